@@ -139,6 +139,18 @@ int rwkv_quantize_u8(rwkv_stream_t stream, const float *weight,
                      int64_t n_out, int64_t n_in,
                      uint8_t *codes, float *range, double *offset);
 
+/* The same codes, ranges and offsets (the offset up to the order in which its
+ * fractions are summed), written straight in any of the three layouts: codes
+ * [n_in, n_out], packed (rwkv_pack_u8's) and packed16 (rwkv_pack_m16's); a NULL
+ * layout is not written, at least one is.  workspace:
+ * rwkv_quantize_workspace_bytes(n_out, n_in) bytes, 8-byte aligned. */
+size_t rwkv_quantize_workspace_bytes(int64_t n_out, int64_t n_in);
+int rwkv_quantize_layouts(rwkv_stream_t stream, const float *weight,
+                          int64_t n_out, int64_t n_in, uint8_t *codes,
+                          uint8_t *packed, uint8_t *packed16,
+                          float *range, double *offset,
+                          void *workspace, size_t workspace_bytes);
+
 /* Device layout the matvec/GEMM kernels stream: 1 KiB blocks of 8 output
  * columns x 128 input rows, blocks ordered [ceil(n_out/8)][ceil(n_in/128)],
  * zero padded.  Within a block, byte 16*(8*s + c) + 4*m + e holds

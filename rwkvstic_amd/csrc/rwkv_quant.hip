@@ -82,6 +82,232 @@ quantize_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in,
 }
 
 // ---------------------------------------------------------------------------
+// The same quantiser for callers with a workspace: four launches that cut the matrix both ways, and the codes leave
+// in any of the three layouts straight from the encoding pass.
+//
+// Bound: memory (the float32 matrix twice, the second time mostly from the memory-side cache, the codes once per
+// layout).  quantize_kernel walks all rows with one workgroup per 64 channels, 40 workgroups at 2560 channels, and
+// the packed layouts then read its codes back byte by byte.  The seven matrices of a layer of width 2560: 5.14 ms
+// that way, 0.315 ms here (host calls included; the 511 MB at copy rate: 0.108).
+//
+//   quant_minmax_kernel   256 channels x one of the row splits: partial minimum and maximum
+//   quant_scale_kernel    one channel per thread: partials -> lo, range, 1 / range
+//   quant_encode_kernel   128 channels x kEncRows rows at a time: codes, layouts, partial sums of the fractions
+//   quant_offset_kernel   fractions in a fixed order -> offset
+// ---------------------------------------------------------------------------
+constexpr int kEncRows = 64;            // rows of one LDS tile: 8 blocks of the P8 layout, 4 x 2 of the M16 layout
+constexpr int kMinMaxSplits = 32;       // enough workgroups at 2560 channels (320); more only lengthens quant_scale_kernel
+
+struct QuantWs {
+    float2 *mm;                 // [splits][n_in]
+    double *lo, *ran, *inv;     // [n_in] each
+    double *frac;               // [parts][n_in]
+    int64_t splits, split_rows; // of the minimum / maximum pass
+    int64_t parts, part_rows;   // of the encoding pass: part_rows a multiple of kEncRows
+    size_t bytes;
+};
+static QuantWs quant_carve(int64_t n_out, int64_t n_in, void *ws) {
+    QuantWs q;
+    q.split_rows = round_up(ceil_div(n_out, kMinMaxSplits), 4);
+    q.splits = ceil_div(n_out, q.split_rows);
+    // one tile per workgroup until there are two workgroups per compute unit, then up to four
+    int64_t tiles = ceil_div(n_out, kEncRows) * ceil_div(n_in, 128) / 512;
+    tiles = tiles < 1 ? 1 : tiles > 4 ? 4 : tiles;
+    q.part_rows = kEncRows * tiles;
+    q.parts = ceil_div(n_out, q.part_rows);
+    unsigned char *p = static_cast<unsigned char *>(ws);
+    size_t at = 0;
+    auto take = [&](int64_t bytes) { unsigned char *r = p + at; at += (size_t)round_up(bytes, 256); return r; };
+    q.mm = reinterpret_cast<float2 *>(take(q.splits * n_in * 8));
+    q.lo = reinterpret_cast<double *>(take(n_in * 8));
+    q.ran = reinterpret_cast<double *>(take(n_in * 8));
+    q.inv = reinterpret_cast<double *>(take(n_in * 8));
+    q.frac = reinterpret_cast<double *>(take(q.parts * n_in * 8));
+    q.bytes = at;
+    return q;
+}
+
+// Four consecutive channels of a row; channels past the end read as `pad`.
+template <bool VEC>
+__device__ __forceinline__ float4 weight4(const float *__restrict__ row, int64_t j, int64_t n_in, float pad) {
+    if (VEC) return j < n_in ? *reinterpret_cast<const float4 *>(row + j) : make_float4(pad, pad, pad, pad);
+    return make_float4(j < n_in ? row[j] : pad, j + 1 < n_in ? row[j + 1] : pad, j + 2 < n_in ? row[j + 2] : pad,
+                       j + 3 < n_in ? row[j + 3] : pad);
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(256)
+quant_minmax_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, QuantWs q) {
+    __shared__ float4 slo[4][64], shi[4][64];
+    const int cq = threadIdx.x & 63, rg = threadIdx.x >> 6;
+    const int64_t j = (int64_t)blockIdx.x * 256 + 4 * cq;
+    const int64_t k0 = (int64_t)blockIdx.y * q.split_rows, k1 = min(k0 + q.split_rows, n_out);
+    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, INFINITY), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+    if (j < n_in) {
+        constexpr int U = 8;                // rows in flight per thread
+        for (int64_t k = k0 + rg; k < k1; k += 4 * U) {
+            float4 x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)     // past the end: the last row again, which changes no extremum
+                x[u] = weight4<VEC>(W + min(k + 4 * u, k1 - 1) * n_in, j, n_in, 0.f);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                lo.x = fminf(lo.x, x[u].x); lo.y = fminf(lo.y, x[u].y); lo.z = fminf(lo.z, x[u].z); lo.w = fminf(lo.w, x[u].w);
+                hi.x = fmaxf(hi.x, x[u].x); hi.y = fmaxf(hi.y, x[u].y); hi.z = fmaxf(hi.z, x[u].z); hi.w = fmaxf(hi.w, x[u].w);
+            }
+        }
+    }
+    slo[rg][cq] = lo; shi[rg][cq] = hi;
+    __syncthreads();
+    const int64_t jj = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (jj < n_in) {
+        const float *l = reinterpret_cast<const float *>(slo), *h = reinterpret_cast<const float *>(shi);
+        const int t = threadIdx.x;
+        q.mm[(int64_t)blockIdx.y * n_in + jj] = make_float2(fminf(fminf(l[t], l[256 + t]), fminf(l[512 + t], l[768 + t])),
+                                                            fmaxf(fmaxf(h[t], h[256 + t]), fmaxf(h[512 + t], h[768 + t])));
+    }
+}
+
+__global__ void __launch_bounds__(64)
+quant_scale_kernel(int64_t n_in, QuantWs q) {
+    const int64_t j = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (j >= n_in) return;
+    float lo = INFINITY, hi = -INFINITY;
+#pragma unroll 8
+    for (int s = 0; s < (int)q.splits; ++s) {
+        const float2 v = q.mm[(int64_t)s * n_in + j];
+        lo = fminf(lo, v.x); hi = fmaxf(hi, v.y);
+    }
+    const double ran = ((double)hi - (double)lo) / 255.0;              // matmul.py:31-33, as quantize_kernel
+    q.lo[j] = (double)lo; q.ran[j] = ran; q.inv[j] = 1.0 / ran;
+}
+
+// The correctly rounded quotient d / b from the correctly rounded reciprocal of b (Markstein: a quotient within one
+// unit in the last place is corrected by its remainder; the first step brings d * inv there): the bits of a division
+// at a third of its instructions, with the reciprocal shared by a whole column.
+__device__ __forceinline__ double quotient(double d, double b, double inv) {
+    double x = d * inv;
+    x = fma(fma(-b, x, d), inv, x);
+    return fma(fma(-b, x, d), inv, x);
+}
+
+__device__ __forceinline__ int slot8(int lane) { return lane ^ ((lane >> 3) & 6); }
+__device__ __forceinline__ int slot16(int lane, int half) { return lane ^ (((lane >> 3) & 6) | (half << 3)); }
+
+template <bool VEC>
+__global__ void __launch_bounds__(256)
+quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, QuantWs q,
+                    uint8_t *__restrict__ codes, uint8_t *__restrict__ packed, uint8_t *__restrict__ packed16) {
+    __shared__ uint32_t p8[8][256], m16[8][256];
+    __shared__ double fsum[8][128];
+    const int cq = threadIdx.x & 31, rg = threadIdx.x >> 5;         // four channels, every eighth row
+    const int64_t j0 = (int64_t)blockIdx.x * 128, j = j0 + 4 * cq;
+    double lo[4], ran[4], inv[4], fr[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int64_t je = min(j + e, n_in - 1);
+        lo[e] = q.lo[je]; ran[e] = q.ran[je]; inv[e] = q.inv[je]; fr[e] = 0.0;
+    }
+    const int64_t kbeg = (int64_t)blockIdx.y * q.part_rows, kend = min(kbeg + q.part_rows, n_out);
+    const int64_t n_ct8 = (n_out + 7) >> 3, n_kb8 = (n_in + 127) >> 7, n_ct16 = (n_out + 15) >> 4, n_kb16 = (n_in + 63) >> 6;
+    const bool words = (n_out & 3) == 0 && (reinterpret_cast<uintptr_t>(codes) & 3) == 0;
+    for (int64_t k0 = kbeg; k0 < kend; k0 += kEncRows) {
+        float4 x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = weight4<VEC>(W + min(k0 + rg + 8 * i, n_out - 1) * n_in, j, n_in, 0.f);
+        if (k0 > kbeg) __syncthreads();                             // the tile before has been written out
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float xe[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
+            const bool row = k0 + rg + 8 * i < n_out;
+            uint32_t c4 = 0, live = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (row && j + e < n_in) {
+                    live |= 0x80u << (8 * e);
+                    if (ran[e] > 0.0) {
+                        const double v = quotient((double)xe[e] - lo[e], ran[e], inv[e]);   // matmul.py:32-34
+                        const double t = trunc(v);
+                        c4 |= (uint32_t)(uint8_t)(int)t << (8 * e);                         // matmul.py:21
+                        fr[e] += v - t;                                                     // matmul.py:35
+                    }
+                }
+            }
+            // P8: block i of the tile, lane 8 s + column, dword m, with channel 32 m + 4 s + e of the block; M16: blocks
+            // (i / 2, half of the 128 channels), lane 16 g + column, dword q, code - 128 with padding 0.  In LDS the
+            // columns of a group are permuted (slot8, slot16) so that the 64 stores of a wavefront hit 64 banks.
+            p8[i][slot8(8 * (cq & 7) + rg) * 4 + (cq >> 3)] = c4;
+            m16[(i >> 1) * 2 + (cq >> 4)][slot16(16 * ((cq & 15) >> 2) + rg + 8 * (i & 1), cq >> 4) * 4 + (cq & 3)] = c4 ^ live;
+        }
+        __syncthreads();
+        const int b = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+        for (int h = 0; h < 8; h += 4) {
+            const int i = b + h;
+            if (packed) {
+                const int64_t ct = (k0 >> 3) + i;
+                if (ct < n_ct8)
+                    *reinterpret_cast<uint4 *>(packed + (ct * n_kb8 + blockIdx.x) * 1024 + lane * 16) = *reinterpret_cast<const uint4 *>(&p8[i][slot8(lane) * 4]);
+            }
+            if (packed16) {
+                const int64_t ct = (k0 >> 4) + (i >> 1), kb = (int64_t)blockIdx.x * 2 + (i & 1);
+                if (ct < n_ct16 && kb < n_kb16)
+                    *reinterpret_cast<uint4 *>(packed16 + (ct * n_kb16 + kb) * 1024 + lane * 16) = *reinterpret_cast<const uint4 *>(&m16[i][slot16(lane, i & 1) * 4]);
+            }
+        }
+        if (codes) {
+            // [n_in][n_out]: channel r of the tile, 16 lanes of four rows each (gathered from the P8 tile's bytes)
+            const uint8_t *tile = reinterpret_cast<const uint8_t *>(p8);
+            for (int r = threadIdx.x >> 4; r < 128; r += 16) {
+                const int kq = 4 * (threadIdx.x & 15);
+                uint32_t v = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int k = kq + e;
+                    v |= (uint32_t)tile[(k >> 3) * 1024 + slot8(8 * ((r & 31) >> 2) + (k & 7)) * 16 + 4 * (r >> 5) + (r & 3)] << (8 * e);
+                }
+                const int64_t jr = j0 + r, k = k0 + kq;
+                if (jr < n_in) {
+                    uint8_t *o = codes + jr * n_out + k;
+                    if (words && k + 4 <= n_out) *reinterpret_cast<uint32_t *>(o) = v;
+                    else
+                        for (int e = 0; e < 4; ++e)
+                            if (k + e < n_out) o[e] = (uint8_t)(v >> (8 * e));
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) fsum[rg][4 * cq + e] = fr[e];
+    __syncthreads();
+    if (threadIdx.x < 128 && j0 + threadIdx.x < n_in) {
+        double s = 0.0;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) s += fsum[r][threadIdx.x];
+        q.frac[(int64_t)blockIdx.y * n_in + j0 + threadIdx.x] = s;
+    }
+}
+
+__global__ void __launch_bounds__(256)
+quant_offset_kernel(int64_t n_out, int64_t n_in, QuantWs q, float *__restrict__ range, double *__restrict__ offset) {
+    __shared__ double part[4][64];
+    const int jx = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int64_t j = (int64_t)blockIdx.x * 64 + jx;
+    double s = 0.0;
+    if (j < n_in) {
+#pragma unroll 8
+        for (int p = g; p < (int)q.parts; p += 4) s += q.frac[(int64_t)p * n_in + j];
+    }
+    part[g][jx] = s;
+    __syncthreads();
+    if (g == 0 && j < n_in) {
+        s = (part[0][jx] + part[1][jx]) + (part[2][jx] + part[3][jx]);
+        offset[j] = q.lo[j] + (s / (double)n_out) * q.ran[j];          // matmul.py:36-37
+        range[j] = (float)q.ran[j];                                    // matmul.py:39
+    }
+}
+
+// ---------------------------------------------------------------------------
 // pack / unpack: one thread per 16-byte lane chunk of a block.
 // ---------------------------------------------------------------------------
 template <bool PACK>
@@ -204,6 +430,41 @@ int rwkv_quantize_u8(rwkv_stream_t stream, const float *weight, int64_t n_out, i
     hipLaunchKernelGGL(quantize_kernel, dim3((unsigned)ceil_div(n_in, 64)), dim3(256), 0,
                        (hipStream_t)stream, weight, n_out, n_in, codes, range, offset);
     RWKV_CHECK_LAUNCH("quantize_kernel");
+    return RWKV_OK;
+}
+
+size_t rwkv_quantize_workspace_bytes(int64_t n_out, int64_t n_in) {
+    if (n_out <= 0 || n_in <= 0) return 0;
+    return quant_carve(n_out, n_in, nullptr).bytes;
+}
+
+int rwkv_quantize_layouts(rwkv_stream_t stream, const float *weight, int64_t n_out, int64_t n_in, uint8_t *codes,
+                          uint8_t *packed, uint8_t *packed16, float *range, double *offset, void *workspace,
+                          size_t workspace_bytes) {
+    RWKV_CHECK_ARG(weight && range && offset && workspace, "rwkv_quantize_layouts: null pointer");
+    RWKV_CHECK_ARG(codes || packed || packed16, "rwkv_quantize_layouts: no output layout");
+    RWKV_CHECK_ARG(n_out > 0 && n_in > 0 && n_out < (1ll << 30) && n_in < (1ll << 30), "rwkv_quantize_layouts: bad sizes");
+    RWKV_CHECK_ALIGN(weight, 4);
+    RWKV_CHECK_ALIGN(range, 4);
+    RWKV_CHECK_ALIGN(offset, 8);
+    RWKV_CHECK_ALIGN(packed, 16);
+    RWKV_CHECK_ALIGN(packed16, 16);
+    RWKV_CHECK_ALIGN(workspace, 8);
+    const QuantWs q = quant_carve(n_out, n_in, workspace);
+    if (workspace_bytes < q.bytes)
+        return set_error(RWKV_ERR_WORKSPACE, "rwkv_quantize_layouts: workspace of %zu bytes needed, %zu given", q.bytes, workspace_bytes);
+    const hipStream_t st = (hipStream_t)stream;
+    const bool vec = n_in % 4 == 0 && reinterpret_cast<uintptr_t>(weight) % 16 == 0;
+    const dim3 mg((unsigned)ceil_div(n_in, 256), (unsigned)q.splits), eg((unsigned)ceil_div(n_in, 128), (unsigned)q.parts);
+    if (q.parts > 65535)
+        return set_error(RWKV_ERR_SIZE, "rwkv_quantize_layouts: n_out %lld is more than one launch covers", (long long)n_out);
+    if (vec) hipLaunchKernelGGL(quant_minmax_kernel<true>, mg, dim3(256), 0, st, weight, n_out, n_in, q);
+    else hipLaunchKernelGGL(quant_minmax_kernel<false>, mg, dim3(256), 0, st, weight, n_out, n_in, q);
+    hipLaunchKernelGGL(quant_scale_kernel, dim3((unsigned)ceil_div(n_in, 64)), dim3(64), 0, st, n_in, q);
+    if (vec) hipLaunchKernelGGL(quant_encode_kernel<true>, eg, dim3(256), 0, st, weight, n_out, n_in, q, codes, packed, packed16);
+    else hipLaunchKernelGGL(quant_encode_kernel<false>, eg, dim3(256), 0, st, weight, n_out, n_in, q, codes, packed, packed16);
+    hipLaunchKernelGGL(quant_offset_kernel, dim3((unsigned)ceil_div(n_in, 64)), dim3(256), 0, st, n_out, n_in, q, range, offset);
+    RWKV_CHECK_LAUNCH("quant_encode_kernel");
     return RWKV_OK;
 }
 

@@ -30,9 +30,9 @@ class QuantMatrix:
     def from_weight(cls, weight: torch.Tensor, device, m16: bool = True, stream: bool = False) -> "QuantMatrix":
         """``weight[out, in]`` in any float dtype, on any device."""
         w = weight.to(device=device, dtype=torch.float32).contiguous()
-        codes, rng, off = ops.quantize(w)
-        n_in, n_out = codes.shape
-        return cls(ops.pack(codes), rng, off, n_in, n_out, ops.pack_m16(codes) if m16 else None)._placed(stream)
+        n_out, n_in = w.shape
+        packed, packed16, rng, off = ops.quantize_packed(w, m16)
+        return cls(packed, rng, off, n_in, n_out, packed16)._placed(stream)
 
     @classmethod
     def from_codes(cls, codes: torch.Tensor, rng: torch.Tensor, off: torch.Tensor, device, stream: bool = False) -> "QuantMatrix":

@@ -127,17 +127,35 @@ def register_torch_ops() -> None:
 
 
 # ---------------------------------------------------------------- quantiser / layouts
+def _quantize(weight: torch.Tensor, codes: bool, packed: bool, packed16: bool):
+    """One quantising pass, its codes written in the layouts asked for (None for the others)."""
+    _req(weight, torch.float32, "weight"); _contig(weight, "weight")
+    n_out, n_in = weight.shape
+    L, dev = N.lib(), weight.device
+    c = torch.empty((n_in, n_out), dtype=torch.uint8, device=dev) if codes else None
+    p = torch.empty(L.rwkv_packed_bytes(n_in, n_out), dtype=torch.uint8, device=dev) if packed else None
+    p16 = torch.empty(L.rwkv_packed_m16_bytes(n_in, n_out), dtype=torch.uint8, device=dev) if packed16 else None
+    rng = torch.empty(n_in, dtype=torch.float32, device=dev)
+    off = torch.empty(n_in, dtype=torch.float64, device=dev)
+    ws = torch.empty(L.rwkv_quantize_workspace_bytes(n_out, n_in), dtype=torch.uint8, device=dev)
+    N.check(L.rwkv_quantize_layouts(_stream(), weight.data_ptr(), n_out, n_in, c.data_ptr() if codes else None,
+                                    p.data_ptr() if packed else None, p16.data_ptr() if packed16 else None,
+                                    rng.data_ptr(), off.data_ptr(), ws.data_ptr(), ws.numel()))
+    return c, p, p16, rng, off
+
+
 def quantize(weight: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """``weight[out, in]`` float32 -> ``(codes[in, out] uint8, range[in] float32, offset[in] float64)``
     (MM8.QuantizeMatrix, matmul.py:24-40)."""
-    _req(weight, torch.float32, "weight"); _contig(weight, "weight")
-    n_out, n_in = weight.shape
-    codes = torch.empty((n_in, n_out), dtype=torch.uint8, device=weight.device)
-    rng = torch.empty(n_in, dtype=torch.float32, device=weight.device)
-    off = torch.empty(n_in, dtype=torch.float64, device=weight.device)
-    N.check(N.lib().rwkv_quantize_u8(_stream(), weight.data_ptr(), n_out, n_in,
-                                     codes.data_ptr(), rng.data_ptr(), off.data_ptr()))
+    codes, _, _, rng, off = _quantize(weight, True, False, False)
     return codes, rng, off
+
+
+def quantize_packed(weight: torch.Tensor, m16: bool = True):
+    """``quantize`` without the intermediate codes: ``(packed, packed16 or None, range, offset)``, the layouts being
+    those of ``pack`` and (``m16``) ``pack_m16``."""
+    _, packed, packed16, rng, off = _quantize(weight, False, True, m16)
+    return packed, packed16, rng, off
 
 
 def pack(codes: torch.Tensor) -> torch.Tensor:

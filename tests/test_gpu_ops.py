@@ -46,6 +46,25 @@ def test_quantiser_constant_channel(ops):
     assert int(codes[3].max()) == 0 and float(rng[3]) == 0.0 and float(off[3]) == 0.125
 
 
+# one tile, its edges on both sides, several tiles per workgroup, ragged rows that rule out 16-byte loads
+@pytest.mark.parametrize("shape", [(1, 1), (64, 128), (63, 127), (65, 129), (300, 132), (1000, 257), (10240, 2560), (50277, 768)])
+def test_quantised_layouts_are_the_packed_codes(ops, shape):
+    _say(f"quantise to layouts {shape}")
+    g = torch.Generator().manual_seed(shape[0] + 5 * shape[1])
+    W = (torch.randn(*shape, generator=g) * 0.02).cuda()
+    W[:, -1] = 0.25
+    codes, rng, off = ops.quantize(W)
+    packed, packed16, rng2, off2 = ops.quantize_packed(W)
+    assert torch.equal(packed, ops.pack(codes)) and torch.equal(packed16, ops.pack_m16(codes))
+    assert torch.equal(rng, rng2) and torch.equal(off, off2)
+    assert ops.quantize_packed(W, m16=False)[1] is None
+    c_ref, r_ref, o_ref = O.quantize_matrix(W.cpu())
+    live = r_ref > 0                                    # (the oracle divides by the range of a constant channel)
+    assert torch.equal(codes.cpu()[live], c_ref[live]) and torch.equal(rng.cpu()[live], r_ref[live])
+    assert torch.allclose(off.cpu()[live], o_ref[live], rtol=1e-13, atol=1e-300)
+    assert int(codes[-1].max()) == 0 and float(off[-1]) == 0.25
+
+
 def test_pack_strided_and_ragged(ops):
     big = torch.randint(0, 256, (200, 400), dtype=torch.uint8, device="cuda")
     view = big[:130, :77]                      # stride 400, ragged in both dims
