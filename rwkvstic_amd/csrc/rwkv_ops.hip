@@ -579,6 +579,95 @@ wkv_f64_ref_kernel(int B, int T, int C, const double *__restrict__ w, const doub
     bb[idx] = bsum * e;
 }
 
+// The same recurrence for longer sequences.  It is linear in (aa, bb), so a block of kW64NC chunks of kW64SB steps is
+// summed up by kW64NC threads per channel side by side, a scan over the chunks in LDS gives each thread the state its
+// chunk starts from, and every thread writes the outputs of its own steps from there (the steps stay in registers
+// between the two passes, k and v are read once).
+//
+// Bound: the chain of float64 exponentials (some fifty dependent instructions each) where there are few channels,
+// memory with many.  32 channels per workgroup keep a row's piece at 256 bytes.  2560 channels, 256 steps: 15.4 us
+// against 101 us of the serial kernel, which stays for sequences of fewer than kW64MinT steps: one pass of the scan
+// costs as much as about that many serial steps.
+constexpr int kW64SB = 8, kW64MinT = 12;
+
+template <int NC>
+__global__ void __launch_bounds__(NC * 32)
+wkv_f64_scan_kernel(int T, int C, const double *__restrict__ w, const double *__restrict__ u, const double *__restrict__ k,
+                    const double *__restrict__ v, double *__restrict__ y, double *__restrict__ aa, double *__restrict__ bb) {
+    __shared__ double sa[2][NC][32], sb[2][NC][32], sp[2][NC][32];
+    constexpr int kBlk = NC * kW64SB;
+    // the last round of the scan writes buffer 1, so that the next block's summaries may enter buffer 0 while other
+    // wavefronts still read the result
+    static_assert(NC == 8 || NC == 32, "an odd number of scan rounds");
+    const int per_b = (C + 31) / 32, b = blockIdx.x / per_b;
+    const int ch = threadIdx.x & 31, j = threadIdx.x >> 5;
+    const int cx = (blockIdx.x % per_b) * 32 + ch;
+    const bool live = cx < C;
+    const int c = live ? cx : C - 1;
+    const size_t base = (size_t)b * T * C + c;
+    const double wc = w[c], uc = u[c];
+    double ca = aa[(size_t)b * C + c], cb = bb[(size_t)b * C + c], cp = 0.0;      // naive (aa, bb) == shifted (aa, bb, pp = 0)
+    if (!(cb > 0.0)) cp = -1e300;                        // empty state: let the first token dominate exactly
+    for (int tb = 0; tb < T; tb += kBlk) {
+        const int t0 = min(tb + j * kW64SB, T), n = min(kW64SB, T - t0);
+        double kc[kW64SB], vc[kW64SB];
+#pragma unroll
+        for (int i = 0; i < kW64SB; ++i) {
+            const size_t o = base + (size_t)min(t0 + i, T - 1) * C;
+            kc[i] = k[o]; vc[i] = v[o];
+        }
+        // the chunk from an empty state, a direct sum: step i contributes e^{k_i + (n - i) w} by the chunk's end
+        double x[kW64SB], p = -1e300, a = 0.0, s = 0.0;
+#pragma unroll
+        for (int i = 0; i < kW64SB; ++i) {
+            x[i] = i < n ? kc[i] + (double)(n - i) * wc : -1e300;
+            p = fmax(p, x[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < kW64SB; ++i) {
+            const double f = i < n ? exp(x[i] - p) : 0.0;
+            a = fma(f, vc[i], a);
+            s += f;
+        }
+        if (j == 0) {                                    // the state before the block, decayed over the first chunk
+            const double e = cp + (double)n * wc, pn = fmax(e, p);
+            const double f0 = exp(e - pn), f1 = exp(p - pn);
+            a = f0 * ca + f1 * a; s = f0 * cb + f1 * s; p = pn;
+        }
+        sa[0][j][ch] = a; sb[0][j][ch] = s; sp[0][j][ch] = p;
+        __syncthreads();
+        int buf = 0;
+#pragma unroll
+        for (int d = 1; d < NC; d <<= 1, buf ^= 1) {     // inclusive scan: add what ends d chunks earlier, decayed to here
+            if (j >= d) {
+                const int len = t0 + n - min(tb + (j - d + 1) * kW64SB, T);
+                const double e = sp[buf][j - d][ch] + (double)len * wc, pn = fmax(e, p);
+                const double f0 = exp(e - pn), f1 = exp(p - pn);
+                a = f0 * sa[buf][j - d][ch] + f1 * a;
+                s = f0 * sb[buf][j - d][ch] + f1 * s;
+                p = pn;
+            }
+            sa[buf ^ 1][j][ch] = a; sb[buf ^ 1][j][ch] = s; sp[buf ^ 1][j][ch] = p;
+            __syncthreads();
+        }
+        if (j > 0) { a = sa[buf][j - 1][ch]; s = sb[buf][j - 1][ch]; p = sp[buf][j - 1][ch]; }
+        else { a = ca; s = cb; p = cp; }
+        ca = sa[buf][NC - 1][ch]; cb = sb[buf][NC - 1][ch]; cp = sp[buf][NC - 1][ch];
+#pragma unroll
+        for (int i = 0; i < kW64SB; ++i) {
+            if (i < n) {
+                const double yv = wkv_step<double>(wc, uc, kc[i], vc[i], a, s, p);
+                if (live) y[base + (size_t)(t0 + i) * C] = yv;
+            }
+        }
+    }
+    if (live && j == 0) {
+        const double e = exp(cp);
+        aa[(size_t)b * C + c] = ca * e;
+        bb[(size_t)b * C + c] = cb * e;
+    }
+}
+
 // First index of the maximum (torch.argmax tie rule is unspecified; greedy
 // decoding here takes the lowest index).
 __global__ void __launch_bounds__(1024)
@@ -608,98 +697,124 @@ argmax_f64_kernel(const double *__restrict__ logits, int V, int64_t *__restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Reference layout w[n_in][n_out] (row stride w_stride), operators32.cu:18-83.
-// Workgroup (ct, sp): columns 256*ct .. +255, rows of split sp.  Lane cx of
-// wave ky handles VEC consecutive columns of rows ky, ky+4, ...; x[j]*r[j] is
-// wave-uniform.  Partials go to scratch[sp][m][k]; mm8_ref_reduce_kernel adds
-// them in split order and accumulates into y (deterministic).
+// Reference layout w[n_in][n_out] (row stride w_stride), operators32.cu:18-83: y[k] += sum_j w[j][k] * (x[j] r[j]).
+//
+// Bound: memory (n_in x n_out bytes, once), in practice one round of loads and a second launch.  A workgroup takes 128
+// columns (whole cache lines of the rows) and up to 256 rows; a lane requests 16 bytes of each of its up to eight rows
+// before the first is used.  One compute unit draws only some 40 bytes per nanosecond, so the rows are cut until the
+// grid covers the device; the slices are added in order by mm8_ref_reduce_kernel (deterministic).  The two
+// launches of [2560 x 2560] take 7.2 + 3.5 us, of [2560 x 10240] and [10240 x 2560] 13.8 + 3.5 us (26 MB at copy rate:
+// 5.5); with 4-byte loads, one row after the other, and a reduction of one thread per column the three averaged
+// 14.3 + 9.1 us.  64 columns and all 2560 rows to a workgroup, which needs no second launch: 16 us on average.
+// Non-temporal loads and row slices dealt out to the XCDs change nothing.
 // ---------------------------------------------------------------------------
-constexpr int kRefSplitRows = 128;
+constexpr int kRefSplitRows = 128;      // rows per slice the workspace is sized for
+constexpr int kRefThreads = 256, kRefRowsPass = kRefThreads / 8, kRefPasses = 8;
+
+template <typename T>
+struct Mm8RefArgs {
+    int n_in, n_out, rows_per_split, splits;
+    const T *x[3], *r[3];
+    const uint8_t *w[3];
+    int64_t stride[3];
+    T *y[3];
+    T *scratch;                 // [split][product][n_out]
+};
 
 // T: float (operators32.cu) or double (operators.cu:58-80, the dispatch of wrapper.cpp:60-77): the type of x, r, y and
-// of the sums.
-template <typename T, int NM, int VEC>
-__global__ void __launch_bounds__(kThreads)
-mm8_ref_partial_kernel(int n_in, int n_out,
-                       const T *x0, const T *x1, const T *x2,
-                       const uint8_t *w0, const uint8_t *w1, const uint8_t *w2,
-                       int64_t s0, int64_t s1, int64_t s2,
-                       const T *r0, const T *r1, const T *r2,
-                       T *__restrict__ scratch) {
-    __shared__ T xs[NM][kRefSplitRows];
-    __shared__ T red[kWaves][NM][64 * VEC];
-    const T *xp[3] = {x0, x1, x2};
-    const T *rp[3] = {r0, r1, r2};
-    const uint8_t *wp[3] = {w0, w1, w2};
-    const int64_t sp_[3] = {s0, s1, s2};
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int j0 = blockIdx.y * kRefSplitRows;
-    const int rows = min(kRefSplitRows, n_in - j0);
-    for (int i = threadIdx.x; i < NM * kRefSplitRows; i += kThreads) {
-        const int m = i / kRefSplitRows, jj = i % kRefSplitRows;
-        // operators32.cu:33-36 multiplies x[j] * (w * r[j]); here x[j]*r[j] is
-        // formed once per row (same rounding as the reference CPU path,
-        // matmul.py:131).
-        xs[m][jj] = jj < rows ? xp[m][j0 + jj] * rp[m][j0 + jj] : (T)0;
-    }
-    __syncthreads();
-    const int k0 = (blockIdx.x * 64 + lane) * VEC;
-    T acc[NM][VEC];
+// of the sums.  WIDE: at least 16 columns; narrower matrices are read byte by byte.
+template <typename T, bool WIDE>
+__global__ void __launch_bounds__(kRefThreads) mm8_ref_kernel(const Mm8RefArgs<T> a) {
+    __shared__ T xs[kRefPasses * kRefRowsPass];
+    __shared__ T red[kRefThreads / 64][128];
+    const int m = blockIdx.z, tid = threadIdx.x;
+    const T *x = m == 0 ? a.x[0] : m == 1 ? a.x[1] : a.x[2], *r = m == 0 ? a.r[0] : m == 1 ? a.r[1] : a.r[2];
+    const uint8_t *w = m == 0 ? a.w[0] : m == 1 ? a.w[1] : a.w[2];
+    const int64_t stride = m == 0 ? a.stride[0] : m == 1 ? a.stride[1] : a.stride[2];
+    const int j0 = blockIdx.y * a.rows_per_split, rows = min(a.rows_per_split, a.n_in - j0);
+    const int q = tid & 7, row0 = tid >> 3;
+    const int c0 = blockIdx.x * 128 + 16 * q;            // this lane's 16 columns
+    // the last piece of a row that is not a multiple of 16 columns is read 16 bytes from the row's end (its first
+    // columns belong to the piece before and are dropped)
+    const int cl = WIDE ? min(c0, a.n_out - 16) : 0;
+    // x and r are requested ahead of the weights: a wavefront's loads return in order
+    const int jx = j0 + min(tid, rows - 1);
+    const T xv = x[jx], rv = r[jx];
+    typedef uint32_t Piece __attribute__((ext_vector_type(4), aligned(1)));     // (rows may start anywhere)
+    Piece wv[kRefPasses];
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
+    for (int p = 0; p < kRefPasses; ++p) {
+        if (p * kRefRowsPass >= rows) break;                            // (uniform)
+        const int j = j0 + min(row0 + p * kRefRowsPass, rows - 1);      // past the end: the last row again, times zero
+        const uint8_t *row = w + (size_t)j * stride + cl;
+        if (WIDE) wv[p] = *reinterpret_cast<const Piece *>(row);
+        else {
+            uint32_t d[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) acc[m][e] = (T)0;
-    if (k0 < n_out) {
-        for (int jj = wave; jj < rows; jj += kWaves) {
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                const uint8_t *row = wp[m] + (size_t)(j0 + jj) * sp_[m] + k0;
-                const T xv = xs[m][jj];
-                if (VEC == 4) {
-                    uint32_t d;
-                    if (k0 + 4 <= n_out) {
-                        d = *reinterpret_cast<const uint32_t *>(row);
-                    } else {   // ragged last group: never read past the row
-                        d = 0;
-                        for (int e = 0; k0 + e < n_out; ++e) d |= (uint32_t)row[e] << (8 * e);
-                    }
-                    acc[m][0] = fma((T)ubyte0(d), xv, acc[m][0]);
-                    acc[m][1] = fma((T)ubyte1(d), xv, acc[m][1]);
-                    acc[m][2] = fma((T)ubyte2(d), xv, acc[m][2]);
-                    acc[m][3] = fma((T)ubyte3(d), xv, acc[m][3]);
-                } else {
-                    acc[m][0] = fma((T)row[0], xv, acc[m][0]);
-                }
-            }
+            for (int e = 0; e < 15; ++e)
+                if (e < a.n_out) d[e >> 2] |= (uint32_t)row[e] << (8 * (e & 3));
+            wv[p] = Piece{d[0], d[1], d[2], d[3]};
         }
     }
-#pragma unroll
-    for (int m = 0; m < NM; ++m)
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) red[wave][m][lane * VEC + e] = acc[m][e];
+    // operators32.cu:33-36 multiplies x[j] * (w * r[j]); here x[j]*r[j] is formed once per row (same rounding as the
+    // reference CPU path, matmul.py:131)
+    xs[tid] = tid < rows ? xv * rv : (T)0;
     __syncthreads();
-    for (int i = threadIdx.x; i < NM * 64 * VEC; i += kThreads) {
-        const int m = i / (64 * VEC), kk = i % (64 * VEC);
-        const int k = blockIdx.x * 64 * VEC + kk;
-        if (k < n_out)
-            scratch[((size_t)blockIdx.y * NM + m) * n_out + k] =
-                (red[0][m][kk] + red[1][m][kk]) + (red[2][m][kk] + red[3][m][kk]);
+    T acc[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = (T)0;
+#pragma unroll
+    for (int p = 0; p < kRefPasses; ++p) {
+        if (p * kRefRowsPass >= rows) break;
+        const T xr = xs[row0 + p * kRefRowsPass];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t d = wv[p][i];
+            acc[4 * i] = fma((T)ubyte0(d), xr, acc[4 * i]);
+            acc[4 * i + 1] = fma((T)ubyte1(d), xr, acc[4 * i + 1]);
+            acc[4 * i + 2] = fma((T)ubyte2(d), xr, acc[4 * i + 2]);
+            acc[4 * i + 3] = fma((T)ubyte3(d), xr, acc[4 * i + 3]);
+        }
     }
+    // Sum over the 8 rows of the wavefront: at each step a lane keeps one half of its columns and hands the other to
+    // the lane that keeps those, so 14 exchanges leave every lane with two of its piece's columns.
+    const int lane = tid & 63, wave = tid >> 6, s = lane >> 3;
+#pragma unroll
+    for (int h = 8; h >= 2; h >>= 1) {
+        const int off = 64 / h;                          // 8, 16, 32
+        const bool up = lane & off;
+        T got[8];
+#pragma unroll
+        for (int e = 0; e < h; ++e) got[e] = __shfl_xor(up ? acc[e] : acc[e + h], off, 64);
+#pragma unroll
+        for (int e = 0; e < h; ++e) acc[e] = (up ? acc[e + h] : acc[e]) + got[e];
+    }
+    const int e = 8 * (s & 1) + 4 * ((s >> 1) & 1) + 2 * (s >> 2);
+    red[wave][16 * q + e] = acc[0];
+    red[wave][16 * q + e + 1] = acc[1];
+    __syncthreads();
+    if (tid >= 128) return;
+    const T sum = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
+    const int piece = blockIdx.x * 128 + (tid & ~15), first = WIDE ? min(piece, a.n_out - 16) : 0, k = first + (tid & 15);
+    if (k < piece || k >= a.n_out) return;
+    a.scratch[((size_t)blockIdx.y * gridDim.z + m) * a.n_out + k] = sum;
 }
 
-template <typename T, int NM>
-__global__ void __launch_bounds__(256)
-mm8_ref_reduce_kernel(int n_out, int n_split, const T *__restrict__ scratch,
-                      T *y0, T *y1, T *y2) {
-    T *yp[3] = {y0, y1, y2};
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n_out) return;
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        T s = (T)0;
-        for (int sp = 0; sp < n_split; ++sp) s += scratch[((size_t)sp * NM + m) * n_out + k];
-        yp[m][k] += s;   // the reference accumulates into y (operators32.cu:38)
+template <typename T>
+__global__ void __launch_bounds__(256) mm8_ref_reduce_kernel(const Mm8RefArgs<T> a) {
+    __shared__ T part[4][64];
+    const int kx = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int k = blockIdx.x * 64 + kx, m = blockIdx.y, nm = gridDim.y;
+    T s = (T)0;
+    if (k < a.n_out) {
+#pragma unroll 8
+        for (int sp = g; sp < a.splits; sp += 4) s += a.scratch[((size_t)sp * nm + m) * a.n_out + k];
     }
+    part[g][kx] = s;
+    __syncthreads();
+    if (g > 0 || k >= a.n_out) return;
+    T *y = m == 0 ? a.y[0] : m == 1 ? a.y[1] : a.y[2];
+    y[k] += (part[0][kx] + part[1][kx]) + (part[2][kx] + part[3][kx]);      // the reference accumulates into y (operators32.cu:38)
 }
 
 template <typename T>
@@ -707,33 +822,33 @@ static int mm8_ref_launch(hipStream_t st, int nm, int64_t n_in, int64_t n_out,
                           const T *const x[3], const uint8_t *const w[3], const int64_t stride[3],
                           T *const y[3], const T *const r[3], void *ws, size_t ws_bytes) {
     RWKV_CHECK_ARG(n_in > 0 && n_out > 0 && n_in < (1 << 30) && n_out < (1 << 30), "mm8: bad sizes");
-    bool vec4 = true;
+    Mm8RefArgs<T> a;
     for (int m = 0; m < nm; ++m) {
         RWKV_CHECK_ARG(x[m] && w[m] && y[m] && r[m], "mm8: null pointer");
         RWKV_CHECK_ARG(stride[m] >= n_out, "mm8: w_stride < n_out");
         RWKV_CHECK_ALIGN(x[m], sizeof(T)); RWKV_CHECK_ALIGN(y[m], sizeof(T)); RWKV_CHECK_ALIGN(r[m], sizeof(T));
-        if (reinterpret_cast<uintptr_t>(w[m]) % 4 || stride[m] % 4) vec4 = false;
+    }
+    for (int m = 0; m < 3; ++m) {
+        const int i = m < nm ? m : 0;
+        a.x[m] = x[i]; a.r[m] = r[i]; a.w[m] = w[i]; a.stride[m] = stride[i]; a.y[m] = y[i];
     }
     const size_t need = (size_t)(ceil_div(n_in, kRefSplitRows) * nm * n_out) * sizeof(T);
     if (!ws || ws_bytes < need)
         return set_error(RWKV_ERR_WORKSPACE, "mm8: workspace of %zu bytes needed, %zu given", need, ws_bytes);
     RWKV_CHECK_ALIGN(ws, sizeof(T));
-    const int n_split = (int)ceil_div(n_in, kRefSplitRows);
-    T *scratch = static_cast<T *>(ws);
-    const int vec = vec4 ? 4 : 1;
-    dim3 grid((unsigned)ceil_div(n_out, 64 * vec), (unsigned)n_split);
-#define LAUNCH_P(NM, VEC) \
-    hipLaunchKernelGGL((mm8_ref_partial_kernel<T, NM, VEC>), grid, dim3(kThreads), 0, st, (int)n_in, (int)n_out, \
-                       x[0], x[1], x[2], w[0], w[1], w[2], stride[0], stride[1], stride[2], r[0], r[1], r[2], scratch)
-    if (nm == 1) { if (vec4) LAUNCH_P(1, 4); else LAUNCH_P(1, 1); }
-    else         { if (vec4) LAUNCH_P(3, 4); else LAUNCH_P(3, 1); }
-#undef LAUNCH_P
-    RWKV_CHECK_LAUNCH("mm8_ref_partial_kernel");
-    dim3 rgrid((unsigned)ceil_div(n_out, 256));
-    if (nm == 1)
-        hipLaunchKernelGGL((mm8_ref_reduce_kernel<T, 1>), rgrid, dim3(256), 0, st, (int)n_out, n_split, scratch, y[0], y[1], y[2]);
-    else
-        hipLaunchKernelGGL((mm8_ref_reduce_kernel<T, 3>), rgrid, dim3(256), 0, st, (int)n_out, n_split, scratch, y[0], y[1], y[2]);
+    a.n_in = (int)n_in; a.n_out = (int)n_out; a.scratch = static_cast<T *>(ws);
+    // 256 rows per workgroup, 128 (the least the workspace allows) where that leaves compute units without one; the number
+    // of matrices does not count, so that mm8_three gives the bits of three mm8_one
+    const int64_t cols = ceil_div(n_out, 128);
+    a.rows_per_split = kRefPasses * kRefRowsPass;
+    if (cols * ceil_div(n_in, a.rows_per_split) < 256) a.rows_per_split = kRefSplitRows;
+    a.splits = (int)ceil_div(n_in, a.rows_per_split);
+    if (a.splits > 65535) return set_error(RWKV_ERR_SIZE, "mm8: n_in %lld is more than one launch covers", (long long)n_in);
+    const dim3 grid((unsigned)cols, (unsigned)a.splits, (unsigned)nm);
+    if (n_out >= 16) hipLaunchKernelGGL((mm8_ref_kernel<T, true>), grid, dim3(kRefThreads), 0, st, a);
+    else hipLaunchKernelGGL((mm8_ref_kernel<T, false>), grid, dim3(kRefThreads), 0, st, a);
+    RWKV_CHECK_LAUNCH("mm8_ref_kernel");
+    hipLaunchKernelGGL(mm8_ref_reduce_kernel<T>, dim3((unsigned)ceil_div(n_out, 64), (unsigned)nm), dim3(256), 0, st, a);
     RWKV_CHECK_LAUNCH("mm8_ref_reduce_kernel");
     return RWKV_OK;
 }
@@ -861,6 +976,16 @@ int rwkv_wkv_forward_f64(rwkv_stream_t stream, int64_t B, int64_t T, int64_t C,
     RWKV_CHECK_ARG(w && u && k && v && y && aa && bb && pp, "rwkv_wkv_forward_f64: null pointer");
     RWKV_CHECK_ARG(B > 0 && T > 0 && C > 0 && B * C < (1ll << 31) && T < (1ll << 31), "rwkv_wkv_forward_f64: bad sizes");
     RWKV_CHECK_ALIGN(k, 8); RWKV_CHECK_ALIGN(v, 8); RWKV_CHECK_ALIGN(y, 8);
+    if (T >= kW64MinT && B * ceil_div(C, 32) < (1ll << 31)) {
+        const dim3 grid((unsigned)(B * ceil_div(C, 32)));
+        // short sequences: 8 chunks cover them and leave fewer threads idle; long ones: 32 chunks per block
+        if (T <= 8 * kW64SB)
+            hipLaunchKernelGGL(wkv_f64_scan_kernel<8>, grid, dim3(8 * 32), 0, (hipStream_t)stream, (int)T, (int)C, w, u, k, v, y, aa, bb);
+        else
+            hipLaunchKernelGGL(wkv_f64_scan_kernel<32>, grid, dim3(32 * 32), 0, (hipStream_t)stream, (int)T, (int)C, w, u, k, v, y, aa, bb);
+        RWKV_CHECK_LAUNCH("wkv_f64_scan_kernel");
+        return RWKV_OK;
+    }
     hipLaunchKernelGGL(wkv_f64_ref_kernel, dim3((unsigned)ceil_div(B * C, 64)), dim3(64), 0, (hipStream_t)stream,
                        (int)B, (int)T, (int)C, w, u, k, v, y, aa, bb);
     RWKV_CHECK_LAUNCH("wkv_f64_ref_kernel");

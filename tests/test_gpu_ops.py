@@ -198,6 +198,25 @@ def test_mm8_one_reference_semantics(ops, n_in, n_out):
     assert (y.cpu().double() - want).abs().max() <= 2.0 ** -23 * 8 * scale + 1e-6 * y0.abs().max()
 
 
+# 16-byte pieces of rows that start anywhere, the last piece of a row, fewer columns than one piece, slices of 128 rows
+# and (from 256 workgroups on) of 256 rows, whole and ragged ones of both
+@pytest.mark.parametrize("n_in,n_out,pad", [(1, 1, 0), (127, 15, 3), (128, 16, 0), (129, 17, 5), (256, 127, 1), (257, 129, 0),
+                                            (5121, 130, 2), (64, 1100, 7), (2560, 3329, 3), (1800, 4097, 0)])
+def test_mm8_one_edges_against_the_float64_product(ops, n_in, n_out, pad):
+    _say(f"mm8_one edges in={n_in} out={n_out} pad={pad}")
+    g = torch.Generator().manual_seed(n_in * 3 + n_out)
+    big = torch.randint(0, 256, (n_in, n_out + pad), generator=g, dtype=torch.uint8)
+    x, r, y0 = torch.randn(n_in, generator=g), torch.rand(n_in, generator=g) * 1e-3, torch.randn(n_out, generator=g)
+    for dt, eps in ((torch.float32, 2.0 ** -24), (torch.float64, 2.0 ** -53)):
+        xd, rd, y = x.to(dt).cuda(), r.to(dt).cuda(), y0.to(dt).cuda()
+        ops.mm8_one(n_in, n_out, xd, big.cuda()[:, :n_out], y, rd)
+        xr, wd = x.double() * r.double(), big[:, :n_out].double()
+        want, mag = y0.double() + xr @ wd, y0.double().abs() + xr.abs() @ wd
+        # at most 8 products per lane, 3 + 2 additions in the trees, the slices, the product x * r and y
+        steps = 8 + 5 + (n_in + 127) // 128 + 2
+        assert ((y.cpu().double() - want).abs() <= steps * eps * mag).all()
+
+
 def test_mm8_three_matches_three_mm8_one(ops):
     n_in, n_out = 512, 520
     g = torch.Generator().manual_seed(11)
@@ -391,6 +410,25 @@ def test_wkv_forward_f64_reference_convention(ops):
     ops.wkv_forward(1, T, C, d(w), d(u), d(k[0].contiguous()), d(v[0].contiguous()), y, aa_d, bb_d, pp_d)
     assert torch.allclose(y.cpu(), yr, rtol=1e-11, atol=1e-12)
     assert torch.allclose(bb_d.cpu(), br, rtol=1e-10)
+
+
+# the serial kernel and both scan forms, at the edges of their chunks (8 steps) and blocks (64 and 256 steps)
+@pytest.mark.parametrize("T", [1, 11, 12, 63, 64, 65, 255, 256, 257, 600])
+@pytest.mark.parametrize("B,C", [(1, 32), (3, 33)])
+def test_wkv_forward_f64_any_length(ops, B, T, C):
+    _say(f"wkv_forward f64 B={B} T={T} C={C}")
+    w, u, k, v = (t.double() for t in _wkv_case(B, T, C, seed=T + C))
+    g = torch.Generator().manual_seed(T)
+    aa, bb = torch.randn(B, C, generator=g).double(), torch.rand(B, C, generator=g).double() + 0.5
+    aa[0, :3], bb[0, :3] = 0.0, 0.0                     # three empty channels among the others
+    pp = torch.full((B, C), -1e30).double()
+    y, ad, bd, pd = torch.empty(B, T, C, dtype=torch.float64, device="cuda"), aa.cuda(), bb.cuda(), pp.cuda()
+    ops.wkv_forward(B, T, C, w.cuda(), u.cuda(), k.cuda(), v.cuda(), y, ad, bd, pd)
+    for b in range(B):
+        yr, ar, br, _ = O.wkv_naive(w, u, k[b], v[b], aa[b], bb[b], pp[b])
+        assert torch.allclose(y[b].cpu(), yr, rtol=1e-11, atol=1e-12)
+        assert torch.allclose(ad[b].cpu(), ar, rtol=1e-10, atol=1e-12) and torch.allclose(bd[b].cpu(), br, rtol=1e-10)
+    assert torch.equal(pd.cpu(), pp)
 
 
 def test_argmax_first_maximum(ops):
