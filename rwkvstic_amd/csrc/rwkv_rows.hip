@@ -511,46 +511,86 @@ __device__ __forceinline__ void dma16(const v4i *g, unsigned lds_byte_offset) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "s"(lds_byte_offset) : "memory");
 }
 
-// Accumulators of one wavefront (GM M-tiles x GN N-tiles from (mt0, nt0)) to totals or, when the
-// contraction is not split, straight through the product's tail.
-template <int GM, int GN>
-__device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat,
-                                              int bz, int lane) {
-    // lane 16g + n, register i  <->  digit i of token 4*mt + g, column 16*nt + n
+// Accumulators of one wavefront (GM M-tiles x GN N-tiles from (mt0, nt0)) to totals or, when the contraction is not
+// split, straight through the product's tail.  Lane 16g + n, register i <-> digit i of token 4*mt + g, column 16*nt + n.
+//
+// Nothing overlaps this part of a workgroup but the other workgroup of its compute unit, so it is kept short: the
+// digit sums are joined in float64 (exact while 64 KB products of 2^30 x 2^7 stay below 2^53; a third of the
+// instructions of the 64-bit integer form), the tail is chosen once and not per element, and a residual tail requests
+// the next M-tile's old values before it stores this one's (a store and the load after it may not be exchanged by the
+// compiler: element by element each of them waited for a round trip).  1024 tokens at width 2560, before and after: k, v, r
+// 75.5 and 71.8 us, ffn key 93.1 and 89.4, att output and ffn receptance 35.1 and 30.2 (median), ffn value 94.8 and 87.7.
+template <int TAIL, int GM, int GN>
+__device__ __forceinline__ void gemm_tail(const GemmArgs &a, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat, int lane) {
     const int g = lane >> 4, n = lane & 15;
     const double *Sv = mat == 0 ? a.S[0] : mat == 1 ? a.S[1] : a.S[2];
     const double *qsv = mat == 0 ? a.qs[0] : mat == 1 ? a.qs[1] : a.qs[2];
     const double *zpv = mat == 0 ? a.zp[0] : mat == 1 ? a.zp[1] : a.zp[2];
     double *outv = mat == 0 ? a.out[0] : mat == 1 ? a.out[1] : a.out[2];
+    constexpr bool kAdd = TAIL == ROW_ADD || TAIL == ROW_GATE_ADD;
+    const bool exact53 = a.KB <= 512;
+    double old[2][GN];
+    float gate[2][GN];
+    auto at = [&](int i, int j) { return (size_t)min(4 * (mt0 + i) + g, a.R - 1) * a.N + min(16 * (nt0 + j) + n, a.N - 1); };   // (clamped: loads stay in bounds)
+    auto fetch = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < GN; ++j) {
+            if (kAdd) old[i & 1][j] = outv[at(i, j)];
+            if (TAIL == ROW_GATE_ADD) gate[i & 1][j] = a.gate[at(i, j)];
+        }
+    };
+    fetch(0);
+#pragma unroll
+    for (int i = 0; i < GM; ++i) {
+        if (i + 1 < GM) fetch(i + 1);
+        const int t = 4 * (mt0 + i) + g;
+        const bool live = t < a.R;
+        const int tc = live ? t : a.R - 1;
+        const double S = Sv[tc], add = 128.0 * (S * qsv[tc]) + zpv[tc];
+#pragma unroll
+        for (int j = 0; j < GN; ++j) {
+            const v4i d = acc[i][j];
+            double tot;
+            if (exact53) tot = fma(fma(fma((double)d.x, 256.0, (double)d.y), 256.0, (double)d.z), 256.0, (double)d.w);
+            else tot = (double)(((((long long)d.x * 256 + d.y) * 256 + d.z) * 256) + d.w);
+            const int col = 16 * (nt0 + j) + n;
+            const double y = S * tot + add;
+            const size_t o = (size_t)t * a.N + col;
+            if (live && col < a.N) {
+                if (TAIL == ROW_STORE) outv[o] = y;
+                else if (TAIL == ROW_STORE_F32) reinterpret_cast<float *>(outv)[o] = (float)y;
+                else if (TAIL == ROW_RELU2) {                                                       // block.py:97, kept as float32 (see RowTail)
+                    const double r = y > 0.0 ? y : 0.0;
+                    reinterpret_cast<float *>(outv)[o] = (float)(r * r);
+                }
+                else if (TAIL == ROW_ADD) outv[o] = old[i & 1][j] + y;                              // block.py:80
+                else outv[o] = old[i & 1][j] + y * (double)sigmoid_f32(gate[i & 1][j]);             // block.py:95-100; the gate in float32 as in the single-token kernel
+            }
+        }
+    }
+}
+
+template <int GM, int GN>
+__device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat,
+                                              int bz, int lane) {
+    switch (a.tail) {
+        case ROW_STORE: return gemm_tail<ROW_STORE, GM, GN>(a, acc, mt0, nt0, mat, lane);
+        case ROW_STORE_F32: return gemm_tail<ROW_STORE_F32, GM, GN>(a, acc, mt0, nt0, mat, lane);
+        case ROW_RELU2: return gemm_tail<ROW_RELU2, GM, GN>(a, acc, mt0, nt0, mat, lane);
+        case ROW_ADD: return gemm_tail<ROW_ADD, GM, GN>(a, acc, mt0, nt0, mat, lane);
+        case ROW_GATE_ADD: return gemm_tail<ROW_GATE_ADD, GM, GN>(a, acc, mt0, nt0, mat, lane);
+        default: break;
+    }
+    const int g = lane >> 4, n = lane & 15;
     long long *totv = a.tot + (size_t)(mat * a.split + bz) * a.slice;      // this part's slice
 #pragma unroll
     for (int i = 0; i < GM; ++i) {
         if (mt0 + i >= a.MT) continue;
-        const int t = 4 * (mt0 + i) + g;
-        double S = 0.0, add = 0.0;
-        if (a.tail >= 0 && t < a.R) { S = Sv[t]; add = 128.0 * (S * qsv[t]) + zpv[t]; }
 #pragma unroll
         for (int j = 0; j < GN; ++j) {
             if (nt0 + j >= a.NT) continue;
             const v4i d = acc[i][j];
-            const long long tot = ((((long long)d.x * 256 + d.y) * 256 + d.z) * 256) + d.w;
-            const int col = 16 * (nt0 + j) + n;
-            if (a.tail >= 0) {
-                if (t < a.R && col < a.N) {
-                    const double y = S * (double)tot + add;
-                    double *o = outv + (size_t)t * a.N + col;
-                    if (a.tail == ROW_STORE) *o = y;
-                    else if (a.tail == ROW_STORE_F32) reinterpret_cast<float *>(outv)[(size_t)t * a.N + col] = (float)y;
-                    else if (a.tail == ROW_RELU2) {                                                                 // block.py:97, kept as float32 (see RowTail)
-                        const double r = y > 0.0 ? y : 0.0;
-                        reinterpret_cast<float *>(outv)[(size_t)t * a.N + col] = (float)(r * r);
-                    }
-                    else if (a.tail == ROW_ADD) *o += y;                                                            // block.py:80
-                    else *o += y * (double)sigmoid_f32(a.gate[(size_t)t * a.N + col]);       // block.py:95-100; the gate in float32 as in the single-token kernel
-                }
-                continue;
-            }
-            totv[(size_t)t * a.ldd + col] = tot;
+            totv[(size_t)(4 * (mt0 + i) + g) * a.ldd + 16 * (nt0 + j) + n] = ((((long long)d.x * 256 + d.y) * 256 + d.z) * 256) + d.w;
         }
     }
 }
