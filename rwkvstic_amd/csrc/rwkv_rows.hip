@@ -30,15 +30,36 @@ constexpr int kRW = kRT / 64;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
+// Sums and maxima over a wavefront without the LDS crossbar: four exchanges inside rows of 16 lanes (DPP: neighbour,
+// pair, half row, row), then the four rows' results through scalar registers.  Every lane ends with the same value.  (A
+// butterfly of 64-bit shuffles is twelve dependent trips through LDS; the row kernels are chains of such reductions.)
+template <int CTRL>
+__device__ __forceinline__ double dpp64(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp32(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false)); }
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+__device__ __forceinline__ double lane64(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l), __builtin_amdgcn_readlane(__double2loint(v), l));
+}
 __device__ __forceinline__ double wsum(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    v += dpp64<kDppXor1>(v);
+    v += dpp64<kDppXor2>(v);
+    v += dpp64<kDppHalfMirror>(v);
+    v += dpp64<kDppMirror>(v);
+    return (lane64(v, 0) + lane64(v, 16)) + (lane64(v, 32) + lane64(v, 48));
 }
 __device__ __forceinline__ float wmaxf(float v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
+    v = fmaxf(v, dpp32<kDppXor1>(v));
+    v = fmaxf(v, dpp32<kDppXor2>(v));
+    v = fmaxf(v, dpp32<kDppHalfMirror>(v));
+    v = fmaxf(v, dpp32<kDppMirror>(v));
+    const int i = __float_as_int(v);
+    return fmaxf(fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 0)), __int_as_float(__builtin_amdgcn_readlane(i, 16))),
+                 fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 32)), __int_as_float(__builtin_amdgcn_readlane(i, 48))));
 }
 
 // Sum of N values per thread over the workgroup (fixed order), broadcast.
