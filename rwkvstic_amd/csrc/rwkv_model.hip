@@ -523,7 +523,7 @@ constexpr int64_t kRowsChunk = 1024;   // rows per pass: bounds the workspace of
 constexpr int64_t kRowsMin = 4;        // shorter prompts go token by token
 
 struct RowsWs {
-    double *x, *kvr, *att, *h, *prev0, *wkv_scr;
+    double *x, *kvr, *att, *h, *prev0;
     RowsOperand q[3];       // quantised left operands: q[0] up to n_ffn wide, q[1], q[2] n_embd wide
     long long *tot;
 };
@@ -544,7 +544,6 @@ size_t rows_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_
     n += round_up((size_t)R * C * 8, 256) * 5;          // x, kvr[3], att
     n += round_up((size_t)R * F * 8, 256);              // h
     n += round_up((size_t)C * 8, 256);                  // prev0
-    n += round_up(rows_wkv_scratch_bytes(R, C), 256);
     n += round_up((size_t)R * 8, 256) * 9;              // S, qs, zp of three operands
     n += round_up(rows_dig_bytes(R, F), 256) + 2 * round_up(rows_dig_bytes(R, C), 256);
     n += round_up(rows_tot_ws_bytes(R, C, n_wide, n_head), 256);
@@ -560,7 +559,6 @@ RowsWs rows_carve(void *ws, int64_t R, int64_t C, int64_t F, int64_t n_wide, int
     w.att = (double *)take((size_t)R * C * 8);
     w.h = (double *)take((size_t)R * F * 8);
     w.prev0 = (double *)take((size_t)C * 8);
-    w.wkv_scr = (double *)take(rows_wkv_scratch_bytes(R, C));
     for (int i = 0; i < 3; ++i) {
         w.q[i].S = (double *)take((size_t)R * 8);
         w.q[i].qs = (double *)take((size_t)R * 8);
@@ -615,7 +613,7 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
         for (int i = 0; i < 3; ++i) { pk[i].a = w.q[i]; pk[i].w16 = kvr[i]->packed16; pk[i].out = reinterpret_cast<double *>(kvr32 + i * RC); }
         RWKV_TRY(rows_products(st, 3, pk, w.tot, R, C, C, ROW_STORE_F32, nullptr, defer ? dk : nullptr));
         RWKV_TRY(rows_wkv(st, R, C, sequence, kvr32, kvr32 + RC, kvr32 + 2 * RC, L.time_decay, L.time_first,
-                          sl + 2 * (size_t)C, state_stride, reinterpret_cast<float *>(w.att), w.wkv_scr, defer ? dk : nullptr));
+                          sl + 2 * (size_t)C, state_stride, reinterpret_cast<float *>(w.att), defer ? dk : nullptr));
         RWKV_TRY(rows_quant(st, R, C, w.att, true, L.att_o.range, L.att_o.offset, w.q[0], (double *)w.tot));    // att and h: float32 arrays
         const RowsProduct po = {w.q[0], L.att_o.packed16, w.x};
         RWKV_TRY(rows_products(st, 1, &po, w.tot, R, C, C, ROW_ADD, nullptr, defer ? &dx : nullptr));

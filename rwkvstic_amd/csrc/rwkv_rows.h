@@ -37,7 +37,6 @@ constexpr int64_t kRowsDeferMax = 128;
 constexpr int kRowsDeferSlices = 4;     // a contraction split further than this is finished by a launch of its own
 size_t rows_dig_bytes(int64_t R, int64_t K);
 size_t rows_tot_bytes(int64_t R, int64_t N);        // integer totals of ONE product (times the products in a launch)
-size_t rows_wkv_scratch_bytes(int64_t R, int64_t C);
 size_t rows_quant_scratch_bytes(int64_t R, int64_t K);   // what rows_quant writes into its scratch area (0: unused)
 // The plan rows_products follows for n products [R, K] x [K, N]: out = {kernel kind, grid x, grid y, splits}.
 void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int out[4]);
@@ -67,7 +66,6 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
 // kvr (null, or 3 entries, batch rows only): k, v, r still pending as split products (ROW_STORE_F32) where tot is set.
 int rows_wkv(hipStream_t st, int64_t R, int C, bool sequence, const float *k, const float *v, const float *r,
              const double *w, const double *u, double *state, int64_t state_stride, float *out,
-             double *scratch /* rows_wkv_scratch_bytes(R, C), or null: serial over the rows */,
              const RowsDeferred *kvr = nullptr);
 
 // Stand-alone product of 1..8 float32 vectors with one matrix in M16 blocks, four-vector dequantisation (row and

@@ -986,117 +986,97 @@ __global__ void __launch_bounds__(64) wkv_rows_kernel(const WkvRowsArgs a) {
 }
 
 
-// Long sequences: the recurrence is linear in (aa, bb), so T steps split into chunks of kWkvChunk:
-// (1) every chunk's own contribution from an empty state, in parallel; (2) a short serial pass that
-// turns them into each chunk's incoming state (a chunk decays its input by e^{n w}); (3) every chunk
-// replays its steps from that state, in parallel.  Same sums as the serial order up to float64 rounding.
-constexpr int kWkvChunk = 32;
+// Longer sequences: the recurrence is linear in (aa, bb), so a workgroup sums up a block of NC chunks of kWkvStep steps
+// side by side (32 channels x NC chunk positions), a scan over the chunks in LDS gives every thread the state its chunk
+// starts from, and each writes the outputs of its own steps: one launch, k and v read once (a chunk stays in
+// registers between the two passes).  Sums float32 and exponents float64 as in the serial form.
+//
+// Bound: the chain of one block (loads, kWkvStep + log2 NC exponentials, kWkvStep steps), with many steps its vector
+// instructions; not memory.  2560 channels and 64 / 128 / 256 / 1024 steps: 5.4 / 6.7 / 8.1 / 24.2 us; as three launches
+// (contributions of 32-step chunks, serial prefix, replay) 19.0 / 19.3 / 20.5 / 32.6 us.  16 channels per workgroup for
+// the long forms: twice the compute units at work (32 channels: 34.9 us at 1024 steps).
+constexpr int kWkvScanMin = 6;      // from kWkvScanMin steps on the scan is faster than the serial form (2560 channels: 8 steps 9.0 us serially, 6.0 as a scan; 1.0 us a step)
 
-// The kernels read their inputs kWkvGroup steps ahead of the serial recurrence (registers, two groups): a
-// thread that fetched each step's k and v when it needed them would wait out a memory round trip per step.
-constexpr int kWkvGroup = 8;
-static_assert(kWkvChunk % kWkvGroup == 0, "whole groups");
-
-__global__ void __launch_bounds__(64) wkv_chunk_local_kernel(const WkvRowsArgs a, double *scr) {
-    const int c = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y;
-    if (c >= a.C) return;
-    const int C = a.C;
-    const double w = a.w[c], u = a.u[c];
-    const int t0 = j * kWkvChunk, t1 = min(t0 + kWkvChunk, a.R);
-    float aa = 0.f, bb = 0.f;
-    double pp = -1e30;
-    float kc[kWkvGroup], vc[kWkvGroup], kn[kWkvGroup], vn[kWkvGroup];
+// One block from step tb; FULL: it lies inside the sequence.  (as, bs, p): the state before the block, on return after it.
+template <int NC, int CH, int kWkvStep, bool FULL>
+__device__ __forceinline__ void wkv_scan_block(const WkvRowsArgs &a, int tb, int c, int ch, int j, double wc, double uw,
+                                               float (*sa)[NC][CH], float (*sb)[NC][CH], double (*sp)[NC][CH],
+                                               float &ca, float &cb, double &cp) {
+    const int C = a.C, T = a.R;
+    const int t0 = FULL ? tb + j * kWkvStep : min(tb + j * kWkvStep, T), n = FULL ? kWkvStep : min(kWkvStep, T - t0);
+    auto row = [&](int i) { return (size_t)(FULL ? t0 + i : min(t0 + i, T - 1)) * C + c; };     // past the end: the last row again, unused
+    float kc[kWkvStep], vc[kWkvStep], rc[kWkvStep];
 #pragma unroll
-    for (int i = 0; i < kWkvGroup; ++i) {
-        const size_t o = (size_t)min(t0 + i, t1 - 1) * C + c;
-        kc[i] = a.k[o]; vc[i] = a.v[o];
+    for (int i = 0; i < kWkvStep; ++i) { kc[i] = a.k[row(i)]; vc[i] = a.v[row(i)]; }
+#pragma unroll
+    for (int i = 0; i < kWkvStep; ++i) rc[i] = a.r[row(i)];
+    // the chunk from an empty state, a direct sum: step i contributes e^{k_i + (n - i) w} by the chunk's end
+    double p = -1e30;
+    float as = 0.f, bs = 0.f;
+#pragma unroll
+    for (int i = 0; i < kWkvStep; ++i) p = fmax(p, FULL || i < n ? fma((double)(n - i), wc, (double)kc[i]) : -1e30);
+#pragma unroll
+    for (int i = 0; i < kWkvStep; ++i) {
+        const float f = FULL || i < n ? expf((float)(fma((double)(n - i), wc, (double)kc[i]) - p)) : 0.f;
+        as = fmaf(f, vc[i], as);
+        bs += f;
     }
-    for (int g = t0; g < t1; g += kWkvGroup) {
+    if (j == 0) {                                        // the state before the block, decayed over the first chunk
+        const double e = cp + (double)n * wc, pn = fmax(e, p);
+        const float f0 = expf((float)(e - pn)), f1 = expf((float)(p - pn));
+        as = f0 * ca + f1 * as; bs = f0 * cb + f1 * bs; p = pn;
+    }
+    sa[0][j][ch] = as; sb[0][j][ch] = bs; sp[0][j][ch] = p;
+    __syncthreads();
+    int buf = 0;
 #pragma unroll
-        for (int i = 0; i < kWkvGroup; ++i) {
-            const size_t o = (size_t)min(g + kWkvGroup + i, t1 - 1) * C + c;      // past the end: the last row again (unused)
-            kn[i] = a.k[o]; vn[i] = a.v[o];
+    for (int d = 1; d < NC; d <<= 1, buf ^= 1) {         // inclusive scan: add what ends d chunks earlier, decayed to here
+        if (j >= d) {
+            const int len = FULL ? d * kWkvStep : t0 + n - min(tb + (j - d + 1) * kWkvStep, T);
+            const double e = sp[buf][j - d][ch] + (double)len * wc, pn = fmax(e, p);
+            const float f0 = expf((float)(e - pn)), f1 = expf((float)(p - pn));
+            as = f0 * sa[buf][j - d][ch] + f1 * as;
+            bs = f0 * sb[buf][j - d][ch] + f1 * bs;
+            p = pn;
         }
-#pragma unroll
-        for (int i = 0; i < kWkvGroup; ++i)
-            if (g + i < t1) (void)wkv_step_f32(w, u, kc[i], vc[i], aa, bb, pp);
-#pragma unroll
-        for (int i = 0; i < kWkvGroup; ++i) { kc[i] = kn[i]; vc[i] = vn[i]; }
+        sa[buf ^ 1][j][ch] = as; sb[buf ^ 1][j][ch] = bs; sp[buf ^ 1][j][ch] = p;
+        __syncthreads();
     }
-    double *o = scr + (size_t)j * 3 * C;
-    o[c] = (double)aa; o[C + c] = (double)bb; o[2 * C + c] = pp;
+    if (j > 0) { as = sa[buf][j - 1][ch]; bs = sb[buf][j - 1][ch]; p = sp[buf][j - 1][ch]; }
+    else { as = ca; bs = cb; p = cp; }
+    ca = sa[buf][NC - 1][ch]; cb = sb[buf][NC - 1][ch]; cp = sp[buf][NC - 1][ch];
+#pragma unroll
+    for (int i = 0; i < kWkvStep; ++i) {
+        if (FULL || i < n) {                             // wkv_step_f32; the gate's division joins the step's
+            const double dk = p - (double)kc[i];
+            const float d2 = (float)dk, d = (float)(dk - uw);
+            const float e = expf(-fabsf(d)), f = expf(-fabsf(d2));
+            const float e1 = d >= 0.f ? 1.f : e, e2 = d >= 0.f ? e : 1.f;
+            a.out[(size_t)(t0 + i) * C + c] = (e1 * as + e2 * vc[i]) / ((e1 * bs + e2) * (1.f + expf(-rc[i])));
+            const float f1 = d2 >= 0.f ? 1.f : f, f2 = d2 >= 0.f ? f : 1.f;
+            as = f1 * as + f2 * vc[i];
+            bs = f1 * bs + f2;
+            p = fmax(p, (double)kc[i]) + wc;
+        }
+    }
 }
 
-__global__ void __launch_bounds__(64) wkv_chunk_prefix_kernel(const WkvRowsArgs a, double *scr, int n_chunks) {
-    const int c = blockIdx.x * 64 + threadIdx.x;
-    if (c >= a.C) return;
-    const int C = a.C;
-    const double w = a.w[c];
-    double aa = a.state[c], bb = a.state[C + c], pp = a.state[2 * C + c];
-    double la[kWkvGroup], lb[kWkvGroup], lp[kWkvGroup], na[kWkvGroup], nb[kWkvGroup], np[kWkvGroup];
-#pragma unroll
-    for (int i = 0; i < kWkvGroup; ++i) {
-        const double *o = scr + (size_t)min(i, n_chunks - 1) * 3 * C;
-        la[i] = o[c]; lb[i] = o[C + c]; lp[i] = o[2 * C + c];
-    }
-    for (int g = 0; g < n_chunks; g += kWkvGroup) {
-#pragma unroll
-        for (int i = 0; i < kWkvGroup; ++i) {
-            const double *o = scr + (size_t)min(g + kWkvGroup + i, n_chunks - 1) * 3 * C;
-            na[i] = o[c]; nb[i] = o[C + c]; np[i] = o[2 * C + c];
-        }
-#pragma unroll
-        for (int i = 0; i < kWkvGroup; ++i) {
-            const int j = g + i;
-            if (j < n_chunks) {
-                double *o = scr + (size_t)j * 3 * C;
-                o[c] = aa; o[C + c] = bb; o[2 * C + c] = pp;              // incoming state of chunk j
-                const int n = min(kWkvChunk, a.R - j * kWkvChunk);
-                const double s = pp + (double)n * w;
-                const double p = fmax(s, lp[i]);
-                const double f1 = (double)expf((float)(s - p)), f2 = (double)expf((float)(lp[i] - p));   // (one of them is e^0)
-                aa = f1 * aa + f2 * la[i];
-                bb = f1 * bb + f2 * lb[i];
-                pp = p;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kWkvGroup; ++i) { la[i] = na[i]; lb[i] = nb[i]; lp[i] = np[i]; }
-    }
-    a.state[c] = aa; a.state[C + c] = bb; a.state[2 * C + c] = pp;
-}
-
-__global__ void __launch_bounds__(64) wkv_chunk_replay_kernel(const WkvRowsArgs a, const double *scr) {
-    const int c = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y;
-    if (c >= a.C) return;
-    const int C = a.C;
-    const double w = a.w[c], u = a.u[c];
-    const int t0 = j * kWkvChunk, t1 = min(t0 + kWkvChunk, a.R);
-    const double *in = scr + (size_t)j * 3 * C;
-    float aa = (float)in[c], bb = (float)in[C + c];
-    double pp = in[2 * C + c];
-    float kc[kWkvGroup], vc[kWkvGroup], rc[kWkvGroup], kn[kWkvGroup], vn[kWkvGroup], rn[kWkvGroup];
-#pragma unroll
-    for (int i = 0; i < kWkvGroup; ++i) {
-        const size_t o = (size_t)min(t0 + i, t1 - 1) * C + c;
-        kc[i] = a.k[o]; vc[i] = a.v[o]; rc[i] = a.r[o];
-    }
-    for (int g = t0; g < t1; g += kWkvGroup) {
-#pragma unroll
-        for (int i = 0; i < kWkvGroup; ++i) {
-            const size_t o = (size_t)min(g + kWkvGroup + i, t1 - 1) * C + c;
-            kn[i] = a.k[o]; vn[i] = a.v[o]; rn[i] = a.r[o];
-        }
-#pragma unroll
-        for (int i = 0; i < kWkvGroup; ++i) {
-            if (g + i < t1) {
-                const float y = wkv_step_f32(w, u, kc[i], vc[i], aa, bb, pp);
-                a.out[(size_t)(g + i) * C + c] = y * sigmoid_f32(rc[i]);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kWkvGroup; ++i) { kc[i] = kn[i]; vc[i] = vn[i]; rc[i] = rn[i]; }
-    }
+template <int NC, int CH, int kWkvStep>
+__global__ void __launch_bounds__(NC * CH) wkv_scan_rows_kernel(const WkvRowsArgs a) {
+    __shared__ float sa[2][NC][CH], sb[2][NC][CH];
+    __shared__ double sp[2][NC][CH];
+    // the last round of the scan writes buffer 1: the next block's summaries may enter buffer 0 while it is still read
+    static_assert(NC == 8 || NC == 32, "an odd number of scan rounds");
+    const int ch = threadIdx.x % CH, j = threadIdx.x / CH;
+    const int C = a.C, c = blockIdx.x * CH + ch;               // (C is a multiple of 64)
+    const double wc = a.w[c], uw = a.u[c] + wc;
+    float ca = (float)a.state[c], cb = (float)a.state[C + c];
+    double cp = a.state[2 * C + c];
+    int tb = 0;
+    for (; tb + NC * kWkvStep <= a.R; tb += NC * kWkvStep)
+        wkv_scan_block<NC, CH, kWkvStep, true>(a, tb, c, ch, j, wc, uw, sa, sb, sp, ca, cb, cp);
+    if (tb < a.R) wkv_scan_block<NC, CH, kWkvStep, false>(a, tb, c, ch, j, wc, uw, sa, sb, sp, ca, cb, cp);
+    if (j == 0) { a.state[c] = (double)ca; a.state[C + c] = (double)cb; a.state[2 * C + c] = cp; }
 }
 
 // ---------------------------------------------------------------------------
@@ -1285,7 +1265,6 @@ __global__ void __launch_bounds__(1024) mv16_kernel(const Mv16Args a) {
 // host side
 // ---------------------------------------------------------------------------
 size_t rows_dig_bytes(int64_t R, int64_t K) { return (size_t)(ceil_div(R, 4) * (K / 64) * 1024); }
-size_t rows_wkv_scratch_bytes(int64_t R, int64_t C) { return (size_t)(ceil_div(R, kWkvChunk) * 3 * C * 8); }
 constexpr int kVecFillWgs = 128;        // products of at most 8 rows: the contraction is split until there are this many workgroups (batch step of 8 / 4 sequences, 3B shape: 3.06 / 2.64 ms at 128, 3.19 / 2.81 at 256, 3.30 / 2.94 at 512)
 constexpr int kMaxSplit = 8;
 constexpr int kGemmWideNum = 10, kGemmWideDen = 9;     // the 64 x 160 variant is taken when its cost is below 9/10 of the 64 x 128 variant's
@@ -1512,8 +1491,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
 }
 
 int rows_wkv(hipStream_t st, int64_t R, int C, bool sequence, const float *k, const float *v, const float *r,
-             const double *w, const double *u, double *state, int64_t state_stride, float *out, double *scratch,
-             const RowsDeferred *kvr) {
+             const double *w, const double *u, double *state, int64_t state_stride, float *out, const RowsDeferred *kvr) {
     WkvRowsArgs a;
     a.C = C; a.R = (int)R; a.sequence = sequence ? 1 : 0; a.k = k; a.v = v; a.r = r; a.w = w; a.u = u;
     a.state = state; a.state_stride = state_stride; a.out = out;
@@ -1523,13 +1501,14 @@ int rows_wkv(hipStream_t st, int64_t R, int C, bool sequence, const float *k, co
         if (a.pend[i].tot && (sequence || a.pend[i].op != ROW_STORE_F32))
             return set_error(RWKV_ERR_ARG, "rows_wkv: a pending product needs batch rows and the float32 store tail");
     }
-    if (sequence && scratch && R >= 2 * kWkvChunk) {
-        const int n_chunks = (int)ceil_div(R, kWkvChunk);
-        const dim3 grid((unsigned)ceil_div(C, 64), (unsigned)n_chunks);
-        hipLaunchKernelGGL(wkv_chunk_local_kernel, grid, dim3(64), 0, st, a, scratch);
-        hipLaunchKernelGGL(wkv_chunk_prefix_kernel, dim3(grid.x), dim3(64), 0, st, a, scratch, n_chunks);
-        hipLaunchKernelGGL(wkv_chunk_replay_kernel, grid, dim3(64), 0, st, a, (const double *)scratch);
-        RWKV_CHECK_LAUNCH("wkv_chunk kernels");
+    if (sequence && R >= kWkvScanMin) {
+        // the smallest block that covers the sequence leaves the fewest threads idle
+        const dim3 g32((unsigned)(C / 32)), g16((unsigned)(C / 16));
+        if (R <= 8 * 8) hipLaunchKernelGGL((wkv_scan_rows_kernel<8, 32, 8>), g32, dim3(8 * 32), 0, st, a);
+        else if (R <= 8 * 16) hipLaunchKernelGGL((wkv_scan_rows_kernel<8, 32, 16>), g32, dim3(8 * 32), 0, st, a);
+        else if (R <= 32 * 8) hipLaunchKernelGGL((wkv_scan_rows_kernel<32, 16, 8>), g16, dim3(32 * 16), 0, st, a);
+        else hipLaunchKernelGGL((wkv_scan_rows_kernel<32, 16, 16>), g16, dim3(32 * 16), 0, st, a);
+        RWKV_CHECK_LAUNCH("wkv_scan_rows_kernel");
         return RWKV_OK;
     }
     hipLaunchKernelGGL(wkv_rows_kernel, dim3((unsigned)ceil_div(C, 64), sequence ? 1u : (unsigned)R), dim3(64), 0, st, a);
