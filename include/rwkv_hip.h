@@ -287,7 +287,9 @@ int rwkv_model_create(const rwkv_model_desc *desc, rwkv_model **out);
 void rwkv_model_destroy(rwkv_model *m);
 
 /* 1 if single-token steps of this handle run as one persistent launch (all
- * matrices have packed16 and the shape is supported), else 0. */
+ * matrices have packed16 and the shape is supported) and its generation loop
+ * can sample on the device, else 0.  At n_embd 512, 768 and 1536 the token
+ * steps are persistent launches too, but sampling stays with the caller. */
 int rwkv_model_has_fused_step(const rwkv_model *m);
 
 /* Diagnostics: when device_buffer is non-NULL, every workgroup g of every

@@ -11,9 +11,9 @@ twice the space and spills; a spilled or copied in-flight register is silent cor
 whole back-wave program is one asm statement with its own register map; it talks to the compiled
 front waves only through LDS and workgroup barriers.
 
-Stream of one back wave (wave wb of 8) of workgroup g, in units of 1 KiB blocks ("positions"):
+Stream of one back wave (wave wb of BW, 8 or, at the two smallest widths, 4) of workgroup g, in units of 1 KiB blocks ("positions"):
   per layer 13 jobs x KW blocks (job = one 16-column tile of a C-row matrix, or a quarter of the
-  F-row ffn value tile; wave wb owns blocks wb, wb+8, ... of the job), padded to PP positions, a
+  F-row ffn value tile; wave wb owns blocks wb, wb+BW, ... of the job; KW = C / (64 BW)), padded to PP positions, a
   multiple of the ring size R, then the head tiles g, g+G, ... .  Position p lives in ring slot
   p % R.  At every position: wait until at most R-1 loads are outstanding (then the slot's block has
   landed), multiply, reload the slot with position p+R.  Every position issues exactly one load -
@@ -81,16 +81,17 @@ class Emit:
 S_TMP = 62        # scratch pair for a block's address where block offsets are added on the scalar side
 
 
-def gen(KW, R, NV, NSH, HELP=False):
+def gen(KW, R, NV, NSH, HELP=False, BW=8):
     """HELP: the four ffn key tiles of a group are not this workgroup's (helper workgroups on the otherwise idle
     compute units own that matrix): 9 jobs per layer instead of 13, and the ffn receptance tile takes its digits
     from the first set of planes."""
-    C = 512 * KW
+    NB = BW * KW                     # 64-channel blocks of a row
+    C = 64 * NB
     F = 4 * C
     PS, PSF = C + 64, F + 64
-    NT = 2 if KW > 8 else 1          # groups of 16 channels (and their tiles) per workgroup
+    NT = 2 if NB > 64 else 1          # groups of 16 channels (and their tiles) per workgroup
     SPG = 5                          # parked-tile slots per group
-    NWG = 32 * KW // NT              # workgroups
+    NWG = 4 * NB // NT              # workgroups
     SADDR = KW > 8                   # no room for one offset register per block of a job: the block offset joins the base address in a scalar pair
     # Compact register map where block offsets travel on the scalar side: one offset register, two A-operand buffers
     # and no register for the flag address leave room for a ring of 26 blocks in 128 registers.
@@ -107,11 +108,12 @@ def gen(KW, R, NV, NSH, HELP=False):
     RB = NV - 4 * R
     assert RB >= V_A + 4 * NA, "ring does not fit"
     assert R <= NREAL and R - 1 <= 63
-    TB = 8 * KW * 1024
+    TB = NB * 1024
+    PARK = BW * 256                  # bytes of a parked tile: 16 columns x 16 bytes per back wave
     DIG = max(12 * PS, 4 * PSF)
     RED = DIG                                 # byte offset of the parked tiles from the start of LDS
     RED_SLOTS = max(SPG * NT, 2 * NSH)
-    FLAG = RED + RED_SLOTS * 2048 + 32 * 8 + NT * 32 * 8 + 2 * 4   # FLAG_ABORT word
+    FLAG = RED + RED_SLOTS * PARK + 32 * 8 + NT * 32 * 8 + 2 * 4   # FLAG_ABORT word
 
     # Jobs of a layer in stream order.  ptr: index of the job's base address in the workgroup's table row (that of
     # its first group; the same tile of the next group lies `stride` bytes further), aset/aoff: digit planes the
@@ -143,7 +145,7 @@ def gen(KW, R, NV, NSH, HELP=False):
         if wh:
             e(f"global_load_dwordx4 {dst}, v{V_OFF}, %[wh]")
         elif SADDR:
-            e(f"s_add_u32 s{S_TMP}, s{sbase}, {extra + 8192 * b}")
+            e(f"s_add_u32 s{S_TMP}, s{sbase}, {extra + 1024 * BW * b}")
             e(f"s_addc_u32 s{S_TMP + 1}, s{sbase + 1}, 0")
             e(f"global_load_dwordx4 {dst}, v{V_OFF}, s[{S_TMP}:{S_TMP + 1}]")
         else:
@@ -169,11 +171,11 @@ def gen(KW, R, NV, NSH, HELP=False):
     def aread(q_layer_pos=None, head_b=None):
         """Issue the A-operand read of a layer position (or of block head_b of a head tile)."""
         if head_b is not None:
-            base, off, k = V_APC, 512 * head_b, head_b % NA
+            base, off, k = V_APC, 64 * BW * head_b, head_b % NA
         else:
             q = q_layer_pos
             j, b = divmod(q, KW)
-            base, off = (V_APC if jobs[j]["aset"] == "C" else V_APF), jobs[j]["aoff"] + 512 * b
+            base, off = (V_APC if jobs[j]["aset"] == "C" else V_APF), jobs[j]["aoff"] + 64 * BW * b
             k = q % NA
         assert off < 65536
         e(f"ds_read_b128 v[{V_A + 4 * k}:{V_A + 4 * k + 3}], v{base} offset:{off}")
@@ -193,7 +195,7 @@ def gen(KW, R, NV, NSH, HELP=False):
     def park_static(dreg, slot):
         e("s_nop 7"); e("s_nop 7"); e("s_nop 7")
         e("s_mov_b64 exec, 0xffff")
-        e(f"ds_write_b128 v{V_PARK}, v[{dreg}:{dreg + 3}] offset:{slot * 2048}")
+        e(f"ds_write_b128 v{V_PARK}, v[{dreg}:{dreg + 3}] offset:{slot * PARK}")
         e("s_mov_b64 exec, -1")
         e.issued += 1
 
@@ -224,7 +226,7 @@ def gen(KW, R, NV, NSH, HELP=False):
     e(f"v_add_u32 v{V_OFF}, s{S_T}, v{V_OFF}")
     if not SADDR:
         for b in range(1, KW):
-            e(f"v_add_u32 v{V_OFF + b}, {8192 * b}, v{V_OFF}")
+            e(f"v_add_u32 v{V_OFF + b}, {1024 * BW * b}, v{V_OFF}")
     e(f"s_mov_b64 s[{S_JT}:{S_JT + 1}], %[jt]")
     e(f"s_mov_b32 s{S_L}, %[L]")
     e(f"s_mov_b32 s{S_SEQ}, 0")
@@ -443,7 +445,7 @@ def gen(KW, R, NV, NSH, HELP=False):
             if b == KW - 1:
                 e("s_nop 7"); e("s_nop 7"); e("s_nop 7")
                 e(f"s_add_u32 s{S_T}, s{S_PAR}, {tq % NSH}")
-                e(f"s_lshl_b32 s{S_T}, s{S_T}, 11")
+                e(f"s_lshl_b32 s{S_T}, s{S_T}, {PARK.bit_length() - 1}")
                 e(f"v_add_u32 v{V_A}, s{S_T}, v{V_PARK}")
                 e("s_mov_b64 exec, 0xffff")
                 e(f"ds_write_b128 v{V_A}, v[{dreg}:{dreg + 3}]")
@@ -464,10 +466,11 @@ def gen(KW, R, NV, NSH, HELP=False):
     return e.lines, dict(KW=KW, R=R, PP=PP, RB=RB, RED=RED, FLAG=FLAG, RED_SLOTS=RED_SLOTS, NS=NSH)
 
 
-# (KW, front waves, ring size): 4 front waves -> 12 waves per workgroup, 168 VGPRs each;
-# 8 front waves -> 16 waves, 128 VGPRs each.
-CONFIGS = [(2, 4, 26), (4, 4, 26), (5, 4, 33), (8, 4, 26),
-           (2, 8, 13), (4, 8, 13), (5, 8, 22), (8, 8, 13), (10, 8, int(os.environ.get("RWKV_BACK_R_WIDE", "26")))]
+# (KW, back waves, front waves, ring size): 12 waves per workgroup -> 168 VGPRs each, 16 waves -> 128.  At the narrow
+# widths the exchanges set the pace and the ring size does not matter: C = 768, 12 layers, 176 / 180 / 177 us per token
+# with rings of 13 / 20 / 39; C = 1536, 24 layers, 478 / 476 with 13 / 20.
+CONFIGS = [(2, 4, 4, 26), (3, 4, 4, 13), (2, 8, 4, 26), (3, 8, 4, 20), (4, 8, 4, 26), (8, 8, 4, 26), (5, 8, 8, 22),
+           (10, 8, 8, int(os.environ.get("RWKV_BACK_R_WIDE", "26")))]
 
 
 def main():
@@ -475,15 +478,15 @@ def main():
     w = out.append
     w("// Generated by gen_decode_back.py - do not edit.  One asm statement per kernel width: the program")
     w("// of a weight-streaming wave of the single-token kernel (see the generator for the register map).")
-    w("template <int KW, int FW> struct BackCfg;")
-    w("template <int KW, int FW> struct BackCfgH;      // with helper workgroups: no ffn key tiles")
-    for KW, FW, R, HELP in [c + (False,) for c in CONFIGS] + [(5, 8, R_HELP, True)]:
-        NV = 168 if FW == 4 else 128
+    w("template <int NB, int FW> struct BackCfg;")
+    w("template <int NB, int FW> struct BackCfgH;      // with helper workgroups: no ffn key tiles")
+    for KW, BW, FW, R, HELP in [c + (False,) for c in CONFIGS] + [(5, 8, 8, R_HELP, True)]:
+        NV = 128 if FW + BW == 16 else 168
         clob = ", ".join(f'"v{i}"' for i in range(V_APC, NV)) + ", " + ", ".join(f'"s{i}"' for i in range(S_CUR, 102 if KW > 8 else 100))
         tiles_per_body = R // math.gcd(R, KW)
         NSH = max(d for d in range(1, 5) if tiles_per_body % d == 0)     # head tiles per barrier round
-        lines, info = gen(KW, R, NV, NSH, HELP)
-        w(f"template <> struct BackCfg{'H' if HELP else ''}<{KW}, {FW}> {{")
+        lines, info = gen(KW, R, NV, NSH, HELP, BW)
+        w(f"template <> struct BackCfg{'H' if HELP else ''}<{BW * KW}, {FW}> {{")
         w(f"    static constexpr int R = {R}, RED = {info['RED']}, FLAG = {info['FLAG']}, RED_SLOTS = {info['RED_SLOTS']}, NS = {info['NS']};")
         w("    static __device__ __forceinline__ void run(const unsigned long long *jt, const uint8_t *wh, int L, int hr, int vt,")
         w("                                                int g, int wb, unsigned lds) {")

@@ -57,14 +57,25 @@ namespace rwkv {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-constexpr int kBW = 8;                 // back (streaming) waves per workgroup
+// Widths.  C = 512, 768 and 1536 are bound by the four exchanges per layer (13.4 us per layer at 768): a token of the
+// 12-layer 768 shape takes 177 us, as one-row prompts through the many-row kernels it took 630 us (146 launches).
+// NB (template parameter throughout): 64-channel blocks of a row of C channels, C = 64 NB.  Back (streaming) waves per
+// workgroup: eight, four at the two smallest widths, whose 8 and 12 blocks per tile they share evenly (12 over eight
+// waves would leave half of them idle every second block).
+constexpr int back_waves(int nb) { return nb <= 12 ? 4 : 8; }
+constexpr int kPrepThreads = 512;
+constexpr int prep_parts(int C) { return (C + kPrepThreads - 1) / kPrepThreads; }      // 512-channel parts of a layer's per-token scalars
 constexpr int kRealJobs = 13;          // tile jobs per layer: k v r | o | ffn_r, 4 x ffn_k | 4 quarters of ffn_v
 constexpr unsigned kSpinLimit = 1u << 20;        // polls before a wait gives up (DArgs::spin_limit; a self-test passes a small one)
 constexpr int kStatRows = 2;           // XR rows 0-1: sum x of a workgroup's 16 channels, and their squared deviations from the workgroup's own mean
 constexpr int kLnRows = kStatRows + 3 * 3;     // rows of the XR record table
 constexpr int kEarlyDiv = 4;           // gathers start when all but G / kEarlyDiv workgroups have published (measured flat from G/20 to G)
 constexpr int kSlotsPerGroup = 5;      // parked-tile slots a group of 16 channels needs at once (ffn receptance + 4 ffn key tiles)
-constexpr int kHeadCsPerThread = 4;    // head column sums a front thread fetches: 16 per head tile of the workgroup
+// Head column sums a front thread fetches, 16 per head tile of the workgroup: narrow models have few workgroups and so
+// many head tiles each (66 at C = 768 with 50277 tokens), and a part of LDS for the sums; the others park them in half
+// an owner record.
+constexpr int head_cs_per_thread(int nb) { return nb <= 12 ? 8 : 4; }
+constexpr int head_cs_lds_bytes(int nb) { return nb <= 12 ? 8 * 256 * 4 : 0; }
 
 // LDS flag words
 enum { FLAG_ARRIVED = 0, FLAG_SCALE = 1, FLAG_ABORT = 2, FLAG_GO = 3, FLAG_COUNT = 4 };   // FLAG_GO: see the reload gate of the generated back-wave program
@@ -89,9 +100,9 @@ __device__ __forceinline__ void gst(T *p, T v) { *(RWKV_GLOBAL T *)p = v; }
 
 // A workgroup owns NT groups of 16 channels (and their tiles): one up to C = 4096, two at C = 5120, whose 320
 // groups would not all be resident on 256 compute units.  Wave gi < NT of the front waves finishes group NT w + gi.
-template <int KW>
+template <int NB>
 struct GroupShape {
-    static constexpr int NT = KW > 8 ? 2 : 1, G = 32 * KW, NWG = G / NT;
+    static constexpr int NT = NB > 64 ? 2 : 1, G = 4 * NB, NWG = G / NT;
 };
 
 // Helper workgroups.  At C = 2560 the grid of C / 16 = 160 owner workgroups leaves 96 compute units without
@@ -101,15 +112,15 @@ struct GroupShape {
 // The owner workgroups then stream 9 tiles per layer instead of 13 and have the ffn receptance tile only to
 // multiply in that phase.
 constexpr int kHelperPace = 20;        // s_sleep units (64 cycles) between groups of three weight loads of a helper (10 and 30: within 0.5 %; 0: +2 %, 60: +3 %)
-template <int KW>
+template <int NB>
 struct DecodeLdsDigBytes {          // bytes of the digit planes at the start of LDS (three C-row sets, or one F-row set)
-    static constexpr int value = (3 * 4 * (512 * KW + 64) > 4 * (2048 * KW + 64)) ? 3 * 4 * (512 * KW + 64) : 4 * (2048 * KW + 64);
+    static constexpr int value = (3 * 4 * (64 * NB + 64) > 4 * (256 * NB + 64)) ? 3 * 4 * (64 * NB + 64) : 4 * (256 * NB + 64);
 };
 
-template <int KW>
+template <int NB>
 struct HelperShape {
-    static constexpr int NH = KW == 5 ? 80 : 0;                    // helper workgroups
-    static constexpr int TILES = NH ? (4 * 32 * KW) / NH : 1;      // ffn key tiles of 16 columns per helper
+    static constexpr int NH = NB == 40 ? 80 : 0;                    // helper workgroups
+    static constexpr int TILES = NH ? (4 * 4 * NB) / NH : 1;      // ffn key tiles of 16 columns per helper
     static constexpr int LDS_BLOCKS = 4;                           // weight blocks per wavefront that wait in LDS instead of registers
 };
 
@@ -372,16 +383,17 @@ __device__ __forceinline__ void settle_quads(Front &fx, xtab_t src, int first, i
     }
 }
 
-// Sum of the 8 back waves' digit sums of column n of parked tile `slot`, digits recombined:
+// Sum of the BW back waves' digit sums of column n of parked tile `slot`, digits recombined:
 // sum_k 256^k sum_c s_k,c w_c.  Every digit sum is below 2^28 in magnitude and the total below 2^52,
 // so each step of the float64 Horner form is exact.
+template <int BW>
 __device__ __forceinline__ double tile_total(const v4i *red, int slot, int n) {
     int d0 = 0, d1 = 0, d2 = 0, d3 = 0;
 #pragma unroll
-    for (int h = 0; h < kBW; h += 4) {
+    for (int h = 0; h < BW; h += 4) {
         v4i v[4];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) v[w] = red[(slot * kBW + h + w) * 16 + n];
+        for (int w = 0; w < 4; ++w) v[w] = red[(slot * BW + h + w) * 16 + n];
 #pragma unroll
         for (int w = 0; w < 4; ++w) { d0 += v[w].x; d1 += v[w].y; d2 += v[w].z; d3 += v[w].w; }
     }
@@ -389,8 +401,9 @@ __device__ __forceinline__ double tile_total(const v4i *red, int slot, int n) {
 }
 // y = S (sum_c q_c (code_c - 128)) + zp  with  sum_c q_c w_c = total + 0x808080 sum_c w_c.  S is a power
 // of two and the sum an integer below 2^53: one rounding, in the addition of zp.
+template <int BW>
 __device__ __forceinline__ double finish_col(const v4i *red, int slot, int n, double S, int colsum, double zp) {
-    return fma(S, tile_total(red, slot, n) + (double)(0x808080LL * (long long)colsum), zp);
+    return fma(S, tile_total<BW>(red, slot, n) + (double)(0x808080LL * (long long)colsum), zp);
 }
 
 // LayerNorm statistics of the 16 channels a DPP row owns, and everything a consumer of x needs that
@@ -548,12 +561,12 @@ __device__ __forceinline__ double ln_zp(const double *stat, const u64 *rec, int 
 // waits for x and its records, leaves mean, rsd and the per-product sums in stat[0..7] and each
 // product's scale and zero-point sum in stat[8 + 2m], stat[9 + 2m], writes NM sets of digit planes.  Contains one workgroup barrier (statistics) and ends with the "digits
 // ready" barrier.  rec: the LDS owner record of the layer (scalars).
-template <int KW, int FW, int NM>
+template <int NB, int FW, int NM>
 __device__ __forceinline__ void ln_front(Front &fx, int &seq, const DArgs &a, const float *P32, const float *Q32,
                                          const u64 *rec, int m0, unsigned epoch, signed char *dig, double *stat,
                                          long long *tr, long long *tp, int xr_m0 = 0) {
     // xr_m0: the first of the NM products among those the publisher wrote records for
-    constexpr int C = 512 * KW, G = 32 * KW, FT = 64 * FW, NQ = C / 4, NQT = (NQ + FT - 1) / FT;
+    constexpr int C = 64 * NB, G = 4 * NB, FT = 64 * FW, NQ = C / 4, NQT = (NQ + FT - 1) / FT;
     constexpr int PS = C + 64;
     static_assert(FW >= 4, "one front wave per product plus wave 0");
     fx.refresh();
@@ -635,7 +648,7 @@ __device__ __forceinline__ void ln_front(Front &fx, int &seq, const DArgs &a, co
 // Front side of a product whose input was scaled by its producers (att output, ffn value):
 // the records carry max |xs| and the shares of the zero-point sum.  Leaves the scale in stat[16],
 // the zero-point sum in stat[17].  Ends with the "digits ready" barrier.
-template <int KW, int FW, int NQT, int G = 32 * KW>     // G: workgroups that publish a record each
+template <int NB, int FW, int NQT, int G = 4 * NB>     // G: workgroups that publish a record each
 __device__ __forceinline__ void vec_front(Front &fx, int &seq, const u64 *src, const u64 *rec, int nq, unsigned epoch,
                                           signed char *dig, int plane_stride, double *stat, long long *tr, long long *tp) {
     constexpr int FT = 64 * FW;
@@ -683,13 +696,13 @@ __device__ __forceinline__ void vec_front(Front &fx, int &seq, const u64 *src, c
 }
 
 // =============================================================================
-template <int KW, int FW, bool HELP> using BackOf = std::conditional_t<HELP, BackCfgH<KW, FW>, BackCfg<KW, FW>>;
+template <int NB, int FW, bool HELP> using BackOf = std::conditional_t<HELP, BackCfgH<NB, FW>, BackCfg<NB, FW>>;
 
-template <int KW, int FW, bool TRACE, bool HELP>
+template <int NB, int FW, bool TRACE, bool HELP>
 __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, const v4i *red, double *stat, double *rf_lds,
                                            lds_flag_t *flags, u64 *own_lds, double *st_lds, long long *trace_lds) {
-    constexpr int C = 512 * KW, F = 4 * C, G = GroupShape<KW>::G, NT = GroupShape<KW>::NT, NWG = GroupShape<KW>::NWG, FT = 64 * FW;
-    constexpr int PS = C + 64, PSF = F + 64;
+    constexpr int C = 64 * NB, F = 4 * C, G = GroupShape<NB>::G, NT = GroupShape<NB>::NT, NWG = GroupShape<NB>::NWG, FT = 64 * FW;
+    constexpr int BW = back_waves(NB), PS = C + 64, PSF = F + 64;
     constexpr int NQH = F / 4, NQTH = (NQH + FT - 1) / FT, NQC = C / 4, NQTC = (NQC + FT - 1) / FT;
     static_assert(FW >= NT, "one finishing wave per group");
     Front fx;
@@ -699,7 +712,7 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
     const bool fin = fx.wave < NT;                       // wave gi finishes the workgroup's group gi of 16 channels
     const int gi = fin ? fx.wave : 0;
     const int g = NT * wg + gi;
-    red += gi * kSlotsPerGroup * kBW * 16;               // the group's parked tiles
+    red += gi * kSlotsPerGroup * BW * 16;               // the group's parked tiles
     rf_lds += gi * 32;
     // stamps are collected in LDS and copied out after the head: a store to memory here would queue behind the weight stream
     long long *trace = TRACE ? trace_lds : nullptr;     // uniform; thread 0 stamps
@@ -709,7 +722,7 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
     RWKV_IDS();
 
 #pragma unroll
-    for (int t = 0; t < NT; ++t) stage_owner_record<FT, KW>(a, 0, NT * wg + t, G, C, own_lds + (2 * t) * kOrSlots, fx.tid);   // read after the first barriers below
+    for (int t = 0; t < NT; ++t) stage_owner_record<FT, prep_parts(C)>(a, 0, NT * wg + t, G, C, own_lds + (2 * t) * kOrSlots, fx.tid);   // read after the first barriers below
     // the residual value of the own channels lives in LDS between the epilogues (rf_lds[16 + n])
     double *x_lds = rf_lds + 16;
     if (fin && row == 0) x_lds[n] = a.m.X0[c_own];
@@ -730,7 +743,7 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
         if (tr && fx.tid == 0) { tr[0] = wall_clock64(); tr[23] = clock64(); }     // [23]: shader clock, for its ratio to the wall clock
 
         // ===================== phase 1: att k, v, r ============================
-        ln_front<KW, FW, 3>(fx, seq, a, P32, Q32, rec, 0, e, dig, stat, tr ? tr + 1 : nullptr, tr ? tr + 16 : nullptr);
+        ln_front<NB, FW, 3>(fx, seq, a, P32, Q32, rec, 0, e, dig, stat, tr ? tr + 1 : nullptr, tr ? tr + 16 : nullptr);
         if (!fx.ok) break;
         RWKV_IDS();
         // while the matrix cores run: the LayerNorm output of the own channel is the new att shift state (block.py:58,63-64)
@@ -740,7 +753,7 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
         if (fin) {
             const int j = row < 3 ? row : 0;             // rows 0..2: columns of k, v, r
             const int cs1 = (int)(j == 0 ? or_lo(rec, OR_CSK_CSV * 16 + n) : (j == 1 ? or_hi(rec, OR_CSK_CSV * 16 + n) : or_lo(rec, OR_CSR_CSFR * 16 + n)));
-            const double y = finish_col(red, j, n, stat[8 + 2 * j], cs1, stat[9 + 2 * j]);
+            const double y = finish_col<BW>(red, j, n, stat[8 + 2 * j], cs1, stat[9 + 2 * j]);
             const double yk = lane_read_f64(y, n), yv = lane_read_f64(y, n + 16), yr = lane_read_f64(y, n + 32);
             if (tr && fx.tid == 0) tr[20] = wall_clock64();
             {                                              // all four rows: the same 16 channels; one store instruction
@@ -773,14 +786,14 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
         RWKV_IDS();
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-            stage_owner_record<FT, KW>(a, l + 1, NT * wg + t, G, C, own_lds + (2 * t + ((l + 1) & 1)) * kOrSlots, fx.tid);
-        vec_front<KW, FW, NQTC>(fx, seq, a.b.A, a.b.AR, NQC, e + 1u, dig, PS, stat, tr ? tr + 5 : nullptr, tr ? tr + 17 : nullptr);
+            stage_owner_record<FT, prep_parts(C)>(a, l + 1, NT * wg + t, G, C, own_lds + (2 * t + ((l + 1) & 1)) * kOrSlots, fx.tid);
+        vec_front<NB, FW, NQTC>(fx, seq, a.b.A, a.b.AR, NQC, e + 1u, dig, PS, stat, tr ? tr + 5 : nullptr, tr ? tr + 17 : nullptr);
         if (!fx.ok) break;
         __syncthreads();
         if (tr && fx.tid == 0) tr[7] = wall_clock64();
         RWKV_IDS();
         if (fin) {                                         // all four rows: the same 16 channels; row 1 + m reduces for product m
-            const double x_own = x_lds[n] + finish_col(red, 0, n, stat[16], (int)or_hi(rec, OR_RNGO_CSO * 16 + n), stat[17]);   // block.py:80
+            const double x_own = x_lds[n] + finish_col<BW>(red, 0, n, stat[16], (int)or_hi(rec, OR_RNGO_CSO * 16 + n), stat[17]);   // block.py:80
             const int m = row == 2 ? 1 : 0;                // [0] ffn_k, [1] ffn_r
             const u64 pf = rec[OR_PF * 16 + n];
             const float Pm = __uint_as_float(m ? (unsigned)(pf >> 32) : (unsigned)pf);
@@ -793,9 +806,9 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
 
         // ===================== phase 3: ffn receptance + key ===================
         if constexpr (HELP)      // the ffn key tiles are the helper workgroups': the receptance alone, second of the two products published
-            ln_front<KW, FW, 1>(fx, seq, a, P32, Q32, rec, 4, e + 2u, dig, stat, tr ? tr + 9 : nullptr, tr ? tr + 18 : nullptr, 1);
+            ln_front<NB, FW, 1>(fx, seq, a, P32, Q32, rec, 4, e + 2u, dig, stat, tr ? tr + 9 : nullptr, tr ? tr + 18 : nullptr, 1);
         else
-            ln_front<KW, FW, 2>(fx, seq, a, P32, Q32, rec, 3, e + 2u, dig, stat, tr ? tr + 9 : nullptr, tr ? tr + 18 : nullptr);   // [0] ffn_k, [1] ffn_r
+            ln_front<NB, FW, 2>(fx, seq, a, P32, Q32, rec, 3, e + 2u, dig, stat, tr ? tr + 9 : nullptr, tr ? tr + 18 : nullptr);   // [0] ffn_k, [1] ffn_r
         if (!fx.ok) break;
         RWKV_IDS();
         // the LayerNorm output of the own channel is the new ffn shift state (block.py:82,87-88)
@@ -804,13 +817,13 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
         if (tr && fx.tid == 0) tr[11] = wall_clock64();
         if constexpr (HELP) {
             if (fin && row == 0) {                         // the receptance gate of the own channels (block.py:95)
-                const double yr = finish_col(red, 0, n, stat[8], (int)or_hi(rec, OR_CSR_CSFR * 16 + n), stat[9]);
+                const double yr = finish_col<BW>(red, 0, n, stat[8], (int)or_hi(rec, OR_CSR_CSFR * 16 + n), stat[9]);
                 rf_lds[n] = (double)sigmoid_f32((float)yr);
             }
         } else if (fin) {
             // parked tiles: 0 = ffn_r, 1..4 = ffn_k tiles g, g+G, g+2G, g+3G
             const int f_own = 16 * (g + G * row) + n;      // column of ffn_k tile `row`
-            const double y = finish_col(red, 1 + row, n, stat[8], (int)or_hi(rec, kOrRngVCs + lane), stat[9]);
+            const double y = finish_col<BW>(red, 1 + row, n, stat[8], (int)or_hi(rec, kOrRngVCs + lane), stat[9]);
             const double h = y > 0.0 ? y : 0.0;                                  // block.py:97-98
             const double hh = h * h;
             const float xs = (float)(hh * (double)__uint_as_float(or_lo(rec, kOrRngVCs + lane)));
@@ -820,21 +833,21 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
             const float hi = (float)so, lo = (float)(so - (double)hi);
             if (lane < 3) put_word(a.b.HR + (size_t)lane * G + g, e + 3u, lane == 0 ? mx : (lane == 1 ? hi : lo));
             if (row == 0) {                                // after H is out: the receptance gate of the own channels (block.py:95)
-                const double yr = finish_col(red, 0, n, stat[10], (int)or_hi(rec, OR_CSR_CSFR * 16 + n), stat[11]);
+                const double yr = finish_col<BW>(red, 0, n, stat[10], (int)or_hi(rec, OR_CSR_CSFR * 16 + n), stat[11]);
                 rf_lds[n] = (double)sigmoid_f32((float)yr);
             }
         }
         if (tr && fx.tid == 0) tr[12] = wall_clock64();
 
         // ===================== phase 4: ffn value ==============================
-        vec_front<KW, FW, NQTH, HELP ? 2 * HelperShape<KW>::NH : G>(fx, seq, a.b.H, a.b.HR, NQH, e + 3u, dig, PSF, stat, tr ? tr + 13 : nullptr,
+        vec_front<NB, FW, NQTH, HELP ? 2 * HelperShape<NB>::NH : G>(fx, seq, a.b.H, a.b.HR, NQH, e + 3u, dig, PSF, stat, tr ? tr + 13 : nullptr,
                                                                 tr ? tr + 19 : nullptr);
         if (!fx.ok) break;
         __syncthreads();
         if (tr && fx.tid == 0) tr[15] = wall_clock64();
         RWKV_IDS();
         if (fin) {                                         // all four rows: the same 16 channels; row 1 + m reduces for product m
-            const double y = finish_col(red, 0, n, stat[16], (int)or_lo(rec, OR_CSFV * 16 + n), stat[17]);
+            const double y = finish_col<BW>(red, 0, n, stat[16], (int)or_lo(rec, OR_CSFV * 16 + n), stat[17]);
             const double x_own = y * rf_lds[n] + x_lds[n];                       // block.py:100
             const int m = row >= 1 ? row - 1 : 0;          // next layer's att k, v, r (or the head: one product)
             const u64 pn = rec[(OR_PN01 + (m >> 1)) * 16 + n];
@@ -849,29 +862,30 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
 
     // ========================= head (opt.py:71-73) ==============================
     const int v_tiles = (V + 15) / 16, head_rounds = (v_tiles + NWG - 1) / NWG;
-    red -= gi * kSlotsPerGroup * kBW * 16;                 // the head's parked tiles belong to the workgroup
+    red -= gi * kSlotsPerGroup * BW * 16;                 // the head's parked tiles belong to the workgroup
     const u64 *rec_h = own_lds + (L & 1) * kOrSlots;
-    // column sums of the workgroup's head tiles: requested now, parked in the LDS half that held the
-    // last layer's record once the wait for x is over (a load inside the loop below would cost a
+    // column sums of the workgroup's head tiles: requested now, parked in LDS (where there is no
+    // room of their own, in the half that held the last layer's record) once the wait for x is over (a load inside the loop below would cost a
     // round trip through the busy memory pipeline in every round)
-    int *csh = reinterpret_cast<int *>(own_lds + ((L + 1) & 1) * kOrSlots);
-    int csv[kHeadCsPerThread];
+    constexpr int HCS = head_cs_per_thread(NB);
+    int *csh = reinterpret_cast<int *>(own_lds + (head_cs_lds_bytes(NB) ? 2 : (L + 1) & 1) * kOrSlots);
+    int csv[HCS];
 #pragma unroll
-    for (int k = 0; k < kHeadCsPerThread; ++k) {
+    for (int k = 0; k < HCS; ++k) {
         const int i = fx.tid + FT * k, v = 16 * (wg + NWG * (i >> 4)) + (i & 15);
         csv[k] = (i < head_rounds * 16 && v < V) ? a.m.cs_head[v] : 0;
     }
     if (fx.ok)
-        ln_front<KW, FW, 1>(fx, seq, a, a.m.P32 + (size_t)L * kLnMats * C, a.m.Q32 + (size_t)L * kLnMats * C, rec_h, 0,
+        ln_front<NB, FW, 1>(fx, seq, a, a.m.P32 + (size_t)L * kLnMats * C, a.m.Q32 + (size_t)L * kLnMats * C, rec_h, 0,
                             a.epoch0 + 4u * (unsigned)L, dig, stat, nullptr, nullptr);
     if (!fx.ok) return;     // every wave leaves after the same barrier: the flag is tested after each one that follows a wait
 #pragma unroll
-    for (int k = 0; k < kHeadCsPerThread; ++k)
+    for (int k = 0; k < HCS; ++k)
         if (fx.tid + FT * k < head_rounds * 16) csh[fx.tid + FT * k] = csv[k];
     RWKV_IDS();
 #undef RWKV_IDS
     unsigned par = 0;
-    constexpr int NS = BackOf<KW, FW, HELP>::NS;          // head tiles per barrier round
+    constexpr int NS = BackOf<NB, FW, HELP>::NS;          // head tiles per barrier round
     double Sh;
     float invSh;
     ln_scale(stat, rec_h, 0, 0, Sh, invSh);
@@ -884,7 +898,7 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
         if (s < NS && h0 + s < head_rounds) {
             const int v = 16 * (wg + NWG * (h0 + s)) + n;
             if (v < V) {
-                const double y = finish_col(red + par * (NS * kBW * 16), s, n, Sh, csh[16 * (h0 + s) + n], zph);
+                const double y = finish_col<BW>(red + par * (NS * BW * 16), s, n, Sh, csh[16 * (h0 + s) + n], zph);
                 a.logits[v] = y;
                 if (y > best) { best = y; best_i = v; }    // v grows with the round: an equal later value does not replace
             }
@@ -915,19 +929,19 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
 // cores), wavefront 0 finishes the columns.
 // Three workgroup barriers per layer, each followed by a test of the abort word, so that every wavefront leaves
 // after the same barrier.
-template <int KW, int FW>
+template <int NB, int FW>
 __device__ __forceinline__ void helper_path(const DArgs &a, signed char *dig, v4i *red, double *stat, lds_flag_t *flags,
                                             v4i *stash) {
-    constexpr int C = 512 * KW, G = GroupShape<KW>::G, NWG = GroupShape<KW>::NWG;
-    constexpr int NH = HelperShape<KW>::NH, TPH = HelperShape<KW>::TILES, NWV = FW + kBW, FT = 64 * NWV;
+    constexpr int C = 64 * NB, G = GroupShape<NB>::G, NWG = GroupShape<NB>::NWG;
+    constexpr int NH = HelperShape<NB>::NH, TPH = HelperShape<NB>::TILES, NWV = FW + back_waves(NB), FT = 64 * NWV;
     // NTW tiles per wavefront, WPT wavefronts (parts of the contraction) per tile, KB blocks per tile, KPW blocks of
     // the contraction per wavefront, BPW weight blocks per wavefront
-    constexpr int NTW = 4, WPT = NWV * NTW / TPH, KB = 8 * KW, KPW = KB / WPT, BPW = NTW * KPW;
+    constexpr int NTW = 4, WPT = NWV * NTW / TPH, KB = NB, KPW = KB / WPT, BPW = NTW * KPW;
     static_assert(TPH % NTW == 0 && (TPH / NTW) * WPT == NWV && WPT * KPW == KB && TPH * 16 == 128 && NWV >= 3, "helper shape");
     // Of a wavefront's BPW blocks the last of every tile waits in LDS (64 lanes x 16 bytes each, `stash`), the others
     // in registers: all of them in registers would leave too few for the gather and the digits, and the compiler
     // would park blocks in scratch memory - a reload from memory in the middle of the phase.
-    constexpr int BLDS = HelperShape<KW>::LDS_BLOCKS, BREG = BPW - BLDS, KREG = BREG / NTW;      // per tile: blocks 0 .. KREG - 1 in registers
+    constexpr int BLDS = HelperShape<NB>::LDS_BLOCKS, BREG = BPW - BLDS, KREG = BREG / NTW;      // per tile: blocks 0 .. KREG - 1 in registers
     static_assert(BLDS == NTW && KREG == KPW - 1, "one block of every tile waits in LDS");
     constexpr int PS = C + 64, NQ = C / 4, NQT = (NQ + FT - 1) / FT, MFK = 3;      // MFK: the ffn key product in the layer's tables
     static_assert(NQT == 1, "one group of four channels per thread");
@@ -937,7 +951,7 @@ __device__ __forceinline__ void helper_path(const DArgs &a, signed char *dig, v4
     int *c_cs = reinterpret_cast<int *>(cQ + NQ);
     float *c_rg = reinterpret_cast<float *>(c_cs + 128);
     double *c_of = reinterpret_cast<double *>(c_rg + 128);
-    static_assert(4 * PS + 2 * NQ * 16 + 128 * 16 <= DecodeLdsDigBytes<KW>::value, "constants fit between the digit planes and the parked sums");
+    static_assert(4 * PS + 2 * NQ * 16 + 128 * 16 <= DecodeLdsDigBytes<NB>::value, "constants fit between the digit planes and the parked sums");
     int *redi = reinterpret_cast<int *>(red);              // [TPH][16 columns][4 digit sums], added to by the WPT parts of a tile
     Front fx;
     fx.abort_flag = a.b.abort_flag; fx.flags = flags; fx.spin_limit = a.spin_limit; fx.ok = true;
@@ -998,11 +1012,11 @@ __device__ __forceinline__ void helper_path(const DArgs &a, signed char *dig, v4
             c_cs[col] = gld(csl + f); c_rg[col] = gld(rv + f); c_of[col] = gld(ov + f);
         }
         if (fx.wave == 2 && fx.lane == 0) {                // the product's scalars (the per-token ones: parts in a fixed order)
-            const DScal *sc = a.m.sc + l, *sp = a.m.scp + (size_t)l * KW;
+            const DScal *sc = a.m.sc + l, *sp = a.m.scp + (size_t)l * prep_parts(C);
             double sq = 0.0;
             float mq = 0.f;
 #pragma unroll
-            for (int q = 0; q < KW; ++q) { sq += gld(&sp[q].sumQO[MFK]); mq = fmaxf(mq, gld(&sp[q].maxQ[MFK])); }
+            for (int q = 0; q < prep_parts(C); ++q) { sq += gld(&sp[q].sumQO[MFK]); mq = fmaxf(mq, gld(&sp[q].maxQ[MFK])); }
             stat[20] = gld(&sc->sumPO[MFK]); stat[21] = sq; stat[22] = (double)gld(&sc->maxP[MFK]); stat[23] = (double)mq;
         }
         ++seq;
@@ -1108,36 +1122,37 @@ __device__ __forceinline__ void helper_path(const DArgs &a, signed char *dig, v4
     }
 }
 
-template <int KW, int FW, bool HELP = false>
+template <int NB, int FW, bool HELP = false>
 struct DecodeLds {
-    using Back = BackOf<KW, FW, HELP>;
-    static constexpr int C = 512 * KW, F = 4 * C, NT = GroupShape<KW>::NT;
+    using Back = BackOf<NB, FW, HELP>;
+    static constexpr int C = 64 * NB, F = 4 * C, NT = GroupShape<NB>::NT;
     static constexpr int PS = C + 64, PSF = F + 64;
     static constexpr int DIG_BYTES = (3 * 4 * PS > 4 * PSF) ? 3 * 4 * PS : 4 * PSF;
     static constexpr int RED_SLOTS = Back::RED_SLOTS;
-    static constexpr int RED_BYTES = RED_SLOTS * kBW * 16 * 16;
+    static constexpr int RED_BYTES = RED_SLOTS * back_waves(NB) * 16 * 16;
     static constexpr int STAT_BYTES = 32 * 8, RF_BYTES = NT * 32 * 8, FLAG_BYTES = FLAG_COUNT * 4;   // RF: gate and residual of the own channels
     static constexpr int OWN_OFFSET = DIG_BYTES + RED_BYTES + STAT_BYTES + RF_BYTES + FLAG_BYTES;
-    static constexpr int STATE_OFFSET = OWN_OFFSET + NT * 2 * kOrSlots * 8;
+    static constexpr int STATE_OFFSET = OWN_OFFSET + NT * 2 * kOrSlots * 8 + head_cs_lds_bytes(NB);      // (the head's column sums, if any, follow the records)
     static __host__ __device__ int state_bytes(int L) { return NT == 1 ? L * 5 * 16 * 8 : 0; }  // the new state rows of the own channels
     // a helper workgroup's stash of weight blocks lies over the owner records and state rows, which it does not have
     static constexpr int STASH_OFFSET = OWN_OFFSET;
-    static constexpr int STASH_BYTES = HELP ? (FW + kBW) * HelperShape<KW>::LDS_BLOCKS * 1024 : 0;
+    static constexpr int STASH_BYTES = HELP ? (FW + back_waves(NB)) * HelperShape<NB>::LDS_BLOCKS * 1024 : 0;
     static __host__ __device__ int total(int L, bool trace = false) {                           // (+ the stamps)
         const int own = STATE_OFFSET + state_bytes(L);
         return (own > STASH_OFFSET + STASH_BYTES ? own : STASH_OFFSET + STASH_BYTES) + (trace ? L * kTraceStampsPerLayer * 8 : 0);
     }
+    static_assert(head_cs_lds_bytes(NB) == 0 || (NT == 1 && head_cs_lds_bytes(NB) >= head_cs_per_thread(NB) * 64 * FW * 4), "head column sums");
     // the generated back-wave program addresses LDS by these offsets
     static_assert(Back::RED == DIG_BYTES, "parked tiles follow the digit planes");
     static_assert(Back::FLAG == DIG_BYTES + RED_BYTES + STAT_BYTES + RF_BYTES + FLAG_ABORT * 4, "abort flag offset");
     static_assert(RED_SLOTS >= kSlotsPerGroup * NT && RED_SLOTS >= 2 * Back::NS, "park slots");
-    static_assert(DIG_BYTES == DecodeLdsDigBytes<KW>::value, "digit planes");
-    static_assert(!HELP || RED_BYTES >= HelperShape<KW>::TILES * 256, "a helper's tile sums");
+    static_assert(DIG_BYTES == DecodeLdsDigBytes<NB>::value, "digit planes");
+    static_assert(!HELP || RED_BYTES >= HelperShape<NB>::TILES * 256, "a helper's tile sums");
 };
 
-template <int KW, int FW, bool TRACE, bool HELP>
-__global__ void __launch_bounds__((FW + kBW) * 64) decode_kernel(const DArgs a) {
-    using Lds = DecodeLds<KW, FW, HELP>;
+template <int NB, int FW, bool TRACE, bool HELP>
+__global__ void __launch_bounds__((FW + back_waves(NB)) * 64) decode_kernel(const DArgs a) {
+    using Lds = DecodeLds<NB, FW, HELP>;
     extern __shared__ __align__(16) unsigned char smem[];
     signed char *dig = reinterpret_cast<signed char *>(smem);
     v4i *red = reinterpret_cast<v4i *>(smem + Lds::DIG_BYTES);
@@ -1149,20 +1164,20 @@ __global__ void __launch_bounds__((FW + kBW) * 64) decode_kernel(const DArgs a) 
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     if constexpr (HELP) {
-        if ((int)blockIdx.x >= GroupShape<KW>::NWG) {          // (uniform for the workgroup)
-            helper_path<KW, FW>(a, dig, red, stat, flags, reinterpret_cast<v4i *>(smem + Lds::STASH_OFFSET));
+        if ((int)blockIdx.x >= GroupShape<NB>::NWG) {          // (uniform for the workgroup)
+            helper_path<NB, FW>(a, dig, red, stat, flags, reinterpret_cast<v4i *>(smem + Lds::STASH_OFFSET));
             return;
         }
     }
     if (wave < FW) {
-        front_path<KW, FW, TRACE, HELP>(a, dig, red, stat, rf_lds, flags, reinterpret_cast<u64 *>(smem + Lds::OWN_OFFSET),
+        front_path<NB, FW, TRACE, HELP>(a, dig, red, stat, rf_lds, flags, reinterpret_cast<u64 *>(smem + Lds::OWN_OFFSET),
                                   reinterpret_cast<double *>(smem + Lds::STATE_OFFSET),
                                   reinterpret_cast<long long *>(smem + Lds::total(a.m.L)));       // (total without the stamps = where they start)
     } else {
-        constexpr int NWG = GroupShape<KW>::NWG;
+        constexpr int NWG = GroupShape<NB>::NWG;
         const int v_tiles = (a.m.V + 15) / 16, head_rounds = (v_tiles + NWG - 1) / NWG;
         const unsigned lds = (unsigned)(uintptr_t)(RWKV_LDS unsigned char *)smem;
-        BackOf<KW, FW, HELP>::run(a.m.jt + (size_t)blockIdx.x * (a.m.L + 1) * 16, a.m.w_head, a.m.L, head_rounds, v_tiles,
+        BackOf<NB, FW, HELP>::run(a.m.jt + (size_t)blockIdx.x * (a.m.L + 1) * 16, a.m.w_head, a.m.L, head_rounds, v_tiles,
                          (int)blockIdx.x, wave - FW, lds);
     }
 }
@@ -1172,8 +1187,6 @@ __global__ void __launch_bounds__((FW + kBW) * 64) decode_kernel(const DArgs a) 
 // (they change with every token); block L computes x0 = ln0(emb[token]) (emb.py:9, opt.py:63-64)
 // and publishes it, with its LayerNorm records, as the input of layer 0.
 // ---------------------------------------------------------------------------
-constexpr int kPrepThreads = 512;
-
 template <int N>
 __device__ __forceinline__ void prep_block_sum(double (&v)[N], double *scr) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1213,15 +1226,17 @@ __device__ __forceinline__ void prep_block_max(float (&v)[N], float *scr) {
 
 // Channels [512 part, 512 part + 512) of layer l: Q32 and this part's share of the scalars.
 __device__ __forceinline__ void prep_layer_part(const DArgs &a, int l, int part, double *scr) {
-    const int C = a.m.C, KWr = C / kPrepThreads;
+    const int C = a.m.C;
     const DPrep &p = a.m.prep[l];
     const double *sl = a.state + (size_t)l * 5 * C;
     const int c = part * kPrepThreads + threadIdx.x;
-    double sq[kLnMats];
-    float mq[kLnMats];
-    const double sh0 = sl[c], sh1 = sl[(size_t)C + c], b1 = p.ln1_b[c], b2 = p.ln2_b[c];
+    double sq[kLnMats] = {0, 0, 0, 0, 0};
+    float mq[kLnMats] = {0, 0, 0, 0, 0};
+    const bool in = c < C;                              // (C = 768: the second part is half a part)
+    const double sh0 = in ? sl[c] : 0.0, sh1 = in ? sl[(size_t)C + c] : 0.0, b1 = in ? p.ln1_b[c] : 0.0, b2 = in ? p.ln2_b[c] : 0.0;
 #pragma unroll
     for (int m = 0; m < kLnMats; ++m) {
+        if (!in) continue;
         const bool att = m < 3;
         const double mu = att ? p.att_mix[(size_t)m * C + c] : p.ffn_mix[(size_t)(m - 3) * C + c];
         const double base = (att ? b1 : b2) * mu + (att ? sh0 : sh1) * (1.0 - mu);   // block.py:67,91 without the x term
@@ -1234,17 +1249,17 @@ __device__ __forceinline__ void prep_layer_part(const DArgs &a, int l, int part,
     prep_block_sum<kLnMats>(sq, scr);
     prep_block_max<kLnMats>(mq, reinterpret_cast<float *>(scr));
     if (threadIdx.x < kLnMats) {
-        DScal &d = a.m.scp[(size_t)l * KWr + part];
+        DScal &d = a.m.scp[(size_t)l * prep_parts(C) + part];
         d.sumQO[threadIdx.x] = sq[threadIdx.x];
         d.maxQ[threadIdx.x] = mq[threadIdx.x];
     }
 }
 
 // x0 = ln0(emb[tok]) (emb.py:9, opt.py:63-64), published with its LayerNorm records as the input
-// of layer 0 under `epoch`.  C is a multiple of 512 and thread t takes channels t, t + 512, ...
+// of layer 0 under `epoch`.  C is a multiple of 64 and thread t takes channels t, t + 512, ...
 __device__ __forceinline__ void prep_token(const DArgs &a, int64_t tok, unsigned epoch, double *scr) {
     constexpr int kMaxParts = 10;                               // C <= 5120
-    const int C = a.m.C, G = a.m.G, parts = C / kPrepThreads;
+    const int C = a.m.C, G = a.m.G;
     if (tok < 0) tok = 0;
     if (tok >= a.m.V) tok = a.m.V - 1;
     // everything this thread needs is requested before the first use: the block is one chain of memory latencies otherwise
@@ -1253,7 +1268,7 @@ __device__ __forceinline__ void prep_token(const DArgs &a, int64_t tok, unsigned
 #pragma unroll
     for (int k = 0; k < kMaxParts; ++k) {
         const int c = threadIdx.x + k * kPrepThreads;
-        if (k < parts) {
+        if (c < C) {
             v[k] = (double)a.m.emb[(size_t)tok * C + c];
             lw[k] = a.m.ln0_w[c]; lb[k] = a.m.ln0_b[c];
 #pragma unroll
@@ -1263,16 +1278,16 @@ __device__ __forceinline__ void prep_token(const DArgs &a, int64_t tok, unsigned
     double s[2] = {0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < kMaxParts; ++k)
-        if (k < parts) { s[0] += v[k]; s[1] += v[k] * v[k]; }
+        if ((int)threadIdx.x + k * kPrepThreads < C) { s[0] += v[k]; s[1] += v[k] * v[k]; }
     prep_block_sum<2>(s, scr);
     const double mean = s[0] / (double)C;
     double var = s[1] / (double)C - mean * mean;
     if (var < 0.0) var = 0.0;
     const double rsd = 1.0 / sqrt(var + 1e-5);
 #pragma unroll
-    for (int k = 0; k < kMaxParts; ++k) {                       // whole waves are in or out: C % 512 == 0
-        if (k < parts) {
-            const int c = threadIdx.x + k * kPrepThreads;
+    for (int k = 0; k < kMaxParts; ++k) {                       // whole waves are in or out: C % 64 == 0
+        const int c = threadIdx.x + k * kPrepThreads;
+        if (c < C) {
             const double x0 = lw[k] * ((v[k] - mean) * rsd) + lb[k];
             a.m.X0[c] = x0;
             publish_ln_input<3>(a.b.X, a.b.XR, G, c >> 4, c & 15, epoch, x0, P[k], PO[k]);
@@ -1280,11 +1295,11 @@ __device__ __forceinline__ void prep_token(const DArgs &a, int64_t tok, unsigned
     }
 }
 
-// grid: L * (C / 512) layer parts, then one block for the token.
+// grid: L * ceil(C / 512) layer parts, then one block for the token.
 __global__ void __launch_bounds__(kPrepThreads) prep_kernel(const DArgs a) {
     __shared__ double scr[8 * (kPrepThreads / 64)];
     if (a.stop && gld(a.stop) != 0) return;
-    const int parts = a.m.C / kPrepThreads;
+    const int parts = prep_parts(a.m.C);
     const int b = blockIdx.x;
     if (b < a.m.L * parts) prep_layer_part(a, b / parts, b % parts, scr);
     else prep_token(a, a.token[0], a.epoch0, scr);
@@ -1293,12 +1308,12 @@ __global__ void __launch_bounds__(kPrepThreads) prep_kernel(const DArgs a) {
 // Between two greedy tokens: the greedy token (the single-token kernel left one candidate per
 // workgroup: the first maximum of the logits it wrote) -> out_token[0], and the preparation of the
 // next step (which reads the state the step before has just updated) in the same launch.
-// grid: L * (C / 512) layer parts, then one block for the token.  a.epoch0: the epoch of the NEXT
+// grid: L * ceil(C / 512) layer parts, then one block for the token.  a.epoch0: the epoch of the NEXT
 // token step.
 __global__ void __launch_bounds__(kPrepThreads) next_token_kernel(const DArgs a, int64_t *__restrict__ out_token) {
     __shared__ double scr[8 * (kPrepThreads / 64)];
     __shared__ int sidx[kPrepThreads / 64];
-    const int parts = a.m.C / kPrepThreads;
+    const int parts = prep_parts(a.m.C);
     const int b = blockIdx.x;
     if (b < a.m.L * parts) { prep_layer_part(a, b / parts, b % parts, scr); return; }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1483,17 +1498,40 @@ __global__ void __launch_bounds__(kPrepThreads) build_consts_kernel(const ConstA
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
+// LDS of the token kernel at width C (0: no such kernel); it grows with the layers, whose new state rows wait there.
+static int decode_lds(int64_t C, int64_t L) {
+    const int l = (int)(L < 4096 ? L : 4096);
+    switch (C) {
+        case 512: return DecodeLds<8, 4>::total(l);
+        case 768: return DecodeLds<12, 4>::total(l);
+        case 1024: return DecodeLds<16, 4>::total(l);
+        case 1536: return DecodeLds<24, 4>::total(l);
+        case 2048: return DecodeLds<32, 4>::total(l);
+        case 2560: return DecodeLds<40, 8, true>::total(l);
+        case 4096: return DecodeLds<64, 4>::total(l);
+        case 5120: return DecodeLds<80, 8>::total(l);
+        default: return 0;
+    }
+}
+
 bool decode_supported(int64_t L, int64_t C, int64_t F, int64_t V) {
     if (L <= 0 || V <= 0 || F != 4 * C) return false;
     // one 16-column tile per workgroup, all workgroups resident: C/16 <= 256 CUs
-    if (!(C == 1024 || C == 2048 || C == 2560 || C == 4096 || C == 5120)) return false;
-    // the column sums of a workgroup's head tiles are staged by its front threads into half an owner record
+    if (decode_lds(C, L) == 0) return false;
+    // the column sums of a workgroup's head tiles are staged in LDS by its front threads
+    const int nb = (int)(C / 64);
     const int64_t NWG = decode_workgroups(C), head_rounds = ((V + 15) / 16 + NWG - 1) / NWG, front_threads = (C == 2560 || C == 5120) ? 512 : 256;
-    return head_rounds * 16 <= kHeadCsPerThread * front_threads && head_rounds * 16 * (int64_t)sizeof(int) <= kOrSlots * 8;
+    return head_rounds * 16 <= head_cs_per_thread(nb) * front_threads &&
+           head_rounds * 16 * (int64_t)sizeof(int) <= (head_cs_lds_bytes(nb) ? head_cs_lds_bytes(nb) : kOrSlots * 8) &&
+           decode_lds(C, L) <= 160 * 1024;
 }
 
+// Widths whose generation loop samples on the device.  The others (512, 768, 1536) run their token steps here too, but
+// their texts are drawn on the host from torch's generator, and a program that seeds it keeps its texts.
+bool decode_samples(int64_t C) { return C == 1024 || C == 2048 || C == 2560 || C == 4096 || C == 5120; }
+
 int64_t decode_workgroups(int64_t C) { return C > 4096 ? C / 32 : C / 16; }
-int64_t decode_helper_workgroups(int64_t C) { return C == 2560 ? HelperShape<5>::NH : 0; }
+int64_t decode_helper_workgroups(int64_t C) { return C == 2560 ? HelperShape<40>::NH : 0; }
 
 unsigned decode_epochs_per_token(int64_t L) { return (unsigned)(4 * L + 1); }
 
@@ -1521,7 +1559,7 @@ BlockPlan plan_block(int64_t L, int64_t C, int64_t F, int64_t V) {
     p.cs = take(((size_t)L * p.cs_layer_ints + (size_t)round_up(V, 16)) * sizeof(int));
     p.ownrec = take((size_t)L * G * kOrSlots * sizeof(u64));
     p.jt = take(G * (size_t)(L + 1) * 16 * sizeof(u64));
-    p.scp = take((size_t)L * (C / 512) * sizeof(DScal));
+    p.scp = take((size_t)L * prep_parts((int)C) * sizeof(DScal));
     p.amax = take((size_t)G * (sizeof(double) + sizeof(int)));
     p.abort = take(256);
     p.total = off;
@@ -1628,11 +1666,11 @@ int decode_clear_exchange(hipStream_t st, const DModel &m, const DecodeBuffers &
 
 constexpr int kMaxDevices = 64;
 
-template <int KW, int FW>
+template <int NB, int FW>
 static int launch_one(hipStream_t st, const DArgs &args, bool with_prep) {
-    constexpr bool HELP = HelperShape<KW>::NH > 0;
+    constexpr bool HELP = HelperShape<NB>::NH > 0;
     const bool trace = args.b.trace != nullptr;
-    const int lds = DecodeLds<KW, FW, HELP>::total(args.m.L, trace);
+    const int lds = DecodeLds<NB, FW, HELP>::total(args.m.L, trace);
     if (lds > 160 * 1024) return set_error(RWKV_ERR_SIZE, "decode kernel: %d layers need %d bytes of LDS", args.m.L, lds);
     // the dynamic LDS limit is a per-device attribute of the function; it only ever grows
     static std::mutex mu;
@@ -1643,34 +1681,37 @@ static int launch_one(hipStream_t st, const DArgs &args, bool with_prep) {
     {
         std::lock_guard<std::mutex> lock(mu);
         if (configured[dev] < lds) {
-            RWKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_kernel<KW, FW, false, HELP>),
+            RWKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_kernel<NB, FW, false, HELP>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-            RWKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_kernel<KW, FW, true, HELP>),
+            RWKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_kernel<NB, FW, true, HELP>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds));
             configured[dev] = lds;
         }
     }
     if (with_prep) {
-        hipLaunchKernelGGL(prep_kernel, dim3((unsigned)(args.m.L * (args.m.C / kPrepThreads) + 1)), dim3(kPrepThreads), 0, st, args);
+        hipLaunchKernelGGL(prep_kernel, dim3((unsigned)(args.m.L * prep_parts(args.m.C) + 1)), dim3(kPrepThreads), 0, st, args);
         RWKV_CHECK_LAUNCH("prep_kernel");
     }
     // owner workgroups first, then the helpers: every one of them is resident at once (one per compute unit)
-    const dim3 grid((unsigned)(args.m.NWG + HelperShape<KW>::NH));
+    const dim3 grid((unsigned)(args.m.NWG + HelperShape<NB>::NH));
     if (trace)
-        hipLaunchKernelGGL((decode_kernel<KW, FW, true, HELP>), grid, dim3((FW + kBW) * 64), lds, st, args);
+        hipLaunchKernelGGL((decode_kernel<NB, FW, true, HELP>), grid, dim3((FW + back_waves(NB)) * 64), lds, st, args);
     else
-        hipLaunchKernelGGL((decode_kernel<KW, FW, false, HELP>), grid, dim3((FW + kBW) * 64), lds, st, args);
+        hipLaunchKernelGGL((decode_kernel<NB, FW, false, HELP>), grid, dim3((FW + back_waves(NB)) * 64), lds, st, args);
     RWKV_CHECK_LAUNCH("decode_kernel");
     return RWKV_OK;
 }
 
 static int launch_step(hipStream_t st, const DArgs &args, bool with_prep) {
     switch (args.m.C) {
-        case 1024: return launch_one<2, 4>(st, args, with_prep);
-        case 2048: return launch_one<4, 4>(st, args, with_prep);
-        case 2560: return launch_one<5, 8>(st, args, with_prep);
-        case 4096: return launch_one<8, 4>(st, args, with_prep);
-        case 5120: return launch_one<10, 8>(st, args, with_prep);
+        case 512: return launch_one<8, 4>(st, args, with_prep);
+        case 768: return launch_one<12, 4>(st, args, with_prep);
+        case 1024: return launch_one<16, 4>(st, args, with_prep);
+        case 1536: return launch_one<24, 4>(st, args, with_prep);
+        case 2048: return launch_one<32, 4>(st, args, with_prep);
+        case 2560: return launch_one<40, 8>(st, args, with_prep);
+        case 4096: return launch_one<64, 4>(st, args, with_prep);
+        case 5120: return launch_one<80, 8>(st, args, with_prep);
         default: return set_error(RWKV_ERR_SIZE, "decode kernel: n_embd %d not supported", args.m.C);
     }
 }
@@ -1690,7 +1731,7 @@ int decode_launch_bracketed(hipStream_t st, const DModel &m, const DecodeBuffers
     DArgs args;
     args.m = m; args.b = b; args.epoch0 = epoch0; args.token = token; args.state = state; args.logits = logits;
     args.stop = nullptr; args.spin_limit = kSpinLimit;
-    hipLaunchKernelGGL(prep_kernel, dim3((unsigned)(m.L * (m.C / kPrepThreads) + 1)), dim3(kPrepThreads), 0, st, args);
+    hipLaunchKernelGGL(prep_kernel, dim3((unsigned)(m.L * prep_parts(m.C) + 1)), dim3(kPrepThreads), 0, st, args);
     RWKV_CHECK_LAUNCH("prep_kernel");
     RWKV_CHECK_HIP(hipEventRecord(before, st));
     const int rc = launch_step(st, args, false);
@@ -1744,7 +1785,7 @@ int decode_launch_greedy(hipStream_t st, const DModel &m, const DecodeBuffers &b
         // argmax -> tokens[i + 1], and the preparation of step i + 1 (harmless after the last step:
         // the next forward call prepares again under the same epoch)
         args.epoch0 += ept;
-        hipLaunchKernelGGL(next_token_kernel, dim3((unsigned)(m.L * (m.C / kPrepThreads) + 1)),
+        hipLaunchKernelGGL(next_token_kernel, dim3((unsigned)(m.L * prep_parts(m.C) + 1)),
                            dim3(kPrepThreads), 0, st, args, tokens + i + 1);
         RWKV_CHECK_LAUNCH("next_token_kernel");
     }

@@ -744,7 +744,7 @@ void rwkv_model_destroy(rwkv_model *m) {
     delete m;
 }
 
-int rwkv_model_has_fused_step(const rwkv_model *m) { return (m && m->fused) ? 1 : 0; }
+int rwkv_model_has_fused_step(const rwkv_model *m) { return (m && m->fused && decode_samples(m->dm.C)) ? 1 : 0; }
 
 int rwkv_model_trace_workgroups(const rwkv_model *m) {
     if (!m || !m->fused) return 0;
@@ -929,9 +929,9 @@ int rwkv_model_decode_sample(rwkv_model *m, rwkv_stream_t stream, int64_t *token
     RWKV_CHECK_ARG(stop_flag && n_done, "rwkv_model_decode_sample: stop_flag and n_done must point to device words");
     RWKV_CHECK_ARG(n_stop >= 0 && (n_stop == 0 || stop_tokens), "rwkv_model_decode_sample: stop list");
     RWKV_CHECK_ARG(greedy || (temp > 0.f && tau >= 0.f), "rwkv_model_decode_sample: temp must be positive, tau non-negative");
-    if (!m->fused)
-        return set_error(RWKV_ERR_SIZE, "rwkv_model_decode_sample: this shape does not run the persistent single-token "
-                                        "kernel; sample on the host from rwkv_model_forward's logits");
+    if (!rwkv_model_has_fused_step(m))
+        return set_error(RWKV_ERR_SIZE, "rwkv_model_decode_sample: this shape does not sample on the device; "
+                                        "sample on the host from rwkv_model_forward's logits");
     if ((rc = fused_epochs(m, (hipStream_t)stream, n))) return rc;
     SampleArgs sa{};
     sa.greedy = greedy ? 1 : 0; sa.temp = temp; sa.tau = tau; sa.end_adj = end_adj; sa.seed = seed; sa.counter = 0;

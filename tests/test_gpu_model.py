@@ -273,6 +273,40 @@ def test_fused_kernel_layernorm_with_large_mean(kind):
     _state_close(sp, se, tol=STATE_TOL)
 
 
+# the narrow widths: four back wavefronts at 512 and 768, a layer of part widths in the per-token preparation at 768;
+# vocabularies of a ragged last head tile, of many head rounds per workgroup, and of fewer tiles than workgroups
+@pytest.mark.parametrize("C,L,V", [(512, 3, 1999), (768, 2, 30011), (768, 3, 333), (1536, 2, 3001)])
+def test_narrow_widths_run_the_persistent_kernel(C, L, V):
+    """Token steps at 512, 768 and 1536 channels against exact accumulation (bounds as for the other widths), bit-identical
+    replay, the greedy loop equal to host argmax; sampling stays with the caller at these widths."""
+    from rwkvstic_amd import _native as N
+    from rwkvstic_amd.model import HipRWKV
+    sd = synth.make_state_dict(L, C, 4 * C, V, seed=C + L, ln="random")
+    exact, hip = O.OracleModel(sd, matmul_dtype=torch.float64), HipRWKV(sd)
+    assert N.lib().rwkv_model_trace_workgroups(hip._handle) == C // 16 and not hip.fused_step
+    toks = synth.random_tokens(5, V=V, seed=6).tolist()
+    se, sg = exact.emptyState.clone(), hip.emptyState.clone()
+    for t in toks:
+        le, se = exact.forward([t], se)
+        lg, sg = hip.forward([t], sg)
+        hip.check()
+        assert (lg.cpu() - le).abs().max() < 2e-5 and int(lg.argmax()) == int(le.argmax())
+    _state_close(sg, se, tol=STATE_TOL)
+    s2 = hip.emptyState.clone()
+    for t in toks:
+        l2, s2 = hip.forward([t], s2)
+    assert torch.equal(l2, lg) and torch.equal(s2, sg)
+    got, lo, sd_ = hip.decode_greedy(toks[0], 6, sg.clone())
+    t, want = toks[0], []
+    for _ in range(6):
+        l2, s2 = hip.forward([t], s2)
+        t = int(l2.argmax()); want.append(t)
+    hip.check()
+    assert got.tolist() == want and torch.equal(lo, l2) and torch.equal(sd_, s2)
+    with pytest.raises(RuntimeError):
+        hip.decode_sample(1, 2, sg.clone())
+
+
 def test_fused_greedy_device_loop_matches_host_loop():
     """rwkv_model_decode_greedy on the persistent kernel: argmax and the preparation of the next step run in one
     launch between the token kernels; tokens, logits and state must equal forward() + host argmax, bit for bit
