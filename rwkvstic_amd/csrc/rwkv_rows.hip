@@ -517,7 +517,13 @@ struct GemmArgs {
     // when the contraction is not split the tail of the product is applied here (see rows_finish_kernel)
     int tail, R, N;                 // tail < 0: totals only
     const float *gate;
+    // NT2 > 0: the launch holds two products of different widths (same rows, same contraction, not split): product 1 has
+    // NT2 tiles, N2 columns and tail2, and its workgroups follow product 0's
+    int NT2, N2, tail2;
 };
+// Columns and tail of the product a workgroup works for (kept apart from the arguments: a modified copy of those would
+// live in scratch memory).
+struct GemmCols { int NT, N, tail; };
 
 constexpr int kGemmNT = 8, kGemmWideNT = 10;     // N-tiles per workgroup (two wavefronts side by side)
 constexpr int kWideRing = 4;                     // LDS buffers of the 64 x 160 variant
@@ -542,7 +548,7 @@ __device__ __forceinline__ void dma16(const v4i *g, unsigned lds_byte_offset) {
 // compiler: element by element each of them waited for a round trip).  1024 tokens at width 2560, before and after: k, v, r
 // 75.5 and 71.8 us, ffn key 93.1 and 89.4, att output and ffn receptance 35.1 and 30.2 (median), ffn value 94.8 and 87.7.
 template <int TAIL, int GM, int GN>
-__device__ __forceinline__ void gemm_tail(const GemmArgs &a, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat, int lane) {
+__device__ __forceinline__ void gemm_tail(const GemmArgs &a, int N, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat, int lane) {
     const int g = lane >> 4, n = lane & 15;
     const double *Sv = mat == 0 ? a.S[0] : mat == 1 ? a.S[1] : a.S[2];
     const double *qsv = mat == 0 ? a.qs[0] : mat == 1 ? a.qs[1] : a.qs[2];
@@ -552,7 +558,7 @@ __device__ __forceinline__ void gemm_tail(const GemmArgs &a, const v4i (&acc)[GM
     const bool exact53 = a.KB <= 512;
     double old[2][GN];
     float gate[2][GN];
-    auto at = [&](int i, int j) { return (size_t)min(4 * (mt0 + i) + g, a.R - 1) * a.N + min(16 * (nt0 + j) + n, a.N - 1); };   // (clamped: loads stay in bounds)
+    auto at = [&](int i, int j) { return (size_t)min(4 * (mt0 + i) + g, a.R - 1) * N + min(16 * (nt0 + j) + n, N - 1); };   // (clamped: loads stay in bounds)
     auto fetch = [&](int i) {
 #pragma unroll
         for (int j = 0; j < GN; ++j) {
@@ -576,8 +582,8 @@ __device__ __forceinline__ void gemm_tail(const GemmArgs &a, const v4i (&acc)[GM
             else tot = (double)(((((long long)d.x * 256 + d.y) * 256 + d.z) * 256) + d.w);
             const int col = 16 * (nt0 + j) + n;
             const double y = S * tot + add;
-            const size_t o = (size_t)t * a.N + col;
-            if (live && col < a.N) {
+            const size_t o = (size_t)t * N + col;
+            if (live && col < N) {
                 if (TAIL == ROW_STORE) outv[o] = y;
                 else if (TAIL == ROW_STORE_F32) reinterpret_cast<float *>(outv)[o] = (float)y;
                 else if (TAIL == ROW_RELU2) {                                                       // block.py:97, kept as float32 (see RowTail)
@@ -592,14 +598,14 @@ __device__ __forceinline__ void gemm_tail(const GemmArgs &a, const v4i (&acc)[GM
 }
 
 template <int GM, int GN>
-__device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat,
+__device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, const GemmCols &cols, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat,
                                               int bz, int lane) {
-    switch (a.tail) {
-        case ROW_STORE: return gemm_tail<ROW_STORE, GM, GN>(a, acc, mt0, nt0, mat, lane);
-        case ROW_STORE_F32: return gemm_tail<ROW_STORE_F32, GM, GN>(a, acc, mt0, nt0, mat, lane);
-        case ROW_RELU2: return gemm_tail<ROW_RELU2, GM, GN>(a, acc, mt0, nt0, mat, lane);
-        case ROW_ADD: return gemm_tail<ROW_ADD, GM, GN>(a, acc, mt0, nt0, mat, lane);
-        case ROW_GATE_ADD: return gemm_tail<ROW_GATE_ADD, GM, GN>(a, acc, mt0, nt0, mat, lane);
+    switch (cols.tail) {
+        case ROW_STORE: return gemm_tail<ROW_STORE, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
+        case ROW_STORE_F32: return gemm_tail<ROW_STORE_F32, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
+        case ROW_RELU2: return gemm_tail<ROW_RELU2, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
+        case ROW_ADD: return gemm_tail<ROW_ADD, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
+        case ROW_GATE_ADD: return gemm_tail<ROW_GATE_ADD, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
         default: break;
     }
     const int g = lane >> 4, n = lane & 15;
@@ -609,7 +615,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, const v4i (&acc
         if (mt0 + i >= a.MT) continue;
 #pragma unroll
         for (int j = 0; j < GN; ++j) {
-            if (nt0 + j >= a.NT) continue;
+            if (nt0 + j >= cols.NT) continue;
             const v4i d = acc[i][j];
             totv[(size_t)(4 * (mt0 + i) + g) * a.ldd + 16 * (nt0 + j) + n] = ((((long long)d.x * 256 + d.y) * 256 + d.z) * 256) + d.w;
         }
@@ -724,7 +730,7 @@ __device__ __forceinline__ void gemm8_body(const GemmArgs a) {
 #undef RWKV_GEMM_STEP
 #undef RWKV_GEMM_DMA
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // nothing of this wavefront may still be writing LDS when it leaves
-    gemm_epilogue<kGM, kGN>(a, acc, mt0, nt0, mat, bz, lane);
+    gemm_epilogue<kGM, kGN>(a, GemmCols{a.NT, a.N, a.tail}, acc, mt0, nt0, mat, bz, lane);
 }
 
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) gemm8_kernel(const GemmArgs a) {
@@ -751,11 +757,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int xcd = blockIdx.x % kXcds;
     int item = blockIdx.x / kXcds;
     const int cslot = item % a.per_xcd; item /= a.per_xcd;      // the XCDs share out the column blocks
-    const int bx = xcd + kXcds * cslot;
+    int bx = xcd + kXcds * cslot;
     int bz = item;
     if (bx >= a.gx || bz >= a.gz) return;
-    const int mat = bz / a.split;
+    int mat = bz / a.split;
     bz -= mat * a.split;
+    GemmCols cols = {a.NT, a.N, a.tail};
+    if (a.NT2 > 0) {                                    // two products side by side: gx counts the column blocks of both
+        const int gx0 = (a.NT + kSkinnyNT - 1) / kSkinnyNT;
+        if (bx >= gx0) { bx -= gx0; mat = 1; cols = GemmCols{a.NT2, a.N2, a.tail2}; }
+    }
     const signed char *dig = mat == 0 ? a.dig[0] : mat == 1 ? a.dig[1] : a.dig[2];
     const uint8_t *w16 = mat == 0 ? a.w16[0] : mat == 1 ? a.w16[1] : a.w16[2];
     const int nt0 = bx * kSkinnyNT + wave * kSkinnyGN;
@@ -774,7 +785,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             src[i] = reinterpret_cast<const v4i *>(dig + ((size_t)mt * a.KB + kb0) * 1024) + lane;
         } else {
             int nt = bx * kSkinnyNT + (f - kSkinnyMT);
-            if (nt >= a.NT) nt = a.NT - 1;
+            if (nt >= cols.NT) nt = cols.NT - 1;
             src[i] = reinterpret_cast<const v4i *>(w16 + ((size_t)nt * a.KB + kb0) * 1024) + lane;
         }
     }
@@ -850,67 +861,95 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #undef RWKV_SKINNY_MOVE
 #undef RWKV_SKINNY_PARK
 #undef RWKV_SKINNY_FETCH
-    gemm_epilogue<kSkinnyMT, kSkinnyGN>(a, acc, 0, nt0, mat, bz, lane);
+    gemm_epilogue<kSkinnyMT, kSkinnyGN>(a, cols, acc, 0, nt0, mat, bz, lane);
 }
 
 // ---------------------------------------------------------------------------
 // The same product for at most 8 rows (MT <= 2 M-tiles: a single token of a shape the persistent kernel does
-// not serve, a small batch): pure weight streaming.  No LDS staging and no barrier in the loop: workgroup =
-// one 16-column tile and one part of the contraction, its 4 wavefronts take every fourth block (together
-// they read the tile's blocks in order) and each keeps 8 blocks of weights in flight on its own, so that a
-// slow load holds up one wavefront, not the workgroup.  The digit fragments (L2-resident) are read by every
-// wavefront itself.  One cross-wavefront sum in LDS at the end, then the common epilogue.
+// not serve, a small batch): pure weight streaming.  No LDS staging and no barrier in the loop: a workgroup has NTW
+// column tiles and the whole contraction, its NW wavefronts take every NW-th block (together they read the tiles'
+// blocks in order) and each keeps U blocks per tile in flight on its own, so that a slow load holds up one wavefront,
+// not the workgroup.  The digit fragments (L2-resident) are read by every wavefront itself, once for its NTW tiles.
+// The wavefronts' sums are added in LDS, each sum by a wavefront of its own that also writes it.
+//
+// Bound: the latency of a few dependent loads per wavefront, then HBM.  So the blocks are spread over as many wavefronts
+// as are resident at once (vec_shape), which needs no split of the contraction and no second launch; wide products take
+// several tiles per wavefront, since for two M-tiles the digits are twice a tile's bytes.  8 rows at 2560 channels (us per
+// launch), 4 wavefronts of one tile with 8 blocks in flight / this: k, v, r 10.1 / 7.3, att output 7.4 / 5.4, ffn key and
+// receptance 12.7 + 6.4 / 10.1, ffn value 15.5 / 13.0, head 43 / 30.5.
 // ---------------------------------------------------------------------------
 constexpr int kVecMT = 2;
 
-// kVecBlocks: weight blocks a wavefront has in flight
-template <int MT, int kVecBlocks>
-__global__ void __launch_bounds__(256) gemv16_kernel(const GemmArgs a) {
-    __shared__ v4i red[4][MT][64];
+template <int MT, int NTW, int NW, int U>
+__global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
+    __shared__ v4i red[NW][MT * NTW][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int item = blockIdx.x;
-    const int nt = item % a.NT; item /= a.NT;
-    const int bz = item % a.split, mat = item / a.split;
+    int item = blockIdx.x, mat, bz = 0, grp;
+    const int groups = (a.NT + NTW - 1) / NTW;
+    GemmCols cols = {a.NT, a.N, a.tail};
+    if (a.NT2 > 0) {                                    // two products of different widths side by side, not split
+        mat = item >= groups ? 1 : 0;
+        grp = item - mat * groups;
+        if (mat) cols = GemmCols{a.NT2, a.N2, a.tail2};
+    } else {
+        grp = item % groups; item /= groups;
+        bz = item % a.split; mat = item / a.split;
+    }
+    const int nt0 = grp * NTW;
     const signed char *dig = mat == 0 ? a.dig[0] : mat == 1 ? a.dig[1] : a.dig[2];
     const uint8_t *w16 = mat == 0 ? a.w16[0] : mat == 1 ? a.w16[1] : a.w16[2];
     const int kb0 = bz * a.kb_per_split;
     int kb1 = kb0 + a.kb_per_split;
     if (kb1 > a.KB) kb1 = a.KB;
-    const v4i *bsrc = reinterpret_cast<const v4i *>(w16 + (size_t)nt * a.KB * 1024) + lane;
-    const v4i *asrc[MT];
+    const v4i *bsrc[NTW], *asrc[MT];
+#pragma unroll
+    for (int j = 0; j < NTW; ++j)                       // (clamped: loads stay in bounds, results are dropped)
+        bsrc[j] = reinterpret_cast<const v4i *>(w16 + (size_t)(nt0 + j < cols.NT ? nt0 + j : cols.NT - 1) * a.KB * 1024) + lane;
 #pragma unroll
     for (int m = 0; m < MT; ++m)
         asrc[m] = reinterpret_cast<const v4i *>(dig + (size_t)(m < a.MT ? m : a.MT - 1) * a.KB * 1024) + lane;
-    v4i acc[MT][1];
+    v4i acc[MT][NTW];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m][0] = v4i{0, 0, 0, 0};
-    for (int k = kb0 + wave; k < kb1; k += 4 * kVecBlocks) {
-        v4i B[kVecBlocks], A[MT][kVecBlocks];
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int i = 0; i < kVecBlocks; ++i) {
-            const size_t o = (size_t)min(k + 4 * i, a.KB - 1) * 64;       // past the end: a block nobody multiplies
-            B[i] = bsrc[o];
+        for (int j = 0; j < NTW; ++j) acc[m][j] = v4i{0, 0, 0, 0};
+    for (int k = kb0 + wave; k < kb1; k += NW * U) {
+        v4i B[NTW][U], A[MT][U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const size_t o = (size_t)min(k + NW * i, a.KB - 1) * 64;      // past the end: a block nobody multiplies
+#pragma unroll
+            for (int j = 0; j < NTW; ++j) B[j][i] = bsrc[j][o];
 #pragma unroll
             for (int m = 0; m < MT; ++m) A[m][i] = asrc[m][o];
         }
 #pragma unroll
-        for (int i = 0; i < kVecBlocks; ++i) {
-            if (k + 4 * i < kb1) {          // uniform for the wavefront
+        for (int i = 0; i < U; ++i) {
+            if (k + NW * i < kb1) {         // uniform for the wavefront
 #pragma unroll
                 for (int m = 0; m < MT; ++m)
-                    acc[m][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[m][i], B[i], acc[m][0], 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < NTW; ++j)
+                        acc[m][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[m][i], B[j][i], acc[m][j], 0, 0, 0);
             }
         }
     }
-    // digit sums of at most a few hundred blocks: far inside int32
+    // digit sums of at most a thousand blocks or so (plan_products splits longer contractions): inside int32
 #pragma unroll
-    for (int m = 0; m < MT; ++m) red[wave][m][lane] = acc[m][0];
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) red[wave][m * NTW + j][lane] = acc[m][j];
     __syncthreads();
-    if (wave != 0) return;
+    for (int i = wave; i < MT * NTW; i += NW) {
+        const int m = i / NTW, nt = nt0 + i % NTW;
+        if (nt >= cols.NT) continue;           // uniform for the wavefront
+        v4i sum[1][1];
+        sum[0][0] = red[0][i][lane];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m][0] = red[0][m][lane] + red[1][m][lane] + red[2][m][lane] + red[3][m][lane];
-    gemm_epilogue<MT, 1>(a, acc, 0, nt, mat, bz, lane);
+        for (int w = 1; w < NW; ++w) sum[0][0] += red[w][i][lane];
+        gemm_epilogue<1, 1>(a, cols, sum, m, nt, mat, bz, lane);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1265,13 +1304,13 @@ __global__ void __launch_bounds__(1024) mv16_kernel(const Mv16Args a) {
 // host side
 // ---------------------------------------------------------------------------
 size_t rows_dig_bytes(int64_t R, int64_t K) { return (size_t)(ceil_div(R, 4) * (K / 64) * 1024); }
-constexpr int kVecFillWgs = 128;        // products of at most 8 rows: the contraction is split until there are this many workgroups (batch step of 8 / 4 sequences, 3B shape: 3.06 / 2.64 ms at 128, 3.19 / 2.81 at 256, 3.30 / 2.94 at 512)
 constexpr int kMaxSplit = 8;
 constexpr int kGemmWideNum = 10, kGemmWideDen = 9;     // the 64 x 160 variant is taken when its cost is below 9/10 of the 64 x 128 variant's
 // ... except a contraction of 200 blocks and more, which splits in two while the grid is below the device (14B shape,
 // 256-token chunks: the [256 x 20480] x [20480 x 5120] product; 14,080 against 13,190 tokens/s)
 constexpr int kGemmLongFillWgs = 256, kGemmLongBlocks = 200;
 constexpr int kSkinnyFillWgs = 128;     // 9..32 rows (weight streaming): the contraction is split until the grid has this many workgroups (batch-32 step: 8.07 ms at 128, 8.73 at 256, 9.17 at 64 for the 14B shape; 4.06 / 4.13 / 4.11 ms for the 3B shape)
+constexpr int kSkinnyPairWgs = 64;      // ffn key and receptance of 9..32 rows in one launch from so many workgroups on
 constexpr int kGemmFillWgs = 96;         // larger products: split until the grid has this many workgroups.  A split costs a second launch and a round trip of the integer totals through memory, so it only pays for grids far below the device (3B shape, tokens/s in chunks of 64 / 128 / 256 / 512 tokens: 13,180 / 23,640 / 37,610 / 52,070 at 96; 12,480 / 21,280 / 34,650 / 49,380 at 256; 12,540 / 21,470 / 31,520 / 51,160 at 64)
 
 // Which kernel serves n products of MT row tiles x NT column tiles over KB contraction blocks, its grid and
@@ -1283,12 +1322,9 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n) {
     ProductPlan p;
     p.split = 1;
     if (MT <= kVecMT) {
-        // a handful of rows: one 16-column tile per workgroup; only products with fewer tiles than compute
-        // units split the contraction (their integer slices are added by the tail kernel)
+        // a handful of rows: whole contractions, as long as a digit's sum of them stays inside int32 (2^20 per block)
         p.kind = PLAN_VEC; p.gx = (int)NT; p.gy = 1;
-        while (NT * n * p.split < kVecFillWgs && KB / (p.split * 2) >= 8 && p.split < kMaxSplit) p.split *= 2;
-        // a very long contraction: one split (the 14B shape's ffn value product, 8 sequences: 6.97 against 7.26 ms per step)
-        if (p.split == 1 && NT * n < 512 && KB >= kGemmLongBlocks) p.split = 2;
+        while (ceil_div(KB, p.split) > 1024 && p.split < kMaxSplit) p.split *= 2;
         return p;
     }
     p.gy = (int)ceil_div(MT, 16);
@@ -1309,6 +1345,34 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n) {
     if (p.kind != PLAN_SKINNY && p.split == 1 && (int64_t)p.gx * p.gy * n < kGemmLongFillWgs && KB >= kGemmLongBlocks) p.split = 2;
     return p;
 }
+// Shape of the few-row kernel for a launch of so many column tiles: tiles per workgroup, wavefronts per workgroup, blocks
+// in flight per wavefront and tile.  All workgroups resident at once, 2000 to 4000 wavefronts where the tiles allow it; one
+// tile per workgroup while that fills the device, more where the digits every wavefront reads would outweigh the weights.
+struct VecShape { int ntw, nw, u; };
+static VecShape vec_shape(int64_t tiles, int64_t KB) {
+    if (tiles > 1280) return VecShape{4, 8, 3};
+    if (tiles > 320) return tiles <= 512 ? VecShape{2, 16, 3} : VecShape{2, 8, 5};
+    if (tiles > 256) return VecShape{1, 8, 5};
+    return KB <= 48 ? VecShape{1, 16, 3} : VecShape{1, 16, 5};
+}
+static void launch_vec(hipStream_t st, const GemmArgs &g) {
+    const int64_t tiles = g.NT2 > 0 ? (int64_t)g.NT + g.NT2 : (int64_t)g.NT * g.gz;
+    const VecShape v = vec_shape(tiles, g.KB);
+    const dim3 grid((unsigned)(g.NT2 > 0 ? ceil_div(g.NT, v.ntw) + ceil_div(g.NT2, v.ntw) : ceil_div(g.NT, v.ntw) * g.gz)), block((unsigned)(64 * v.nw));
+#define RWKV_VEC(NTW, NW, U)                                                                          \
+    if (v.ntw == NTW && v.nw == NW && v.u == U) {                                                     \
+        if (g.MT == 1) hipLaunchKernelGGL((gemv16_kernel<1, NTW, NW, U>), grid, block, 0, st, g);     \
+        else hipLaunchKernelGGL((gemv16_kernel<2, NTW, NW, U>), grid, block, 0, st, g);               \
+    }
+    RWKV_VEC(4, 8, 3)
+    RWKV_VEC(2, 16, 3)
+    RWKV_VEC(2, 8, 5)
+    RWKV_VEC(1, 8, 5)
+    RWKV_VEC(1, 16, 3)
+    RWKV_VEC(1, 16, 5)
+#undef RWKV_VEC
+}
+
 // Upper bound of the splits plan_products chooses for R rows and N columns, whatever the contraction length and
 // the number of products in the launch: a longer contraction only lifts the limit on the split, so the
 // plan for an unbounded one bounds every real one.
@@ -1454,11 +1518,10 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     g.slice = (size_t)g.MT * 4 * g.ldd;
     g.gz = split * n;
     g.tail = split > 1 ? -1 : op;
+    g.NT2 = g.N2 = g.tail2 = 0;
     if (pl.kind == PLAN_VEC) {
         g.gx = g.NT; g.gy = 1; g.by_rows = 0; g.per_xcd = 0;
-        const dim3 grid((unsigned)(g.NT * g.gz));
-        if (g.MT == 1) hipLaunchKernelGGL((gemv16_kernel<1, 8>), grid, dim3(256), 0, st, g);
-        else hipLaunchKernelGGL((gemv16_kernel<2, 8>), grid, dim3(256), 0, st, g);
+        launch_vec(st, g);
         RWKV_CHECK_LAUNCH("gemv16_kernel");
     } else {
         g.gx = pl.gx; g.gy = gy; g.by_rows = gy >= kXcds;
@@ -1487,6 +1550,36 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
         default: hipLaunchKernelGGL(rows_finish_kernel<ROW_GATE_ADD>, fg, fb, 0, st, f); break;
     }
     RWKV_CHECK_LAUNCH("rows_finish_kernel");
+    return RWKV_OK;
+}
+
+// Few rows: both in one launch, whole contractions (the receptance's column blocks find room beside the key's; apart they
+// were up to four launches, two of them only adding slices).  With gemv16_kernel's shapes: 8 sequences at 3B 2.96 -> 2.40 ms
+// a step, 32 at 14B 7.38 -> 6.66 ms (its two launches and the receptance's sum of slices: 31.8 + 13.5 + 4.6 us, one launch 37.5).
+int rows_ffn_key_receptance(hipStream_t st, const RowsProduct &k, const RowsProduct &r, long long *tot, int64_t R, int64_t C, int64_t F) {
+    GemmArgs g;
+    const RowsProduct *p[2] = {&k, &r};
+    for (int m = 0; m < kRowsMaxProducts; ++m) {
+        const RowsProduct &q = *p[m == 1];
+        g.dig[m] = q.a.dig; g.w16[m] = q.w16; g.S[m] = q.a.S; g.qs[m] = q.a.qs; g.zp[m] = q.a.zp; g.out[m] = q.out;
+    }
+    g.tot = nullptr; g.slice = 0; g.gate = nullptr;
+    g.MT = (int)ceil_div(R, 4); g.NT = (int)ceil_div(F, 16); g.KB = (int)(C / 64); g.ldd = g.NT * 16;
+    g.kb_per_split = g.KB; g.split = 1; g.gz = 1; g.gy = 1; g.by_rows = 0;
+    g.tail = ROW_RELU2; g.R = (int)R; g.N = (int)F;
+    g.NT2 = (int)ceil_div(C, 16); g.N2 = (int)C; g.tail2 = ROW_STORE_F32;
+    const int gx = (int)(ceil_div(g.NT, kSkinnyNT) + ceil_div(g.NT2, kSkinnyNT));
+    if (C % 64 == 0 && g.MT <= kVecMT && g.KB <= 1024) {
+        g.gx = g.NT; g.per_xcd = 0;
+        launch_vec(st, g);
+    } else if (C % 64 == 0 && g.MT <= kSkinnyMT && gx >= kSkinnyPairWgs) {
+        g.gx = gx; g.per_xcd = (gx + kXcds - 1) / kXcds;
+        hipLaunchKernelGGL(gemm8_skinny_kernel, dim3((unsigned)(kXcds * g.per_xcd)), dim3(256), 0, st, g);
+    } else {
+        const int rc = rows_products(st, 1, &k, tot, R, C, F, ROW_RELU2, nullptr);
+        return rc ? rc : rows_products(st, 1, &r, tot, R, C, C, ROW_STORE_F32, nullptr);
+    }
+    RWKV_CHECK_LAUNCH("ffn key and receptance");
     return RWKV_OK;
 }
 

@@ -481,6 +481,27 @@ def test_gemm8_matches_fp64_dense(ops, T, K, N):
     assert err < 2e-7                                         # float32 rounding of x*range, nothing else
 
 
+# at most 8 rows: both sides of the column tiles at which the kernel changes its shape (256 | 320 | 512 | 1280), of the
+# contraction length at which it does (48 blocks), fewer blocks than wavefronts, one block past a round, a split contraction
+@pytest.mark.parametrize("T,K,N", [(1, 64, 16), (8, 17 * 64, 4096), (8, 17 * 64, 4100), (3, 192, 5120), (5, 41 * 64, 5121), (4, 448, 8192),
+                                   (8, 41 * 64, 8200), (8, 192, 20480), (7, 25 * 64, 20490), (6, 49 * 64, 4096), (8, 81 * 64, 256),
+                                   (2, 1025 * 64, 20)])
+def test_few_row_products_match_fp64_dense(ops, T, K, N):
+    g = torch.Generator().manual_seed(T * 7 + K + N)
+    codes = torch.randint(0, 256, (K, N), generator=g, dtype=torch.uint8)
+    rng, off = torch.rand(K, generator=g) * 1e-3, torch.randn(K, generator=g, dtype=torch.float64) * 0.01
+    x = torch.randn(T, K, generator=g, dtype=torch.float64)
+    x[0, : K // 2] *= 50.0
+    xr = (x * rng.double()).float().double()                 # what the kernel is given to multiply, rounded once
+    want = (xr @ codes.double()) + (x @ off)[:, None]
+    p16 = ops.pack_m16(codes.cuda())
+    got = ops.gemm8(x.cuda(), p16, rng.cuda(), off.cuda(), K, N).cpu()
+    # fixed point of 30 bits below a row's largest |xr| (half a unit each, codes up to 255), float64 beyond that
+    bound = K * 255 * xr.abs().max(dim=1, keepdim=True).values * 2.0 ** -30 + 1e-12 * (x.abs() @ off.abs())[:, None]
+    print(f"few-row product T={T} K={K} N={N}: max err / bound {((got - want).abs() / bound).max():.2e}", flush=True)
+    assert ((got - want).abs() <= bound).all()
+
+
 def test_gemm8_rows_do_not_depend_on_batching(ops):
     """Integer accumulation: a row's result is bit-identical whether the contraction is split (few rows)
     or not (many rows), and wherever the row sits in its tile."""
