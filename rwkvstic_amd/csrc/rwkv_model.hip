@@ -524,6 +524,7 @@ constexpr int64_t kRowsMin = 4;        // shorter prompts go token by token
 
 struct RowsWs {
     double *x, *kvr, *att, *h, *prev0;
+    double *x2, *sh1, *sh2; // fewer than kRowsDeferMax rows: x after a pending update, the two newest shift rows (see RowsFew)
     RowsOperand q[3];       // quantised left operands: q[0] up to n_ffn wide, q[1], q[2] n_embd wide
     long long *tot;
 };
@@ -544,6 +545,7 @@ size_t rows_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_
     n += round_up((size_t)R * C * 8, 256) * 5;          // x, kvr[3], att
     n += round_up((size_t)R * F * 8, 256);              // h
     n += round_up((size_t)C * 8, 256);                  // prev0
+    n += round_up((size_t)(R < kRowsDeferMax ? R : kRowsDeferMax - 1) * C * 8, 256) * 3;    // x2, sh1, sh2
     n += round_up((size_t)R * 8, 256) * 9;              // S, qs, zp of three operands
     n += round_up(rows_dig_bytes(R, F), 256) + 2 * round_up(rows_dig_bytes(R, C), 256);
     n += round_up(rows_tot_ws_bytes(R, C, n_wide, n_head), 256);
@@ -559,6 +561,7 @@ RowsWs rows_carve(void *ws, int64_t R, int64_t C, int64_t F, int64_t n_wide, int
     w.att = (double *)take((size_t)R * C * 8);
     w.h = (double *)take((size_t)R * F * 8);
     w.prev0 = (double *)take((size_t)C * 8);
+    for (double **b : {&w.x2, &w.sh1, &w.sh2}) *b = (double *)take((size_t)(R < kRowsDeferMax ? R : kRowsDeferMax - 1) * C * 8);
     for (int i = 0; i < 3; ++i) {
         w.q[i].S = (double *)take((size_t)R * 8);
         w.q[i].qs = (double *)take((size_t)R * 8);
@@ -581,10 +584,11 @@ bool rows_supported(const rwkv_model *m) {
 
 // R rows through every layer.  sequence: rows are consecutive tokens of one sequence whose state is
 // `state` [L,5,C]; otherwise row b is one token of sequence b with state at state + b * state_stride.
-// pending (batch rows only, or null): the last layer's ffn value product may come back unfinished, for the
-// LayerNorm kernel in front of the head to finish.
+// tail: what is left to the LayerNorm kernel in front of the head: its input x, the last layer's ffn value product where it
+// is still pending (batch rows), and the last shift rows to be committed.
+struct RowsTailWork { const double *x; RowsFew few; };
 int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R, bool sequence, double *state,
-                int64_t state_stride, const RowsWs &w, RowsDeferred *pending = nullptr) {
+                int64_t state_stride, const RowsWs &w, RowsTailWork &tail) {
     const rwkv_model_desc &d = m->d;
     const int C = (int)d.n_embd, F = (int)d.n_ffn, V = (int)d.n_vocab;
     const size_t RC = (size_t)R * C;
@@ -593,8 +597,18 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     // row-wise kernel (k, v, r -> WKV; the two residual updates -> the next LayerNorm) leave the sum of their slices
     // to that kernel instead of a launch of their own.
     const bool defer = !sequence && R < kRowsDeferMax;
-    RowsDeferred dk[3], dx;
-    dx.tot = nullptr;
+    RowsDeferred dk[3];
+    // Few rows whose shift rows are read straight from the state: the LayerNorm kernels leave the new ones aside, and each
+    // commits what the one before it left.
+    const bool aside = R < kRowsDeferMax && (!sequence || R == 1);
+    RowsFew few{};
+    double *x = w.x;
+    // (after a launch of the LayerNorm kernel: x is where a pending update went, its shift rows wait in `left` for `home`)
+    auto advance = [&](const double *left, double *home) {
+        if (few.add.tot) { x = few.x_out; few.add.tot = nullptr; }
+        few.commit_src = aside ? left : nullptr; few.commit_dst = home;
+    };
+    auto prepare = [&](double *left) { few.x_out = x == w.x ? w.x2 : w.x; few.shift_out = aside ? left : nullptr; };
     for (int64_t l = 0; l < d.n_layer; ++l) {
         const rwkv_layer_desc &L = m->layers[l];
         double *sl = state + (size_t)l * 5 * C;
@@ -605,8 +619,10 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
         const rwkv_qmat *kvr[3] = {&L.att_k, &L.att_v, &L.att_r};
         const float *rg[3] = {kvr[0]->range, kvr[1]->range, kvr[2]->range};
         const double *of[3] = {kvr[0]->offset, kvr[1]->offset, kvr[2]->offset};
-        RWKV_TRY(rows_ln_mix_quant(st, 3, R, C, sequence, w.x, L.ln1_w, L.ln1_b, L.att_mix, copy_prev ? w.prev0 : sl, sl,
-                                   state_stride, rg, of, w.q, &dx));
+        prepare(w.sh1);
+        RWKV_TRY(rows_ln_mix_quant(st, 3, R, C, sequence, x, L.ln1_w, L.ln1_b, L.att_mix, copy_prev ? w.prev0 : sl, sl,
+                                   state_stride, rg, of, w.q, &few));
+        advance(w.sh1, sl);
         // k, v, r (and the ffn receptance below) are kept as float32 arrays in the kvr slab
         float *kvr32 = reinterpret_cast<float *>(w.kvr);
         RowsProduct pk[3];
@@ -615,24 +631,25 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
         RWKV_TRY(rows_wkv(st, R, C, sequence, kvr32, kvr32 + RC, kvr32 + 2 * RC, L.time_decay, L.time_first,
                           sl + 2 * (size_t)C, state_stride, reinterpret_cast<float *>(w.att), defer ? dk : nullptr));
         RWKV_TRY(rows_quant(st, R, C, w.att, true, L.att_o.range, L.att_o.offset, w.q[0], (double *)w.tot));    // att and h: float32 arrays
-        const RowsProduct po = {w.q[0], L.att_o.packed16, w.x};
-        RWKV_TRY(rows_products(st, 1, &po, w.tot, R, C, C, ROW_ADD, nullptr, defer ? &dx : nullptr));
+        const RowsProduct po = {w.q[0], L.att_o.packed16, x};
+        RWKV_TRY(rows_products(st, 1, &po, w.tot, R, C, C, ROW_ADD, nullptr, defer ? &few.add : nullptr));
         // ChannelMix (block.py:82-100)
         if (copy_prev) RWKV_CHECK_HIP(hipMemcpyAsync(w.prev0, sl + C, (size_t)C * 8, hipMemcpyDeviceToDevice, st));
         const float *rg2[2] = {L.ffn_k.range, L.ffn_r.range};
         const double *of2[2] = {L.ffn_k.offset, L.ffn_r.offset};
-        RWKV_TRY(rows_ln_mix_quant(st, 2, R, C, sequence, w.x, L.ln2_w, L.ln2_b, L.ffn_mix, copy_prev ? w.prev0 : sl + C,
-                                   sl + C, state_stride, rg2, of2, w.q + 1, &dx));
-        dx.tot = nullptr;
+        prepare(w.sh2);
+        RWKV_TRY(rows_ln_mix_quant(st, 2, R, C, sequence, x, L.ln2_w, L.ln2_b, L.ffn_mix, copy_prev ? w.prev0 : sl + C,
+                                   sl + C, state_stride, rg2, of2, w.q + 1, &few));
+        advance(w.sh2, sl + C);
         const RowsProduct pfk = {w.q[1], L.ffn_k.packed16, w.h}, pfr = {w.q[2], L.ffn_r.packed16, w.kvr};
         RWKV_TRY(rows_ffn_key_receptance(st, pfk, pfr, w.tot, R, C, F));
         RWKV_TRY(rows_quant(st, R, F, w.h, true, L.ffn_v.range, L.ffn_v.offset, w.q[0], (double *)w.tot));
-        const RowsProduct pfv = {w.q[0], L.ffn_v.packed16, w.x};
+        const RowsProduct pfv = {w.q[0], L.ffn_v.packed16, x};
         // (the ffn receptance stays in the kvr slab and the totals untouched until the next LayerNorm kernel has run)
-        const bool hand_on = defer && (l + 1 < d.n_layer || pending);
-        RWKV_TRY(rows_products(st, 1, &pfv, w.tot, R, F, C, ROW_GATE_ADD, kvr32, hand_on ? &dx : nullptr));
+        RWKV_TRY(rows_products(st, 1, &pfv, w.tot, R, F, C, ROW_GATE_ADD, kvr32, defer ? &few.add : nullptr));
     }
-    if (pending) *pending = dx;
+    few.x_out = few.shift_out = nullptr;
+    tail = RowsTailWork{x, few};
     return RWKV_OK;
 }
 
@@ -651,15 +668,16 @@ int rows_sequence(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t 
     const RowsWs rw = rows_carve(rows_base, Rmax, C, F, F, m->d.n_vocab);
     for (int64_t t0 = 0; t0 < T; t0 += kRowsChunk) {
         const int64_t R = T - t0 < kRowsChunk ? T - t0 : kRowsChunk;
-        int rc = rows_layers(m, st, tokens + t0, R, true, state, 0, rw);
+        RowsTailWork tail;
+        int rc = rows_layers(m, st, tokens + t0, R, true, state, 0, rw, tail);
         if (rc) return rc;
         if (t0 + R == T) {
             // ln_out and the head on the last row (opt.py:72-74), as a one-row product with integer sums
             const rwkv_model_desc &d = m->d;
             const float *rg[1] = {d.head.range};
             const double *of[1] = {d.head.offset};
-            rc = rows_ln_mix_quant(st, 0, 1, (int)C, false, rw.x + (size_t)(R - 1) * C, d.ln_out_w, d.ln_out_b, nullptr,
-                                   nullptr, nullptr, 0, rg, of, rw.q);
+            rc = rows_ln_mix_quant(st, 0, 1, (int)C, false, tail.x + (size_t)(R - 1) * C, d.ln_out_w, d.ln_out_b, nullptr,
+                                   nullptr, nullptr, 0, rg, of, rw.q, &tail.few);
             if (rc) return rc;
             const RowsProduct ph = {rw.q[0], d.head.packed16, logits};
             rc = rows_products(st, 1, &ph, rw.tot, 1, C, d.n_vocab, ROW_STORE, nullptr);
@@ -863,13 +881,13 @@ int rwkv_model_forward_batch(rwkv_model *m, rwkv_stream_t stream, const int64_t 
     const rwkv_model_desc &d = m->d;
     const int64_t C = d.n_embd, F = d.n_ffn, V = d.n_vocab;
     const RowsWs rw = rows_carve(workspace, batch, C, F, F > V ? F : V, 0);
-    RowsDeferred pending;
-    int rc = rows_layers(m, st, tokens, batch, false, states, d.n_layer * 5 * C, rw, &pending);
+    RowsTailWork tail;
+    int rc = rows_layers(m, st, tokens, batch, false, states, d.n_layer * 5 * C, rw, tail);
     if (rc) return rc;
     const float *rg[1] = {d.head.range};
     const double *of[1] = {d.head.offset};
-    rc = rows_ln_mix_quant(st, 0, batch, (int)C, false, rw.x, d.ln_out_w, d.ln_out_b, nullptr, nullptr, nullptr, 0, rg, of,
-                           rw.q, &pending);
+    rc = rows_ln_mix_quant(st, 0, batch, (int)C, false, tail.x, d.ln_out_w, d.ln_out_b, nullptr, nullptr, nullptr, d.n_layer * 5 * C, rg, of,
+                           rw.q, &tail.few);
     if (rc) return rc;
     const RowsProduct ph = {rw.q[0], d.head.packed16, logits};
     return rows_products(st, 1, &ph, rw.tot, batch, C, V, ROW_STORE, nullptr);

@@ -35,6 +35,15 @@ struct RowsDeferred {
 };
 constexpr int64_t kRowsDeferMax = 128;
 constexpr int kRowsDeferSlices = 4;     // a contraction split further than this is finished by a launch of its own
+// What the LayerNorm kernel of fewer than kRowsDeferMax rows does besides (several workgroups share a row there, and none
+// may overwrite what another reads).
+struct RowsFew {
+    RowsDeferred add;           // a residual update of x still pending (tot null: none); batch rows only
+    double *x_out;              // where the updated x goes: another buffer than x (null: it is not needed)
+    double *shift_out;          // [R, C]: the newest shift rows, instead of the state; needed wherever prev0 is the state itself
+    const double *commit_src;   // [R, C]: shift rows left by the launch before (null: none) ...
+    double *commit_dst;         // ... and their place in the state, row stride prev_stride
+};
 size_t rows_dig_bytes(int64_t R, int64_t K);
 size_t rows_tot_bytes(int64_t R, int64_t N);        // integer totals of ONE product (times the products in a launch)
 size_t rows_quant_scratch_bytes(int64_t R, int64_t K);   // what rows_quant writes into its scratch area (0: unused)
@@ -50,8 +59,7 @@ int rows_embed(hipStream_t st, const int64_t *tokens, int64_t R, int V, int C, c
 int rows_ln_mix_quant(hipStream_t st, int n_mix, int64_t R, int C, bool sequence, const double *x, const double *ln_w,
                       const double *ln_b, const double *mu, const double *prev0, double *shift_dst,
                       int64_t prev_stride, const float *const *range, const double *const *offset,
-                      const RowsOperand *out, const RowsDeferred *add = nullptr /* pending residual update of x: applied
-                      and stored first (x is then written too); batch rows only */);
+                      const RowsOperand *out, const RowsFew *few = nullptr);
 // Rows of float64 values quantised for a matrix with the given per-input-channel range / offset.
 // scratch: rows_quant_scratch_bytes(R, K) bytes (any buffer free until the product starts, e.g. its totals), or null.
 int rows_quant(hipStream_t st, int64_t R, int64_t K, const void *in, bool in_f32, const float *range, const double *offset,

@@ -208,8 +208,11 @@ __device__ __forceinline__ double deferred_value(const RowsDeferred &d, int t, i
 struct LnQuantArgs {
     int C, R, sequence;
     const double *x;            // [R, C]
-    RowsDeferred add;           // batch rows, 512 threads per row: x += this product first, stored to x_rw (tot null: none)
-    double *x_rw;
+    RowsDeferred add;           // batch rows, few-row form: x += this product first, stored to x_out (tot null: none)
+    double *x_out;              // null: nobody reads x again
+    double *shift_out;          // few-row form, [R, C]: the newest xy rows go here instead of to shift_dst (null: sequences, to shift_dst)
+    const double *commit_src;   // few-row form: [R, C] rows an earlier launch left in its shift_out (null: none) ...
+    double *commit_dst;         // ... copied to commit_dst + row * prev_stride
     const double *ln_w, *ln_b;  // [C]
     const double *mu;           // [NM, C]
     const double *prev0;        // sequence: [C]; batch: row t at prev0 + t * prev_stride
@@ -221,7 +224,7 @@ struct LnQuantArgs {
     double *S[3], *qs[3], *zp[3];
 };
 
-constexpr int kLnMaxThreads = 512;      // the LayerNorm kernel runs 512 threads per row for few rows, 256 for many
+constexpr int kLnMaxWidth = 6144;       // widest row the LayerNorm kernels hold in registers
 
 // Sum of N values per thread over the kLW wavefronts of the workgroup (fixed order), broadcast.
 template <int N, int kLW>
@@ -241,6 +244,178 @@ __device__ __forceinline__ void lsum(double (&v)[N], double *red /*[N*kLW]*/) {
         v[i] = s;
     }
     __syncthreads();
+}
+
+// Sum of N values per thread over the nw <= 16 wavefronts of the workgroup (fixed order), broadcast; red[N * 16] is used
+// by no other reduction, so one barrier does.  Every wavefront adds up the wavefronts' sums for itself: each row of 16
+// lanes reads them side by side.
+__device__ __forceinline__ double row16_sum(double v) {
+    v += dpp64<kDppXor1>(v);
+    v += dpp64<kDppXor2>(v);
+    v += dpp64<kDppHalfMirror>(v);
+    return v + dpp64<kDppMirror>(v);
+}
+__device__ __forceinline__ float row16_max(float v) {
+    v = fmaxf(v, dpp32<kDppXor1>(v));
+    v = fmaxf(v, dpp32<kDppXor2>(v));
+    v = fmaxf(v, dpp32<kDppHalfMirror>(v));
+    return fmaxf(v, dpp32<kDppMirror>(v));
+}
+template <int N>
+__device__ __forceinline__ void bsum(double (&v)[N], double *red, int nw) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const double s = wsum(v[i]);
+        if (lane == 0) red[i * 16 + wave] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = row16_sum((lane & 15) < nw ? red[i * 16 + (lane & 15)] : 0.0);
+}
+__device__ __forceinline__ void ld4(double (&v)[4], const double *p) {
+    const double2 a = *reinterpret_cast<const double2 *>(p), b = *reinterpret_cast<const double2 *>(p + 2);
+    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+}
+__device__ __forceinline__ void ld4(float (&v)[4], const float *p) {
+    const float4 a = *reinterpret_cast<const float4 *>(p);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+}
+
+__device__ __forceinline__ void st4(double *p, const double (&v)[4]) {
+    *reinterpret_cast<double2 *>(p) = make_double2(v[0], v[1]);
+    *reinterpret_cast<double2 *>(p + 2) = make_double2(v[2], v[3]);
+}
+
+// The same for fewer than kRowsDeferMax rows, where one row's chain of dependent steps is the whole kernel.  Most of it is
+// instruction fetch: a launch begins with cold instruction caches and runs straight through code it uses once, so the three
+// mixes are not unrolled into one workgroup but go to workgroups of their own (blockIdx.y), which take the row's statistics
+// each for themselves.  As many threads as the row has groups of four channels (above 4096 channels half as many), all
+// loads requested before the first reduction.
+//
+// The workgroups of a row may not write what the others still read.  So the row's new x (a residual update that a split
+// product left pending is applied here) goes to x_out, another buffer than x, and its newest shift row to shift_out; the next
+// launch of this kernel copies that one into the state (commit).
+//
+// 8 rows of 2560 channels, three / two mixes: 8.4 / 8.5 us, 32 rows of 5120 15.8 / 15.0 us (one workgroup of 512 threads for
+// the row and all its mixes: 11.1 / 9.7 and 19.6 / 15.4; the same with every parameter vector requested ahead: no faster).
+template <bool MIX, int NSEG, int MAXT>
+__global__ void __launch_bounds__(MAXT) rows_ln_mix_quant_row_kernel(const LnQuantArgs a) {
+    __shared__ double red0[2 * 16], red1[2 * 16], red2[16], red3[16];
+    __shared__ float redf[16];
+    const int t = blockIdx.x, m = blockIdx.y, C = a.C, tid = threadIdx.x, nt = blockDim.x, nw = nt >> 6, lane = tid & 63;
+    const bool need_prev = MIX && a.sequence && t > 0;
+    const double *xr = a.x + (size_t)t * C;
+    const double *pr = !MIX ? xr : need_prev ? xr - C : a.sequence ? a.prev0 : a.prev0 + (size_t)t * a.prev_stride;
+    const double *mur = MIX ? a.mu + (size_t)m * C : nullptr;
+    const float *range = m == 0 ? a.range[0] : m == 1 ? a.range[1] : a.range[2];
+    const double *offset = m == 0 ? a.offset[0] : m == 1 ? a.offset[1] : a.offset[2];
+    double xv[NSEG][4], pv[NSEG][4], lw[NSEG][4], lb[NSEG][4], mu[NSEG][4], of[NSEG][4];
+    float rg[NSEG][4];
+#pragma unroll
+    for (int g = 0; g < NSEG; ++g) {
+        const int c0 = 4 * (tid + g * nt);
+        if (c0 < C) {
+            ld4(xv[g], xr + c0);
+            if (MIX) ld4(pv[g], pr + c0);
+            ld4(lw[g], a.ln_w + c0);
+            ld4(lb[g], a.ln_b + c0);
+            if (MIX) ld4(mu[g], mur + c0);
+            ld4(rg[g], range + c0);
+            ld4(of[g], offset + c0);
+            if (a.commit_src && m == 0) {
+                double v[4];
+                ld4(v, a.commit_src + (size_t)t * C + c0);
+                st4(a.commit_dst + (size_t)t * a.prev_stride + c0, v);
+            }
+        }
+    }
+    if (a.add.tot) {
+        // The product before this kernel was handed on unfinished: x += y (block.py:80) or x += y * sigmoid(r)
+        // (block.py:95-100), as rows_finish_kernel would have done.
+        const bool gated = a.add.op == ROW_GATE_ADD;
+#pragma unroll
+        for (int g = 0; g < NSEG; ++g) {
+            const int c0 = 4 * (tid + g * nt);
+            if (c0 < C) {
+                long long tot[4] = {0, 0, 0, 0};
+                float gt[4] = {0.f, 0.f, 0.f, 0.f};
+                slices_sum4(a.add.tot + (size_t)t * a.add.ldd + c0, a.add.slice, a.add.slices, tot);
+                if (gated) ld4(gt, a.add.gate + (size_t)t * C + c0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const double y = deferred_y(a.add, t, tot[i]);
+                    xv[g][i] += gated ? y * (double)sigmoid_f32(gt[i]) : y;
+                }
+                if (a.x_out && m == 0) st4(a.x_out + (size_t)t * C + c0, xv[g]);
+            }
+        }
+    }
+    double s[2] = {0.0, 0.0};
+#pragma unroll
+    for (int g = 0; g < NSEG; ++g) {
+        if (4 * (tid + g * nt) < C) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { s[0] += xv[g][i]; if (MIX) s[1] += pv[g][i]; }
+        }
+    }
+    bsum<2>(s, red0, nw);
+    const double mean = s[0] / (double)C, meanp = s[1] / (double)C;
+    double q[2] = {0.0, 0.0};
+#pragma unroll
+    for (int g = 0; g < NSEG; ++g) {
+        if (4 * (tid + g * nt) < C) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double d = xv[g][i] - mean;
+                q[0] += d * d;
+                if (MIX) { const double dp = pv[g][i] - meanp; q[1] += dp * dp; }
+            }
+        }
+    }
+    bsum<2>(q, red1, nw);
+    const double rsd = 1.0 / sqrt(q[0] / (double)C + 1e-5), rsdp = MIX ? 1.0 / sqrt(q[1] / (double)C + 1e-5) : 0.0;
+    float xs[NSEG][4];
+    float amax = 0.f;
+    double z[1] = {0.0};
+    double *sh = !MIX || m != 0 ? nullptr : a.shift_out ? a.shift_out + (size_t)t * C : t == a.R - 1 ? a.shift_dst : nullptr;
+#pragma unroll
+    for (int g = 0; g < NSEG; ++g) {
+        const int c0 = 4 * (tid + g * nt);
+        if (c0 < C) {
+            double xy[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                xy[i] = lw[g][i] * ((xv[g][i] - mean) * rsd) + lb[g][i];
+                double v = xy[i];
+                if (MIX) {
+                    const double prev = need_prev ? lw[g][i] * ((pv[g][i] - meanp) * rsdp) + lb[g][i] : pv[g][i];
+                    v = xy[i] * mu[g][i] + prev * (1.0 - mu[g][i]);
+                }
+                xs[g][i] = (float)(v * (double)rg[g][i]);
+                amax = fmaxf(amax, fabsf(xs[g][i]));
+                z[0] += v * of[g][i];
+            }
+            if (sh) st4(sh + c0, xy);
+        }
+    }
+    amax = wmaxf(amax);
+    if (lane == 0) redf[tid >> 6] = amax;
+    bsum<1>(z, red2, nw);                       // (its barrier also publishes redf)
+    double S, invS, qsum[1] = {0.0};
+    row_scale(row16_max((lane & 15) < nw ? redf[lane & 15] : 0.f), S, invS);
+    signed char *dig = m == 0 ? a.dig[0] : m == 1 ? a.dig[1] : a.dig[2];
+#pragma unroll
+    for (int g = 0; g < NSEG; ++g) {
+        const int c0 = 4 * (tid + g * nt);
+        if (c0 < C) qsum[0] += emit_quad(xs[g], invS, c0, t, C >> 6, dig);
+    }
+    bsum<1>(qsum, red3, nw);
+    if (tid == 0) {
+        (m == 0 ? a.S[0] : m == 1 ? a.S[1] : a.S[2])[t] = S;
+        (m == 0 ? a.qs[0] : m == 1 ? a.qs[1] : a.qs[2])[t] = qsum[0];
+        (m == 0 ? a.zp[0] : m == 1 ? a.zp[1] : a.zp[2])[t] = z[0];
+    }
 }
 
 template <int NM, int NSEG, int kLT>
@@ -1408,24 +1583,26 @@ int rows_embed(hipStream_t st, const int64_t *tokens, int64_t R, int V, int C, c
     return RWKV_OK;
 }
 
-bool rows_ln_width_supported(int64_t C) { return C % 4 == 0 && C <= 3 * 4 * kLnMaxThreads; }
+bool rows_ln_width_supported(int64_t C) { return C % 4 == 0 && C <= kLnMaxWidth; }
 
 int rows_ln_mix_quant(hipStream_t st, int n_mix, int64_t R, int C, bool sequence, const double *x, const double *ln_w,
                       const double *ln_b, const double *mu, const double *prev0, double *shift_dst,
                       int64_t prev_stride, const float *const *range, const double *const *offset,
-                      const RowsOperand *out, const RowsDeferred *add) {
+                      const RowsOperand *out, const RowsFew *few) {
     if (C % 64 != 0 || !rows_ln_width_supported(C))
-        return set_error(RWKV_ERR_SIZE, "rows_ln_mix_quant: width %d is not a multiple of 64 up to %d", C, 3 * 4 * kLnMaxThreads);
+        return set_error(RWKV_ERR_SIZE, "rows_ln_mix_quant: width %d is not a multiple of 64 up to %d", C, kLnMaxWidth);
     LnQuantArgs a;
     a.C = C; a.R = (int)R; a.sequence = sequence ? 1 : 0; a.x = x; a.ln_w = ln_w; a.ln_b = ln_b; a.mu = mu;
-    a.add.tot = nullptr; a.x_rw = nullptr;
-    if (add && add->tot) {
-        // every row is read and rewritten by its own workgroup only: rows of a sequence read their neighbour's x too
-        if (sequence || R >= kRowsDeferMax || (add->op != ROW_ADD && add->op != ROW_GATE_ADD))
-            return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: a pending product needs fewer than %d batch rows and a residual tail",
-                             (int)kRowsDeferMax);
-        a.add = *add; a.x_rw = const_cast<double *>(x);
+    a.add.tot = nullptr; a.x_out = nullptr; a.shift_out = nullptr; a.commit_src = nullptr; a.commit_dst = nullptr;
+    if (few) {
+        if (few->add.tot && (sequence || (few->add.op != ROW_ADD && few->add.op != ROW_GATE_ADD) || few->x_out == x))
+            return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: a pending product needs batch rows, a residual tail and another buffer for the new x");
+        if (R >= kRowsDeferMax && (few->add.tot || few->shift_out || few->commit_src))
+            return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: pending work needs fewer than %d rows", (int)kRowsDeferMax);
+        a.add = few->add; a.x_out = few->x_out; a.shift_out = few->shift_out; a.commit_src = few->commit_src; a.commit_dst = few->commit_dst;
     }
+    if (n_mix > 0 && R < kRowsDeferMax && !a.shift_out && !(sequence && R > 1 && prev0 != shift_dst))
+        return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: few rows need their shift rows kept apart");
     a.prev0 = prev0; a.shift_dst = shift_dst; a.prev_stride = prev_stride;
     const int n_out = n_mix > 0 ? n_mix : 1;
     for (int m = 0; m < 3; ++m) {
@@ -1433,18 +1610,29 @@ int rows_ln_mix_quant(hipStream_t st, int n_mix, int64_t R, int C, bool sequence
         a.range[m] = range[k]; a.offset[m] = offset[k];
         a.dig[m] = out[k].dig; a.S[m] = out[k].S; a.qs[m] = out[k].qs; a.zp[m] = out[k].zp;
     }
-    // few rows: 512 threads per row shorten the chain of dependent steps; many rows: 256 threads with twice
-    // the channels each keep more rows resident per compute unit
-    const bool many = R >= kRowsDeferMax;           // (a pending product is only ever handed to the 512-thread form)
-    const dim3 grid((unsigned)R), block(many ? 256 : 512);
-    const bool small = many ? C <= 3 * 4 * 256 : C <= 2 * 4 * 512;
+    // few rows: a workgroup per row and mix; many rows: one per row, 256 threads with more channels each, which keeps more
+    // rows resident per compute unit
+    const bool many = R >= kRowsDeferMax;
+    if (!many) {
+        const int nseg = C <= 4 * 1024 ? 1 : 2;
+        const dim3 grid((unsigned)R, (unsigned)n_out), block((unsigned)round_up(ceil_div(C, 4 * nseg), 64));
+        if (n_mix == 0) {
+            if (nseg == 1) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<false, 1, 1024>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<false, 2, 768>), grid, block, 0, st, a);
+        } else {
+            if (nseg == 1) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 1, 1024>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 2, 768>), grid, block, 0, st, a);
+        }
+        RWKV_CHECK_LAUNCH("rows_ln_mix_quant_row_kernel");
+        return RWKV_OK;
+    }
+    const bool small = C <= 3 * 4 * 256;
+    const dim3 grid((unsigned)R), block(256);
 #define RWKV_LNQ(NM)                                                                                  \
     do {                                                                                              \
-        if (many && small && R <= 512) hipLaunchKernelGGL((rows_ln_mix_quant_few_kernel<NM, 3, 256>), grid, block, 0, st, a);   \
-        else if (many && small) hipLaunchKernelGGL((rows_ln_mix_quant_kernel<NM, 3, 256>), grid, block, 0, st, a);   \
-        else if (many) hipLaunchKernelGGL((rows_ln_mix_quant_kernel<NM, 6, 256>), grid, block, 0, st, a);       \
-        else if (small) hipLaunchKernelGGL((rows_ln_mix_quant_kernel<NM, 2, 512>), grid, block, 0, st, a);      \
-        else hipLaunchKernelGGL((rows_ln_mix_quant_kernel<NM, 3, 512>), grid, block, 0, st, a);                 \
+        if (small && R <= 512) hipLaunchKernelGGL((rows_ln_mix_quant_few_kernel<NM, 3, 256>), grid, block, 0, st, a);   \
+        else if (small) hipLaunchKernelGGL((rows_ln_mix_quant_kernel<NM, 3, 256>), grid, block, 0, st, a);   \
+        else hipLaunchKernelGGL((rows_ln_mix_quant_kernel<NM, 6, 256>), grid, block, 0, st, a);       \
     } while (0)
     switch (n_mix) {
         case 0: RWKV_LNQ(0); break;

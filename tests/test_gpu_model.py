@@ -499,6 +499,29 @@ def test_shapes_chunkings_and_batches_against_the_exact_oracle(L, C, F, V, T, cu
     hip.check()
 
 
+# few rows: a workgroup per row and mix.  Ragged thread counts, the widest row with one group of channels per thread (4096),
+# the narrowest with two (4160), and on both sides of the rows (8, 32) and launch sizes at which the products around them change
+@pytest.mark.parametrize("C,F,B", [(64, 64, 2), (1088, 4352, 8), (1088, 4352, 9), (1984, 8192, 12), (4096, 8192, 3), (4096, 8192, 32),
+                                   (4160, 4160, 1), (4160, 4160, 33)])
+def test_batch_steps_of_ragged_and_wide_rows_match_single_steps(C, F, B):
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"batch of {B} at C={C} F={F}")
+    m = HipRWKV(synth.make_state_dict(2, C, F, V=100, seed=C + B, ln="random"))
+    states = torch.stack([m.emptyState.clone() for _ in range(B)])
+    for b in range(B):
+        m.forward(synth.random_tokens(1 + b % 3, V=100, seed=b).tolist(), states[b])
+    singles = states.clone()
+    for step in range(2):
+        toks = synth.random_tokens(B, V=100, seed=50 + step)
+        lb, states = m.forward_batch(toks.cuda(), states)
+        for b in range(B):
+            l1, _ = m.forward([int(toks[b])], singles[b])
+            # exact integer products on both sides; the float32 recurrence and gates in the same order
+            assert float((lb[b] - l1).norm() / l1.norm()) < 2e-6, (step, b)
+    for row in range(5):
+        assert float((states[:, :, row] - singles[:, :, row]).norm() / singles[:, :, row].norm()) < 2e-6, row
+
+
 def test_rwkv_shell_loads_checkpoint_file_and_generates(tmp_path, tiny):
     """RWKV(path) -> RWKVMaster surface (load.py:18,42-47; rwkvMaster.py:28-105) over the HIP model."""
     from rwkvstic_amd.master import RWKV, greedy
