@@ -143,14 +143,14 @@ def gen(KW, R, NV, NSH, HELP=False, BW=8):
     def block_load(dst, sbase, extra, b, wh=False):
         """16-byte-per-lane load of block b of a job whose base address is in s[sbase:sbase+1] (+ extra bytes)."""
         if wh:
-            e(f"global_load_dwordx4 {dst}, v{V_OFF}, %[wh]")
+            e(f"global_load_dwordx4 {dst}, v{V_OFF}, %[wh]{POLICY}")
         elif SADDR:
             e(f"s_add_u32 s{S_TMP}, s{sbase}, {extra + 1024 * BW * b}")
             e(f"s_addc_u32 s{S_TMP + 1}, s{sbase + 1}, 0")
-            e(f"global_load_dwordx4 {dst}, v{V_OFF}, s[{S_TMP}:{S_TMP + 1}]")
+            e(f"global_load_dwordx4 {dst}, v{V_OFF}, s[{S_TMP}:{S_TMP + 1}]{POLICY}")
         else:
             assert extra == 0
-            e(f"global_load_dwordx4 {dst}, v{V_OFF + b}, s[{sbase}:{sbase + 1}]")
+            e(f"global_load_dwordx4 {dst}, v{V_OFF + b}, s[{sbase}:{sbase + 1}]{POLICY}")
     LH = R * KW // math.gcd(R, KW)
     e = Emit(NA)
 
@@ -473,11 +473,15 @@ CONFIGS = [(2, 4, 4, 26), (3, 4, 4, 13), (2, 8, 4, 26), (3, 8, 4, 20), (4, 8, 4,
            (10, 8, 8, int(os.environ.get("RWKV_BACK_R_WIDE", "26")))]
 
 
+POLICY = "@policy@"       # suffix of every weight load, see RWKV_BACK_POLICY
+
+
 def main():
     out = []
     w = out.append
     w("// Generated by gen_decode_back.py - do not edit.  One asm statement per kernel width: the program")
     w("// of a weight-streaming wave of the single-token kernel (see the generator for the register map).")
+    w("// RWKV_BACK_POLICY: cache policy of the weight loads, an assembler suffix; the includer defines it (and a namespace).")
     w("template <int NB, int FW> struct BackCfg;")
     w("template <int NB, int FW> struct BackCfgH;      // with helper workgroups: no ffn key tiles")
     for KW, BW, FW, R, HELP in [c + (False,) for c in CONFIGS] + [(5, 8, 8, R_HELP, True)]:
@@ -494,7 +498,7 @@ def main():
         w("        const unsigned whhi = (unsigned)((unsigned long long)(uintptr_t)wh >> 32);")
         w("        asm volatile(")
         for ln in lines:
-            w(f'            "{ln}\\n"')
+            w(f'            "{ln}\\n"'.replace(POLICY, '" RWKV_BACK_POLICY "'))
         w('            :')
         w('            : [jt] "s"(jt), [wh] "s"(wh), [whlo] "s"(whlo), [whhi] "s"(whhi), [L] "s"(L), [hr] "s"(hr), [vt] "s"(vt),')
         w('              [g] "s"(g), [wb] "s"(wb), [lds] "s"(lds)')

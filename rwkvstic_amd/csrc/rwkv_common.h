@@ -133,6 +133,12 @@ __device__ __forceinline__ float wkv_step_f32(double w, double u, float k, float
     return y;
 }
 
+// Whether a model's quantised matrices are too many for the 256 MB Infinity Cache to hold from one token to the next:
+// their loads then go past the caches.  222 MB are faster kept, 242 MB streamed (figures beside back_streamed in
+// rwkv_decode.hip, gemv16_kernel in rwkv_rows.hip).
+constexpr int64_t kStreamWeightBytes = 230000000;
+inline bool weights_streamed(int64_t L, int64_t C, int64_t F, int64_t V) { return L * (5 * C * C + 2 * C * F) + V * C > kStreamWeightBytes; }
+
 // ---- the streaming tile product ---------------------------------------------
 // One workgroup computes, for NM matrices that share n_in, the dot products of
 // one 8-column tile with NB activation vectors held in LDS.

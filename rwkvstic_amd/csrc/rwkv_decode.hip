@@ -140,7 +140,23 @@ struct DArgs {
 // Their program is generated (gen_decode_back.py -> rwkv_decode_back.inc): one asm statement with
 // its own register map, so that the ring of in-flight weight blocks sits in fixed registers that
 // are reloaded in place.  It meets the compiled front waves only at LDS and workgroup barriers.
+//
+// Two cache policies for the weight loads.  A model that fits the 256 MB Infinity Cache finds part of its weights there
+// again at the next token; of a larger one nothing is left by then, and loads that do not displace what else is cached
+// (exchange words, constants, instructions) are faster.  8 tokens, cached / streamed: 1024 channels and 8, 14, 18 layers
+// (160, 242, 296 MB) 1055 / 1124, 1804 / 1767, 2265 / 2213 us; 768 and 24 layers (222 MB) 2684 / 2745; 1536 and 4, 8
+// layers (200, 322 MB) 747 / 858, 1459 / 1416; 32 layers of 4096 12367 / 11747; 16 tokens of the 3B shape 11696 / 11296
+// (11446 without the helpers' loads), 4 of 14B 11430 / 11169.
+namespace back_cached {
+#define RWKV_BACK_POLICY ""
 #include "rwkv_decode_back.inc"
+#undef RWKV_BACK_POLICY
+}
+namespace back_streamed {
+#define RWKV_BACK_POLICY " nt"
+#include "rwkv_decode_back.inc"
+#undef RWKV_BACK_POLICY
+}
 
 // ---- cross-lane reductions (DPP, fixed order) --------------------------------
 template <int CTRL>
@@ -696,7 +712,9 @@ __device__ __forceinline__ void vec_front(Front &fx, int &seq, const u64 *src, c
 }
 
 // =============================================================================
-template <int NB, int FW, bool HELP> using BackOf = std::conditional_t<HELP, BackCfgH<NB, FW>, BackCfg<NB, FW>>;
+template <int NB, int FW, bool HELP, bool STREAM = true>       // (the two policies differ in nothing but the loads)
+using BackOf = std::conditional_t<STREAM, std::conditional_t<HELP, back_streamed::BackCfgH<NB, FW>, back_streamed::BackCfg<NB, FW>>,
+                                  std::conditional_t<HELP, back_cached::BackCfgH<NB, FW>, back_cached::BackCfg<NB, FW>>>;
 
 template <int NB, int FW, bool TRACE, bool HELP>
 __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, const v4i *red, double *stat, double *rf_lds,
@@ -976,12 +994,12 @@ __device__ __forceinline__ void helper_path(const DArgs &a, signed char *dig, v4
 #pragma unroll
         for (int i = 0; i < BLDS; ++i) {
             if (paced && i % 3 == 0) asm volatile("s_sleep %0" :: "n"(kHelperPace) : "memory");
-            T[i] = *blk(i, KREG);
+            T[i] = __builtin_nontemporal_load(blk(i, KREG));
         }
 #pragma unroll
         for (int i = 0; i < BREG; ++i) {
             if (paced && i % 3 == 0) asm volatile("s_sleep %0" :: "n"(kHelperPace) : "memory");
-            W[i] = *blk(i / KREG, i % KREG);
+            W[i] = __builtin_nontemporal_load(blk(i / KREG, i % KREG));
         }
 #pragma unroll
         for (int i = 0; i < BLDS; ++i) stash[(wv * BLDS + i) * 64 + (tid & 63)] = T[i];
@@ -1150,7 +1168,7 @@ struct DecodeLds {
     static_assert(!HELP || RED_BYTES >= HelperShape<NB>::TILES * 256, "a helper's tile sums");
 };
 
-template <int NB, int FW, bool TRACE, bool HELP>
+template <int NB, int FW, bool TRACE, bool HELP, bool STREAM>
 __global__ void __launch_bounds__((FW + back_waves(NB)) * 64) decode_kernel(const DArgs a) {
     using Lds = DecodeLds<NB, FW, HELP>;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1177,7 +1195,7 @@ __global__ void __launch_bounds__((FW + back_waves(NB)) * 64) decode_kernel(cons
         constexpr int NWG = GroupShape<NB>::NWG;
         const int v_tiles = (a.m.V + 15) / 16, head_rounds = (v_tiles + NWG - 1) / NWG;
         const unsigned lds = (unsigned)(uintptr_t)(RWKV_LDS unsigned char *)smem;
-        BackOf<NB, FW, HELP>::run(a.m.jt + (size_t)blockIdx.x * (a.m.L + 1) * 16, a.m.w_head, a.m.L, head_rounds, v_tiles,
+        BackOf<NB, FW, HELP, STREAM>::run(a.m.jt + (size_t)blockIdx.x * (a.m.L + 1) * 16, a.m.w_head, a.m.L, head_rounds, v_tiles,
                          (int)blockIdx.x, wave - FW, lds);
     }
 }
@@ -1666,7 +1684,7 @@ int decode_clear_exchange(hipStream_t st, const DModel &m, const DecodeBuffers &
 
 constexpr int kMaxDevices = 64;
 
-template <int NB, int FW>
+template <int NB, int FW, bool STREAM>
 static int launch_one(hipStream_t st, const DArgs &args, bool with_prep) {
     constexpr bool HELP = HelperShape<NB>::NH > 0;
     const bool trace = args.b.trace != nullptr;
@@ -1681,9 +1699,9 @@ static int launch_one(hipStream_t st, const DArgs &args, bool with_prep) {
     {
         std::lock_guard<std::mutex> lock(mu);
         if (configured[dev] < lds) {
-            RWKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_kernel<NB, FW, false, HELP>),
+            RWKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_kernel<NB, FW, false, HELP, STREAM>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-            RWKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_kernel<NB, FW, true, HELP>),
+            RWKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&decode_kernel<NB, FW, true, HELP, STREAM>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds));
             configured[dev] = lds;
         }
@@ -1695,23 +1713,25 @@ static int launch_one(hipStream_t st, const DArgs &args, bool with_prep) {
     // owner workgroups first, then the helpers: every one of them is resident at once (one per compute unit)
     const dim3 grid((unsigned)(args.m.NWG + HelperShape<NB>::NH));
     if (trace)
-        hipLaunchKernelGGL((decode_kernel<NB, FW, true, HELP>), grid, dim3((FW + back_waves(NB)) * 64), lds, st, args);
+        hipLaunchKernelGGL((decode_kernel<NB, FW, true, HELP, STREAM>), grid, dim3((FW + back_waves(NB)) * 64), lds, st, args);
     else
-        hipLaunchKernelGGL((decode_kernel<NB, FW, false, HELP>), grid, dim3((FW + back_waves(NB)) * 64), lds, st, args);
+        hipLaunchKernelGGL((decode_kernel<NB, FW, false, HELP, STREAM>), grid, dim3((FW + back_waves(NB)) * 64), lds, st, args);
     RWKV_CHECK_LAUNCH("decode_kernel");
     return RWKV_OK;
 }
 
 static int launch_step(hipStream_t st, const DArgs &args, bool with_prep) {
+    // (from 2048 channels on a model is larger than the cache from a few layers on)
+    const bool stream = weights_streamed(args.m.L, args.m.C, args.m.F, args.m.V);
     switch (args.m.C) {
-        case 512: return launch_one<8, 4>(st, args, with_prep);
-        case 768: return launch_one<12, 4>(st, args, with_prep);
-        case 1024: return launch_one<16, 4>(st, args, with_prep);
-        case 1536: return launch_one<24, 4>(st, args, with_prep);
-        case 2048: return launch_one<32, 4>(st, args, with_prep);
-        case 2560: return launch_one<40, 8>(st, args, with_prep);
-        case 4096: return launch_one<64, 4>(st, args, with_prep);
-        case 5120: return launch_one<80, 8>(st, args, with_prep);
+        case 512: return stream ? launch_one<8, 4, true>(st, args, with_prep) : launch_one<8, 4, false>(st, args, with_prep);
+        case 768: return stream ? launch_one<12, 4, true>(st, args, with_prep) : launch_one<12, 4, false>(st, args, with_prep);
+        case 1024: return stream ? launch_one<16, 4, true>(st, args, with_prep) : launch_one<16, 4, false>(st, args, with_prep);
+        case 1536: return stream ? launch_one<24, 4, true>(st, args, with_prep) : launch_one<24, 4, false>(st, args, with_prep);
+        case 2048: return launch_one<32, 4, true>(st, args, with_prep);
+        case 2560: return launch_one<40, 8, true>(st, args, with_prep);
+        case 4096: return launch_one<64, 4, true>(st, args, with_prep);
+        case 5120: return launch_one<80, 8, true>(st, args, with_prep);
         default: return set_error(RWKV_ERR_SIZE, "decode kernel: n_embd %d not supported", args.m.C);
     }
 }

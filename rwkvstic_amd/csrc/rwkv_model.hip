@@ -596,6 +596,7 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     // Few batch rows: the products split their contraction, and the three whose result goes straight into one
     // row-wise kernel (k, v, r -> WKV; the two residual updates -> the next LayerNorm) leave the sum of their slices
     // to that kernel instead of a launch of their own.
+    const bool stream = weights_streamed(d.n_layer, d.n_embd, d.n_ffn, d.n_vocab);
     const bool defer = !sequence && R < kRowsDeferMax;
     RowsDeferred dk[3];
     // Few rows whose shift rows are read straight from the state: the LayerNorm kernels leave the new ones aside, and each
@@ -626,12 +627,12 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
         // k, v, r (and the ffn receptance below) are kept as float32 arrays in the kvr slab
         float *kvr32 = reinterpret_cast<float *>(w.kvr);
         RowsProduct pk[3];
-        for (int i = 0; i < 3; ++i) { pk[i].a = w.q[i]; pk[i].w16 = kvr[i]->packed16; pk[i].out = reinterpret_cast<double *>(kvr32 + i * RC); }
+        for (int i = 0; i < 3; ++i) { pk[i].a = w.q[i]; pk[i].w16 = kvr[i]->packed16; pk[i].out = reinterpret_cast<double *>(kvr32 + i * RC); pk[i].stream = stream; }
         RWKV_TRY(rows_products(st, 3, pk, w.tot, R, C, C, ROW_STORE_F32, nullptr, defer ? dk : nullptr));
         RWKV_TRY(rows_wkv(st, R, C, sequence, kvr32, kvr32 + RC, kvr32 + 2 * RC, L.time_decay, L.time_first,
                           sl + 2 * (size_t)C, state_stride, reinterpret_cast<float *>(w.att), defer ? dk : nullptr));
         RWKV_TRY(rows_quant(st, R, C, w.att, true, L.att_o.range, L.att_o.offset, w.q[0], (double *)w.tot));    // att and h: float32 arrays
-        const RowsProduct po = {w.q[0], L.att_o.packed16, x};
+        const RowsProduct po = {w.q[0], L.att_o.packed16, x, stream};
         RWKV_TRY(rows_products(st, 1, &po, w.tot, R, C, C, ROW_ADD, nullptr, defer ? &few.add : nullptr));
         // ChannelMix (block.py:82-100)
         if (copy_prev) RWKV_CHECK_HIP(hipMemcpyAsync(w.prev0, sl + C, (size_t)C * 8, hipMemcpyDeviceToDevice, st));
@@ -641,10 +642,10 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
         RWKV_TRY(rows_ln_mix_quant(st, 2, R, C, sequence, x, L.ln2_w, L.ln2_b, L.ffn_mix, copy_prev ? w.prev0 : sl + C,
                                    sl + C, state_stride, rg2, of2, w.q + 1, &few));
         advance(w.sh2, sl + C);
-        const RowsProduct pfk = {w.q[1], L.ffn_k.packed16, w.h}, pfr = {w.q[2], L.ffn_r.packed16, w.kvr};
+        const RowsProduct pfk = {w.q[1], L.ffn_k.packed16, w.h, stream}, pfr = {w.q[2], L.ffn_r.packed16, w.kvr, stream};
         RWKV_TRY(rows_ffn_key_receptance(st, pfk, pfr, w.tot, R, C, F));
         RWKV_TRY(rows_quant(st, R, F, w.h, true, L.ffn_v.range, L.ffn_v.offset, w.q[0], (double *)w.tot));
-        const RowsProduct pfv = {w.q[0], L.ffn_v.packed16, x};
+        const RowsProduct pfv = {w.q[0], L.ffn_v.packed16, x, stream};
         // (the ffn receptance stays in the kvr slab and the totals untouched until the next LayerNorm kernel has run)
         RWKV_TRY(rows_products(st, 1, &pfv, w.tot, R, F, C, ROW_GATE_ADD, kvr32, defer ? &few.add : nullptr));
     }
@@ -679,7 +680,7 @@ int rows_sequence(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t 
             rc = rows_ln_mix_quant(st, 0, 1, (int)C, false, tail.x + (size_t)(R - 1) * C, d.ln_out_w, d.ln_out_b, nullptr,
                                    nullptr, nullptr, 0, rg, of, rw.q, &tail.few);
             if (rc) return rc;
-            const RowsProduct ph = {rw.q[0], d.head.packed16, logits};
+            const RowsProduct ph = {rw.q[0], d.head.packed16, logits, weights_streamed(d.n_layer, d.n_embd, d.n_ffn, d.n_vocab)};
             rc = rows_products(st, 1, &ph, rw.tot, 1, C, d.n_vocab, ROW_STORE, nullptr);
         }
         if (rc) return rc;
@@ -889,7 +890,7 @@ int rwkv_model_forward_batch(rwkv_model *m, rwkv_stream_t stream, const int64_t 
     rc = rows_ln_mix_quant(st, 0, batch, (int)C, false, tail.x, d.ln_out_w, d.ln_out_b, nullptr, nullptr, nullptr, d.n_layer * 5 * C, rg, of,
                            rw.q, &tail.few);
     if (rc) return rc;
-    const RowsProduct ph = {rw.q[0], d.head.packed16, logits};
+    const RowsProduct ph = {rw.q[0], d.head.packed16, logits, weights_streamed(d.n_layer, d.n_embd, d.n_ffn, d.n_vocab)};
     return rows_products(st, 1, &ph, rw.tot, batch, C, V, ROW_STORE, nullptr);
 }
 

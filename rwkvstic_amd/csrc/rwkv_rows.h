@@ -20,6 +20,7 @@ struct RowsProduct {        // out[R, N] (tail op) a x quantised matrix in M16 b
     RowsOperand a;
     const uint8_t *w16;
     double *out;
+    bool stream = false;    // few rows: read the weights past the caches (see weights_streamed; of the first product of a launch)
 };
 constexpr int kRowsMaxProducts = 3;     // products of equal shape and tail that share one launch
 // A product whose contraction was split, handed on unfinished: its consumer (the LayerNorm kernel for the two

@@ -700,6 +700,12 @@ struct GemmArgs {
 // live in scratch memory).
 struct GemmCols { int NT, N, tail; };
 
+// Weights of the few-row kernels.  STREAM: past the caches, which keeps the digits and the next kernels' vectors there: 8
+// sequences at 3B 2.25 -> 2.08 ms a step, at 14B 5.75 -> 5.30; 32 sequences (9..32-row kernel) 3.20 -> 3.15 and 6.66 -> 6.59.  Of a
+// model that fits the Infinity Cache the weights are kept: 8 layers of 1024, 8 sequences 334 us, streamed 360.
+template <bool STREAM>
+__device__ __forceinline__ v4i ldw(const v4i *p) { return STREAM ? __builtin_nontemporal_load(p) : *p; }
+
 constexpr int kGemmNT = 8, kGemmWideNT = 10;     // N-tiles per workgroup (two wavefronts side by side)
 constexpr int kWideRing = 4;                     // LDS buffers of the 64 x 160 variant
 
@@ -925,6 +931,7 @@ constexpr int kSkinnyMT = 8, kSkinnyGN = 2, kSkinnyNT = 4 * kSkinnyGN;
 constexpr int kSkinnyFrags = kSkinnyMT + kSkinnyNT;     // 16: wave w fetches fragments w, w + 4, w + 8, w + 12
 constexpr int kSkinnyAhead = 6;
 
+template <bool STREAM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm8_skinny_kernel(const GemmArgs a) {
     __shared__ v4i frag[2][kSkinnyFrags][64];
     const int lane = threadIdx.x & 63;
@@ -976,7 +983,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #define RWKV_SKINNY_FETCH(F, K)                                                                      \
     do {                                                                                             \
         const size_t o_ = (size_t)((K) < nk ? (K) : nk - 1) * 64; /* past the end: the last block again (unused) */ \
-        F.v0 = src[0][o_]; F.v1 = src[1][o_]; F.v2 = src[2][o_]; F.v3 = src[3][o_];                  \
+        F.v0 = src[0][o_]; F.v1 = src[1][o_]; F.v2 = ldw<STREAM>(src[2] + o_); F.v3 = ldw<STREAM>(src[3] + o_); \
     } while (0)
 #define RWKV_SKINNY_PARK(F, B)                                                                       \
     do {                                                                                             \
@@ -986,7 +993,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     // (same step as gemm8_body: the next block is parked, and its registers refilled, piece by piece between
     // this block's groups of matrix instructions)
 #define RWKV_SKINNY_MOVE(FN, I, V, B, O)                                                             \
-    { frag[B][wave + 4 * (I)][lane] = FN.V; FN.V = src[I][O]; }
+    { frag[B][wave + 4 * (I)][lane] = FN.V; FN.V = (I) < 2 ? src[I][O] : ldw<STREAM>(src[I] + (O)); }
 #define RWKV_SKINNY_STEP(FN, K)                                                                      \
     {                                                                                                \
         const int buf_ = (K) & 1;                                                                    \
@@ -1055,7 +1062,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 // ---------------------------------------------------------------------------
 constexpr int kVecMT = 2;
 
-template <int MT, int NTW, int NW, int U>
+template <int MT, int NTW, int NW, int U, bool STREAM>
 __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
     __shared__ v4i red[NW][MT * NTW][64];
     const int lane = threadIdx.x & 63;
@@ -1095,7 +1102,7 @@ __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
         for (int i = 0; i < U; ++i) {
             const size_t o = (size_t)min(k + NW * i, a.KB - 1) * 64;      // past the end: a block nobody multiplies
 #pragma unroll
-            for (int j = 0; j < NTW; ++j) B[j][i] = bsrc[j][o];
+            for (int j = 0; j < NTW; ++j) B[j][i] = ldw<STREAM>(bsrc[j] + o);
 #pragma unroll
             for (int m = 0; m < MT; ++m) A[m][i] = asrc[m][o];
         }
@@ -1530,14 +1537,16 @@ static VecShape vec_shape(int64_t tiles, int64_t KB) {
     if (tiles > 256) return VecShape{1, 8, 5};
     return KB <= 48 ? VecShape{1, 16, 3} : VecShape{1, 16, 5};
 }
-static void launch_vec(hipStream_t st, const GemmArgs &g) {
+static void launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
     const int64_t tiles = g.NT2 > 0 ? (int64_t)g.NT + g.NT2 : (int64_t)g.NT * g.gz;
     const VecShape v = vec_shape(tiles, g.KB);
     const dim3 grid((unsigned)(g.NT2 > 0 ? ceil_div(g.NT, v.ntw) + ceil_div(g.NT2, v.ntw) : ceil_div(g.NT, v.ntw) * g.gz)), block((unsigned)(64 * v.nw));
 #define RWKV_VEC(NTW, NW, U)                                                                          \
     if (v.ntw == NTW && v.nw == NW && v.u == U) {                                                     \
-        if (g.MT == 1) hipLaunchKernelGGL((gemv16_kernel<1, NTW, NW, U>), grid, block, 0, st, g);     \
-        else hipLaunchKernelGGL((gemv16_kernel<2, NTW, NW, U>), grid, block, 0, st, g);               \
+        if (g.MT == 1 && stream) hipLaunchKernelGGL((gemv16_kernel<1, NTW, NW, U, true>), grid, block, 0, st, g);     \
+        else if (g.MT == 1) hipLaunchKernelGGL((gemv16_kernel<1, NTW, NW, U, false>), grid, block, 0, st, g);         \
+        else if (stream) hipLaunchKernelGGL((gemv16_kernel<2, NTW, NW, U, true>), grid, block, 0, st, g);             \
+        else hipLaunchKernelGGL((gemv16_kernel<2, NTW, NW, U, false>), grid, block, 0, st, g);        \
     }
     RWKV_VEC(4, 8, 3)
     RWKV_VEC(2, 16, 3)
@@ -1709,13 +1718,14 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     g.NT2 = g.N2 = g.tail2 = 0;
     if (pl.kind == PLAN_VEC) {
         g.gx = g.NT; g.gy = 1; g.by_rows = 0; g.per_xcd = 0;
-        launch_vec(st, g);
+        launch_vec(st, g, p[0].stream);
         RWKV_CHECK_LAUNCH("gemv16_kernel");
     } else {
         g.gx = pl.gx; g.gy = gy; g.by_rows = gy >= kXcds;
         g.per_xcd = ((g.by_rows ? gy : pl.gx) + kXcds - 1) / kXcds;
         const dim3 grid((unsigned)(kXcds * g.per_xcd * (g.by_rows ? pl.gx : gy) * g.gz));
-        if (pl.kind == PLAN_SKINNY) hipLaunchKernelGGL(gemm8_skinny_kernel, grid, dim3(256), 0, st, g);
+        if (pl.kind == PLAN_SKINNY && p[0].stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
+        else if (pl.kind == PLAN_SKINNY) hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
         else if (pl.kind == PLAN_WIDE) hipLaunchKernelGGL(gemm8_wide_kernel, grid, dim3(512), 0, st, g);
         else hipLaunchKernelGGL(gemm8_kernel, grid, dim3(512), 0, st, g);
         RWKV_CHECK_LAUNCH("gemm8_kernel");
@@ -1759,10 +1769,12 @@ int rows_ffn_key_receptance(hipStream_t st, const RowsProduct &k, const RowsProd
     const int gx = (int)(ceil_div(g.NT, kSkinnyNT) + ceil_div(g.NT2, kSkinnyNT));
     if (C % 64 == 0 && g.MT <= kVecMT && g.KB <= 1024) {
         g.gx = g.NT; g.per_xcd = 0;
-        launch_vec(st, g);
+        launch_vec(st, g, k.stream);
     } else if (C % 64 == 0 && g.MT <= kSkinnyMT && gx >= kSkinnyPairWgs) {
         g.gx = gx; g.per_xcd = (gx + kXcds - 1) / kXcds;
-        hipLaunchKernelGGL(gemm8_skinny_kernel, dim3((unsigned)(kXcds * g.per_xcd)), dim3(256), 0, st, g);
+        const dim3 grid((unsigned)(kXcds * g.per_xcd));
+        if (k.stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
+        else hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
     } else {
         const int rc = rows_products(st, 1, &k, tot, R, C, F, ROW_RELU2, nullptr);
         return rc ? rc : rows_products(st, 1, &r, tot, R, C, C, ROW_STORE_F32, nullptr);
