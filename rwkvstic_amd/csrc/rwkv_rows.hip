@@ -719,6 +719,11 @@ __device__ __forceinline__ void dma16(const v4i *g, unsigned lds_byte_offset) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "s"(lds_byte_offset) : "memory");
 }
 
+// The same past the caches (as ldw).
+__device__ __forceinline__ void dma16_stream(const v4i *g, unsigned lds_byte_offset) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" :: "v"(g), "s"(lds_byte_offset) : "memory");
+}
+
 // Accumulators of one wavefront (GM M-tiles x GN N-tiles from (mt0, nt0)) to totals or, when the contraction is not
 // split, straight through the product's tail.  Lane 16g + n, register i <-> digit i of token 4*mt + g, column 16*nt + n.
 //
@@ -807,7 +812,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, const GemmCols 
 // N-tiles, RING LDS buffers.  <4, 4, 3> is the general shape (8 wavefronts of 4 x 4 tiles, two workgroups per
 // compute unit); <5, 4, 4> (4 x 5 tiles, one workgroup per compute unit) is used where it turns a grid of 1.25
 // workgroups per compute unit into exactly one (2560 columns: 16 column blocks instead of 20).
-template <int GN, int WM, int RING>
+template <int GN, int WM, int RING, bool STREAM>
 __device__ __forceinline__ void gemm8_body(const GemmArgs a) {
     // Both operands of a contraction block are fetched once per workgroup into LDS and read from there by
     // the wavefronts that need each fragment (one barrier per block).
@@ -870,8 +875,10 @@ __device__ __forceinline__ void gemm8_body(const GemmArgs a) {
 #define RWKV_GEMM_DMA(SLOT, K)                                                                       \
     do {                                                                                             \
         const size_t o_ = (size_t)((K) < nk ? (K) : nk - 1) * 64; /* past the end: the last block again (unused) */ \
-        _Pragma("unroll") for (int i = 0; i < kGemmLoads; ++i)                                       \
-            dma16(src[i] + o_, lds0 + (unsigned)(((SLOT) * kSlots + kNW * i) * 1024));               \
+        _Pragma("unroll") for (int i = 0; i < kGemmLoads; ++i) {                                     \
+            if (STREAM && kNW * i >= 16) dma16_stream(src[i] + o_, lds0 + (unsigned)(((SLOT) * kSlots + kNW * i) * 1024)); \
+            else dma16(src[i] + o_, lds0 + (unsigned)(((SLOT) * kSlots + kNW * i) * 1024));          \
+        }                                                                                            \
     } while (0)
 #define RWKV_GEMM_STEP(SLOT, K)                                                                      \
     {                                                                                                \
@@ -914,11 +921,12 @@ __device__ __forceinline__ void gemm8_body(const GemmArgs a) {
     gemm_epilogue<kGM, kGN>(a, GemmCols{a.NT, a.N, a.tail}, acc, mt0, nt0, mat, bz, lane);
 }
 
+template <bool STREAM>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) gemm8_kernel(const GemmArgs a) {
-    gemm8_body<4, 4, 3>(a);
+    gemm8_body<4, 4, 3, STREAM>(a);
 }
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm8_wide_kernel(const GemmArgs a) {
-    gemm8_body<5, 4, kWideRing>(a);
+    gemm8_body<5, 4, kWideRing, false>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -1492,6 +1500,10 @@ constexpr int kGemmWideNum = 10, kGemmWideDen = 9;     // the 64 x 160 variant i
 // 256-token chunks: the [256 x 20480] x [20480 x 5120] product; 14,080 against 13,190 tokens/s)
 constexpr int kGemmLongFillWgs = 256, kGemmLongBlocks = 200;
 constexpr int kSkinnyFillWgs = 128;     // 9..32 rows (weight streaming): the contraction is split until the grid has this many workgroups (batch-32 step: 8.07 ms at 128, 8.73 at 256, 9.17 at 64 for the 14B shape; 4.06 / 4.13 / 4.11 ms for the 3B shape)
+// Row blocks of 64 tokens up to which the general kernel reads the weights past the caches: more of them find each other's weight
+// blocks there (prompts, kept / streamed: 77 tokens of 24 layers of 1024 2274 / 2193 us, 100 of the 3B shape 4565 / 4416, 256 of it
+// 6158 / 6248, 256 of 14B 17786 / 18992)
+constexpr int kStreamRowBlocks = 2;
 constexpr int kSkinnyPairWgs = 64;      // ffn key and receptance of 9..32 rows in one launch from so many workgroups on
 constexpr int kGemmFillWgs = 96;         // larger products: split until the grid has this many workgroups.  A split costs a second launch and a round trip of the integer totals through memory, so it only pays for grids far below the device (3B shape, tokens/s in chunks of 64 / 128 / 256 / 512 tokens: 13,180 / 23,640 / 37,610 / 52,070 at 96; 12,480 / 21,280 / 34,650 / 49,380 at 256; 12,540 / 21,470 / 31,520 / 51,160 at 64)
 
@@ -1727,7 +1739,8 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
         if (pl.kind == PLAN_SKINNY && p[0].stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
         else if (pl.kind == PLAN_SKINNY) hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
         else if (pl.kind == PLAN_WIDE) hipLaunchKernelGGL(gemm8_wide_kernel, grid, dim3(512), 0, st, g);
-        else hipLaunchKernelGGL(gemm8_kernel, grid, dim3(512), 0, st, g);
+        else if (p[0].stream && gy <= kStreamRowBlocks) hipLaunchKernelGGL(gemm8_kernel<true>, grid, dim3(512), 0, st, g);
+        else hipLaunchKernelGGL(gemm8_kernel<false>, grid, dim3(512), 0, st, g);
         RWKV_CHECK_LAUNCH("gemm8_kernel");
     }
     for (int m = 0; defer && m < n; ++m) defer[m].tot = nullptr;
