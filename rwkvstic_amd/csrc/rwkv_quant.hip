@@ -88,7 +88,7 @@ quantize_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in,
 // Bound: memory (the float32 matrix twice, the second time mostly from the memory-side cache, the codes once per
 // layout).  quantize_kernel walks all rows with one workgroup per 64 channels, 40 workgroups at 2560 channels, and
 // the packed layouts then read its codes back byte by byte.  The seven matrices of a layer of width 2560: 5.14 ms
-// that way, 0.315 ms here (host calls included; the 511 MB at copy rate: 0.108).
+// that way, 0.288 ms here (host calls included; the 511 MB at copy rate: 0.108).
 //
 //   quant_minmax_kernel   256 channels x one of the row splits: partial minimum and maximum
 //   quant_scale_kernel    one channel per thread: partials -> lo, range, 1 / range
@@ -191,6 +191,10 @@ __device__ __forceinline__ double quotient(double d, double b, double inv) {
     return fma(fma(-b, x, d), inv, x);
 }
 
+// 16 bytes of a packed layout.  They are stored past the caches, which leaves the float32 matrix there for the encoding pass
+// (the seven matrices of a layer of width 2560: 0.315 -> 0.288 ms).
+typedef uint32_t Chunk __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ int slot8(int lane) { return lane ^ ((lane >> 3) & 6); }
 __device__ __forceinline__ int slot16(int lane, int half) { return lane ^ (((lane >> 3) & 6) | (half << 3)); }
 
@@ -247,12 +251,12 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
             if (packed) {
                 const int64_t ct = (k0 >> 3) + i;
                 if (ct < n_ct8)
-                    *reinterpret_cast<uint4 *>(packed + (ct * n_kb8 + blockIdx.x) * 1024 + lane * 16) = *reinterpret_cast<const uint4 *>(&p8[i][slot8(lane) * 4]);
+                    __builtin_nontemporal_store(*reinterpret_cast<const Chunk *>(&p8[i][slot8(lane) * 4]), reinterpret_cast<Chunk *>(packed + (ct * n_kb8 + blockIdx.x) * 1024 + lane * 16));
             }
             if (packed16) {
                 const int64_t ct = (k0 >> 4) + (i >> 1), kb = (int64_t)blockIdx.x * 2 + (i & 1);
                 if (ct < n_ct16 && kb < n_kb16)
-                    *reinterpret_cast<uint4 *>(packed16 + (ct * n_kb16 + kb) * 1024 + lane * 16) = *reinterpret_cast<const uint4 *>(&m16[i][slot16(lane, i & 1) * 4]);
+                    __builtin_nontemporal_store(*reinterpret_cast<const Chunk *>(&m16[i][slot16(lane, i & 1) * 4]), reinterpret_cast<Chunk *>(packed16 + (ct * n_kb16 + kb) * 1024 + lane * 16));
             }
         }
         if (codes) {
