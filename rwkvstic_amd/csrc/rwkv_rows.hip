@@ -695,6 +695,12 @@ struct GemmArgs {
     // NT2 > 0: the launch holds two products of different widths (same rows, same contraction, not split): product 1 has
     // NT2 tiles, N2 columns and tail2, and its workgroups follow product 0's
     int NT2, N2, tail2;
+    // part non-null (few rows, product 0 with the relu^2 tail): what the quantiser of its result needs of every row and column
+    // tile, {max |xs|, zero-point share} at [row][tile], and qs of the operand to be, cleared
+    double2 *part;
+    const float *next_range;
+    const double *next_offset;
+    double *next_qs;
 };
 // Columns and tail of the product a workgroup works for (kept apart from the arguments: a modified copy of those would
 // live in scratch memory).
@@ -1070,6 +1076,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 // ---------------------------------------------------------------------------
 constexpr int kVecMT = 2;
 
+// The relu^2 tail of one tile (as gemm_tail's), and the tile's share of what rows_quant_tiles_kernel needs to know of the rows.
+__device__ __forceinline__ void relu2_part(const GemmArgs &a, const v4i d, int m, int nt, int lane) {
+    const int g = lane >> 4, n = lane & 15, t = 4 * m + g, col = 16 * nt + n;
+    const bool live = t < a.R;
+    const int tc = live ? t : a.R - 1;
+    const double tot = (double)(((((long long)d.x * 256 + d.y) * 256 + d.z) * 256) + d.w);
+    const double y = a.S[0][tc] * tot + (128.0 * (a.S[0][tc] * a.qs[0][tc]) + a.zp[0][tc]), r = y > 0.0 ? y : 0.0;
+    const float h = (float)(r * r);
+    if (live) reinterpret_cast<float *>(a.out[0])[(size_t)t * a.N + col] = h;
+    const double v = live ? (double)h : 0.0;
+    const float amax = row16_max(fabsf((float)(v * (double)a.next_range[col])));
+    const double z = row16_sum(v * a.next_offset[col]);
+    if (live && n == 0) {
+        a.part[(size_t)t * a.NT + nt] = make_double2((double)amax, z);
+        if (nt == 0) a.next_qs[t] = 0.0;
+    }
+}
+
 template <int MT, int NTW, int NW, int U, bool STREAM>
 __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
     __shared__ v4i red[NW][MT * NTW][64];
@@ -1138,7 +1162,44 @@ __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
         sum[0][0] = red[0][i][lane];
 #pragma unroll
         for (int w = 1; w < NW; ++w) sum[0][0] += red[w][i][lane];
-        gemm_epilogue<1, 1>(a, cols, sum, m, nt, mat, bz, lane);
+        if (mat == 0 && a.part) relu2_part(a, sum[0][0], m, nt, lane);
+        else gemm_epilogue<1, 1>(a, cols, sum, m, nt, mat, bz, lane);
+    }
+}
+
+// Quantiser of a product whose tiles left their share of every row (relu2_part): a part of 1024 values per workgroup, one launch
+// instead of a pass for the rows' maxima and one for the digits (8 rows of 10240: 4.7 us against 3.9 + 4.0).  A step of 8
+// sequences at 3B 2.08 -> 2.04 ms, of 5 at 24 layers of 2048 1.40 -> 1.34, of 8 at 24 layers of 1024 1.033 -> 1.019; not for rows
+// up to 3072, which one workgroup each quantises as fast (12 layers of 768, 8 sequences: 451 us that way, 458 this).  The sum of
+// the fixed-point values is added up with atomics: integers below 2^53, exact in
+// any order.
+__global__ void __launch_bounds__(kRT) rows_quant_tiles_kernel(const QuantArgs a, const double2 *part, int tiles) {
+    __shared__ double red0[16], red1[16];
+    __shared__ float redf[16];
+    const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, c0 = 4 * (blockIdx.x * kRT + tid);
+    const bool live = c0 < a.K;                            // (whole groups of four lanes: K is a multiple of 64)
+    float v[4] = {0.f, 0.f, 0.f, 0.f}, rg[4] = {0.f, 0.f, 0.f, 0.f}, amax = 0.f;
+    if (live) { ld4(v, static_cast<const float *>(a.in) + (size_t)t * a.K + c0); ld4(rg, a.range + c0); }
+    double z[1] = {0.0};
+    for (int i = tid; i < tiles; i += kRT) {
+        const double2 p = part[(size_t)t * tiles + i];
+        amax = fmaxf(amax, (float)p.x); z[0] += p.y;
+    }
+    amax = wmaxf(amax);
+    if (lane == 0) redf[tid >> 6] = amax;
+    bsum<1>(z, red0, kRW);                                 // (its barrier also publishes redf)
+    double S, invS, qsum[1] = {0.0};
+    row_scale(row16_max((lane & 15) < kRW ? redf[lane & 15] : 0.f), S, invS);
+    if (live) {
+        float xs[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xs[i] = (float)((double)v[i] * (double)rg[i]);
+        qsum[0] = emit_quad(xs, invS, c0, t, a.K >> 6, a.dig);
+    }
+    bsum<1>(qsum, red1, kRW);
+    if (tid == 0) {
+        atomicAdd(a.qs + t, qsum[0]);
+        if (blockIdx.x == 0) { a.S[t] = S; a.zp[t] = z[0]; }
     }
 }
 
@@ -1728,6 +1789,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     g.gz = split * n;
     g.tail = split > 1 ? -1 : op;
     g.NT2 = g.N2 = g.tail2 = 0;
+    g.part = nullptr;
     if (pl.kind == PLAN_VEC) {
         g.gx = g.NT; g.gy = 1; g.by_rows = 0; g.per_xcd = 0;
         launch_vec(st, g, p[0].stream);
@@ -1767,7 +1829,8 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
 // Few rows: both in one launch, whole contractions (the receptance's column blocks find room beside the key's; apart they
 // were up to four launches, two of them only adding slices).  With gemv16_kernel's shapes: 8 sequences at 3B 2.96 -> 2.40 ms
 // a step, 32 at 14B 7.38 -> 6.66 ms (its two launches and the receptance's sum of slices: 31.8 + 13.5 + 4.6 us, one launch 37.5).
-int rows_ffn_key_receptance(hipStream_t st, const RowsProduct &k, const RowsProduct &r, long long *tot, int64_t R, int64_t C, int64_t F) {
+int rows_ffn_key_receptance(hipStream_t st, const RowsProduct &k, const RowsProduct &r, long long *tot, int64_t R, int64_t C, int64_t F,
+                            const float *range, const double *offset, const RowsOperand &out) {
     GemmArgs g;
     const RowsProduct *p[2] = {&k, &r};
     for (int m = 0; m < kRowsMaxProducts; ++m) {
@@ -1778,22 +1841,33 @@ int rows_ffn_key_receptance(hipStream_t st, const RowsProduct &k, const RowsProd
     g.MT = (int)ceil_div(R, 4); g.NT = (int)ceil_div(F, 16); g.KB = (int)(C / 64); g.ldd = g.NT * 16;
     g.kb_per_split = g.KB; g.split = 1; g.gz = 1; g.gy = 1; g.by_rows = 0;
     g.tail = ROW_RELU2; g.R = (int)R; g.N = (int)F;
+    g.part = nullptr;
     g.NT2 = (int)ceil_div(C, 16); g.N2 = (int)C; g.tail2 = ROW_STORE_F32;
     const int gx = (int)(ceil_div(g.NT, kSkinnyNT) + ceil_div(g.NT2, kSkinnyNT));
     if (C % 64 == 0 && g.MT <= kVecMT && g.KB <= 1024) {
         g.gx = g.NT; g.per_xcd = 0;
+        if (F > 3072) g.part = reinterpret_cast<double2 *>(tot);       // (16 bytes per row and tile: no more than a slice of totals)
+        g.next_range = range; g.next_offset = offset; g.next_qs = out.qs;
         launch_vec(st, g, k.stream);
+        RWKV_CHECK_LAUNCH("gemv16_kernel");
+        if (!g.part) return rows_quant(st, R, F, k.out, true, range, offset, out, nullptr);
+        QuantArgs q;
+        q.K = (int)F; q.in = k.out; q.range = range; q.offset = offset; q.dig = out.dig; q.S = out.S; q.qs = out.qs; q.zp = out.zp;
+        hipLaunchKernelGGL(rows_quant_tiles_kernel, dim3((unsigned)ceil_div(F, 4 * kRT), (unsigned)R), dim3(kRT), 0, st, q, g.part, g.NT);
+        RWKV_CHECK_LAUNCH("rows_quant_tiles_kernel");
+        return RWKV_OK;
     } else if (C % 64 == 0 && g.MT <= kSkinnyMT && gx >= kSkinnyPairWgs) {
         g.gx = gx; g.per_xcd = (gx + kXcds - 1) / kXcds;
         const dim3 grid((unsigned)(kXcds * g.per_xcd));
         if (k.stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
         else hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
     } else {
-        const int rc = rows_products(st, 1, &k, tot, R, C, F, ROW_RELU2, nullptr);
-        return rc ? rc : rows_products(st, 1, &r, tot, R, C, C, ROW_STORE_F32, nullptr);
+        int rc = rows_products(st, 1, &k, tot, R, C, F, ROW_RELU2, nullptr);
+        if (!rc) rc = rows_products(st, 1, &r, tot, R, C, C, ROW_STORE_F32, nullptr);
+        if (rc) return rc;
     }
-    RWKV_CHECK_LAUNCH("ffn key and receptance");
-    return RWKV_OK;
+    RWKV_CHECK_LAUNCH("gemm8_skinny_kernel");
+    return rows_quant(st, R, F, k.out, true, range, offset, out, (double *)tot);
 }
 
 int rows_wkv(hipStream_t st, int64_t R, int C, bool sequence, const float *k, const float *v, const float *r,
