@@ -10,6 +10,11 @@
 // per round.  One workgroup of 1024 threads; thread t owns the tokens t, t + 1024, ... (coalesced reads of the
 // logits).  The probabilities stay in registers; of the keys the first kSKeysLds per thread live in LDS and the
 // rest in registers: both arrays in registers would not fit the 128 registers a wave of a 1024-thread workgroup has.
+//
+// Bound: vector instructions of one compute unit (a pass of three thresholds over 50277 tokens is 3 us) and code run once
+// from a cold instruction cache, so passes and code are what is saved.  50277 tokens, typical: 69 us with eight passes from the
+// key's top bits, exp(t) recomputed or spilled, and the temperature's power skipped token by token; 58 us with one pass for
+// the top eight bits, exp(t) kept and t in the key's place, and the power in a block of its own.
 #include "rwkv_common.h"
 #include "rwkv_sample.h"
 
@@ -21,7 +26,9 @@ namespace {
 
 constexpr int kST = 1024;            // threads
 constexpr int kSMaxPer = 52;         // tokens per thread: vocabularies up to 53248
-constexpr int kSFirstBit = 16;       // full passes settle the key's bits down to this one before the first attempt to list the undecided tokens
+// Full passes settle the key's bits down to this one before the first attempt to list the undecided tokens (16, 18, 20: 60, 58
+// and 70 us at 50277 tokens, where the list overflows at 20).
+constexpr int kSFirstBit = 18;
 constexpr int kSList = 2048;         // tokens that share the upper half of the cut's key: finished by one wave
 constexpr int kSKeysLds = 32;        // keys per thread kept in LDS ([k][thread]: conflict-free), 128 KiB
 
@@ -61,7 +68,7 @@ __global__ void __launch_bounds__(kST)
 sample_kernel(SampleArgs a) {
     constexpr int KL = PER < kSKeysLds ? PER : kSKeysLds, KR = PER - KL > 0 ? PER - KL : 1;
     extern __shared__ unsigned key_lds[];            // [KL][kST]
-    __shared__ float scr[3 * (kST / 64)];
+    __shared__ float scr[4 * (kST / 64)];
     __shared__ float wsum[kST / 64];
     __shared__ int s_tok, s_cnt;
     __shared__ unsigned s_prefix;
@@ -106,29 +113,33 @@ sample_kernel(SampleArgs a) {
         }
         mx = block_max_f(mx, scr);
         // softmax in float32 (typical.py:5); the hardware exponential (about one ulp) is enough here: only a tie at
-        // the edge of the kept set could fall the other way.  p[k] holds t = logit - max until the last pass.
+        // the edge of the kept set could fall the other way.  p[k] holds exp(t), t = logit - max; t itself waits where its
+        // search key will be (both in registers would not fit).
+        unsigned kreg[KR];
+#define RWKV_KEY(k) ((k) < KL ? key_lds[(k) * kST + tid] : kreg[(k) - KL < KR ? (k) - KL : 0])
+#define RWKV_SET_KEY(k, v) { const unsigned v_ = (v); if ((k) < KL) key_lds[(k) * kST + tid] = v_; else kreg[(k) - KL < KR ? (k) - KL : 0] = v_; }   /* (each thread reads back only its own) */
         float z = 0.f;
 #pragma unroll
-        for (int k = 0; k < PER; ++k) { p[k] -= mx; z += __expf(p[k]); }          // exp(-inf) = 0 past the end
+        for (int k = 0; k < PER; ++k) {
+            const float t = p[k] - mx;
+            RWKV_SET_KEY(k, __float_as_uint(t))
+            p[k] = __expf(t);                            // exp(-inf) = 0 past the end
+            z += p[k];
+        }
         z = block_sum_f(z, scr);
         const float rz = 1.0f / z, logz = logf(z);
         // surprise s = -log p = log z - t (no logarithm per token), entropy (nansum: terms with p == 0 are skipped)
         float h = 0.f;
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
-            const float pk = __expf(p[k]) * rz;
-            if (pk > 0.f) h += (logz - p[k]) * pk;
+            p[k] *= rz;
+            if (p[k] > 0.f) h += (logz - __uint_as_float(RWKV_KEY(k))) * p[k];
         }
         h = block_sum_f(h, scr);
         // distance from the entropy as the search key
-        unsigned kreg[KR];
-#define RWKV_KEY(k) ((k) < KL ? key_lds[(k) * kST + tid] : kreg[(k) - KL < KR ? (k) - KL : 0])
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
-            const float pk = __expf(p[k]) * rz;
-            const unsigned key = pk > 0.f ? __float_as_uint(fabsf(logz - p[k] - h)) : 0x7f800000u;   // p == 0: d = inf
-            if (k < KL) key_lds[k * kST + tid] = key; else kreg[k - KL < KR ? k - KL : 0] = key;      // (each thread reads back only its own)
-            p[k] = pk;
+            RWKV_SET_KEY(k, p[k] > 0.f ? __float_as_uint(fabsf(logz - __uint_as_float(RWKV_KEY(k)) - h)) : 0x7f800000u)      // p == 0: d = inf
         }
         // Radix search, most significant bits first, two bits per round: the largest prefix P with mass{key < P} < tau.
         // `below` = mass{key < prefix}.
@@ -156,9 +167,40 @@ sample_kernel(SampleArgs a) {
             if (RWKV_BELOW(t3)) { prefix = c3; below = t3; } else if (RWKV_BELOW(t2)) { prefix = c2; below = t2; }       \
             else if (RWKV_BELOW(t1)) { prefix = c1; below = t1; }                                                        \
         }
-        // After 16 (or 20, 24, 28) bits only the tokens that share those bits with the cut can still decide the rest.
+        // After 14 (or 18, 22, 26, 30) bits only the tokens that share those bits with the cut can still decide the rest.
         // As soon as they fit a list of kSList entries, one wave finishes alone: no pass over all tokens, no barriers.
         int shift = 30;
+        {
+            // One round over four thresholds that settles the top eight bits where the cut lies between 1/8 and 8, as it does
+            // unless the distribution is nearly one token or tau nearly everything; else the rounds start at the top.  (The
+            // sums grow with the threshold, rounding included: the cut does not depend on the thresholds tried before.)
+            constexpr unsigned c1 = 0x3e000000u, c2 = 0x3f000000u, c3 = 0x40000000u, c4 = 0x41000000u;       // 1/8, 1/2, 2, 8
+            float m1 = 0.f, m2 = 0.f, m3 = 0.f, m4 = 0.f;
+#pragma unroll
+            for (int k = 0; k < PER; ++k) {
+                const unsigned key = RWKV_KEY(k);
+                m1 += key < c1 ? p[k] : 0.f;
+                m2 += key < c2 ? p[k] : 0.f;
+                m3 += key < c3 ? p[k] : 0.f;
+                m4 += key < c4 ? p[k] : 0.f;
+            }
+            m1 = wave_sum(m1); m2 = wave_sum(m2); m3 = wave_sum(m3); m4 = wave_sum(m4);
+            __syncthreads();
+            if ((tid & 63) == 0) {
+                scr[tid >> 6] = m1; scr[kST / 64 + (tid >> 6)] = m2; scr[2 * (kST / 64) + (tid >> 6)] = m3; scr[3 * (kST / 64) + (tid >> 6)] = m4;
+            }
+            __syncthreads();
+            float t1 = 0.f, t2 = 0.f, t3 = 0.f, t4 = 0.f;
+#pragma unroll
+            for (int w = 0; w < kST / 64; ++w) {
+                t1 += scr[w]; t2 += scr[kST / 64 + w]; t3 += scr[2 * (kST / 64) + w]; t4 += scr[3 * (kST / 64) + w];
+            }
+            if (RWKV_BELOW(t1) && !RWKV_BELOW(t4)) {
+                if (RWKV_BELOW(t3)) { prefix = c3; below = t3; } else if (RWKV_BELOW(t2)) { prefix = c2; below = t2; }
+                else { prefix = c1; below = t1; }
+                shift = 22;
+            }
+        }
         for (; shift >= kSFirstBit; shift -= 2) RWKV_FULL_ROUND(shift)
         bool listed = false;
         while (shift >= 0) {                           // (uniform) shift = next undecided bit pair
@@ -208,11 +250,15 @@ sample_kernel(SampleArgs a) {
         float q = 0.f;
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
-            float w = (RWKV_KEY(k) <= prefix && p[k] > 0.f) ? p[k] : 0.f;
-            if (a.temp != 1.0f && w > 0.f) w = __powf(w, inv_t);      // hardware log2 / exp2: a few ulp, immaterial for a sampling weight
-            p[k] = w;
-            q += w;
+            p[k] = (RWKV_KEY(k) <= prefix && p[k] > 0.f) ? p[k] : 0.f;
         }
+        if (a.temp != 1.0f) {        // (as one block: skipped token by token it is 50 KB of code to jump through)
+#pragma unroll
+            for (int k = 0; k < PER; ++k)
+                if (p[k] > 0.f) p[k] = __powf(p[k], inv_t);           // hardware log2 / exp2: a few ulp, immaterial for a sampling weight
+        }
+#pragma unroll
+        for (int k = 0; k < PER; ++k) q += p[k];
         // inverse CDF in the order (thread, k): scan of the per-thread sums, then a walk inside one thread's tokens
         float own = q;
         float incl = own;
@@ -267,6 +313,7 @@ sample_kernel(SampleArgs a) {
             __syncthreads();
         }
 #undef RWKV_KEY
+#undef RWKV_SET_KEY
         token = s_tok;
     }
     if (tid == 0) {

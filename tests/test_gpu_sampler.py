@@ -99,6 +99,28 @@ def test_typical_cut_on_a_nearly_flat_distribution(spread, tau):
     assert chi < dof + 5.0 * (2 * dof) ** 0.5 + 10
 
 
+@pytest.mark.parametrize("V,top,spread,tau,lo,hi", [
+    (5000, 0.0, 0.05, 0.6, 0.0, 0.125), (5000, 0.0, 0.3, 0.6, 0.125, 0.5), (50277, 0.0, 1.0, 0.7, 0.5, 2.0),
+    (50277, 0.0, 3.0, 0.95, 2.0, 8.0), (1000, 10.0, 0.0, 0.98, 8.0, 16.0)])
+def test_typical_cut_in_every_range_of_the_first_round(V, top, spread, tau, lo, hi):
+    """The cut's distance from the entropy in each range that the search's first round tells apart, and on both sides of
+    them: a cut set wrongly moves the mean distance of the drawn tokens, known to its standard error."""
+    from rwkvstic_amd import ops
+    g = torch.Generator().manual_seed(V + int(100 * spread))
+    logits = torch.randn(V, generator=g, dtype=torch.float64) * spread
+    logits[0] += top
+    want = O.typical_distribution(logits, 1.0, tau).double()
+    p = torch.softmax(logits, 0)
+    d = (-torch.log(p) + (p * torch.log(p)).sum()).abs()
+    assert lo < float(d[want > 0].max()) < hi
+    n = 4000
+    got = _draws(ops, logits, n, temp=1.0, tau=tau, seed=77)
+    assert int((want[got] == 0).sum()) <= n * 2e-3          # (one borderline token may differ)
+    mean = float((want * d).sum())
+    sigma = float((want * (d - mean) ** 2).sum()) ** 0.5 / n ** 0.5
+    assert abs(float(d[got].mean()) - mean) < 5 * sigma
+
+
 def test_greedy_mode_end_adj_and_determinism():
     from rwkvstic_amd import ops
     g = torch.Generator().manual_seed(3)
