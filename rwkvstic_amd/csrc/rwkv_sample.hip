@@ -14,7 +14,8 @@
 // Bound: vector instructions of one compute unit (a pass of three thresholds over 50277 tokens is 3 us) and code run once
 // from a cold instruction cache, so passes and code are what is saved.  50277 tokens, typical: 69 us with eight passes from the
 // key's top bits, exp(t) recomputed or spilled, and the temperature's power skipped token by token; 58 us with one pass for
-// the top eight bits, exp(t) kept and t in the key's place, and the power in a block of its own.
+// the top eight bits, exp(t) kept and t in the key's place, and the power in a block of its own (60 us with the list started at
+// bit 16 as before).
 #include "rwkv_common.h"
 #include "rwkv_sample.h"
 
@@ -26,9 +27,11 @@ namespace {
 
 constexpr int kST = 1024;            // threads
 constexpr int kSMaxPer = 52;         // tokens per thread: vocabularies up to 53248
-// Full passes settle the key's bits down to this one before the first attempt to list the undecided tokens (16, 18, 20: 60, 58
-// and 70 us at 50277 tokens, where the list overflows at 20).
-constexpr int kSFirstBit = 18;
+// Full passes settle the key's bits down to this one before the first attempt to list the undecided tokens.  It is part of
+// the results: the mass below a threshold is rounded differently when it is the sum of the listed tokens on top of what
+// lies below them, and a cut that moves by one token moves every draw of a seed.  (16, 18, 20: 60, 58 and 70 us at 50277
+// tokens, where the list overflows at 20; 18 changed 8 of 24000 draws.)
+constexpr int kSFirstBit = 16;
 constexpr int kSList = 2048;         // tokens that share the upper half of the cut's key: finished by one wave
 constexpr int kSKeysLds = 32;        // keys per thread kept in LDS ([k][thread]: conflict-free), 128 KiB
 
@@ -167,7 +170,7 @@ sample_kernel(SampleArgs a) {
             if (RWKV_BELOW(t3)) { prefix = c3; below = t3; } else if (RWKV_BELOW(t2)) { prefix = c2; below = t2; }       \
             else if (RWKV_BELOW(t1)) { prefix = c1; below = t1; }                                                        \
         }
-        // After 14 (or 18, 22, 26, 30) bits only the tokens that share those bits with the cut can still decide the rest.
+        // After 16 (or 20, 24, 28) bits only the tokens that share those bits with the cut can still decide the rest.
         // As soon as they fit a list of kSList entries, one wave finishes alone: no pass over all tokens, no barriers.
         int shift = 30;
         {
