@@ -1247,21 +1247,23 @@ __device__ __forceinline__ void prep_layer_part(const DArgs &a, int l, int part,
     const int C = a.m.C;
     const DPrep &p = a.m.prep[l];
     const double *sl = a.state + (size_t)l * 5 * C;
-    const int c = part * kPrepThreads + threadIdx.x;
-    double sq[kLnMats] = {0, 0, 0, 0, 0};
-    float mq[kLnMats] = {0, 0, 0, 0, 0};
-    const bool in = c < C;                              // (C = 768: the second part is half a part)
-    const double sh0 = in ? sl[c] : 0.0, sh1 = in ? sl[(size_t)C + c] : 0.0, b1 = in ? p.ln1_b[c] : 0.0, b2 = in ? p.ln2_b[c] : 0.0;
+    // Past the row's end (C = 768: the second part is half a part) a thread works on the last channel again and counts
+    // for nothing.  The terms are formed without a branch: the compiler joins the product below with the first addition
+    // of the sum (one rounding), which a value from two sides of a branch would rule out and so change the sums' last bits.
+    const bool in = part * kPrepThreads + (int)threadIdx.x < C;
+    const int c = in ? part * kPrepThreads + (int)threadIdx.x : C - 1;
+    double sq[kLnMats];
+    float mq[kLnMats];
+    const double sh0 = sl[c], sh1 = sl[(size_t)C + c], b1 = p.ln1_b[c], b2 = p.ln2_b[c];
 #pragma unroll
     for (int m = 0; m < kLnMats; ++m) {
-        if (!in) continue;
         const bool att = m < 3;
         const double mu = att ? p.att_mix[(size_t)m * C + c] : p.ffn_mix[(size_t)(m - 3) * C + c];
         const double base = (att ? b1 : b2) * mu + (att ? sh0 : sh1) * (1.0 - mu);   // block.py:67,91 without the x term
         const double rg = (double)p.range[m][c];
         const float q = (float)(base * rg);
-        a.m.Q32[((size_t)l * kLnMats + m) * C + c] = q;
-        sq[m] = base * (p.offset[m][c] + 128.0 * rg);
+        if (in) a.m.Q32[((size_t)l * kLnMats + m) * C + c] = q;
+        sq[m] = (in ? base : 0.0) * (p.offset[m][c] + 128.0 * rg);
         mq[m] = fabsf(q);
     }
     prep_block_sum<kLnMats>(sq, scr);

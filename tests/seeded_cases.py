@@ -34,6 +34,54 @@ def draws():
     return out
 
 
+def _models():
+    """Models made of random codes, so that no quantiser has a part in them: (name, model)."""
+    from rwkvstic_amd.model import HipRWKV
+    for L, C, V in ((2, 1024, 1000), (2, 2560, 1000), (1, 5120, 1000)):
+        g = torch.Generator().manual_seed(C)
+        F = 4 * C
+
+        def u(*shape, lo=0.0, hi=1.0, dtype=torch.float64):
+            return (torch.rand(*shape, generator=g) * (hi - lo) + lo).to(dtype)
+
+        tree = {"emb.w": u(V, C, lo=-0.04, hi=0.04, dtype=torch.float32)}
+
+        def mat(prefix, suffix, n_in, n_out):
+            tree[f"{prefix}weight{suffix}"] = torch.randint(0, 256, (n_in, n_out), generator=g, dtype=torch.uint8)
+            tree[f"{prefix}range{suffix}"] = u(n_in, lo=2e-4, hi=6e-4, dtype=torch.float32)
+            tree[f"{prefix}offset{suffix}"] = u(n_in, lo=-0.06, hi=-0.04)
+
+        for ln in ("ln_in", "ln_out") + tuple(f"blocks.{i}.ln{k}" for i in range(L) for k in (1, 2)):
+            tree[ln + ".weight"], tree[ln + ".bias"] = u(C, lo=0.5, hi=1.5), u(C, lo=-0.1, hi=0.1)
+        mat("head.weights.0.", "", C, V)
+        for i in range(L):
+            p = f"blocks.{i}."
+            tree[p + "attmix"], tree[p + "ffnmix"] = u(3, 1, C), u(2, 1, C)
+            tree[p + "time_first"], tree[p + "time_decay"] = u(C, lo=-1.0), -torch.exp(u(C, lo=-5.0))
+            for s in ("", "1", "2"):
+                mat(p + "att.weights.0.", s, C, C)
+            mat(p + "attout.weights.0.", "", C, C)
+            mat(p + "ffnkey.weights.0.", "", C, F)
+            mat(p + "ffnreceptance.weights.0.", "", C, C)
+            mat(p + "ffnvalue.weights.0.", "", F, C)
+        yield str(C), HipRWKV.from_quantized(tree)
+
+
+def _tokens(n, seed):
+    return torch.randint(0, 1000, (n,), generator=torch.Generator().manual_seed(seed)).tolist()
+
+
+def steps():
+    """Logits and state after token steps, one by one."""
+    out = {}
+    for name, m in _models():
+        st = m.emptyState.clone()
+        for i, t in enumerate(_tokens(6, 1)):
+            lg, st = m.forward([t], st)
+            out[f"{name} step {i}"] = _digest(lg, st)
+    return out
+
+
 if __name__ == "__main__":
     sys.path.insert(0, os.getcwd())
     print(json.dumps({name: globals()[name]() for name in sys.argv[1:]}))
