@@ -139,8 +139,7 @@ int rwkv_quantize_u8(rwkv_stream_t stream, const float *weight,
                      int64_t n_out, int64_t n_in,
                      uint8_t *codes, float *range, double *offset);
 
-/* The same codes, ranges and offsets (the offset up to the order in which its
- * fractions are summed), written straight in any of the three layouts: codes
+/* The same codes, ranges and offsets, bit for bit, written straight in any of the three layouts: codes
  * [n_in, n_out], packed (rwkv_pack_u8's) and packed16 (rwkv_pack_m16's); a NULL
  * layout is not written, at least one is.  workspace:
  * rwkv_quantize_workspace_bytes(n_out, n_in) bytes, 8-byte aligned. */

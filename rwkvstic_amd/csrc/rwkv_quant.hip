@@ -82,28 +82,30 @@ quantize_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in,
 }
 
 // ---------------------------------------------------------------------------
-// The same quantiser for callers with a workspace: four launches that cut the matrix both ways, and the codes leave
-// in any of the three layouts straight from the encoding pass.
+// The same quantiser for callers with a workspace: three launches that cut the matrix both ways, and the codes leave
+// in any of the three layouts straight from the encoding pass.  Codes, ranges and offsets have quantize_kernel's bits.
 //
 // Bound: memory (the float32 matrix twice, the second time mostly from the memory-side cache, the codes once per
 // layout).  quantize_kernel walks all rows with one workgroup per 64 channels, 40 workgroups at 2560 channels, and
 // the packed layouts then read its codes back byte by byte.  The seven matrices of a layer of width 2560: 5.14 ms
-// that way, 0.288 ms here (host calls included; the 511 MB at copy rate: 0.108).
+// that way, 0.325 ms here (host calls included; the 511 MB at copy rate: 0.108).  The offsets' serial sums are 0.03 of it, and
+// more where there are few channels for many rows: a head of 768 x 50277 takes 268 us (97 with the fractions added in
+// parallel), the layer of width 5120 1.18 ms (0.88).
 //
 //   quant_minmax_kernel   256 channels x one of the row splits: partial minimum and maximum
 //   quant_scale_kernel    one channel per thread: partials -> lo, range, 1 / range
-//   quant_encode_kernel   128 channels x kEncRows rows at a time: codes, layouts, partial sums of the fractions
-//   quant_offset_kernel   fractions in a fixed order -> offset
+//   quant_encode_kernel   128 channels x kEncRows rows at a time: codes, layouts; in workgroups of its own the offsets
 // ---------------------------------------------------------------------------
 constexpr int kEncRows = 64;            // rows of one LDS tile: 8 blocks of the P8 layout, 4 x 2 of the M16 layout
+constexpr int kChainChannels = 8;       // channels of a workgroup that adds up fractions
 constexpr int kMinMaxSplits = 32;       // enough workgroups at 2560 channels (320); more only lengthens quant_scale_kernel
 
 struct QuantWs {
     float2 *mm;                 // [splits][n_in]
     double *lo, *ran, *inv;     // [n_in] each
-    double *frac;               // [parts][n_in]
     int64_t splits, split_rows; // of the minimum / maximum pass
     int64_t parts, part_rows;   // of the encoding pass: part_rows a multiple of kEncRows
+    int64_t chain_blocks, col_blocks;   // its workgroups: the offsets' first, then col_blocks x parts
     size_t bytes;
 };
 static QuantWs quant_carve(int64_t n_out, int64_t n_in, void *ws) {
@@ -115,6 +117,8 @@ static QuantWs quant_carve(int64_t n_out, int64_t n_in, void *ws) {
     tiles = tiles < 1 ? 1 : tiles > 4 ? 4 : tiles;
     q.part_rows = kEncRows * tiles;
     q.parts = ceil_div(n_out, q.part_rows);
+    q.chain_blocks = round_up(ceil_div(n_in, kChainChannels), 32);
+    q.col_blocks = ceil_div(n_in, 128);
     unsigned char *p = static_cast<unsigned char *>(ws);
     size_t at = 0;
     auto take = [&](int64_t bytes) { unsigned char *r = p + at; at += (size_t)round_up(bytes, 256); return r; };
@@ -122,7 +126,6 @@ static QuantWs quant_carve(int64_t n_out, int64_t n_in, void *ws) {
     q.lo = reinterpret_cast<double *>(take(n_in * 8));
     q.ran = reinterpret_cast<double *>(take(n_in * 8));
     q.inv = reinterpret_cast<double *>(take(n_in * 8));
-    q.frac = reinterpret_cast<double *>(take(q.parts * n_in * 8));
     q.bytes = at;
     return q;
 }
@@ -192,27 +195,100 @@ __device__ __forceinline__ double quotient(double d, double b, double inv) {
 }
 
 // 16 bytes of a packed layout.  They are stored past the caches, which leaves the float32 matrix there for the encoding pass
-// (the seven matrices of a layer of width 2560: 0.315 -> 0.288 ms).
+// (the seven matrices of a layer of width 2560, offsets added in parallel: 0.315 -> 0.288 ms).
 typedef uint32_t Chunk __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int slot8(int lane) { return lane ^ ((lane >> 3) & 6); }
 __device__ __forceinline__ int slot16(int lane, int half) { return lane ^ (((lane >> 3) & 6) | (half << 3)); }
 
+// Offsets of eight channels.  The fractions of a channel are added in quantize_kernel's order, four serial float64 sums over
+// the rows k = 0, 1, 2, 3 (mod 4), so that both give the same bits (an offset that differs in its last bit moves every logit of
+// a model by rounding, and with it seeded texts).  Bound: that chain of n_out / 4 dependent additions.  Three wavefronts form
+// the fractions of 96 rows at a time and leave them in LDS, kChainAhead such tiles requested ahead; the fourth adds, a lane
+// per sum.  These workgroups run beside those that encode (launched first: they take longest).
+constexpr int kChainRows = 96, kChainAhead = 4, kChainStride = kChainRows / 4 + 2;     // (+ 2: 16-byte aligned, fewer bank conflicts)
+constexpr int kChainLds = 2 * 4 * kChainChannels * kChainStride * 8;
+
+__device__ __forceinline__ void quant_offsets(const float *__restrict__ W, int n_out, int n_in, const QuantWs &q, int group, double *lds,
+                                              float *__restrict__ range, double *__restrict__ offset) {
+    constexpr int kChains = 4 * kChainChannels;
+    double (*fr)[kChains][kChainStride] = reinterpret_cast<double (*)[kChains][kChainStride]>(lds);
+    const int tiles = (n_out + kChainRows - 1) / kChainRows;
+    if (threadIdx.x >= 64) {
+        const int pt = threadIdx.x - 64, ch = pt & 7, r = pt >> 3;          // rows r, r + 24, r + 48, r + 72 of a tile
+        const int j = min(group * kChainChannels + ch, n_in - 1);
+        const double lo = q.lo[j], ran = q.ran[j], inv = q.inv[j];
+        const float *col = W + (size_t)r * n_in + j;
+        float x[kChainAhead][4];
+        auto fetch = [&](float (&v)[4], int t) {
+            const int k = t * kChainRows;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)     // past the end: the last row again, counted as zero
+                v[e] = k + kChainRows <= n_out ? col[(size_t)(k + 24 * e) * n_in] : W[(size_t)min(k + 24 * e + r, n_out - 1) * n_in + j];
+        };
+#pragma unroll
+        for (int d = 0; d < kChainAhead; ++d) fetch(x[d], d);
+        for (int t0 = 0; t0 < tiles; t0 += kChainAhead) {
+#pragma unroll
+            for (int d = 0; d < kChainAhead; ++d) {
+                const int t = t0 + d;
+                if (t >= tiles) break;                                      // (uniform)
+                double f[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const double v = quotient((double)x[d][e] - lo, ran, inv);                      // matmul.py:32-34
+                    f[e] = ran > 0.0 && t * kChainRows + 24 * e + r < n_out ? v - trunc(v) : 0.0;   // matmul.py:35 (adding zero changes no bit)
+                }
+                fetch(x[d], t + kChainAhead);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) fr[t & 1][4 * ch + (r & 3)][(r >> 2) + 6 * e] = f[e];
+                __syncthreads();                                            // tile t is there; tile t - 1 has been added
+            }
+        }
+        return;
+    }
+    const int lane = threadIdx.x, chain = lane & (kChains - 1);
+    double sum = 0.0;
+    for (int t = 0; t < tiles; ++t) {
+        __syncthreads();
+        const double2 *v = reinterpret_cast<const double2 *>(fr[t & 1][chain]);
+#pragma unroll
+        for (int i = 0; i < kChainRows / 8; ++i) { const double2 p = v[i]; sum += p.x; sum += p.y; }
+    }
+    const int first = lane & ~3;
+    const double f0 = __shfl(sum, first, 64), f1 = __shfl(sum, first + 1, 64), f2 = __shfl(sum, first + 2, 64), f3 = __shfl(sum, first + 3, 64);
+    const int j = group * kChainChannels + (lane >> 2);
+    if (lane < kChains && (lane & 3) == 0 && j < n_in) {
+        const double fsum = (f0 + f1) + (f2 + f3), ran = q.ran[j];
+        offset[j] = q.lo[j] + (fsum / (double)n_out) * ran;                 // matmul.py:36-37
+        range[j] = (float)ran;                                              // matmul.py:39
+    }
+}
+
 template <bool VEC>
 __global__ void __launch_bounds__(256)
 quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, QuantWs q,
-                    uint8_t *__restrict__ codes, uint8_t *__restrict__ packed, uint8_t *__restrict__ packed16) {
-    __shared__ uint32_t p8[8][256], m16[8][256];
-    __shared__ double fsum[8][128];
+                    uint8_t *__restrict__ codes, uint8_t *__restrict__ packed, uint8_t *__restrict__ packed16,
+                    float *__restrict__ range, double *__restrict__ offset) {
+    __shared__ __align__(16) uint32_t lds[2][8][256];
+    static_assert(kChainLds <= (int)sizeof(lds), "the fractions fit");
+    if (blockIdx.x < q.chain_blocks) {
+        // (workgroups go to the XCDs round robin: the four groups that share a 128-byte line of a row go to the same one)
+        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, group = (slot >> 2) * 32 + xcd * 4 + (slot & 3);
+        if (group * kChainChannels < n_in) quant_offsets(W, (int)n_out, (int)n_in, q, group, reinterpret_cast<double *>(lds), range, offset);
+        return;
+    }
+    uint32_t (*p8)[256] = lds[0], (*m16)[256] = lds[1];
+    const int64_t item = blockIdx.x - q.chain_blocks, col_block = item % q.col_blocks, part = item / q.col_blocks;
     const int cq = threadIdx.x & 31, rg = threadIdx.x >> 5;         // four channels, every eighth row
-    const int64_t j0 = (int64_t)blockIdx.x * 128, j = j0 + 4 * cq;
-    double lo[4], ran[4], inv[4], fr[4];
+    const int64_t j0 = col_block * 128, j = j0 + 4 * cq;
+    double lo[4], ran[4], inv[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int64_t je = min(j + e, n_in - 1);
-        lo[e] = q.lo[je]; ran[e] = q.ran[je]; inv[e] = q.inv[je]; fr[e] = 0.0;
+        lo[e] = q.lo[je]; ran[e] = q.ran[je]; inv[e] = q.inv[je];
     }
-    const int64_t kbeg = (int64_t)blockIdx.y * q.part_rows, kend = min(kbeg + q.part_rows, n_out);
+    const int64_t kbeg = part * q.part_rows, kend = min(kbeg + q.part_rows, n_out);
     const int64_t n_ct8 = (n_out + 7) >> 3, n_kb8 = (n_in + 127) >> 7, n_ct16 = (n_out + 15) >> 4, n_kb16 = (n_in + 63) >> 6;
     const bool words = (n_out & 3) == 0 && (reinterpret_cast<uintptr_t>(codes) & 3) == 0;
     for (int64_t k0 = kbeg; k0 < kend; k0 += kEncRows) {
@@ -231,9 +307,7 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
                     live |= 0x80u << (8 * e);
                     if (ran[e] > 0.0) {
                         const double v = quotient((double)xe[e] - lo[e], ran[e], inv[e]);   // matmul.py:32-34
-                        const double t = trunc(v);
-                        c4 |= (uint32_t)(uint8_t)(int)t << (8 * e);                         // matmul.py:21
-                        fr[e] += v - t;                                                     // matmul.py:35
+                        c4 |= (uint32_t)(uint8_t)(int)v << (8 * e);                         // matmul.py:21
                     }
                 }
             }
@@ -251,10 +325,10 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
             if (packed) {
                 const int64_t ct = (k0 >> 3) + i;
                 if (ct < n_ct8)
-                    __builtin_nontemporal_store(*reinterpret_cast<const Chunk *>(&p8[i][slot8(lane) * 4]), reinterpret_cast<Chunk *>(packed + (ct * n_kb8 + blockIdx.x) * 1024 + lane * 16));
+                    __builtin_nontemporal_store(*reinterpret_cast<const Chunk *>(&p8[i][slot8(lane) * 4]), reinterpret_cast<Chunk *>(packed + (ct * n_kb8 + col_block) * 1024 + lane * 16));
             }
             if (packed16) {
-                const int64_t ct = (k0 >> 4) + (i >> 1), kb = (int64_t)blockIdx.x * 2 + (i & 1);
+                const int64_t ct = (k0 >> 4) + (i >> 1), kb = col_block * 2 + (i & 1);
                 if (ct < n_ct16 && kb < n_kb16)
                     __builtin_nontemporal_store(*reinterpret_cast<const Chunk *>(&m16[i][slot16(lane, i & 1) * 4]), reinterpret_cast<Chunk *>(packed16 + (ct * n_kb16 + kb) * 1024 + lane * 16));
             }
@@ -280,34 +354,6 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
                 }
             }
         }
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) fsum[rg][4 * cq + e] = fr[e];
-    __syncthreads();
-    if (threadIdx.x < 128 && j0 + threadIdx.x < n_in) {
-        double s = 0.0;
-#pragma unroll
-        for (int r = 0; r < 8; ++r) s += fsum[r][threadIdx.x];
-        q.frac[(int64_t)blockIdx.y * n_in + j0 + threadIdx.x] = s;
-    }
-}
-
-__global__ void __launch_bounds__(256)
-quant_offset_kernel(int64_t n_out, int64_t n_in, QuantWs q, float *__restrict__ range, double *__restrict__ offset) {
-    __shared__ double part[4][64];
-    const int jx = threadIdx.x & 63, g = threadIdx.x >> 6;
-    const int64_t j = (int64_t)blockIdx.x * 64 + jx;
-    double s = 0.0;
-    if (j < n_in) {
-#pragma unroll 8
-        for (int p = g; p < (int)q.parts; p += 4) s += q.frac[(int64_t)p * n_in + j];
-    }
-    part[g][jx] = s;
-    __syncthreads();
-    if (g == 0 && j < n_in) {
-        s = (part[0][jx] + part[1][jx]) + (part[2][jx] + part[3][jx]);
-        offset[j] = q.lo[j] + (s / (double)n_out) * q.ran[j];          // matmul.py:36-37
-        range[j] = (float)q.ran[j];                                    // matmul.py:39
     }
 }
 
@@ -459,15 +505,15 @@ int rwkv_quantize_layouts(rwkv_stream_t stream, const float *weight, int64_t n_o
         return set_error(RWKV_ERR_WORKSPACE, "rwkv_quantize_layouts: workspace of %zu bytes needed, %zu given", q.bytes, workspace_bytes);
     const hipStream_t st = (hipStream_t)stream;
     const bool vec = n_in % 4 == 0 && reinterpret_cast<uintptr_t>(weight) % 16 == 0;
-    const dim3 mg((unsigned)ceil_div(n_in, 256), (unsigned)q.splits), eg((unsigned)ceil_div(n_in, 128), (unsigned)q.parts);
-    if (q.parts > 65535)
-        return set_error(RWKV_ERR_SIZE, "rwkv_quantize_layouts: n_out %lld is more than one launch covers", (long long)n_out);
+    const int64_t blocks = q.chain_blocks + q.col_blocks * q.parts;
+    if (blocks >= (1ll << 31))
+        return set_error(RWKV_ERR_SIZE, "rwkv_quantize_layouts: %lld x %lld is more than one launch covers", (long long)n_out, (long long)n_in);
+    const dim3 mg((unsigned)ceil_div(n_in, 256), (unsigned)q.splits), eg((unsigned)blocks);
     if (vec) hipLaunchKernelGGL(quant_minmax_kernel<true>, mg, dim3(256), 0, st, weight, n_out, n_in, q);
     else hipLaunchKernelGGL(quant_minmax_kernel<false>, mg, dim3(256), 0, st, weight, n_out, n_in, q);
     hipLaunchKernelGGL(quant_scale_kernel, dim3((unsigned)ceil_div(n_in, 64)), dim3(64), 0, st, n_in, q);
-    if (vec) hipLaunchKernelGGL(quant_encode_kernel<true>, eg, dim3(256), 0, st, weight, n_out, n_in, q, codes, packed, packed16);
-    else hipLaunchKernelGGL(quant_encode_kernel<false>, eg, dim3(256), 0, st, weight, n_out, n_in, q, codes, packed, packed16);
-    hipLaunchKernelGGL(quant_offset_kernel, dim3((unsigned)ceil_div(n_in, 64)), dim3(256), 0, st, n_out, n_in, q, range, offset);
+    if (vec) hipLaunchKernelGGL(quant_encode_kernel<true>, eg, dim3(256), 0, st, weight, n_out, n_in, q, codes, packed, packed16, range, offset);
+    else hipLaunchKernelGGL(quant_encode_kernel<false>, eg, dim3(256), 0, st, weight, n_out, n_in, q, codes, packed, packed16, range, offset);
     RWKV_CHECK_LAUNCH("quant_encode_kernel");
     return RWKV_OK;
 }
