@@ -1276,97 +1276,162 @@ __global__ void __launch_bounds__(64) wkv_rows_kernel(const WkvRowsArgs a) {
 }
 
 
-// Longer sequences: the recurrence is linear in (aa, bb), so a workgroup sums up a block of NC chunks of kWkvStep steps
-// side by side (32 channels x NC chunk positions), a scan over the chunks in LDS gives every thread the state its chunk
-// starts from, and each writes the outputs of its own steps: one launch, k and v read once (a chunk stays in
-// registers between the two passes).  Sums float32 and exponents float64 as in the serial form.
+// Longer sequences, in one launch and with the same roundings as token by token: sequences of fewer than kWkvChunked steps
+// are one serial recurrence; longer ones are cut into chunks of kWkvChunk steps (the recurrence is linear in (aa, bb)): every
+// chunk's own sums from an empty state in float32, a serial float64 pass over the chunks for the state each of them starts from
+// (a chunk decays its input by e^{n w}; float64 is also what the state keeps), and the steps again from there.  These
+// orders are part of the results: logits that move by rounding move the texts of a seeded sampler.
 //
-// Bound: the chain of one block (loads, kWkvStep + log2 NC exponentials, kWkvStep steps), with many steps its vector
-// instructions; not memory.  2560 channels and 64 / 128 / 256 / 1024 steps: 5.4 / 6.7 / 8.1 / 24.2 us; as three launches
-// (contributions of 32-step chunks, serial prefix, replay) 19.0 / 19.3 / 20.5 / 32.6 us.  16 channels per workgroup for
-// the long forms: twice the compute units at work (32 channels: 34.9 us at 1024 steps).
-constexpr int kWkvScanMin = 6;      // from kWkvScanMin steps on the scan is faster than the serial form (2560 channels: 8 steps 9.0 us serially, 6.0 as a scan; 1.0 us a step)
+// A serial recurrence need not be a chain of exponentials: the exponent pp depends on k alone (an addition and a maximum
+// a step), all factors follow from it side by side, and (aa, bb) are two fused multiply-adds a step.  So SL lanes share a
+// chunk, S steps each: pp and then (aa, bb) are handed from lane to lane in SL - 1 rounds (every lane runs its steps in every
+// round; what it was handed counts from the round in which it is right), and the rest is done by all lanes at once.
+//
+// Bound: vector instructions, some 200 a step.  2560 channels and 24 / 64 / 128 / 256 / 1024 steps: 5.1 / 7.5 / 6.2 / 8.6 /
+// 27.2 us; a thread per channel below 64 steps and three launches from there on, with the same results, 19.6 / 19.3 / 19.1 /
+// 19.8 / 31.0 us; a log-step scan over chunk sums, in another order of additions, 5.8 / 5.6 / 6.3 / 8.0 / 23.3 us.
+constexpr int kWkvSeqMin = 6;       // from here on faster than a thread per channel (1.0 us a step)
+constexpr int kWkvChunk = 32, kWkvChunked = 64;
+// Channels from which on there is a workgroup for every compute unit: blocks of 4 chunks, two workgroups to a unit, beat blocks
+// of 8 (5120 channels, 257 / 512 / 1024 steps: 18.3 / 25.2 / 47.2 against 25.6 / 29.4 / 56.2 us; 2560: 13.8 / 18.3 / 34.6 against
+// 13.3 / 14.6 / 27.2; 16 chunks spill registers: 31 us).
+constexpr int kWkvWide = 4096;
 
-// One block from step tb; FULL: it lies inside the sequence.  (as, bs, p): the state before the block, on return after it.
-template <int NC, int CH, int kWkvStep, bool FULL>
-__device__ __forceinline__ void wkv_scan_block(const WkvRowsArgs &a, int tb, int c, int ch, int j, double wc, double uw,
-                                               float (*sa)[NC][CH], float (*sb)[NC][CH], double (*sp)[NC][CH],
-                                               float &ca, float &cb, double &cp) {
-    const int C = a.C, T = a.R;
-    const int t0 = FULL ? tb + j * kWkvStep : min(tb + j * kWkvStep, T), n = FULL ? kWkvStep : min(kWkvStep, T - t0);
-    auto row = [&](int i) { return (size_t)(FULL ? t0 + i : min(t0 + i, T - 1)) * C + c; };     // past the end: the last row again, unused
-    float kc[kWkvStep], vc[kWkvStep], rc[kWkvStep];
+__device__ __forceinline__ float shfl_from(float v, int lane) { return __shfl(v, lane, 64); }
+__device__ __forceinline__ double shfl_from(double v, int lane) { return __shfl(v, lane, 64); }
+
+// The S steps of one lane: k, v and what the exponents make of them.  FULL: all of them lie inside the sequence.
+template <int S, bool FULL>
+struct WkvSteps {
+    int n;                          // live steps
+    float k[S], v[S], f1[S], f2[S];
+    double w;
+    __device__ __forceinline__ bool on(int i) const { return FULL || i < n; }
+    __device__ __forceinline__ double exponent(double p) const {        // pp after the steps
 #pragma unroll
-    for (int i = 0; i < kWkvStep; ++i) { kc[i] = a.k[row(i)]; vc[i] = a.v[row(i)]; }
-#pragma unroll
-    for (int i = 0; i < kWkvStep; ++i) rc[i] = a.r[row(i)];
-    // the chunk from an empty state, a direct sum: step i contributes e^{k_i + (n - i) w} by the chunk's end
-    double p = -1e30;
-    float as = 0.f, bs = 0.f;
-#pragma unroll
-    for (int i = 0; i < kWkvStep; ++i) p = fmax(p, FULL || i < n ? fma((double)(n - i), wc, (double)kc[i]) : -1e30);
-#pragma unroll
-    for (int i = 0; i < kWkvStep; ++i) {
-        const float f = FULL || i < n ? expf((float)(fma((double)(n - i), wc, (double)kc[i]) - p)) : 0.f;
-        as = fmaf(f, vc[i], as);
-        bs += f;
+        for (int i = 0; i < S; ++i) { const double q = fmax(p + w, (double)k[i] + w); p = on(i) ? q : p; }
+        return p;
     }
-    if (j == 0) {                                        // the state before the block, decayed over the first chunk
-        const double e = cp + (double)n * wc, pn = fmax(e, p);
-        const float f0 = expf((float)(e - pn)), f1 = expf((float)(p - pn));
-        as = f0 * ca + f1 * as; bs = f0 * cb + f1 * bs; p = pn;
-    }
-    sa[0][j][ch] = as; sb[0][j][ch] = bs; sp[0][j][ch] = p;
-    __syncthreads();
-    int buf = 0;
+    __device__ __forceinline__ double factors(double p) {               // as in wkv_step_f32; pp after the steps
 #pragma unroll
-    for (int d = 1; d < NC; d <<= 1, buf ^= 1) {         // inclusive scan: add what ends d chunks earlier, decayed to here
-        if (j >= d) {
-            const int len = FULL ? d * kWkvStep : t0 + n - min(tb + (j - d + 1) * kWkvStep, T);
-            const double e = sp[buf][j - d][ch] + (double)len * wc, pn = fmax(e, p);
-            const float f0 = expf((float)(e - pn)), f1 = expf((float)(p - pn));
-            as = f0 * sa[buf][j - d][ch] + f1 * as;
-            bs = f0 * sb[buf][j - d][ch] + f1 * bs;
-            p = pn;
+        for (int i = 0; i < S; ++i) {
+            const double s = p + w, r = (double)k[i] + w, d2 = s - r;
+            const float f = expf(-fabsf((float)d2));
+            f1[i] = d2 >= 0.0 ? 1.f : f; f2[i] = d2 >= 0.0 ? f : 1.f;
+            p = on(i) ? fmax(s, r) : p;
         }
-        sa[buf ^ 1][j][ch] = as; sb[buf ^ 1][j][ch] = bs; sp[buf ^ 1][j][ch] = p;
+        return p;
+    }
+    __device__ __forceinline__ void sums(float &aa, float &bb) const {  // (aa, bb) after the steps
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            const float x = fmaf(f1[i], aa, f2[i] * v[i]), y = fmaf(f1[i], bb, f2[i]);
+            aa = on(i) ? x : aa; bb = on(i) ? y : bb;
+        }
+    }
+};
+
+// One block from step tb on: NCH chunks of SL lanes x S steps for each of CH channels.  CHUNKED: (ca, cb, cp) is the float64
+// state before the block, on return after it; else the block is the whole sequence, and the state comes back in the last lane
+// of every channel.
+template <int CH, int SL, int S, int NCH, bool CHUNKED, bool FULL>
+__device__ __forceinline__ void wkv_seq_block(const WkvRowsArgs &a, int tb, int c, double w, double u, double (*sh)[NCH][CH],
+                                              double &ca, double &cb, double &cp) {
+    const int C = a.C, R = a.R;
+    const int ch = threadIdx.x % CH, pos = threadIdx.x / CH, slot = pos % SL, lane = threadIdx.x & 63;
+    // (a wavefront is one chunk: its number is uniform)
+    const int chunk = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int t0 = tb + pos * S;
+    WkvSteps<S, FULL> st;
+    st.w = w;
+    st.n = FULL ? S : max(0, min(S, R - t0));
+    float r[S];
+    auto row = [&](int i) { return (size_t)(FULL ? t0 + i : min(t0 + i, R - 1)) * C + c; };     // past the end: the last row again, unused
+#pragma unroll
+    for (int i = 0; i < S; ++i) { st.k[i] = a.k[row(i)]; st.v[i] = a.v[row(i)]; }
+#pragma unroll
+    for (int i = 0; i < S; ++i) r[i] = a.r[row(i)];
+    // what a lane starts from, handed on from the lane before it
+    auto hand_exponent = [&](double p) {
+#pragma unroll
+        for (int j = 1; j < SL; ++j) { const double q = shfl_from(st.exponent(p), lane - CH); p = slot >= j ? q : p; }
+        return p;
+    };
+    auto hand_sums = [&](float &aa, float &bb) {
+#pragma unroll
+        for (int j = 1; j < SL; ++j) {
+            float x = aa, y = bb;
+            st.sums(x, y);
+            x = shfl_from(x, lane - CH); y = shfl_from(y, lane - CH);
+            aa = slot >= j ? x : aa; bb = slot >= j ? y : bb;
+        }
+    };
+    double pp = cp;
+    float aa = (float)ca, bb = (float)cb;
+    if (CHUNKED) {
+        // the chunk's own sums
+        const double lp = st.factors(hand_exponent(-1e30));
+        float la = 0.f, lb = 0.f;
+        hand_sums(la, lb);
+        st.sums(la, lb);
+        if (tb > 0) __syncthreads();                     // the block before has been read
+        if (slot == SL - 1) { sh[0][chunk][ch] = lp; sh[1][chunk][ch] = (double)la; sh[2][chunk][ch] = (double)lb; }
         __syncthreads();
-    }
-    if (j > 0) { as = sa[buf][j - 1][ch]; bs = sb[buf][j - 1][ch]; p = sp[buf][j - 1][ch]; }
-    else { as = ca; bs = cb; p = cp; }
-    ca = sa[buf][NC - 1][ch]; cb = sb[buf][NC - 1][ch]; cp = sp[buf][NC - 1][ch];
+        // the exponents before every chunk; this chunk's factors
+        double p = cp, s_own = 0.0, p_own = 0.0;
+        const int live = FULL ? NCH : (R - tb + SL * S - 1) / (SL * S);
 #pragma unroll
-    for (int i = 0; i < kWkvStep; ++i) {
-        if (FULL || i < n) {                             // wkv_step_f32; the gate's division joins the step's
-            const double dk = p - (double)kc[i];
-            const float d2 = (float)dk, d = (float)(dk - uw);
-            const float e = expf(-fabsf(d)), f = expf(-fabsf(d2));
-            const float e1 = d >= 0.f ? 1.f : e, e2 = d >= 0.f ? e : 1.f;
-            a.out[(size_t)(t0 + i) * C + c] = (e1 * as + e2 * vc[i]) / ((e1 * bs + e2) * (1.f + expf(-rc[i])));
-            const float f1 = d2 >= 0.f ? 1.f : f, f2 = d2 >= 0.f ? f : 1.f;
-            as = f1 * as + f2 * vc[i];
-            bs = f1 * bs + f2;
-            p = fmax(p, (double)kc[i]) + wc;
+        for (int j = 0; j < NCH; ++j) {
+            const int nj = FULL ? SL * S : min(SL * S, R - tb - j * SL * S);
+            const double s = fma((double)nj, w, p), q = fmax(s, sh[0][j][ch]);
+            if (j == chunk) { pp = p; s_own = s; p_own = q; }
+            p = FULL || j < live ? q : p;
+        }
+        cp = p;
+        const double g1 = (double)expf((float)(s_own - p_own)), g2 = (double)expf((float)(sh[0][chunk][ch] - p_own));
+        const double ga = g2 * sh[1][chunk][ch], gb = g2 * sh[2][chunk][ch];
+        __syncthreads();
+        if (slot == SL - 1) { sh[0][chunk][ch] = g1; sh[1][chunk][ch] = ga; sh[2][chunk][ch] = gb; }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) {
+            const double f = sh[0][j][ch], x = fma(f, ca, sh[1][j][ch]), y = fma(f, cb, sh[2][j][ch]);
+            if (j == chunk) { aa = (float)ca; bb = (float)cb; }
+            ca = FULL || j < live ? x : ca; cb = FULL || j < live ? y : cb;
         }
     }
+    pp = hand_exponent(pp);
+    st.factors(pp);
+    hand_sums(aa, bb);
+    const double uw = u + w;
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+        if (st.on(i)) {                                  // wkv_step_f32, its second pair of exponentials taken from above
+            const double d = pp - (uw + (double)st.k[i]);
+            const float e = expf(-fabsf((float)d));
+            const float e1 = d >= 0.0 ? 1.f : e, e2 = d >= 0.0 ? e : 1.f;
+            const float y = fmaf(e1, aa, e2 * st.v[i]) / fmaf(e1, bb, e2);
+            a.out[row(i)] = y * sigmoid_f32(r[i]);
+            aa = fmaf(st.f1[i], aa, st.f2[i] * st.v[i]);
+            bb = fmaf(st.f1[i], bb, st.f2[i]);
+            pp = fmax(pp + w, (double)st.k[i] + w);
+        }
+    }
+    if (!CHUNKED) { ca = (double)aa; cb = (double)bb; cp = pp; }
 }
 
-template <int NC, int CH, int kWkvStep>
-__global__ void __launch_bounds__(NC * CH) wkv_scan_rows_kernel(const WkvRowsArgs a) {
-    __shared__ float sa[2][NC][CH], sb[2][NC][CH];
-    __shared__ double sp[2][NC][CH];
-    // the last round of the scan writes buffer 1: the next block's summaries may enter buffer 0 while it is still read
-    static_assert(NC == 8 || NC == 32, "an odd number of scan rounds");
-    const int ch = threadIdx.x % CH, j = threadIdx.x / CH;
-    const int C = a.C, c = blockIdx.x * CH + ch;               // (C is a multiple of 64)
-    const double wc = a.w[c], uw = a.u[c] + wc;
-    float ca = (float)a.state[c], cb = (float)a.state[C + c];
-    double cp = a.state[2 * C + c];
+template <int CH, int SL, int S, int NCH, bool CHUNKED>
+__global__ void __launch_bounds__(CH * SL * NCH) wkv_seq_kernel(const WkvRowsArgs a) {
+    static_assert(CH * SL == 64, "a chunk is a wavefront");
+    __shared__ double sh[CHUNKED ? 3 : 1][NCH][CH];
+    const int ch = threadIdx.x % CH, C = a.C, c = blockIdx.x * CH + ch;        // (C is a multiple of 64)
+    const double w = a.w[c], u = a.u[c];
+    double ca = a.state[c], cb = a.state[C + c], cp = a.state[2 * C + c];
+    constexpr int kBlock = NCH * SL * S;
     int tb = 0;
-    for (; tb + NC * kWkvStep <= a.R; tb += NC * kWkvStep)
-        wkv_scan_block<NC, CH, kWkvStep, true>(a, tb, c, ch, j, wc, uw, sa, sb, sp, ca, cb, cp);
-    if (tb < a.R) wkv_scan_block<NC, CH, kWkvStep, false>(a, tb, c, ch, j, wc, uw, sa, sb, sp, ca, cb, cp);
-    if (j == 0) { a.state[c] = (double)ca; a.state[C + c] = (double)cb; a.state[2 * C + c] = cp; }
+    for (; tb + kBlock <= a.R; tb += kBlock) wkv_seq_block<CH, SL, S, NCH, CHUNKED, true>(a, tb, c, w, u, sh, ca, cb, cp);
+    if (tb < a.R) wkv_seq_block<CH, SL, S, NCH, CHUNKED, false>(a, tb, c, w, u, sh, ca, cb, cp);
+    if ((int)threadIdx.x / CH == (CHUNKED ? 0 : SL - 1)) { a.state[c] = ca; a.state[C + c] = cb; a.state[2 * C + c] = cp; }
 }
 
 // ---------------------------------------------------------------------------
@@ -1881,14 +1946,14 @@ int rows_wkv(hipStream_t st, int64_t R, int C, bool sequence, const float *k, co
         if (a.pend[i].tot && (sequence || a.pend[i].op != ROW_STORE_F32))
             return set_error(RWKV_ERR_ARG, "rows_wkv: a pending product needs batch rows and the float32 store tail");
     }
-    if (sequence && R >= kWkvScanMin) {
-        // the smallest block that covers the sequence leaves the fewest threads idle
-        const dim3 g32((unsigned)(C / 32)), g16((unsigned)(C / 16));
-        if (R <= 8 * 8) hipLaunchKernelGGL((wkv_scan_rows_kernel<8, 32, 8>), g32, dim3(8 * 32), 0, st, a);
-        else if (R <= 8 * 16) hipLaunchKernelGGL((wkv_scan_rows_kernel<8, 32, 16>), g32, dim3(8 * 32), 0, st, a);
-        else if (R <= 32 * 8) hipLaunchKernelGGL((wkv_scan_rows_kernel<32, 16, 8>), g16, dim3(32 * 16), 0, st, a);
-        else hipLaunchKernelGGL((wkv_scan_rows_kernel<32, 16, 16>), g16, dim3(32 * 16), 0, st, a);
-        RWKV_CHECK_LAUNCH("wkv_scan_rows_kernel");
+    if (sequence && R >= kWkvSeqMin) {
+        // short sequences: the smallest block that covers them leaves the fewest lanes idle
+        const dim3 g8((unsigned)(C / 8)), g16((unsigned)(C / 16));
+        if (R <= 32) hipLaunchKernelGGL((wkv_seq_kernel<8, 8, 4, 1, false>), g8, dim3(64), 0, st, a);
+        else if (R < kWkvChunked) hipLaunchKernelGGL((wkv_seq_kernel<8, 8, 8, 1, false>), g8, dim3(64), 0, st, a);
+        else if (R <= 4 * kWkvChunk || C >= kWkvWide) hipLaunchKernelGGL((wkv_seq_kernel<16, 4, 8, 4, true>), g16, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((wkv_seq_kernel<16, 4, 8, 8, true>), g16, dim3(512), 0, st, a);
+        RWKV_CHECK_LAUNCH("wkv_seq_kernel");
         return RWKV_OK;
     }
     hipLaunchKernelGGL(wkv_rows_kernel, dim3((unsigned)ceil_div(C, 64), sequence ? 1u : (unsigned)R), dim3(64), 0, st, a);

@@ -693,3 +693,30 @@ def test_a_prompt_equals_its_tokens_one_by_one(T):
     assert float((lg - l1).norm() / l1.norm()) < 5e-6
     for row in range(5):
         assert float((sp[:, row] - st[:, row]).norm() / st[:, row].norm()) < 5e-6, row
+
+
+# both sides of the serial kernels' sizes: a thread per channel below 6 steps, blocks of 32 and of 63 steps
+@pytest.mark.parametrize("T", [4, 5, 6, 8, 9, 31, 32, 33, 48, 63])
+def test_a_short_prompt_has_the_bits_of_its_tokens_one_by_one(T):
+    """Below 64 tokens the recurrence is one serial float32 chain, however it is shared out; everything else of a prompt is
+    exact integers or the same float64 sums for any number of rows."""
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"prompt of {T} tokens, bits of single tokens")
+    m = HipRWKV(synth.make_state_dict(2, 128, V=300, seed=9, ln="random"))
+    toks = synth.random_tokens(T + 3, V=300, seed=T)
+    _, st = m.forward(toks[:1], m.emptyState.clone())
+    lg, sp = m.forward(toks[1:T + 1], st.clone())
+    for t in toks[1:T + 1].tolist():
+        l1, st = m.forward([t], st)
+    assert torch.equal(sp, st) and torch.equal(lg, l1)
+
+
+# one chunk past the serial sizes, ragged chunks, one and several blocks of 4 and of 8 chunks
+@pytest.mark.parametrize("C,T", [(128, 64), (128, 129), (128, 257), (128, 700), (4160, 65), (4160, 300)])
+def test_long_prompts_keep_float64_sums_between_their_chunks(C, T):
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"float64 state after a prompt of {T} tokens at C={C}")
+    m = HipRWKV(synth.make_state_dict(1, C, C, V=100, seed=9, ln="random"))
+    _, st = m.forward(synth.random_tokens(T, V=100, seed=T), m.emptyState.clone())
+    for row in (2, 3):                                  # aa, bb: sums of float32 parts weighted in float64
+        assert bool((st[0, row].float().double() != st[0, row]).any()), row
