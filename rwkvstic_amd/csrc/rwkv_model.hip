@@ -643,7 +643,7 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
                                    sl + C, state_stride, rg2, of2, w.q + 1, &few));
         advance(w.sh2, sl + C);
         const RowsProduct pfk = {w.q[1], L.ffn_k.packed16, w.h, stream}, pfr = {w.q[2], L.ffn_r.packed16, w.kvr, stream};
-        RWKV_TRY(rows_ffn_key_receptance(st, pfk, pfr, w.tot, R, C, F, L.ffn_v.range, L.ffn_v.offset, w.q[0]));
+        RWKV_TRY(rows_ffn_key_receptance(st, sequence, pfk, pfr, w.tot, R, C, F, L.ffn_v.range, L.ffn_v.offset, w.q[0]));
         const RowsProduct pfv = {w.q[0], L.ffn_v.packed16, x, stream};
         // (the ffn receptance stays in the kvr slab and the totals untouched until the next LayerNorm kernel has run)
         RWKV_TRY(rows_products(st, 1, &pfv, w.tot, R, F, C, ROW_GATE_ADD, kvr32, defer ? &few.add : nullptr));

@@ -74,7 +74,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
                   const float *gate, RowsDeferred *defer = nullptr);
 // ffn key (relu squared) [R, C] x [C, F] and ffn receptance [R, C] x [C, C], both stored float32, and the key's rows quantised
 // for the ffn value matrix (range, offset -> out); tot as for either.
-int rows_ffn_key_receptance(hipStream_t st, const RowsProduct &k, const RowsProduct &r, long long *tot, int64_t R, int64_t C, int64_t F,
+int rows_ffn_key_receptance(hipStream_t st, bool sequence, const RowsProduct &k, const RowsProduct &r, long long *tot, int64_t R, int64_t C, int64_t F,
                             const float *range, const double *offset, const RowsOperand &out);
 // kvr (null, or 3 entries, batch rows only): k, v, r still pending as split products (ROW_STORE_F32) where tot is set.
 int rows_wkv(hipStream_t st, int64_t R, int C, bool sequence, const float *k, const float *v, const float *r,

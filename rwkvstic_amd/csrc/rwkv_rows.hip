@@ -30,9 +30,11 @@ constexpr int kRW = kRT / 64;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-// Sums and maxima over a wavefront without the LDS crossbar: four exchanges inside rows of 16 lanes (DPP: neighbour,
-// pair, half row, row), then the four rows' results through scalar registers.  Every lane ends with the same value.  (A
-// butterfly of 64-bit shuffles is twelve dependent trips through LDS; the row kernels are chains of such reductions.)
+// Sums and maxima over a wavefront without the LDS crossbar (a butterfly of 64-bit shuffles is twelve dependent trips
+// through LDS; the row kernels are chains of such reductions).  Every lane ends with the same value.  The sum is that of the
+// butterfly, lanes 32, 16, 8, 4, 2, 1 apart in this order: its last bit reaches the logits, and with them the texts of a
+// seeded sampler.  Halves and rows of 16 lanes change places by permlane swaps, and inside a row DPP rotations stand for the
+// butterfly's steps, since what lanes 8 and then 4 apart have just added up repeats with that period.
 template <int CTRL>
 __device__ __forceinline__ double dpp64(double v) {
     const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
@@ -41,16 +43,22 @@ __device__ __forceinline__ double dpp64(double v) {
 }
 template <int CTRL>
 __device__ __forceinline__ float dpp32(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false)); }
-constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
-__device__ __forceinline__ double lane64(double v, int l) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l), __builtin_amdgcn_readlane(__double2loint(v), l));
-}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140, kDppRor4 = 0x124, kDppRor8 = 0x128;
 __device__ __forceinline__ double wsum(double v) {
-    v += dpp64<kDppXor1>(v);
+    {
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+        v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    }
+    {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+        v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    }
+    v += dpp64<kDppRor8>(v);
+    v += dpp64<kDppRor4>(v);
     v += dpp64<kDppXor2>(v);
-    v += dpp64<kDppHalfMirror>(v);
-    v += dpp64<kDppMirror>(v);
-    return (lane64(v, 0) + lane64(v, 16)) + (lane64(v, 32) + lane64(v, 48));
+    return v + dpp64<kDppXor1>(v);
 }
 __device__ __forceinline__ float wmaxf(float v) {
     v = fmaxf(v, dpp32<kDppXor1>(v));
@@ -246,9 +254,8 @@ __device__ __forceinline__ void lsum(double (&v)[N], double *red /*[N*kLW]*/) {
     __syncthreads();
 }
 
-// Sum of N values per thread over the nw <= 16 wavefronts of the workgroup (fixed order), broadcast; red[N * 16] is used
-// by no other reduction, so one barrier does.  Every wavefront adds up the wavefronts' sums for itself: each row of 16
-// lanes reads them side by side.
+// Sum of N values per thread over the nw <= 8 wavefronts of the workgroup (fixed order, that of lsum), broadcast; red[N * 8]
+// is used by no other reduction, so one barrier does.
 __device__ __forceinline__ double row16_sum(double v) {
     v += dpp64<kDppXor1>(v);
     v += dpp64<kDppXor2>(v);
@@ -267,11 +274,16 @@ __device__ __forceinline__ void bsum(double (&v)[N], double *red, int nw) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         const double s = wsum(v[i]);
-        if (lane == 0) red[i * 16 + wave] = s;
+        if (lane == 0) red[i * 8 + wave] = s;
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = row16_sum((lane & 15) < nw ? red[i * 16 + (lane & 15)] : 0.0);
+    for (int i = 0; i < N; ++i) {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) s += w < nw ? red[i * 8 + w] : 0.0;
+        v[i] = s;
+    }
 }
 __device__ __forceinline__ void ld4(double (&v)[4], const double *p) {
     const double2 a = *reinterpret_cast<const double2 *>(p), b = *reinterpret_cast<const double2 *>(p + 2);
@@ -290,8 +302,8 @@ __device__ __forceinline__ void st4(double *p, const double (&v)[4]) {
 // The same for fewer than kRowsDeferMax rows, where one row's chain of dependent steps is the whole kernel.  Most of it is
 // instruction fetch: a launch begins with cold instruction caches and runs straight through code it uses once, so the three
 // mixes are not unrolled into one workgroup but go to workgroups of their own (blockIdx.y), which take the row's statistics
-// each for themselves.  As many threads as the row has groups of four channels (above 4096 channels half as many), all
-// loads requested before the first reduction.
+// each for themselves.  A thread per group of four channels, at most 512 (the sums' order: wider rows give a thread two or three
+// groups, 2048 channels apart), all loads requested before the first reduction.
 //
 // The workgroups of a row may not write what the others still read.  So the row's new x (a residual update that a split
 // product left pending is applied here) goes to x_out, another buffer than x, and its newest shift row to shift_out; the next
@@ -299,9 +311,10 @@ __device__ __forceinline__ void st4(double *p, const double (&v)[4]) {
 //
 // 8 rows of 2560 channels, three / two mixes: 8.4 / 8.5 us, 32 rows of 5120 15.8 / 15.0 us (one workgroup of 512 threads for
 // the row and all its mixes: 11.1 / 9.7 and 19.6 / 15.4; the same with every parameter vector requested ahead: no faster).
-template <bool MIX, int NSEG, int MAXT>
-__global__ void __launch_bounds__(MAXT) rows_ln_mix_quant_row_kernel(const LnQuantArgs a) {
-    __shared__ double red0[2 * 16], red1[2 * 16], red2[16], red3[16];
+constexpr int kLnRowThreads = 512;
+template <bool MIX, int NSEG>
+__global__ void __launch_bounds__(kLnRowThreads) rows_ln_mix_quant_row_kernel(const LnQuantArgs a) {
+    __shared__ double red0[2 * 8], red1[2 * 8], red2[8], red3[8];
     __shared__ float redf[16];
     const int t = blockIdx.x, m = blockIdx.y, C = a.C, tid = threadIdx.x, nt = blockDim.x, nw = nt >> 6, lane = tid & 63;
     const bool need_prev = MIX && a.sequence && t > 0;
@@ -695,6 +708,7 @@ struct GemmArgs {
     // NT2 > 0: the launch holds two products of different widths (same rows, same contraction, not split): product 1 has
     // NT2 tiles, N2 columns and tail2, and its workgroups follow product 0's
     int NT2, N2, tail2;
+    int apart, apart2;              // few rows: round y as rows_finish_kernel does (see rounded_apart)
     // part non-null (few rows, product 0 with the relu^2 tail): what the quantiser of its result needs of every row and column
     // tile, {max |xs|, zero-point share} at [row][tile], and qs of the operand to be, cleared
     double2 *part;
@@ -704,7 +718,7 @@ struct GemmArgs {
 };
 // Columns and tail of the product a workgroup works for (kept apart from the arguments: a modified copy of those would
 // live in scratch memory).
-struct GemmCols { int NT, N, tail; };
+struct GemmCols { int NT, N, tail; bool apart = false; };
 
 // Weights of the few-row kernels.  STREAM: past the caches, which keeps the digits and the next kernels' vectors there: 8
 // sequences at 3B 2.25 -> 2.08 ms a step, at 14B 5.75 -> 5.30; 32 sequences (9..32-row kernel) 3.20 -> 3.15 and 6.66 -> 6.59.  Of a
@@ -740,7 +754,7 @@ __device__ __forceinline__ void dma16_stream(const v4i *g, unsigned lds_byte_off
 // compiler: element by element each of them waited for a round trip).  1024 tokens at width 2560, before and after: k, v, r
 // 75.5 and 71.8 us, ffn key 93.1 and 89.4, att output and ffn receptance 35.1 and 30.2 (median), ffn value 94.8 and 87.7.
 template <int TAIL, int GM, int GN>
-__device__ __forceinline__ void gemm_tail(const GemmArgs &a, int N, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat, int lane) {
+__device__ __forceinline__ void gemm_tail(const GemmArgs &a, int N, bool apart, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat, int lane) {
     const int g = lane >> 4, n = lane & 15;
     const double *Sv = mat == 0 ? a.S[0] : mat == 1 ? a.S[1] : a.S[2];
     const double *qsv = mat == 0 ? a.qs[0] : mat == 1 ? a.qs[1] : a.qs[2];
@@ -765,7 +779,8 @@ __device__ __forceinline__ void gemm_tail(const GemmArgs &a, int N, const v4i (&
         const int t = 4 * (mt0 + i) + g;
         const bool live = t < a.R;
         const int tc = live ? t : a.R - 1;
-        const double S = Sv[tc], add = 128.0 * (S * qsv[tc]) + zpv[tc];
+        // y = S tot + (128 S q + zp), or with zp added last, as where slices are added up (-0.0 changes nothing)
+        const double S = Sv[tc], sq = 128.0 * (S * qsv[tc]), zp = zpv[tc], add = apart ? sq : sq + zp, last = apart ? zp : -0.0;
 #pragma unroll
         for (int j = 0; j < GN; ++j) {
             const v4i d = acc[i][j];
@@ -773,7 +788,7 @@ __device__ __forceinline__ void gemm_tail(const GemmArgs &a, int N, const v4i (&
             if (exact53) tot = fma(fma(fma((double)d.x, 256.0, (double)d.y), 256.0, (double)d.z), 256.0, (double)d.w);
             else tot = (double)(((((long long)d.x * 256 + d.y) * 256 + d.z) * 256) + d.w);
             const int col = 16 * (nt0 + j) + n;
-            const double y = S * tot + add;
+            const double y = (S * tot + add) + last;
             const size_t o = (size_t)t * N + col;
             if (live && col < N) {
                 if (TAIL == ROW_STORE) outv[o] = y;
@@ -793,11 +808,11 @@ template <int GM, int GN>
 __device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, const GemmCols &cols, const v4i (&acc)[GM][GN], int mt0, int nt0, int mat,
                                               int bz, int lane) {
     switch (cols.tail) {
-        case ROW_STORE: return gemm_tail<ROW_STORE, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
-        case ROW_STORE_F32: return gemm_tail<ROW_STORE_F32, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
-        case ROW_RELU2: return gemm_tail<ROW_RELU2, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
-        case ROW_ADD: return gemm_tail<ROW_ADD, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
-        case ROW_GATE_ADD: return gemm_tail<ROW_GATE_ADD, GM, GN>(a, cols.N, acc, mt0, nt0, mat, lane);
+        case ROW_STORE: return gemm_tail<ROW_STORE, GM, GN>(a, cols.N, cols.apart, acc, mt0, nt0, mat, lane);
+        case ROW_STORE_F32: return gemm_tail<ROW_STORE_F32, GM, GN>(a, cols.N, cols.apart, acc, mt0, nt0, mat, lane);
+        case ROW_RELU2: return gemm_tail<ROW_RELU2, GM, GN>(a, cols.N, cols.apart, acc, mt0, nt0, mat, lane);
+        case ROW_ADD: return gemm_tail<ROW_ADD, GM, GN>(a, cols.N, cols.apart, acc, mt0, nt0, mat, lane);
+        case ROW_GATE_ADD: return gemm_tail<ROW_GATE_ADD, GM, GN>(a, cols.N, cols.apart, acc, mt0, nt0, mat, lane);
         default: break;
     }
     const int g = lane >> 4, n = lane & 15;
@@ -958,10 +973,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     if (bx >= a.gx || bz >= a.gz) return;
     int mat = bz / a.split;
     bz -= mat * a.split;
-    GemmCols cols = {a.NT, a.N, a.tail};
+    GemmCols cols = {a.NT, a.N, a.tail, a.apart != 0};
     if (a.NT2 > 0) {                                    // two products side by side: gx counts the column blocks of both
         const int gx0 = (a.NT + kSkinnyNT - 1) / kSkinnyNT;
-        if (bx >= gx0) { bx -= gx0; mat = 1; cols = GemmCols{a.NT2, a.N2, a.tail2}; }
+        if (bx >= gx0) { bx -= gx0; mat = 1; cols = GemmCols{a.NT2, a.N2, a.tail2, a.apart2 != 0}; }
     }
     const signed char *dig = mat == 0 ? a.dig[0] : mat == 1 ? a.dig[1] : a.dig[2];
     const uint8_t *w16 = mat == 0 ? a.w16[0] : mat == 1 ? a.w16[1] : a.w16[2];
@@ -1101,11 +1116,11 @@ __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int item = blockIdx.x, mat, bz = 0, grp;
     const int groups = (a.NT + NTW - 1) / NTW;
-    GemmCols cols = {a.NT, a.N, a.tail};
+    GemmCols cols = {a.NT, a.N, a.tail, a.apart != 0};
     if (a.NT2 > 0) {                                    // two products of different widths side by side, not split
         mat = item >= groups ? 1 : 0;
         grp = item - mat * groups;
-        if (mat) cols = GemmCols{a.NT2, a.N2, a.tail2};
+        if (mat) cols = GemmCols{a.NT2, a.N2, a.tail2, a.apart2 != 0};
     } else {
         grp = item % groups; item /= groups;
         bz = item % a.split; mat = item / a.split;
@@ -1174,7 +1189,7 @@ __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
 // the fixed-point values is added up with atomics: integers below 2^53, exact in
 // any order.
 __global__ void __launch_bounds__(kRT) rows_quant_tiles_kernel(const QuantArgs a, const double2 *part, int tiles) {
-    __shared__ double red0[16], red1[16];
+    __shared__ double red0[8], red1[8];
     __shared__ float redf[16];
     const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, c0 = 4 * (blockIdx.x * kRT + tid);
     const bool live = c0 < a.K;                            // (whole groups of four lanes: K is a multiple of 64)
@@ -1665,6 +1680,14 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n) {
     if (p.kind != PLAN_SKINNY && p.split == 1 && (int64_t)p.gx * p.gy * n < kGemmLongFillWgs && KB >= kGemmLongBlocks) p.split = 2;
     return p;
 }
+// Which of two roundings a product's y has: one of S (tot + 128 q) + zp, exact but for the last addition, where slices of the
+// contraction are added up by a launch of their own, or S tot + (128 S q + zp) in a product's own epilogue.  Products of at
+// most 32 rows that once were split run whole contractions now and keep the first: the last bit of y reaches the logits, and
+// with them the texts of a seeded sampler.
+static bool rounded_apart(int64_t MT, int64_t NT, int64_t KB, int n) {
+    if (MT > kVecMT) return plan_products(MT, NT, KB, n).split > 1;
+    return KB >= 16 && (NT * n < 128 || (NT * n < 512 && KB >= kGemmLongBlocks));
+}
 // Shape of the few-row kernel for a launch of so many column tiles: tiles per workgroup, wavefronts per workgroup, blocks
 // in flight per wavefront and tile.  All workgroups resident at once, 2000 to 4000 wavefronts where the tiles allow it; one
 // tile per workgroup while that fills the device, more where the digits every wavefront reads would outweigh the weights.
@@ -1761,14 +1784,17 @@ int rows_ln_mix_quant(hipStream_t st, int n_mix, int64_t R, int C, bool sequence
     // rows resident per compute unit
     const bool many = R >= kRowsDeferMax;
     if (!many) {
-        const int nseg = C <= 4 * 1024 ? 1 : 2;
-        const dim3 grid((unsigned)R, (unsigned)n_out), block((unsigned)round_up(ceil_div(C, 4 * nseg), 64));
+        const int64_t threads = round_up(ceil_div(C, 4), 64);
+        const dim3 grid((unsigned)R, (unsigned)n_out), block((unsigned)(threads < kLnRowThreads ? threads : kLnRowThreads));
+        const int nseg = (int)ceil_div(C, 4 * kLnRowThreads);           // 1 .. 3 (kLnMaxWidth)
         if (n_mix == 0) {
-            if (nseg == 1) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<false, 1, 1024>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<false, 2, 768>), grid, block, 0, st, a);
+            if (nseg == 1) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<false, 1>), grid, block, 0, st, a);
+            else if (nseg == 2) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<false, 2>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<false, 3>), grid, block, 0, st, a);
         } else {
-            if (nseg == 1) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 1, 1024>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 2, 768>), grid, block, 0, st, a);
+            if (nseg == 1) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 1>), grid, block, 0, st, a);
+            else if (nseg == 2) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 2>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 3>), grid, block, 0, st, a);
         }
         RWKV_CHECK_LAUNCH("rows_ln_mix_quant_row_kernel");
         return RWKV_OK;
@@ -1854,6 +1880,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     g.gz = split * n;
     g.tail = split > 1 ? -1 : op;
     g.NT2 = g.N2 = g.tail2 = 0;
+    g.apart = rounded_apart(g.MT, g.NT, g.KB, n); g.apart2 = 0;
     g.part = nullptr;
     if (pl.kind == PLAN_VEC) {
         g.gx = g.NT; g.gy = 1; g.by_rows = 0; g.per_xcd = 0;
@@ -1894,7 +1921,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
 // Few rows: both in one launch, whole contractions (the receptance's column blocks find room beside the key's; apart they
 // were up to four launches, two of them only adding slices).  With gemv16_kernel's shapes: 8 sequences at 3B 2.96 -> 2.40 ms
 // a step, 32 at 14B 7.38 -> 6.66 ms (its two launches and the receptance's sum of slices: 31.8 + 13.5 + 4.6 us, one launch 37.5).
-int rows_ffn_key_receptance(hipStream_t st, const RowsProduct &k, const RowsProduct &r, long long *tot, int64_t R, int64_t C, int64_t F,
+int rows_ffn_key_receptance(hipStream_t st, bool sequence, const RowsProduct &k, const RowsProduct &r, long long *tot, int64_t R, int64_t C, int64_t F,
                             const float *range, const double *offset, const RowsOperand &out) {
     GemmArgs g;
     const RowsProduct *p[2] = {&k, &r};
@@ -1908,14 +1935,17 @@ int rows_ffn_key_receptance(hipStream_t st, const RowsProduct &k, const RowsProd
     g.tail = ROW_RELU2; g.R = (int)R; g.N = (int)F;
     g.part = nullptr;
     g.NT2 = (int)ceil_div(C, 16); g.N2 = (int)C; g.tail2 = ROW_STORE_F32;
+    g.apart = rounded_apart(g.MT, g.NT, g.KB, 1); g.apart2 = rounded_apart(g.MT, g.NT2, g.KB, 1);
     const int gx = (int)(ceil_div(g.NT, kSkinnyNT) + ceil_div(g.NT2, kSkinnyNT));
     if (C % 64 == 0 && g.MT <= kVecMT && g.KB <= 1024) {
         g.gx = g.NT; g.per_xcd = 0;
-        if (F > 3072) g.part = reinterpret_cast<double2 *>(tot);       // (16 bytes per row and tile: no more than a slice of totals)
+        // (not for the rows of a sequence: the tiles add up the zero-point term in another order than rows_quant does, and the
+        // last bit of it reaches the logits and a seeded sampler's texts)
+        if (F > 3072 && !sequence) g.part = reinterpret_cast<double2 *>(tot);       // (16 bytes per row and tile: no more than a slice of totals)
         g.next_range = range; g.next_offset = offset; g.next_qs = out.qs;
         launch_vec(st, g, k.stream);
         RWKV_CHECK_LAUNCH("gemv16_kernel");
-        if (!g.part) return rows_quant(st, R, F, k.out, true, range, offset, out, nullptr);
+        if (!g.part) return rows_quant(st, R, F, k.out, true, range, offset, out, (double *)tot);
         QuantArgs q;
         q.K = (int)F; q.in = k.out; q.range = range; q.offset = offset; q.dig = out.dig; q.S = out.S; q.qs = out.qs; q.zp = out.zp;
         hipLaunchKernelGGL(rows_quant_tiles_kernel, dim3((unsigned)ceil_div(F, 4 * kRT), (unsigned)R), dim3(kRT), 0, st, q, g.part, g.NT);

@@ -82,6 +82,33 @@ def steps():
     return out
 
 
+def prompts():
+    """Logits and state after prompts of every path's lengths, from a state that is not empty."""
+    out = {}
+    for name, m in _models():
+        _, start = m.forward(_tokens(3, 2), m.emptyState.clone())
+        for T in (4, 5, 6, 8, 9, 24, 32, 33, 63, 64, 65, 77, 127, 128, 300, 513, 1030):
+            lg, st = m.forward(_tokens(T, T), start.clone())
+            out[f"{name} prompt {T}"] = _digest(lg, st)
+    return out
+
+
+def replies():
+    """Sampled answers to prompts, from a checkpoint that is quantised here: 24 layers of 1024 channels."""
+    from rwkvstic_amd import synth
+    from rwkvstic_amd.master import RWKVMaster, typical
+    from rwkvstic_amd.model import HipRWKV
+    m = HipRWKV(synth.iter_tensors(24, 1024, 4096, 50277, seed=11, device="cuda", ln="random"))
+    ma = RWKVMaster(m, m.emptyState, typical)
+    out = {}
+    for s in range(40):
+        torch.manual_seed(s)
+        ma.resetState()
+        ma.loadContext(newctx=synth.random_tokens(77 if s % 2 else 3 + s, seed=s).tolist())
+        out[str(s)] = ma.encode(ma.forward(number=24)["output"])
+    return out
+
+
 if __name__ == "__main__":
     sys.path.insert(0, os.getcwd())
     print(json.dumps({name: globals()[name]() for name in sys.argv[1:]}))
