@@ -526,6 +526,7 @@ struct RowsWs {
     double *x, *kvr, *att, *h, *prev0;
     double *x2, *sh1, *sh2; // fewer than kRowsDeferMax rows: x after a pending update, the two newest shift rows (see RowsFew)
     RowsOperand q[3];       // quantised left operands: q[0] up to n_ffn wide, q[1], q[2] n_embd wide
+    RowsOperand qv;         // ffn value's: the digits of q[0], row constants of its own (see rows_layers)
     long long *tot;
 };
 
@@ -546,7 +547,7 @@ size_t rows_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_
     n += round_up((size_t)R * F * 8, 256);              // h
     n += round_up((size_t)C * 8, 256);                  // prev0
     n += round_up((size_t)(R < kRowsDeferMax ? R : kRowsDeferMax - 1) * C * 8, 256) * 3;    // x2, sh1, sh2
-    n += round_up((size_t)R * 8, 256) * 9;              // S, qs, zp of three operands
+    n += round_up((size_t)R * 8, 256) * 12;             // S, qs, zp of four operands
     n += round_up(rows_dig_bytes(R, F), 256) + 2 * round_up(rows_dig_bytes(R, C), 256);
     n += round_up(rows_tot_ws_bytes(R, C, n_wide, n_head), 256);
     return n;
@@ -568,6 +569,8 @@ RowsWs rows_carve(void *ws, int64_t R, int64_t C, int64_t F, int64_t n_wide, int
         w.q[i].zp = (double *)take((size_t)R * 8);
         w.q[i].dig = (signed char *)take(rows_dig_bytes(R, i == 0 ? F : C));
     }
+    w.qv.dig = w.q[0].dig;
+    for (double **b : {&w.qv.S, &w.qv.qs, &w.qv.zp}) *b = (double *)take((size_t)R * 8);
     w.tot = (long long *)take(rows_tot_ws_bytes(R, C, n_wide, n_head));
     return w;
 }
@@ -593,9 +596,19 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     const int C = (int)d.n_embd, F = (int)d.n_ffn, V = (int)d.n_vocab;
     const size_t RC = (size_t)R * C;
     RWKV_TRY(rows_embed(st, tokens, R, V, C, d.emb, d.ln0_w, d.ln0_b, w.x));
-    // Few batch rows: the products split their contraction, and the three whose result goes straight into one
-    // row-wise kernel (k, v, r -> WKV; the two residual updates -> the next LayerNorm) leave the sum of their slices
-    // to that kernel instead of a launch of their own.
+    // Few batch rows: where a product splits its contraction (from 9 rows on), and its result goes straight into one row-wise
+    // kernel (k, v, r -> WKV; the two residual updates -> the next LayerNorm), the sum of the slices is left to that kernel
+    // instead of a launch of its own.
+    //
+    // Several workgroups share a row in the LayerNorm kernel of few rows, one for each mix, and no order holds between them.
+    // What one of them reads another may not write in the same launch:
+    //   x                        the updated x goes to the other of two buffers (few.x_out)
+    //   the shift rows           the newest go aside (few.shift_out); the next launch commits them, for batch rows and a single
+    //                            row; longer sequences read a copy (prev0)
+    //   S, qs, zp of a pending product    ffn value's, which the next layer's first LayerNorm reads while it writes those of k, v
+    //                            and r, are a set of their own (w.qv); att output's are q[0]'s, while ffn key and receptance have
+    //                            q[1] and q[2].  In front of the head one workgroup has the row.
+    // A pending product's totals and gate are written by later launches only.
     const bool stream = weights_streamed(d.n_layer, d.n_embd, d.n_ffn, d.n_vocab);
     const bool defer = !sequence && R < kRowsDeferMax;
     RowsDeferred dk[3];
@@ -613,8 +626,8 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     for (int64_t l = 0; l < d.n_layer; ++l) {
         const rwkv_layer_desc &L = m->layers[l];
         double *sl = state + (size_t)l * 5 * C;
-        // TimeMix (block.py:58-80).  Row 0 of a sequence reads the shift state while the last row replaces it,
-        // hence the copy; a single row is read and written by the same threads, in that order, and needs none.
+        // TimeMix (block.py:58-80).  Row 0 of a sequence reads the shift state while the last row replaces it, hence the copy;
+        // a single row's workgroups all read it, and its newest goes aside instead.
         const bool copy_prev = sequence && R > 1;
         if (copy_prev) RWKV_CHECK_HIP(hipMemcpyAsync(w.prev0, sl, (size_t)C * 8, hipMemcpyDeviceToDevice, st));
         const rwkv_qmat *kvr[3] = {&L.att_k, &L.att_v, &L.att_r};
@@ -643,8 +656,8 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
                                    sl + C, state_stride, rg2, of2, w.q + 1, &few));
         advance(w.sh2, sl + C);
         const RowsProduct pfk = {w.q[1], L.ffn_k.packed16, w.h, stream}, pfr = {w.q[2], L.ffn_r.packed16, w.kvr, stream};
-        RWKV_TRY(rows_ffn_key_receptance(st, sequence, pfk, pfr, w.tot, R, C, F, L.ffn_v.range, L.ffn_v.offset, w.q[0]));
-        const RowsProduct pfv = {w.q[0], L.ffn_v.packed16, x, stream};
+        RWKV_TRY(rows_ffn_key_receptance(st, sequence, pfk, pfr, w.tot, R, C, F, L.ffn_v.range, L.ffn_v.offset, w.qv));
+        const RowsProduct pfv = {w.qv, L.ffn_v.packed16, x, stream};
         // (the ffn receptance stays in the kvr slab and the totals untouched until the next LayerNorm kernel has run)
         RWKV_TRY(rows_products(st, 1, &pfv, w.tot, R, F, C, ROW_GATE_ADD, kvr32, defer ? &few.add : nullptr));
     }

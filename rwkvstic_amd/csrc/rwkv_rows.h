@@ -39,7 +39,7 @@ constexpr int kRowsDeferSlices = 4;     // a contraction split further than this
 // What the LayerNorm kernel of fewer than kRowsDeferMax rows does besides (several workgroups share a row there, and none
 // may overwrite what another reads).
 struct RowsFew {
-    RowsDeferred add;           // a residual update of x still pending (tot null: none); batch rows only
+    RowsDeferred add;           // a residual update of x still pending (tot null: none); batch rows only; with mixes, its S, qs and zp are no output's
     double *x_out;              // where the updated x goes: another buffer than x (null: it is not needed)
     double *shift_out;          // [R, C]: the newest shift rows, instead of the state; needed wherever prev0 is the state itself
     const double *commit_src;   // [R, C]: shift rows left by the launch before (null: none) ...

@@ -1771,6 +1771,10 @@ int rows_ln_mix_quant(hipStream_t st, int n_mix, int64_t R, int C, bool sequence
             return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: pending work needs fewer than %d rows", (int)kRowsDeferMax);
         a.add = few->add; a.x_out = few->x_out; a.shift_out = few->shift_out; a.commit_src = few->commit_src; a.commit_dst = few->commit_dst;
     }
+    // (a row has a workgroup for each mix: none may write what another still reads)
+    for (int k = 0; n_mix > 1 && a.add.tot && k < n_mix; ++k)
+        if (out[k].S == a.add.S || out[k].qs == a.add.qs || out[k].zp == a.add.zp)
+            return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: the row constants of a pending product may not be those of an output");
     if (n_mix > 0 && R < kRowsDeferMax && !a.shift_out && !(sequence && R > 1 && prev0 != shift_dst))
         return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: few rows need their shift rows kept apart");
     a.prev0 = prev0; a.shift_dst = shift_dst; a.prev_stride = prev_stride;

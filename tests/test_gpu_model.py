@@ -522,6 +522,30 @@ def test_batch_steps_of_ragged_and_wide_rows_match_single_steps(C, F, B):
         assert float((states[:, :, row] - singles[:, :, row]).norm() / singles[:, :, row].norm()) < 2e-6, row
 
 
+# so many rows that not all of their workgroups are resident at once, with the ffn value product left pending for the next
+# layer's LayerNorm: 86 rows are 258 workgroups of three mixes, one to a compute unit at 4096 and 5120 channels
+@pytest.mark.parametrize("C,B", [(4096, 86), (4096, 127), (5120, 100), (2560, 127)])
+def test_batch_steps_of_more_rows_than_are_resident_match_single_steps(C, B):
+    from rwkvstic_amd import _native as N
+    import ctypes
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"batch of {B} at C={C}")
+    plan, tot = (ctypes.c_int * 4)(), ctypes.c_size_t()
+    N.check(N.lib().rwkv_gemm8_plan(B, 4 * C, C, 1, plan, ctypes.byref(tot)))
+    assert plan[3] > 1                                  # ffn value is split, so it is handed on
+    m = HipRWKV(synth.iter_tensors(3, C, 4 * C, 100, seed=C + B, device="cuda", ln="random"))
+    states = m.emptyState.repeat(B, 1, 1, 1).contiguous()
+    singles = states.clone()
+    for step in range(2):
+        toks = synth.random_tokens(B, V=100, seed=50 + step)
+        lb, states = m.forward_batch(toks.cuda(), states)
+        for b in range(B):
+            l1, _ = m.forward([int(toks[b])], singles[b])
+            assert float((lb[b] - l1).norm() / l1.norm()) < 2e-6, (step, b)
+    for row in range(5):
+        assert float((states[:, :, row] - singles[:, :, row]).norm() / singles[:, :, row].norm()) < 2e-6, row
+
+
 def test_rwkv_shell_loads_checkpoint_file_and_generates(tmp_path, tiny):
     """RWKV(path) -> RWKVMaster surface (load.py:18,42-47; rwkvMaster.py:28-105) over the HIP model."""
     from rwkvstic_amd.master import RWKV, greedy

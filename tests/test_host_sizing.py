@@ -72,3 +72,32 @@ def test_gemm8_workspace_covers_quantiser_scratch(lib):
             need = T * -(-K // (4 * 256 * 3)) * 16
             fixed = 3 * (-(-T * 8 // 256) * 256) + (-(-(-(-T // 4) * (K // 64) * 1024) // 256) * 256)
             assert lib.rwkv_gemm8_workspace_bytes(T, K, 16) - fixed >= need, (T, K)
+
+
+def test_a_pending_product_keeps_its_row_constants_apart(lib):
+    """Few rows: a row of the LayerNorm kernel has one workgroup per mix, all of which read S, qs and zp of a product handed on
+    unfinished; outputs in the same arrays would be written by one while another still reads.  The call is refused on the
+    host, before anything is launched, for each of the three arrays and each output."""
+    P, i64, D = C.c_void_p, C.c_int64, C.c_void_p
+
+    class Operand(C.Structure):
+        _fields_ = [("dig", P), ("S", P), ("qs", P), ("zp", P)]
+
+    class Deferred(C.Structure):
+        _fields_ = [("tot", P), ("slice", C.c_size_t), ("slices", C.c_int), ("ldd", C.c_int), ("op", C.c_int),
+                    ("S", P), ("qs", P), ("zp", P), ("gate", P)]
+
+    class Few(C.Structure):
+        _fields_ = [("add", Deferred), ("x_out", P), ("shift_out", P), ("commit_src", P), ("commit_dst", P)]
+
+    fn = getattr(lib, "_ZN4rwkv17rows_ln_mix_quantEP12ihipStream_tilibPKdS3_S3_S3_S3_PdlPKPKfPKS3_PKNS_11RowsOperandEPKNS_7RowsFewE")
+    fn.restype, fn.argtypes = C.c_int, [P, C.c_int, i64, C.c_int, C.c_bool, D, D, D, D, D, D, i64, P, P, P, P]
+    ptrs = (P * 3)(16, 16, 16)
+    for n_mix in (2, 3):
+        for k in range(n_mix):
+            for field in ("S", "qs", "zp"):
+                out = (Operand * 3)(*[Operand(16, 1024 * (i + 1), 1024 * (i + 1) + 256, 1024 * (i + 1) + 512) for i in range(3)])
+                few = Few(Deferred(16, 0, 1, 64, 2, 8192, 8448, 8704, None), 32, 48, None, None)     # op 2: ROW_ADD
+                setattr(few.add, field, getattr(out[k], field))
+                assert fn(None, n_mix, 100, 64, False, 64, 16, 16, 16, 16, 16, 320, ptrs, ptrs, C.byref(out), C.byref(few)) == -1
+                assert b"row constants" in lib.rwkv_last_error(), (n_mix, k, field)
