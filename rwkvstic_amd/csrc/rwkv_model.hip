@@ -531,9 +531,9 @@ struct RowsWs {
 };
 
 // n_head > 0: one more product, of a single row with n_head columns (the head after a prompt)
-size_t rows_tot_ws_bytes(int64_t R, int64_t C, int64_t n_wide, int64_t n_head) {
-    const size_t a = rows_tot_bytes(R, n_wide), b = 3 * rows_tot_bytes(R, C);     // k, v, r share a launch
-    const size_t c = n_head > 0 ? rows_tot_bytes(1, n_head) : 0;
+size_t rows_tot_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_head) {
+    const size_t a = rows_tot_bytes(R, n_wide, C), b = 3 * rows_tot_bytes(R, C, F > C ? F : C);     // k, v, r share a launch; ffn value
+    const size_t c = n_head > 0 ? rows_tot_bytes(1, n_head, C) : 0;
     // the quantisers of the att output and of h park their partial records here before the product starts
     const size_t q = rows_quant_scratch_bytes(R, n_wide > C ? n_wide : C);
     const size_t m = a > b ? (a > c ? a : c) : (b > c ? b : c);
@@ -549,7 +549,7 @@ size_t rows_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_
     n += round_up((size_t)(R < kRowsDeferMax ? R : kRowsDeferMax - 1) * C * 8, 256) * 3;    // x2, sh1, sh2
     n += round_up((size_t)R * 8, 256) * 12;             // S, qs, zp of four operands
     n += round_up(rows_dig_bytes(R, F), 256) + 2 * round_up(rows_dig_bytes(R, C), 256);
-    n += round_up(rows_tot_ws_bytes(R, C, n_wide, n_head), 256);
+    n += round_up(rows_tot_ws_bytes(R, C, F, n_wide, n_head), 256);
     return n;
 }
 
@@ -571,7 +571,7 @@ RowsWs rows_carve(void *ws, int64_t R, int64_t C, int64_t F, int64_t n_wide, int
     }
     w.qv.dig = w.q[0].dig;
     for (double **b : {&w.qv.S, &w.qv.qs, &w.qv.zp}) *b = (double *)take((size_t)R * 8);
-    w.tot = (long long *)take(rows_tot_ws_bytes(R, C, n_wide, n_head));
+    w.tot = (long long *)take(rows_tot_ws_bytes(R, C, F, n_wide, n_head));
     return w;
 }
 
@@ -935,7 +935,7 @@ int rwkv_gemm8(rwkv_stream_t stream, int64_t T, int64_t n_in, int64_t n_out, con
 
 size_t rwkv_gemm8_workspace_bytes(int64_t T, int64_t n_in, int64_t n_out) {
     if (T <= 0 || n_in <= 0 || n_out <= 0) return 0;
-    const size_t tot = rows_tot_bytes(T, n_out), qs = rows_quant_scratch_bytes(T, n_in);   // share one area
+    const size_t tot = rows_tot_bytes(T, n_out, n_in), qs = rows_quant_scratch_bytes(T, n_in);   // share one area
     return round_up((size_t)T * 8, 256) * 3 + round_up(rows_dig_bytes(T, n_in), 256) + round_up(tot > qs ? tot : qs, 256);
 }
 
@@ -977,7 +977,7 @@ int rwkv_gemm8_plan(int64_t T, int64_t n_in, int64_t n_out, int n_products, int 
                    "rwkv_gemm8_plan: bad sizes");
     if (n_in % 64) return set_error(RWKV_ERR_SIZE, "rwkv_gemm8_plan: n_in must be a multiple of 64");
     rows_plan_describe(T, n_in, n_out, n_products, plan);
-    *tot_bytes_per_product = rows_tot_bytes(T, n_out);
+    *tot_bytes_per_product = rows_tot_bytes(T, n_out, n_in);
     return RWKV_OK;
 }
 

@@ -46,7 +46,7 @@ struct RowsFew {
     double *commit_dst;         // ... and their place in the state, row stride prev_stride
 };
 size_t rows_dig_bytes(int64_t R, int64_t K);
-size_t rows_tot_bytes(int64_t R, int64_t N);        // integer totals of ONE product (times the products in a launch)
+size_t rows_tot_bytes(int64_t R, int64_t N, int64_t K);     // integer totals of ONE product (times the products in a launch) of a contraction of up to K
 size_t rows_quant_scratch_bytes(int64_t R, int64_t K);   // what rows_quant writes into its scratch area (0: unused)
 // The plan rows_products follows for n products [R, K] x [K, N]: out = {kernel kind, grid x, grid y, splits}.
 void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int out[4]);

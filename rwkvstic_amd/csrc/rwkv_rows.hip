@@ -1718,20 +1718,20 @@ static void launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
 #undef RWKV_VEC
 }
 
-// Upper bound of the splits plan_products chooses for R rows and N columns, whatever the contraction length and
-// the number of products in the launch: a longer contraction only lifts the limit on the split, so the
-// plan for an unbounded one bounds every real one.
-static int gemm_split_bound(int64_t R, int64_t N) {
+// Upper bound of the splits plan_products chooses for R rows, N columns and contractions of up to K, whatever the number of
+// products in the launch.  A longer contraction only lifts the limit on the split, so from 9 rows on the plan for an
+// unbounded one bounds every real one; at most 8 rows split for the length's sake alone, which for no model's is needed.
+static int gemm_split_bound(int64_t R, int64_t N, int64_t K) {
     const int64_t MT = ceil_div(R, 4), NT = ceil_div(N, 16);
     int s = 1;
     for (int n = 1; n <= kRowsMaxProducts; ++n) {
-        const int sp = plan_products(MT, NT, (int64_t)1 << 40, n).split;
+        const int sp = plan_products(MT, NT, MT <= kVecMT ? ceil_div(K, 64) : (int64_t)1 << 40, n).split;
         if (sp > s) s = sp;
     }
     return s;
 }
-size_t rows_tot_bytes(int64_t R, int64_t N) {
-    return (size_t)(ceil_div(R, 4) * 4 * round_up(N, 16) * 8) * (size_t)gemm_split_bound(R, N);
+size_t rows_tot_bytes(int64_t R, int64_t N, int64_t K) {
+    return (size_t)(ceil_div(R, 4) * 4 * round_up(N, 16) * 8) * (size_t)gemm_split_bound(R, N, K);
 }
 // What rows_quant keeps in its scratch area for R rows of K values (0: that shape does not use it).
 // (a few long rows are quantised by several workgroups each, in two launches: one workgroup per row leaves most of the

@@ -65,6 +65,16 @@ def test_split_contractions_are_where_the_grid_is_small(lib):
     assert _plan(lib, 256, 5120, 5120, 1)[0][3] == 1
 
 
+@pytest.mark.parametrize("T", [1, 4, 5, 8])
+def test_few_rows_reserve_the_slices_they_write(lib, T):
+    """At most 8 rows run whole contractions up to 65536, so the totals of one slice are reserved, and those of the slices
+    there are beyond: for a head of 50277 columns eight slices are 13 MB of workspace in every forward call."""
+    for K, N, n in ((5120, 50277, 1), (20480, 5120, 1), (2560, 2560, 3), (65536, 16, 1), (65537 + 63, 16, 1), (4 * 65536, 300, 1)):
+        slice_bytes = -(-T // 4) * 4 * (-(-N // 16) * 16) * 8
+        (kind, gx, gy, split), tot = _plan(lib, T, K, N, n)
+        assert kind == 0 and split == (1 if K <= 65536 else 2 if K <= 2 * 65536 else 4) and tot == split * slice_bytes, (K, N)
+
+
 def test_gemm8_workspace_covers_quantiser_scratch(lib):
     """A few rows of a long contraction are quantised in parts whose records sit in the totals area."""
     for T in (1, 4, 8):
