@@ -133,10 +133,12 @@ __device__ __forceinline__ float wkv_step_f32(double w, double u, float k, float
     return y;
 }
 
-// Whether a model's quantised matrices are too many for the 256 MB Infinity Cache to hold from one token to the next:
-// their loads then go past the caches.  222 MB are faster kept, 242 MB streamed (figures beside back_streamed in
-// rwkv_decode.hip, gemv16_kernel in rwkv_rows.hip).
-constexpr int64_t kStreamWeightBytes = 230000000;
+// Whether a model's quantised matrices are too many for the 256 MiB Infinity Cache to hold from one token to the next: their
+// loads then go past the caches.  Us per token kept / streamed: at 2048 channels 65 / 72 (212 MB), 79 / 88 (245), 105 / 104 (280),
+// 113 / 111 (321); at 2560 56.2 / 57.8 (214), 70.4 / 72.0 (247), 81 / 79 (299); at 4096 66 / 68 (226), 70.2 / 71.6 (251), 81 / 78 (300);
+// at 1024 216 / 218 (242), 252 / 245 (270).  The rows of batches and prompts cross at the same place (2048 channels, 245 MB, 8 and 32
+// sequences: 194 / 205, 269 / 281; figures for larger models beside gemv16_kernel in rwkv_rows.hip).
+constexpr int64_t kStreamWeightBytes = 258000000;
 inline bool weights_streamed(int64_t L, int64_t C, int64_t F, int64_t V) { return L * (5 * C * C + 2 * C * F) + V * C > kStreamWeightBytes; }
 
 // ---- the streaming tile product ---------------------------------------------

@@ -143,10 +143,10 @@ struct DArgs {
 //
 // Two cache policies for the weight loads.  A model that fits the 256 MB Infinity Cache finds part of its weights there
 // again at the next token; of a larger one nothing is left by then, and loads that do not displace what else is cached
-// (exchange words, constants, instructions) are faster.  8 tokens, cached / streamed: 1024 channels and 8, 14, 18 layers
-// (160, 242, 296 MB) 1055 / 1124, 1804 / 1767, 2265 / 2213 us; 768 and 24 layers (222 MB) 2684 / 2745; 1536 and 4, 8
-// layers (200, 322 MB) 747 / 858, 1459 / 1416; 32 layers of 4096 12367 / 11747; 16 tokens of the 3B shape 11696 / 11296
-// (11446 without the helpers' loads), 4 of 14B 11430 / 11169.
+// (exchange words, constants, instructions) are faster.  Where the line lies: weights_streamed.  On both sides of it, 8 tokens,
+// cached / streamed: 1024 channels and 8, 18 layers (160, 296 MB) 1055 / 1124, 2265 / 2213 us; 768 and 24 layers (222 MB) 2684 /
+// 2745; 1536 and 4, 8 layers (200, 322 MB) 747 / 858, 1459 / 1416; 32 layers of 4096 12367 / 11747; 16 tokens of the 3B shape
+// 11696 / 11296 (11446 without the helpers' loads), 4 of 14B 11430 / 11169.
 namespace back_cached {
 #define RWKV_BACK_POLICY ""
 #include "rwkv_decode_back.inc"
@@ -947,7 +947,7 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
 // cores), wavefront 0 finishes the columns.
 // Three workgroup barriers per layer, each followed by a test of the abort word, so that every wavefront leaves
 // after the same barrier.
-template <int NB, int FW>
+template <int NB, int FW, bool STREAM>
 __device__ __forceinline__ void helper_path(const DArgs &a, signed char *dig, v4i *red, double *stat, lds_flag_t *flags,
                                             v4i *stash) {
     constexpr int C = 64 * NB, G = GroupShape<NB>::G, NWG = GroupShape<NB>::NWG;
@@ -987,6 +987,7 @@ __device__ __forceinline__ void helper_path(const DArgs &a, signed char *dig, v4
         const uint8_t *base = gld(&a.m.layers[l].w[MAT_FFN_K]) + ((size_t)(tile0 + NTW * (wv / WPT)) * KB + (size_t)(wv % WPT) * KPW) * 1024 + (tid & 63) * 16;
 #endif
         auto blk = [&](int t, int b) { return (const RWKV_GLOBAL v4i *)(base + ((size_t)t * KB + b) * 1024); };
+        auto weight = [](const RWKV_GLOBAL v4i *p) -> v4i { return STREAM ? __builtin_nontemporal_load(p) : *p; };
         // The helpers' 26 MB per layer are not wanted anywhere for a whole layer: they are requested a few blocks at a
         // time with pauses in between, so that they never stand as one burst in front of the owners' polls, gathers
         // and weight stream.  (`paced` is off for the first layer, before anything runs.)
@@ -994,12 +995,12 @@ __device__ __forceinline__ void helper_path(const DArgs &a, signed char *dig, v4
 #pragma unroll
         for (int i = 0; i < BLDS; ++i) {
             if (paced && i % 3 == 0) asm volatile("s_sleep %0" :: "n"(kHelperPace) : "memory");
-            T[i] = __builtin_nontemporal_load(blk(i, KREG));
+            T[i] = weight(blk(i, KREG));
         }
 #pragma unroll
         for (int i = 0; i < BREG; ++i) {
             if (paced && i % 3 == 0) asm volatile("s_sleep %0" :: "n"(kHelperPace) : "memory");
-            W[i] = __builtin_nontemporal_load(blk(i / KREG, i % KREG));
+            W[i] = weight(blk(i / KREG, i % KREG));
         }
 #pragma unroll
         for (int i = 0; i < BLDS; ++i) stash[(wv * BLDS + i) * 64 + (tid & 63)] = T[i];
@@ -1183,7 +1184,7 @@ __global__ void __launch_bounds__((FW + back_waves(NB)) * 64) decode_kernel(cons
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     if constexpr (HELP) {
         if ((int)blockIdx.x >= GroupShape<NB>::NWG) {          // (uniform for the workgroup)
-            helper_path<NB, FW>(a, dig, red, stat, flags, reinterpret_cast<v4i *>(smem + Lds::STASH_OFFSET));
+            helper_path<NB, FW, STREAM>(a, dig, red, stat, flags, reinterpret_cast<v4i *>(smem + Lds::STASH_OFFSET));
             return;
         }
     }
@@ -1723,19 +1724,20 @@ static int launch_one(hipStream_t st, const DArgs &args, bool with_prep) {
 }
 
 static int launch_step(hipStream_t st, const DArgs &args, bool with_prep) {
-    // (from 2048 channels on a model is larger than the cache from a few layers on)
     const bool stream = weights_streamed(args.m.L, args.m.C, args.m.F, args.m.V);
+#define RWKV_STEP(NB, FW) return stream ? launch_one<NB, FW, true>(st, args, with_prep) : launch_one<NB, FW, false>(st, args, with_prep)
     switch (args.m.C) {
-        case 512: return stream ? launch_one<8, 4, true>(st, args, with_prep) : launch_one<8, 4, false>(st, args, with_prep);
-        case 768: return stream ? launch_one<12, 4, true>(st, args, with_prep) : launch_one<12, 4, false>(st, args, with_prep);
-        case 1024: return stream ? launch_one<16, 4, true>(st, args, with_prep) : launch_one<16, 4, false>(st, args, with_prep);
-        case 1536: return stream ? launch_one<24, 4, true>(st, args, with_prep) : launch_one<24, 4, false>(st, args, with_prep);
-        case 2048: return launch_one<32, 4, true>(st, args, with_prep);
-        case 2560: return launch_one<40, 8, true>(st, args, with_prep);
-        case 4096: return launch_one<64, 4, true>(st, args, with_prep);
-        case 5120: return launch_one<80, 8, true>(st, args, with_prep);
+        case 512: RWKV_STEP(8, 4);
+        case 768: RWKV_STEP(12, 4);
+        case 1024: RWKV_STEP(16, 4);
+        case 1536: RWKV_STEP(24, 4);
+        case 2048: RWKV_STEP(32, 4);
+        case 2560: RWKV_STEP(40, 8);
+        case 4096: RWKV_STEP(64, 4);
+        case 5120: return launch_one<80, 8, true>(st, args, with_prep);        // (one layer alone is 340 MB)
         default: return set_error(RWKV_ERR_SIZE, "decode kernel: n_embd %d not supported", args.m.C);
     }
+#undef RWKV_STEP
 }
 
 int decode_launch(hipStream_t st, const DModel &m, const DecodeBuffers &b, unsigned epoch0,

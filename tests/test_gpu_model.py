@@ -744,3 +744,59 @@ def test_long_prompts_keep_float64_sums_between_their_chunks(C, T):
     _, st = m.forward(synth.random_tokens(T, V=100, seed=T), m.emptyState.clone())
     for row in (2, 3):                                  # aa, bb: sums of float32 parts weighted in float64
         assert bool((st[0, row].float().double() != st[0, row]).any()), row
+
+
+# every width that has both cache policies: layers that fit the cache with a small head and not with a large one
+@pytest.mark.parametrize("C,L,V", [(512, 70, 60000), (768, 30, 50000), (1024, 15, 60000), (1536, 7, 40000), (2048, 3, 60000),
+                                   (2560, 2, 50000), (4096, 1, 20000)])
+def test_weights_kept_in_the_cache_and_read_past_it_give_the_same_bits(C, L, V):
+    """One model, and the same with columns added to its head until it is too large for the cache (258 MB): token steps, a
+    batch step and a prompt give the same state, and the token steps the same first logits."""
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"both cache policies at C={C}, {L} layers")
+    few, mb = 1000, lambda v: (L * 13 * C * C + v * C) / 1e6
+    assert mb(few) < 258 < mb(V)
+    g = torch.Generator(device="cuda").manual_seed(C)
+
+    def u(*shape, lo=0.0, hi=1.0, dtype=torch.float64):
+        return (torch.rand(*shape, generator=g, device="cuda") * (hi - lo) + lo).to(dtype)
+
+    tree = {"emb.w": u(V, C, lo=-0.04, hi=0.04, dtype=torch.float32)}
+
+    def mat(prefix, suffix, n_in, n_out):
+        tree[f"{prefix}weight{suffix}"] = torch.randint(0, 256, (n_in, n_out), generator=g, dtype=torch.uint8, device="cuda")
+        tree[f"{prefix}range{suffix}"] = u(n_in, lo=2e-4, hi=6e-4, dtype=torch.float32)
+        tree[f"{prefix}offset{suffix}"] = u(n_in, lo=-0.06, hi=-0.04)
+
+    for ln in ("ln_in", "ln_out") + tuple(f"blocks.{i}.ln{k}" for i in range(L) for k in (1, 2)):
+        tree[ln + ".weight"], tree[ln + ".bias"] = u(C, lo=0.5, hi=1.5), u(C, lo=-0.1, hi=0.1)
+    mat("head.weights.0.", "", C, V)
+    for i in range(L):
+        p = f"blocks.{i}."
+        tree[p + "attmix"], tree[p + "ffnmix"] = u(3, 1, C), u(2, 1, C)
+        tree[p + "time_first"], tree[p + "time_decay"] = u(C, lo=-1.0), -torch.exp(u(C, lo=-5.0))
+        for s in ("", "1", "2"):
+            mat(p + "att.weights.0.", s, C, C)
+        for name, n_in, n_out in (("attout", C, C), ("ffnkey", C, 4 * C), ("ffnreceptance", C, C), ("ffnvalue", 4 * C, C)):
+            mat(p + name + ".weights.0.", "", n_in, n_out)
+
+    def outputs(m):
+        st = m.emptyState.clone()
+        out = []
+        for t in (3, 700, 9):
+            lg, st = m.forward([t], st)
+            out += [lg[:few], st.clone()]
+        lg, st = m.forward([5, 6, 7, 8, 9, 10, 11, 12, 13, 14], st)
+        lb, sb = m.forward_batch([1, 2, 999], torch.stack([st, st, m.emptyState]))
+        m.check()
+        return out + [st, sb], [lg[:few], lb[:, :few]]
+
+    large = outputs(HipRWKV.from_quantized(tree))
+    tree["emb.w"] = tree["emb.w"][:few]
+    tree["head.weights.0.weight"] = tree["head.weights.0.weight"][:, :few].contiguous()
+    small = outputs(HipRWKV.from_quantized(tree))
+    for a, b in zip(large[0], small[0]):
+        assert torch.equal(a, b)
+    for a, b in zip(large[1], small[1]):                # (a head's width decides where the many-row product rounds: a few float64
+        # roundings of its terms, the zero points' up to C x 0.06 times an input)
+        assert float((a - b).abs().max()) <= 2.0 ** -50 * 8 * float(a.abs().max() + 128 * C * 0.06)
