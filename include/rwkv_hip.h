@@ -338,9 +338,12 @@ size_t rwkv_model_workspace_bytes(const rwkv_model *m, int64_t max_tokens);
  * the reference's empty state (0, 0, 0, 0, -1e30) is valid as is.
  * logits: float64 [V].  Path: T >= 4 with the M16 layout of every matrix and
  * n_embd, n_ffn multiples of 64 takes the many-row (GEMM) kernels; fewer tokens
- * go one at a time through the persistent single-token kernel where
- * rwkv_model_has_fused_step, else as one-row prompts through the many-row
- * kernels, and only without the M16 layout as one launch per phase. */
+ * go one at a time through the persistent single-token kernel where there is
+ * one (rwkv_model_trace_workgroups is not 0), else through the many-row kernels
+ * as a short prompt, and only without the M16 layout as one launch per phase.
+ * Calls recorded into a graph take the many-row kernels whatever T is: the
+ * single-token kernel cannot be replayed.  The same holds for
+ * rwkv_model_decode_greedy; rwkv_model_decode_sample cannot be recorded. */
 int rwkv_model_forward(rwkv_model *m, rwkv_stream_t stream,
                        const int64_t *tokens, int64_t T,
                        double *state, double *logits,

@@ -671,6 +671,15 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
 // phase with float32 sums both in time and in accuracy).
 bool use_rows(const rwkv_model *m, int64_t T) { return rows_supported(m) && (T >= kRowsMin || !m->fused); }
 
+// Whether a call on this stream is being recorded.  The token kernel carries an epoch from the host that must grow with
+// every run, which a recorded launch cannot do: replays would meet their own last exchange words.  Recorded calls of few tokens
+// take the many-row kernels, which keep nothing between runs.
+bool recorded(hipStream_t st) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) { (void)hipGetLastError(); return false; }
+    return status == hipStreamCaptureStatusActive;
+}
+
 // T consecutive tokens of one sequence through the many-row kernels, in chunks of kRowsChunk rows; logits
 // from the last row only.  workspace: as rwkv_model_workspace_bytes(m, T) sizes it.
 int rows_sequence(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t T, double *state, double *logits,
@@ -847,7 +856,7 @@ int rwkv_model_selftest_timeout(rwkv_model *m, rwkv_stream_t stream, double *sta
 size_t rwkv_model_workspace_bytes(const rwkv_model *m, int64_t max_tokens) {
     if (!m || max_tokens <= 0) return 0;
     size_t n = round_up(ws_doubles(m->d.n_embd, m->d.n_ffn) * sizeof(double), 256);
-    if (use_rows(m, max_tokens)) {
+    if (rows_supported(m)) {            // (also where the token kernel serves eager calls: see recorded)
         const int64_t R = max_tokens < kRowsChunk ? max_tokens : kRowsChunk;
         n += rows_ws_bytes(R, m->d.n_embd, m->d.n_ffn, m->d.n_ffn, m->d.n_vocab);
     }
@@ -865,7 +874,8 @@ int rwkv_model_forward(rwkv_model *m, rwkv_stream_t stream, const int64_t *token
     int rc = check_forward_args(m, tokens, state, logits, workspace, workspace_bytes, T, "rwkv_model_forward");
     if (rc) return rc;
     const Workspace w = carve(workspace, m->d.n_embd, m->d.n_ffn);
-    if (use_rows(m, T)) return rows_sequence(m, (hipStream_t)stream, tokens, T, state, logits, workspace);
+    if (use_rows(m, T) || (m->fused && recorded((hipStream_t)stream)))
+        return rows_sequence(m, (hipStream_t)stream, tokens, T, state, logits, workspace);
     for (int64_t t = 0; t < T; ++t) {
         if (m->fused) rc = fused_token(m, (hipStream_t)stream, tokens + t, state, logits);
         else rc = step_token(m, (hipStream_t)stream, tokens + t, state, logits, w, t == T - 1);
@@ -987,14 +997,15 @@ int rwkv_model_decode_greedy(rwkv_model *m, rwkv_stream_t stream, int64_t *token
     if (rc) return rc;
     RWKV_CHECK_ARG(n > 0, "rwkv_model_decode_greedy: n must be positive");
     const Workspace w = carve(workspace, m->d.n_embd, m->d.n_ffn);
-    if (m->fused) {
+    const bool replayed = m->fused && recorded((hipStream_t)stream);
+    if (m->fused && !replayed) {
         if ((rc = fused_epochs(m, (hipStream_t)stream, n))) return rc;
         rc = decode_launch_greedy((hipStream_t)stream, m->dm, m->db, m->epoch, tokens, n, state, logits);
         m->epoch += (unsigned)n * decode_epochs_per_token(m->d.n_layer);
         return rc;
     }
     for (int64_t i = 0; i < n; ++i) {
-        if (use_rows(m, 1)) rc = rows_sequence(m, (hipStream_t)stream, tokens + i, 1, state, logits, workspace);
+        if (use_rows(m, 1) || replayed) rc = rows_sequence(m, (hipStream_t)stream, tokens + i, 1, state, logits, workspace);
         else rc = step_token(m, (hipStream_t)stream, tokens + i, state, logits, w, true);
         if (rc) return rc;
         rc = rwkv_argmax_f64(stream, logits, m->d.n_vocab, tokens + i + 1);

@@ -800,3 +800,40 @@ def test_weights_kept_in_the_cache_and_read_past_it_give_the_same_bits(C, L, V):
     for a, b in zip(large[1], small[1]):                # (a head's width decides where the many-row product rounds: a few float64
         # roundings of its terms, the zero points' up to C x 0.06 times an input)
         assert float((a - b).abs().max()) <= 2.0 ** -50 * 8 * float(a.abs().max() + 128 * C * 0.06)
+
+
+@pytest.mark.parametrize("C,n", [(768, 1), (768, 3), (1024, 1), (128, 1)])
+def test_recorded_token_steps_replay(C, n):
+    """A forward of fewer than four tokens and a greedy loop recorded into a graph and replayed, with eager steps of the same
+    handle between the replays: every replay does what the eager call does from the same state."""
+    from rwkvstic_amd import _native as N
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"recorded steps at C={C}, {n} tokens")
+    m = HipRWKV(synth.make_state_dict(2, C, 4 * C, V=500, seed=C, ln="random"))
+    toks, st, gs = torch.zeros(n, dtype=torch.int64, device="cuda"), m.emptyState.clone(), m.emptyState.clone()
+    out = torch.full((4,), 3, dtype=torch.int64, device="cuda")
+    gl, ws = torch.empty(500, dtype=torch.float64, device="cuda"), m._workspace(n)
+
+    def greedy(state):                                  # (the Python entry point uploads its token)
+        N.check(N.lib().rwkv_model_decode_greedy(m._handle, torch.cuda.current_stream().cuda_stream, out.data_ptr(), 3, state.data_ptr(),
+                                                 gl.data_ptr(), ws.data_ptr(), ws.numel()))
+
+    m.forward(toks, st.clone()); greedy(gs.clone())     # workspaces and code are there
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        lg, _ = m.forward(toks, st)
+        greedy(gs)
+    for i in range(4):
+        toks.copy_(synth.random_tokens(n, V=500, seed=i))
+        s0, g0 = st.clone(), gs.clone()
+        graph.replay()
+        l1, s0 = m.forward(toks, s0)
+        o1, l2, g0 = m.decode_greedy(3, 3, g0)
+        torch.cuda.synchronize()
+        m.check()
+        assert float((lg - l1).norm() / l1.norm()) < 5e-6 and float((gl - l2).norm() / l2.norm()) < 5e-6, i
+        assert out[1:].tolist() == o1.tolist(), i
+        for row in range(5):
+            assert float((st[:, row] - s0[:, row]).norm() / s0[:, row].norm()) < 5e-6, (i, row)
+            assert float((gs[:, row] - g0[:, row]).norm() / g0[:, row].norm()) < 5e-6, (i, row)
