@@ -586,9 +586,18 @@ wkv_f64_ref_kernel(int B, int T, int C, const double *__restrict__ w, const doub
 //
 // Bound: the chain of float64 exponentials (some fifty dependent instructions each) where there are few channels,
 // memory with many.  32 channels per workgroup keep a row's piece at 256 bytes.  2560 channels, 256 steps: 15.4 us
-// against 101 us of the serial kernel, which stays for sequences of fewer than kW64MinT steps: one pass of the scan
-// costs as much as about that many serial steps.
-constexpr int kW64SB = 8, kW64MinT = 12;
+// against 101 us of the serial kernel.
+constexpr int kW64SB = 8;
+
+// The serial kernel stays where it is the faster one: for few steps, since one pass of the scan costs as much as about twelve
+// of them, and for many channels, which hide the chain and leave the scan its threefold instructions.  Us serial / scan, calls
+// included: 10240 channels (of all sequences) and 16, 32 steps 12 / 12, 14 / 12; 40960 and 32, 48: 15 / 18, 26 / 20; 81920 and 48, 64:
+// 30 / 30, 38 / 34; above 64 steps (blocks of 256) 40960 and 100, 128: 47 / 50, 59 / 53; 81920 and 200, 256: 154 / 154, 201 / 163;
+// 163840 and 512: 492 / 596.
+static bool wkv_f64_scanned(int64_t channels, int64_t T) {
+    if (T <= 8 * kW64SB) return T >= 12 + channels / 1600;
+    return channels <= 100000 && T >= channels / 400;
+}
 
 template <int NC>
 __global__ void __launch_bounds__(NC * 32)
@@ -976,7 +985,7 @@ int rwkv_wkv_forward_f64(rwkv_stream_t stream, int64_t B, int64_t T, int64_t C,
     RWKV_CHECK_ARG(w && u && k && v && y && aa && bb && pp, "rwkv_wkv_forward_f64: null pointer");
     RWKV_CHECK_ARG(B > 0 && T > 0 && C > 0 && B * C < (1ll << 31) && T < (1ll << 31), "rwkv_wkv_forward_f64: bad sizes");
     RWKV_CHECK_ALIGN(k, 8); RWKV_CHECK_ALIGN(v, 8); RWKV_CHECK_ALIGN(y, 8);
-    if (T >= kW64MinT && B * ceil_div(C, 32) < (1ll << 31)) {
+    if (wkv_f64_scanned(B * C, T)) {
         const dim3 grid((unsigned)(B * ceil_div(C, 32)));
         // short sequences: 8 chunks cover them and leave fewer threads idle; long ones: 32 chunks per block
         if (T <= 8 * kW64SB)

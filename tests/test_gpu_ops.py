@@ -436,6 +436,16 @@ def test_wkv_forward_f64_reference_convention(ops):
 @pytest.mark.parametrize("T", [1, 11, 12, 63, 64, 65, 255, 256, 257, 600])
 @pytest.mark.parametrize("B,C", [(1, 32), (3, 33)])
 def test_wkv_forward_f64_any_length(ops, B, T, C):
+    _wkv_f64_case(ops, B, T, C)
+
+
+# both sides of the lengths from which so many channels are scanned, and more channels than are scanned at all
+@pytest.mark.parametrize("B,C,T", [(50, 640, 31), (50, 640, 32), (50, 640, 79), (50, 640, 80), (100, 1001, 65), (7, 160, 12)])
+def test_wkv_forward_f64_of_many_channels(ops, B, C, T):
+    _wkv_f64_case(ops, B, T, C)
+
+
+def _wkv_f64_case(ops, B, T, C):
     _say(f"wkv_forward f64 B={B} T={T} C={C}")
     w, u, k, v = (t.double() for t in _wkv_case(B, T, C, seed=T + C))
     g = torch.Generator().manual_seed(T)
