@@ -731,8 +731,8 @@ struct Mm8RefArgs {
 };
 
 // T: float (operators32.cu) or double (operators.cu:58-80, the dispatch of wrapper.cpp:60-77): the type of x, r, y and
-// of the sums.  WIDE: at least 16 columns; narrower matrices are read byte by byte.
-template <typename T, bool WIDE>
+// of the sums.  WIDE: at least 16 columns; narrower matrices are read byte by byte.  LONG: more than 256 rows to a workgroup.
+template <typename T, bool WIDE, bool LONG>
 __global__ void __launch_bounds__(kRefThreads) mm8_ref_kernel(const Mm8RefArgs<T> a) {
     __shared__ T xs[kRefPasses * kRefRowsPass];
     __shared__ T red[kRefThreads / 64][128];
@@ -740,50 +740,55 @@ __global__ void __launch_bounds__(kRefThreads) mm8_ref_kernel(const Mm8RefArgs<T
     const T *x = m == 0 ? a.x[0] : m == 1 ? a.x[1] : a.x[2], *r = m == 0 ? a.r[0] : m == 1 ? a.r[1] : a.r[2];
     const uint8_t *w = m == 0 ? a.w[0] : m == 1 ? a.w[1] : a.w[2];
     const int64_t stride = m == 0 ? a.stride[0] : m == 1 ? a.stride[1] : a.stride[2];
-    const int j0 = blockIdx.y * a.rows_per_split, rows = min(a.rows_per_split, a.n_in - j0);
+    const int j_end = min((int)(blockIdx.y + 1) * a.rows_per_split, a.n_in);
     const int q = tid & 7, row0 = tid >> 3;
     const int c0 = blockIdx.x * 128 + 16 * q;            // this lane's 16 columns
     // the last piece of a row that is not a multiple of 16 columns is read 16 bytes from the row's end (its first
     // columns belong to the piece before and are dropped)
     const int cl = WIDE ? min(c0, a.n_out - 16) : 0;
-    // x and r are requested ahead of the weights: a wavefront's loads return in order
-    const int jx = j0 + min(tid, rows - 1);
-    const T xv = x[jx], rv = r[jx];
     typedef uint32_t Piece __attribute__((ext_vector_type(4), aligned(1)));     // (rows may start anywhere)
-    Piece wv[kRefPasses];
-#pragma unroll
-    for (int p = 0; p < kRefPasses; ++p) {
-        if (p * kRefRowsPass >= rows) break;                            // (uniform)
-        const int j = j0 + min(row0 + p * kRefRowsPass, rows - 1);      // past the end: the last row again, times zero
-        const uint8_t *row = w + (size_t)j * stride + cl;
-        if (WIDE) wv[p] = *reinterpret_cast<const Piece *>(row);
-        else {
-            uint32_t d[4] = {0, 0, 0, 0};
-#pragma unroll
-            for (int e = 0; e < 15; ++e)
-                if (e < a.n_out) d[e >> 2] |= (uint32_t)row[e] << (8 * (e & 3));
-            wv[p] = Piece{d[0], d[1], d[2], d[3]};
-        }
-    }
-    // operators32.cu:33-36 multiplies x[j] * (w * r[j]); here x[j]*r[j] is formed once per row (same rounding as the
-    // reference CPU path, matmul.py:131)
-    xs[tid] = tid < rows ? xv * rv : (T)0;
-    __syncthreads();
     T acc[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = (T)0;
+    for (int j0 = blockIdx.y * a.rows_per_split; j0 < j_end; j0 += kRefPasses * kRefRowsPass) {      // (!LONG: once)
+        const int rows = min(kRefPasses * kRefRowsPass, j_end - j0);
+        // x and r are requested ahead of the weights: a wavefront's loads return in order
+        const int jx = j0 + min(tid, rows - 1);
+        const T xv = x[jx], rv = r[jx];
+        Piece wv[kRefPasses];
 #pragma unroll
-    for (int p = 0; p < kRefPasses; ++p) {
-        if (p * kRefRowsPass >= rows) break;
-        const T xr = xs[row0 + p * kRefRowsPass];
+        for (int p = 0; p < kRefPasses; ++p) {
+            if (p * kRefRowsPass >= rows) break;                            // (uniform)
+            const int j = j0 + min(row0 + p * kRefRowsPass, rows - 1);      // past the end: the last row again, times zero
+            const uint8_t *row = w + (size_t)j * stride + cl;
+            if (WIDE) wv[p] = *reinterpret_cast<const Piece *>(row);
+            else {
+                uint32_t d[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t d = wv[p][i];
-            acc[4 * i] = fma((T)ubyte0(d), xr, acc[4 * i]);
-            acc[4 * i + 1] = fma((T)ubyte1(d), xr, acc[4 * i + 1]);
-            acc[4 * i + 2] = fma((T)ubyte2(d), xr, acc[4 * i + 2]);
-            acc[4 * i + 3] = fma((T)ubyte3(d), xr, acc[4 * i + 3]);
+                for (int e = 0; e < 15; ++e)
+                    if (e < a.n_out) d[e >> 2] |= (uint32_t)row[e] << (8 * (e & 3));
+                wv[p] = Piece{d[0], d[1], d[2], d[3]};
+            }
         }
+        // operators32.cu:33-36 multiplies x[j] * (w * r[j]); here x[j]*r[j] is formed once per row (same rounding as the
+        // reference CPU path, matmul.py:131)
+        xs[tid] = tid < rows ? xv * rv : (T)0;
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < kRefPasses; ++p) {
+            if (p * kRefRowsPass >= rows) break;
+            const T xr = xs[row0 + p * kRefRowsPass];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t d = wv[p][i];
+                acc[4 * i] = fma((T)ubyte0(d), xr, acc[4 * i]);
+                acc[4 * i + 1] = fma((T)ubyte1(d), xr, acc[4 * i + 1]);
+                acc[4 * i + 2] = fma((T)ubyte2(d), xr, acc[4 * i + 2]);
+                acc[4 * i + 3] = fma((T)ubyte3(d), xr, acc[4 * i + 3]);
+            }
+        }
+        if (!LONG) break;
+        __syncthreads();                                     // xs has been read
     }
     // Sum over the 8 rows of the wavefront: at each step a lane keeps one half of its columns and hands the other to
     // the lane that keeps those, so 14 exchanges leave every lane with two of its piece's columns.
@@ -851,11 +856,19 @@ static int mm8_ref_launch(hipStream_t st, int nm, int64_t n_in, int64_t n_out,
     const int64_t cols = ceil_div(n_out, 128);
     a.rows_per_split = kRefPasses * kRefRowsPass;
     if (cols * ceil_div(n_in, a.rows_per_split) < 256) a.rows_per_split = kRefSplitRows;
+    // In float64 the reduction at a workgroup's end is a quarter of its time, so it takes two or four times the rows where enough
+    // workgroups are left (us a call: 2560 x 10240 19.1 -> 14.8, three of them 36.8 -> 26.5, 5120 x 20480 49.5 -> 35.2).
+    const bool wide = n_out >= 16;
+    int64_t more = 1;
+    if (sizeof(T) == 8 && wide) more = cols * ceil_div(n_in, 4 * a.rows_per_split) >= 512 ? 4 : cols * ceil_div(n_in, 2 * a.rows_per_split) >= 256 ? 2 : 1;
+    const bool longer = more > 1;
+    a.rows_per_split *= (int)more;
     a.splits = (int)ceil_div(n_in, a.rows_per_split);
     if (a.splits > 65535) return set_error(RWKV_ERR_SIZE, "mm8: n_in %lld is more than one launch covers", (long long)n_in);
     const dim3 grid((unsigned)cols, (unsigned)a.splits, (unsigned)nm);
-    if (n_out >= 16) hipLaunchKernelGGL((mm8_ref_kernel<T, true>), grid, dim3(kRefThreads), 0, st, a);
-    else hipLaunchKernelGGL((mm8_ref_kernel<T, false>), grid, dim3(kRefThreads), 0, st, a);
+    if (longer) hipLaunchKernelGGL((mm8_ref_kernel<T, true, sizeof(T) == 8>), grid, dim3(kRefThreads), 0, st, a);
+    else if (wide) hipLaunchKernelGGL((mm8_ref_kernel<T, true, false>), grid, dim3(kRefThreads), 0, st, a);
+    else hipLaunchKernelGGL((mm8_ref_kernel<T, false, false>), grid, dim3(kRefThreads), 0, st, a);
     RWKV_CHECK_LAUNCH("mm8_ref_kernel");
     hipLaunchKernelGGL(mm8_ref_reduce_kernel<T>, dim3((unsigned)ceil_div(n_out, 64), (unsigned)nm), dim3(256), 0, st, a);
     RWKV_CHECK_LAUNCH("mm8_ref_reduce_kernel");

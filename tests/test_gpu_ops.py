@@ -237,6 +237,26 @@ def test_mm8_one_edges_against_the_float64_product(ops, n_in, n_out, pad):
         assert ((y.cpu().double() - want).abs() <= steps * eps * mag).all()
 
 
+# float64: 512 and 1024 rows to a workgroup, the last ones ragged, one row into a further round of 256
+@pytest.mark.parametrize("n_in,n_out,pad", [(2049, 8200, 3), (1793, 8321, 0), (5000, 13200, 0), (4097, 16384, 1)])
+def test_mm8_float64_of_long_slices_against_the_exact_product(ops, n_in, n_out, pad):
+    _say(f"mm8 float64 long slices in={n_in} out={n_out}")
+    g = torch.Generator(device="cuda").manual_seed(n_in + n_out)
+    big = torch.randint(0, 256, (n_in, n_out + pad), generator=g, dtype=torch.uint8, device="cuda")
+    x = torch.randn(n_in, generator=g, device="cuda", dtype=torch.float64)
+    r = torch.rand(n_in, generator=g, device="cuda", dtype=torch.float64) * 1e-3
+    y0 = torch.randn(n_out, generator=g, device="cuda", dtype=torch.float64)
+    y, z = y0.clone(), [y0.clone() for _ in range(3)]
+    w = big[:, :n_out]
+    ops.mm8_one(n_in, n_out, x, w, y, r)
+    ops.mm8_three(n_in, n_out, x, x, x, w, w, w, z[0], z[1], z[2], r, r, r)
+    xr, wd = x * r, w.double()
+    # at most 32 products per lane, 3 + 2 additions in the trees, the slices, x * r and y on each side
+    bound = (2 * (32 + 5 + n_in // 512 + 3)) * 2.0 ** -53 * (y0.abs() + xr.abs() @ wd) + n_in * 2.0 ** -53 * (xr.abs() @ wd)
+    assert ((y - (y0 + xr @ wd)).abs() <= bound).all()
+    assert all(torch.equal(t, y) for t in z)
+
+
 def test_mm8_three_matches_three_mm8_one(ops):
     n_in, n_out = 512, 520
     g = torch.Generator().manual_seed(11)
