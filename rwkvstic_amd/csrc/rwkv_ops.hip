@@ -861,12 +861,13 @@ static int mm8_ref_launch(hipStream_t st, int nm, int64_t n_in, int64_t n_out,
     const bool wide = n_out >= 16;
     int64_t more = 1;
     if (sizeof(T) == 8 && wide) more = cols * ceil_div(n_in, 4 * a.rows_per_split) >= 512 ? 4 : cols * ceil_div(n_in, 2 * a.rows_per_split) >= 256 ? 2 : 1;
-    const bool longer = more > 1;
     a.rows_per_split *= (int)more;
+    while (ceil_div(n_in, a.rows_per_split) > 65535) a.rows_per_split *= 2;        // (slices of a grid)
+    const bool longer = a.rows_per_split > kRefPasses * kRefRowsPass;
     a.splits = (int)ceil_div(n_in, a.rows_per_split);
-    if (a.splits > 65535) return set_error(RWKV_ERR_SIZE, "mm8: n_in %lld is more than one launch covers", (long long)n_in);
     const dim3 grid((unsigned)cols, (unsigned)a.splits, (unsigned)nm);
-    if (longer) hipLaunchKernelGGL((mm8_ref_kernel<T, true, sizeof(T) == 8>), grid, dim3(kRefThreads), 0, st, a);
+    if (longer && wide) hipLaunchKernelGGL((mm8_ref_kernel<T, true, true>), grid, dim3(kRefThreads), 0, st, a);
+    else if (longer) hipLaunchKernelGGL((mm8_ref_kernel<T, false, true>), grid, dim3(kRefThreads), 0, st, a);
     else if (wide) hipLaunchKernelGGL((mm8_ref_kernel<T, true, false>), grid, dim3(kRefThreads), 0, st, a);
     else hipLaunchKernelGGL((mm8_ref_kernel<T, false, false>), grid, dim3(kRefThreads), 0, st, a);
     RWKV_CHECK_LAUNCH("mm8_ref_kernel");

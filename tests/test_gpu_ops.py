@@ -257,6 +257,24 @@ def test_mm8_float64_of_long_slices_against_the_exact_product(ops, n_in, n_out, 
     assert all(torch.equal(t, y) for t in z)
 
 
+# one row more than 65535 slices of 256 rows, in whole cache lines of columns and byte by byte
+@pytest.mark.parametrize("n_out", [16, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_mm8_takes_more_rows_than_a_grid_has_slices(ops, n_out, dtype):
+    n_in = 65535 * 256 + 1
+    _say(f"mm8 in={n_in} out={n_out} {dtype}")
+    g = torch.Generator(device="cuda").manual_seed(n_out)
+    w = torch.randint(0, 256, (n_in, n_out), generator=g, dtype=torch.uint8, device="cuda")
+    # a few thousand rows of +-1/4, the first and the last ones among them: sums of multiples of 1/4 below 2^20 are exact
+    rows = torch.unique(torch.cat([torch.randint(0, n_in, (3000,), generator=g, device="cuda"), torch.arange(4, device="cuda"),
+                                   torch.arange(n_in - 600, n_in, device="cuda")]))
+    x = torch.zeros(n_in, dtype=dtype, device="cuda")
+    x[rows] = (torch.randint(0, 2, rows.shape, generator=g, device="cuda") * 2 - 1).to(dtype)
+    y = torch.zeros(n_out, dtype=dtype, device="cuda")
+    ops.mm8_one(n_in, n_out, x, w, y, torch.full((n_in,), 0.25, dtype=dtype, device="cuda"))
+    assert torch.equal(y.double(), (x[rows].double()[:, None] * w[rows].double()).sum(0) * 0.25)
+
+
 def test_mm8_three_matches_three_mm8_one(ops):
     n_in, n_out = 512, 520
     g = torch.Generator().manual_seed(11)
