@@ -2,6 +2,7 @@
 // packed weight layout: pack / unpack / canonical dequantisation.
 #include "rwkv_common.h"
 
+#include <algorithm>
 #include <string>
 
 namespace rwkv {
@@ -101,6 +102,7 @@ quantize_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in,
 constexpr int kOneLaunchRows = 64;
 constexpr int kEncRows = 64;            // rows of one LDS tile: 8 blocks of the P8 layout, 4 x 2 of the M16 layout
 constexpr int kChainChannels = 8;       // channels of a workgroup that adds up fractions
+constexpr int64_t kChainMaxBlocks = 1 << 20;    // such workgroups (a launch has at most 2^32 threads); of more channels each takes several groups
 constexpr int kMinMaxSplits = 32;       // enough workgroups at 2560 channels (320); more only lengthens quant_scale_kernel
 
 struct QuantWs {
@@ -120,7 +122,7 @@ static QuantWs quant_carve(int64_t n_out, int64_t n_in, void *ws) {
     tiles = tiles < 1 ? 1 : tiles > 4 ? 4 : tiles;
     q.part_rows = kEncRows * tiles;
     q.parts = ceil_div(n_out, q.part_rows);
-    q.chain_blocks = round_up(ceil_div(n_in, kChainChannels), 32);
+    q.chain_blocks = std::min(round_up(ceil_div(n_in, kChainChannels), (int64_t)32), kChainMaxBlocks);
     q.col_blocks = ceil_div(n_in, 128);
     unsigned char *p = static_cast<unsigned char *>(ws);
     size_t at = 0;
@@ -277,8 +279,11 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
     static_assert(kChainLds <= (int)sizeof(lds), "the fractions fit");
     if (blockIdx.x < q.chain_blocks) {
         // (workgroups go to the XCDs round robin: the four groups that share a 128-byte line of a row go to the same one)
-        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, group = (slot >> 2) * 32 + xcd * 4 + (slot & 3);
-        if (group * kChainChannels < n_in) quant_offsets(W, (int)n_out, (int)n_in, q, group, reinterpret_cast<double *>(lds), range, offset);
+        for (int64_t b = blockIdx.x; b * kChainChannels < n_in + 32 * kChainChannels; b += q.chain_blocks) {
+            const int64_t xcd = b & 7, slot = b >> 3, group = (slot >> 2) * 32 + xcd * 4 + (slot & 3);
+            if (group * kChainChannels < n_in) quant_offsets(W, (int)n_out, (int)n_in, q, (int)group, reinterpret_cast<double *>(lds), range, offset);
+            __syncthreads();                                        // the last rows of this group have been added
+        }
         return;
     }
     uint32_t (*p8)[256] = lds[0], (*m16)[256] = lds[1];
@@ -511,7 +516,7 @@ int rwkv_quantize_layouts(rwkv_stream_t stream, const float *weight, int64_t n_o
     const hipStream_t st = (hipStream_t)stream;
     const bool vec = n_in % 4 == 0 && reinterpret_cast<uintptr_t>(weight) % 16 == 0;
     const int64_t blocks = q.chain_blocks + q.col_blocks * q.parts;
-    if (blocks >= (1ll << 31))
+    if (blocks >= (1ll << 24))
         return set_error(RWKV_ERR_SIZE, "rwkv_quantize_layouts: %lld x %lld is more than one launch covers", (long long)n_out, (long long)n_in);
     const dim3 mg((unsigned)ceil_div(n_in, 256), (unsigned)q.splits), eg((unsigned)blocks);
     if (vec) hipLaunchKernelGGL(quant_minmax_kernel<true>, mg, dim3(256), 0, st, weight, n_out, n_in, q);

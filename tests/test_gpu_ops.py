@@ -85,6 +85,19 @@ def test_both_quantisers_give_the_same_bits(ops, shape):
     assert torch.equal(codes, c) and torch.equal(rng, r) and torch.equal(off, o)
 
 
+def test_layouts_of_more_channels_than_one_launch_has_workgroups_for(ops):
+    """Eight channels to a workgroup would be more than the 2^32 threads of a launch; the plain codes of three rows come from
+    the one-launch kernel and have the same bits."""
+    n_out, n_in = 3, (1 << 27) + 1000
+    _say(f"quantise {n_out} x {n_in}")
+    g = torch.Generator(device="cuda").manual_seed(5)
+    W = torch.randn(n_out, n_in, generator=g, device="cuda") * 0.02
+    codes, rng, off = ops.quantize(W)
+    packed, packed16, r, o = ops.quantize_packed(W)
+    assert torch.equal(rng, r) and torch.equal(off, o)
+    assert torch.equal(ops.unpack(packed, n_in, n_out), codes) and torch.equal(ops.unpack_m16(packed16, n_in, n_out), codes)
+
+
 def test_pack_strided_and_ragged(ops):
     big = torch.randint(0, 256, (200, 400), dtype=torch.uint8, device="cuda")
     view = big[:130, :77]                      # stride 400, ragged in both dims
