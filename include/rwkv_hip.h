@@ -285,10 +285,11 @@ typedef struct rwkv_model rwkv_model;
 int rwkv_model_create(const rwkv_model_desc *desc, rwkv_model **out);
 void rwkv_model_destroy(rwkv_model *m);
 
-/* 1 if single-token steps of this handle run as one persistent launch (all
- * matrices have packed16 and the shape is supported) and its generation loop
- * can sample on the device, else 0.  At n_embd 512, 768 and 1536 the token
- * steps are persistent launches too, but sampling stays with the caller. */
+/* 1 if the generation loop of this handle can sample on the device
+ * (rwkv_model_decode_sample), else 0.  It can wherever single-token steps run as
+ * one persistent launch, except at n_embd 512, 768 and 1536, where sampling
+ * stays with the caller.  Whether the persistent kernel is in use (all matrices
+ * have packed16 and the shape is supported) is rwkv_model_trace_workgroups > 0. */
 int rwkv_model_has_fused_step(const rwkv_model *m);
 
 /* Diagnostics: when device_buffer is non-NULL, every workgroup g of every
@@ -298,7 +299,8 @@ int rwkv_model_has_fused_step(const rwkv_model *m);
  * the owner workgroups (n_embd / 16, or n_embd / 32 at n_embd = 5120) followed
  * by the helper workgroups of the ffn key matrix where the kernel has them
  * (80 at n_embd = 2560), whose six stamps are: records seen, statistics,
- * digits written, tiles multiplied, results published, next weights fetched. */
+ * digits written, tiles multiplied, results published, next weights fetched.
+ * 0 workgroups: this handle does not run the persistent kernel. */
 int rwkv_model_trace_workgroups(const rwkv_model *m);
 int rwkv_model_set_trace(rwkv_model *m, int64_t *device_buffer);
 
@@ -313,8 +315,8 @@ int rwkv_model_check(rwkv_model *m);
  * immediately before and after each launch of the persistent single-token
  * kernel - the per-token preparation launch stays outside the pair - then
  * synchronises the stream and returns the kernel's average duration in
- * microseconds.  Creates and destroys 2 n events.  Only models with
- * rwkv_model_has_fused_step. */
+ * microseconds.  Creates and destroys 2 n events.  Only models that run the
+ * persistent kernel (rwkv_model_trace_workgroups > 0). */
 int rwkv_model_time_token_kernel(rwkv_model *m, rwkv_stream_t stream, const int64_t *token, double *state,
                                  double *logits, int n, float *avg_us);
 
@@ -325,7 +327,7 @@ int rwkv_model_time_token_kernel(rwkv_model *m, rwkv_stream_t stream, const int6
  * leaves - the launch ends normally within a millisecond.  state and logits
  * are left untouched.  The next rwkv_model_check reports the aborted step
  * (and clears the flag); token steps after that run as usual.  Only models
- * with rwkv_model_has_fused_step. */
+ * that run the persistent kernel (rwkv_model_trace_workgroups > 0). */
 int rwkv_model_selftest_timeout(rwkv_model *m, rwkv_stream_t stream, double *state, double *logits);
 
 /* Scratch needed by rwkv_model_forward for chunks of up to max_tokens tokens. */

@@ -35,8 +35,8 @@
 // first drain whatever it had prefetched.  The workgroup is therefore split:
 // "front" waves talk to the other workgroups (one of them polls, the others
 // wait on LDS flags), do the per-channel arithmetic, write the digit planes to
-// LDS and finish the 16 owned columns of each product; 8 "back" waves own the
-// weight stream.  A back wave's program is one generated assembly statement
+// LDS and finish the 16 owned columns of each product; 8 "back" waves (4 at the
+// two smallest widths) own the weight stream.  A back wave's program is one generated assembly statement
 // (gen_decode_back.py -> rwkv_decode_back.inc): the 1 KiB blocks of its share
 // of the workgroup's 13 tiles per layer form one sequence of positions,
 // position p lives in register slot p % R of a fixed ring that is reloaded in
@@ -1548,7 +1548,9 @@ bool decode_supported(int64_t L, int64_t C, int64_t F, int64_t V) {
 }
 
 // Widths whose generation loop samples on the device.  The others (512, 768, 1536) run their token steps here too, but
-// their texts are drawn on the host from torch's generator, and a program that seeds it keeps its texts.
+// their texts are drawn on the host from torch's generator: a program that seeds it keeps its random numbers.  (Not every
+// text: the logits of a token step are this kernel's, within 1e-7 of the many-row kernels' that served these widths before
+// and no further from exact sums, and a draw that falls that close to an edge goes the other way.)
 bool decode_samples(int64_t C) { return C == 1024 || C == 2048 || C == 2560 || C == 4096 || C == 5120; }
 
 int64_t decode_workgroups(int64_t C) { return C > 4096 ? C / 32 : C / 16; }

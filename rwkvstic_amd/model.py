@@ -363,10 +363,10 @@ class HipRWKV:
         agnostic/samplers/typical.py:1-17, or argmax), with ``end_adj`` added to logit 0 before every choice
         and the loop ending at the first chosen stop token (which is part of the output).  Returns
         ``(tokens int64 on the device, logits, state)``; ``state`` and ``logits`` are those of the last step
-        that ran.  Needs the persistent single-token kernel (``fused_step``)."""
+        that ran.  Only where the loop can sample on the device (``fused_step``)."""
         self._check_state(state)
         if not self.fused_step:
-            raise RuntimeError("decode_sample needs the persistent single-token kernel (fused_step)")
+            raise RuntimeError("decode_sample: this model does not sample on the device (fused_step); sample from forward's logits")
         if not 0 <= int(token) < self.vocab:
             raise IndexError(f"token id out of range for a vocabulary of {self.vocab}")
         toks = torch.empty(n + 1, dtype=torch.int64, device=self.device)
