@@ -309,7 +309,7 @@ __device__ __forceinline__ void st4(double *p, const double (&v)[4]) {
 // product left pending is applied here) goes to x_out, another buffer than x, and its newest shift row to shift_out; the next
 // launch of this kernel copies that one into the state (commit).
 //
-// 8 rows of 2560 channels, three / two mixes: 8.4 / 8.5 us, 32 rows of 5120 15.8 / 15.0 us (one workgroup of 512 threads for
+// 8 rows of 2560 channels, three / two mixes: 6.9 / 7.4 us, 32 rows of 5120 15.2 / 14.8 us (one workgroup of 512 threads for
 // the row and all its mixes: 11.1 / 9.7 and 19.6 / 15.4; the same with every parameter vector requested ahead: no faster).
 constexpr int kLnRowThreads = 512;
 template <bool MIX, int NSEG>
