@@ -97,9 +97,6 @@ quantize_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in,
 //   quant_scale_kernel    one channel per thread: partials -> lo, range, 1 / range
 //   quant_encode_kernel   128 channels x kEncRows rows at a time: codes, layouts; in workgroups of its own the offsets
 // ---------------------------------------------------------------------------
-// Plain codes of so few rows come from quantize_kernel's one launch, with the same bits (64 x 64: 16 us against 28 for three
-// launches, host calls included; it walks 64 rows in 11 us).
-constexpr int kOneLaunchRows = 64;
 constexpr int kEncRows = 64;            // rows of one LDS tile: 8 blocks of the P8 layout, 4 x 2 of the M16 layout
 constexpr int kChainChannels = 8;       // channels of a workgroup that adds up fractions
 constexpr int64_t kChainMaxBlocks = 1 << 20;    // such workgroups (a launch has at most 2^32 threads); of more channels each takes several groups
@@ -509,8 +506,6 @@ int rwkv_quantize_layouts(rwkv_stream_t stream, const float *weight, int64_t n_o
     RWKV_CHECK_ALIGN(packed16, 16);
     RWKV_CHECK_ALIGN(workspace, 8);
     const QuantWs q = quant_carve(n_out, n_in, workspace);
-    if (workspace_bytes >= q.bytes && n_out <= kOneLaunchRows && codes && !packed && !packed16)
-        return rwkv_quantize_u8(stream, weight, n_out, n_in, codes, range, offset);
     if (workspace_bytes < q.bytes)
         return set_error(RWKV_ERR_WORKSPACE, "rwkv_quantize_layouts: workspace of %zu bytes needed, %zu given", q.bytes, workspace_bytes);
     const hipStream_t st = (hipStream_t)stream;

@@ -147,7 +147,19 @@ def _quantize(weight: torch.Tensor, codes: bool, packed: bool, packed16: bool):
 def quantize(weight: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """``weight[out, in]`` float32 -> ``(codes[in, out] uint8, range[in] float32, offset[in] float64)``
     (MM8.QuantizeMatrix, matmul.py:24-40)."""
-    codes, _, _, rng, off = _quantize(weight, True, False, False)
+    _req(weight, torch.float32, "weight"); _contig(weight, "weight")
+    n_out, n_in = weight.shape
+    # One launch without a workspace, with the same bits, where it is no slower than three that cut the matrix both ways.  It
+    # walks the rows with a workgroup per 64 channels; us of both, 144 / 192 / 208 / 256 rows: of 64 to 8192 channels 18 / 21 / 25 / 28
+    # against 20, of 1 channel 16 / 18 / 21 / 23 against 20; 16384 channels 19 / 22 / 25 / 28 against 22 / 23 / 26 / 27; 65536
+    # channels 35 / 43 / 49 / 56 against 62 / 65 / 76 / 80.  (64 rows 12 against 18.5.)
+    if n_out > max(200, n_in // 64):
+        codes, _, _, rng, off = _quantize(weight, True, False, False)
+        return codes, rng, off
+    codes = torch.empty((n_in, n_out), dtype=torch.uint8, device=weight.device)
+    rng = torch.empty(n_in, dtype=torch.float32, device=weight.device)
+    off = torch.empty(n_in, dtype=torch.float64, device=weight.device)
+    N.check(N.lib().rwkv_quantize_u8(_stream(), weight.data_ptr(), n_out, n_in, codes.data_ptr(), rng.data_ptr(), off.data_ptr()))
     return codes, rng, off
 
 

@@ -66,8 +66,8 @@ def test_quantised_layouts_are_the_packed_codes(ops, shape):
 
 
 # rows on both sides of a step of the serial sums (16), of the eight steps requested together (128) and of an encoding
-# tile (64); channels on both sides of a workgroup's 16 and 128; more rows than 65535 encoding tiles of 256
-@pytest.mark.parametrize("shape", [(1, 1), (15, 16), (17, 15), (64, 17), (127, 128), (129, 129), (300, 132), (1000, 257),
+# tile (64); channels on both sides of a workgroup's 16 and 128; the rows up to which ops.quantize takes the one and the other; more rows than 65535 encoding tiles of 256
+@pytest.mark.parametrize("shape", [(1, 1), (15, 16), (17, 15), (64, 17), (127, 128), (129, 129), (200, 70), (201, 70), (300, 132), (1000, 257),
                                    (2560, 640), (50277, 64), (65535 * 256 + 5, 1)])
 def test_both_quantisers_give_the_same_bits(ops, shape):
     """rwkv_quantize_u8 (no workspace, one workgroup per 64 channels) and rwkv_quantize_layouts: codes, ranges and offsets."""
@@ -78,11 +78,12 @@ def test_both_quantisers_give_the_same_bits(ops, shape):
     W = torch.randn(n_out, n_in, generator=g, device="cuda") * 0.02
     if n_in > 2:
         W[:, 1] = 0.25                                  # a constant channel
-    codes, rng, off = ops.quantize(W)
+    codes, _, _, rng, off = ops._quantize(W, True, False, False)
     c = torch.empty_like(codes)
     r, o = torch.empty_like(rng), torch.empty_like(off)
     N.check(N.lib().rwkv_quantize_u8(torch.cuda.current_stream().cuda_stream, W.data_ptr(), n_out, n_in, c.data_ptr(), r.data_ptr(), o.data_ptr()))
     assert torch.equal(codes, c) and torch.equal(rng, r) and torch.equal(off, o)
+    assert all(torch.equal(a, b) for a, b in zip(ops.quantize(W), (codes, rng, off)))
 
 
 def test_layouts_of_more_channels_than_one_launch_has_workgroups_for(ops):
