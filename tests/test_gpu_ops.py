@@ -65,9 +65,9 @@ def test_quantised_layouts_are_the_packed_codes(ops, shape):
     assert int(codes[-1].max()) == 0 and float(off[-1]) == 0.25
 
 
-# rows on both sides of a step of the serial sums (16), of the eight steps requested together (128) and of an encoding
-# tile (64); channels on both sides of a workgroup's 16 and 128; the rows up to which ops.quantize takes the one and the other; more rows than 65535 encoding tiles of 256
-@pytest.mark.parametrize("shape", [(1, 1), (15, 16), (17, 15), (64, 17), (127, 128), (129, 129), (200, 70), (201, 70), (300, 132), (1000, 257),
+# rows on both sides of a tile of the serial sums (96), of the four tiles requested together (384) and of an encoding
+# tile (64); channels on both sides of a workgroup's 8 and 128; the rows up to which ops.quantize takes the one and the other; more rows than 65535 encoding tiles of 256
+@pytest.mark.parametrize("shape", [(1, 1), (15, 16), (17, 15), (64, 17), (96, 8), (97, 9), (127, 128), (129, 129), (384, 7), (385, 8), (200, 70), (201, 70), (300, 132), (1000, 257),
                                    (2560, 640), (50277, 64), (65535 * 256 + 5, 1)])
 def test_both_quantisers_give_the_same_bits(ops, shape):
     """rwkv_quantize_u8 (no workspace, one workgroup per 64 channels) and rwkv_quantize_layouts: codes, ranges and offsets."""
