@@ -202,8 +202,11 @@ sample_kernel(SampleArgs a) {
                 if (RWKV_BELOW(t3)) { prefix = c3; below = t3; } else if (RWKV_BELOW(t2)) { prefix = c2; below = t2; }
                 else { prefix = c1; below = t1; }
                 shift = 22;
-            } else if (!RWKV_BELOW(t1)) {
-                shift = 28;         // the cut lies below 1/8: its two top bits are zero
+            } else {
+                // the cut lies below 1/8: its two top bits are 00; or at 8 and above (a peaked distribution, nearly all of it
+                // kept): they are 01, and the mass below 2 is that below them
+                if (RWKV_BELOW(t4)) { prefix = c3; below = t3; }
+                shift = 28;
             }
         }
         for (; shift >= kSFirstBit; shift -= 2) RWKV_FULL_ROUND(shift)
