@@ -857,10 +857,12 @@ static int mm8_ref_launch(hipStream_t st, int nm, int64_t n_in, int64_t n_out,
     a.rows_per_split = kRefPasses * kRefRowsPass;
     if (cols * ceil_div(n_in, a.rows_per_split) < 256) a.rows_per_split = kRefSplitRows;
     // In float64 the reduction at a workgroup's end is a quarter of its time, so it takes two or four times the rows where enough
-    // workgroups are left (us a call: 2560 x 10240 19.1 -> 14.8, three of them 36.8 -> 26.5, 5120 x 20480 49.5 -> 35.2).
+    // workgroups are left (us a call with 1, 2, 4 times 256 rows: 2560 x 10240 18.8, 14.4, 13.4, of 240 workgroups the last, and 20.9,
+    // 17.4, 18.0 from memory; 2560 x 20480 29.2, 25.2, 21.0, of 480, and 30.4, 27.6, 22.8; 768 x 50277 24.5, 26.2, 21.3, of 393;
+    // 5120 x 20480 47.9, 38.0, 35.1).
     const bool wide = n_out >= 16;
     int64_t more = 1;
-    if (sizeof(T) == 8 && wide) more = cols * ceil_div(n_in, 4 * a.rows_per_split) >= 512 ? 4 : cols * ceil_div(n_in, 2 * a.rows_per_split) >= 256 ? 2 : 1;
+    if (sizeof(T) == 8 && wide) more = cols * ceil_div(n_in, 4 * a.rows_per_split) >= 384 ? 4 : cols * ceil_div(n_in, 2 * a.rows_per_split) >= 256 ? 2 : 1;
     a.rows_per_split *= (int)more;
     while (ceil_div(n_in, a.rows_per_split) > 65535) a.rows_per_split *= 2;        // (slices of a grid)
     const bool longer = a.rows_per_split > kRefPasses * kRefRowsPass;
