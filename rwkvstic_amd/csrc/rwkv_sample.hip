@@ -175,8 +175,8 @@ sample_kernel(SampleArgs a) {
         int shift = 30;
         {
             // One round over four thresholds that settles the top eight bits where the cut lies between 1/8 and 8, as it does
-            // unless the distribution is nearly one token or tau nearly everything; else the rounds start at the top.  (The
-            // sums grow with the threshold, rounding included: the cut does not depend on the thresholds tried before.)
+            // unless the distribution is nearly one token or tau nearly everything; else it settles the top two.  (The sums
+            // grow with the threshold, rounding included: the cut does not depend on the thresholds tried before.)
             constexpr unsigned c1 = 0x3e000000u, c2 = 0x3f000000u, c3 = 0x40000000u, c4 = 0x41000000u;       // 1/8, 1/2, 2, 8
             float m1 = 0.f, m2 = 0.f, m3 = 0.f, m4 = 0.f;
 #pragma unroll
