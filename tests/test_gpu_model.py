@@ -701,8 +701,8 @@ def test_timed_token_steps_advance_the_state_like_forward():
     assert 1.0 < us < 5000.0
 
 
-# both sides of every block length of the sequence WKV kernel (64, 128, 256 and 512 steps), of its serial form (5 steps)
-# and of the rows one pass takes (1024)
+# both sides of where the sequence WKV kernels take over (6 steps) and cut into chunks (64), of their blocks (128 and 256
+# steps, one and several) and of the rows one pass takes (1024)
 @pytest.mark.parametrize("T", [4, 5, 6, 8, 9, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1023, 1025])
 def test_a_prompt_equals_its_tokens_one_by_one(T):
     from rwkvstic_amd.model import HipRWKV
@@ -713,7 +713,7 @@ def test_a_prompt_equals_its_tokens_one_by_one(T):
     lg, sp = m.forward(toks[3:], st.clone())
     for t in toks[3:].tolist():
         l1, st = m.forward([t], st)
-    # the same float32 recurrence in another order: float32 rounding of the WKV output, a few layers of it
+    # from 64 steps on the recurrence is joined in another order: float32 rounding of the WKV output, a few layers of it
     assert float((lg - l1).norm() / l1.norm()) < 5e-6
     for row in range(5):
         assert float((sp[:, row] - st[:, row]).norm() / st[:, row].norm()) < 5e-6, row
