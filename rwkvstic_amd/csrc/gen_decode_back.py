@@ -11,7 +11,7 @@ twice the space and spills; a spilled or copied in-flight register is silent cor
 whole back-wave program is one asm statement with its own register map; it talks to the compiled
 front waves only through LDS and workgroup barriers.
 
-Stream of one back wave (wave wb of BW, 8 or, at the two smallest widths, 4) of workgroup g, in units of 1 KiB blocks ("positions"):
+Stream of one back wave (wave wb of BW, 8 or, up to 1024 channels, 4) of workgroup g, in units of 1 KiB blocks ("positions"):
   per layer 13 jobs x KW blocks (job = one 16-column tile of a C-row matrix, or a quarter of the
   F-row ffn value tile; wave wb owns blocks wb, wb+BW, ... of the job; KW = C / (64 BW)), padded to PP positions, a
   multiple of the ring size R, then the head tiles g, g+G, ... .  Position p lives in ring slot
@@ -468,8 +468,9 @@ def gen(KW, R, NV, NSH, HELP=False, BW=8):
 
 # (KW, back waves, front waves, ring size): 12 waves per workgroup -> 168 VGPRs each, 16 waves -> 128.  At the narrow
 # widths the exchanges set the pace and the ring size does not matter: C = 768, 12 layers, 176 / 180 / 177 us per token
-# with rings of 13 / 20 / 39; C = 1536, 24 layers, 478 / 476 with 13 / 20.
-CONFIGS = [(2, 4, 4, 26), (3, 4, 4, 13), (2, 8, 4, 26), (3, 8, 4, 20), (4, 8, 4, 26), (8, 8, 4, 26), (5, 8, 8, 22),
+# with rings of 13 / 20 / 39; C = 1536, 24 layers, 478 / 476 with 13 / 20 (both with four front waves).  Rings that divide
+# a layer's positions, or nearly: what is left over is loaded as padding.
+CONFIGS = [(2, 4, 8, 26), (3, 4, 8, 13), (4, 4, 8, 26), (3, 8, 8, 20), (4, 8, 8, 18), (8, 8, 8, 21), (5, 8, 8, 22),
            (10, 8, 8, int(os.environ.get("RWKV_BACK_R_WIDE", "26")))]
 
 
@@ -488,7 +489,7 @@ def main():
         NV = 128 if FW + BW == 16 else 168
         clob = ", ".join(f'"v{i}"' for i in range(V_APC, NV)) + ", " + ", ".join(f'"s{i}"' for i in range(S_CUR, 102 if KW > 8 else 100))
         tiles_per_body = R // math.gcd(R, KW)
-        NSH = max(d for d in range(1, 5) if tiles_per_body % d == 0)     # head tiles per barrier round
+        NSH = max(d for d in range(1, 5) if tiles_per_body % d == 0 and d != 3)     # head tiles per barrier round (three: no faster, and more LDS than the phases need)
         lines, info = gen(KW, R, NV, NSH, HELP, BW)
         w(f"template <> struct BackCfg{'H' if HELP else ''}<{BW * KW}, {FW}> {{")
         w(f"    static constexpr int R = {R}, RED = {info['RED']}, FLAG = {info['FLAG']}, RED_SLOTS = {info['RED_SLOTS']}, NS = {info['NS']};")

@@ -35,8 +35,8 @@
 // first drain whatever it had prefetched.  The workgroup is therefore split:
 // "front" waves talk to the other workgroups (one of them polls, the others
 // wait on LDS flags), do the per-channel arithmetic, write the digit planes to
-// LDS and finish the 16 owned columns of each product; 8 "back" waves (4 at the
-// two smallest widths) own the weight stream.  A back wave's program is one generated assembly statement
+// LDS and finish the 16 owned columns of each product; 8 "back" waves (4 up to
+// 1024 channels) own the weight stream.  A back wave's program is one generated assembly statement
 // (gen_decode_back.py -> rwkv_decode_back.inc): the 1 KiB blocks of its share
 // of the workgroup's 13 tiles per layer form one sequence of positions,
 // position p lives in register slot p % R of a fixed ring that is reloaded in
@@ -57,12 +57,16 @@ namespace rwkv {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-// Widths.  C = 512, 768 and 1536 are bound by the four exchanges per layer (13.4 us per layer at 768): a token of the
-// 12-layer 768 shape takes 177 us, as one-row prompts through the many-row kernels it took 630 us (146 launches).
+// Widths.  C = 512, 768 and 1536 are bound by the four exchanges per layer (12.3 us per layer at 768): a token of the
+// 12-layer 768 shape takes 170 us, as one-row prompts through the many-row kernels it took 630 us (146 launches).
 // NB (template parameter throughout): 64-channel blocks of a row of C channels, C = 64 NB.  Back (streaming) waves per
-// workgroup: eight, four at the two smallest widths, whose 8 and 12 blocks per tile they share evenly (12 over eight
-// waves would leave half of them idle every second block).
-constexpr int back_waves(int nb) { return nb <= 12 ? 4 : 8; }
+// workgroup: eight, four up to 1024 channels, where the exchanges and not the stream set the pace and a tile's sums come
+// from four parts instead of eight (24 layers of 1024: 336 us a token, with eight 344; at 1536 they are equal, at 2048 four
+// cost 9 %).  Front waves: eight, which gather, quantise and write the digits of a vector between them (four / eight, us
+// a token: 12 layers of 512 172 / 168, of 768 178 / 170, of 1536 246 / 225, of 2048 267 / 248, 8 of 4096 408 / 387; twelve
+// lose again: 172 at 768, 243 at 1536).
+constexpr int back_waves(int nb) { return nb <= 16 ? 4 : 8; }
+constexpr int kFrontWaves = 8;
 constexpr int kPrepThreads = 512;
 constexpr int prep_parts(int C) { return (C + kPrepThreads - 1) / kPrepThreads; }      // 512-channel parts of a layer's per-token scalars
 constexpr int kRealJobs = 13;          // tile jobs per layer: k v r | o | ffn_r, 4 x ffn_k | 4 quarters of ffn_v
@@ -74,8 +78,8 @@ constexpr int kSlotsPerGroup = 5;      // parked-tile slots a group of 16 channe
 // Head column sums a front thread fetches, 16 per head tile of the workgroup: narrow models have few workgroups and so
 // many head tiles each (66 at C = 768 with 50277 tokens), and a part of LDS for the sums; the others park them in half
 // an owner record.
-constexpr int head_cs_per_thread(int nb) { return nb <= 12 ? 8 : 4; }
-constexpr int head_cs_lds_bytes(int nb) { return nb <= 12 ? 8 * 256 * 4 : 0; }
+constexpr int kHeadCsPerThread = 4;
+constexpr int head_cs_lds_bytes(int nb) { return nb <= 12 ? kHeadCsPerThread * 64 * kFrontWaves * 4 : 0; }
 
 // LDS flag words
 enum { FLAG_ARRIVED = 0, FLAG_SCALE = 1, FLAG_ABORT = 2, FLAG_GO = 3, FLAG_COUNT = 4 };   // FLAG_GO: see the reload gate of the generated back-wave program
@@ -885,7 +889,7 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
     // column sums of the workgroup's head tiles: requested now, parked in LDS (where there is no
     // room of their own, in the half that held the last layer's record) once the wait for x is over (a load inside the loop below would cost a
     // round trip through the busy memory pipeline in every round)
-    constexpr int HCS = head_cs_per_thread(NB);
+    constexpr int HCS = kHeadCsPerThread;
     int *csh = reinterpret_cast<int *>(own_lds + (head_cs_lds_bytes(NB) ? 2 : (L + 1) & 1) * kOrSlots);
     int csv[HCS];
 #pragma unroll
@@ -1160,7 +1164,7 @@ struct DecodeLds {
         const int own = STATE_OFFSET + state_bytes(L);
         return (own > STASH_OFFSET + STASH_BYTES ? own : STASH_OFFSET + STASH_BYTES) + (trace ? L * kTraceStampsPerLayer * 8 : 0);
     }
-    static_assert(head_cs_lds_bytes(NB) == 0 || (NT == 1 && head_cs_lds_bytes(NB) >= head_cs_per_thread(NB) * 64 * FW * 4), "head column sums");
+    static_assert(FW == kFrontWaves && (head_cs_lds_bytes(NB) == 0 || NT == 1), "head column sums");
     // the generated back-wave program addresses LDS by these offsets
     static_assert(Back::RED == DIG_BYTES, "parked tiles follow the digit planes");
     static_assert(Back::FLAG == DIG_BYTES + RED_BYTES + STAT_BYTES + RF_BYTES + FLAG_ABORT * 4, "abort flag offset");
@@ -1525,14 +1529,14 @@ __global__ void __launch_bounds__(kPrepThreads) build_consts_kernel(const ConstA
 static int decode_lds(int64_t C, int64_t L) {
     const int l = (int)(L < 4096 ? L : 4096);
     switch (C) {
-        case 512: return DecodeLds<8, 4>::total(l);
-        case 768: return DecodeLds<12, 4>::total(l);
-        case 1024: return DecodeLds<16, 4>::total(l);
-        case 1536: return DecodeLds<24, 4>::total(l);
-        case 2048: return DecodeLds<32, 4>::total(l);
-        case 2560: return DecodeLds<40, 8, true>::total(l);
-        case 4096: return DecodeLds<64, 4>::total(l);
-        case 5120: return DecodeLds<80, 8>::total(l);
+        case 512: return DecodeLds<8, kFrontWaves>::total(l);
+        case 768: return DecodeLds<12, kFrontWaves>::total(l);
+        case 1024: return DecodeLds<16, kFrontWaves>::total(l);
+        case 1536: return DecodeLds<24, kFrontWaves>::total(l);
+        case 2048: return DecodeLds<32, kFrontWaves>::total(l);
+        case 2560: return DecodeLds<40, kFrontWaves, true>::total(l);
+        case 4096: return DecodeLds<64, kFrontWaves>::total(l);
+        case 5120: return DecodeLds<80, kFrontWaves>::total(l);
         default: return 0;
     }
 }
@@ -1543,8 +1547,8 @@ bool decode_supported(int64_t L, int64_t C, int64_t F, int64_t V) {
     if (decode_lds(C, L) == 0) return false;
     // the column sums of a workgroup's head tiles are staged in LDS by its front threads
     const int nb = (int)(C / 64);
-    const int64_t NWG = decode_workgroups(C), head_rounds = ((V + 15) / 16 + NWG - 1) / NWG, front_threads = (C == 2560 || C == 5120) ? 512 : 256;
-    return head_rounds * 16 <= head_cs_per_thread(nb) * front_threads &&
+    const int64_t NWG = decode_workgroups(C), head_rounds = ((V + 15) / 16 + NWG - 1) / NWG;
+    return head_rounds * 16 <= kHeadCsPerThread * 64 * kFrontWaves &&
            head_rounds * 16 * (int64_t)sizeof(int) <= (head_cs_lds_bytes(nb) ? head_cs_lds_bytes(nb) : kOrSlots * 8) &&
            decode_lds(C, L) <= 160 * 1024;
 }
@@ -1731,14 +1735,14 @@ static int launch_step(hipStream_t st, const DArgs &args, bool with_prep) {
     const bool stream = weights_streamed(args.m.L, args.m.C, args.m.F, args.m.V);
 #define RWKV_STEP(NB, FW) return stream ? launch_one<NB, FW, true>(st, args, with_prep) : launch_one<NB, FW, false>(st, args, with_prep)
     switch (args.m.C) {
-        case 512: RWKV_STEP(8, 4);
-        case 768: RWKV_STEP(12, 4);
-        case 1024: RWKV_STEP(16, 4);
-        case 1536: RWKV_STEP(24, 4);
-        case 2048: RWKV_STEP(32, 4);
-        case 2560: RWKV_STEP(40, 8);
-        case 4096: RWKV_STEP(64, 4);
-        case 5120: return launch_one<80, 8, true>(st, args, with_prep);        // (one layer alone is 340 MB)
+        case 512: RWKV_STEP(8, kFrontWaves);
+        case 768: RWKV_STEP(12, kFrontWaves);
+        case 1024: RWKV_STEP(16, kFrontWaves);
+        case 1536: RWKV_STEP(24, kFrontWaves);
+        case 2048: RWKV_STEP(32, kFrontWaves);
+        case 2560: RWKV_STEP(40, kFrontWaves);
+        case 4096: RWKV_STEP(64, kFrontWaves);
+        case 5120: return launch_one<80, kFrontWaves, true>(st, args, with_prep);        // (one layer alone is 340 MB)
         default: return set_error(RWKV_ERR_SIZE, "decode kernel: n_embd %d not supported", args.m.C);
     }
 #undef RWKV_STEP
