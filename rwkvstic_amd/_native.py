@@ -133,6 +133,24 @@ def lib() -> C.CDLL:
     return L
 
 
+_host = None
+
+
+def host():
+    """The native host side of the operator calls (csrc/rwkv_torch.cpp), bound to the library ``lib()`` has loaded."""
+    global _host
+    if _host is None or _host[0] is not lib():
+        try:
+            from . import _rwkv_torch
+        except ImportError as e:
+            raise RuntimeError(f"{os.path.join(HERE, '_rwkv_torch.so')} is missing or was built for another torch: build it "
+                               f"with `python -m rwkvstic_amd.build` ({e})") from e
+        L = lib()
+        _rwkv_torch.bind({n: C.cast(getattr(L, n), C.c_void_p).value for n in EXPORTS})
+        _host = (L, _rwkv_torch)
+    return _host[1]
+
+
 def check(code: int) -> None:
     if code != 0:
         raise RwkvHipError(code, lib().rwkv_last_error().decode())

@@ -1,0 +1,227 @@
+// Host side of the operator calls, native: torch.ops.rwkv.* (reference src/rwkvstic/agnostic/backends/cuda/wrapper.cpp:45-141)
+// and the stand-alone products and recurrence of rwkvstic_amd.ops.  A call checks its tensors, takes its workspace from torch's
+// allocator (so that it belongs to the stream the call runs on) and hands device pointers to librwkv_hip.so.
+//
+// What bounds these calls is the host: a matrix of the 3B shape is 10 us of kernels, and a call that goes through Python
+// (dispatcher to interpreter, checks, ctypes) takes 16.
+//
+// Anything out of the ordinary - an argument that does not fit, an error of the library - is left to the Python function of the
+// same name, which raises what it always raised.
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
+#include <torch/library.h>
+
+#include <map>
+#include <string>
+
+#include "../../include/rwkv_hip.h"
+
+namespace {
+
+// Entry points of the library that the Python side has loaded (it decides which file that is).
+struct Entries {
+    decltype(&rwkv_mm8_workspace_bytes) mm8_workspace_bytes, mm8_f64_workspace_bytes;
+    decltype(&rwkv_mm8_one) mm8_one;
+    decltype(&rwkv_mm8_one_f64) mm8_one_f64;
+    decltype(&rwkv_mm8_three) mm8_three;
+    decltype(&rwkv_mm8_three_f64) mm8_three_f64;
+    decltype(&rwkv_wkv_forward_f64) wkv_forward_f64;
+    decltype(&rwkv_packed_bytes) packed_bytes, packed_m16_bytes;
+    decltype(&rwkv_mm8_packed) mm8_packed;
+    decltype(&rwkv_mm8_m16_workspace_bytes) mm8_m16_workspace_bytes;
+    decltype(&rwkv_mm8_m16) mm8_m16;
+    decltype(&rwkv_wkv_f32) wkv_f32;
+} lib;
+
+void bind(const std::map<std::string, uintptr_t> &at) {
+#define BIND(field, name) lib.field = reinterpret_cast<decltype(lib.field)>(at.at(#name))
+    BIND(mm8_workspace_bytes, rwkv_mm8_workspace_bytes); BIND(mm8_f64_workspace_bytes, rwkv_mm8_f64_workspace_bytes);
+    BIND(mm8_one, rwkv_mm8_one); BIND(mm8_one_f64, rwkv_mm8_one_f64);
+    BIND(mm8_three, rwkv_mm8_three); BIND(mm8_three_f64, rwkv_mm8_three_f64);
+    BIND(wkv_forward_f64, rwkv_wkv_forward_f64);
+    BIND(packed_bytes, rwkv_packed_bytes); BIND(packed_m16_bytes, rwkv_packed_m16_bytes);
+    BIND(mm8_packed, rwkv_mm8_packed);
+    BIND(mm8_m16_workspace_bytes, rwkv_mm8_m16_workspace_bytes); BIND(mm8_m16, rwkv_mm8_m16);
+    BIND(wkv_f32, rwkv_wkv_f32);
+#undef BIND
+}
+
+rwkv_stream_t stream() { return reinterpret_cast<rwkv_stream_t>(c10::hip::getCurrentHIPStream().stream()); }
+
+// A recorded call keeps its scratch for as long as it is replayed: the buffer the Python side holds on to.
+bool recording() {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(c10::hip::getCurrentHIPStream().stream(), &s) != hipSuccess || s != hipStreamCaptureStatusNone;
+}
+
+at::Tensor bytes(size_t n, const at::Tensor &like) {
+    return at::empty({static_cast<int64_t>(n > 0 ? n : 1)}, like.options().dtype(at::kByte));
+}
+
+bool on_gpu(const at::Tensor &t, at::ScalarType dt) { return t.defined() && t.is_cuda() && t.scalar_type() == dt && !t.requires_grad(); }
+bool vec(const at::Tensor &t, at::ScalarType dt) { return on_gpu(t, dt) && t.dim() >= 1 && t.stride(0) == 1; }
+bool codes(const at::Tensor &w, int64_t n, int64_t m) {
+    return on_gpu(w, at::kByte) && w.dim() == 2 && w.stride(1) == 1 && w.size(0) >= n && w.size(1) >= m;
+}
+bool whole(const at::Tensor &t, at::ScalarType dt) { return on_gpu(t, dt) && t.is_contiguous(); }
+
+template <typename T>
+T *ptr(const at::Tensor &t) { return static_cast<T *>(t.data_ptr()); }
+const uint8_t *u8(const at::Tensor &t) { return ptr<const uint8_t>(t); }
+
+// ---- torch.ops.rwkv.* ------------------------------------------------------------------------------------------------
+template <typename... A>
+void in_python(const char *name, A &&...args) {
+    pybind11::gil_scoped_acquire gil;
+    pybind11::module_::import("rwkvstic_amd.ops").attr(name)(std::forward<A>(args)...);
+}
+
+bool try_one(int64_t N, int64_t M, const at::Tensor &x, const at::Tensor &w, const at::Tensor &y, const at::Tensor &r) {
+    const auto dt = x.scalar_type();
+    if ((dt != at::kFloat && dt != at::kDouble) || recording()) return false;
+    if (!vec(x, dt) || x.dim() != 1 || !vec(y, dt) || !vec(r, dt) || !codes(w, N, M)) return false;
+    if (N <= 0 || M <= 0 || x.numel() < N || r.numel() < N || y.numel() < M) return false;
+    if (dt == at::kFloat) {
+        const at::Tensor ws = bytes(lib.mm8_workspace_bytes(N, M, 1), x);
+        return lib.mm8_one(stream(), N, M, ptr<float>(x), u8(w), w.stride(0), ptr<float>(y), ptr<float>(r), ws.data_ptr(), ws.numel()) == RWKV_OK;
+    }
+    const at::Tensor ws = bytes(lib.mm8_f64_workspace_bytes(N, M, 1), x);
+    return lib.mm8_one_f64(stream(), N, M, ptr<double>(x), u8(w), w.stride(0), ptr<double>(y), ptr<double>(r), ws.data_ptr(), ws.numel()) == RWKV_OK;
+}
+
+void mm8_one(int64_t N, int64_t M, at::Tensor &x, at::Tensor &w, at::Tensor &y, at::Tensor &r) {
+    if (!try_one(N, M, x, w, y, r)) in_python("mm8_one", N, M, x, w, y, r);
+}
+
+using T3 = const at::Tensor *const (&)[3];
+bool try_three(int64_t N, int64_t M, T3 x, T3 w, T3 y, T3 r) {
+    const auto dt = x[0]->scalar_type();
+    if ((dt != at::kFloat && dt != at::kDouble) || N <= 0 || M <= 0 || recording()) return false;
+    for (int i = 0; i < 3; ++i) {
+        if (!vec(*x[i], dt) || !vec(*y[i], dt) || !vec(*r[i], dt) || !codes(*w[i], N, M)) return false;
+        if (x[i]->numel() < N || r[i]->numel() < N || y[i]->numel() < M) return false;
+    }
+    auto call = [&](auto fn, auto bytes_fn, auto zero) {
+        using T = decltype(zero);
+        const at::Tensor ws = bytes(bytes_fn(N, M, 3), *x[0]);
+        return fn(stream(), N, M, ptr<T>(*x[0]), ptr<T>(*x[1]), ptr<T>(*x[2]), u8(*w[0]), w[0]->stride(0), u8(*w[1]), w[1]->stride(0),
+                  u8(*w[2]), w[2]->stride(0), ptr<T>(*y[0]), ptr<T>(*y[1]), ptr<T>(*y[2]), ptr<T>(*r[0]), ptr<T>(*r[1]), ptr<T>(*r[2]),
+                  ws.data_ptr(), ws.numel()) == RWKV_OK;
+    };
+    return dt == at::kFloat ? call(lib.mm8_three, lib.mm8_workspace_bytes, 0.f) : call(lib.mm8_three_f64, lib.mm8_f64_workspace_bytes, 0.0);
+}
+
+void mm8_three(int64_t N, int64_t M, at::Tensor &x, at::Tensor &x1, at::Tensor &x2, at::Tensor &w, at::Tensor &w1, at::Tensor &w2,
+               at::Tensor &y, at::Tensor &y1, at::Tensor &y2, at::Tensor &r, at::Tensor &r1, at::Tensor &r2) {
+    const at::Tensor *const xs[3] = {&x, &x1, &x2}, *const ws[3] = {&w, &w1, &w2}, *const ys[3] = {&y, &y1, &y2}, *const rs[3] = {&r, &r1, &r2};
+    if (!try_three(N, M, xs, ws, ys, rs)) in_python("mm8_three", N, M, x, x1, x2, w, w1, w2, y, y1, y2, r, r1, r2);
+}
+
+void wkv_forward(int64_t B, int64_t T, int64_t C, at::Tensor &w, at::Tensor &u, at::Tensor &k, at::Tensor &v, at::Tensor &y,
+                 at::Tensor &aa, at::Tensor &bb, at::Tensor &pp) {
+    bool ok = B > 0 && T > 0 && C > 0;
+    for (const at::Tensor *t : {&w, &u, &k, &v, &y, &aa, &bb, &pp}) ok = ok && whole(*t, at::kDouble);
+    for (const at::Tensor *t : {&k, &v, &y}) ok = ok && t->numel() / C / T >= B;
+    for (const at::Tensor *t : {&aa, &bb, &pp}) ok = ok && t->numel() / C >= B;
+    for (const at::Tensor *t : {&w, &u}) ok = ok && t->numel() >= C;
+    if (!ok || lib.wkv_forward_f64(stream(), B, T, C, ptr<double>(w), ptr<double>(u), ptr<double>(k), ptr<double>(v), ptr<double>(y),
+                                   ptr<double>(aa), ptr<double>(bb), ptr<double>(pp)) != RWKV_OK)
+        in_python("wkv_forward", B, T, C, w, u, k, v, y, aa, bb, pp);
+}
+
+// The reference's schemas (wrapper.cpp:131-141).
+void register_ops() {
+    static torch::Library *published = nullptr;      // (lives as long as the process: operators are looked up until its end)
+    if (published) return;
+    auto *l = new torch::Library(torch::Library::DEF, "rwkv", std::nullopt, __FILE__, __LINE__);
+    l->def("wkv_forward(int B, int T, int C, Tensor(a!) w, Tensor(b!) u, Tensor(c!) k, Tensor(d!) v, Tensor(e!) y, Tensor(f!) aa, "
+           "Tensor(g!) bb, Tensor(h!) pp) -> ()");
+    l->def("mm8_one(int N, int M, Tensor(a!) x, Tensor(b!) w, Tensor(c!) y, Tensor(d!) r) -> ()");
+    l->def("mm8_three(int N, int M, Tensor(a!) x, Tensor(b!) x1, Tensor(c!) x2, Tensor(d!) w, Tensor(e!) w1, Tensor(f!) w2, "
+           "Tensor(g!) y, Tensor(h!) y1, Tensor(i!) y2, Tensor(j!) r, Tensor(k!) r1, Tensor(l!) r2) -> ()");
+    l->impl("wkv_forward", c10::DispatchKey::CUDA, TORCH_FN(wkv_forward));
+    l->impl("mm8_one", c10::DispatchKey::CUDA, TORCH_FN(mm8_one));
+    l->impl("mm8_three", c10::DispatchKey::CUDA, TORCH_FN(mm8_three));
+    published = l;
+}
+
+// ---- stand-alone kernels: the result, or None where the Python function has to look at the call ------------------------
+using Arg = pybind11::handle;
+const at::Tensor *tensor(Arg a) { return THPVariable_CheckExact(a.ptr()) ? &THPVariable_Unpack(a.ptr()) : nullptr; }
+
+struct Product {
+    const at::Tensor *x, *packed, *r_row, *m_row, *r_col = nullptr, *m_col = nullptr;
+    at::Tensor y;
+    const float *col(const at::Tensor *t) const { return t ? ptr<const float>(*t) : nullptr; }
+};
+
+bool product(Product &p, decltype(lib.packed_bytes) bytes_fn, Arg x, Arg packed, int64_t n_in, int64_t n_out, Arg r_row, Arg m_row,
+             Arg r_col, Arg m_col, Arg out) {
+    p.x = tensor(x); p.packed = tensor(packed); p.r_row = tensor(r_row); p.m_row = tensor(m_row);
+    if (!p.x || !p.packed || !p.r_row || !p.m_row || n_in <= 0 || n_out <= 0) return false;
+    if (!whole(*p.x, at::kFloat) || p.x->dim() != 2 || p.x->size(1) != n_in || !on_gpu(*p.packed, at::kByte) ||
+        !on_gpu(*p.r_row, at::kFloat) || !on_gpu(*p.m_row, at::kDouble)) return false;
+    if (p.packed->numel() < (int64_t)bytes_fn(n_in, n_out) || p.r_row->numel() < n_in || p.m_row->numel() < n_in) return false;
+    for (auto [h, t] : {std::pair{r_col, &p.r_col}, std::pair{m_col, &p.m_col}}) {
+        if (h.is_none()) continue;
+        *t = tensor(h);
+        if (!*t || !on_gpu(**t, at::kFloat) || (*t)->numel() < n_out) return false;
+    }
+    if (out.is_none()) p.y = at::empty({p.x->size(0), n_out}, p.x->options().dtype(at::kDouble));
+    else {
+        const at::Tensor *t = tensor(out);
+        if (!t || !whole(*t, at::kDouble)) return false;
+        p.y = *t;
+    }
+    return true;
+}
+
+pybind11::object mm8_packed(Arg x, Arg packed, int64_t n_in, int64_t n_out, Arg r_row, Arg m_row, Arg r_col, Arg m_col, Arg out) {
+    Product p;
+    if (!product(p, lib.packed_bytes, x, packed, n_in, n_out, r_row, m_row, r_col, m_col, out)) return pybind11::none();
+    if (lib.mm8_packed(stream(), p.x->size(0), n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
+                       p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y)) != RWKV_OK) return pybind11::none();
+    return out.is_none() ? pybind11::cast(p.y) : pybind11::reinterpret_borrow<pybind11::object>(out);
+}
+
+pybind11::object mm8_m16(Arg x, Arg packed, int64_t n_in, int64_t n_out, Arg r_row, Arg m_row, Arg r_col, Arg m_col, Arg out, Arg workspace) {
+    Product p;
+    if (!product(p, lib.packed_m16_bytes, x, packed, n_in, n_out, r_row, m_row, r_col, m_col, out)) return pybind11::none();
+    const int64_t B = p.x->size(0);
+    at::Tensor ws;
+    if (workspace.is_none()) ws = bytes(lib.mm8_m16_workspace_bytes(B, n_in), *p.x);
+    else if (const at::Tensor *t = tensor(workspace)) ws = *t;
+    else return pybind11::none();
+    if (lib.mm8_m16(stream(), B, n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
+                    p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y), ws.data_ptr(), ws.numel()) != RWKV_OK) return pybind11::none();
+    return out.is_none() ? pybind11::cast(p.y) : pybind11::reinterpret_borrow<pybind11::object>(out);
+}
+
+pybind11::object wkv_f32(Arg w, Arg u, Arg k, Arg v, Arg aa, Arg bb, Arg pp) {
+    const Arg args[7] = {w, u, k, v, aa, bb, pp};
+    const at::Tensor *t[7];
+    for (int i = 0; i < 7; ++i) {
+        t[i] = tensor(args[i]);
+        if (!t[i] || !whole(*t[i], at::kFloat)) return pybind11::none();
+    }
+    if (t[2]->dim() != 3 || t[3]->sizes() != t[2]->sizes()) return pybind11::none();
+    const int64_t B = t[2]->size(0), T = t[2]->size(1), C = t[2]->size(2);
+    for (int i : {4, 5, 6}) if (t[i]->numel() < B * C) return pybind11::none();
+    for (int i : {0, 1}) if (t[i]->numel() < C) return pybind11::none();
+    at::Tensor y = at::empty_like(*t[2]);
+    if (lib.wkv_f32(stream(), B, T, C, ptr<float>(*t[0]), ptr<float>(*t[1]), ptr<float>(*t[2]), ptr<float>(*t[3]), ptr<float>(y),
+                    ptr<float>(*t[4]), ptr<float>(*t[5]), ptr<float>(*t[6])) != RWKV_OK) return pybind11::none();
+    return pybind11::cast(y);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_rwkv_torch, m) {
+    m.def("bind", &bind);
+    m.def("register_ops", &register_ops);
+    m.def("mm8_packed", &mm8_packed);
+    m.def("mm8_m16", &mm8_m16);
+    m.def("wkv_f32", &wkv_f32);
+}

@@ -355,6 +355,55 @@ def test_torch_ops_registered_with_reference_schema(ops):
     assert (y.double() - (x.double() * r.double()) @ w.double()).abs().max() < 1e-2
 
 
+def _calls(ops):
+    """Calls of the published operators, ordinary and odd: (name, arguments).  The last tensors are what they write."""
+    g = torch.Generator().manual_seed(5)
+    n_in, n_out = 96, 40
+    for dt in (torch.float32, torch.float64):
+        x, r, y = torch.randn(n_in, generator=g, dtype=dt).cuda(), torch.rand(n_in, generator=g, dtype=dt).cuda(), torch.zeros(n_out, dtype=dt, device="cuda")
+        w = torch.randint(0, 256, (n_in, n_out + 8), generator=g, dtype=torch.uint8).cuda()
+        yield "mm8_one", (n_in, n_out, x, w[:, :n_out].contiguous(), y, r)
+        yield "mm8_one", (n_in, n_out, x, w[:, 3:3 + n_out], y, r)                              # strided rows that start anywhere
+        yield "mm8_one", (n_in, n_out, x, w[:, :n_out], y, torch.stack((r, r), 1)[:, 0])         # (a strided r is read as it lies)
+        yield "mm8_one", (n_in - 1, n_out, x, w, y, r)                                           # larger tensors than the product
+        yield "mm8_one", (n_in, n_out, x.clone().requires_grad_(), w, y, r)
+        yield "mm8_one", (n_in, n_out, x[::2], w, y, r)                                          # refused: stride
+        yield "mm8_one", (n_in, n_out, x, w.t(), y, r)
+        yield "mm8_one", (n_in, n_out, x, w, y[:-1], r)                                          # refused: size
+        yield "mm8_one", (n_in, n_out, x, w, y.half(), r)                                        # refused: type
+        yield "mm8_one", (0, n_out, x, w, y, r)
+        yield "mm8_three", (n_in, n_out, x, x, x, w, w[:, 1:1 + n_out], w, y, y.clone(), y.clone(), r, r, r)
+        yield "mm8_three", (n_in, n_out, x, x[:-1], x, w, w, w, y, y.clone(), y.clone(), r, r, r)
+    f = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64).cuda()
+    wkv = lambda T, C: (2, T, C, -f(C), f(C), f(2, T, C), f(2, T, C), f(2, T, C), f(2, C), f(2, C) + 0.5, f(2, C))
+    yield "wkv_forward", wkv(3, 5)
+    yield "wkv_forward", wkv(20, 33)
+    yield "wkv_forward", wkv(3, 5)[:5] + (f(5, 6).t(),) + wkv(3, 5)[6:]
+    yield "wkv_forward", (2, 4, 5) + wkv(3, 5)[3:]
+
+
+def test_published_operators_do_what_the_functions_do(ops):
+    """Results, and what is refused with which exception: the operators' native side leaves odd calls to the functions."""
+    ops.register_torch_ops()
+    for i, (name, args) in enumerate(_calls(ops)):
+        print(f"operator call {i}: {name}", flush=True)
+        seen = []
+        for fn in (getattr(ops, name), getattr(torch.ops.rwkv, name)):
+            mine = [a.detach().clone(memory_format=torch.preserve_format).requires_grad_(a.requires_grad)
+                    if isinstance(a, torch.Tensor) and a.is_contiguous() else a for a in args]
+            try:
+                fn(*mine)
+            except Exception as e:
+                seen.append((type(e), str(e)))
+            else:
+                seen.append([a.detach().cpu() for a in mine if isinstance(a, torch.Tensor)])
+        if isinstance(seen[0], tuple):
+            assert seen[0] == seen[1], (i, seen)
+        else:
+            assert not isinstance(seen[1], tuple), (i, seen[1])
+            assert all(torch.equal(a, b) for a, b in zip(*seen)), i
+
+
 # ------------------------------------------------------------------ WKV
 def _wkv_case(B, T, C, seed, lo=-8.0):
     g = torch.Generator().manual_seed(seed)
