@@ -585,8 +585,8 @@ wkv_f64_ref_kernel(int B, int T, int C, const double *__restrict__ w, const doub
 // between the two passes, k and v are read once).
 //
 // Bound: the chain of float64 exponentials (some fifty dependent instructions each) where there are few channels,
-// memory with many.  32 channels per workgroup keep a row's piece at 256 bytes.  2560 channels, 256 steps: 15.4 us
-// against 101 us of the serial kernel.
+// memory with many.  2560 channels, 256 steps: 9.7 us (with 32 channels to a workgroup, on 80 compute units, 14.5), the
+// serial kernel 101.
 constexpr int kW64SB = 8;
 
 // The serial kernel stays where it is the faster one: for few steps, since one pass of the scan costs as much as about twelve
@@ -599,18 +599,28 @@ static bool wkv_f64_scanned(int64_t channels, int64_t T) {
     return channels <= 100000 && T >= channels / 400;
 }
 
-template <int NC>
-__global__ void __launch_bounds__(NC * 32)
+// Channels per workgroup (CW).  A thread's chain is the same for each, so the fewest that leave no compute unit with two
+// workgroups; with more, 16, whose rounds are shorter, but for the few more that 256 workgroups of 32 still take in one.  Us with
+// 32 / 16 / 8, 256 steps: 512 channels (of all sequences) 13.9 / 9.0 / 7.1, 2048 14.3 / 9.7 / 7.8, 3072 14.5 / 10.0 / 10.7, 4096
+// 15.0 / 10.2 / 12.1, 4600 15.5 / 16.2 / 15.3, 8192 18.0 / 17.6 / 20.3, 9216 29.6 / 23.3 / 22.8, 40960 77.9 / 66.7 / 74.2; up to 64
+// steps they are equal or 32 is the fastest.
+static int wkv_f64_scan_width(int64_t channels, int64_t T) {
+    if (T <= 8 * kW64SB) return 32;
+    return channels <= 256 * 8 ? 8 : channels > 256 * 16 && channels <= 256 * 32 ? 32 : 16;
+}
+
+template <int NC, int CW>
+__global__ void __launch_bounds__(NC * CW)
 wkv_f64_scan_kernel(int T, int C, const double *__restrict__ w, const double *__restrict__ u, const double *__restrict__ k,
                     const double *__restrict__ v, double *__restrict__ y, double *__restrict__ aa, double *__restrict__ bb) {
-    __shared__ double sa[2][NC][32], sb[2][NC][32], sp[2][NC][32];
+    __shared__ double sa[2][NC][CW], sb[2][NC][CW], sp[2][NC][CW];
     constexpr int kBlk = NC * kW64SB;
     // the last round of the scan writes buffer 1, so that the next block's summaries may enter buffer 0 while other
     // wavefronts still read the result
     static_assert(NC == 8 || NC == 32, "an odd number of scan rounds");
-    const int per_b = (C + 31) / 32, b = blockIdx.x / per_b;
-    const int ch = threadIdx.x & 31, j = threadIdx.x >> 5;
-    const int cx = (blockIdx.x % per_b) * 32 + ch;
+    const int per_b = (C + CW - 1) / CW, b = blockIdx.x / per_b;
+    const int ch = threadIdx.x % CW, j = threadIdx.x / CW;
+    const int cx = (blockIdx.x % per_b) * CW + ch;
     const bool live = cx < C;
     const int c = live ? cx : C - 1;
     const size_t base = (size_t)b * T * C + c;
@@ -1002,12 +1012,16 @@ int rwkv_wkv_forward_f64(rwkv_stream_t stream, int64_t B, int64_t T, int64_t C,
     RWKV_CHECK_ARG(B > 0 && T > 0 && C > 0 && B * C < (1ll << 31) && T < (1ll << 31), "rwkv_wkv_forward_f64: bad sizes");
     RWKV_CHECK_ALIGN(k, 8); RWKV_CHECK_ALIGN(v, 8); RWKV_CHECK_ALIGN(y, 8);
     if (wkv_f64_scanned(B * C, T)) {
-        const dim3 grid((unsigned)(B * ceil_div(C, 32)));
+        const int cw = wkv_f64_scan_width(B * C, T);
+        const dim3 grid((unsigned)(B * ceil_div(C, cw)));
+#define RWKV_SCAN(NC, CW) \
+        hipLaunchKernelGGL((wkv_f64_scan_kernel<NC, CW>), grid, dim3(NC * CW), 0, (hipStream_t)stream, (int)T, (int)C, w, u, k, v, y, aa, bb)
         // short sequences: 8 chunks cover them and leave fewer threads idle; long ones: 32 chunks per block
-        if (T <= 8 * kW64SB)
-            hipLaunchKernelGGL(wkv_f64_scan_kernel<8>, grid, dim3(8 * 32), 0, (hipStream_t)stream, (int)T, (int)C, w, u, k, v, y, aa, bb);
-        else
-            hipLaunchKernelGGL(wkv_f64_scan_kernel<32>, grid, dim3(32 * 32), 0, (hipStream_t)stream, (int)T, (int)C, w, u, k, v, y, aa, bb);
+        if (T <= 8 * kW64SB) RWKV_SCAN(8, 32);
+        else if (cw == 8) RWKV_SCAN(32, 8);
+        else if (cw == 16) RWKV_SCAN(32, 16);
+        else RWKV_SCAN(32, 32);
+#undef RWKV_SCAN
         RWKV_CHECK_LAUNCH("wkv_f64_scan_kernel");
         return RWKV_OK;
     }

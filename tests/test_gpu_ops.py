@@ -373,7 +373,7 @@ def _calls(ops):
         yield "mm8_one", (n_in, n_out, x, w, y.half(), r)                                        # refused: type
         yield "mm8_one", (0, n_out, x, w, y, r)
         yield "mm8_three", (n_in, n_out, x, x, x, w, w[:, 1:1 + n_out], w, y, y.clone(), y.clone(), r, r, r)
-        yield "mm8_three", (n_in, n_out, x, x[:-1], x, w, w, w, y, y.clone(), y.clone(), r, r, r)
+        yield "mm8_three", (n_in, n_out, x, x, x, w, w[:-1], w, y, y.clone(), y.clone(), r, r, r)     # refused: size
     f = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64).cuda()
     wkv = lambda T, C: (2, T, C, -f(C), f(C), f(2, T, C), f(2, T, C), f(2, T, C), f(2, C), f(2, C) + 0.5, f(2, C))
     yield "wkv_forward", wkv(3, 5)
@@ -543,6 +543,12 @@ def test_wkv_forward_f64_any_length(ops, B, T, C):
 # both sides of the lengths from which so many channels are scanned, and more channels than are scanned at all
 @pytest.mark.parametrize("B,C,T", [(50, 640, 31), (50, 640, 32), (50, 640, 79), (50, 640, 80), (100, 1001, 65), (7, 160, 12)])
 def test_wkv_forward_f64_of_many_channels(ops, B, C, T):
+    _wkv_f64_case(ops, B, T, C)
+
+
+# the widths of the scan's workgroups: 8, 16, 32 and 16 channels, at the edges of the rule and with a ragged last one
+@pytest.mark.parametrize("B,C,T", [(1, 2048, 65), (1, 2049, 65), (2, 1030, 257), (1, 4096, 100), (1, 4097, 100), (8, 1024, 70), (3, 2731, 70)])
+def test_wkv_forward_f64_workgroup_widths(ops, B, C, T):
     _wkv_f64_case(ops, B, T, C)
 
 
