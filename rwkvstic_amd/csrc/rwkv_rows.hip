@@ -1109,7 +1109,10 @@ __device__ __forceinline__ void relu2_part(const GemmArgs &a, const v4i d, int m
     }
 }
 
-template <int MT, int NTW, int NW, int U, bool STREAM>
+// ROUNDS: more blocks to a wavefront than it has in flight (U a tile).  Each slot is then asked for again as soon as its block
+// has been multiplied, not when the whole round has.  (Where one round is all, that code would only be fetched: 24 layers of 1024,
+// 8 sequences, 965 -> 975 us.)
+template <int MT, int NTW, int NW, int U, bool STREAM, bool ROUNDS>
 __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
     __shared__ v4i red[NW][MT * NTW][64];
     const int lane = threadIdx.x & 63;
@@ -1143,16 +1146,18 @@ __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int j = 0; j < NTW; ++j) acc[m][j] = v4i{0, 0, 0, 0};
-    for (int k = kb0 + wave; k < kb1; k += NW * U) {
-        v4i B[NTW][U], A[MT][U];
+    v4i B[NTW][U], A[MT][U];
+    auto fetch = [&](int i, int kb) {
+        const size_t o = (size_t)min(kb, a.KB - 1) * 64;                  // past the end: a block nobody multiplies
 #pragma unroll
-        for (int i = 0; i < U; ++i) {
-            const size_t o = (size_t)min(k + NW * i, a.KB - 1) * 64;      // past the end: a block nobody multiplies
+        for (int j = 0; j < NTW; ++j) B[j][i] = ldw<STREAM>(bsrc[j] + o);
 #pragma unroll
-            for (int j = 0; j < NTW; ++j) B[j][i] = ldw<STREAM>(bsrc[j] + o);
+        for (int m = 0; m < MT; ++m) A[m][i] = asrc[m][o];
+    };
+    int k = kb0 + wave;
 #pragma unroll
-            for (int m = 0; m < MT; ++m) A[m][i] = asrc[m][o];
-        }
+    for (int i = 0; i < U; ++i) fetch(i, k + NW * i);
+    for (; k < kb1; k += NW * U) {
 #pragma unroll
         for (int i = 0; i < U; ++i) {
             if (k + NW * i < kb1) {         // uniform for the wavefront
@@ -1162,6 +1167,7 @@ __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
                     for (int j = 0; j < NTW; ++j)
                         acc[m][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[m][i], B[j][i], acc[m][j], 0, 0, 0);
             }
+            if (ROUNDS && k + NW * (U + i) < kb1) fetch(i, k + NW * (U + i));      // the slot is free
         }
     }
     // digit sums of at most a thousand blocks or so (plan_products splits longer contractions): inside int32
@@ -1689,33 +1695,55 @@ static bool rounded_apart(int64_t MT, int64_t NT, int64_t KB, int n) {
     return KB >= 16 && (NT * n < 128 || (NT * n < 512 && KB >= kGemmLongBlocks));
 }
 // Shape of the few-row kernel for a launch of so many column tiles: tiles per workgroup, wavefronts per workgroup, blocks
-// in flight per wavefront and tile.  All workgroups resident at once, 2000 to 4000 wavefronts where the tiles allow it; one
+// in flight per wavefront and tile (at most).  All workgroups resident at once, 2000 to 4000 wavefronts where the tiles allow it; one
 // tile per workgroup while that fills the device, more where the digits every wavefront reads would outweigh the weights.
 struct VecShape { int ntw, nw, u; };
 static VecShape vec_shape(int64_t tiles, int64_t KB) {
-    if (tiles > 1280) return VecShape{4, 8, 3};
-    if (tiles > 320) return tiles <= 512 ? VecShape{2, 16, 3} : VecShape{2, 8, 5};
-    if (tiles > 256) return VecShape{1, 8, 5};
-    return KB <= 48 ? VecShape{1, 16, 3} : VecShape{1, 16, 5};
+    VecShape v;
+    if (tiles > 1280) v = VecShape{4, 8, 3};
+    else if (tiles > 320) v = tiles <= 512 ? VecShape{2, 16, 3} : VecShape{2, 8, 5};
+    else if (tiles > 256) v = VecShape{1, 8, 5};
+    else v = VecShape{1, 16, 5};
+    // No more in flight than a wavefront has: what is past the end is loaded all the same.  With this and the refilled slots, us a
+    // step of 8 sequences before / now: 12 layers of 512 437 / 433, of 768 464 / 457, 24 of 1024 1014 / 965, 12 of 1536 625 / 597, 8
+    // of 2048 479 / 457, 12 of 2560 780 / 766, 8 of 4096 820 / 776, 4 of 5120 586 / 576.
+    const int64_t each = ceil_div(KB, v.nw);
+    if (each < v.u) v.u = each <= 1 ? 1 : each == 2 ? 2 : each == 3 ? 3 : v.u;
+    return v;
 }
 static void launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
     const int64_t tiles = g.NT2 > 0 ? (int64_t)g.NT + g.NT2 : (int64_t)g.NT * g.gz;
     const VecShape v = vec_shape(tiles, g.KB);
     const dim3 grid((unsigned)(g.NT2 > 0 ? ceil_div(g.NT, v.ntw) + ceil_div(g.NT2, v.ntw) : ceil_div(g.NT, v.ntw) * g.gz)), block((unsigned)(64 * v.nw));
-#define RWKV_VEC(NTW, NW, U)                                                                          \
-    if (v.ntw == NTW && v.nw == NW && v.u == U) {                                                     \
-        if (g.MT == 1 && stream) hipLaunchKernelGGL((gemv16_kernel<1, NTW, NW, U, true>), grid, block, 0, st, g);     \
-        else if (g.MT == 1) hipLaunchKernelGGL((gemv16_kernel<1, NTW, NW, U, false>), grid, block, 0, st, g);         \
-        else if (stream) hipLaunchKernelGGL((gemv16_kernel<2, NTW, NW, U, true>), grid, block, 0, st, g);             \
-        else hipLaunchKernelGGL((gemv16_kernel<2, NTW, NW, U, false>), grid, block, 0, st, g);        \
+#define RWKV_VEC_LAUNCH(MT, NTW, NW, U, ROUNDS)                                                                               \
+        if (stream) hipLaunchKernelGGL((gemv16_kernel<MT, NTW, NW, U, true, ROUNDS>), grid, block, 0, st, g);                 \
+        else hipLaunchKernelGGL((gemv16_kernel<MT, NTW, NW, U, false, ROUNDS>), grid, block, 0, st, g)
+#define RWKV_VEC(NTW, NW, U, ROUNDS)                                                                  \
+    if (v.ntw == NTW && v.nw == NW && v.u == U && (g.kb_per_split > NW * U) == ROUNDS) {              \
+        if (g.MT == 1) { RWKV_VEC_LAUNCH(1, NTW, NW, U, ROUNDS); }                                    \
+        else { RWKV_VEC_LAUNCH(2, NTW, NW, U, ROUNDS); }                                              \
     }
-    RWKV_VEC(4, 8, 3)
-    RWKV_VEC(2, 16, 3)
-    RWKV_VEC(2, 8, 5)
-    RWKV_VEC(1, 8, 5)
-    RWKV_VEC(1, 16, 3)
-    RWKV_VEC(1, 16, 5)
+    // (more than one round only with the most blocks in flight)
+    RWKV_VEC(4, 8, 1, false)
+    RWKV_VEC(4, 8, 2, false)
+    RWKV_VEC(4, 8, 3, false) RWKV_VEC(4, 8, 3, true)
+    RWKV_VEC(2, 16, 1, false)
+    RWKV_VEC(2, 16, 2, false)
+    RWKV_VEC(2, 16, 3, false) RWKV_VEC(2, 16, 3, true)
+    RWKV_VEC(2, 8, 1, false)
+    RWKV_VEC(2, 8, 2, false)
+    RWKV_VEC(2, 8, 3, false)
+    RWKV_VEC(2, 8, 5, false) RWKV_VEC(2, 8, 5, true)
+    RWKV_VEC(1, 8, 1, false)
+    RWKV_VEC(1, 8, 2, false)
+    RWKV_VEC(1, 8, 3, false)
+    RWKV_VEC(1, 8, 5, false) RWKV_VEC(1, 8, 5, true)
+    RWKV_VEC(1, 16, 1, false)
+    RWKV_VEC(1, 16, 2, false)
+    RWKV_VEC(1, 16, 3, false)
+    RWKV_VEC(1, 16, 5, false) RWKV_VEC(1, 16, 5, true)
 #undef RWKV_VEC
+#undef RWKV_VEC_LAUNCH
 }
 
 // Upper bound of the splits plan_products chooses for R rows, N columns and contractions of up to K, whatever the number of
