@@ -1077,7 +1077,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 
 // ---------------------------------------------------------------------------
 // The same product for at most 8 rows (MT <= 2 M-tiles: a single token of a shape the persistent kernel does
-// not serve, a small batch): pure weight streaming.  No LDS staging and no barrier in the loop: a workgroup has NTW
+// not serve, a small batch), and for up to 32 where the matrix is small (vec_rows): pure weight streaming.  No LDS staging and no barrier in the loop: a workgroup has NTW
 // column tiles and the whole contraction, its NW wavefronts take every NW-th block (together they read the tiles'
 // blocks in order) and each keeps U blocks per tile in flight on its own, so that a slow load holds up one wavefront,
 // not the workgroup.  The digit fragments (L2-resident) are read by every wavefront itself, once for its NTW tiles.
@@ -1089,7 +1089,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 // launch), 4 wavefronts of one tile with 8 blocks in flight / this: k, v, r 10.1 / 7.3, att output 7.4 / 5.4, ffn key and
 // receptance 12.7 + 6.4 / 10.1, ffn value 15.5 / 13.0, head 43 / 30.5.
 // ---------------------------------------------------------------------------
-constexpr int kVecMT = 2;
+constexpr int kVecMT = 2, kVecMTMax = 8;
 
 // The relu^2 tail of one tile (as gemm_tail's), and the tile's share of what rows_quant_tiles_kernel needs to know of the rows.
 __device__ __forceinline__ void relu2_part(const GemmArgs &a, const v4i d, int m, int nt, int lane) {
@@ -1097,7 +1097,9 @@ __device__ __forceinline__ void relu2_part(const GemmArgs &a, const v4i d, int m
     const bool live = t < a.R;
     const int tc = live ? t : a.R - 1;
     const double tot = (double)(((((long long)d.x * 256 + d.y) * 256 + d.z) * 256) + d.w);
-    const double y = a.S[0][tc] * tot + (128.0 * (a.S[0][tc] * a.qs[0][tc]) + a.zp[0][tc]), r = y > 0.0 ? y : 0.0;
+    const double sq = 128.0 * (a.S[0][tc] * a.qs[0][tc]), zp = a.zp[0][tc];
+    const bool apart = a.MT > 2 && a.apart;             // (up to 8 rows whole contractions always ended here)
+    const double y = (a.S[0][tc] * tot + (apart ? sq : sq + zp)) + (apart ? zp : -0.0), r = y > 0.0 ? y : 0.0;
     const float h = (float)(r * r);
     if (live) reinterpret_cast<float *>(a.out[0])[(size_t)t * a.N + col] = h;
     const double v = live ? (double)h : 0.0;
@@ -1191,7 +1193,8 @@ __global__ void __launch_bounds__(64 * NW) gemv16_kernel(const GemmArgs a) {
 // Quantiser of a product whose tiles left their share of every row (relu2_part): a part of 1024 values per workgroup, one launch
 // instead of a pass for the rows' maxima and one for the digits (8 rows of 10240: 4.7 us against 3.9 + 4.0).  A step of 8
 // sequences at 3B 2.08 -> 2.04 ms, of 5 at 24 layers of 2048 1.40 -> 1.34, of 8 at 24 layers of 1024 1.033 -> 1.019; not for rows
-// up to 3072, which one workgroup each quantises as fast (12 layers of 768, 8 sequences: 451 us that way, 458 this).  The sum of
+// up to 3072, which one workgroup each quantises as fast (12 layers of 768, 8 sequences: 451 us that way, 458 this).  9 and 16
+// sequences: 12 layers of 2560 855 -> 834 and 928 -> 906, 24 of 1024 1050 -> 1015 and 1089 -> 1058.  The sum of
 // the fixed-point values is added up with atomics: integers below 2^53, exact in
 // any order.
 __global__ void __launch_bounds__(kRT) rows_quant_tiles_kernel(const QuantArgs a, const double2 *part, int tiles) {
@@ -1659,11 +1662,29 @@ constexpr int kGemmFillWgs = 96;         // larger products: split until the gri
 // totals buffer both call it, so the buffer always holds every slice the kernel writes.
 enum { PLAN_VEC = 0, PLAN_SKINNY, PLAN_GENERAL, PLAN_WIDE };
 struct ProductPlan { int kind, gx, gy, split; };
+// Which products of 9 to 32 rows go through gemv16_kernel.  Every workgroup of it reads the digits of all rows, gemm8_skinny_kernel
+// shares them between four wavefronts of eight tiles but needs slices of the contraction, and launches that add them up, to fill
+// the device.  So: few tiles, short contractions.  Us a step of 9, 16 / 17, 32 sequences, all through the other kernel / by this rule:
+// 12 layers of 512 658, 668 / 684, 722 against 448, 460 / 475, 497; 24 of 1024 1500, 1549 / 1590, 1750 against 1048, 1086 / 1151,
+// 1300; 12 of 1536 884, 908 / 935, 1036 against 652, 690 / 744, 815; 8 of 2048 582, 600 / 615, 665 against 512, 538 / 590, 645; 12 of 2560
+// 985, 1028 / 1057, 1165 against 860, 935 / 1005, 1096; 8 of 4096 905, 920 / 950, 1025 against 865, 905 / 930, 1024.  Beyond it that
+// kernel wins: three M-tiles of 5120 channels 561 against 572, four 601 against 615 to 646, five of 4096 951 against 978 with its 768 tiles of k, v, r.
+static bool vec_rows(int64_t MT, int64_t tiles, int64_t KB) {
+    if (MT <= kVecMT) return true;
+    if (MT <= 4) return tiles <= 1280 && MT * KB <= (tiles <= 256 ? 700 : 200);
+    return MT <= kVecMTMax && tiles <= 512 && MT * KB <= 400;
+}
+// Slices of a contraction of 9 to 32 rows in gemm8_skinny_kernel, whether it is the kernel that runs or not (see rounded_apart).
+static int skinny_split(int64_t NT, int64_t KB, int n) {
+    int split = 1;
+    while (ceil_div(NT, kSkinnyNT) * n * split < kSkinnyFillWgs && KB / (split * 2) >= 8 && split < kMaxSplit) split *= 2;
+    return split;
+}
 static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n) {
     ProductPlan p;
     p.split = 1;
-    if (MT <= kVecMT) {
-        // a handful of rows: whole contractions, as long as a digit's sum of them stays inside int32 (2^20 per block)
+    if (vec_rows(MT, NT * n, KB)) {
+        // few rows: whole contractions, as long as a digit's sum of them stays inside int32 (2^20 per block)
         p.kind = PLAN_VEC; p.gx = (int)NT; p.gy = 1;
         while (ceil_div(KB, p.split) > 1024 && p.split < kMaxSplit) p.split *= 2;
         return p;
@@ -1680,8 +1701,9 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n) {
     }
     p.gx = (int)ceil_div(NT, p.kind == PLAN_SKINNY ? kSkinnyNT : p.kind == PLAN_WIDE ? kGemmWideNT : kGemmNT);
     // Split the contraction until the grid has a few workgroups per compute unit.
-    const int fill = p.kind == PLAN_SKINNY ? kSkinnyFillWgs : kGemmFillWgs;
-    while ((int64_t)p.gx * p.gy * n * p.split < fill && KB / (p.split * 2) >= 8 && p.split < kMaxSplit) p.split *= 2;
+    if (p.kind == PLAN_SKINNY) p.split = skinny_split(NT, KB, n);
+    else
+        while ((int64_t)p.gx * p.gy * n * p.split < kGemmFillWgs && KB / (p.split * 2) >= 8 && p.split < kMaxSplit) p.split *= 2;
     // a long contraction on a grid still below the device: one split more (two slices at most)
     if (p.kind != PLAN_SKINNY && p.split == 1 && (int64_t)p.gx * p.gy * n < kGemmLongFillWgs && KB >= kGemmLongBlocks) p.split = 2;
     return p;
@@ -1691,19 +1713,21 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n) {
 // most 32 rows that once were split run whole contractions now and keep the first: the last bit of y reaches the logits, and
 // with them the texts of a seeded sampler.
 static bool rounded_apart(int64_t MT, int64_t NT, int64_t KB, int n) {
-    if (MT > kVecMT) return plan_products(MT, NT, KB, n).split > 1;
+    if (MT > kVecMT) return MT <= kSkinnyMT ? skinny_split(NT, KB, n) > 1 : plan_products(MT, NT, KB, n).split > 1;
     return KB >= 16 && (NT * n < 128 || (NT * n < 512 && KB >= kGemmLongBlocks));
 }
 // Shape of the few-row kernel for a launch of so many column tiles: tiles per workgroup, wavefronts per workgroup, blocks
 // in flight per wavefront and tile (at most).  All workgroups resident at once, 2000 to 4000 wavefronts where the tiles allow it; one
 // tile per workgroup while that fills the device, more where the digits every wavefront reads would outweigh the weights.
 struct VecShape { int ntw, nw, u; };
-static VecShape vec_shape(int64_t tiles, int64_t KB) {
+static VecShape vec_shape(int64_t tiles, int64_t KB, int MT) {
     VecShape v;
-    if (tiles > 1280) v = VecShape{4, 8, 3};
+    if (MT > 4) v = tiles > 256 ? VecShape{2, 8, 2} : VecShape{1, 16, 2};       // (128 KB of sums in LDS)
+    else if (tiles > 1280) v = VecShape{4, 8, 3};
     else if (tiles > 320) v = tiles <= 512 ? VecShape{2, 16, 3} : VecShape{2, 8, 5};
     else if (tiles > 256) v = VecShape{1, 8, 5};
     else v = VecShape{1, 16, 5};
+    if (MT > 2 && v.u > 3) v.u = 3;                     // (registers)
     // No more in flight than a wavefront has: what is past the end is loaded all the same.  With this and the refilled slots, us a
     // step of 8 sequences before / now: 12 layers of 512 437 / 433, of 768 464 / 457, 24 of 1024 1014 / 965, 12 of 1536 625 / 597, 8
     // of 2048 479 / 457, 12 of 2560 780 / 766, 8 of 4096 820 / 776, 4 of 5120 586 / 576.
@@ -1713,37 +1737,62 @@ static VecShape vec_shape(int64_t tiles, int64_t KB) {
 }
 static void launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
     const int64_t tiles = g.NT2 > 0 ? (int64_t)g.NT + g.NT2 : (int64_t)g.NT * g.gz;
-    const VecShape v = vec_shape(tiles, g.KB);
+    const VecShape v = vec_shape(tiles, g.KB, g.MT);
     const dim3 grid((unsigned)(g.NT2 > 0 ? ceil_div(g.NT, v.ntw) + ceil_div(g.NT2, v.ntw) : ceil_div(g.NT, v.ntw) * g.gz)), block((unsigned)(64 * v.nw));
 #define RWKV_VEC_LAUNCH(MT, NTW, NW, U, ROUNDS)                                                                               \
         if (stream) hipLaunchKernelGGL((gemv16_kernel<MT, NTW, NW, U, true, ROUNDS>), grid, block, 0, st, g);                 \
         else hipLaunchKernelGGL((gemv16_kernel<MT, NTW, NW, U, false, ROUNDS>), grid, block, 0, st, g)
-#define RWKV_VEC(NTW, NW, U, ROUNDS)                                                                  \
-    if (v.ntw == NTW && v.nw == NW && v.u == U && (g.kb_per_split > NW * U) == ROUNDS) {              \
-        if (g.MT == 1) { RWKV_VEC_LAUNCH(1, NTW, NW, U, ROUNDS); }                                    \
-        else { RWKV_VEC_LAUNCH(2, NTW, NW, U, ROUNDS); }                                              \
+#define RWKV_VEC(MT_, LO, HI, NTW, NW, U, ROUNDS)                                                     \
+    if (g.MT >= LO && g.MT <= HI && v.ntw == NTW && v.nw == NW && v.u == U && (g.kb_per_split > NW * U) == ROUNDS) { \
+        RWKV_VEC_LAUNCH(MT_, NTW, NW, U, ROUNDS); return;                                             \
     }
+#define RWKV_VEC12(NTW, NW, U, ROUNDS) RWKV_VEC(1, 1, 1, NTW, NW, U, ROUNDS) RWKV_VEC(2, 2, 2, NTW, NW, U, ROUNDS)
+#define RWKV_VEC34(NTW, NW, U, ROUNDS) RWKV_VEC(3, 3, 3, NTW, NW, U, ROUNDS) RWKV_VEC(4, 4, 4, NTW, NW, U, ROUNDS)
+// (above 16 rows one kernel for two counts of M-tiles: the last one may be a copy)
+#define RWKV_VEC68(NTW, NW, U, ROUNDS) RWKV_VEC(6, 5, 6, NTW, NW, U, ROUNDS) RWKV_VEC(8, 7, 8, NTW, NW, U, ROUNDS)
     // (more than one round only with the most blocks in flight)
-    RWKV_VEC(4, 8, 1, false)
-    RWKV_VEC(4, 8, 2, false)
-    RWKV_VEC(4, 8, 3, false) RWKV_VEC(4, 8, 3, true)
-    RWKV_VEC(2, 16, 1, false)
-    RWKV_VEC(2, 16, 2, false)
-    RWKV_VEC(2, 16, 3, false) RWKV_VEC(2, 16, 3, true)
-    RWKV_VEC(2, 8, 1, false)
-    RWKV_VEC(2, 8, 2, false)
-    RWKV_VEC(2, 8, 3, false)
-    RWKV_VEC(2, 8, 5, false) RWKV_VEC(2, 8, 5, true)
-    RWKV_VEC(1, 8, 1, false)
-    RWKV_VEC(1, 8, 2, false)
-    RWKV_VEC(1, 8, 3, false)
-    RWKV_VEC(1, 8, 5, false) RWKV_VEC(1, 8, 5, true)
-    RWKV_VEC(1, 16, 1, false)
-    RWKV_VEC(1, 16, 2, false)
-    RWKV_VEC(1, 16, 3, false)
-    RWKV_VEC(1, 16, 5, false) RWKV_VEC(1, 16, 5, true)
+    RWKV_VEC12(4, 8, 1, false)
+    RWKV_VEC12(4, 8, 2, false)
+    RWKV_VEC12(4, 8, 3, false) RWKV_VEC12(4, 8, 3, true)
+    RWKV_VEC12(2, 16, 1, false)
+    RWKV_VEC12(2, 16, 2, false)
+    RWKV_VEC12(2, 16, 3, false) RWKV_VEC12(2, 16, 3, true)
+    RWKV_VEC12(2, 8, 1, false)
+    RWKV_VEC12(2, 8, 2, false)
+    RWKV_VEC12(2, 8, 3, false)
+    RWKV_VEC12(2, 8, 5, false) RWKV_VEC12(2, 8, 5, true)
+    RWKV_VEC12(1, 8, 1, false)
+    RWKV_VEC12(1, 8, 2, false)
+    RWKV_VEC12(1, 8, 3, false)
+    RWKV_VEC12(1, 8, 5, false) RWKV_VEC12(1, 8, 5, true)
+    RWKV_VEC12(1, 16, 1, false)
+    RWKV_VEC12(1, 16, 2, false)
+    RWKV_VEC12(1, 16, 3, false)
+    RWKV_VEC12(1, 16, 5, false) RWKV_VEC12(1, 16, 5, true)
+    RWKV_VEC34(4, 8, 1, false)
+    RWKV_VEC34(4, 8, 2, false)
+    RWKV_VEC34(4, 8, 3, false) RWKV_VEC34(4, 8, 3, true)
+    RWKV_VEC34(2, 16, 1, false)
+    RWKV_VEC34(2, 16, 2, false)
+    RWKV_VEC34(2, 16, 3, false) RWKV_VEC34(2, 16, 3, true)
+    RWKV_VEC34(2, 8, 1, false)
+    RWKV_VEC34(2, 8, 2, false)
+    RWKV_VEC34(2, 8, 3, false) RWKV_VEC34(2, 8, 3, true)
+    RWKV_VEC34(1, 8, 1, false)
+    RWKV_VEC34(1, 8, 2, false)
+    RWKV_VEC34(1, 8, 3, false) RWKV_VEC34(1, 8, 3, true)
+    RWKV_VEC34(1, 16, 1, false)
+    RWKV_VEC34(1, 16, 2, false)
+    RWKV_VEC34(1, 16, 3, false) RWKV_VEC34(1, 16, 3, true)
+    RWKV_VEC68(2, 8, 1, false)
+    RWKV_VEC68(2, 8, 2, false) RWKV_VEC68(2, 8, 2, true)
+    RWKV_VEC68(1, 16, 1, false)
+    RWKV_VEC68(1, 16, 2, false) RWKV_VEC68(1, 16, 2, true)
 #undef RWKV_VEC
 #undef RWKV_VEC_LAUNCH
+#undef RWKV_VEC12
+#undef RWKV_VEC34
+#undef RWKV_VEC68
 }
 
 // Upper bound of the splits plan_products chooses for R rows, N columns and contractions of up to K, whatever the number of
@@ -1969,7 +2018,7 @@ int rows_ffn_key_receptance(hipStream_t st, bool sequence, const RowsProduct &k,
     g.NT2 = (int)ceil_div(C, 16); g.N2 = (int)C; g.tail2 = ROW_STORE_F32;
     g.apart = rounded_apart(g.MT, g.NT, g.KB, 1); g.apart2 = rounded_apart(g.MT, g.NT2, g.KB, 1);
     const int gx = (int)(ceil_div(g.NT, kSkinnyNT) + ceil_div(g.NT2, kSkinnyNT));
-    if (C % 64 == 0 && g.MT <= kVecMT && g.KB <= 1024) {
+    if (C % 64 == 0 && vec_rows(g.MT, g.NT + g.NT2, g.KB) && g.KB <= 1024) {
         g.gx = g.NT; g.per_xcd = 0;
         // (not for the rows of a sequence: the tiles add up the zero-point term in another order than rows_quant does, and the
         // last bit of it reaches the logits and a seeded sampler's texts)

@@ -618,11 +618,17 @@ def test_gemm8_matches_fp64_dense(ops, T, K, N):
     assert err < 2e-7                                         # float32 rounding of x*range, nothing else
 
 
-# at most 8 rows: both sides of the column tiles at which the kernel changes its shape (256 | 320 | 512 | 1280), of the
-# contraction length at which it does (48 blocks), fewer blocks than wavefronts, one block past a round, a split contraction
+# at most 8 rows: both sides of the column tiles at which the kernel changes its shape (256 | 320 | 512 | 1280),
+# fewer blocks than wavefronts, one block past a round, a split contraction
 @pytest.mark.parametrize("T,K,N", [(1, 64, 16), (8, 17 * 64, 4096), (8, 17 * 64, 4100), (3, 192, 5120), (5, 41 * 64, 5121), (4, 448, 8192),
                                    (8, 41 * 64, 8200), (8, 192, 20480), (7, 25 * 64, 20490), (6, 49 * 64, 4096), (8, 81 * 64, 256),
-                                   (2, 1025 * 64, 20)])
+                                   (2, 1025 * 64, 20),
+                                   # 9 to 32 rows of small matrices: every count of M-tiles, tiles (256 | 320 | 512 | 1280) and
+                                   # contractions (blocks times M-tiles 200 | 700, 400) on both sides of the rules' edges
+                                   (9, 64, 16), (12, 17 * 64, 4100), (13, 50 * 64, 4112), (16, 50 * 64, 4112), (16, 51 * 64, 4112), (10, 100 * 64, 8192),
+                                   (16, 175 * 64, 4096), (15, 176 * 64, 4096), (11, 33 * 64, 8200), (14, 5 * 64, 20480), (9, 6 * 64, 20490),
+                                   (17, 64, 16), (20, 80 * 64, 4096), (24, 66 * 64, 4097), (25, 50 * 64, 8192), (32, 50 * 64, 8192), (32, 51 * 64, 8192),
+                                   (29, 17 * 64, 8193), (32, 64, 50), (21, 33 * 64, 4100)])
 def test_few_row_products_match_fp64_dense(ops, T, K, N):
     g = torch.Generator().manual_seed(T * 7 + K + N)
     codes = torch.randint(0, 256, (K, N), generator=g, dtype=torch.uint8)
