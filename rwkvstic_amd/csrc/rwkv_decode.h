@@ -48,6 +48,7 @@ static_assert(sizeof(DScal) == 128, "DScal is read as a 128-byte record");
 struct DModel {
     int L, C, F, V, G;           // G = C / 16 groups of 16 channels
     int NWG;                     // workgroups of the single-token kernel: G, or G / 2 where a workgroup owns two groups (C = 5120)
+    int n_cand;                  // workgroups that leave a candidate for the greedy token
     const float *emb;
     const double *ln0_w, *ln0_b;
     const uint8_t *w_head;
@@ -67,7 +68,7 @@ struct DModel {
     double *PO;                  // [L+1][5][C]
     DScal *sc;                   // [L+1]
     DScal *scp;                  // [L][C/512] per-token scalars (sumQO, maxQ) of each 512-channel part of a layer
-    double *amax_val;            // [NWG] device-side argmax: first maximum of the logits each workgroup wrote, and its index
+    double *amax_val;            // [n_cand] device-side argmax: first maximum of the logits each workgroup wrote, and its index
     int *amax_idx;
     double *X0;                  // [C] ln0(emb[token]) of the launch in flight
 };

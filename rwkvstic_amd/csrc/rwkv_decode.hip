@@ -3,8 +3,8 @@
 //
 // One launch of decode_kernel = one token through every layer and the head; a
 // small launch of prep_kernel before it turns the token and the shift state
-// into the per-token constants.  The grid is C/16 workgroups, all resident at
-// once; workgroup g owns the 16 channels [16g, 16g+16) for the whole token
+// into the per-token constants.  The grid is C/16 workgroups (and those of
+// HelperShape and HeadShape), all resident at once; workgroup g owns the 16 channels [16g, 16g+16) for the whole token
 // (their residual value, WKV state and receptance gate stay in its LDS) and
 // the matching 16-column tiles of every matrix.
 //
@@ -58,7 +58,7 @@ namespace rwkv {
 typedef int v4i __attribute__((ext_vector_type(4)));
 
 // Widths.  C = 512, 768 and 1536 are bound by the four exchanges per layer (12.3 us per layer at 768): a token of the
-// 12-layer 768 shape takes 170 us, as one-row prompts through the many-row kernels it took 630 us (146 launches).
+// 12-layer 768 shape takes 158 us, as one-row prompts through the many-row kernels it took 630 us (146 launches).
 // NB (template parameter throughout): 64-channel blocks of a row of C channels, C = 64 NB.  Back (streaming) waves per
 // workgroup: eight, four up to 1024 channels, where the exchanges and not the stream set the pace and a tile's sums come
 // from four parts instead of eight (24 layers of 1024: 336 us a token, with eight 344; at 1536 they are equal, at 2048 four
@@ -128,6 +128,22 @@ struct HelperShape {
     static constexpr int LDS_BLOCKS = 4;                           // weight blocks per wavefront that wait in LDS instead of registers
 };
 
+// Head workgroups.  Up to 1024 channels the owners are 32 to 64 workgroups, and the head, a third of a small model's bytes, took
+// them as long as one or two layers: 18 us of a 170 us token at 768 channels.  Compute units they leave free get a workgroup each
+// that holds its share of the head on chip, fetched while the layers run, waits for the last residual and finishes the
+// logits; the owners have no head tiles.  Us a token before / now: 12 layers of 768 172 / 158, 2 of 768 53 / 40, 24 of 512 302 / 289,
+// 12 and 24 of 1024 179 / 167, 337 / 327.  Owners and head workgroups together leave 64 compute units to other streams (with
+// those used too: the same within 1 us; with 128 in all 337 us for 24 layers of 1024).
+constexpr int kHeadGrid = 192;
+// s_sleep units (64 cycles) per layer between two blocks a head workgroup asks for, so that its fetches last about half a token: as
+// one burst they stood in the way of the first layers' (24 layers of 1024, with 1 / 4 / 8 / 12 and in a burst: 329 / 328 / 327 / 329, 336 us).
+constexpr int kHeadPace = 8;
+template <int NB>
+struct HeadShape {
+    static constexpr int NH = NB <= 16 ? kHeadGrid - 4 * NB : 0;   // head workgroups (every workgroup has a compute unit of its own)
+    static constexpr int HELD = 2 * NB < 24 ? 2 * NB : 24;          // weight blocks a wavefront holds
+};
+
 struct DArgs {
     DModel m;
     DecodeBuffers b;
@@ -139,6 +155,15 @@ struct DArgs {
     const int *stop;        // device word or null: when it reads non-zero the launch does nothing (a sampled stop token
                             // ended the sequence; the remaining launches of a generation loop then leave the state alone)
 };
+
+// The kernel's arguments read again from where they lie.  What a workgroup's part needs of them is kept in scalar registers from
+// the kernel's entry on, for all parts together, and what does not fit is parked in vector registers and fetched back lane
+// by lane; the pointer here is opaque, so a part that reads its arguments through it costs the others none.
+__device__ __forceinline__ const DArgs &arguments_again() {
+    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const DArgs *)p;       // (the first argument)
+}
 
 // ---- the back (weight-streaming) waves ------------------------------------------
 // Their program is generated (gen_decode_back.py -> rwkv_decode_back.inc): one asm statement with
@@ -730,7 +755,7 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
     Front fx;
     fx.abort_flag = a.b.abort_flag; fx.flags = flags; fx.spin_limit = a.spin_limit; fx.ok = true;
     fx.refresh();
-    const int wg = blockIdx.x, L = a.m.L, V = a.m.V;
+    const int wg = blockIdx.x, L = a.m.L;
     const bool fin = fx.wave < NT;                       // wave gi finishes the workgroup's group gi of 16 channels
     const int gi = fin ? fx.wave : 0;
     const int g = NT * wg + gi;
@@ -882,8 +907,17 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
         }
     }
 
+    if constexpr (HeadShape<NB>::NH > 0) {                // the head is other workgroups'
+        if (!fx.ok) return;
+        __syncthreads(); __syncthreads();                 // (the back waves' program passes the head's two barriers)
+        for (int i = fx.tid; i < L * 5 * 16; i += FT) a.state[(size_t)(i >> 4) * C + 16 * wg + (i & 15)] = st_lds[i];
+        if (TRACE)
+            for (int i = fx.tid; i < L * kTraceStampsPerLayer; i += FT) a.b.trace[(size_t)wg * L * kTraceStampsPerLayer + i] = trace_lds[i];
+        return;
+    }
     // ========================= head (opt.py:71-73) ==============================
-    const int v_tiles = (V + 15) / 16, head_rounds = (v_tiles + NWG - 1) / NWG;
+    const DArgs &ah = arguments_again();
+    const int V = ah.m.V, v_tiles = (V + 15) / 16, head_rounds = (v_tiles + NWG - 1) / NWG;
     red -= gi * kSlotsPerGroup * BW * 16;                 // the head's parked tiles belong to the workgroup
     const u64 *rec_h = own_lds + (L & 1) * kOrSlots;
     // column sums of the workgroup's head tiles: requested now, parked in LDS (where there is no
@@ -895,11 +929,11 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
 #pragma unroll
     for (int k = 0; k < HCS; ++k) {
         const int i = fx.tid + FT * k, v = 16 * (wg + NWG * (i >> 4)) + (i & 15);
-        csv[k] = (i < head_rounds * 16 && v < V) ? a.m.cs_head[v] : 0;
+        csv[k] = (i < head_rounds * 16 && v < V) ? ah.m.cs_head[v] : 0;
     }
     if (fx.ok)
-        ln_front<NB, FW, 1>(fx, seq, a, a.m.P32 + (size_t)L * kLnMats * C, a.m.Q32 + (size_t)L * kLnMats * C, rec_h, 0,
-                            a.epoch0 + 4u * (unsigned)L, dig, stat, nullptr, nullptr);
+        ln_front<NB, FW, 1>(fx, seq, ah, ah.m.P32 + (size_t)L * kLnMats * C, ah.m.Q32 + (size_t)L * kLnMats * C, rec_h, 0,
+                            ah.epoch0 + 4u * (unsigned)L, dig, stat, nullptr, nullptr);
     if (!fx.ok) return;     // every wave leaves after the same barrier: the flag is tested after each one that follows a wait
 #pragma unroll
     for (int k = 0; k < HCS; ++k)
@@ -921,7 +955,7 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
             const int v = 16 * (wg + NWG * (h0 + s)) + n;
             if (v < V) {
                 const double y = finish_col<BW>(red + par * (NS * BW * 16), s, n, Sh, csh[16 * (h0 + s) + n], zph);
-                a.logits[v] = y;
+                ah.logits[v] = y;
                 if (y > best) { best = y; best_i = v; }    // v grows with the round: an equal later value does not replace
             }
         }
@@ -934,13 +968,13 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
             const int oi = __shfl_xor(best_i, off, 64);
             if (ob > best || (ob == best && oi < best_i)) { best = ob; best_i = oi; }
         }
-        if (fx.lane == 0) { a.m.amax_val[wg] = best; a.m.amax_idx[wg] = best_i; }
+        if (fx.lane == 0) { ah.m.amax_val[wg] = best; ah.m.amax_idx[wg] = best_i; }
     }
     // the state rows of the own channels: st_lds[l][row][n] -> state[l][row][16 g + n]
     if constexpr (NT == 1)
-        for (int i = fx.tid; i < L * 5 * 16; i += FT) a.state[(size_t)(i >> 4) * C + 16 * wg + (i & 15)] = st_lds[i];
+        for (int i = fx.tid; i < L * 5 * 16; i += FT) ah.state[(size_t)(i >> 4) * C + 16 * wg + (i & 15)] = st_lds[i];
     if (TRACE)
-        for (int i = fx.tid; i < L * kTraceStampsPerLayer; i += FT) a.b.trace[(size_t)wg * L * kTraceStampsPerLayer + i] = trace_lds[i];
+        for (int i = fx.tid; i < L * kTraceStampsPerLayer; i += FT) ah.b.trace[(size_t)wg * L * kTraceStampsPerLayer + i] = trace_lds[i];
 }
 
 
@@ -1145,6 +1179,109 @@ __device__ __forceinline__ void helper_path(const DArgs &a, signed char *dig, v4
     }
 }
 
+// =============================================================================
+// A head workgroup (see HeadShape).  All its wavefronts gather and quantise the last residual; wavefront w multiplies tiles
+// h + NH (w + NWV r), r = 0, 1, ..., whole contractions, and finishes their 16 columns itself.  Of the first two tiles the
+// first HELD blocks have been waiting in registers.
+template <int NB, int FW, bool STREAM>
+__device__ __forceinline__ void head_path(const DArgs &a, signed char *dig, double *stat, lds_flag_t *flags, u64 *rec, double *best_lds) {
+    constexpr int NWG = GroupShape<NB>::NWG, NH = HeadShape<NB>::NH, HELD = HeadShape<NB>::HELD, NWV = FW + back_waves(NB), FT = 64 * NWV;
+    constexpr int C = 64 * NB, PS = C + 64, LATE = 2 * NB - HELD;
+    static_assert(HELD >= NB, "the first tile is held whole");
+    Front fx;
+    fx.abort_flag = a.b.abort_flag; fx.flags = flags; fx.spin_limit = a.spin_limit; fx.ok = true;
+    fx.refresh();
+    const int h = (int)blockIdx.x - NWG, L = a.m.L, V = a.m.V, v_tiles = (V + 15) / 16;
+    const int tile0 = h + NH * fx.wave, tile1 = tile0 + NH * NWV;
+    auto blk = [&](int tile, int b) {                      // (clamped: a tile past the end is loaded and not used)
+        return (const RWKV_GLOBAL v4i *)(a.m.w_head + ((size_t)(tile < v_tiles ? tile : v_tiles - 1) * NB + b) * 1024 + fx.lane * 16);
+    };
+    auto weight = [](const RWKV_GLOBAL v4i *p) -> v4i { return STREAM ? __builtin_nontemporal_load(p) : *p; };
+    v4i W[HELD];
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+        for (int l = 0; l < L; ++l) asm volatile("s_sleep %0" :: "n"(kHeadPace) : "memory");
+        W[i] = weight(blk(i < NB ? tile0 : tile1, i % NB));
+    }
+    const int n = fx.lane & 15;
+    auto colsum = [&](int tile) { return gld(a.m.cs_head + min(16 * tile + n, V - 1)); };
+    const int cs0 = colsum(tile0), cs1 = colsum(tile1);
+    if (fx.tid < 16) rec[kOrScal + fx.tid] = gld(reinterpret_cast<const u64 *>(a.m.sc + L) + fx.tid);       // the head's scalars
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) asm volatile("" : "+v"(W[i]));       // (here, not where they are used)
+    // The last residual is a whole token away.  One word of X says how far the layers are: a look, then a sleep of two
+    // thirds of what a layer takes for each one still to come, so that hardly anybody looks while they run.
+    const unsigned last = a.epoch0 + 4u * (unsigned)L;
+    if (fx.wave == 0) {
+        for (unsigned looks = 0;; ++looks) {
+            const unsigned behind = min(last - (unsigned)(ALOAD(a.b.X) >> 32), 4u * (unsigned)L);       // (an older token's word: everything)
+            if (behind <= 2) break;
+            if (looks > fx.spin_limit || ALOAD32(fx.abort_flag) != 0u) { fx.fail(); break; }
+            for (unsigned i = 0; i < behind - 2; ++i) __builtin_amdgcn_s_sleep(75);                     // 4800 cycles, 2 us
+        }
+    }
+    __syncthreads();
+    if (flags[FLAG_ABORT]) return;
+    int seq = 0;
+    ln_front<NB, NWV, 1>(fx, seq, a, a.m.P32 + (size_t)L * kLnMats * C, a.m.Q32 + (size_t)L * kLnMats * C, rec, 0, last, dig, stat, nullptr, nullptr);
+    if (!fx.ok) return;
+    double S;
+    float invS;
+    ln_scale(stat, rec, 0, 0, S, invS);
+    const double zp = ln_zp(stat, rec, 0, 0);
+    double best = -INFINITY;
+    int best_i = 0x7fffffff;
+    // rows 0 .. 3 of a product are the four digit sums of column lane < 16: finish_col of one part
+    auto finish = [&](int tile, const v4i d, int cs) {
+        const int v = 16 * tile + n;
+        if (fx.lane < 16 && v < V) {
+            const double tot = fma(fma(fma((double)d.x, 256.0, (double)d.y), 256.0, (double)d.z), 256.0, (double)d.w);
+            const double y = fma(S, tot + (double)(0x808080LL * (long long)cs), zp);
+            a.logits[v] = y;
+            if (y > best) { best = y; best_i = v; }        // v grows from tile to tile
+        }
+    };
+    const signed char *ap = dig + (fx.lane & 3) * PS + 16 * (fx.lane >> 4);
+    {
+        v4i late[LATE > 0 ? LATE : 1];
+#pragma unroll
+        for (int i = 0; i < LATE; ++i) late[i] = weight(blk(tile1, NB - LATE + i));
+        v4i acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const v4i A = *reinterpret_cast<const v4i *>(ap + 64 * b);
+            acc0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, W[b], acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, b < NB - LATE ? W[b < NB - LATE ? NB + b : 0] : late[b < NB - LATE ? 0 : b - (NB - LATE)], acc1, 0, 0, 0);
+        }
+        finish(tile0, acc0, cs0);
+        finish(tile1, acc1, cs1);
+    }
+    for (int tile = tile1 + NH * NWV; tile < v_tiles; tile += NH * NWV) {       // vocabularies beyond two tiles a wavefront
+        v4i w[NB], acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int b = 0; b < NB; ++b) w[b] = weight(blk(tile, b));
+        const int cs = colsum(tile);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(*reinterpret_cast<const v4i *>(ap + 64 * b), w[b], acc, 0, 0, 0);
+        finish(tile, acc, cs);
+    }
+    // the workgroup's candidate for the greedy token
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) {
+        const double ob = __shfl_xor(best, off, 64);
+        const int oi = __shfl_xor(best_i, off, 64);
+        if (ob > best || (ob == best && oi < best_i)) { best = ob; best_i = oi; }
+    }
+    int *idx_lds = reinterpret_cast<int *>(best_lds + NWV);
+    if (fx.lane == 0) { best_lds[fx.wave] = best; idx_lds[fx.wave] = best_i; }
+    __syncthreads();
+    if (fx.tid == 0) {
+        for (int w = 1; w < NWV; ++w)
+            if (best_lds[w] > best || (best_lds[w] == best && idx_lds[w] < best_i)) { best = best_lds[w]; best_i = idx_lds[w]; }
+        a.m.amax_val[h] = best; a.m.amax_idx[h] = best_i;
+    }
+}
+
 template <int NB, int FW, bool HELP = false>
 struct DecodeLds {
     using Back = BackOf<NB, FW, HELP>;
@@ -1188,7 +1325,13 @@ __global__ void __launch_bounds__((FW + back_waves(NB)) * 64) decode_kernel(cons
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     if constexpr (HELP) {
         if ((int)blockIdx.x >= GroupShape<NB>::NWG) {          // (uniform for the workgroup)
-            helper_path<NB, FW, STREAM>(a, dig, red, stat, flags, reinterpret_cast<v4i *>(smem + Lds::STASH_OFFSET));
+            helper_path<NB, FW, STREAM>(arguments_again(), dig, red, stat, flags, reinterpret_cast<v4i *>(smem + Lds::STASH_OFFSET));
+            return;
+        }
+    }
+    if constexpr (HeadShape<NB>::NH > 0) {
+        if ((int)blockIdx.x >= GroupShape<NB>::NWG) {          // (uniform for the workgroup)
+            head_path<NB, FW, STREAM>(arguments_again(), dig, stat, flags, reinterpret_cast<u64 *>(smem + Lds::OWN_OFFSET), reinterpret_cast<double *>(red));
             return;
         }
     }
@@ -1198,9 +1341,10 @@ __global__ void __launch_bounds__((FW + back_waves(NB)) * 64) decode_kernel(cons
                                   reinterpret_cast<long long *>(smem + Lds::total(a.m.L)));       // (total without the stamps = where they start)
     } else {
         constexpr int NWG = GroupShape<NB>::NWG;
-        const int v_tiles = (a.m.V + 15) / 16, head_rounds = (v_tiles + NWG - 1) / NWG;
+        const DArgs &ab = arguments_again();
+        const int v_tiles = (ab.m.V + 15) / 16, head_rounds = HeadShape<NB>::NH > 0 ? 0 : (v_tiles + NWG - 1) / NWG;
         const unsigned lds = (unsigned)(uintptr_t)(RWKV_LDS unsigned char *)smem;
-        BackOf<NB, FW, HELP, STREAM>::run(a.m.jt + (size_t)blockIdx.x * (a.m.L + 1) * 16, a.m.w_head, a.m.L, head_rounds, v_tiles,
+        BackOf<NB, FW, HELP, STREAM>::run(ab.m.jt + (size_t)blockIdx.x * (ab.m.L + 1) * 16, ab.m.w_head, ab.m.L, head_rounds, v_tiles,
                          (int)blockIdx.x, wave - FW, lds);
     }
 }
@@ -1347,7 +1491,7 @@ __global__ void __launch_bounds__(kPrepThreads) next_token_kernel(const DArgs a,
     auto better = [](double v, int i, double bv, int bi) { return v > bv || (v == bv && i < bi); };
     double best = -INFINITY;
     int bi = 0x7fffffff;
-    if ((int)threadIdx.x < a.m.NWG) { best = a.m.amax_val[threadIdx.x]; bi = a.m.amax_idx[threadIdx.x]; }   // NWG <= 256
+    if ((int)threadIdx.x < a.m.n_cand) { best = a.m.amax_val[threadIdx.x]; bi = a.m.amax_idx[threadIdx.x]; }   // at most 256
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         const double ob = __shfl_xor(best, off, 64);
@@ -1437,7 +1581,7 @@ __global__ void __launch_bounds__(kOrSlots) build_ownrec_kernel(const DPrep *__r
 // tiles of the workgroup (tiles past the end of the vocabulary point at tile 0, whose blocks stay
 // hot in L2 and whose products are never used).  grid (G), any block size.
 __global__ void build_jobtab_kernel(const DLayer *__restrict__ layers, const uint8_t *w_head, int L, int G, int NWG, int n_kb,
-                                    int v_tiles, u64 *__restrict__ jt) {
+                                    int v_tiles, bool head, u64 *__restrict__ jt) {
     const int wg = blockIdx.x, g = (G / NWG) * wg;     // the workgroup's first group; the tiles of its next group follow at fixed strides
     const size_t TB = (size_t)n_kb * 1024;
     for (int i = threadIdx.x; i < (L + 1) * 16; i += blockDim.x) {
@@ -1450,7 +1594,7 @@ __global__ void build_jobtab_kernel(const DLayer *__restrict__ layers, const uin
             else if (j == 4) p = Ly.w[MAT_FFN_R] + (size_t)g * TB;
             else if (j <= 8) p = Ly.w[MAT_FFN_K] + (size_t)(g + G * (j - 5)) * TB;
             else p = Ly.w[MAT_FFN_V] + ((size_t)g * 4 + (j - 9)) * TB;
-        } else if (l == L) {
+        } else if (l == L && head) {                  // (no head tiles: what the ring fetches at the end stays hot)
             const int tile = wg + NWG * j;
             p = w_head + (size_t)(tile < v_tiles ? tile : 0) * TB;
         }
@@ -1567,6 +1711,11 @@ unsigned decode_epochs_per_token(int64_t L) { return (unsigned)(4 * L + 1); }
 // 8-byte words of the exchange buffers (X, XR, A, AR, H, HR), one contiguous range starting at X
 static size_t exchange_words(int64_t C, int64_t F) { return (size_t)(2 * C + F + (kLnRows + 6) * (C / 16)); }
 
+// Workgroups that only have head tiles (launched last), and those that leave a candidate for the greedy token.
+static int64_t head_workgroups(int64_t C) { return C <= 1024 ? kHeadGrid - C / 16 : 0; }
+static int64_t candidates(int64_t C) { return head_workgroups(C) > 0 ? head_workgroups(C) : decode_workgroups(C); }
+static_assert(HeadShape<8>::NH == kHeadGrid - 512 / 16 && HeadShape<16>::NH == kHeadGrid - 1024 / 16 && HeadShape<24>::NH == 0, "head_workgroups");
+
 namespace {
 struct BlockPlan {
     size_t layers, prep, P32, Q32, PO, sc, X0, cs, ownrec, jt, scp, amax, abort, total;
@@ -1589,7 +1738,7 @@ BlockPlan plan_block(int64_t L, int64_t C, int64_t F, int64_t V) {
     p.ownrec = take((size_t)L * G * kOrSlots * sizeof(u64));
     p.jt = take(G * (size_t)(L + 1) * 16 * sizeof(u64));
     p.scp = take((size_t)L * prep_parts((int)C) * sizeof(DScal));
-    p.amax = take((size_t)G * (sizeof(double) + sizeof(int)));
+    p.amax = take((size_t)candidates(C) * (sizeof(double) + sizeof(int)));
     p.abort = take(256);
     p.total = off;
     return p;
@@ -1641,13 +1790,13 @@ int decode_setup(void *block, void *exchange, const DSetup &s, DModel *dm, Decod
     RWKV_CHECK_HIP(hipMemcpy(base + p.layers, tab.data(), (size_t)L * sizeof(DLayer), hipMemcpyHostToDevice));
     RWKV_CHECK_HIP(hipMemcpy(base + p.prep, prep.data(), (size_t)L * sizeof(DPrep), hipMemcpyHostToDevice));
 
-    dm->L = (int)L; dm->C = (int)C; dm->F = (int)F; dm->V = (int)V; dm->G = (int)G; dm->NWG = (int)decode_workgroups(C);
+    dm->L = (int)L; dm->C = (int)C; dm->F = (int)F; dm->V = (int)V; dm->G = (int)G; dm->NWG = (int)decode_workgroups(C); dm->n_cand = (int)candidates(C);
     dm->emb = s.emb; dm->ln0_w = s.ln0_w; dm->ln0_b = s.ln0_b;
     dm->w_head = s.head.w16; dm->cs = cs; dm->cs_head = cs_head;
     dm->ownrec = reinterpret_cast<const u64 *>(base + p.ownrec);
     dm->scp = reinterpret_cast<DScal *>(base + p.scp);
     dm->amax_val = reinterpret_cast<double *>(base + p.amax);
-    dm->amax_idx = reinterpret_cast<int *>(base + p.amax + (size_t)G * sizeof(double));
+    dm->amax_idx = reinterpret_cast<int *>(base + p.amax + (size_t)candidates(C) * sizeof(double));
     dm->layers = reinterpret_cast<const DLayer *>(base + p.layers);
     dm->prep = reinterpret_cast<const DPrep *>(base + p.prep);
     dm->P32 = reinterpret_cast<float *>(base + p.P32);
@@ -1659,7 +1808,7 @@ int decode_setup(void *block, void *exchange, const DSetup &s, DModel *dm, Decod
     ConstArgs ca;
     dm->jt = reinterpret_cast<const u64 *>(base + p.jt);
     hipLaunchKernelGGL(build_jobtab_kernel, dim3((unsigned)dm->NWG), dim3(256), 0, nullptr, dm->layers, s.head.w16, (int)L,
-                       (int)G, dm->NWG, c_kb, (int)ceil_div(V, 16), reinterpret_cast<u64 *>(base + p.jt));
+                       (int)G, dm->NWG, c_kb, (int)ceil_div(V, 16), head_workgroups(C) == 0, reinterpret_cast<u64 *>(base + p.jt));
     RWKV_CHECK_LAUNCH("build_jobtab_kernel");
     ca.L = (int)L; ca.C = (int)C; ca.prep = dm->prep;
     ca.lnout_w = s.lnout_w; ca.lnout_b = s.lnout_b; ca.range_h = s.head.range; ca.offset_h = s.head.offset;
@@ -1721,8 +1870,8 @@ static int launch_one(hipStream_t st, const DArgs &args, bool with_prep) {
         hipLaunchKernelGGL(prep_kernel, dim3((unsigned)(args.m.L * prep_parts(args.m.C) + 1)), dim3(kPrepThreads), 0, st, args);
         RWKV_CHECK_LAUNCH("prep_kernel");
     }
-    // owner workgroups first, then the helpers: every one of them is resident at once (one per compute unit)
-    const dim3 grid((unsigned)(args.m.NWG + HelperShape<NB>::NH));
+    // owner workgroups first, then those that help: every one of them is resident at once (one per compute unit)
+    const dim3 grid((unsigned)(args.m.NWG + HelperShape<NB>::NH + HeadShape<NB>::NH));
     if (trace)
         hipLaunchKernelGGL((decode_kernel<NB, FW, true, HELP, STREAM>), grid, dim3((FW + back_waves(NB)) * 64), lds, st, args);
     else

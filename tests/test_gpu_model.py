@@ -655,6 +655,31 @@ def test_host_resident_weights_give_identical_results():
     assert torch.equal(la, lb) and torch.equal(sa, sb)
 
 
+# up to 1024 channels the head belongs to workgroups of its own: fewer tiles than there are of them, one tile each exactly,
+# some with one and some with two, and more than the two a wavefront holds
+@pytest.mark.parametrize("C,V", [(512, 15), (512, 2561), (512, 61500), (768, 17), (768, 2304), (768, 27700), (768, 56000), (1024, 2049), (1024, 49153)])
+def test_token_steps_of_any_vocabulary_match_the_many_row_path(C, V):
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"token steps, C={C} V={V}")
+    m = HipRWKV(synth.iter_tensors(2, C, 4 * C, V, seed=C + V, device="cuda", ln="random"))
+    toks = synth.random_tokens(4, V=V, seed=V).tolist()
+    s, sb = m.emptyState.clone(), m.emptyState[None].clone()
+    for t in toks:
+        lg, s = m.forward([t], s)
+        lb, sb = m.forward_batch([t], sb)
+        # integer products on both sides; the rest differs by the float32 rounding of LayerNorm'd inputs
+        assert float((lg - lb[0]).norm() / lb[0].norm()) < 2e-6
+    first = cur = int(lg.argmax())
+    chain, st = [], s.clone()
+    for _ in range(3):
+        lg, st = m.forward([cur], st)
+        cur = int(lg.argmax())
+        chain.append(cur)
+    got, _, _ = m.decode_greedy(first, 3, s.clone())
+    assert got.tolist() == chain
+    m.check()
+
+
 @pytest.mark.parametrize("C,L", [(1024, 2), (2560, 1), (5120, 1)])
 def test_a_token_step_that_never_gets_its_input_drains_and_is_reported(C, L):
     """The failure path of the persistent kernel, forced from the host without anything that could hang: a token
