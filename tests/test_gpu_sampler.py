@@ -121,6 +121,52 @@ def test_typical_cut_in_every_range_of_the_first_round(V, top, spread, tau, lo, 
     assert abs(float(d[got].mean()) - mean) < 5 * sigma
 
 
+@pytest.mark.parametrize("V,shape,tau", [
+    (8192, "normal", 0.8), (8193, "normal", 0.8), (8194, "normal", 0.2), (50277, "normal", 0.999), (53248, "normal", 0.8), (53247, "zipf", 0.95),
+    (20001, "zipf", 0.2), (50277, "one", 0.5), (50277, "equal", 0.5), (9001, "peaked", 0.9), (50277, "peaked", 0.99999), (50277, "masked", 0.8),
+    (8191, "peaked", 1.0), (50277, "normal", 1.5)])
+def test_typical_keeps_the_tokens_of_a_float64_cut(V, shape, tau):
+    """Either way of loading the logits (two a load from 8193 tokens on), odd vocabularies, logits that are not 16-byte aligned,
+    and cuts the masses by bin find, miss (equal keys, one token with everything, tau of about one) or need not look for (tau
+    above one).  A token is inside or outside the cut by its distance from the entropy; the float32 sums around the cut move it
+    by no more than their rounding, V * 2^-24 of the mass at most, here twice that on either side."""
+    from rwkvstic_amd import ops
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(V, generator=g, dtype=torch.float64) * 1.5
+    if shape == "zipf":
+        x = -1.3 * torch.log(torch.arange(1, V + 1, dtype=torch.float64))
+    elif shape == "one":
+        x = x * 0 - 200.0
+        x[V - 2] = 30.0
+    elif shape == "equal":
+        x = x * 0 + 0.25
+    elif shape == "peaked":
+        x[V - 1] += 14.0
+        x[3] += 16.0
+    elif shape == "masked":
+        x[: V // 2] = -float("inf")
+    buf = torch.zeros(V + 1, dtype=torch.float64, device="cuda")
+    buf[1:] = x.cuda()
+    out = torch.empty(400, dtype=torch.int64, device="cuda")
+    for i in range(400):
+        ops.sample_token(buf[1:], temp=1.0, tau=tau, seed=3, counter=i, out=out[i:i + 1])
+    got = out.cpu()
+    assert torch.equal(buf[1:].cpu(), x)
+    p = torch.softmax(x, 0)
+    s = -torch.log(p)
+    d = torch.where(p > 0, (s - torch.nansum(s * p)).abs(), float("inf"))
+    order = torch.argsort(d)
+    mass = torch.empty(V, dtype=torch.float64)
+    mass[order] = torch.cumsum(p[order], 0) - p[order]              # what lies nearer than each token
+    slack = 2 * V * 2.0 ** -24
+    edge = d[order][min(int((torch.cumsum(p[order], 0) < tau + slack).sum()), V - 1)]
+    assert bool((d[got] <= edge * (1 + 1e-4) + 1e-5).all())         # (distances themselves: float32 logarithms of up to 2^4)
+    if shape in ("normal", "masked"):                               # and the kept tokens are all drawn from: half of them by mass lie beyond the median
+        far = mass[got] > 0.5 * min(tau, 1.0)
+        assert abs(float(far.double().mean()) - 0.5) < 5 * 0.5 / 400 ** 0.5 + 0.02
+    assert int(got.unique().numel()) == 1 if shape == "one" else int(got.unique().numel()) > 1
+
+
 def test_greedy_mode_end_adj_and_determinism():
     from rwkvstic_amd import ops
     g = torch.Generator().manual_seed(3)
