@@ -857,8 +857,13 @@ __device__ __forceinline__ void gemm8_body(const GemmArgs a) {
         bx = xcd + kXcds * cslot;
     }
     if (by >= a.gy || bx >= a.gx || bz >= a.gz) return;
-    const int mat = bz / a.split;                       // which product; then which part of its contraction
+    int mat = bz / a.split;                             // which product; then which part of its contraction
     bz -= mat * a.split;
+    GemmCols cols = {a.NT, a.N, a.tail, a.apart != 0};
+    if (a.NT2 > 0) {                                    // two products side by side: gx counts the column blocks of both
+        const int gx0 = (a.NT + kNT - 1) / kNT;
+        if (bx >= gx0) { bx -= gx0; mat = 1; cols = GemmCols{a.NT2, a.N2, a.tail2, a.apart2 != 0}; }
+    }
     const signed char *dig = mat == 0 ? a.dig[0] : mat == 1 ? a.dig[1] : a.dig[2];
     const uint8_t *w16 = mat == 0 ? a.w16[0] : mat == 1 ? a.w16[1] : a.w16[2];
     const int mt0 = by * 16 + wm * kGM, nt0 = bx * kNT + wn * kGN;
@@ -878,7 +883,7 @@ __device__ __forceinline__ void gemm8_body(const GemmArgs a) {
             src[i] = reinterpret_cast<const v4i *>(dig + ((size_t)mt * a.KB + kb0) * 1024) + lane;
         } else {
             int nt = bx * kNT + (f - 16 < kNT ? f - 16 : 0);   // (slots past the last fragment: a copy nobody reads)
-            if (nt >= a.NT) nt = a.NT - 1;
+            if (nt >= cols.NT) nt = cols.NT - 1;
             src[i] = reinterpret_cast<const v4i *>(w16 + ((size_t)nt * a.KB + kb0) * 1024) + lane;
         }
     }
@@ -939,7 +944,7 @@ __device__ __forceinline__ void gemm8_body(const GemmArgs a) {
 #undef RWKV_GEMM_STEP
 #undef RWKV_GEMM_DMA
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // nothing of this wavefront may still be writing LDS when it leaves
-    gemm_epilogue<kGM, kGN>(a, GemmCols{a.NT, a.N, a.tail}, acc, mt0, nt0, mat, bz, lane);
+    gemm_epilogue<kGM, kGN>(a, cols, acc, mt0, nt0, mat, bz, lane);
 }
 
 template <bool STREAM>
@@ -1680,6 +1685,13 @@ static int skinny_split(int64_t NT, int64_t KB, int n) {
     while (ceil_div(NT, kSkinnyNT) * n * split < kSkinnyFillWgs && KB / (split * 2) >= 8 && split < kMaxSplit) split *= 2;
     return split;
 }
+// Rounds of workgroups on 256 compute units, in matrix instructions per step: two general workgroups (w4 in all) share a
+// compute unit (2 x 32), a wide one (w5) has it alone (40).
+static int64_t general_cost(int64_t w4) {
+    const int64_t rem = w4 % 512;
+    return (w4 / 512) * 64 + (rem == 0 ? 0 : rem <= 256 ? 32 : 64);
+}
+static bool general_wide(int64_t w4, int64_t w5) { return w4 >= 256 && kGemmWideNum * ceil_div(w5, 256) * 40 < kGemmWideDen * general_cost(w4); }
 static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n) {
     ProductPlan p;
     p.split = 1;
@@ -1691,14 +1703,7 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n) {
     }
     p.gy = (int)ceil_div(MT, 16);
     p.kind = MT <= kSkinnyMT ? PLAN_SKINNY : PLAN_GENERAL;      // few rows: the weight-streaming variant
-    if (p.kind == PLAN_GENERAL) {
-        // Rounds of workgroups on 256 compute units, in matrix instructions per step: two general workgroups
-        // share a compute unit (2 x 32), a wide one has it alone (40).
-        const int64_t w4 = ceil_div(NT, kGemmNT) * p.gy * n, w5 = ceil_div(NT, kGemmWideNT) * p.gy * n;
-        const int64_t rem = w4 % 512;
-        const int64_t cost4 = (w4 / 512) * 64 + (rem == 0 ? 0 : rem <= 256 ? 32 : 64), cost5 = ceil_div(w5, 256) * 40;
-        if (w4 >= 256 && kGemmWideNum * cost5 < kGemmWideDen * cost4) p.kind = PLAN_WIDE;
-    }
+    if (p.kind == PLAN_GENERAL && general_wide(ceil_div(NT, kGemmNT) * p.gy * n, ceil_div(NT, kGemmWideNT) * p.gy * n)) p.kind = PLAN_WIDE;
     p.gx = (int)ceil_div(NT, p.kind == PLAN_SKINNY ? kSkinnyNT : p.kind == PLAN_WIDE ? kGemmWideNT : kGemmNT);
     // Split the contraction until the grid has a few workgroups per compute unit.
     if (p.kind == PLAN_SKINNY) p.split = skinny_split(NT, KB, n);
@@ -1936,6 +1941,15 @@ int rows_quant(hipStream_t st, int64_t R, int64_t K, const void *in, bool in_f32
     return RWKV_OK;
 }
 
+static void launch_general(hipStream_t st, GemmArgs &g, bool wide, int gx, bool stream) {
+    g.gx = gx; g.gy = (int)ceil_div(g.MT, 16); g.by_rows = g.gy >= kXcds;
+    g.per_xcd = ((g.by_rows ? g.gy : gx) + kXcds - 1) / kXcds;
+    const dim3 grid((unsigned)(kXcds * g.per_xcd * (g.by_rows ? gx : g.gy) * g.gz));
+    if (wide) hipLaunchKernelGGL(gemm8_wide_kernel, grid, dim3(512), 0, st, g);
+    else if (stream && g.gy <= kStreamRowBlocks) hipLaunchKernelGGL(gemm8_kernel<true>, grid, dim3(512), 0, st, g);
+    else hipLaunchKernelGGL(gemm8_kernel<false>, grid, dim3(512), 0, st, g);
+}
+
 int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, int64_t R, int64_t K, int64_t N, int op,
                   const float *gate, RowsDeferred *defer) {
     if (K % 64 != 0) return set_error(RWKV_ERR_SIZE, "rows_products: contraction length %lld is not a multiple of 64",
@@ -1951,7 +1965,6 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     }
     g.tot = tot;
     g.MT = (int)ceil_div(R, 4); g.NT = (int)ceil_div(N, 16); g.KB = (int)(K / 64); g.ldd = g.NT * 16;
-    const int gy = (int)ceil_div(g.MT, 16);
     g.R = (int)R; g.N = (int)N; g.gate = gate;
     const ProductPlan pl = plan_products(g.MT, g.NT, g.KB, n);
     const int split = pl.split;
@@ -1967,15 +1980,14 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
         g.gx = g.NT; g.gy = 1; g.by_rows = 0; g.per_xcd = 0;
         launch_vec(st, g, p[0].stream);
         RWKV_CHECK_LAUNCH("gemv16_kernel");
+    } else if (pl.kind == PLAN_SKINNY) {
+        g.gx = pl.gx; g.gy = 1; g.by_rows = 0; g.per_xcd = (pl.gx + kXcds - 1) / kXcds;
+        const dim3 grid((unsigned)(kXcds * g.per_xcd * g.gz));
+        if (p[0].stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
+        else hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
+        RWKV_CHECK_LAUNCH("gemm8_skinny_kernel");
     } else {
-        g.gx = pl.gx; g.gy = gy; g.by_rows = gy >= kXcds;
-        g.per_xcd = ((g.by_rows ? gy : pl.gx) + kXcds - 1) / kXcds;
-        const dim3 grid((unsigned)(kXcds * g.per_xcd * (g.by_rows ? pl.gx : gy) * g.gz));
-        if (pl.kind == PLAN_SKINNY && p[0].stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
-        else if (pl.kind == PLAN_SKINNY) hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
-        else if (pl.kind == PLAN_WIDE) hipLaunchKernelGGL(gemm8_wide_kernel, grid, dim3(512), 0, st, g);
-        else if (p[0].stream && gy <= kStreamRowBlocks) hipLaunchKernelGGL(gemm8_kernel<true>, grid, dim3(512), 0, st, g);
-        else hipLaunchKernelGGL(gemm8_kernel<false>, grid, dim3(512), 0, st, g);
+        launch_general(st, g, pl.kind == PLAN_WIDE, pl.gx, p[0].stream);
         RWKV_CHECK_LAUNCH("gemm8_kernel");
     }
     for (int m = 0; defer && m < n; ++m) defer[m].tot = nullptr;
@@ -1997,6 +2009,25 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     }
     RWKV_CHECK_LAUNCH("rows_finish_kernel");
     return RWKV_OK;
+}
+
+// Whether ffn key (NT tiles) and receptance (NT2) of more than 32 rows share a launch of the general kernel, whole contractions:
+// what it saves is a launch, about 3 us at a third of a microsecond a contraction block, and part of another where slices had to
+// be added up; what it may cost is a round of workgroups more.  Us a prompt apart / together: 24 layers of
+// 1024, 33 / 77 / 127 / 500 tokens 2055 / 2143 / 2368 / 2912 against 1792 / 1890 / 2019 / 2763; 12 of 2560, 64 / 77 / 200 / 500 1525 / 1572 / 2198 / 3327
+// against 1383 / 1416 / 2097 / 3279; 6 of 5120, 33 / 300 1244 / 3032 against 1155 / 2921.  Together all the same where the rule says apart: 6
+// of 4096, 77 1255 / 1268; 12 of 1536, 300 1671 / 1702; 12 of 2560, 1000 (the receptance alone: one round of the wide kernel) 4846 / 4971.
+static bool pair_general(int64_t MT, int64_t NT, int64_t NT2, int64_t KB) {
+    if (MT <= kSkinnyMT || KB > 1024) return false;
+    const int64_t gy = ceil_div(MT, 16);
+    int64_t saved = 290;
+    auto alone = [&](int64_t nt) {                          // in ninths, as kGemmWideDen weighs the wide kernel
+        const ProductPlan p = plan_products(MT, nt, KB, 1);
+        if (p.split > 1) saved += 60;
+        return p.kind == PLAN_WIDE ? kGemmWideNum * 40 * ceil_div((int64_t)p.gx * p.gy, 256) : kGemmWideDen * general_cost((int64_t)p.gx * p.gy * p.split) / p.split;
+    };
+    const int64_t more = kGemmWideDen * general_cost((ceil_div(NT, kGemmNT) + ceil_div(NT2, kGemmNT)) * gy) - alone(NT) - alone(NT2);
+    return more * KB <= kGemmWideDen * saved;
 }
 
 // Few rows: both in one launch, whole contractions (the receptance's column blocks find room beside the key's; apart they
@@ -2037,6 +2068,8 @@ int rows_ffn_key_receptance(hipStream_t st, bool sequence, const RowsProduct &k,
         const dim3 grid((unsigned)(kXcds * g.per_xcd));
         if (k.stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
         else hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
+    } else if (pair_general(g.MT, g.NT, g.NT2, g.KB)) {
+        launch_general(st, g, false, (int)(ceil_div(g.NT, kGemmNT) + ceil_div(g.NT2, kGemmNT)), k.stream);
     } else {
         int rc = rows_products(st, 1, &k, tot, R, C, F, ROW_RELU2, nullptr);
         if (!rc) rc = rows_products(st, 1, &r, tot, R, C, C, ROW_STORE_F32, nullptr);

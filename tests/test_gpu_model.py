@@ -503,7 +503,8 @@ def test_shapes_chunkings_and_batches_against_the_exact_oracle(L, C, F, V, T, cu
 # the narrowest with two (4160), and on both sides of the rows (8, 32) and launch sizes at which the products around them change
 @pytest.mark.parametrize("C,F,B", [(64, 64, 2), (1088, 4352, 8), (1088, 4352, 9), (1984, 8192, 12), (4096, 8192, 3), (4096, 8192, 32),
                                    (4160, 4160, 1), (4160, 4160, 33), (576, 2304, 13), (1024, 4096, 16), (1024, 4096, 17), (1536, 6144, 25),
-                                   (1024, 4096, 32), (2048, 8192, 31)])
+                                   (1024, 4096, 32), (2048, 8192, 31),
+                                   (576, 2304, 33), (1088, 4352, 65), (1984, 8192, 64)])     # ffn key and receptance side by side
 def test_batch_steps_of_ragged_and_wide_rows_match_single_steps(C, F, B):
     from rwkvstic_amd.model import HipRWKV
     _say(f"batch of {B} at C={C} F={F}")
