@@ -523,8 +523,8 @@ constexpr int64_t kRowsChunk = 1024;   // rows per pass: bounds the workspace of
 constexpr int64_t kRowsMin = 4;        // shorter prompts go token by token
 
 struct RowsWs {
-    double *x, *kvr, *att, *h, *prev0;
-    double *x2, *sh1, *sh2; // fewer than kRowsDeferMax rows: x after a pending update, the two newest shift rows (see RowsFew)
+    double *x, *kvr, *att, *h;
+    double *x2, *sh1, *sh2; // fewer than kRowsDeferMax rows: x after a pending update, the two newest shift rows (of any sequence; see RowsFew)
     RowsOperand q[3];       // quantised left operands: q[0] up to n_ffn wide, q[1], q[2] n_embd wide
     RowsOperand qv;         // ffn value's: the digits of q[0], row constants of its own (see rows_layers)
     long long *tot;
@@ -545,7 +545,6 @@ size_t rows_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_
     size_t n = 0;
     n += round_up((size_t)R * C * 8, 256) * 5;          // x, kvr[3], att
     n += round_up((size_t)R * F * 8, 256);              // h
-    n += round_up((size_t)C * 8, 256);                  // prev0
     n += round_up((size_t)(R < kRowsDeferMax ? R : kRowsDeferMax - 1) * C * 8, 256) * 3;    // x2, sh1, sh2
     n += round_up((size_t)R * 8, 256) * 12;             // S, qs, zp of four operands
     n += round_up(rows_dig_bytes(R, F), 256) + 2 * round_up(rows_dig_bytes(R, C), 256);
@@ -561,7 +560,6 @@ RowsWs rows_carve(void *ws, int64_t R, int64_t C, int64_t F, int64_t n_wide, int
     w.kvr = (double *)take((size_t)R * C * 8 * 3);
     w.att = (double *)take((size_t)R * C * 8);
     w.h = (double *)take((size_t)R * F * 8);
-    w.prev0 = (double *)take((size_t)C * 8);
     for (double **b : {&w.x2, &w.sh1, &w.sh2}) *b = (double *)take((size_t)(R < kRowsDeferMax ? R : kRowsDeferMax - 1) * C * 8);
     for (int i = 0; i < 3; ++i) {
         w.q[i].S = (double *)take((size_t)R * 8);
@@ -588,8 +586,8 @@ bool rows_supported(const rwkv_model *m) {
 // R rows through every layer.  sequence: rows are consecutive tokens of one sequence whose state is
 // `state` [L,5,C]; otherwise row b is one token of sequence b with state at state + b * state_stride.
 // tail: what is left to the LayerNorm kernel in front of the head: its input x, the last layer's ffn value product where it
-// is still pending (batch rows), and the last shift rows to be committed.
-struct RowsTailWork { const double *x; RowsFew few; };
+// is still pending (batch rows), and the last shift rows to be committed; or to the sequence's next pass.
+struct RowsTailWork { const double *x = nullptr; RowsFew few{}; };
 int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R, bool sequence, double *state,
                 int64_t state_stride, const RowsWs &w, RowsTailWork &tail) {
     const rwkv_model_desc &d = m->d;
@@ -603,8 +601,9 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     // Several workgroups share a row in the LayerNorm kernel of few rows, one for each mix, and no order holds between them.
     // What one of them reads another may not write in the same launch:
     //   x                        the updated x goes to the other of two buffers (few.x_out)
-    //   the shift rows           the newest go aside (few.shift_out); the next launch commits them, for batch rows and a single
-    //                            row; longer sequences read a copy (prev0)
+    //   the shift rows           the newest go aside (few.shift_out); the next launch commits them.  So for sequences of any length,
+    //                            whose row 0 reads what their last row replaces (copied before each launch they cost 12 layers
+    //                            of 2560 3.5 us a time)
     //   S, qs, zp of a pending product    ffn value's, which the next layer's first LayerNorm reads while it writes those of k, v
     //                            and r, are a set of their own (w.qv); att output's are q[0]'s, while ffn key and receptance have
     //                            q[1] and q[2].  In front of the head one workgroup has the row.
@@ -612,10 +611,9 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     const bool stream = weights_streamed(d.n_layer, d.n_embd, d.n_ffn, d.n_vocab);
     const bool defer = !sequence && R < kRowsDeferMax;
     RowsDeferred dk[3];
-    // Few rows whose shift rows are read straight from the state: the LayerNorm kernels leave the new ones aside, and each
-    // commits what the one before it left.
-    const bool aside = R < kRowsDeferMax && (!sequence || R == 1);
-    RowsFew few{};
+    // The LayerNorm kernels leave the new shift rows aside, and each commits what the one before it left.
+    const bool aside = R < kRowsDeferMax || sequence;
+    RowsFew few = tail.few;                             // (a sequence's next pass: the last shift row of the one before)
     double *x = w.x;
     // (after a launch of the LayerNorm kernel: x is where a pending update went, its shift rows wait in `left` for `home`)
     auto advance = [&](const double *left, double *home) {
@@ -626,15 +624,12 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     for (int64_t l = 0; l < d.n_layer; ++l) {
         const rwkv_layer_desc &L = m->layers[l];
         double *sl = state + (size_t)l * 5 * C;
-        // TimeMix (block.py:58-80).  Row 0 of a sequence reads the shift state while the last row replaces it, hence the copy;
-        // a single row's workgroups all read it, and its newest goes aside instead.
-        const bool copy_prev = sequence && R > 1;
-        if (copy_prev) RWKV_CHECK_HIP(hipMemcpyAsync(w.prev0, sl, (size_t)C * 8, hipMemcpyDeviceToDevice, st));
+        // TimeMix (block.py:58-80)
         const rwkv_qmat *kvr[3] = {&L.att_k, &L.att_v, &L.att_r};
         const float *rg[3] = {kvr[0]->range, kvr[1]->range, kvr[2]->range};
         const double *of[3] = {kvr[0]->offset, kvr[1]->offset, kvr[2]->offset};
         prepare(w.sh1);
-        RWKV_TRY(rows_ln_mix_quant(st, 3, R, C, sequence, x, L.ln1_w, L.ln1_b, L.att_mix, copy_prev ? w.prev0 : sl, sl,
+        RWKV_TRY(rows_ln_mix_quant(st, 3, R, C, sequence, x, L.ln1_w, L.ln1_b, L.att_mix, sl, sl,
                                    state_stride, rg, of, w.q, &few));
         advance(w.sh1, sl);
         // k, v, r (and the ffn receptance below) are kept as float32 arrays in the kvr slab
@@ -648,12 +643,11 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
         const RowsProduct po = {w.q[0], L.att_o.packed16, x, stream};
         RWKV_TRY(rows_products(st, 1, &po, w.tot, R, C, C, ROW_ADD, nullptr, defer ? &few.add : nullptr));
         // ChannelMix (block.py:82-100)
-        if (copy_prev) RWKV_CHECK_HIP(hipMemcpyAsync(w.prev0, sl + C, (size_t)C * 8, hipMemcpyDeviceToDevice, st));
         const float *rg2[2] = {L.ffn_k.range, L.ffn_r.range};
         const double *of2[2] = {L.ffn_k.offset, L.ffn_r.offset};
         prepare(w.sh2);
-        RWKV_TRY(rows_ln_mix_quant(st, 2, R, C, sequence, x, L.ln2_w, L.ln2_b, L.ffn_mix, copy_prev ? w.prev0 : sl + C,
-                                   sl + C, state_stride, rg2, of2, w.q + 1, &few));
+        RWKV_TRY(rows_ln_mix_quant(st, 2, R, C, sequence, x, L.ln2_w, L.ln2_b, L.ffn_mix, sl + C, sl + C,
+                                   state_stride, rg2, of2, w.q + 1, &few));
         advance(w.sh2, sl + C);
         const RowsProduct pfk = {w.q[1], L.ffn_k.packed16, w.h, stream}, pfr = {w.q[2], L.ffn_r.packed16, w.kvr, stream};
         RWKV_TRY(rows_ffn_key_receptance(st, sequence, pfk, pfr, w.tot, R, C, F, L.ffn_v.range, L.ffn_v.offset, w.qv));
@@ -688,9 +682,9 @@ int rows_sequence(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t 
     unsigned char *rows_base = static_cast<unsigned char *>(workspace) + round_up(ws_doubles(C, F) * sizeof(double), 256);
     const int64_t Rmax = T < kRowsChunk ? T : kRowsChunk;
     const RowsWs rw = rows_carve(rows_base, Rmax, C, F, F, m->d.n_vocab);
+    RowsTailWork tail;
     for (int64_t t0 = 0; t0 < T; t0 += kRowsChunk) {
         const int64_t R = T - t0 < kRowsChunk ? T - t0 : kRowsChunk;
-        RowsTailWork tail;
         int rc = rows_layers(m, st, tokens + t0, R, true, state, 0, rw, tail);
         if (rc) return rc;
         if (t0 + R == T) {

@@ -37,12 +37,12 @@ struct RowsDeferred {
 constexpr int64_t kRowsDeferMax = 128;
 constexpr int kRowsDeferSlices = 4;     // a contraction split further than this is finished by a launch of its own
 // What the LayerNorm kernel of fewer than kRowsDeferMax rows does besides (several workgroups share a row there, and none
-// may overwrite what another reads).
+// may overwrite what another reads); of a sequence of any length, the shift rows (row 0 reads what the last row replaces).
 struct RowsFew {
     RowsDeferred add;           // a residual update of x still pending (tot null: none); batch rows only; with mixes, its S, qs and zp are no output's
     double *x_out;              // where the updated x goes: another buffer than x (null: it is not needed)
-    double *shift_out;          // [R, C]: the newest shift rows, instead of the state; needed wherever prev0 is the state itself
-    const double *commit_src;   // [R, C]: shift rows left by the launch before (null: none) ...
+    double *shift_out;          // [R, C], of a sequence [C]: the newest shift rows, instead of the state
+    const double *commit_src;   // shift rows left by the launch before (null: none) ...
     double *commit_dst;         // ... and their place in the state, row stride prev_stride
 };
 size_t rows_dig_bytes(int64_t R, int64_t K);

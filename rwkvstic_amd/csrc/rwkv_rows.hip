@@ -218,13 +218,13 @@ struct LnQuantArgs {
     const double *x;            // [R, C]
     RowsDeferred add;           // batch rows, few-row form: x += this product first, stored to x_out (tot null: none)
     double *x_out;              // null: nobody reads x again
-    double *shift_out;          // few-row form, [R, C]: the newest xy rows go here instead of to shift_dst (null: sequences, to shift_dst)
-    const double *commit_src;   // few-row form: [R, C] rows an earlier launch left in its shift_out (null: none) ...
+    double *shift_out;          // few-row form of batch rows, [R, C]: the newest xy rows go here instead of to shift_dst (null: to shift_dst)
+    const double *commit_src;   // few-row form or sequence: [R, C] rows (sequence: one) an earlier launch left aside (null: none) ...
     double *commit_dst;         // ... copied to commit_dst + row * prev_stride
     const double *ln_w, *ln_b;  // [C]
     const double *mu;           // [NM, C]
     const double *prev0;        // sequence: [C]; batch: row t at prev0 + t * prev_stride
-    double *shift_dst;          // sequence: [C] (written by row R-1); batch: row t at shift_dst + t * prev_stride
+    double *shift_dst;          // sequence: [C] aside (written by row R-1, while row 0 reads the state); batch: row t at shift_dst + t * prev_stride
     int64_t prev_stride;
     const float *range[3];      // per output: the matrix's per-input-channel range / offset
     const double *offset[3];
@@ -336,7 +336,7 @@ __global__ void __launch_bounds__(kLnRowThreads) rows_ln_mix_quant_row_kernel(co
             if (MIX) ld4(mu[g], mur + c0);
             ld4(rg[g], range + c0);
             ld4(of[g], offset + c0);
-            if (a.commit_src && m == 0) {
+            if (a.commit_src && m == 0 && (!a.sequence || t == 0)) {
                 double v[4];
                 ld4(v, a.commit_src + (size_t)t * C + c0);
                 st4(a.commit_dst + (size_t)t * a.prev_stride + c0, v);
@@ -1849,16 +1849,18 @@ int rows_ln_mix_quant(hipStream_t st, int n_mix, int64_t R, int C, bool sequence
     if (few) {
         if (few->add.tot && (sequence || (few->add.op != ROW_ADD && few->add.op != ROW_GATE_ADD) || few->x_out == x))
             return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: a pending product needs batch rows, a residual tail and another buffer for the new x");
-        if (R >= kRowsDeferMax && (few->add.tot || few->shift_out || few->commit_src))
+        if (R >= kRowsDeferMax && (few->add.tot || (!sequence && (few->shift_out || few->commit_src))))
             return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: pending work needs fewer than %d rows", (int)kRowsDeferMax);
-        a.add = few->add; a.x_out = few->x_out; a.shift_out = few->shift_out; a.commit_src = few->commit_src; a.commit_dst = few->commit_dst;
+        a.add = few->add; a.x_out = few->x_out; a.commit_src = few->commit_src; a.commit_dst = few->commit_dst;
+        if (sequence && few->shift_out) shift_dst = few->shift_out;      // (its last row alone)
+        else a.shift_out = few->shift_out;
     }
     // (a row has a workgroup for each mix: none may write what another still reads)
     for (int k = 0; n_mix > 1 && a.add.tot && k < n_mix; ++k)
         if (out[k].S == a.add.S || out[k].qs == a.add.qs || out[k].zp == a.add.zp)
             return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: the row constants of a pending product may not be those of an output");
-    if (n_mix > 0 && R < kRowsDeferMax && !a.shift_out && !(sequence && R > 1 && prev0 != shift_dst))
-        return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: few rows need their shift rows kept apart");
+    if (n_mix > 0 && (sequence ? prev0 == shift_dst : R < kRowsDeferMax && !a.shift_out))
+        return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: few rows and sequences need their shift rows kept apart");
     a.prev0 = prev0; a.shift_dst = shift_dst; a.prev_stride = prev_stride;
     const int n_out = n_mix > 0 ? n_mix : 1;
     for (int m = 0; m < 3; ++m) {
