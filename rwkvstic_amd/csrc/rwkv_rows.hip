@@ -433,12 +433,26 @@ __global__ void __launch_bounds__(kLnRowThreads) rows_ln_mix_quant_row_kernel(co
 
 template <int NM, int NSEG, int kLT>
 __global__ void __launch_bounds__(kLT) rows_ln_mix_quant_kernel(const LnQuantArgs a) {
+    constexpr int m0 = 0;
 #include "rwkv_rows_ln_body.inc"
 }
 // The same for so few rows that at most two workgroups share a compute unit: twice the registers, so that the
 // parameter vectors of all of a thread's channels can be on their way at once instead of one group after the other.
 template <int NM, int NSEG, int kLT>
 __global__ void __launch_bounds__(kLT) __attribute__((amdgpu_waves_per_eu(1, 2))) rows_ln_mix_quant_few_kernel(const LnQuantArgs a) {
+    constexpr int m0 = 0;
+#include "rwkv_rows_ln_body.inc"
+}
+// The same with a workgroup to each mix of a row (blockIdx.y): up to 256 rows of a sequence leave a compute unit one row, four
+// wavefronts that wait for its parameter vectors one group of channels after the other, of all mixes in turn.  Two or three times
+// the wavefronts for the same waits, and the statistics, a few additions, done again.  Bound: those dependent loads.  Not for
+// batches, whose shift rows are replaced in place: a workgroup may not write what the others of its row still read.  With the
+// quantiser below, prompts of 256 tokens, before / now: 10 layers of 5120 4321 / 4049 us, 16 of 4096 4813 / 4474, 24 of 2560
+// 4215 / 4057, 24 of 1024 2037 / 1998; of 150 tokens 24 of 2560 3879 / 3741.
+template <int NSEG, int kLT>
+__global__ void __launch_bounds__(kLT) __attribute__((amdgpu_waves_per_eu(1, 3))) rows_ln_mix_quant_split_kernel(const LnQuantArgs a) {
+    constexpr int NM = 1;
+    const int m0 = blockIdx.y;
 #include "rwkv_rows_ln_body.inc"
 }
 
@@ -600,6 +614,86 @@ __global__ void __launch_bounds__(kRT) rows_quant4_kernel(const QuantArgs a) {
     }
     rsum<1>(qsum, red);
     if (tid == 0) { a.S[t] = S; a.qs[t] = qsum[0]; a.zp[t] = z[0]; }
+}
+
+// Long rows, too few of them to fill the device with workgroups of 256 threads: four threads for each one of the kernel above, with
+// a quarter of its groups each (NP consecutive ones), so that four times the loads are on their way from a compute unit that has
+// a row or two.  Bound: those loads.  The sums are in that kernel's order, the bits its own.  256 rows of 20480 / 16384 values, caches warm:
+// 13.8 / 11.4 us by the kernel above, 10.7 / 8.5 by this.
+template <int NP, typename TIn>
+__global__ void __launch_bounds__(4 * kRT) rows_quant_long_kernel(const QuantArgs a) {
+    __shared__ double zs[kRT], red0[8], red1[4 * kRW];
+    __shared__ float redf[4 * kRW];
+    const int t = blockIdx.x, K = a.K, tid = threadIdx.x, part = tid / kRT, col = tid % kRT, wave = tid >> 6, lane = tid & 63;
+    const TIn *row = static_cast<const TIn *>(a.in) + (size_t)t * K;
+    TIn v[NP][4];
+    float r[NP][4];
+    double o[NP][4];
+#pragma unroll
+    for (int g = 0; g < NP; ++g) {
+        const int c0 = 4 * (col + (part * NP + g) * kRT);
+        if (c0 < K) {
+            ld4(v[g], row + c0);
+            ld4(r[g], a.range + c0);
+            ld4(o[g], a.offset + c0);
+        }
+    }
+    float xs[NP][4];
+    float amax = 0.f;
+#pragma unroll
+    for (int g = 0; g < NP; ++g) {
+        if (4 * (col + (part * NP + g) * kRT) < K) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                xs[g][i] = (float)((double)v[g][i] * (double)r[g][i]);
+                amax = fmaxf(amax, fabsf(xs[g][i]));
+            }
+        }
+    }
+    amax = wmaxf(amax);
+    if (lane == 0) redf[wave] = amax;
+    // the zero-point sum in that kernel's order: a quarter goes on from where the one before it ended
+    double z = 0.0;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        if (part == p) {
+            if (p > 0) z = zs[col];
+#pragma unroll
+            for (int g = 0; g < NP; ++g) {
+                if (4 * (col + (part * NP + g) * kRT) < K) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) z += (double)v[g][i] * o[g][i];
+                }
+            }
+            if (p < 3) zs[col] = z;
+            else {
+                z = wsum(z);
+                if (lane == 0) red0[wave - 3 * kRW] = z;
+            }
+        }
+        __syncthreads();
+    }
+    double zp = 0.0;
+    amax = redf[0];
+#pragma unroll
+    for (int w = 0; w < kRW; ++w) zp += red0[w];
+#pragma unroll
+    for (int w = 1; w < 4 * kRW; ++w) amax = fmaxf(amax, redf[w]);
+    double S, invS;
+    row_scale(amax, S, invS);
+    double qsum = 0.0;
+#pragma unroll
+    for (int g = 0; g < NP; ++g) {
+        const int c0 = 4 * (col + (part * NP + g) * kRT);
+        if (c0 < K) qsum += emit_quad(xs[g], invS, c0, t, K >> 6, a.dig);
+    }
+    qsum = wsum(qsum);
+    if (lane == 0) red1[wave] = qsum;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < 4 * kRW; ++w) qsum += red1[w];
+        a.S[t] = S; a.qs[t] = qsum; a.zp[t] = zp;
+    }
 }
 
 // A handful of long rows (one token of a wide ffn): one workgroup per row would pull the whole row and its
@@ -1819,6 +1913,11 @@ size_t rows_tot_bytes(int64_t R, int64_t N, int64_t K) {
 // (a few long rows are quantised by several workgroups each, in two launches: one workgroup per row leaves most of the
 // device idle - 14B shape, batch step of 32 sequences: 7.78 against 8.10 ms)
 static bool quant_uses_parts(int64_t R, int64_t K) { return R <= 64 && K >= 8192; }
+// Rows that have four times the threads: up to 384 of them (300 tokens, 10 layers of 5120 4883 / 4849 us a prompt, 16 of 4096 5760 / 5701; from
+// 500 on, and at 2560 channels from 300 on, it makes no difference, and alone with warm caches 400 rows are 10 % slower), and of so many
+// values that a wavefront of the narrower form has more than two groups a lane (from 6144 values on: 256 tokens of 5120 channels
+// 4067 us, this 4049).
+constexpr int kLongQuantRows = 384, kLongQuantFrom = 2048;
 size_t rows_quant_scratch_bytes(int64_t R, int64_t K) {
     if (!quant_uses_parts(R, K)) return 0;
     return (size_t)(R * ceil_div(K, 4 * kRT * kQuantPartSeg) * 2 * 8);
@@ -1889,6 +1988,15 @@ int rows_ln_mix_quant(hipStream_t st, int n_mix, int64_t R, int C, bool sequence
     }
     const bool small = C <= 3 * 4 * 256;
     const dim3 grid((unsigned)R), block(256);
+    // A workgroup to each mix where the rows alone are too few (us a prompt of 300, 400, 500 tokens, a workgroup to each row / mix:
+    // 10 layers of 5120 4884, 6350 / 4813, 6307; 16 of 4096, 300 and 500 5760, 7572 / 5666, 7708; 24 of 2560 5339, 5765, 6308 / 5344, 5845, 6517).
+    if (sequence && n_mix > 1 && R <= (small ? 256 : 384)) {
+        const dim3 apart((unsigned)R, (unsigned)n_mix);
+        if (small) hipLaunchKernelGGL((rows_ln_mix_quant_split_kernel<3, 256>), apart, block, 0, st, a);
+        else hipLaunchKernelGGL((rows_ln_mix_quant_split_kernel<6, 256>), apart, block, 0, st, a);
+        RWKV_CHECK_LAUNCH("rows_ln_mix_quant_split_kernel");
+        return RWKV_OK;
+    }
 #define RWKV_LNQ(NM)                                                                                  \
     do {                                                                                              \
         if (small && R <= 512) hipLaunchKernelGGL((rows_ln_mix_quant_few_kernel<NM, 3, 256>), grid, block, 0, st, a);   \
@@ -1926,6 +2034,14 @@ int rows_quant(hipStream_t st, int64_t R, int64_t K, const void *in, bool in_f32
             hipLaunchKernelGGL((rows_quant_part_kernel<true, double>), pg, block, 0, st, pa);
         }
         RWKV_CHECK_LAUNCH("rows_quant_part_kernel");
+        return RWKV_OK;
+    }
+    if (R <= kLongQuantRows && K > kLongQuantFrom && K <= 20 * 4 * kRT && in_f32) {
+        if (K <= 4 * 4 * kRT) hipLaunchKernelGGL((rows_quant_long_kernel<1, float>), grid, dim3(4 * kRT), 0, st, q);
+        else if (K <= 8 * 4 * kRT) hipLaunchKernelGGL((rows_quant_long_kernel<2, float>), grid, dim3(4 * kRT), 0, st, q);
+        else if (K <= 12 * 4 * kRT) hipLaunchKernelGGL((rows_quant_long_kernel<3, float>), grid, dim3(4 * kRT), 0, st, q);
+        else hipLaunchKernelGGL((rows_quant_long_kernel<5, float>), grid, dim3(4 * kRT), 0, st, q);
+        RWKV_CHECK_LAUNCH("rows_quant_long_kernel");
         return RWKV_OK;
     }
 #define RWKV_QUANT_LAUNCH(T)                                                                          \

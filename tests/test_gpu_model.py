@@ -746,6 +746,25 @@ def test_a_prompt_equals_its_tokens_one_by_one(T):
         assert float((sp[:, row] - st[:, row]).norm() / st[:, row].norm()) < 5e-6, row
 
 
+# rows of a prompt that share a launch of the row kernels: on both sides of the rows (256 for up to 3072 channels, 384 for more) up to
+# which each mix, and of the row lengths (2048, 4096, 8192, 12288, 20480) from which each quarter of a row, has threads of its own
+@pytest.mark.parametrize("C,F,T", [(64, 2048, 128), (64, 2112, 256), (64, 4096, 257), (128, 4160, 384), (128, 8256, 385), (192, 12352, 300),
+                                   (2112, 20480, 130), (64, 20544, 200), (3072, 3072, 256), (3136, 3136, 257), (3136, 3136, 384), (3136, 3136, 385)])
+def test_prompts_of_a_few_hundred_rows_equal_their_tokens_in_pieces(C, F, T):
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"prompt of {T} tokens at C={C} F={F}")
+    m = HipRWKV(synth.make_state_dict(2, C, F, V=100, seed=C + T, ln="random"))
+    toks = synth.random_tokens(T + 3, V=100, seed=T)
+    _, st = m.forward(toks[:3], m.emptyState.clone())
+    lg, sp = m.forward(toks[3:], st.clone())
+    for i in range(3, T + 3, 50):                       # (a workgroup to each row and mix, 256 threads or parts to each row)
+        l1, st = m.forward(toks[i:min(i + 50, T + 3)], st)
+    # exact integer products; LayerNorm and WKV sums joined in another order
+    assert float((lg - l1).norm() / l1.norm()) < 5e-6
+    for row in range(5):
+        assert float((sp[:, row] - st[:, row]).norm() / st[:, row].norm()) < 5e-6, row
+
+
 # both sides of the serial kernels' sizes: a thread per channel below 6 steps, blocks of 32 and of 63 steps
 @pytest.mark.parametrize("T", [4, 5, 6, 8, 9, 31, 32, 33, 48, 63])
 def test_a_short_prompt_has_the_bits_of_its_tokens_one_by_one(T):
