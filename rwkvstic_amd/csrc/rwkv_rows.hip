@@ -1419,6 +1419,12 @@ constexpr int kWkvChunk = 32, kWkvChunked = 64;
 // of 8 (5120 channels, 257 / 512 / 1024 steps: 18.3 / 25.2 / 47.2 against 25.6 / 29.4 / 56.2 us; 2560: 13.8 / 18.3 / 34.6 against
 // 13.3 / 14.6 / 27.2; 16 chunks spill registers: 31 us).
 constexpr int kWkvWide = 4096;
+// Channels up to which eight of them to a workgroup, each chunk shared by eight lanes of four steps, still leave at most one workgroup
+// to a compute unit: half the steps for a lane to work out, for four more rounds of handing on.  Us a prompt with 16 channels / with 8:
+// 12 layers of 512, 1024 tokens 1188 / 1149, 12 of 768, 2000 2914 / 2803, 24 of 1024, 1024 3813 / 3722, 16 of 1536, 700 3283 / 3229, 24 of
+// 2048, 1000 6829 / 6751; 120 tokens, 24 of 1024 1853 / 1838.  With one block of 4 chunks half as
+// many channels are enough: 80 tokens, 24 layers of 2048 2289 / 2305.  At 2560 channels, 320 workgroups, 9904 / 10087 with 1024 tokens.
+constexpr int kWkvNarrow = 2048;
 
 __device__ __forceinline__ float shfl_from(float v, int lane) { return __shfl(v, lane, 64); }
 __device__ __forceinline__ double shfl_from(double v, int lane) { return __shfl(v, lane, 64); }
@@ -1547,7 +1553,10 @@ template <int CH, int SL, int S, int NCH, bool CHUNKED>
 __global__ void __launch_bounds__(CH * SL * NCH) wkv_seq_kernel(const WkvRowsArgs a) {
     static_assert(CH * SL == 64, "a chunk is a wavefront");
     __shared__ double sh[CHUNKED ? 3 : 1][NCH][CH];
-    const int ch = threadIdx.x % CH, C = a.C, c = blockIdx.x * CH + ch;        // (C is a multiple of 64)
+    const int ch = threadIdx.x % CH, C = a.C, n = gridDim.x;                   // (C is a multiple of 64)
+    // Neighbouring channels, which share their cache lines, go to one XCD: workgroup i runs on XCD i % 8, whose channels are consecutive
+    // (24 layers of 2560, 500 / 1024 tokens 6721 / 9963 us a prompt without, 6661 / 9904 with this).
+    const int x = blockIdx.x % kXcds, c = (x * (n / kXcds) + min(x, n % kXcds) + (int)blockIdx.x / kXcds) * CH + ch;
     const double w = a.w[c], u = a.u[c];
     double ca = a.state[c], cb = a.state[C + c], cp = a.state[2 * C + c];
     constexpr int kBlock = NCH * SL * S;
@@ -2213,6 +2222,8 @@ int rows_wkv(hipStream_t st, int64_t R, int C, bool sequence, const float *k, co
         const dim3 g8((unsigned)(C / 8)), g16((unsigned)(C / 16));
         if (R <= 32) hipLaunchKernelGGL((wkv_seq_kernel<8, 8, 4, 1, false>), g8, dim3(64), 0, st, a);
         else if (R < kWkvChunked) hipLaunchKernelGGL((wkv_seq_kernel<8, 8, 8, 1, false>), g8, dim3(64), 0, st, a);
+        else if (C <= kWkvNarrow / 2 && R <= 4 * kWkvChunk) hipLaunchKernelGGL((wkv_seq_kernel<8, 8, 4, 4, true>), g8, dim3(256), 0, st, a);
+        else if (C <= kWkvNarrow && R > 4 * kWkvChunk) hipLaunchKernelGGL((wkv_seq_kernel<8, 8, 4, 8, true>), g8, dim3(512), 0, st, a);
         else if (R <= 4 * kWkvChunk || C >= kWkvWide) hipLaunchKernelGGL((wkv_seq_kernel<16, 4, 8, 4, true>), g16, dim3(256), 0, st, a);
         else hipLaunchKernelGGL((wkv_seq_kernel<16, 4, 8, 8, true>), g16, dim3(512), 0, st, a);
         RWKV_CHECK_LAUNCH("wkv_seq_kernel");

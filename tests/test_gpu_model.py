@@ -792,6 +792,22 @@ def test_long_prompts_keep_float64_sums_between_their_chunks(C, T):
         assert bool((st[0, row].float().double() != st[0, row]).any()), row
 
 
+# channels on both sides of 2048, where a chunk's steps are shared by eight lanes or by four, and counts of workgroups (the channels
+# by 8 or 16) that the XCDs share evenly and not
+@pytest.mark.parametrize("C,T", [(64, 129), (448, 128), (1088, 256), (2048, 130), (2112, 130), (2112, 257), (4160, 130)])
+def test_long_prompts_of_every_width_end_in_the_state_of_their_tokens(C, T):
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"state after a prompt of {T} tokens at C={C}")
+    m = HipRWKV(synth.make_state_dict(1, C, C, V=100, seed=9, ln="random"))
+    toks = synth.random_tokens(T, V=100, seed=T)
+    _, sp = m.forward(toks, m.emptyState.clone())
+    st = m.emptyState.clone()
+    for i in range(0, T, 60):                           # (serial: fewer than 64 steps)
+        _, st = m.forward(toks[i:min(i + 60, T)], st)
+    # each channel for itself: a chunk's sums are joined in another order, a few float32 roundings of 6e-8
+    assert torch.allclose(sp[:, 2:], st[:, 2:], rtol=5e-6, atol=5e-6 * float(st[:, 3].abs().max()))
+
+
 # every width that has both cache policies: layers that fit the cache with a small head and not with a large one
 @pytest.mark.parametrize("C,L,V", [(512, 70, 60000), (768, 30, 50000), (1024, 15, 60000), (1536, 7, 40000), (2048, 3, 60000),
                                    (2560, 2, 50000), (4096, 1, 20000)])
