@@ -5,8 +5,9 @@
 // What bounds these calls is the host: a matrix of the 3B shape is 10 us of kernels, and a call that goes through Python
 // (dispatcher to interpreter, checks, ctypes) takes 16.
 //
-// Anything out of the ordinary - an argument that does not fit, an error of the library - is left to the Python function of the
-// same name, which raises what it always raised.
+// An argument that does not fit is left to the Python function of the same name, which raises what it always raised.  Only
+// arguments are: what the library reports is raised here, since it may report an error after it has launched (one that an
+// earlier HIP call of the thread left behind), and the operators write in place: a second call would add y twice.
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -53,7 +54,15 @@ rwkv_stream_t stream() { return reinterpret_cast<rwkv_stream_t>(c10::hip::getCur
 // A recorded call keeps its scratch for as long as it is replayed: the buffer the Python side holds on to.
 bool recording() {
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(c10::hip::getCurrentHIPStream().stream(), &s) != hipSuccess || s != hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream().stream(), &s) != hipSuccess) { (void)hipGetLastError(); return true; }
+    return s != hipStreamCaptureStatusNone;
+}
+
+// What the library answers to a call: RwkvHipError with its text for anything but RWKV_OK.
+void check(int code) {
+    if (code == RWKV_OK) return;
+    pybind11::gil_scoped_acquire gil;
+    pybind11::module_::import("rwkvstic_amd._native").attr("check")(code);
 }
 
 at::Tensor bytes(size_t n, const at::Tensor &like) {
@@ -85,10 +94,12 @@ bool try_one(int64_t N, int64_t M, const at::Tensor &x, const at::Tensor &w, con
     if (N <= 0 || M <= 0 || x.numel() < N || r.numel() < N || y.numel() < M) return false;
     if (dt == at::kFloat) {
         const at::Tensor ws = bytes(lib.mm8_workspace_bytes(N, M, 1), x);
-        return lib.mm8_one(stream(), N, M, ptr<float>(x), u8(w), w.stride(0), ptr<float>(y), ptr<float>(r), ws.data_ptr(), ws.numel()) == RWKV_OK;
+        check(lib.mm8_one(stream(), N, M, ptr<float>(x), u8(w), w.stride(0), ptr<float>(y), ptr<float>(r), ws.data_ptr(), ws.numel()));
+    } else {
+        const at::Tensor ws = bytes(lib.mm8_f64_workspace_bytes(N, M, 1), x);
+        check(lib.mm8_one_f64(stream(), N, M, ptr<double>(x), u8(w), w.stride(0), ptr<double>(y), ptr<double>(r), ws.data_ptr(), ws.numel()));
     }
-    const at::Tensor ws = bytes(lib.mm8_f64_workspace_bytes(N, M, 1), x);
-    return lib.mm8_one_f64(stream(), N, M, ptr<double>(x), u8(w), w.stride(0), ptr<double>(y), ptr<double>(r), ws.data_ptr(), ws.numel()) == RWKV_OK;
+    return true;
 }
 
 void mm8_one(int64_t N, int64_t M, at::Tensor &x, at::Tensor &w, at::Tensor &y, at::Tensor &r) {
@@ -106,11 +117,13 @@ bool try_three(int64_t N, int64_t M, T3 x, T3 w, T3 y, T3 r) {
     auto call = [&](auto fn, auto bytes_fn, auto zero) {
         using T = decltype(zero);
         const at::Tensor ws = bytes(bytes_fn(N, M, 3), *x[0]);
-        return fn(stream(), N, M, ptr<T>(*x[0]), ptr<T>(*x[1]), ptr<T>(*x[2]), u8(*w[0]), w[0]->stride(0), u8(*w[1]), w[1]->stride(0),
-                  u8(*w[2]), w[2]->stride(0), ptr<T>(*y[0]), ptr<T>(*y[1]), ptr<T>(*y[2]), ptr<T>(*r[0]), ptr<T>(*r[1]), ptr<T>(*r[2]),
-                  ws.data_ptr(), ws.numel()) == RWKV_OK;
+        check(fn(stream(), N, M, ptr<T>(*x[0]), ptr<T>(*x[1]), ptr<T>(*x[2]), u8(*w[0]), w[0]->stride(0), u8(*w[1]), w[1]->stride(0),
+                 u8(*w[2]), w[2]->stride(0), ptr<T>(*y[0]), ptr<T>(*y[1]), ptr<T>(*y[2]), ptr<T>(*r[0]), ptr<T>(*r[1]), ptr<T>(*r[2]),
+                 ws.data_ptr(), ws.numel()));
     };
-    return dt == at::kFloat ? call(lib.mm8_three, lib.mm8_workspace_bytes, 0.f) : call(lib.mm8_three_f64, lib.mm8_f64_workspace_bytes, 0.0);
+    if (dt == at::kFloat) call(lib.mm8_three, lib.mm8_workspace_bytes, 0.f);
+    else call(lib.mm8_three_f64, lib.mm8_f64_workspace_bytes, 0.0);
+    return true;
 }
 
 void mm8_three(int64_t N, int64_t M, at::Tensor &x, at::Tensor &x1, at::Tensor &x2, at::Tensor &w, at::Tensor &w1, at::Tensor &w2,
@@ -126,9 +139,9 @@ void wkv_forward(int64_t B, int64_t T, int64_t C, at::Tensor &w, at::Tensor &u, 
     for (const at::Tensor *t : {&k, &v, &y}) ok = ok && t->numel() / C / T >= B;
     for (const at::Tensor *t : {&aa, &bb, &pp}) ok = ok && t->numel() / C >= B;
     for (const at::Tensor *t : {&w, &u}) ok = ok && t->numel() >= C;
-    if (!ok || lib.wkv_forward_f64(stream(), B, T, C, ptr<double>(w), ptr<double>(u), ptr<double>(k), ptr<double>(v), ptr<double>(y),
-                                   ptr<double>(aa), ptr<double>(bb), ptr<double>(pp)) != RWKV_OK)
-        in_python("wkv_forward", B, T, C, w, u, k, v, y, aa, bb, pp);
+    if (!ok) return in_python("wkv_forward", B, T, C, w, u, k, v, y, aa, bb, pp);
+    check(lib.wkv_forward_f64(stream(), B, T, C, ptr<double>(w), ptr<double>(u), ptr<double>(k), ptr<double>(v), ptr<double>(y),
+                              ptr<double>(aa), ptr<double>(bb), ptr<double>(pp)));
 }
 
 // The reference's schemas (wrapper.cpp:131-141).
@@ -181,8 +194,8 @@ bool product(Product &p, decltype(lib.packed_bytes) bytes_fn, Arg x, Arg packed,
 pybind11::object mm8_packed(Arg x, Arg packed, int64_t n_in, int64_t n_out, Arg r_row, Arg m_row, Arg r_col, Arg m_col, Arg out) {
     Product p;
     if (!product(p, lib.packed_bytes, x, packed, n_in, n_out, r_row, m_row, r_col, m_col, out)) return pybind11::none();
-    if (lib.mm8_packed(stream(), p.x->size(0), n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
-                       p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y)) != RWKV_OK) return pybind11::none();
+    check(lib.mm8_packed(stream(), p.x->size(0), n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
+                         p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y)));
     return out.is_none() ? pybind11::cast(p.y) : pybind11::reinterpret_borrow<pybind11::object>(out);
 }
 
@@ -194,8 +207,8 @@ pybind11::object mm8_m16(Arg x, Arg packed, int64_t n_in, int64_t n_out, Arg r_r
     if (workspace.is_none()) ws = bytes(lib.mm8_m16_workspace_bytes(B, n_in), *p.x);
     else if (const at::Tensor *t = tensor(workspace)) ws = *t;
     else return pybind11::none();
-    if (lib.mm8_m16(stream(), B, n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
-                    p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y), ws.data_ptr(), ws.numel()) != RWKV_OK) return pybind11::none();
+    check(lib.mm8_m16(stream(), B, n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
+                      p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y), ws.data_ptr(), ws.numel()));
     return out.is_none() ? pybind11::cast(p.y) : pybind11::reinterpret_borrow<pybind11::object>(out);
 }
 
@@ -211,8 +224,8 @@ pybind11::object wkv_f32(Arg w, Arg u, Arg k, Arg v, Arg aa, Arg bb, Arg pp) {
     for (int i : {4, 5, 6}) if (t[i]->numel() < B * C) return pybind11::none();
     for (int i : {0, 1}) if (t[i]->numel() < C) return pybind11::none();
     at::Tensor y = at::empty_like(*t[2]);
-    if (lib.wkv_f32(stream(), B, T, C, ptr<float>(*t[0]), ptr<float>(*t[1]), ptr<float>(*t[2]), ptr<float>(*t[3]), ptr<float>(y),
-                    ptr<float>(*t[4]), ptr<float>(*t[5]), ptr<float>(*t[6])) != RWKV_OK) return pybind11::none();
+    check(lib.wkv_f32(stream(), B, T, C, ptr<float>(*t[0]), ptr<float>(*t[1]), ptr<float>(*t[2]), ptr<float>(*t[3]), ptr<float>(y),
+                      ptr<float>(*t[4]), ptr<float>(*t[5]), ptr<float>(*t[6])));
     return pybind11::cast(y);
 }
 

@@ -1,0 +1,95 @@
+"""The native host side of the operators (csrc/rwkv_torch.cpp): what it does with the answers of the library, checked with
+entry points bound to functions of the test in place of the library's, so that nothing wrong is ever launched."""
+import contextlib
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from rwkvstic_amd import ops as _ops
+    _ops.register_torch_ops()
+    return _ops
+
+
+@contextlib.contextmanager
+def _bound(**entries):
+    """The host side with some of its entry points replaced by the addresses given."""
+    from rwkvstic_amd import _native as N
+    own = {n: C.cast(getattr(N.lib(), n), C.c_void_p).value for n in N.EXPORTS}
+    N.host().bind({**own, **entries})
+    try:
+        yield
+    finally:
+        N.host().bind(own)
+
+
+def _calls(ops):
+    """Each operator once: (library entry, call, the tensors it writes)."""
+    g = torch.Generator().manual_seed(1)
+    n_in, n_out = 256, 48
+    codes = torch.randint(0, 256, (n_in, n_out), generator=g, dtype=torch.uint8).cuda()
+    for dt, suffix in ((torch.float32, ""), (torch.float64, "_f64")):
+        x, r = torch.randn(n_in, generator=g, dtype=dt).cuda(), torch.rand(n_in, generator=g, dtype=dt).cuda()
+        ys = [torch.randn(n_out, generator=g, dtype=dt).cuda() for _ in range(4)]
+        yield "rwkv_mm8_one" + suffix, lambda: torch.ops.rwkv.mm8_one(n_in, n_out, x, codes, ys[0], r), ys[:1]
+        yield "rwkv_mm8_three" + suffix, lambda: torch.ops.rwkv.mm8_three(n_in, n_out, x, x, x, codes, codes, codes, *ys[1:], r, r, r), ys[1:]
+    for dt, entry in ((torch.float64, "rwkv_wkv_forward_f64"), (torch.float32, "rwkv_wkv_f32")):
+        f = lambda *s: torch.rand(*s, generator=g, dtype=dt).cuda()
+        w, u, k, v, y = -f(32), f(32), f(2, 5, 32), f(2, 5, 32), f(2, 5, 32)
+        state = [f(2, 32), f(2, 32) + 0.5, f(2, 32)]
+        if dt == torch.float64:
+            yield entry, lambda: torch.ops.rwkv.wkv_forward(2, 5, 32, w, u, k, v, y, *state), state + [y]
+        else:
+            yield entry, lambda: ops.wkv_f32(w, u, k, v, *state), state
+    x, r, m = torch.randn(2, n_in, generator=g).cuda(), torch.rand(n_in, generator=g).cuda(), torch.randn(n_in, generator=g).double().cuda()
+    y = torch.randn(2, n_out, generator=g).double().cuda()
+    p, p16 = ops.pack(codes), ops.pack_m16(codes)
+    yield "rwkv_mm8_packed", lambda: ops.mm8_packed(x, p, n_in, n_out, r, m, out=y), [y]
+    yield "rwkv_mm8_m16", lambda: ops.mm8_m16(x, p16, n_in, n_out, r, m, out=y), [y]
+
+
+def test_an_error_of_the_library_is_raised_and_nothing_is_done_again(ops):
+    """A library that answers RWKV_ERR_HIP may have launched all the same, so the call is not repeated by other means."""
+    from rwkvstic_amd import _native as N
+    for entry, call, written in _calls(ops):
+        print(f"error from {entry}", flush=True)
+        before, seen = [t.clone() for t in written], []
+        fails = C.CFUNCTYPE(C.c_int)(lambda: seen.append(1) or -5)
+        with _bound(**{entry: C.cast(fails, C.c_void_p).value}):
+            with pytest.raises(N.RwkvHipError) as e:
+                call()
+        torch.cuda.synchronize()
+        assert e.value.code == -5 and len(seen) == 1, entry
+        assert all(torch.equal(a, b) for a, b in zip(before, written)), entry
+
+
+def test_an_error_left_by_another_hip_call_does_not_repeat_an_operator(ops):
+    """The same from the other end: a HIP call of this thread has failed (an allocation of 2^60 bytes) and nobody has read
+    its error, which the library then reports after its own launch.  Each operator raises, and has run at most once."""
+    from rwkvstic_amd import _native as N
+    L = N.lib()
+    at = C.c_void_p()
+    for entry, call, written in _calls(ops):
+        print(f"error left before {entry}", flush=True)
+        start = [t.clone() for t in written]
+        call()
+        torch.cuda.synchronize()
+        once = [t.clone() for t in written]
+        for t, b in zip(written, start):
+            t.copy_(b)
+        torch.cuda.synchronize()
+        assert L.hipMalloc(C.byref(at), C.c_size_t(1 << 60)) != 0
+        try:
+            call()
+        except N.RwkvHipError as e:
+            assert e.code == -5
+        finally:
+            L.hipGetLastError()
+        torch.cuda.synchronize()
+        for t, a, b in zip(written, start, once):
+            assert torch.equal(t, a) or torch.equal(t, b), entry
