@@ -29,9 +29,10 @@ int set_error(int code, const char *fmt, ...);
 #define RWKV_CHECK_ALIGN(ptr, a) \
     do { if ((reinterpret_cast<uintptr_t>(ptr) % (a)) != 0) \
         return ::rwkv::set_error(RWKV_ERR_ALIGN, #ptr " must be %d-byte aligned", int(a)); } while (0)
+// (the runtime keeps a failed call's error until it is read: left there, the next launch of this thread would be blamed for it)
 #define RWKV_CHECK_HIP(expr) \
-    do { hipError_t e_ = (expr); if (e_ != hipSuccess) \
-        return ::rwkv::set_error(RWKV_ERR_HIP, "%s: %s", #expr, hipGetErrorString(e_)); } while (0)
+    do { hipError_t e_ = (expr); if (e_ != hipSuccess) { (void)hipGetLastError(); \
+        return ::rwkv::set_error(RWKV_ERR_HIP, "%s: %s", #expr, hipGetErrorString(e_)); } } while (0)
 #define RWKV_CHECK_LAUNCH(name) \
     do { hipError_t e_ = hipGetLastError(); if (e_ != hipSuccess) \
         return ::rwkv::set_error(RWKV_ERR_HIP, "launch of %s: %s", name, hipGetErrorString(e_)); } while (0)

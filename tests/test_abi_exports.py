@@ -75,3 +75,30 @@ def test_single_token_kernels_do_not_spill_ring_registers():
         regs |= set(r + i for r in list(regs) for i in range(4))
         clob = set(int(x) for x in re.findall(r'"v(\d+)"', block))
         assert regs and regs <= clob
+
+
+def test_a_failed_hip_call_leaves_no_error_behind(tmp_path):
+    """The runtime keeps an error until somebody reads it, and a launch check that reads it blames its own kernel.  The
+    checking macros, compiled against a runtime of a few lines that keeps errors as HIP does."""
+    import shutil
+    import subprocess
+    if not shutil.which("g++"):
+        pytest.skip("no g++")
+    (tmp_path / "hip").mkdir()
+    (tmp_path / "hip" / "hip_runtime.h").write_text(
+        "#pragma once\n#define __host__\n#define __device__\n#define __forceinline__ inline\n"
+        "enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2 };\n"
+        "inline hipError_t kept = hipSuccess;\n"
+        "inline hipError_t hipGetLastError() { const hipError_t e = kept; kept = hipSuccess; return e; }\n"
+        "inline const char *hipGetErrorString(hipError_t e) { return e ? \"out of memory\" : \"none\"; }\n")
+    (tmp_path / "main.cpp").write_text(
+        '#include "rwkv_common.h"\n'
+        "int rwkv::set_error(int code, const char *, ...) { return code; }\n"
+        "hipError_t fails() { return kept = hipErrorOutOfMemory; }\n"
+        "int allocate() { RWKV_CHECK_HIP(fails()); return RWKV_OK; }\n"
+        'int launch() { RWKV_CHECK_LAUNCH("kernel"); return RWKV_OK; }\n'
+        "int main() { return allocate() == RWKV_ERR_HIP && launch() == RWKV_OK ? 0 : 1; }\n")
+    exe = str(tmp_path / "main")
+    subprocess.run(["g++", "-std=c++17", "-I", str(tmp_path), "-I", os.path.join(ROOT, "rwkvstic_amd", "csrc"), "-o", exe,
+                    str(tmp_path / "main.cpp")], check=True)
+    assert subprocess.run([exe]).returncode == 0
