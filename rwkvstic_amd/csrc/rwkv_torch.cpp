@@ -70,7 +70,7 @@ at::Tensor bytes(size_t n, const at::Tensor &like) {
 }
 
 bool on_gpu(const at::Tensor &t, at::ScalarType dt) { return t.defined() && t.is_cuda() && t.scalar_type() == dt && !t.requires_grad(); }
-bool vec(const at::Tensor &t, at::ScalarType dt) { return on_gpu(t, dt) && t.dim() >= 1 && t.stride(0) == 1; }
+bool vec(const at::Tensor &t, at::ScalarType dt) { return on_gpu(t, dt) && t.dim() == 1 && t.stride(0) == 1; }
 bool codes(const at::Tensor &w, int64_t n, int64_t m) {
     return on_gpu(w, at::kByte) && w.dim() == 2 && w.stride(1) == 1 && w.size(0) >= n && w.size(1) >= m;
 }
@@ -90,7 +90,7 @@ void in_python(const char *name, A &&...args) {
 bool try_one(int64_t N, int64_t M, const at::Tensor &x, const at::Tensor &w, const at::Tensor &y, const at::Tensor &r) {
     const auto dt = x.scalar_type();
     if ((dt != at::kFloat && dt != at::kDouble) || recording()) return false;
-    if (!vec(x, dt) || x.dim() != 1 || !vec(y, dt) || !vec(r, dt) || !codes(w, N, M)) return false;
+    if (!vec(x, dt) || !vec(y, dt) || !vec(r, dt) || !codes(w, N, M)) return false;
     if (N <= 0 || M <= 0 || x.numel() < N || r.numel() < N || y.numel() < M) return false;
     if (dt == at::kFloat) {
         const at::Tensor ws = bytes(lib.mm8_workspace_bytes(N, M, 1), x);

@@ -56,13 +56,19 @@ def _mm8_dtype(x: torch.Tensor, others, what: str) -> torch.dtype:
     return x.dtype
 
 
+def _holds(t: torch.Tensor, n: int) -> bool:
+    """Whether the kernels may read or write ``n`` values one after the other from the tensor's first on (a view can have as
+    many elements and less memory)."""
+    return t.numel() >= n and t.untyped_storage().nbytes() // t.element_size() - t.storage_offset() >= n
+
+
 def mm8_one(N_in: int, M_out: int, x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, r: torch.Tensor) -> None:
     """``y[k] += sum_j x[j]*(w[j,k]*r[j])``; argument meaning of wrapper.cpp:52-54 (N=in, M=out); x, y, r all
     float32 or all float64 (wrapper.cpp:60-77)."""
     dt = _mm8_dtype(x, (x, y, r), "mm8_one"); _req(w, torch.uint8, "w")
     if x.dim() != 1 or x.stride(0) != 1 or y.stride(0) != 1 or w.dim() != 2 or w.stride(1) != 1:
         raise ValueError("mm8_one: x, y need unit stride and w.stride(1) == 1 (wrapper.cpp:55-57)")
-    if x.numel() < N_in or r.numel() < N_in or y.numel() < M_out or w.shape[0] < N_in or w.shape[1] < M_out:
+    if not (_holds(x, N_in) and _holds(r, N_in) and _holds(y, M_out)) or w.shape[0] < N_in or w.shape[1] < M_out:
         raise ValueError("mm8_one: tensor smaller than (N, M)")
     L = N.lib()
     f64 = dt == torch.float64
@@ -77,6 +83,8 @@ def mm8_three(N_in: int, M_out: int, x0, x1, x2, w0, w1, w2, y0, y1, y2, r0, r1,
     for t in (x0, x1, x2, y0, y1, y2, r0, r1, r2):
         if t.stride(0) != 1:
             raise ValueError("mm8_three: x, y, r need unit stride")
+    if not (all(_holds(t, N_in) for t in (x0, x1, x2, r0, r1, r2)) and all(_holds(t, M_out) for t in (y0, y1, y2))):
+        raise ValueError("mm8_three: tensor smaller than (N, M)")
     for t in (w0, w1, w2):
         _req(t, torch.uint8, "w")
         if t.dim() != 2 or t.stride(1) != 1 or t.shape[0] < N_in or t.shape[1] < M_out:

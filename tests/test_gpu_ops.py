@@ -374,6 +374,11 @@ def _calls(ops):
         yield "mm8_one", (0, n_out, x, w, y, r)
         yield "mm8_three", (n_in, n_out, x, x, x, w, w[:, 1:1 + n_out], w, y, y.clone(), y.clone(), r, r, r)
         yield "mm8_three", (n_in, n_out, x, x, x, w, w[:-1], w, y, y.clone(), y.clone(), r, r, r)     # refused: size
+        yield "mm8_three", (n_in, n_out, x, x[:-1], x, w, w, w, y, y.clone(), y.clone(), r, r, r)
+        yield "mm8_three", (n_in, n_out, x, x, x, w, w, w, y, y.clone(), y.clone()[:-1], r, r, r)
+        yield "mm8_three", (n_in, n_out, x, x, x, w, w, w, y, y.clone(), y.clone(), r[1:], r, r)
+        yield "mm8_one", (n_in, n_out, x, w, y, r.new_ones(1).expand(n_in))                              # refused: as many values, less memory
+        yield "mm8_one", (n_in, n_out, x, w, y.new_ones(1, 1).expand(1, n_out), r)
     f = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64).cuda()
     wkv = lambda T, C: (2, T, C, -f(C), f(C), f(2, T, C), f(2, T, C), f(2, T, C), f(2, C), f(2, C) + 0.5, f(2, C))
     yield "wkv_forward", wkv(3, 5)
