@@ -174,18 +174,18 @@ bool product(Product &p, decltype(lib.packed_bytes) bytes_fn, Arg x, Arg packed,
              Arg r_col, Arg m_col, Arg out) {
     p.x = tensor(x); p.packed = tensor(packed); p.r_row = tensor(r_row); p.m_row = tensor(m_row);
     if (!p.x || !p.packed || !p.r_row || !p.m_row || n_in <= 0 || n_out <= 0) return false;
-    if (!whole(*p.x, at::kFloat) || p.x->dim() != 2 || p.x->size(1) != n_in || !on_gpu(*p.packed, at::kByte) ||
-        !on_gpu(*p.r_row, at::kFloat) || !on_gpu(*p.m_row, at::kDouble)) return false;
+    if (!whole(*p.x, at::kFloat) || p.x->dim() != 2 || p.x->size(1) != n_in || !whole(*p.packed, at::kByte) ||
+        !whole(*p.r_row, at::kFloat) || !whole(*p.m_row, at::kDouble)) return false;
     if (p.packed->numel() < (int64_t)bytes_fn(n_in, n_out) || p.r_row->numel() < n_in || p.m_row->numel() < n_in) return false;
     for (auto [h, t] : {std::pair{r_col, &p.r_col}, std::pair{m_col, &p.m_col}}) {
         if (h.is_none()) continue;
         *t = tensor(h);
-        if (!*t || !on_gpu(**t, at::kFloat) || (*t)->numel() < n_out) return false;
+        if (!*t || !whole(**t, at::kFloat) || (*t)->numel() < n_out) return false;
     }
     if (out.is_none()) p.y = at::empty({p.x->size(0), n_out}, p.x->options().dtype(at::kDouble));
     else {
         const at::Tensor *t = tensor(out);
-        if (!t || !whole(*t, at::kDouble)) return false;
+        if (!t || !whole(*t, at::kDouble) || t->numel() < p.x->size(0) * n_out) return false;
         p.y = *t;
     }
     return true;
@@ -205,7 +205,7 @@ pybind11::object mm8_m16(Arg x, Arg packed, int64_t n_in, int64_t n_out, Arg r_r
     const int64_t B = p.x->size(0);
     at::Tensor ws;
     if (workspace.is_none()) ws = bytes(lib.mm8_m16_workspace_bytes(B, n_in), *p.x);
-    else if (const at::Tensor *t = tensor(workspace)) ws = *t;
+    else if (const at::Tensor *t = tensor(workspace); t && t->is_cuda() && t->is_contiguous()) ws = *t;
     else return pybind11::none();
     check(lib.mm8_m16(stream(), B, n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
                       p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y), ws.data_ptr(), ws.numel()));

@@ -225,6 +225,28 @@ def dequant_packed(packed, rng, off, n_in: int, n_out: int) -> torch.Tensor:
 
 
 # ---------------------------------------------------------------- stand-alone kernels
+def _buffer(t: torch.Tensor, dtype, n: int, name: str) -> None:
+    """``n`` values that the kernels read or write one after the other."""
+    _req(t, dtype, name); _contig(t, name)
+    if t.numel() < n:
+        raise ValueError(f"{name} too small")
+
+
+def _matvec_args(x, packed, packed_bytes: int, n_in: int, n_out: int, r_row, m_row, r_col, m_col, out) -> torch.Tensor:
+    """Checks what ``mm8_packed`` and ``mm8_m16`` are given; returns the tensor their results go to."""
+    _req(x, torch.float32, "x"); _contig(x, "x")
+    if x.dim() != 2 or x.shape[1] != n_in:
+        raise ValueError("x must be [B, n_in]")
+    _buffer(packed, torch.uint8, packed_bytes, "packed weights")
+    _buffer(r_row, torch.float32, n_in, "r_row"); _buffer(m_row, torch.float64, n_in, "m_row")
+    for t, nm in ((r_col, "r_col"), (m_col, "m_col")):
+        if t is not None:
+            _buffer(t, torch.float32, n_out, nm)
+    y = out if out is not None else torch.empty((x.shape[0], n_out), dtype=torch.float64, device=x.device)
+    _buffer(y, torch.float64, x.shape[0] * n_out, "out")
+    return y
+
+
 def mm8_packed(x: torch.Tensor, packed: torch.Tensor, n_in: int, n_out: int,
                r_row: torch.Tensor, m_row: torch.Tensor,
                r_col: Optional[torch.Tensor] = None, m_col: Optional[torch.Tensor] = None,
@@ -233,21 +255,9 @@ def mm8_packed(x: torch.Tensor, packed: torch.Tensor, n_in: int, n_out: int,
     y = N.host().mm8_packed(x, packed, n_in, n_out, r_row, m_row, r_col, m_col, out)
     if y is not None:
         return y
-    _req(x, torch.float32, "x"); _contig(x, "x")
-    _req(packed, torch.uint8, "packed"); _req(r_row, torch.float32, "r_row"); _req(m_row, torch.float64, "m_row")
-    if x.dim() != 2 or x.shape[1] != n_in:
-        raise ValueError("x must be [B, n_in]")
     L = N.lib()
-    if packed.numel() < L.rwkv_packed_bytes(n_in, n_out) or r_row.numel() < n_in or m_row.numel() < n_in:
-        raise ValueError("buffer too small")
-    for t, nm in ((r_col, "r_col"), (m_col, "m_col")):
-        if t is not None:
-            _req(t, torch.float32, nm)
-            if t.numel() < n_out:
-                raise ValueError(f"{nm} too small")
+    y = _matvec_args(x, packed, L.rwkv_packed_bytes(n_in, n_out), n_in, n_out, r_row, m_row, r_col, m_col, out)
     B = x.shape[0]
-    y = out if out is not None else torch.empty((B, n_out), dtype=torch.float64, device=x.device)
-    _req(y, torch.float64, "out"); _contig(y, "out")
     N.check(L.rwkv_mm8_packed(_stream(), B, n_in, n_out, x.data_ptr(), packed.data_ptr(), r_row.data_ptr(),
                               m_row.data_ptr(), r_col.data_ptr() if r_col is not None else None,
                               m_col.data_ptr() if m_col is not None else None, y.data_ptr()))
@@ -263,23 +273,12 @@ def mm8_m16(x: torch.Tensor, packed16: torch.Tensor, n_in: int, n_out: int,
     y = N.host().mm8_m16(x, packed16, n_in, n_out, r_row, m_row, r_col, m_col, out, workspace)
     if y is not None:
         return y
-    _req(x, torch.float32, "x"); _contig(x, "x")
-    _req(packed16, torch.uint8, "packed16"); _req(r_row, torch.float32, "r_row"); _req(m_row, torch.float64, "m_row")
-    if x.dim() != 2 or x.shape[1] != n_in:
-        raise ValueError("x must be [B, n_in]")
     L = N.lib()
-    if packed16.numel() < L.rwkv_packed_m16_bytes(n_in, n_out) or r_row.numel() < n_in or m_row.numel() < n_in:
-        raise ValueError("buffer too small")
-    for t, nm in ((r_col, "r_col"), (m_col, "m_col")):
-        if t is not None:
-            _req(t, torch.float32, nm)
-            if t.numel() < n_out:
-                raise ValueError(f"{nm} too small")
+    y = _matvec_args(x, packed16, L.rwkv_packed_m16_bytes(n_in, n_out), n_in, n_out, r_row, m_row, r_col, m_col, out)
     B = x.shape[0]
-    y = out if out is not None else torch.empty((B, n_out), dtype=torch.float64, device=x.device)
-    _req(y, torch.float64, "out"); _contig(y, "out")
     need = L.rwkv_mm8_m16_workspace_bytes(B, n_in)
     ws = workspace if workspace is not None else torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+    _buffer(ws, ws.dtype, 0, "workspace")               # (its bytes are counted by the library)
     N.check(L.rwkv_mm8_m16(_stream(), B, n_in, n_out, x.data_ptr(), packed16.data_ptr(), r_row.data_ptr(),
                            m_row.data_ptr(), r_col.data_ptr() if r_col is not None else None,
                            m_col.data_ptr() if m_col is not None else None, y.data_ptr(), ws.data_ptr(), ws.numel()))
