@@ -162,6 +162,15 @@ void register_ops() {
 
 // ---- stand-alone kernels: the result, or None where the Python function has to look at the call ------------------------
 using Arg = pybind11::handle;
+
+// The library's answer to a call from Python, made without the interpreter's lock: a launch waits where the queue is full.
+// (The operators above come through torch's dispatcher, which has let go of it.)
+template <typename F, typename... A>
+void unlocked(F fn, A... args) {
+    pybind11::gil_scoped_release gil;
+    check(fn(stream(), args...));
+}
+
 const at::Tensor *tensor(Arg a) { return THPVariable_CheckExact(a.ptr()) ? &THPVariable_Unpack(a.ptr()) : nullptr; }
 
 struct Product {
@@ -194,8 +203,8 @@ bool product(Product &p, decltype(lib.packed_bytes) bytes_fn, Arg x, Arg packed,
 pybind11::object mm8_packed(Arg x, Arg packed, int64_t n_in, int64_t n_out, Arg r_row, Arg m_row, Arg r_col, Arg m_col, Arg out) {
     Product p;
     if (!product(p, lib.packed_bytes, x, packed, n_in, n_out, r_row, m_row, r_col, m_col, out)) return pybind11::none();
-    check(lib.mm8_packed(stream(), p.x->size(0), n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
-                         p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y)));
+    unlocked(lib.mm8_packed, p.x->size(0), n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
+             p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y));
     return out.is_none() ? pybind11::cast(p.y) : pybind11::reinterpret_borrow<pybind11::object>(out);
 }
 
@@ -207,8 +216,8 @@ pybind11::object mm8_m16(Arg x, Arg packed, int64_t n_in, int64_t n_out, Arg r_r
     if (workspace.is_none()) ws = bytes(lib.mm8_m16_workspace_bytes(B, n_in), *p.x);
     else if (const at::Tensor *t = tensor(workspace); t && t->is_cuda() && t->is_contiguous()) ws = *t;
     else return pybind11::none();
-    check(lib.mm8_m16(stream(), B, n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
-                      p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y), ws.data_ptr(), ws.numel()));
+    unlocked(lib.mm8_m16, B, n_in, n_out, ptr<float>(*p.x), u8(*p.packed), ptr<float>(*p.r_row), ptr<double>(*p.m_row),
+             p.col(p.r_col), p.col(p.m_col), ptr<double>(p.y), ws.data_ptr(), (size_t)ws.numel());
     return out.is_none() ? pybind11::cast(p.y) : pybind11::reinterpret_borrow<pybind11::object>(out);
 }
 
@@ -224,8 +233,8 @@ pybind11::object wkv_f32(Arg w, Arg u, Arg k, Arg v, Arg aa, Arg bb, Arg pp) {
     for (int i : {4, 5, 6}) if (t[i]->numel() < B * C) return pybind11::none();
     for (int i : {0, 1}) if (t[i]->numel() < C) return pybind11::none();
     at::Tensor y = at::empty_like(*t[2]);
-    check(lib.wkv_f32(stream(), B, T, C, ptr<float>(*t[0]), ptr<float>(*t[1]), ptr<float>(*t[2]), ptr<float>(*t[3]), ptr<float>(y),
-                      ptr<float>(*t[4]), ptr<float>(*t[5]), ptr<float>(*t[6])));
+    unlocked(lib.wkv_f32, B, T, C, ptr<float>(*t[0]), ptr<float>(*t[1]), ptr<float>(*t[2]), ptr<float>(*t[3]), ptr<float>(y),
+             ptr<float>(*t[4]), ptr<float>(*t[5]), ptr<float>(*t[6]));
     return pybind11::cast(y);
 }
 

@@ -93,3 +93,37 @@ def test_an_error_left_by_another_hip_call_does_not_repeat_an_operator(ops):
         torch.cuda.synchronize()
         for t, a, b in zip(written, start, once):
             assert torch.equal(t, a) or torch.equal(t, b), entry
+
+
+def test_other_threads_run_while_a_launch_waits(ops):
+    """A launch waits where the stream's queue is full.  poll(0, 0, ms) stands for one that does: of no vectors of 300 values (or
+    no sequences of 300 steps) on the default stream, the entries' first arguments are just that."""
+    import threading
+    import time
+    ms, f = 300, lambda *s, dt=torch.float32: torch.zeros(*s, dtype=dt, device="cuda")
+    codes = torch.zeros(ms, 16, dtype=torch.uint8, device="cuda")
+    args = f(ms), f(ms, dt=torch.float64)
+    calls = {"rwkv_mm8_packed": lambda p=ops.pack(codes): ops.mm8_packed(f(0, ms), p, ms, 16, *args),
+             "rwkv_mm8_m16": lambda p=ops.pack_m16(codes): ops.mm8_m16(f(0, ms), p, ms, 16, *args),
+             "rwkv_wkv_f32": lambda: ops.wkv_f32(f(4), f(4), f(0, ms, 4), f(0, ms, 4), f(0, 4), f(0, 4), f(0, 4))}
+    assert torch.cuda.current_stream().cuda_stream == 0
+    poll = C.cast(C.CDLL(None).poll, C.c_void_p).value
+    for entry, call in calls.items():
+        rounds, stop = [0], threading.Event()
+
+        def count():
+            while not stop.wait(0.001):
+                rounds[0] += 1
+
+        t = threading.Thread(target=count)
+        t.start()
+        try:
+            with _bound(**{entry: poll}):
+                before, start = rounds[0], time.monotonic()
+                call()
+                took, ran = time.monotonic() - start, rounds[0] - before
+        finally:
+            stop.set()
+            t.join()
+        print(f"{entry}: {took:.3f} s, {ran} rounds of another thread", flush=True)
+        assert took >= ms * 1e-3 and ran >= 50, entry
