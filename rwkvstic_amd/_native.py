@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "librwkv_hip.so")
@@ -137,17 +138,19 @@ _host = None
 
 
 def host():
-    """The native host side of the operator calls (csrc/rwkv_torch.cpp), bound to the library ``lib()`` has loaded."""
+    """The native host side of the operator calls (csrc/rwkv_torch.cpp), bound to the library ``lib()`` has loaded.  None, with
+    a warning, where it is missing or was built for another torch: the operators' Python functions launch the same kernels."""
     global _host
     if _host is None or _host[0] is not lib():
+        L, module = lib(), None
         try:
-            from . import _rwkv_torch
+            import torch  # noqa: F401  (its libraries, which the module is linked against)
+            from . import _rwkv_torch as module
+            module.bind({n: C.cast(getattr(L, n), C.c_void_p).value for n in EXPORTS})
         except ImportError as e:
-            raise RuntimeError(f"{os.path.join(HERE, '_rwkv_torch.so')} is missing or was built for another torch: build it "
-                               f"with `python -m rwkvstic_amd.build` ({e})") from e
-        L = lib()
-        _rwkv_torch.bind({n: C.cast(getattr(L, n), C.c_void_p).value for n in EXPORTS})
-        _host = (L, _rwkv_torch)
+            warnings.warn(f"{os.path.join(HERE, '_rwkv_torch.so')} is missing or was built for another torch: operator calls go through "
+                          f"Python, which takes microseconds more each; build it with `python -m rwkvstic_amd.build` ({e})", stacklevel=3)
+        _host = (L, module)
     return _host[1]
 
 

@@ -16,6 +16,7 @@
 
 #include <map>
 #include <string>
+#include <vector>
 
 #include "../../include/rwkv_hip.h"
 
@@ -144,16 +145,11 @@ void wkv_forward(int64_t B, int64_t T, int64_t C, at::Tensor &w, at::Tensor &u, 
                               ptr<double>(aa), ptr<double>(bb), ptr<double>(pp)));
 }
 
-// The reference's schemas (wrapper.cpp:131-141).
-void register_ops() {
+void register_ops(const std::vector<std::string> &schemas) {
     static torch::Library *published = nullptr;      // (lives as long as the process: operators are looked up until its end)
     if (published) return;
     auto *l = new torch::Library(torch::Library::DEF, "rwkv", std::nullopt, __FILE__, __LINE__);
-    l->def("wkv_forward(int B, int T, int C, Tensor(a!) w, Tensor(b!) u, Tensor(c!) k, Tensor(d!) v, Tensor(e!) y, Tensor(f!) aa, "
-           "Tensor(g!) bb, Tensor(h!) pp) -> ()");
-    l->def("mm8_one(int N, int M, Tensor(a!) x, Tensor(b!) w, Tensor(c!) y, Tensor(d!) r) -> ()");
-    l->def("mm8_three(int N, int M, Tensor(a!) x, Tensor(b!) x1, Tensor(c!) x2, Tensor(d!) w, Tensor(e!) w1, Tensor(f!) w2, "
-           "Tensor(g!) y, Tensor(h!) y1, Tensor(i!) y2, Tensor(j!) r, Tensor(k!) r1, Tensor(l!) r2) -> ()");
+    for (const std::string &s : schemas) l->def(s.c_str());
     l->impl("wkv_forward", c10::DispatchKey::CUDA, TORCH_FN(wkv_forward));
     l->impl("mm8_one", c10::DispatchKey::CUDA, TORCH_FN(mm8_one));
     l->impl("mm8_three", c10::DispatchKey::CUDA, TORCH_FN(mm8_three));

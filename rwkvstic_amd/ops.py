@@ -112,16 +112,32 @@ def wkv_forward(B: int, T: int, C: int, w, u, k, v, y, aa, bb, pp) -> None:
 
 
 _registered = False
+_SCHEMAS = (
+    "wkv_forward(int B, int T, int C, Tensor(a!) w, Tensor(b!) u, Tensor(c!) k, Tensor(d!) v, Tensor(e!) y, Tensor(f!) aa, "
+    "Tensor(g!) bb, Tensor(h!) pp) -> ()",
+    "mm8_one(int N, int M, Tensor(a!) x, Tensor(b!) w, Tensor(c!) y, Tensor(d!) r) -> ()",
+    "mm8_three(int N, int M, Tensor(a!) x, Tensor(b!) x1, Tensor(c!) x2, Tensor(d!) w, Tensor(e!) w1, Tensor(f!) w2, "
+    "Tensor(g!) y, Tensor(h!) y1, Tensor(i!) y2, Tensor(j!) r, Tensor(k!) r1, Tensor(l!) r2) -> ()",
+)
 
 
 def register_torch_ops() -> None:
     """Publish ``torch.ops.rwkv.{wkv_forward,mm8_one,mm8_three}`` with the
     reference's schemas (wrapper.cpp:131-141: TORCH_LIBRARY(rwkv, m)).  Their calls run in csrc/rwkv_torch.cpp; what does not
-    fit there comes back to the functions above."""
+    fit there comes back to the functions above, and all calls do where it is not built."""
     global _registered
     if _registered:
         return
-    N.host().register_ops()
+    host = N.host()
+    if host is not None:
+        host.register_ops(_SCHEMAS)
+    else:
+        lib = torch.library.Library("rwkv", "DEF")
+        for schema in _SCHEMAS:
+            lib.define(schema)
+        for fn in (wkv_forward, mm8_one, mm8_three):
+            lib.impl(fn.__name__, fn, "CUDA")
+        register_torch_ops._lib = lib     # keep alive
     _registered = True
 
 
@@ -252,7 +268,8 @@ def mm8_packed(x: torch.Tensor, packed: torch.Tensor, n_in: int, n_out: int,
                r_col: Optional[torch.Tensor] = None, m_col: Optional[torch.Tensor] = None,
                out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``y[B, out]`` float64 for ``x[B, in]`` float32, B in {1, 2, 4, 8}."""
-    y = N.host().mm8_packed(x, packed, n_in, n_out, r_row, m_row, r_col, m_col, out)
+    host = N.host()
+    y = host and host.mm8_packed(x, packed, n_in, n_out, r_row, m_row, r_col, m_col, out)
     if y is not None:
         return y
     L = N.lib()
@@ -270,7 +287,8 @@ def mm8_m16(x: torch.Tensor, packed16: torch.Tensor, n_in: int, n_out: int,
             out: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``mm8_packed`` on the matrix cores: ``y[B, out]`` float64 for ``x[B, in]`` float32, any B in 1..8, weights in
     the M16 layout (``pack_m16``); exact integer sums instead of float32 accumulation."""
-    y = N.host().mm8_m16(x, packed16, n_in, n_out, r_row, m_row, r_col, m_col, out, workspace)
+    host = N.host()
+    y = host and host.mm8_m16(x, packed16, n_in, n_out, r_row, m_row, r_col, m_col, out, workspace)
     if y is not None:
         return y
     L = N.lib()
@@ -307,7 +325,8 @@ def gemm8(x: torch.Tensor, packed16: torch.Tensor, rng: torch.Tensor, off: torch
 
 def wkv_f32(w, u, k, v, aa, bb, pp) -> torch.Tensor:
     """Max-shifted float32 WKV; ``k, v`` are ``[B, T, C]``; state ``[B, C]`` updated in place."""
-    y = N.host().wkv_f32(w, u, k, v, aa, bb, pp)
+    host = N.host()
+    y = host and host.wkv_f32(w, u, k, v, aa, bb, pp)
     if y is not None:
         return y
     for name, t in (("w", w), ("u", u), ("k", k), ("v", v), ("aa", aa), ("bb", bb), ("pp", pp)):
