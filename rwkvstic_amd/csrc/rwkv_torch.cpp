@@ -9,6 +9,7 @@
 // arguments are: what the library reports is raised here, since it may report an error after it has launched (one that an
 // earlier HIP call of the thread left behind), and the operators write in place: a second call would add y twice.
 #include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
@@ -66,6 +67,10 @@ void check(int code) {
     pybind11::module_::import("rwkvstic_amd._native").attr("check")(code);
 }
 
+// The launch goes to a stream of the current device, and scratch from the allocator belongs to one of its tensor's: only if they
+// are the same device may it be handed out again after the call.
+bool here(const at::Tensor &t) { return t.is_cuda() && t.get_device() == c10::hip::current_device(); }
+
 at::Tensor bytes(size_t n, const at::Tensor &like) {
     return at::empty({static_cast<int64_t>(n > 0 ? n : 1)}, like.options().dtype(at::kByte));
 }
@@ -90,7 +95,7 @@ void in_python(const char *name, A &&...args) {
 
 bool try_one(int64_t N, int64_t M, const at::Tensor &x, const at::Tensor &w, const at::Tensor &y, const at::Tensor &r) {
     const auto dt = x.scalar_type();
-    if ((dt != at::kFloat && dt != at::kDouble) || recording()) return false;
+    if ((dt != at::kFloat && dt != at::kDouble) || !here(x) || recording()) return false;
     if (!vec(x, dt) || !vec(y, dt) || !vec(r, dt) || !codes(w, N, M)) return false;
     if (N <= 0 || M <= 0 || x.numel() < N || r.numel() < N || y.numel() < M) return false;
     if (dt == at::kFloat) {
@@ -110,7 +115,7 @@ void mm8_one(int64_t N, int64_t M, at::Tensor &x, at::Tensor &w, at::Tensor &y, 
 using T3 = const at::Tensor *const (&)[3];
 bool try_three(int64_t N, int64_t M, T3 x, T3 w, T3 y, T3 r) {
     const auto dt = x[0]->scalar_type();
-    if ((dt != at::kFloat && dt != at::kDouble) || N <= 0 || M <= 0 || recording()) return false;
+    if ((dt != at::kFloat && dt != at::kDouble) || N <= 0 || M <= 0 || !here(*x[0]) || recording()) return false;
     for (int i = 0; i < 3; ++i) {
         if (!vec(*x[i], dt) || !vec(*y[i], dt) || !vec(*r[i], dt) || !codes(*w[i], N, M)) return false;
         if (x[i]->numel() < N || r[i]->numel() < N || y[i]->numel() < M) return false;
