@@ -1843,22 +1843,16 @@ static VecShape vec_shape(int64_t tiles, int64_t KB, int MT) {
     if (each < v.u) v.u = each <= 1 ? 1 : each == 2 ? 2 : each == 3 ? 3 : v.u;
     return v;
 }
-static void launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
-    const int64_t tiles = g.NT2 > 0 ? (int64_t)g.NT + g.NT2 : (int64_t)g.NT * g.gz;
-    const VecShape v = vec_shape(tiles, g.KB, g.MT);
-    const dim3 grid((unsigned)(g.NT2 > 0 ? ceil_div(g.NT, v.ntw) + ceil_div(g.NT2, v.ntw) : ceil_div(g.NT, v.ntw) * g.gz)), block((unsigned)(64 * v.nw));
-#define RWKV_VEC_LAUNCH(MT, NTW, NW, U, ROUNDS)                                                                               \
-        if (stream) hipLaunchKernelGGL((gemv16_kernel<MT, NTW, NW, U, true, ROUNDS>), grid, block, 0, st, g);                 \
-        else hipLaunchKernelGGL((gemv16_kernel<MT, NTW, NW, U, false, ROUNDS>), grid, block, 0, st, g)
+// The kernel of that shape; null where there is none.  (More than one round only with the most blocks in flight.)
+using VecKernel = void (*)(const GemmArgs);
+static VecKernel vec_kernel(int MT, const VecShape &v, bool rounds, bool stream) {
 #define RWKV_VEC(MT_, LO, HI, NTW, NW, U, ROUNDS)                                                     \
-    if (g.MT >= LO && g.MT <= HI && v.ntw == NTW && v.nw == NW && v.u == U && (g.kb_per_split > NW * U) == ROUNDS) { \
-        RWKV_VEC_LAUNCH(MT_, NTW, NW, U, ROUNDS); return;                                             \
-    }
+    if (MT >= LO && MT <= HI && v.ntw == NTW && v.nw == NW && v.u == U && rounds == ROUNDS)           \
+        return stream ? gemv16_kernel<MT_, NTW, NW, U, true, ROUNDS> : gemv16_kernel<MT_, NTW, NW, U, false, ROUNDS>;
 #define RWKV_VEC12(NTW, NW, U, ROUNDS) RWKV_VEC(1, 1, 1, NTW, NW, U, ROUNDS) RWKV_VEC(2, 2, 2, NTW, NW, U, ROUNDS)
 #define RWKV_VEC34(NTW, NW, U, ROUNDS) RWKV_VEC(3, 3, 3, NTW, NW, U, ROUNDS) RWKV_VEC(4, 4, 4, NTW, NW, U, ROUNDS)
 // (above 16 rows one kernel for two counts of M-tiles: the last one may be a copy)
 #define RWKV_VEC68(NTW, NW, U, ROUNDS) RWKV_VEC(6, 5, 6, NTW, NW, U, ROUNDS) RWKV_VEC(8, 7, 8, NTW, NW, U, ROUNDS)
-    // (more than one round only with the most blocks in flight)
     RWKV_VEC12(4, 8, 1, false)
     RWKV_VEC12(4, 8, 2, false)
     RWKV_VEC12(4, 8, 3, false) RWKV_VEC12(4, 8, 3, true)
@@ -1877,9 +1871,6 @@ static void launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
     RWKV_VEC12(1, 16, 2, false)
     RWKV_VEC12(1, 16, 3, false)
     RWKV_VEC12(1, 16, 5, false) RWKV_VEC12(1, 16, 5, true)
-    RWKV_VEC34(4, 8, 1, false)
-    RWKV_VEC34(4, 8, 2, false)
-    RWKV_VEC34(4, 8, 3, false) RWKV_VEC34(4, 8, 3, true)
     RWKV_VEC34(2, 16, 1, false)
     RWKV_VEC34(2, 16, 2, false)
     RWKV_VEC34(2, 16, 3, false) RWKV_VEC34(2, 16, 3, true)
@@ -1897,10 +1888,27 @@ static void launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
     RWKV_VEC68(1, 16, 1, false)
     RWKV_VEC68(1, 16, 2, false) RWKV_VEC68(1, 16, 2, true)
 #undef RWKV_VEC
-#undef RWKV_VEC_LAUNCH
 #undef RWKV_VEC12
 #undef RWKV_VEC34
 #undef RWKV_VEC68
+    return nullptr;
+}
+// What a launch of so many M-tiles, column tiles and blocks would run; null without a kernel for it, or another kernel's.
+const void *vec_kernel_of(int64_t MT, int64_t tiles, int64_t KB, int64_t kb_per_split) {
+    if (!vec_rows(MT, tiles, KB)) return nullptr;
+    const VecShape v = vec_shape(tiles, KB, (int)MT);
+    return reinterpret_cast<const void *>(vec_kernel((int)MT, v, kb_per_split > v.nw * v.u, false));
+}
+static int launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
+    const int64_t tiles = g.NT2 > 0 ? (int64_t)g.NT + g.NT2 : (int64_t)g.NT * g.gz;
+    const VecShape v = vec_shape(tiles, g.KB, g.MT);
+    const VecKernel kernel = vec_kernel(g.MT, v, g.kb_per_split > v.nw * v.u, stream);
+    if (!kernel)
+        return set_error(RWKV_ERR_SIZE, "gemv16_kernel: no instance for %d M-tiles, %lld column tiles, %d blocks", g.MT, (long long)tiles, g.KB);
+    const dim3 grid((unsigned)(g.NT2 > 0 ? ceil_div(g.NT, v.ntw) + ceil_div(g.NT2, v.ntw) : ceil_div(g.NT, v.ntw) * g.gz)), block((unsigned)(64 * v.nw));
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, g);
+    RWKV_CHECK_LAUNCH("gemv16_kernel");
+    return RWKV_OK;
 }
 
 // Upper bound of the splits plan_products chooses for R rows, N columns and contractions of up to K, whatever the number of
@@ -2068,13 +2076,15 @@ int rows_quant(hipStream_t st, int64_t R, int64_t K, const void *in, bool in_f32
     return RWKV_OK;
 }
 
-static void launch_general(hipStream_t st, GemmArgs &g, bool wide, int gx, bool stream) {
+static int launch_general(hipStream_t st, GemmArgs &g, bool wide, int gx, bool stream) {
     g.gx = gx; g.gy = (int)ceil_div(g.MT, 16); g.by_rows = g.gy >= kXcds;
     g.per_xcd = ((g.by_rows ? g.gy : gx) + kXcds - 1) / kXcds;
     const dim3 grid((unsigned)(kXcds * g.per_xcd * (g.by_rows ? gx : g.gy) * g.gz));
     if (wide) hipLaunchKernelGGL(gemm8_wide_kernel, grid, dim3(512), 0, st, g);
     else if (stream && g.gy <= kStreamRowBlocks) hipLaunchKernelGGL(gemm8_kernel<true>, grid, dim3(512), 0, st, g);
     else hipLaunchKernelGGL(gemm8_kernel<false>, grid, dim3(512), 0, st, g);
+    RWKV_CHECK_LAUNCH(wide ? "gemm8_wide_kernel" : "gemm8_kernel");
+    return RWKV_OK;
 }
 
 int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, int64_t R, int64_t K, int64_t N, int op,
@@ -2105,8 +2115,8 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     g.part = nullptr;
     if (pl.kind == PLAN_VEC) {
         g.gx = g.NT; g.gy = 1; g.by_rows = 0; g.per_xcd = 0;
-        launch_vec(st, g, p[0].stream);
-        RWKV_CHECK_LAUNCH("gemv16_kernel");
+        const int rc = launch_vec(st, g, p[0].stream);
+        if (rc) return rc;
     } else if (pl.kind == PLAN_SKINNY) {
         g.gx = pl.gx; g.gy = 1; g.by_rows = 0; g.per_xcd = (pl.gx + kXcds - 1) / kXcds;
         const dim3 grid((unsigned)(kXcds * g.per_xcd * g.gz));
@@ -2114,8 +2124,8 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
         else hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
         RWKV_CHECK_LAUNCH("gemm8_skinny_kernel");
     } else {
-        launch_general(st, g, pl.kind == PLAN_WIDE, pl.gx, p[0].stream);
-        RWKV_CHECK_LAUNCH("gemm8_kernel");
+        const int rc = launch_general(st, g, pl.kind == PLAN_WIDE, pl.gx, p[0].stream);
+        if (rc) return rc;
     }
     for (int m = 0; defer && m < n; ++m) defer[m].tot = nullptr;
     if (split == 1) return RWKV_OK;     // the tail was applied in the product's epilogue
@@ -2182,8 +2192,8 @@ int rows_ffn_key_receptance(hipStream_t st, bool sequence, const RowsProduct &k,
         // last bit of it reaches the logits and a seeded sampler's texts)
         if (F > 3072 && !sequence) g.part = reinterpret_cast<double2 *>(tot);       // (16 bytes per row and tile: no more than a slice of totals)
         g.next_range = range; g.next_offset = offset; g.next_qs = out.qs;
-        launch_vec(st, g, k.stream);
-        RWKV_CHECK_LAUNCH("gemv16_kernel");
+        const int rc = launch_vec(st, g, k.stream);
+        if (rc) return rc;
         if (!g.part) return rows_quant(st, R, F, k.out, true, range, offset, out, (double *)tot);
         QuantArgs q;
         q.K = (int)F; q.in = k.out; q.range = range; q.offset = offset; q.dig = out.dig; q.S = out.S; q.qs = out.qs; q.zp = out.zp;
@@ -2195,14 +2205,15 @@ int rows_ffn_key_receptance(hipStream_t st, bool sequence, const RowsProduct &k,
         const dim3 grid((unsigned)(kXcds * g.per_xcd));
         if (k.stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
         else hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
+        RWKV_CHECK_LAUNCH("gemm8_skinny_kernel");
     } else if (pair_general(g.MT, g.NT, g.NT2, g.KB)) {
-        launch_general(st, g, false, (int)(ceil_div(g.NT, kGemmNT) + ceil_div(g.NT2, kGemmNT)), k.stream);
+        const int rc = launch_general(st, g, false, (int)(ceil_div(g.NT, kGemmNT) + ceil_div(g.NT2, kGemmNT)), k.stream);
+        if (rc) return rc;
     } else {
         int rc = rows_products(st, 1, &k, tot, R, C, F, ROW_RELU2, nullptr);
         if (!rc) rc = rows_products(st, 1, &r, tot, R, C, C, ROW_STORE_F32, nullptr);
         if (rc) return rc;
     }
-    RWKV_CHECK_LAUNCH("gemm8_skinny_kernel");
     return rows_quant(st, R, F, k.out, true, range, offset, out, (double *)tot);
 }
 

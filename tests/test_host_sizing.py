@@ -111,3 +111,22 @@ def test_a_pending_product_keeps_its_row_constants_apart(lib):
                 setattr(few.add, field, getattr(out[k], field))
                 assert fn(None, n_mix, 100, 64, False, 64, 16, 16, 16, 16, 16, 320, ptrs, ptrs, C.byref(out), C.byref(few)) == -1
                 assert b"row constants" in lib.rwkv_last_error(), (n_mix, k, field)
+
+
+def test_every_few_row_product_has_its_kernel_and_every_kernel_a_product(lib):
+    """gemv16_kernel: the rules that say which products it takes and in which shape, against the list of its instances."""
+    import re
+    kernel_of = getattr(lib, "_ZN4rwkv13vec_kernel_ofEllll")
+    kernel_of.restype, kernel_of.argtypes = C.c_void_p, [C.c_int64] * 4
+    plan, tot = (C.c_int * 4)(), C.c_size_t()
+    reached = set()
+    for MT in range(1, 9):
+        for tiles in list(range(1, 60)) + [100, 127, 128, 200, 255, 256, 257, 300, 319, 320, 321, 400, 511, 512, 513, 900, 1279, 1280, 1281, 2000, 3143, 5000]:
+            for KB in list(range(1, 130)) + [160, 175, 176, 200, 233, 234, 240, 320, 350, 351, 512, 700, 701, 1023, 1024, 1025, 2048, 2049]:
+                assert lib.rwkv_gemm8_plan(4 * MT, 64 * KB, 16 * tiles, 1, C.byref(plan), C.byref(tot)) == 0
+                kind, _, _, split = plan
+                at = kernel_of(MT, tiles * split, KB, -(-KB // split))
+                assert (kind == 0) == bool(at), (MT, tiles, KB)
+                reached.add(at)
+    source = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rwkvstic_amd", "csrc", "rwkv_rows.hip")).read()
+    assert len(reached - {None}) == 2 * len(re.findall(r"RWKV_VEC(?:12|34|68)\(\d", source))
