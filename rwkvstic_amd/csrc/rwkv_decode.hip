@@ -76,11 +76,9 @@ constexpr int kStatRows = 2;           // XR rows 0-1: sum x of a workgroup's 16
 constexpr int kLnRows = kStatRows + 3 * 3;     // rows of the XR record table
 constexpr int kEarlyDiv = 4;           // gathers start when all but G / kEarlyDiv workgroups have published (measured flat from G/20 to G)
 constexpr int kSlotsPerGroup = 5;      // parked-tile slots a group of 16 channels needs at once (ffn receptance + 4 ffn key tiles)
-// Head column sums a front thread fetches, 16 per head tile of the workgroup: narrow models have few workgroups and so
-// many head tiles each (66 at C = 768 with 50277 tokens), and a part of LDS for the sums; the others park them in half
-// an owner record.
+// Head column sums a front thread fetches, 16 per head tile of the workgroup (where owners have head tiles, see HeadShape); they
+// are parked in half an owner record.
 constexpr int kHeadCsPerThread = 4;
-constexpr int head_cs_lds_bytes(int nb) { return nb <= 12 ? kHeadCsPerThread * 64 * kFrontWaves * 4 : 0; }
 
 // LDS flag words
 enum { FLAG_ARRIVED = 0, FLAG_SCALE = 1, FLAG_ABORT = 2, FLAG_GO = 3, FLAG_COUNT = 4 };   // FLAG_GO: see the reload gate of the generated back-wave program
@@ -914,68 +912,68 @@ __device__ __forceinline__ void front_path(const DArgs &a, signed char *dig, con
         for (int i = fx.tid; i < L * 5 * 16; i += FT) a.state[(size_t)(i >> 4) * C + 16 * wg + (i & 15)] = st_lds[i];
         if (TRACE)
             for (int i = fx.tid; i < L * kTraceStampsPerLayer; i += FT) a.b.trace[(size_t)wg * L * kTraceStampsPerLayer + i] = trace_lds[i];
-        return;
-    }
-    // ========================= head (opt.py:71-73) ==============================
-    const DArgs &ah = arguments_again();
-    const int V = ah.m.V, v_tiles = (V + 15) / 16, head_rounds = (v_tiles + NWG - 1) / NWG;
-    red -= gi * kSlotsPerGroup * BW * 16;                 // the head's parked tiles belong to the workgroup
-    const u64 *rec_h = own_lds + (L & 1) * kOrSlots;
-    // column sums of the workgroup's head tiles: requested now, parked in LDS (where there is no
-    // room of their own, in the half that held the last layer's record) once the wait for x is over (a load inside the loop below would cost a
-    // round trip through the busy memory pipeline in every round)
-    constexpr int HCS = kHeadCsPerThread;
-    int *csh = reinterpret_cast<int *>(own_lds + (head_cs_lds_bytes(NB) ? 2 : (L + 1) & 1) * kOrSlots);
-    int csv[HCS];
+    } else {
+        // ========================= head (opt.py:71-73) ==============================
+        const DArgs &ah = arguments_again();
+        const int V = ah.m.V, v_tiles = (V + 15) / 16, head_rounds = (v_tiles + NWG - 1) / NWG;
+        red -= gi * kSlotsPerGroup * BW * 16;                 // the head's parked tiles belong to the workgroup
+        const u64 *rec_h = own_lds + (L & 1) * kOrSlots;
+        // column sums of the workgroup's head tiles: requested now, parked in LDS (in the half that held the last layer's
+        // record) once the wait for x is over (a load inside the loop below would cost a round trip through the busy
+        // memory pipeline in every round)
+        constexpr int HCS = kHeadCsPerThread;
+        int *csh = reinterpret_cast<int *>(own_lds + ((L + 1) & 1) * kOrSlots);
+        int csv[HCS];
 #pragma unroll
-    for (int k = 0; k < HCS; ++k) {
-        const int i = fx.tid + FT * k, v = 16 * (wg + NWG * (i >> 4)) + (i & 15);
-        csv[k] = (i < head_rounds * 16 && v < V) ? ah.m.cs_head[v] : 0;
-    }
-    if (fx.ok)
-        ln_front<NB, FW, 1>(fx, seq, ah, ah.m.P32 + (size_t)L * kLnMats * C, ah.m.Q32 + (size_t)L * kLnMats * C, rec_h, 0,
-                            ah.epoch0 + 4u * (unsigned)L, dig, stat, nullptr, nullptr);
-    if (!fx.ok) return;     // every wave leaves after the same barrier: the flag is tested after each one that follows a wait
+        for (int k = 0; k < HCS; ++k) {
+            const int i = fx.tid + FT * k, v = 16 * (wg + NWG * (i >> 4)) + (i & 15);
+            csv[k] = (i < head_rounds * 16 && v < V) ? ah.m.cs_head[v] : 0;
+        }
+        if (fx.ok)
+            ln_front<NB, FW, 1>(fx, seq, ah, ah.m.P32 + (size_t)L * kLnMats * C, ah.m.Q32 + (size_t)L * kLnMats * C, rec_h, 0,
+                                ah.epoch0 + 4u * (unsigned)L, dig, stat, nullptr, nullptr);
+        if (!fx.ok) return;     // every wave leaves after the same barrier: the flag is tested after each one that follows a wait
 #pragma unroll
-    for (int k = 0; k < HCS; ++k)
-        if (fx.tid + FT * k < head_rounds * 16) csh[fx.tid + FT * k] = csv[k];
-    RWKV_IDS();
+        for (int k = 0; k < HCS; ++k)
+            if (fx.tid + FT * k < head_rounds * 16) csh[fx.tid + FT * k] = csv[k];
+        RWKV_IDS();
 #undef RWKV_IDS
-    unsigned par = 0;
-    constexpr int NS = BackOf<NB, FW, HELP>::NS;          // head tiles per barrier round
-    double Sh;
-    float invSh;
-    ln_scale(stat, rec_h, 0, 0, Sh, invSh);
-    const double zph = ln_zp(stat, rec_h, 0, 0);
-    double best = -INFINITY;                               // first maximum of the logits this thread writes
-    int best_i = 0x7fffffff;
-    for (int h0 = 0; h0 < head_rounds; h0 += NS, par ^= 1u) {
-        __syncthreads();                                   // (the first one also orders the csh writes above)
-        const int s = fx.tid >> 4;                         // parked tile of this round
-        if (s < NS && h0 + s < head_rounds) {
-            const int v = 16 * (wg + NWG * (h0 + s)) + n;
-            if (v < V) {
-                const double y = finish_col<BW>(red + par * (NS * BW * 16), s, n, Sh, csh[16 * (h0 + s) + n], zph);
-                ah.logits[v] = y;
-                if (y > best) { best = y; best_i = v; }    // v grows with the round: an equal later value does not replace
+        unsigned par = 0;
+        constexpr int NS = BackOf<NB, FW, HELP>::NS;          // head tiles per barrier round
+        double Sh;
+        float invSh;
+        ln_scale(stat, rec_h, 0, 0, Sh, invSh);
+        const double zph = ln_zp(stat, rec_h, 0, 0);
+        double best = -INFINITY;                               // first maximum of the logits this thread writes
+        int best_i = 0x7fffffff;
+        for (int h0 = 0; h0 < head_rounds; h0 += NS, par ^= 1u) {
+            __syncthreads();                                   // (the first one also orders the csh writes above)
+            const int s = fx.tid >> 4;                         // parked tile of this round
+            if (s < NS && h0 + s < head_rounds) {
+                const int v = 16 * (wg + NWG * (h0 + s)) + n;
+                if (v < V) {
+                    const double y = finish_col<BW>(red + par * (NS * BW * 16), s, n, Sh, csh[16 * (h0 + s) + n], zph);
+                    ah.logits[v] = y;
+                    if (y > best) { best = y; best_i = v; }    // v grows with the round: an equal later value does not replace
+                }
             }
         }
-    }
-    // the workgroup's candidate for the greedy token: threads 0 .. 16 NS - 1 of wave 0 hold the values
-    if (fx.wave == 0) {
+        // the workgroup's candidate for the greedy token: threads 0 .. 16 NS - 1 of wave 0 hold the values
+        if (fx.wave == 0) {
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            const double ob = __shfl_xor(best, off, 64);
-            const int oi = __shfl_xor(best_i, off, 64);
-            if (ob > best || (ob == best && oi < best_i)) { best = ob; best_i = oi; }
+            for (int off = 32; off >= 1; off >>= 1) {
+                const double ob = __shfl_xor(best, off, 64);
+                const int oi = __shfl_xor(best_i, off, 64);
+                if (ob > best || (ob == best && oi < best_i)) { best = ob; best_i = oi; }
+            }
+            if (fx.lane == 0) { ah.m.amax_val[wg] = best; ah.m.amax_idx[wg] = best_i; }
         }
-        if (fx.lane == 0) { ah.m.amax_val[wg] = best; ah.m.amax_idx[wg] = best_i; }
+        // the state rows of the own channels: st_lds[l][row][n] -> state[l][row][16 g + n]
+        if constexpr (NT == 1)
+            for (int i = fx.tid; i < L * 5 * 16; i += FT) ah.state[(size_t)(i >> 4) * C + 16 * wg + (i & 15)] = st_lds[i];
+        if (TRACE)
+            for (int i = fx.tid; i < L * kTraceStampsPerLayer; i += FT) ah.b.trace[(size_t)wg * L * kTraceStampsPerLayer + i] = trace_lds[i];
     }
-    // the state rows of the own channels: st_lds[l][row][n] -> state[l][row][16 g + n]
-    if constexpr (NT == 1)
-        for (int i = fx.tid; i < L * 5 * 16; i += FT) ah.state[(size_t)(i >> 4) * C + 16 * wg + (i & 15)] = st_lds[i];
-    if (TRACE)
-        for (int i = fx.tid; i < L * kTraceStampsPerLayer; i += FT) ah.b.trace[(size_t)wg * L * kTraceStampsPerLayer + i] = trace_lds[i];
 }
 
 
@@ -1293,7 +1291,7 @@ struct DecodeLds {
     static constexpr int RED_BYTES = RED_SLOTS * back_waves(NB) * 16 * 16;
     static constexpr int STAT_BYTES = 32 * 8, RF_BYTES = NT * 32 * 8, FLAG_BYTES = FLAG_COUNT * 4;   // RF: gate and residual of the own channels
     static constexpr int OWN_OFFSET = DIG_BYTES + RED_BYTES + STAT_BYTES + RF_BYTES + FLAG_BYTES;
-    static constexpr int STATE_OFFSET = OWN_OFFSET + NT * 2 * kOrSlots * 8 + head_cs_lds_bytes(NB);      // (the head's column sums, if any, follow the records)
+    static constexpr int STATE_OFFSET = OWN_OFFSET + NT * 2 * kOrSlots * 8;
     static __host__ __device__ int state_bytes(int L) { return NT == 1 ? L * 5 * 16 * 8 : 0; }  // the new state rows of the own channels
     // a helper workgroup's stash of weight blocks lies over the owner records and state rows, which it does not have
     static constexpr int STASH_OFFSET = OWN_OFFSET;
@@ -1302,7 +1300,7 @@ struct DecodeLds {
         const int own = STATE_OFFSET + state_bytes(L);
         return (own > STASH_OFFSET + STASH_BYTES ? own : STASH_OFFSET + STASH_BYTES) + (trace ? L * kTraceStampsPerLayer * 8 : 0);
     }
-    static_assert(FW == kFrontWaves && (head_cs_lds_bytes(NB) == 0 || NT == 1), "head column sums");
+    static_assert(FW == kFrontWaves, "head column sums");
     // the generated back-wave program addresses LDS by these offsets
     static_assert(Back::RED == DIG_BYTES, "parked tiles follow the digit planes");
     static_assert(Back::FLAG == DIG_BYTES + RED_BYTES + STAT_BYTES + RF_BYTES + FLAG_ABORT * 4, "abort flag offset");
@@ -1695,11 +1693,11 @@ bool decode_supported(int64_t L, int64_t C, int64_t F, int64_t V) {
     if (L <= 0 || V <= 0 || F != 4 * C) return false;
     // one 16-column tile per workgroup, all workgroups resident: C/16 <= 256 CUs
     if (decode_lds(C, L) == 0) return false;
-    // the column sums of a workgroup's head tiles are staged in LDS by its front threads
-    const int nb = (int)(C / 64);
+    // the column sums of an owner's head tiles are fetched by its front threads and parked in half an owner record.  Head
+    // workgroups have no such limit; models of up to 768 channels, whose owners had room of their own, keep it where it was all
+    // the same (65536 and 98304 tokens): larger vocabularies stay with the many-row kernels, and with the last bits of theirs.
     const int64_t NWG = decode_workgroups(C), head_rounds = ((V + 15) / 16 + NWG - 1) / NWG;
-    return head_rounds * 16 <= kHeadCsPerThread * 64 * kFrontWaves &&
-           head_rounds * 16 * (int64_t)sizeof(int) <= (head_cs_lds_bytes(nb) ? head_cs_lds_bytes(nb) : kOrSlots * 8) &&
+    return head_rounds * 16 <= kHeadCsPerThread * 64 * kFrontWaves && (C <= 768 || head_rounds * 16 * (int64_t)sizeof(int) <= kOrSlots * 8) &&
            decode_lds(C, L) <= 160 * 1024;
 }
 

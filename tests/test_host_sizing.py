@@ -130,3 +130,13 @@ def test_every_few_row_product_has_its_kernel_and_every_kernel_a_product(lib):
                 reached.add(at)
     source = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rwkvstic_amd", "csrc", "rwkv_rows.hip")).read()
     assert len(reached - {None}) == 2 * len(re.findall(r"RWKV_VEC(?:12|34|68)\(\d", source))
+
+
+@pytest.mark.parametrize("C_,layers,vocab", [(512, 208, 65536), (768, 201, 98304), (1024, 200, 65536), (1536, 177, 98304), (2048, 174, 131072),
+                                             (2560, 161, 163840), (4096, 123, 262144), (5120, 1000, 163840)])
+def test_models_the_token_kernel_takes(lib, C_, layers, vocab):
+    """At least so many layers (their state rows lie in LDS), and vocabularies up to a line that stays: a model on the other
+    side of it would change kernels, and with them the last bits of its logits."""
+    takes = getattr(lib, "_ZN4rwkv16decode_supportedEllll")
+    takes.restype, takes.argtypes = C.c_bool, [C.c_int64] * 4
+    assert takes(layers, C_, 4 * C_, vocab) and not takes(2, C_, 4 * C_, vocab + 1) and not takes(2, C_, 4 * C_ + 64, vocab)
