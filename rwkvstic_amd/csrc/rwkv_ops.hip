@@ -601,9 +601,11 @@ static bool wkv_f64_scanned(int64_t channels, int64_t T) {
 
 // Channels per workgroup (CW).  A thread's chain is the same for each, so the fewest that leave no compute unit with two
 // workgroups; with more, 16, whose rounds are shorter, but for the few more that 256 workgroups of 32 still take in one.  Us with
-// 32 / 16 / 8, 256 steps: 512 channels (of all sequences) 13.9 / 9.0 / 7.1, 2048 14.3 / 9.7 / 7.8, 3072 14.5 / 10.0 / 10.7, 4096
-// 15.0 / 10.2 / 12.1, 4600 15.5 / 16.2 / 15.3, 8192 18.0 / 17.6 / 20.3, 9216 29.6 / 23.3 / 22.8, 40960 77.9 / 66.7 / 74.2; up to 64
-// steps they are equal or 32 is the fastest.
+// 32 / 16 / 8, 256 steps: 512 channels (of all sequences) 13.9 / 9.0 / 7.1, 2048 14.3 / 9.7 / 7.8, 3072 13.8 / 9.1 / 9.9, 4096
+// 14.2 / 9.4 / 11.5, 4600 14.6 / 15.2 / 14.5, 5144 15.0 / 15.9 / 14.8, 6144 15.1 / 15.3 / 16.2, 8192 17.0 / 16.8 / 19.4, 9216 28.5 / 22.4 /
+// 22.0, 40960 77.9 / 66.7 / 74.2; up to 64 steps they are equal or 32 is the fastest.  (From 4097 to 8192 channels 32 is within
+// 2 % of the fastest up to 256 steps; with 1024, up to 6144 channels, 8 is 5 to 17 % ahead: 4104 49.6 / 49.5 / 41.3, 5120 50.1 / 50.8 /
+// 46.5, but 7168 52.2 / 50.9 / 58.8.)
 static int wkv_f64_scan_width(int64_t channels, int64_t T) {
     if (T <= 8 * kW64SB) return 32;
     return channels <= 256 * 8 ? 8 : channels > 256 * 16 && channels <= 256 * 32 ? 32 : 16;

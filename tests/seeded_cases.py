@@ -34,6 +34,33 @@ def draws():
     return out
 
 
+def edge_draws():
+    """Tokens chosen by the typical sampler from distributions of other shapes, vocabularies on both sides of the 8192 from
+    which logits are loaded in pairs, and cuts from a few tokens to all of them.  (Recorded from the sampler that
+    searched the cut bit by bit in passes over all tokens.)"""
+    from rwkvstic_amd import ops
+    out = {}
+    for V in (300, 8191, 8192, 8193, 20001, 50277, 53247, 53248):
+        for shape in ("normal", "zipf", "peaked", "masked", "equal"):
+            x = torch.randn(V, generator=torch.Generator().manual_seed(V), dtype=torch.float64) * 1.5
+            if shape == "zipf":
+                x = -1.3 * torch.log(torch.arange(1, V + 1, dtype=torch.float64))
+            elif shape == "peaked":
+                x[V - 1] += 14.0
+                x[3] += 16.0
+            elif shape == "masked":
+                x[: V // 2] = -float("inf")
+            elif shape == "equal":
+                x = x * 0 + 0.25
+            logits = x.cuda()
+            for tau, temp in ((0.2, 1.0), (0.8, 1.0), (0.95, 0.7), (0.99999, 1.3), (1.0, 1.0), (1.5, 1.0)):
+                toks = torch.empty(24, dtype=torch.int64, device="cuda")
+                for k in range(24):
+                    ops.sample_token(logits, temp=temp, tau=tau, seed=V, counter=k, out=toks[k:k + 1])
+                out[f"{V} {shape} {tau} {temp}"] = _digest(toks)
+    return out
+
+
 def _models():
     """Models made of random codes, so that no quantiser has a part in them: (name, model)."""
     from rwkvstic_amd.model import HipRWKV

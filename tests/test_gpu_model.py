@@ -681,6 +681,40 @@ def test_token_steps_of_any_vocabulary_match_the_many_row_path(C, V):
     m.check()
 
 
+def test_two_narrow_models_generate_at_once():
+    """Two token kernels of 192 workgroups, more than the device has compute units for, from two threads and streams: the owners,
+    who wait for each other, are dispatched first and wait for no head workgroup, so both come to their ends."""
+    import threading
+    from rwkvstic_amd.model import HipRWKV
+    models = [HipRWKV(synth.iter_tensors(3, C, 4 * C, 20011, seed=C, device="cuda", ln="random")) for C in (768, 1024)]
+    n, times = 48, 4
+    want = [m.decode_greedy(7, n, m.emptyState.clone()) for m in models]
+    torch.cuda.synchronize()
+    got, errors = [[], []], []
+
+    def generate(i):
+        try:
+            m = models[i]
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(times):
+                    got[i].append(m.decode_greedy(7, n, m.emptyState.clone()))
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=generate, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for i, m in enumerate(models):
+        m.check()
+        _say(f"two models at once: model {i}")
+        assert len(got[i]) == times and all(torch.equal(a, b) for g in got[i] for a, b in zip(want[i], g))
+
+
 @pytest.mark.parametrize("C,L", [(1024, 2), (2560, 1), (5120, 1)])
 def test_a_token_step_that_never_gets_its_input_drains_and_is_reported(C, L):
     """The failure path of the persistent kernel, forced from the host without anything that could hang: a token

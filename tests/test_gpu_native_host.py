@@ -127,3 +127,44 @@ def test_other_threads_run_while_a_launch_waits(ops):
             t.join()
         print(f"{entry}: {took:.3f} s, {ran} rounds of another thread", flush=True)
         assert took >= ms * 1e-3 and ran >= 50, entry
+
+
+def test_products_of_two_threads_on_two_streams(ops):
+    """Each call has scratch of its own: threads that multiply at the same time, with products of several workgroup rows whose
+    partial sums go through it, get what each gets alone."""
+    import threading
+    g = torch.Generator(device="cuda").manual_seed(8)
+    work = []
+    for n_in, n_out, dt in ((4096, 1024, torch.float32), (2560, 1536, torch.float64)):
+        x, r = torch.randn(n_in, generator=g, device="cuda").to(dt), torch.rand(n_in, generator=g, device="cuda").to(dt)
+        work.append((n_in, n_out, x, torch.randint(0, 256, (n_in, n_out), generator=g, device="cuda", dtype=torch.uint8), torch.zeros(n_out, device="cuda", dtype=dt), r))
+
+    def run(n_in, n_out, x, w, y, r):
+        three = [torch.zeros_like(y) for _ in range(3)]
+        for _ in range(100):
+            torch.ops.rwkv.mm8_one(n_in, n_out, x, w, y, r)
+            torch.ops.rwkv.mm8_three(n_in, n_out, x, x, x, w, w, w, *three, r, r, r)
+        return [y, *three]
+
+    want = [[t.clone() for t in run(*a)] for a in work]
+    for a in work:
+        a[4].zero_()
+    torch.cuda.synchronize()
+    got, errors = [None, None], []
+
+    def thread(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                got[i] = run(*work[i])
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=thread, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for i in range(2):
+        assert all(torch.equal(a, b) for a, b in zip(want[i], got[i])), i

@@ -9,7 +9,7 @@ import seeded_cases
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("name", ["draws", "steps", "prompts", "replies"])
+@pytest.mark.parametrize("name", ["draws", "edge_draws", "steps", "prompts", "replies"])
 def test_seeded_values_stay(name):
     with open(seeded_cases.GOLDEN) as f:
         want = json.load(f)[name]
