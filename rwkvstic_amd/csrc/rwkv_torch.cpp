@@ -9,7 +9,6 @@
 // arguments are: what the library reports is raised here, since it may report an error after it has launched (one that an
 // earlier HIP call of the thread left behind), and the operators write in place: a second call would add y twice.
 #include <ATen/ATen.h>
-#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
@@ -51,12 +50,14 @@ void bind(const std::map<std::string, uintptr_t> &at) {
 #undef BIND
 }
 
-rwkv_stream_t stream() { return reinterpret_cast<rwkv_stream_t>(c10::hip::getCurrentHIPStream().stream()); }
+using Stream = c10::hip::HIPStream;
+Stream current() { return c10::hip::getCurrentHIPStream(); }
+rwkv_stream_t handle(const Stream &st) { return reinterpret_cast<rwkv_stream_t>(st.stream()); }
 
 // A recorded call keeps its scratch for as long as it is replayed: the buffer the Python side holds on to.
-bool recording() {
+bool recording(const Stream &st) {
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream().stream(), &s) != hipSuccess) { (void)hipGetLastError(); return true; }
+    if (hipStreamIsCapturing(st.stream(), &s) != hipSuccess) { (void)hipGetLastError(); return true; }
     return s != hipStreamCaptureStatusNone;
 }
 
@@ -67,9 +68,9 @@ void check(int code) {
     pybind11::module_::import("rwkvstic_amd._native").attr("check")(code);
 }
 
-// The launch goes to a stream of the current device, and scratch from the allocator belongs to one of its tensor's: only if they
-// are the same device may it be handed out again after the call.
-bool here(const at::Tensor &t) { return t.is_cuda() && t.get_device() == c10::hip::current_device(); }
+// Whether a call on this stream may take scratch from the allocator: that belongs to x's device, and only where the stream does too may
+// it be handed out again after the call.
+bool scratch_fits(const Stream &st, const at::Tensor &x) { return x.is_cuda() && x.get_device() == st.device_index() && !recording(st); }
 
 at::Tensor bytes(size_t n, const at::Tensor &like) {
     return at::empty({static_cast<int64_t>(n > 0 ? n : 1)}, like.options().dtype(at::kByte));
@@ -95,15 +96,16 @@ void in_python(const char *name, A &&...args) {
 
 bool try_one(int64_t N, int64_t M, const at::Tensor &x, const at::Tensor &w, const at::Tensor &y, const at::Tensor &r) {
     const auto dt = x.scalar_type();
-    if ((dt != at::kFloat && dt != at::kDouble) || !here(x) || recording()) return false;
+    const Stream st = current();
+    if ((dt != at::kFloat && dt != at::kDouble) || !scratch_fits(st, x)) return false;
     if (!vec(x, dt) || !vec(y, dt) || !vec(r, dt) || !codes(w, N, M)) return false;
     if (N <= 0 || M <= 0 || x.numel() < N || r.numel() < N || y.numel() < M) return false;
     if (dt == at::kFloat) {
         const at::Tensor ws = bytes(lib.mm8_workspace_bytes(N, M, 1), x);
-        check(lib.mm8_one(stream(), N, M, ptr<float>(x), u8(w), w.stride(0), ptr<float>(y), ptr<float>(r), ws.data_ptr(), ws.numel()));
+        check(lib.mm8_one(handle(st), N, M, ptr<float>(x), u8(w), w.stride(0), ptr<float>(y), ptr<float>(r), ws.data_ptr(), ws.numel()));
     } else {
         const at::Tensor ws = bytes(lib.mm8_f64_workspace_bytes(N, M, 1), x);
-        check(lib.mm8_one_f64(stream(), N, M, ptr<double>(x), u8(w), w.stride(0), ptr<double>(y), ptr<double>(r), ws.data_ptr(), ws.numel()));
+        check(lib.mm8_one_f64(handle(st), N, M, ptr<double>(x), u8(w), w.stride(0), ptr<double>(y), ptr<double>(r), ws.data_ptr(), ws.numel()));
     }
     return true;
 }
@@ -115,7 +117,8 @@ void mm8_one(int64_t N, int64_t M, at::Tensor &x, at::Tensor &w, at::Tensor &y, 
 using T3 = const at::Tensor *const (&)[3];
 bool try_three(int64_t N, int64_t M, T3 x, T3 w, T3 y, T3 r) {
     const auto dt = x[0]->scalar_type();
-    if ((dt != at::kFloat && dt != at::kDouble) || N <= 0 || M <= 0 || !here(*x[0]) || recording()) return false;
+    const Stream st = current();
+    if ((dt != at::kFloat && dt != at::kDouble) || N <= 0 || M <= 0 || !scratch_fits(st, *x[0])) return false;
     for (int i = 0; i < 3; ++i) {
         if (!vec(*x[i], dt) || !vec(*y[i], dt) || !vec(*r[i], dt) || !codes(*w[i], N, M)) return false;
         if (x[i]->numel() < N || r[i]->numel() < N || y[i]->numel() < M) return false;
@@ -123,7 +126,7 @@ bool try_three(int64_t N, int64_t M, T3 x, T3 w, T3 y, T3 r) {
     auto call = [&](auto fn, auto bytes_fn, auto zero) {
         using T = decltype(zero);
         const at::Tensor ws = bytes(bytes_fn(N, M, 3), *x[0]);
-        check(fn(stream(), N, M, ptr<T>(*x[0]), ptr<T>(*x[1]), ptr<T>(*x[2]), u8(*w[0]), w[0]->stride(0), u8(*w[1]), w[1]->stride(0),
+        check(fn(handle(st), N, M, ptr<T>(*x[0]), ptr<T>(*x[1]), ptr<T>(*x[2]), u8(*w[0]), w[0]->stride(0), u8(*w[1]), w[1]->stride(0),
                  u8(*w[2]), w[2]->stride(0), ptr<T>(*y[0]), ptr<T>(*y[1]), ptr<T>(*y[2]), ptr<T>(*r[0]), ptr<T>(*r[1]), ptr<T>(*r[2]),
                  ws.data_ptr(), ws.numel()));
     };
@@ -146,7 +149,7 @@ void wkv_forward(int64_t B, int64_t T, int64_t C, at::Tensor &w, at::Tensor &u, 
     for (const at::Tensor *t : {&aa, &bb, &pp}) ok = ok && t->numel() / C >= B;
     for (const at::Tensor *t : {&w, &u}) ok = ok && t->numel() >= C;
     if (!ok) return in_python("wkv_forward", B, T, C, w, u, k, v, y, aa, bb, pp);
-    check(lib.wkv_forward_f64(stream(), B, T, C, ptr<double>(w), ptr<double>(u), ptr<double>(k), ptr<double>(v), ptr<double>(y),
+    check(lib.wkv_forward_f64(handle(current()), B, T, C, ptr<double>(w), ptr<double>(u), ptr<double>(k), ptr<double>(v), ptr<double>(y),
                               ptr<double>(aa), ptr<double>(bb), ptr<double>(pp)));
 }
 
@@ -169,7 +172,7 @@ using Arg = pybind11::handle;
 template <typename F, typename... A>
 void unlocked(F fn, A... args) {
     pybind11::gil_scoped_release gil;
-    check(fn(stream(), args...));
+    check(fn(handle(current()), args...));
 }
 
 const at::Tensor *tensor(Arg a) { return THPVariable_CheckExact(a.ptr()) ? &THPVariable_Unpack(a.ptr()) : nullptr; }
