@@ -37,8 +37,12 @@ def _contig(t: torch.Tensor, name: str) -> None:
 
 
 def _workspace(nbytes: int, device) -> torch.Tensor:
-    """Grow-only per-device scratch for the reference-layout operators."""
-    key = (device.index if device.index is not None else torch.cuda.current_device())
+    """Scratch of one product, from torch's allocator: it belongs to the stream the call runs on, so that calls of other streams
+    have others.  A call that is recorded, or runs on another device than its tensors', takes a buffer kept per device."""
+    here = torch.cuda.current_device()
+    key = device.index if device.index is not None else here
+    if key == here and not torch.cuda.is_current_stream_capturing():
+        return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
     buf = _scratch.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)

@@ -129,32 +129,44 @@ def test_other_threads_run_while_a_launch_waits(ops):
         assert took >= ms * 1e-3 and ran >= 50, entry
 
 
-def test_products_of_two_threads_on_two_streams(ops):
+@pytest.mark.parametrize("native", [True, False])
+def test_products_of_two_threads_on_two_streams(ops, native):
     """Each call has scratch of its own: threads that multiply at the same time, with products of several workgroup rows whose
-    partial sums go through it, get what each gets alone."""
+    partial sums go through it, get what each gets alone; with the native side, and through the Python functions."""
     import threading
     g = torch.Generator(device="cuda").manual_seed(8)
+    fns = torch.ops.rwkv if native else ops
     work = []
     for n_in, n_out, dt in ((4096, 1024, torch.float32), (2560, 1536, torch.float64)):
         x, r = torch.randn(n_in, generator=g, device="cuda").to(dt), torch.rand(n_in, generator=g, device="cuda").to(dt)
-        work.append((n_in, n_out, x, torch.randint(0, 256, (n_in, n_out), generator=g, device="cuda", dtype=torch.uint8), torch.zeros(n_out, device="cuda", dtype=dt), r))
+        codes = torch.randint(0, 256, (n_in, n_out), generator=g, device="cuda", dtype=torch.uint8)
+        rows = torch.randn(24, n_in, generator=g, device="cuda").double()
+        work.append((n_in, n_out, x, codes, torch.zeros(n_out, device="cuda", dtype=dt), r, rows, ops.pack_m16(codes), r.float(), r.double()))
 
-    def run(n_in, n_out, x, w, y, r):
-        three = [torch.zeros_like(y) for _ in range(3)]
+    def run(n_in, n_out, x, w, y, r, rows, w16, rng, off):
+        three, products = [torch.zeros_like(y) for _ in range(3)], []
         for _ in range(100):
-            torch.ops.rwkv.mm8_one(n_in, n_out, x, w, y, r)
-            torch.ops.rwkv.mm8_three(n_in, n_out, x, x, x, w, w, w, *three, r, r, r)
-        return [y, *three]
+            fns.mm8_one(n_in, n_out, x, w, y, r)
+            fns.mm8_three(n_in, n_out, x, x, x, w, w, w, *three, r, r, r)
+            products.append(ops.gemm8(rows, w16, rng, off, n_in, n_out))
+        return [y, *three, *products]
 
     want = [[t.clone() for t in run(*a)] for a in work]
     for a in work:
         a[4].zero_()
     torch.cuda.synchronize()
+    # both streams wait for a long product, so that their calls are queued by then and run at the same time
+    wide = torch.randn(8192, 8192, device="cuda")
+    for _ in range(10):
+        wide = torch.mm(wide, wide)
+    queued = torch.cuda.Event()
+    queued.record()
     got, errors = [None, None], []
 
     def thread(i):
         try:
             with torch.cuda.stream(torch.cuda.Stream()):
+                queued.wait()
                 got[i] = run(*work[i])
                 torch.cuda.current_stream().synchronize()
         except Exception as e:
