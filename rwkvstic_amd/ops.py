@@ -38,16 +38,16 @@ def _contig(t: torch.Tensor, name: str) -> None:
 
 def _workspace(nbytes: int, device) -> torch.Tensor:
     """Scratch of one product, from torch's allocator: it belongs to the stream the call runs on, so that calls of other streams
-    have others.  A call that is recorded, or runs on another device than its tensors', takes a buffer kept per device."""
+    have others.  A call that is recorded, or runs on another device than its tensors', takes a buffer kept per device: it may be
+    replayed at any time, so where a larger one is needed the smaller ones stay (each at least twice the one before)."""
     here = torch.cuda.current_device()
     key = device.index if device.index is not None else here
     if key == here and not torch.cuda.is_current_stream_capturing():
         return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-    buf = _scratch.get(key)
-    if buf is None or buf.numel() < nbytes:
-        buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _scratch[key] = buf
-    return buf
+    kept = _scratch.setdefault(key, [])
+    if not kept or kept[-1].numel() < nbytes:
+        kept.append(torch.empty(max(nbytes, 2 * kept[-1].numel() if kept else 1 << 20), dtype=torch.uint8, device=device))
+    return kept[-1]
 
 
 # ---------------------------------------------------------------- reference operators

@@ -180,3 +180,39 @@ def test_products_of_two_threads_on_two_streams(ops, native):
     assert not errors, errors
     for i in range(2):
         assert all(torch.equal(a, b) for a, b in zip(want[i], got[i])), i
+
+
+def test_scratch_of_a_recorded_product_is_not_given_back(ops):
+    """A graph that holds an operator call writes its scratch whenever it is replayed, also after a larger product has been
+    recorded: nobody else may have been given that memory."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+
+    def product(n_in, n_out):
+        x, r = torch.randn(n_in, generator=g, device="cuda"), torch.rand(n_in, generator=g, device="cuda")
+        w = torch.randint(0, 256, (n_in, n_out), generator=g, device="cuda", dtype=torch.uint8)
+        return n_in, n_out, x, w, torch.zeros(n_out, device="cuda"), r
+
+    def record(a):
+        graph, st = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(graph, stream=st):
+            torch.ops.rwkv.mm8_one(*a)
+        return graph
+
+    def buffers():
+        return [b for kept in ops._scratch.values() for b in (kept if isinstance(kept, list) else [kept])]
+
+    ops._scratch.clear()
+    small, large = product(4096, 1024), product(8192, 16384)
+    want = torch.zeros_like(small[4])
+    torch.ops.rwkv.mm8_one(*small[:4], want, small[5])
+    graphs = [record(small)]
+    at, size = buffers()[0].data_ptr(), buffers()[0].numel()
+    graphs.append(record(large))
+    assert any(b.data_ptr() == at for b in buffers()), "the first recording's scratch was given back"
+    assert len(buffers()) == 2 and max(b.numel() for b in buffers()) >= 2 * size
+    for i in range(3):
+        for a, graph in zip((small, large), graphs):
+            a[4].zero_()
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(small[4], want), f"replay {i}"
