@@ -352,6 +352,7 @@ def sample_token(logits: torch.Tensor, *, greedy: bool = False, temp: float = 1.
     rwkvMaster.py:37); the uniform number is a hash of ``(seed, counter)``."""
     _req(logits, torch.float64, "logits"); _contig(logits, "logits")
     out = out if out is not None else torch.empty(1, dtype=torch.int64, device=logits.device)
+    _buffer(out, torch.int64, 1, "out")
     N.check(N.lib().rwkv_sample_token(_stream(), logits.data_ptr(), logits.numel(), 1 if greedy else 0, float(temp),
                                       float(tau), float(end_adj), int(seed) & (2 ** 64 - 1), int(counter), out.data_ptr()))
     return out
@@ -360,5 +361,6 @@ def sample_token(logits: torch.Tensor, *, greedy: bool = False, temp: float = 1.
 def argmax(logits: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     _req(logits, torch.float64, "logits"); _contig(logits, "logits")
     out = out if out is not None else torch.empty(1, dtype=torch.int64, device=logits.device)
+    _buffer(out, torch.int64, 1, "out")
     N.check(N.lib().rwkv_argmax_f64(_stream(), logits.data_ptr(), logits.numel(), out.data_ptr()))
     return out

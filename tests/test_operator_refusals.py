@@ -69,3 +69,14 @@ def test_matvec_buffers_that_do_not_hold_the_product_are_refused(ops, tensors, l
         ws = {"workspace": a["workspace"]} if layout == "m16" else {}
         with pytest.raises(ValueError):
             (ops.mm8_packed if layout == "packed" else ops.mm8_m16)(a["x"], a["packed"], N_IN, N_OUT, a["r_row"], a["m_row"], a["r_col"], a["m_col"], out=a["out"], **ws)
+
+
+@ON
+@pytest.mark.parametrize("out", [dict(size=(1,), dtype=torch.int64, device="cpu"), dict(size=(1,), dtype=torch.int32, device="cuda"), dict(size=(0,), dtype=torch.int64, device="cuda")])
+def test_tokens_go_nowhere_but_to_a_word_of_the_device(ops, tensors, out):
+    with tensors():
+        logits, out = torch.empty(64, dtype=torch.float64, device="cuda"), torch.empty(**out)
+        for call in (ops.argmax, ops.sample_token):
+            with pytest.raises((ValueError, TypeError)) as e:
+                call(logits, out=out)
+            assert "out" in str(e.value)
