@@ -377,11 +377,12 @@ struct RowPoll {
     }
 };
 
-// Spin on an LDS sequence word written by wave 0.
+// Spin on an LDS sequence word written by wave 0.  (Without a sleep between the looks: 24 layers of 1024 327 -> 322 us a token, at other
+// widths the same.)
 __device__ __forceinline__ void wait_flag(Front &fx, int which, int seq) {
     unsigned spins = 0;
     while (fx.ok && fx.flags[which] < seq) {
-        __builtin_amdgcn_s_sleep(1);
+        __builtin_amdgcn_s_sleep(0);
         if ((++spins & 255u) == 0u && (spins > (fx.spin_limit << 4) || fx.flags[FLAG_ABORT])) fx.fail();
     }
 }
@@ -545,46 +546,45 @@ __device__ __forceinline__ float or_maxP(const u64 *rec, int m) { return reinter
 __device__ __forceinline__ float or_maxQ(const u64 *rec, int m) { return reinterpret_cast<const float *>(rec + kOrScal)[26 + m]; }
 
 // l == L stages the head's scalars only.
+// Everything a wavefront needs is requested before its first wait: with a branch for each kind of slot, and a load and a wait in each, the
+// last wavefront made four trips to memory, which on a compute unit that streams weights are several microseconds and at 2560
+// channels reached the att output phase's barrier.  Us a token before / now, with vec_front's scale and wait_flag as they are
+// now: 12 layers of 512 148.4 / 145.3, of 768 157.4 / 155.3, 24 of 1024 326 / 320.5, 12 of 1536 222.3 / 220.6, 32 of 2560 701.4 / 694.7,
+// 8 of 4096 386.1 / 385.3 (this alone: 2560 701 / 694, narrower ones within 1).
 template <int FT, int PARTS>
 __device__ __forceinline__ void stage_owner_record(const DArgs &a, int l, int g, int G, int C, u64 *dst, int tid) {
     const bool layer = l < a.m.L;
 #pragma unroll
     for (int i = 0; i < kOrSlots / FT; ++i) {
-        const int t = tid + FT * i;
+        const int t = tid + FT * i, first = __builtin_amdgcn_readfirstlane(t);
+        const u64 *own = a.m.ownrec + ((size_t)l * G + g) * kOrSlots;
         u64 v = 0;
-        if (t < kOrStatic) {
-            if (layer) v = a.m.ownrec[((size_t)l * G + g) * kOrSlots + t];
-        } else if (t < kOrScal) {
-            const int k = (t - kOrState) >> 4, n = (t - kOrState) & 15;
-            if (layer) v = (u64)__double_as_longlong(a.state[((size_t)l * 5 + 2 + k) * C + 16 * g + n]);
-        } else if (t < kOrScal + 16) {
-            // slots 0-4 sum PO, 5-9 sum QO, 10-12 max P, 13-15 max Q (float pairs); the per-token
+        if (first + 63 < kOrStatic) {                       // (uniform: most wavefronts copy the static record alone)
+            if (layer) v = gld(own + t);
+        } else {
+            // scalars: slots 0-4 sum PO, 5-9 sum QO, 10-12 max P, 13-15 max Q (float pairs); the per-token
             // ones of a layer are the combination, in a fixed order, of its parts
-            const int sidx = t - kOrScal;
-            v = reinterpret_cast<const u64 *>(a.m.sc + l)[sidx];
-            const bool per_token = (sidx >= 5 && sidx < 10) || sidx >= 13;
-            if (layer && per_token) {
-                const DScal *sp = a.m.scp + (size_t)l * PARTS;
-                if (sidx < 10) {
-                    double part[PARTS];
+            const int k = (t - kOrState) >> 4, n = (t - kOrState) & 15, sidx = t < kOrScal || t >= kOrScal + 16 ? 0 : t - kOrScal;
+            const u64 *src = reinterpret_cast<const u64 *>(a.m.sc + l) + sidx;
+            if (layer && t < kOrStatic) src = own + t;
+            else if (layer && t < kOrScal) src = reinterpret_cast<const u64 *>(a.state) + ((size_t)l * 5 + 2 + k) * C + 16 * g + n;
+            v = gld(src);
+            if (layer && first + 63 >= kOrScal) {           // (uniform)
+                u64 part[PARTS];
 #pragma unroll
-                    for (int q = 0; q < PARTS; ++q) part[q] = sp[q].sumQO[sidx - 5];     // independent loads
-                    double acc = 0.0;
+                for (int q = 0; q < PARTS; ++q) part[q] = gld(reinterpret_cast<const u64 *>(a.m.scp + (size_t)l * PARTS + q) + sidx);
+                double acc = 0.0;
+                float lo = 0.f, hi = 0.f;
 #pragma unroll
-                    for (int q = 0; q < PARTS; ++q) acc += part[q];
-                    v = (u64)__double_as_longlong(acc);
-                } else {
-                    const int i0 = 2 * (sidx - 13), i1 = i0 + 1 < kLnMats ? i0 + 1 : i0;
-                    float plo[PARTS], phi[PARTS];
-#pragma unroll
-                    for (int q = 0; q < PARTS; ++q) { plo[q] = sp[q].maxQ[i0]; phi[q] = sp[q].maxQ[i1]; }
-                    float lo = 0.f, hi = 0.f;
-#pragma unroll
-                    for (int q = 0; q < PARTS; ++q) { lo = fmaxf(lo, plo[q]); hi = fmaxf(hi, phi[q]); }
-                    if (i0 + 1 >= kLnMats) hi = 0.f;
-                    v = ((u64)__float_as_uint(hi) << 32) | (u64)__float_as_uint(lo);
+                for (int q = 0; q < PARTS; ++q) {
+                    acc += __longlong_as_double((long long)part[q]);
+                    lo = fmaxf(lo, __uint_as_float((unsigned)part[q])); hi = fmaxf(hi, __uint_as_float((unsigned)(part[q] >> 32)));
                 }
+                static_assert(kLnMats == 5, "slot 15: max Q of product 4, and padding");
+                if (sidx >= 5 && sidx < 10) v = (u64)__double_as_longlong(acc);
+                if (sidx >= 13) v = ((u64)(sidx == 15 ? 0u : __float_as_uint(hi)) << 32) | (u64)__float_as_uint(lo);
             }
+            if (t >= kOrScal + 16 || (!layer && t < kOrScal)) v = 0;
         }
         dst[t] = v;
     }
@@ -708,10 +708,13 @@ __device__ __forceinline__ void vec_front(Front &fx, int &seq, const u64 *src, c
         if (fx.lane == 0) fx.flags[FLAG_GO] = seq;
         if (tp && fx.tid == 0) tp[0] = wall_clock64();
         const float mx = wave_max_dpp(r.lane_max(fx, 0));
-        const double so = wave_sum_dpp(r.lane_sum(fx, 1) + r.lane_sum(fx, 2));
         double S;
         scale_from_amax(mx, S, invS);
-        if (fx.lane == 0) { stat[16] = S; stat[17] = so; stat[18] = (double)invS; fx.flags[FLAG_SCALE] = seq; }
+        if (fx.lane == 0) { stat[16] = S; stat[18] = (double)invS; fx.flags[FLAG_SCALE] = seq; }
+        // (the other wavefronts wait for the scale alone; the zero-point sum is the epilogue's, behind the next barrier)
+        asm volatile("" ::: "memory");
+        const double so = wave_sum_dpp(r.lane_sum(fx, 1) + r.lane_sum(fx, 2));
+        if (fx.lane == 0) stat[17] = so;
     } else {
         wait_flag(fx, FLAG_ARRIVED, seq);
         issue_quads<FT, CH>(st, fx.tid, 0, nq, w[0]);
