@@ -720,14 +720,19 @@ argmax_f64_kernel(const double *__restrict__ logits, int V, int64_t *__restrict_
 // ---------------------------------------------------------------------------
 // Reference layout w[n_in][n_out] (row stride w_stride), operators32.cu:18-83: y[k] += sum_j w[j][k] * (x[j] r[j]).
 //
-// Bound: memory (n_in x n_out bytes, once), in practice one round of loads and a second launch.  A workgroup takes 128
-// columns (whole cache lines of the rows) and up to 256 rows; a lane requests 16 bytes of each of its up to eight rows
-// before the first is used.  One compute unit draws only some 40 bytes per nanosecond, so the rows are cut until the
-// grid covers the device; the slices are added in order by mm8_ref_reduce_kernel (deterministic).  The two
-// launches of [2560 x 2560] take 7.2 + 3.5 us, of [2560 x 10240] and [10240 x 2560] 13.8 + 3.5 us (26 MB at copy rate:
-// 5.5); with 4-byte loads, one row after the other, and a reduction of one thread per column the three averaged
-// 14.3 + 9.1 us.  64 columns and all 2560 rows to a workgroup, which needs no second launch: 16 us on average.
-// Non-temporal loads and row slices dealt out to the XCDs change nothing.
+// Bound: memory (n_in x n_out bytes, once), in practice one round of loads and a second launch.  Slices of rows are cut until
+// the grid covers the device, and added in order by mm8_ref_reduce_kernel (deterministic).
+//
+// float32, 16 columns and more (mm8_ref_rows_kernel): 1024 columns and 128 rows to a workgroup.  Every wavefront reads whole rows of
+// its own, 16 bytes to a lane, eight of them requested before the first is used, so that a lane keeps its columns and nothing is
+// exchanged between lanes; the 16 wavefronts' sums meet in LDS.  Us for both launches, by the other kernel / by this: 768 x 768 7.6 / 6.6,
+// 2560 x 2560 10.2 / 8.6, three of them 16.8 / 11.1, 2560 x 10240 17.0 / 12.3, 10240 x 2560 17.0 / 12.6, 5120 x 5120 17.8 / 11.7, 5120 x 20480
+// 36.6 / 26.0, 768 x 50277 21.0 / 17.8 (26 MB at copy rate: 5.5).  512 columns: 8.9 for 2560 x 2560, 14.2 for the 26 MB shapes; 256 rows,
+// 16 of them in flight, 10.4 and 13.7.  Whole contractions of 16, 32 or 64 columns, one launch: 13.1, 19.9 and 32.7 at best.
+//
+// The others (mm8_ref_kernel): 128 columns (whole cache lines of the rows) and up to 256 rows, eight lanes to a row, sums
+// exchanged between the lanes of a column.  float64 stays here: its conversions and sums bind a compute unit, and this
+// spreads them over more of them (768 x 768 7.4 us, by the other kernel 8.7; 512 x 2048 7.2, 9.1).
 // ---------------------------------------------------------------------------
 constexpr int kRefSplitRows = 128;      // rows per slice the workspace is sized for
 constexpr int kRefThreads = 256, kRefRowsPass = kRefThreads / 8, kRefPasses = 8;
@@ -744,6 +749,74 @@ struct Mm8RefArgs {
 
 // T: float (operators32.cu) or double (operators.cu:58-80, the dispatch of wrapper.cpp:60-77): the type of x, r, y and
 // of the sums.  WIDE: at least 16 columns; narrower matrices are read byte by byte.  LONG: more than 256 rows to a workgroup.
+typedef uint32_t RefPiece __attribute__((ext_vector_type(4), aligned(1)));     // 16 columns (rows may start anywhere)
+template <typename T>
+__device__ __forceinline__ void ref_piece(const RefPiece &w, T xr, T (&acc)[16]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t d = w[i];
+        acc[4 * i] = fma((T)ubyte0(d), xr, acc[4 * i]);
+        acc[4 * i + 1] = fma((T)ubyte1(d), xr, acc[4 * i + 1]);
+        acc[4 * i + 2] = fma((T)ubyte2(d), xr, acc[4 * i + 2]);
+        acc[4 * i + 3] = fma((T)ubyte3(d), xr, acc[4 * i + 3]);
+    }
+}
+
+constexpr int kRefRowsThreads = 1024, kRefRowsWaves = kRefRowsThreads / 64, kRefRowsCols = 1024;
+__global__ void __launch_bounds__(kRefRowsThreads) mm8_ref_rows_kernel(const Mm8RefArgs<float> a) {
+    constexpr int kRound = kRefRowsWaves * kRefPasses, kPitch = 65;
+    static_assert(kRound == kRefSplitRows, "a slice is one round");
+    __shared__ float xs[kRound];
+    __shared__ float red[kRefRowsWaves / 2][16 * kPitch];      // [wavefront][column of a lane's 16][lane]
+    const int m = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const float *x = m == 0 ? a.x[0] : m == 1 ? a.x[1] : a.x[2], *r = m == 0 ? a.r[0] : m == 1 ? a.r[1] : a.r[2];
+    const uint8_t *w = m == 0 ? a.w[0] : m == 1 ? a.w[1] : a.w[2];
+    const int64_t stride = m == 0 ? a.stride[0] : m == 1 ? a.stride[1] : a.stride[2];
+    const int j_end = min((int)(blockIdx.y + 1) * a.rows_per_split, a.n_in);
+    // (the last piece of a row: as in mm8_ref_kernel)
+    const int c0 = blockIdx.x * kRefRowsCols, cl = min(c0 + 16 * lane, a.n_out - 16);
+    float acc[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+    for (int j0 = blockIdx.y * a.rows_per_split; j0 < j_end; j0 += kRound) {       // (more than once only where a grid has too few slices)
+        const int rows = min(kRound, j_end - j0);
+        // x and r are requested ahead of the weights: a wavefront's loads return in order
+        const int jx = j0 + min(tid, rows - 1);
+        float xv = 0.f, rv = 0.f;
+        if (tid < kRound) { xv = x[jx]; rv = r[jx]; }
+        RefPiece wv[kRefPasses];
+#pragma unroll
+        for (int p = 0; p < kRefPasses; ++p) {
+            const int j = wave + p * kRefRowsWaves;
+            if (j >= rows) break;                           // (uniform for the wavefront)
+            wv[p] = *reinterpret_cast<const RefPiece *>(w + (size_t)(j0 + j) * stride + cl);
+        }
+        if (tid < kRound) xs[tid] = xv * rv;                // (as in mm8_ref_kernel)
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < kRefPasses; ++p) {
+            const int j = wave + p * kRefRowsWaves;
+            if (j >= rows) break;
+            ref_piece(wv[p], xs[j], acc);
+        }
+        __syncthreads();                                     // xs has been read
+    }
+    // the upper eight wavefronts' sums are added by the lower ones, then eight sums a column
+    if (wave >= kRefRowsWaves / 2)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) red[wave - kRefRowsWaves / 2][e * kPitch + lane] = acc[e];
+    __syncthreads();
+    if (wave < kRefRowsWaves / 2)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) red[wave][e * kPitch + lane] += acc[e];
+    __syncthreads();
+    const int at = (tid & 15) * kPitch + (tid >> 4);
+    const float sum = ((red[0][at] + red[1][at]) + (red[2][at] + red[3][at])) + ((red[4][at] + red[5][at]) + (red[6][at] + red[7][at]));
+    const int piece = c0 + (tid & ~15), k = min(piece, a.n_out - 16) + (tid & 15);
+    if (k < piece || k >= a.n_out) return;
+    a.scratch[((size_t)blockIdx.y * gridDim.z + m) * a.n_out + k] = sum;
+}
+
 template <typename T, bool WIDE, bool LONG>
 __global__ void __launch_bounds__(kRefThreads) mm8_ref_kernel(const Mm8RefArgs<T> a) {
     __shared__ T xs[kRefPasses * kRefRowsPass];
@@ -758,7 +831,6 @@ __global__ void __launch_bounds__(kRefThreads) mm8_ref_kernel(const Mm8RefArgs<T
     // the last piece of a row that is not a multiple of 16 columns is read 16 bytes from the row's end (its first
     // columns belong to the piece before and are dropped)
     const int cl = WIDE ? min(c0, a.n_out - 16) : 0;
-    typedef uint32_t Piece __attribute__((ext_vector_type(4), aligned(1)));     // (rows may start anywhere)
     T acc[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = (T)0;
@@ -767,19 +839,19 @@ __global__ void __launch_bounds__(kRefThreads) mm8_ref_kernel(const Mm8RefArgs<T
         // x and r are requested ahead of the weights: a wavefront's loads return in order
         const int jx = j0 + min(tid, rows - 1);
         const T xv = x[jx], rv = r[jx];
-        Piece wv[kRefPasses];
+        RefPiece wv[kRefPasses];
 #pragma unroll
         for (int p = 0; p < kRefPasses; ++p) {
             if (p * kRefRowsPass >= rows) break;                            // (uniform)
             const int j = j0 + min(row0 + p * kRefRowsPass, rows - 1);      // past the end: the last row again, times zero
             const uint8_t *row = w + (size_t)j * stride + cl;
-            if (WIDE) wv[p] = *reinterpret_cast<const Piece *>(row);
+            if (WIDE) wv[p] = *reinterpret_cast<const RefPiece *>(row);
             else {
                 uint32_t d[4] = {0, 0, 0, 0};
 #pragma unroll
                 for (int e = 0; e < 15; ++e)
                     if (e < a.n_out) d[e >> 2] |= (uint32_t)row[e] << (8 * (e & 3));
-                wv[p] = Piece{d[0], d[1], d[2], d[3]};
+                wv[p] = RefPiece{d[0], d[1], d[2], d[3]};
             }
         }
         // operators32.cu:33-36 multiplies x[j] * (w * r[j]); here x[j]*r[j] is formed once per row (same rounding as the
@@ -789,15 +861,7 @@ __global__ void __launch_bounds__(kRefThreads) mm8_ref_kernel(const Mm8RefArgs<T
 #pragma unroll
         for (int p = 0; p < kRefPasses; ++p) {
             if (p * kRefRowsPass >= rows) break;
-            const T xr = xs[row0 + p * kRefRowsPass];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t d = wv[p][i];
-                acc[4 * i] = fma((T)ubyte0(d), xr, acc[4 * i]);
-                acc[4 * i + 1] = fma((T)ubyte1(d), xr, acc[4 * i + 1]);
-                acc[4 * i + 2] = fma((T)ubyte2(d), xr, acc[4 * i + 2]);
-                acc[4 * i + 3] = fma((T)ubyte3(d), xr, acc[4 * i + 3]);
-            }
+            ref_piece(wv[p], xs[row0 + p * kRefRowsPass], acc);
         }
         if (!LONG) break;
         __syncthreads();                                     // xs has been read
@@ -863,16 +927,16 @@ static int mm8_ref_launch(hipStream_t st, int nm, int64_t n_in, int64_t n_out,
         return set_error(RWKV_ERR_WORKSPACE, "mm8: workspace of %zu bytes needed, %zu given", need, ws_bytes);
     RWKV_CHECK_ALIGN(ws, sizeof(T));
     a.n_in = (int)n_in; a.n_out = (int)n_out; a.scratch = static_cast<T *>(ws);
-    // 256 rows per workgroup, 128 (the least the workspace allows) where that leaves compute units without one; the number
-    // of matrices does not count, so that mm8_three gives the bits of three mm8_one
-    const int64_t cols = ceil_div(n_out, 128);
+    // 256 rows per workgroup of mm8_ref_kernel, 128 (the least the workspace allows) where that leaves compute units without one; the
+    // number of matrices does not count, so that mm8_three gives the bits of three mm8_one
+    const bool wide = n_out >= 16, rows_whole = wide && sizeof(T) == 4;
+    const int64_t cols = ceil_div(n_out, rows_whole ? kRefRowsCols : 128);
     a.rows_per_split = kRefPasses * kRefRowsPass;
-    if (cols * ceil_div(n_in, a.rows_per_split) < 256) a.rows_per_split = kRefSplitRows;
+    if (rows_whole || cols * ceil_div(n_in, a.rows_per_split) < 256) a.rows_per_split = kRefSplitRows;
     // In float64 the reduction at a workgroup's end is a quarter of its time, so it takes two or four times the rows where enough
     // workgroups are left (us a call with 1, 2, 4 times 256 rows: 2560 x 10240 18.8, 14.4, 13.4, of 240 workgroups the last, and 20.9,
     // 17.4, 18.0 from memory; 2560 x 20480 29.2, 25.2, 21.0, of 480, and 30.4, 27.6, 22.8; 768 x 50277 24.5, 26.2, 21.3, of 393;
     // 5120 x 20480 47.9, 38.0, 35.1).
-    const bool wide = n_out >= 16;
     int64_t more = 1;
     if (sizeof(T) == 8 && wide) more = cols * ceil_div(n_in, 4 * a.rows_per_split) >= 384 ? 4 : cols * ceil_div(n_in, 2 * a.rows_per_split) >= 256 ? 2 : 1;
     a.rows_per_split *= (int)more;
@@ -880,10 +944,16 @@ static int mm8_ref_launch(hipStream_t st, int nm, int64_t n_in, int64_t n_out,
     const bool longer = a.rows_per_split > kRefPasses * kRefRowsPass;
     a.splits = (int)ceil_div(n_in, a.rows_per_split);
     const dim3 grid((unsigned)cols, (unsigned)a.splits, (unsigned)nm);
-    if (longer && wide) hipLaunchKernelGGL((mm8_ref_kernel<T, true, true>), grid, dim3(kRefThreads), 0, st, a);
-    else if (longer) hipLaunchKernelGGL((mm8_ref_kernel<T, false, true>), grid, dim3(kRefThreads), 0, st, a);
-    else if (wide) hipLaunchKernelGGL((mm8_ref_kernel<T, true, false>), grid, dim3(kRefThreads), 0, st, a);
-    else hipLaunchKernelGGL((mm8_ref_kernel<T, false, false>), grid, dim3(kRefThreads), 0, st, a);
+    if constexpr (sizeof(T) == 4) {
+        if (wide) hipLaunchKernelGGL(mm8_ref_rows_kernel, grid, dim3(kRefRowsThreads), 0, st, a);
+        else if (longer) hipLaunchKernelGGL((mm8_ref_kernel<T, false, true>), grid, dim3(kRefThreads), 0, st, a);
+        else hipLaunchKernelGGL((mm8_ref_kernel<T, false, false>), grid, dim3(kRefThreads), 0, st, a);
+    } else {
+        if (longer && wide) hipLaunchKernelGGL((mm8_ref_kernel<T, true, true>), grid, dim3(kRefThreads), 0, st, a);
+        else if (longer) hipLaunchKernelGGL((mm8_ref_kernel<T, false, true>), grid, dim3(kRefThreads), 0, st, a);
+        else if (wide) hipLaunchKernelGGL((mm8_ref_kernel<T, true, false>), grid, dim3(kRefThreads), 0, st, a);
+        else hipLaunchKernelGGL((mm8_ref_kernel<T, false, false>), grid, dim3(kRefThreads), 0, st, a);
+    }
     RWKV_CHECK_LAUNCH("mm8_ref_kernel");
     hipLaunchKernelGGL(mm8_ref_reduce_kernel<T>, dim3((unsigned)ceil_div(n_out, 64), (unsigned)nm), dim3(256), 0, st, a);
     RWKV_CHECK_LAUNCH("mm8_ref_reduce_kernel");

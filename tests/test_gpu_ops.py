@@ -251,6 +251,28 @@ def test_mm8_one_edges_against_the_float64_product(ops, n_in, n_out, pad):
         assert ((y.cpu().double() - want).abs() <= steps * eps * mag).all()
 
 
+# float32 by whole rows: 1024 columns and 128 rows to a workgroup, whole and ragged ones of both, rows that start anywhere, fewer rows
+# than the workgroup has wavefronts, three matrices in a call
+@pytest.mark.parametrize("n_in,n_out,pad", [(1, 1024, 0), (15, 1023, 2), (128, 1025, 0), (129, 1040, 7), (300, 2047, 1), (1000, 16, 3)])
+def test_mm8_by_rows_against_the_float64_product(ops, n_in, n_out, pad):
+    _say(f"mm8 by rows in={n_in} out={n_out} pad={pad}")
+    g = torch.Generator(device="cuda").manual_seed(n_in * 7 + n_out)
+    big = torch.randint(0, 256, (3, n_in, n_out + pad), generator=g, dtype=torch.uint8, device="cuda")
+    x, r = torch.randn(n_in, generator=g, device="cuda"), torch.rand(n_in, generator=g, device="cuda") * 1e-3
+    y0 = torch.randn(n_out, generator=g, device="cuda")
+    z = [y0.clone() for _ in range(3)]
+    w = [big[i, :, :n_out] for i in range(3)]
+    ops.mm8_three(n_in, n_out, x, x, x, *w, *z, r, r, r)
+    for i in range(3):
+        y = y0.clone()
+        ops.mm8_one(n_in, n_out, x, w[i], y, r)
+        assert torch.equal(y, z[i])
+        xr, wd = x.double() * r.double(), w[i].double()
+        # at most 8 products per lane, 4 additions over the wavefronts, the slices, x * r and y
+        steps = 8 + 4 + (n_in + 127) // 128 + 2
+        assert ((y.double() - (y0.double() + xr @ wd)).abs() <= steps * 2.0 ** -24 * (y0.double().abs() + xr.abs() @ wd)).all()
+
+
 # float64: 512 and 1024 rows to a workgroup, the last ones ragged, one row into a further round of 256
 @pytest.mark.parametrize("n_in,n_out,pad", [(2049, 8200, 3), (1793, 8321, 0), (5000, 13200, 0), (4097, 16384, 1)])
 def test_mm8_float64_of_long_slices_against_the_exact_product(ops, n_in, n_out, pad):
