@@ -537,7 +537,8 @@ size_t rows_tot_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_
     // the quantisers of the att output and of h park their partial records here before the product starts
     const size_t q = rows_quant_scratch_bytes(R, n_wide > C ? n_wide : C);
     const size_t m = a > b ? (a > c ? a : c) : (b > c ? b : c);
-    return m > q ? m : q;
+    const size_t h = rows_deferred_bytes(R, C);         // a residual update handed on in slices
+    return std::max(std::max(m, q), h);
 }
 
 // n_wide = widest product output (n_ffn, or the vocabulary when every row needs logits)
@@ -594,7 +595,7 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     const int C = (int)d.n_embd, F = (int)d.n_ffn, V = (int)d.n_vocab;
     const size_t RC = (size_t)R * C;
     RWKV_TRY(rows_embed(st, tokens, R, V, C, d.emb, d.ln0_w, d.ln0_b, w.x));
-    // Few batch rows: where a product splits its contraction (from 9 rows on), and its result goes straight into one row-wise
+    // Few batch rows: where a product splits its contraction, and its result goes straight into one row-wise
     // kernel (k, v, r -> WKV; the two residual updates -> the next LayerNorm), the sum of the slices is left to that kernel
     // instead of a launch of its own.
     //

@@ -31,6 +31,7 @@ struct RowsDeferred {
     const long long *tot;   // [slices][slice] totals of this product; element (t, j) at t * ldd + j
     size_t slice;
     int slices, ldd, op;    // op: the RowTail still to be applied
+    bool apart, fused;      // see rounded_apart; the gated update as one fused multiply-add, as in the product's own epilogue
     const double *S, *qs, *zp;
     const float *gate;      // ROW_GATE_ADD
 };
@@ -47,6 +48,7 @@ struct RowsFew {
 };
 size_t rows_dig_bytes(int64_t R, int64_t K);
 size_t rows_tot_bytes(int64_t R, int64_t N, int64_t K);     // integer totals of ONE product (times the products in a launch) of a contraction of up to K
+size_t rows_deferred_bytes(int64_t R, int64_t N);           // integer totals of one product handed on in slices (see RowsDeferred)
 size_t rows_quant_scratch_bytes(int64_t R, int64_t K);   // what rows_quant writes into its scratch area (0: unused)
 // The plan rows_products follows for n products [R, K] x [K, N]: out = {kernel kind, grid x, grid y, splits}.
 void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int out[4]);

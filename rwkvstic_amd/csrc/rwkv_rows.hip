@@ -182,12 +182,12 @@ __device__ __forceinline__ void row_scale(float amax, double &S, double &invS) {
 // Element (t, j) of a product handed on unfinished: the slices added up (integers: exact in any order), then
 // y = S_t * tot + 128 * S_t * sum q_t + zp_t as in rows_finish_kernel.
 __device__ __forceinline__ double deferred_y(const RowsDeferred &d, int t, long long tot) {
-    const double S = d.S[t];
-    return S * (double)tot + 128.0 * (S * d.qs[t]) + d.zp[t];
+    const double S = d.S[t], sq = 128.0 * (S * d.qs[t]), zp = d.zp[t];
+    return d.apart ? S * (double)tot + sq + zp : S * (double)tot + (sq + zp);
 }
 // The slices are requested together, without a branch (always kRowsDeferSlices of them: one past the last reads
 // slice 0 again and is not counted): a loop over a run-time count would wait for every slice before asking for the
-// next, and a branch would keep the loads of a thread's channel groups apart.
+// next.  (slices_sum4: of exactly so many, behind one branch for all of a thread's channel groups.)
 __device__ __forceinline__ long long slices_sum1(const long long *tp, size_t slice, int slices) {
     long long u[kRowsDeferSlices], tot = 0;
 #pragma unroll
@@ -196,18 +196,17 @@ __device__ __forceinline__ long long slices_sum1(const long long *tp, size_t sli
     for (int z = 0; z < kRowsDeferSlices; ++z) tot += z < slices ? u[z] : 0;
     return tot;
 }
-__device__ __forceinline__ void slices_sum4(const long long *tp, size_t slice, int slices, long long (&tot)[4]) {
-    longlong2 u[kRowsDeferSlices][2];
+template <int SLICES>
+__device__ __forceinline__ void slices_sum4(const long long *tp, size_t slice, long long (&tot)[4]) {
+    longlong2 u[SLICES][2];
 #pragma unroll
-    for (int z = 0; z < kRowsDeferSlices; ++z) {
-        const long long *q = tp + (size_t)(z < slices ? z : 0) * slice;
+    for (int z = 0; z < SLICES; ++z) {
+        const long long *q = tp + (size_t)z * slice;
         u[z][0] = *reinterpret_cast<const longlong2 *>(q); u[z][1] = *reinterpret_cast<const longlong2 *>(q + 2);
     }
+    tot[0] = tot[1] = tot[2] = tot[3] = 0;
 #pragma unroll
-    for (int z = 0; z < kRowsDeferSlices; ++z) {
-        const bool on = z < slices;
-        tot[0] += on ? u[z][0].x : 0; tot[1] += on ? u[z][0].y : 0; tot[2] += on ? u[z][1].x : 0; tot[3] += on ? u[z][1].y : 0;
-    }
+    for (int z = 0; z < SLICES; ++z) { tot[0] += u[z][0].x; tot[1] += u[z][0].y; tot[2] += u[z][1].x; tot[3] += u[z][1].y; }
 }
 __device__ __forceinline__ double deferred_value(const RowsDeferred &d, int t, int j) {
     return deferred_y(d, t, slices_sum1(d.tot + (size_t)t * d.ldd + j, d.slice, d.slices));
@@ -312,6 +311,27 @@ __device__ __forceinline__ void st4(double *p, const double (&v)[4]) {
 // 8 rows of 2560 channels, three / two mixes: 6.9 / 7.4 us, 32 rows of 5120 15.2 / 14.8 us (one workgroup of 512 threads for
 // the row and all its mixes: 11.1 / 9.7 and 19.6 / 15.4; the same with every parameter vector requested ahead: no faster).
 constexpr int kLnRowThreads = 512;
+template <int NSEG, int SLICES>
+__device__ __forceinline__ void add_pending(const RowsDeferred &d, int t, int c, int step, int C, double *x_out, double (&xv)[NSEG][4]) {
+    const bool gated = d.op == ROW_GATE_ADD;
+#pragma unroll
+    for (int g = 0; g < NSEG; ++g) {
+        const int c0 = c + g * step;
+        if (c0 < C) {
+            long long tot[4];
+            float gt[4] = {0.f, 0.f, 0.f, 0.f};
+            slices_sum4<SLICES>(d.tot + (size_t)t * d.ldd + c0, d.slice, tot);
+            if (gated) ld4(gt, d.gate + (size_t)t * C + c0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double y = deferred_y(d, t, tot[i]), f = gated ? (double)sigmoid_f32(gt[i]) : 1.0;
+                if (d.fused) xv[g][i] = fma(y, f, xv[g][i]);
+                else xv[g][i] += gated ? y * f : y;
+            }
+            if (x_out) st4(x_out + c0, xv[g]);
+        }
+    }
+}
 template <bool MIX, int NSEG>
 __global__ void __launch_bounds__(kLnRowThreads) rows_ln_mix_quant_row_kernel(const LnQuantArgs a) {
     __shared__ double red0[2 * 8], red1[2 * 8], red2[8], red3[8];
@@ -346,23 +366,11 @@ __global__ void __launch_bounds__(kLnRowThreads) rows_ln_mix_quant_row_kernel(co
     if (a.add.tot) {
         // The product before this kernel was handed on unfinished: x += y (block.py:80) or x += y * sigmoid(r)
         // (block.py:95-100), as rows_finish_kernel would have done.
-        const bool gated = a.add.op == ROW_GATE_ADD;
-#pragma unroll
-        for (int g = 0; g < NSEG; ++g) {
-            const int c0 = 4 * (tid + g * nt);
-            if (c0 < C) {
-                long long tot[4] = {0, 0, 0, 0};
-                float gt[4] = {0.f, 0.f, 0.f, 0.f};
-                slices_sum4(a.add.tot + (size_t)t * a.add.ldd + c0, a.add.slice, a.add.slices, tot);
-                if (gated) ld4(gt, a.add.gate + (size_t)t * C + c0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const double y = deferred_y(a.add, t, tot[i]);
-                    xv[g][i] += gated ? y * (double)sigmoid_f32(gt[i]) : y;
-                }
-                if (a.x_out && m == 0) st4(a.x_out + (size_t)t * C + c0, xv[g]);
-            }
-        }
+        const int c = 4 * tid, step = 4 * nt;
+        double *xo = a.x_out && m == 0 ? a.x_out + (size_t)t * C : nullptr;
+        if (a.add.slices == 2) add_pending<NSEG, 2>(a.add, t, c, step, C, xo, xv);
+        else if (a.add.slices == 3) add_pending<NSEG, 3>(a.add, t, c, step, C, xo, xv);
+        else add_pending<NSEG, 4>(a.add, t, c, step, C, xo, xv);
     }
     double s[2] = {0.0, 0.0};
 #pragma unroll
@@ -1185,8 +1193,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 // Bound: the latency of a few dependent loads per wavefront, then HBM.  So the blocks are spread over as many wavefronts
 // as are resident at once (vec_shape), which needs no split of the contraction and no second launch; wide products take
 // several tiles per wavefront, since for two M-tiles the digits are twice a tile's bytes.  8 rows at 2560 channels (us per
-// launch), 4 wavefronts of one tile with 8 blocks in flight / this: k, v, r 10.1 / 7.3, att output 7.4 / 5.4, ffn key and
-// receptance 12.7 + 6.4 / 10.1, ffn value 15.5 / 13.0, head 43 / 30.5.
+// launch), 4 wavefronts of one tile with 8 blocks in flight / this: k, v, r 10.1 / 6.4, att output 7.4 / 4.9, ffn key and
+// receptance 12.7 + 6.4 / 8.4, ffn value 15.5 / 11.1 (7.5 in three slices: see vec_split), head 43 / 24.9.
 // ---------------------------------------------------------------------------
 constexpr int kVecMT = 2, kVecMTMax = 8;
 
@@ -1795,13 +1803,16 @@ static int64_t general_cost(int64_t w4) {
     return (w4 / 512) * 64 + (rem == 0 ? 0 : rem <= 256 ? 32 : 64);
 }
 static bool general_wide(int64_t w4, int64_t w5) { return w4 >= 256 && kGemmWideNum * ceil_div(w5, 256) * 40 < kGemmWideDen * general_cost(w4); }
-static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n) {
+static int vec_split(int64_t MT, int64_t NT, int64_t KB);
+// handed_on: the consumer adds up the slices of a contraction of at most 8 rows.
+static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n, bool handed_on = false) {
     ProductPlan p;
     p.split = 1;
     if (vec_rows(MT, NT * n, KB)) {
         // few rows: whole contractions, as long as a digit's sum of them stays inside int32 (2^20 per block)
         p.kind = PLAN_VEC; p.gx = (int)NT; p.gy = 1;
         while (ceil_div(KB, p.split) > 1024 && p.split < kMaxSplit) p.split *= 2;
+        if (handed_on && MT <= kVecMT && n == 1 && p.split == 1) p.split = vec_split(MT, NT, KB);
         return p;
     }
     p.gy = (int)ceil_div(MT, 16);
@@ -1825,23 +1836,70 @@ static bool rounded_apart(int64_t MT, int64_t NT, int64_t KB, int n) {
     return KB >= 16 && (NT * n < 128 || (NT * n < 512 && KB >= kGemmLongBlocks));
 }
 // Shape of the few-row kernel for a launch of so many column tiles: tiles per workgroup, wavefronts per workgroup, blocks
-// in flight per wavefront and tile (at most).  All workgroups resident at once, 2000 to 4000 wavefronts where the tiles allow it; one
-// tile per workgroup while that fills the device, more where the digits every wavefront reads would outweigh the weights.
+// in flight per wavefront and tile (at most).  All workgroups resident at once; KB: the blocks of a workgroup's part of the contraction.
+//
+// Bound: what the busiest compute unit draws, some 40 KB a us, beside 3 us of launch and first loads.  Per contraction block a workgroup
+// of ntw tiles reads their weights (ntw KB) and the digits of all rows (MT KB).  So up to 8 rows take the ntw that leaves that unit the least,
+// a larger one only where it saves 32 KB or so; four tiles only where the workgroups fill four fifths of the device.  Us a launch of 8
+// rows, 1 / 2 / 4 tiles: 800 tiles of 40 blocks 10.9 / 9.3 / 8.4, 480 of 40 7.2 / 6.4 / 8.0, 288 of 24 5.3 / 4.9 / 5.9, 960 of 80
+// 20.2 / 16.3 / 15.1, 320 of 80 11.1 / 9.0 / 12.2, 1280 of 64 20.6 / 17.9 / 24.2; 160 of 40 4.9 / 5.9 / 7.5.  320 of 16 4.35 / 4.21 / 5.0,
+// but a step of 24 layers of 1024 962 us with one tile, 975 with two.
 struct VecShape { int ntw, nw, u; };
+static int64_t vec_draw(int64_t tiles, int ntw, int MT) { return ceil_div(ceil_div(tiles, ntw), 256) * (ntw + MT); }
 static VecShape vec_shape(int64_t tiles, int64_t KB, int MT) {
     VecShape v;
-    if (MT > 4) v = tiles > 256 ? VecShape{2, 8, 2} : VecShape{1, 16, 2};       // (128 KB of sums in LDS)
-    else if (tiles > 1280) v = VecShape{4, 8, 3};
-    else if (tiles > 320) v = tiles <= 512 ? VecShape{2, 16, 3} : VecShape{2, 8, 5};
-    else if (tiles > 256) v = VecShape{1, 8, 5};
-    else v = VecShape{1, 16, 5};
-    if (MT > 2 && v.u > 3) v.u = 3;                     // (registers)
-    // No more in flight than a wavefront has: what is past the end is loaded all the same.  With this and the refilled slots, us a
-    // step of 8 sequences before / now: 12 layers of 512 437 / 433, of 768 464 / 457, 24 of 1024 1014 / 965, 12 of 1536 625 / 597, 8
-    // of 2048 479 / 457, 12 of 2560 780 / 766, 8 of 4096 820 / 776, 4 of 5120 586 / 576.
-    const int64_t each = ceil_div(KB, v.nw);
-    if (each < v.u) v.u = each <= 1 ? 1 : each == 2 ? 2 : each == 3 ? 3 : v.u;
+    if (MT > kVecMT) {
+        if (MT > 4) v = tiles > 256 ? VecShape{2, 8, 2} : VecShape{1, 16, 2};       // (128 KB of sums in LDS)
+        else if (tiles > 1280) v = VecShape{4, 8, 3};
+        else if (tiles > 320) v = tiles <= 512 ? VecShape{2, 16, 3} : VecShape{2, 8, 5};
+        else if (tiles > 256) v = VecShape{1, 8, 5};
+        else v = VecShape{1, 16, 5};
+        if (v.u > 3) v.u = 3;                               // (registers)
+        // No more in flight than a wavefront has: what is past the end is loaded all the same.  With this and the refilled slots, us a
+        // step of 8 sequences before / now: 12 layers of 512 437 / 433, of 768 464 / 457, 24 of 1024 1014 / 965, 12 of 1536 625 / 597, 8
+        // of 2048 479 / 457, 12 of 2560 780 / 766, 8 of 4096 820 / 776, 4 of 5120 586 / 576.
+        const int64_t each = ceil_div(KB, v.nw);
+        if (each < v.u) v.u = each <= 1 ? 1 : each == 2 ? 2 : each == 3 ? 3 : v.u;
+        return v;
+    }
+    const int64_t one = vec_draw(tiles, 1, MT), two = vec_draw(tiles, 2, MT), four = vec_draw(tiles, 4, MT);
+    v.ntw = 1;
+    if (tiles > 320 || (one - two) * KB >= 40) v.ntw = 2;
+    if (tiles > 1280) v.ntw = 4;
+    else if (v.ntw == 2 && (two - four) * KB >= 32 && 32 * ceil_div(tiles, 4) >= 25 * round_up(ceil_div(tiles, 4), 256)) v.ntw = 4;
+    // as many wavefronts and blocks in flight as leave the fewest loads past the end (480 tiles of 32 blocks, two to a workgroup: 16
+    // wavefronts of 2 blocks 5.4 us, 8 of 5 5.8; of 40 blocks 8 of 5 6.4, 16 of 3 6.8)
+    const int64_t each = ceil_div(KB, 8);
+    if (each <= 3) { v.nw = 8; v.u = (int)each; }
+    else if (v.ntw == 4) { v.nw = 8; v.u = tiles > 1280 ? 3 : 5; }
+    else if (KB <= 32) { v.nw = 16; v.u = 2; }
+    else if (KB <= 40) { v.nw = 8; v.u = 5; }
+    else if (KB <= 48) { v.nw = 16; v.u = 3; }
+    else if (v.ntw == 1) { v.nw = 16; v.u = 5; }
+    else if (ceil_div(tiles, 2) <= 256) { v.nw = 16; v.u = 3; }
+    else { v.nw = 8; v.u = 5; }
     return v;
+}
+// Slices of a contraction of at most 8 rows whose consumer, the LayerNorm kernel behind the two residual products of a batch step,
+// adds them up.  The ffn value product has few tiles and a long contraction, so whole contractions make a few compute units draw much: cut in
+// slices, with more tiles to a workgroup, all of them draw, and share the digits.  8 rows, us a launch with 1 / 2 / 3 / 4 slices: 2560 channels
+// 11.1 / 9.0 / 7.5 / 8.1, 5120 27.0 / 22.8 / 18.5 / 22.2, 1024 6.3 / 4.4 / 4.1 / 3.7.  The LayerNorm workgroups, one for each row and mix, pay
+// for it: 8 bytes a channel and slice, and the gate's 4, measured at 1.2 to 3.4 us.  Hence the 32 KB and the line at 7/10: 4 rows and fewer
+// (2560 channels 8.7 / 7.6 / 6.8 / 7.3) and 4096 channels gain no more than that costs (step of 8 layers 767 us both ways).  Us a step of 8
+// sequences, before (one tile to every workgroup of up to 320) / whole contractions / this: 24 layers of 1024 970 / 962 / 925, 12 of 1536
+// 589 / 579 / 560, 8 of 2048 453 / 447 / 439, 12 of 2560 764 / 744 / 722, 4 of 5120 566 / 519 / 497; all with the same bits.
+static int vec_split(int64_t MT, int64_t NT, int64_t KB) {
+    auto draw = [&](int s) {
+        const int64_t kb = ceil_div(KB, s);
+        return vec_draw(NT * s, vec_shape(NT * s, kb, (int)MT).ntw, (int)MT) * kb;
+    };
+    int best = 1;
+    int64_t least = draw(1) * 7 / 10;
+    for (int s = 2; s <= kRowsDeferSlices; ++s) {
+        const int64_t cost = draw(s) + 32 + (2 * s + 1) * NT / 16;
+        if (cost < least) { least = cost; best = s; }
+    }
+    return best;
 }
 // The kernel of that shape; null where there is none.  (More than one round only with the most blocks in flight.)
 using VecKernel = void (*)(const GemmArgs);
@@ -1856,7 +1914,7 @@ static VecKernel vec_kernel(int MT, const VecShape &v, bool rounds, bool stream)
     RWKV_VEC12(4, 8, 1, false)
     RWKV_VEC12(4, 8, 2, false)
     RWKV_VEC12(4, 8, 3, false) RWKV_VEC12(4, 8, 3, true)
-    RWKV_VEC12(2, 16, 1, false)
+    RWKV_VEC12(4, 8, 5, false) RWKV_VEC12(4, 8, 5, true)
     RWKV_VEC12(2, 16, 2, false)
     RWKV_VEC12(2, 16, 3, false) RWKV_VEC12(2, 16, 3, true)
     RWKV_VEC12(2, 8, 1, false)
@@ -1866,8 +1924,7 @@ static VecKernel vec_kernel(int MT, const VecShape &v, bool rounds, bool stream)
     RWKV_VEC12(1, 8, 1, false)
     RWKV_VEC12(1, 8, 2, false)
     RWKV_VEC12(1, 8, 3, false)
-    RWKV_VEC12(1, 8, 5, false) RWKV_VEC12(1, 8, 5, true)
-    RWKV_VEC12(1, 16, 1, false)
+    RWKV_VEC12(1, 8, 5, false)
     RWKV_VEC12(1, 16, 2, false)
     RWKV_VEC12(1, 16, 3, false)
     RWKV_VEC12(1, 16, 5, false) RWKV_VEC12(1, 16, 5, true)
@@ -1896,12 +1953,12 @@ static VecKernel vec_kernel(int MT, const VecShape &v, bool rounds, bool stream)
 // What a launch of so many M-tiles, column tiles and blocks would run; null without a kernel for it, or another kernel's.
 const void *vec_kernel_of(int64_t MT, int64_t tiles, int64_t KB, int64_t kb_per_split) {
     if (!vec_rows(MT, tiles, KB)) return nullptr;
-    const VecShape v = vec_shape(tiles, KB, (int)MT);
+    const VecShape v = vec_shape(tiles, kb_per_split, (int)MT);
     return reinterpret_cast<const void *>(vec_kernel((int)MT, v, kb_per_split > v.nw * v.u, false));
 }
 static int launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
     const int64_t tiles = g.NT2 > 0 ? (int64_t)g.NT + g.NT2 : (int64_t)g.NT * g.gz;
-    const VecShape v = vec_shape(tiles, g.KB, g.MT);
+    const VecShape v = vec_shape(tiles, g.kb_per_split, g.MT);
     const VecKernel kernel = vec_kernel(g.MT, v, g.kb_per_split > v.nw * v.u, stream);
     if (!kernel)
         return set_error(RWKV_ERR_SIZE, "gemv16_kernel: no instance for %d M-tiles, %lld column tiles, %d blocks", g.MT, (long long)tiles, g.KB);
@@ -1925,6 +1982,9 @@ static int gemm_split_bound(int64_t R, int64_t N, int64_t K) {
 }
 size_t rows_tot_bytes(int64_t R, int64_t N, int64_t K) {
     return (size_t)(ceil_div(R, 4) * 4 * round_up(N, 16) * 8) * (size_t)gemm_split_bound(R, N, K);
+}
+size_t rows_deferred_bytes(int64_t R, int64_t N) {
+    return R < kRowsDeferMax ? (size_t)(ceil_div(R, 4) * 4 * round_up(N, 16) * 8) * kRowsDeferSlices : 0;
 }
 // What rows_quant keeps in its scratch area for R rows of K values (0: that shape does not use it).
 // (a few long rows are quantised by several workgroups each, in two launches: one workgroup per row leaves most of the
@@ -2103,7 +2163,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     g.tot = tot;
     g.MT = (int)ceil_div(R, 4); g.NT = (int)ceil_div(N, 16); g.KB = (int)(K / 64); g.ldd = g.NT * 16;
     g.R = (int)R; g.N = (int)N; g.gate = gate;
-    const ProductPlan pl = plan_products(g.MT, g.NT, g.KB, n);
+    const ProductPlan pl = plan_products(g.MT, g.NT, g.KB, n, defer && R < kRowsDeferMax);
     const int split = pl.split;
     g.kb_per_split = (int)ceil_div(g.KB, split);
     g.split = split;
@@ -2131,7 +2191,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     if (split == 1) return RWKV_OK;     // the tail was applied in the product's epilogue
     if (defer && R < kRowsDeferMax && split <= kRowsDeferSlices) {   // the consumer adds the slices up
         for (int m = 0; m < n; ++m)
-            defer[m] = RowsDeferred{tot + (size_t)m * split * g.slice, g.slice, split, g.ldd, op, p[m].a.S, p[m].a.qs, p[m].a.zp, gate};
+            defer[m] = RowsDeferred{tot + (size_t)m * split * g.slice, g.slice, split, g.ldd, op, g.apart != 0, pl.kind == PLAN_VEC, p[m].a.S, p[m].a.qs, p[m].a.zp, gate};
         return RWKV_OK;
     }
 

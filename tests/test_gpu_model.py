@@ -548,6 +548,25 @@ def test_batch_steps_of_more_rows_than_are_resident_match_single_steps(C, B):
         assert float((states[:, :, row] - singles[:, :, row]).norm() / singles[:, :, row].norm()) < 2e-6, row
 
 
+# at most 8 rows, ffn value handed on in 3 or 4 slices (5 to 8 rows) or finished in its own launch (a row alone, 2048 channels of
+# 2048 hidden values): integer totals, exact in any order, rounded in the same place, so the bits of a row do not depend on the others
+@pytest.mark.parametrize("C,F,B", [(1024, 4096, 8), (1088, 4352, 5), (1536, 6144, 7), (2560, 10240, 8), (5120, 20480, 6), (2048, 2048, 8)])
+def test_rows_of_a_small_batch_have_the_bits_of_a_batch_of_one(C, F, B):
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"batch of {B} at C={C} F={F}")
+    m = HipRWKV(synth.iter_tensors(2, C, F, 100, seed=C + B, device="cuda", ln="random"))
+    states = m.emptyState.repeat(B, 1, 1, 1).contiguous()
+    singles = states.clone()
+    for step in range(3):
+        toks = synth.random_tokens(B, V=100, seed=50 + step).cuda()
+        lb, states = m.forward_batch(toks, states)
+        for b in range(B):
+            l1, s1 = m.forward_batch(toks[b:b + 1], singles[b:b + 1].clone())
+            singles[b] = s1[0]
+            assert torch.equal(lb[b], l1[0]), (step, b)
+    assert torch.equal(states, singles)
+
+
 def test_rwkv_shell_loads_checkpoint_file_and_generates(tmp_path, tiny):
     """RWKV(path) -> RWKVMaster surface (load.py:18,42-47; rwkvMaster.py:28-105) over the HIP model."""
     from rwkvstic_amd.master import RWKV, greedy
