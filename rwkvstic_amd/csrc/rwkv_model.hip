@@ -27,6 +27,7 @@
 #include "rwkv_decode.h"
 #include "rwkv_rows.h"
 
+#include <algorithm>
 #include <mutex>
 #include <new>
 #include <string>
@@ -525,7 +526,7 @@ constexpr int64_t kRowsMin = 4;        // shorter prompts go token by token
 struct RowsWs {
     double *x, *kvr, *att, *h;
     double *x2, *sh1, *sh2; // fewer than kRowsDeferMax rows: x after a pending update, the two newest shift rows (of any sequence; see RowsFew)
-    RowsOperand q[3];       // quantised left operands: q[0] up to n_ffn wide, q[1], q[2] n_embd wide
+    RowsOperand q[3];       // quantised left operands: q[0] up to n_ffn or n_embd wide, q[1], q[2] n_embd wide
     RowsOperand qv;         // ffn value's: the digits of q[0], row constants of its own (see rows_layers)
     long long *tot;
 };
@@ -548,7 +549,7 @@ size_t rows_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_
     n += round_up((size_t)R * F * 8, 256);              // h
     n += round_up((size_t)(R < kRowsDeferMax ? R : kRowsDeferMax - 1) * C * 8, 256) * 3;    // x2, sh1, sh2
     n += round_up((size_t)R * 8, 256) * 12;             // S, qs, zp of four operands
-    n += round_up(rows_dig_bytes(R, F), 256) + 2 * round_up(rows_dig_bytes(R, C), 256);
+    n += round_up(rows_dig_bytes(R, std::max(F, C)), 256) + 2 * round_up(rows_dig_bytes(R, C), 256);
     n += round_up(rows_tot_ws_bytes(R, C, F, n_wide, n_head), 256);
     return n;
 }
@@ -566,7 +567,7 @@ RowsWs rows_carve(void *ws, int64_t R, int64_t C, int64_t F, int64_t n_wide, int
         w.q[i].S = (double *)take((size_t)R * 8);
         w.q[i].qs = (double *)take((size_t)R * 8);
         w.q[i].zp = (double *)take((size_t)R * 8);
-        w.q[i].dig = (signed char *)take(rows_dig_bytes(R, i == 0 ? F : C));
+        w.q[i].dig = (signed char *)take(rows_dig_bytes(R, i == 0 ? std::max(F, C) : C));
     }
     w.qv.dig = w.q[0].dig;
     for (double **b : {&w.qv.S, &w.qv.qs, &w.qv.zp}) *b = (double *)take((size_t)R * 8);

@@ -550,7 +550,8 @@ def test_batch_steps_of_more_rows_than_are_resident_match_single_steps(C, B):
 
 # at most 8 rows, ffn value handed on in 3 or 4 slices (5 to 8 rows) or finished in its own launch (a row alone, 2048 channels of
 # 2048 hidden values): integer totals, exact in any order, rounded in the same place, so the bits of a row do not depend on the others
-@pytest.mark.parametrize("C,F,B", [(1024, 4096, 8), (1088, 4352, 5), (1536, 6144, 7), (2560, 10240, 8), (5120, 20480, 6), (2048, 2048, 8)])
+@pytest.mark.parametrize("C,F,B", [(1024, 4096, 8), (1088, 4352, 5), (1536, 6144, 7), (2560, 10240, 8), (5120, 20480, 6), (2048, 2048, 8),
+                                   (2048, 512, 8), (1024, 64, 3)])     # the widest rows are not the hidden ones
 def test_rows_of_a_small_batch_have_the_bits_of_a_batch_of_one(C, F, B):
     from rwkvstic_amd.model import HipRWKV
     _say(f"batch of {B} at C={C} F={F}")
