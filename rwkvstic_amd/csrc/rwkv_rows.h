@@ -36,7 +36,7 @@ struct RowsDeferred {
     const float *gate;      // ROW_GATE_ADD
 };
 constexpr int64_t kRowsDeferMax = 128;
-constexpr int kRowsDeferSlices = 4;     // a contraction split further than this is finished by a launch of its own
+constexpr int kRowsDeferSlices = 6;     // a contraction split further than this is finished by a launch of its own
 // What the LayerNorm kernel of fewer than kRowsDeferMax rows does besides (several workgroups share a row there, and none
 // may overwrite what another reads); of a sequence of any length, the shift rows (row 0 reads what the last row replaces).
 struct RowsFew {

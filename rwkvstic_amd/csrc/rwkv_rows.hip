@@ -21,6 +21,8 @@
 // hands it to the matrix instruction unchanged.
 #include "rwkv_rows.h"
 
+#include <type_traits>
+
 namespace rwkv {
 
 namespace {
@@ -185,15 +187,15 @@ __device__ __forceinline__ double deferred_y(const RowsDeferred &d, int t, long 
     const double S = d.S[t], sq = 128.0 * (S * d.qs[t]), zp = d.zp[t];
     return d.apart ? S * (double)tot + sq + zp : S * (double)tot + (sq + zp);
 }
-// The slices are requested together, without a branch (always kRowsDeferSlices of them: one past the last reads
-// slice 0 again and is not counted): a loop over a run-time count would wait for every slice before asking for the
-// next.  (slices_sum4: of exactly so many, behind one branch for all of a thread's channel groups.)
-__device__ __forceinline__ long long slices_sum1(const long long *tp, size_t slice, int slices) {
-    long long u[kRowsDeferSlices], tot = 0;
+// The slices are requested together, of exactly so many and behind one branch for all that a thread adds up: a loop over a run-time count
+// would wait for every slice before asking for the next, and a branch for each value would keep their loads apart.
+template <int SLICES>
+__device__ __forceinline__ long long slices_sum1(const long long *tp, size_t slice) {
+    long long u[SLICES], tot = 0;
 #pragma unroll
-    for (int z = 0; z < kRowsDeferSlices; ++z) u[z] = tp[(size_t)(z < slices ? z : 0) * slice];
+    for (int z = 0; z < SLICES; ++z) u[z] = tp[(size_t)z * slice];
 #pragma unroll
-    for (int z = 0; z < kRowsDeferSlices; ++z) tot += z < slices ? u[z] : 0;
+    for (int z = 0; z < SLICES; ++z) tot += u[z];
     return tot;
 }
 template <int SLICES>
@@ -208,8 +210,15 @@ __device__ __forceinline__ void slices_sum4(const long long *tp, size_t slice, l
 #pragma unroll
     for (int z = 0; z < SLICES; ++z) { tot[0] += u[z][0].x; tot[1] += u[z][0].y; tot[2] += u[z][1].x; tot[3] += u[z][1].y; }
 }
-__device__ __forceinline__ double deferred_value(const RowsDeferred &d, int t, int j) {
-    return deferred_y(d, t, slices_sum1(d.tot + (size_t)t * d.ldd + j, d.slice, d.slices));
+// F(count), the count a constant, for each of the counts that slices may have.
+static_assert(kRowsDeferSlices == 6, "the counts below");
+template <typename F>
+__device__ __forceinline__ void with_slices(int slices, F &&f) {
+    if (slices == 2) f(std::integral_constant<int, 2>());
+    else if (slices == 3) f(std::integral_constant<int, 3>());
+    else if (slices == 4) f(std::integral_constant<int, 4>());
+    else if (slices == 5) f(std::integral_constant<int, 5>());
+    else f(std::integral_constant<int, 6>());
 }
 
 struct LnQuantArgs {
@@ -368,9 +377,7 @@ __global__ void __launch_bounds__(kLnRowThreads) rows_ln_mix_quant_row_kernel(co
         // (block.py:95-100), as rows_finish_kernel would have done.
         const int c = 4 * tid, step = 4 * nt;
         double *xo = a.x_out && m == 0 ? a.x_out + (size_t)t * C : nullptr;
-        if (a.add.slices == 2) add_pending<NSEG, 2>(a.add, t, c, step, C, xo, xv);
-        else if (a.add.slices == 3) add_pending<NSEG, 3>(a.add, t, c, step, C, xo, xv);
-        else add_pending<NSEG, 4>(a.add, t, c, step, C, xo, xv);
+        with_slices(a.add.slices, [&](auto count) { add_pending<NSEG, decltype(count)::value>(a.add, t, c, step, C, xo, xv); });
     }
     double s[2] = {0.0, 0.0};
 #pragma unroll
@@ -1061,15 +1068,16 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 // The same product for at most 32 rows (a batch of single tokens): the weights are read once and
 // hardly reused, so what counts is how many weight bytes a compute unit has in flight.  Workgroup =
 // 4 wavefronts side by side = 8 M-tiles x 8 N-tiles (wavefront: 8 x 2); a contraction block is 8 digit
-// fragments + 8 weight fragments, fetched kSkinnyAhead blocks ahead (48 KiB of weights per workgroup).
+// fragments + 8 weight fragments, fetched kSkinnyAhead blocks ahead (48 KiB of weights per workgroup).  Up to 16 rows
+// have four M-tiles: a compute unit draws 12 instead of 16 KB a block (8 layers of 4096, 16 sequences 905 -> 869 us a step, of 5120, 9 1054 -> 1017).
 // ---------------------------------------------------------------------------
 constexpr int kSkinnyMT = 8, kSkinnyGN = 2, kSkinnyNT = 4 * kSkinnyGN;
-constexpr int kSkinnyFrags = kSkinnyMT + kSkinnyNT;     // 16: wave w fetches fragments w, w + 4, w + 8, w + 12
 constexpr int kSkinnyAhead = 6;
 
-template <bool STREAM>
+template <int MT, bool STREAM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm8_skinny_kernel(const GemmArgs a) {
-    __shared__ v4i frag[2][kSkinnyFrags][64];
+    static_assert(MT == 4 || MT == 8, "wavefront w fetches the digit fragments w and, of eight, w + 4, and the weight fragments w and w + 4");
+    __shared__ v4i frag[2][MT + kSkinnyNT][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int xcd = blockIdx.x % kXcds;
@@ -1096,20 +1104,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     const v4i *src[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int f = wave + 4 * i;
-        if (f < kSkinnyMT) {
-            const int mt = f < a.MT ? f : a.MT - 1;     // clamped: loads stay unconditional, results are dropped
-            src[i] = reinterpret_cast<const v4i *>(dig + ((size_t)mt * a.KB + kb0) * 1024) + lane;
-        } else {
-            int nt = bx * kSkinnyNT + (f - kSkinnyMT);
-            if (nt >= cols.NT) nt = cols.NT - 1;
-            src[i] = reinterpret_cast<const v4i *>(w16 + ((size_t)nt * a.KB + kb0) * 1024) + lane;
-        }
+    for (int i = 0; i < 2; ++i) {                       // clamped: loads stay unconditional, results are dropped
+        const int mt = min(wave + 4 * i, a.MT - 1), nt = min(bx * kSkinnyNT + wave + 4 * i, cols.NT - 1);
+        src[i] = reinterpret_cast<const v4i *>(dig + ((size_t)mt * a.KB + kb0) * 1024) + lane;
+        src[2 + i] = reinterpret_cast<const v4i *>(w16 + ((size_t)nt * a.KB + kb0) * 1024) + lane;
     }
-    v4i acc[kSkinnyMT][kSkinnyGN];
+    v4i acc[MT][kSkinnyGN];
 #pragma unroll
-    for (int i = 0; i < kSkinnyMT; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < kSkinnyGN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
 
@@ -1119,17 +1121,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #define RWKV_SKINNY_FETCH(F, K)                                                                      \
     do {                                                                                             \
         const size_t o_ = (size_t)((K) < nk ? (K) : nk - 1) * 64; /* past the end: the last block again (unused) */ \
-        F.v0 = src[0][o_]; F.v1 = src[1][o_]; F.v2 = ldw<STREAM>(src[2] + o_); F.v3 = ldw<STREAM>(src[3] + o_); \
+        F.v0 = src[0][o_]; if (MT == 8) F.v1 = src[1][o_]; F.v2 = ldw<STREAM>(src[2] + o_); F.v3 = ldw<STREAM>(src[3] + o_); \
     } while (0)
 #define RWKV_SKINNY_PARK(F, B)                                                                       \
     do {                                                                                             \
-        frag[B][wave][lane] = F.v0; frag[B][wave + 4][lane] = F.v1;                                  \
-        frag[B][wave + 8][lane] = F.v2; frag[B][wave + 12][lane] = F.v3;                             \
+        frag[B][wave][lane] = F.v0; if (MT == 8) frag[B][wave + 4][lane] = F.v1;                     \
+        frag[B][MT + wave][lane] = F.v2; frag[B][MT + 4 + wave][lane] = F.v3;                        \
     } while (0)
     // (same step as gemm8_body: the next block is parked, and its registers refilled, piece by piece between
     // this block's groups of matrix instructions)
 #define RWKV_SKINNY_MOVE(FN, I, V, B, O)                                                             \
-    { frag[B][wave + 4 * (I)][lane] = FN.V; FN.V = (I) < 2 ? src[I][O] : ldw<STREAM>(src[I] + (O)); }
+    { frag[B][((I) < 2 ? 0 : MT - 8) + wave + 4 * (I)][lane] = FN.V; FN.V = (I) < 2 ? src[I][O] : ldw<STREAM>(src[I] + (O)); }
 #define RWKV_SKINNY_STEP(FN, K)                                                                      \
     {                                                                                                \
         const int buf_ = (K) & 1;                                                                    \
@@ -1137,24 +1139,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         lds_barrier();                                                                               \
         v4i Bv_[kSkinnyGN];                                                                          \
         _Pragma("unroll") for (int j = 0; j < kSkinnyGN; ++j)                                        \
-            Bv_[j] = frag[buf_][kSkinnyMT + wave * kSkinnyGN + j][lane];                             \
+            Bv_[j] = frag[buf_][MT + wave * kSkinnyGN + j][lane];                                    \
         v4i Av_ = frag[buf_][0][lane];                                                               \
-        _Pragma("unroll") for (int i = 0; i < kSkinnyMT; ++i) {                                      \
-            const v4i An_ = frag[buf_][i + 1 < kSkinnyMT ? i + 1 : i][lane];                         \
+        _Pragma("unroll") for (int i = 0; i < MT; ++i) {                                             \
+            const v4i An_ = frag[buf_][i + 1 < MT ? i + 1 : i][lane];                                \
             if (i == 0) RWKV_SKINNY_MOVE(FN, 0, v0, buf_ ^ 1, on_)                                   \
-            if (i == 2) RWKV_SKINNY_MOVE(FN, 1, v1, buf_ ^ 1, on_)                                   \
-            if (i == 4) RWKV_SKINNY_MOVE(FN, 2, v2, buf_ ^ 1, on_)                                   \
-            if (i == 6) RWKV_SKINNY_MOVE(FN, 3, v3, buf_ ^ 1, on_)                                   \
+            if (MT == 8 && i == 2) RWKV_SKINNY_MOVE(FN, 1, v1, buf_ ^ 1, on_)                        \
+            if (i == MT / 2) RWKV_SKINNY_MOVE(FN, 2, v2, buf_ ^ 1, on_)                              \
+            if (i == MT - (MT == 8 ? 2 : 1)) RWKV_SKINNY_MOVE(FN, 3, v3, buf_ ^ 1, on_)              \
             _Pragma("unroll") for (int j = 0; j < kSkinnyGN; ++j)                                    \
                 acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(Av_, Bv_[j], acc[i][j], 0, 0, 0);  \
             Av_ = An_;                                                                               \
         }                                                                                            \
         __builtin_amdgcn_sched_group_barrier(0x100, kSkinnyGN + 2, 0);                               \
-        _Pragma("unroll") for (int i = 0; i < kSkinnyMT; ++i) {                                      \
-            if (i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);                       \
+        _Pragma("unroll") for (int i = 0; i < MT; ++i) {                                             \
+            const bool moves_ = MT == 8 ? i % 2 == 0 : i != 1;                                       \
+            if (moves_) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);                           \
             __builtin_amdgcn_sched_group_barrier(0x008, kSkinnyGN, 0);                               \
-            if (i + 2 < kSkinnyMT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                \
-            if (i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                       \
+            if (i + 2 < MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                       \
+            if (moves_) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                           \
         }                                                                                            \
     }
     RWKV_SKINNY_FETCH(fly0, 0); RWKV_SKINNY_FETCH(fly1, 1); RWKV_SKINNY_FETCH(fly2, 2);
@@ -1179,7 +1182,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #undef RWKV_SKINNY_MOVE
 #undef RWKV_SKINNY_PARK
 #undef RWKV_SKINNY_FETCH
-    gemm_epilogue<kSkinnyMT, kSkinnyGN>(a, cols, acc, 0, nt0, mat, bz, lane);
+    gemm_epilogue<MT, kSkinnyGN>(a, cols, acc, 0, nt0, mat, bz, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1382,7 +1385,7 @@ struct WkvRowsArgs {
     double *state;              // rows aa, bb, pp of the layer: state + 2C; batch: + row * state_stride
     int64_t state_stride;
     float *out;                 // [R, C]  wkv * sigmoid(r): a float32 product
-    RowsDeferred pend[3];       // batch rows: k, v, r still in slices (tot null: read from the arrays above)
+    RowsDeferred pend[3];       // batch rows: k, v, r still in slices, as many of each (tot null: all are read from the arrays above)
 };
 
 __global__ void __launch_bounds__(64) wkv_rows_kernel(const WkvRowsArgs a) {
@@ -1396,10 +1399,16 @@ __global__ void __launch_bounds__(64) wkv_rows_kernel(const WkvRowsArgs a) {
     double pp = st[2 * C + c];
     for (int t = t0; t < t1; ++t) {
         const size_t i = (size_t)t * C + c;
-        // (uniform branches; a pending product is rounded to float32 exactly as ROW_STORE_F32 would have stored it)
-        const float kk = a.pend[0].tot ? (float)deferred_value(a.pend[0], t, c) : a.k[i];
-        const float vv = a.pend[1].tot ? (float)deferred_value(a.pend[1], t, c) : a.v[i];
-        const float rr = a.pend[2].tot ? (float)deferred_value(a.pend[2], t, c) : a.r[i];
+        float kk, vv, rr;
+        if (a.pend[0].tot) {                            // (uniform; rounded to float32 exactly as ROW_STORE_F32 would have stored them)
+            long long tot[3];
+            with_slices(a.pend[0].slices, [&](auto count) {
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    tot[j] = slices_sum1<decltype(count)::value>(a.pend[j].tot + (size_t)t * a.pend[j].ldd + c, a.pend[j].slice);
+            });
+            kk = (float)deferred_y(a.pend[0], t, tot[0]); vv = (float)deferred_y(a.pend[1], t, tot[1]); rr = (float)deferred_y(a.pend[2], t, tot[2]);
+        } else { kk = a.k[i]; vv = a.v[i]; rr = a.r[i]; }
         const float y = wkv_step_f32(w, u, kk, vv, aa, bb, pp);
         a.out[i] = y * sigmoid_f32(rr);
     }
@@ -1790,11 +1799,24 @@ static bool vec_rows(int64_t MT, int64_t tiles, int64_t KB) {
     if (MT <= 4) return tiles <= 1280 && MT * KB <= (tiles <= 256 ? 700 : 200);
     return MT <= kVecMTMax && tiles <= 512 && MT * KB <= 400;
 }
-// Slices of a contraction of 9 to 32 rows in gemm8_skinny_kernel, whether it is the kernel that runs or not (see rounded_apart).
-static int skinny_split(int64_t NT, int64_t KB, int n) {
-    int split = 1;
-    while (ceil_div(NT, kSkinnyNT) * n * split < kSkinnyFillWgs && KB / (split * 2) >= 8 && split < kMaxSplit) split *= 2;
-    return split;
+// Whether a contraction of 9 to 32 rows is cut in gemm8_skinny_kernel, whether it is the kernel that runs or not (see rounded_apart).
+static bool skinny_cut(int64_t NT, int64_t KB, int n) { return ceil_div(NT, kSkinnyNT) * n < kSkinnyFillWgs && KB >= 16; }
+// In how many slices: as vec_split, what the busiest compute unit draws (eight tiles' weights and the digits of 16 or 32 rows), and what it
+// costs to add them up: in the LayerNorm kernel as there, in the WKV kernel, whose workgroups are many, little, in a launch of its own 4 to 5 us, and
+// the two that then wait for it.  (So no power of two: 40 column blocks of 5120 channels fill 240 compute units in six slices, 160 in four.)  Us a
+// step of 32 sequences before (the power of two that brings 128 workgroups, up to eight) / now: 24 layers of 1024 1308 / 1220, 12 of 2560 1096 /
+// 1071, 8 of 4096 1023 / 1011, 8 of 5120 1289 / 1254; of 16, with four M-tiles (gemm8_skinny_kernel), 905 / 848 of 4096 and 1106 / 1031 of 5120.
+static int skinny_split(int64_t MT, int64_t NT, int64_t KB, int n, bool handed_on) {
+    if (!skinny_cut(NT, KB, n)) return 1;
+    int best = 2;
+    int64_t least = INT64_MAX;
+    for (int s = 2; s <= kMaxSplit && KB >= 8 * s; ++s) {
+        const bool sum = handed_on && s <= kRowsDeferSlices;
+        const int64_t cost = ceil_div(ceil_div(NT, kSkinnyNT) * n * s, 256) * (kSkinnyNT + (MT <= 4 ? 4 : 8)) * ceil_div(KB, s) +
+                             (sum && n > 1 ? 8 * s : sum ? 32 + (2 * s + 1) * NT / 16 : 420 + 30 * s * n);
+        if (cost < least) { least = cost; best = s; }
+    }
+    return best;
 }
 // Rounds of workgroups on 256 compute units, in matrix instructions per step: two general workgroups (w4 in all) share a
 // compute unit (2 x 32), a wide one (w5) has it alone (40).
@@ -1820,7 +1842,7 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n, bool
     if (p.kind == PLAN_GENERAL && general_wide(ceil_div(NT, kGemmNT) * p.gy * n, ceil_div(NT, kGemmWideNT) * p.gy * n)) p.kind = PLAN_WIDE;
     p.gx = (int)ceil_div(NT, p.kind == PLAN_SKINNY ? kSkinnyNT : p.kind == PLAN_WIDE ? kGemmWideNT : kGemmNT);
     // Split the contraction until the grid has a few workgroups per compute unit.
-    if (p.kind == PLAN_SKINNY) p.split = skinny_split(NT, KB, n);
+    if (p.kind == PLAN_SKINNY) p.split = skinny_split(MT, NT, KB, n, handed_on);
     else
         while ((int64_t)p.gx * p.gy * n * p.split < kGemmFillWgs && KB / (p.split * 2) >= 8 && p.split < kMaxSplit) p.split *= 2;
     // a long contraction on a grid still below the device: one split more (two slices at most)
@@ -1832,7 +1854,7 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n, bool
 // most 32 rows that once were split run whole contractions now and keep the first: the last bit of y reaches the logits, and
 // with them the texts of a seeded sampler.
 static bool rounded_apart(int64_t MT, int64_t NT, int64_t KB, int n) {
-    if (MT > kVecMT) return MT <= kSkinnyMT ? skinny_split(NT, KB, n) > 1 : plan_products(MT, NT, KB, n).split > 1;
+    if (MT > kVecMT) return MT <= kSkinnyMT ? skinny_cut(NT, KB, n) : plan_products(MT, NT, KB, n).split > 1;
     return KB >= 16 && (NT * n < 128 || (NT * n < 512 && KB >= kGemmLongBlocks));
 }
 // Shape of the few-row kernel for a launch of so many column tiles: tiles per workgroup, wavefronts per workgroup, blocks
@@ -1969,13 +1991,15 @@ static int launch_vec(hipStream_t st, const GemmArgs &g, bool stream) {
 }
 
 // Upper bound of the splits plan_products chooses for R rows, N columns and contractions of up to K, whatever the number of
-// products in the launch.  A longer contraction only lifts the limit on the split, so from 9 rows on the plan for an
-// unbounded one bounds every real one; at most 8 rows split for the length's sake alone, which for no model's is needed.
+// products in the launch.  A longer contraction only lifts the limit on the split, so from 33 rows on the plan for an
+// unbounded one bounds every real one; 9 to 32 rows are cut in any number of slices or not at all; at most 8 rows split for the
+// length's sake alone, which for no model's is needed (slices that are handed on: rows_deferred_bytes).
 static int gemm_split_bound(int64_t R, int64_t N, int64_t K) {
-    const int64_t MT = ceil_div(R, 4), NT = ceil_div(N, 16);
+    const int64_t MT = ceil_div(R, 4), NT = ceil_div(N, 16), any = (int64_t)1 << 40;
+    if (MT > kVecMT && MT <= kSkinnyMT) return skinny_cut(NT, any, 1) ? kMaxSplit : 1;
     int s = 1;
     for (int n = 1; n <= kRowsMaxProducts; ++n) {
-        const int sp = plan_products(MT, NT, MT <= kVecMT ? ceil_div(K, 64) : (int64_t)1 << 40, n).split;
+        const int sp = plan_products(MT, NT, MT <= kVecMT ? ceil_div(K, 64) : any, n).split;
         if (sp > s) s = sp;
     }
     return s;
@@ -2136,6 +2160,13 @@ int rows_quant(hipStream_t st, int64_t R, int64_t K, const void *in, bool in_f32
     return RWKV_OK;
 }
 
+static int launch_skinny(hipStream_t st, const GemmArgs &g, const dim3 &grid, bool stream) {
+    const bool four = g.MT <= 4;
+    hipLaunchKernelGGL(four ? (stream ? gemm8_skinny_kernel<4, true> : gemm8_skinny_kernel<4, false>)
+                            : (stream ? gemm8_skinny_kernel<8, true> : gemm8_skinny_kernel<8, false>), grid, dim3(256), 0, st, g);
+    RWKV_CHECK_LAUNCH("gemm8_skinny_kernel");
+    return RWKV_OK;
+}
 static int launch_general(hipStream_t st, GemmArgs &g, bool wide, int gx, bool stream) {
     g.gx = gx; g.gy = (int)ceil_div(g.MT, 16); g.by_rows = g.gy >= kXcds;
     g.per_xcd = ((g.by_rows ? g.gy : gx) + kXcds - 1) / kXcds;
@@ -2180,9 +2211,8 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     } else if (pl.kind == PLAN_SKINNY) {
         g.gx = pl.gx; g.gy = 1; g.by_rows = 0; g.per_xcd = (pl.gx + kXcds - 1) / kXcds;
         const dim3 grid((unsigned)(kXcds * g.per_xcd * g.gz));
-        if (p[0].stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
-        else hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
-        RWKV_CHECK_LAUNCH("gemm8_skinny_kernel");
+        const int rc = launch_skinny(st, g, grid, p[0].stream);
+        if (rc) return rc;
     } else {
         const int rc = launch_general(st, g, pl.kind == PLAN_WIDE, pl.gx, p[0].stream);
         if (rc) return rc;
@@ -2263,9 +2293,8 @@ int rows_ffn_key_receptance(hipStream_t st, bool sequence, const RowsProduct &k,
     } else if (C % 64 == 0 && g.MT <= kSkinnyMT && gx >= kSkinnyPairWgs) {
         g.gx = gx; g.per_xcd = (gx + kXcds - 1) / kXcds;
         const dim3 grid((unsigned)(kXcds * g.per_xcd));
-        if (k.stream) hipLaunchKernelGGL(gemm8_skinny_kernel<true>, grid, dim3(256), 0, st, g);
-        else hipLaunchKernelGGL(gemm8_skinny_kernel<false>, grid, dim3(256), 0, st, g);
-        RWKV_CHECK_LAUNCH("gemm8_skinny_kernel");
+        const int rc = launch_skinny(st, g, grid, k.stream);
+        if (rc) return rc;
     } else if (pair_general(g.MT, g.NT, g.NT2, g.KB)) {
         const int rc = launch_general(st, g, false, (int)(ceil_div(g.NT, kGemmNT) + ceil_div(g.NT2, kGemmNT)), k.stream);
         if (rc) return rc;
@@ -2287,6 +2316,8 @@ int rows_wkv(hipStream_t st, int64_t R, int C, bool sequence, const float *k, co
         else a.pend[i].tot = nullptr;
         if (a.pend[i].tot && (sequence || a.pend[i].op != ROW_STORE_F32))
             return set_error(RWKV_ERR_ARG, "rows_wkv: a pending product needs batch rows and the float32 store tail");
+        if ((a.pend[i].tot == nullptr) != (a.pend[0].tot == nullptr) || (a.pend[i].tot && a.pend[i].slices != a.pend[0].slices))
+            return set_error(RWKV_ERR_ARG, "rows_wkv: k, v and r are pending together, in as many slices, or none of them is");
     }
     if (sequence && R >= kWkvSeqMin) {
         // short sequences: the smallest block that covers them leaves the fewest lanes idle

@@ -568,6 +568,13 @@ def test_rows_of_a_small_batch_have_the_bits_of_a_batch_of_one(C, F, B):
     assert torch.equal(states, singles)
 
 
+# four and eight M-tiles, ffn value in five or six slices that are handed on, att output and k, v, r in as many as fill the device
+@pytest.mark.parametrize("C,F,B", [(4096, 16384, 9), (4096, 16384, 16), (4096, 16384, 17), (5120, 20480, 16), (5120, 20480, 32), (2560, 10240, 20),
+                                   (640, 24576, 32)])
+def test_batch_steps_in_slices_that_fill_the_device_match_single_steps(C, F, B):
+    test_batch_steps_of_ragged_and_wide_rows_match_single_steps(C, F, B)
+
+
 def test_rwkv_shell_loads_checkpoint_file_and_generates(tmp_path, tiny):
     """RWKV(path) -> RWKVMaster surface (load.py:18,42-47; rwkvMaster.py:28-105) over the HIP model."""
     from rwkvstic_amd.master import RWKV, greedy
