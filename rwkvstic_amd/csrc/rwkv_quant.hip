@@ -94,17 +94,17 @@ quantize_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in,
 // parallel), the layer of width 5120 1.18 ms (0.88).
 //
 //   quant_minmax_kernel   256 channels x one of the row splits: partial minimum and maximum
-//   quant_scale_kernel    one channel per thread: partials -> lo, range, 1 / range
-//   quant_encode_kernel   128 channels x kEncRows rows at a time: codes, layouts; in workgroups of its own the offsets
+//   quant_encode_kernel   128 channels x kEncRows rows at a time: codes, layouts; in workgroups of its own the offsets.  Every workgroup
+//                         makes lo, range and 1 / range of its channels from the partials, while its first rows travel (a launch between
+//                         the two that did only that took 27 of the 320 us of a layer of width 2560)
 // ---------------------------------------------------------------------------
 constexpr int kEncRows = 64;            // rows of one LDS tile: 8 blocks of the P8 layout, 4 x 2 of the M16 layout
 constexpr int kChainChannels = 8;       // channels of a workgroup that adds up fractions
 constexpr int64_t kChainMaxBlocks = 1 << 20;    // such workgroups (a launch has at most 2^32 threads); of more channels each takes several groups
-constexpr int kMinMaxSplits = 32;       // enough workgroups at 2560 channels (320); more only lengthens quant_scale_kernel
+constexpr int kMinMaxSplits = 32;       // enough workgroups at 2560 channels (320); a partial to each 8 threads of quant_offsets
 
 struct QuantWs {
     float2 *mm;                 // [splits][n_in]
-    double *lo, *ran, *inv;     // [n_in] each
     int64_t splits, split_rows; // of the minimum / maximum pass
     int64_t parts, part_rows;   // of the encoding pass: part_rows a multiple of kEncRows
     int64_t chain_blocks, col_blocks;   // its workgroups: the offsets' first, then col_blocks x parts
@@ -125,9 +125,6 @@ static QuantWs quant_carve(int64_t n_out, int64_t n_in, void *ws) {
     size_t at = 0;
     auto take = [&](int64_t bytes) { unsigned char *r = p + at; at += (size_t)round_up(bytes, 256); return r; };
     q.mm = reinterpret_cast<float2 *>(take(q.splits * n_in * 8));
-    q.lo = reinterpret_cast<double *>(take(n_in * 8));
-    q.ran = reinterpret_cast<double *>(take(n_in * 8));
-    q.inv = reinterpret_cast<double *>(take(n_in * 8));
     q.bytes = at;
     return q;
 }
@@ -173,18 +170,11 @@ quant_minmax_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
     }
 }
 
-__global__ void __launch_bounds__(64)
-quant_scale_kernel(int64_t n_in, QuantWs q) {
-    const int64_t j = (int64_t)blockIdx.x * 64 + threadIdx.x;
-    if (j >= n_in) return;
-    float lo = INFINITY, hi = -INFINITY;
-#pragma unroll 8
-    for (int s = 0; s < (int)q.splits; ++s) {
-        const float2 v = q.mm[(int64_t)s * n_in + j];
-        lo = fminf(lo, v.x); hi = fmaxf(hi, v.y);
-    }
+// A channel's extrema -> lo, range, 1 / range.
+struct QuantScale { double lo, ran, inv; };
+__device__ __forceinline__ QuantScale quant_scale(float lo, float hi) {
     const double ran = ((double)hi - (double)lo) / 255.0;              // matmul.py:31-33, as quantize_kernel
-    q.lo[j] = (double)lo; q.ran[j] = ran; q.inv[j] = 1.0 / ran;
+    return QuantScale{(double)lo, ran, 1.0 / ran};
 }
 
 // The correctly rounded quotient d / b from the correctly rounded reciprocal of b (Markstein: a quotient within one
@@ -216,10 +206,23 @@ __device__ __forceinline__ void quant_offsets(const float *__restrict__ W, int n
     constexpr int kChains = 4 * kChainChannels;
     double (*fr)[kChains][kChainStride] = reinterpret_cast<double (*)[kChains][kChainStride]>(lds);
     const int tiles = (n_out + kChainRows - 1) / kChainRows;
+    // a partial to a thread; the eight of a wavefront's channel meet in the wavefront, its four in LDS
+    static_assert(kMinMaxSplits == 256 / kChainChannels && kChainChannels == 8, "a partial to each thread");
+    float2 (*ends)[kChainChannels] = reinterpret_cast<float2 (*)[kChainChannels]>(reinterpret_cast<char *>(lds) + kChainLds);
+    {
+        const int64_t jm = min(group * kChainChannels + (int)(threadIdx.x & 7), n_in - 1), split = min((int64_t)threadIdx.x >> 3, q.splits - 1);
+        float2 e = q.mm[split * n_in + jm];
+#pragma unroll
+        for (int off = 8; off < 64; off <<= 1) { e.x = fminf(e.x, __shfl_xor(e.x, off, 64)); e.y = fmaxf(e.y, __shfl_xor(e.y, off, 64)); }
+        if ((threadIdx.x & 63) < kChainChannels) ends[threadIdx.x >> 6][threadIdx.x & 63] = e;
+    }
+    auto scale_of = [&](int c) {
+        return quant_scale(fminf(fminf(ends[0][c].x, ends[1][c].x), fminf(ends[2][c].x, ends[3][c].x)),
+                           fmaxf(fmaxf(ends[0][c].y, ends[1][c].y), fmaxf(ends[2][c].y, ends[3][c].y)));
+    };
     if (threadIdx.x >= 64) {
         const int pt = threadIdx.x - 64, ch = pt & 7, r = pt >> 3;          // rows r, r + 24, r + 48, r + 72 of a tile
         const int j = min(group * kChainChannels + ch, n_in - 1);
-        const double lo = q.lo[j], ran = q.ran[j], inv = q.inv[j];
         const float *col = W + (size_t)r * n_in + j;
         float x[kChainAhead][4];
         auto fetch = [&](float (&v)[4], int t) {
@@ -230,6 +233,9 @@ __device__ __forceinline__ void quant_offsets(const float *__restrict__ W, int n
         };
 #pragma unroll
         for (int d = 0; d < kChainAhead; ++d) fetch(x[d], d);
+        __syncthreads();                                                    // the extrema are there
+        const QuantScale sc = scale_of(ch);
+        const double lo = sc.lo, ran = sc.ran, inv = sc.inv;
         for (int t0 = 0; t0 < tiles; t0 += kChainAhead) {
 #pragma unroll
             for (int d = 0; d < kChainAhead; ++d) {
@@ -251,6 +257,7 @@ __device__ __forceinline__ void quant_offsets(const float *__restrict__ W, int n
     }
     const int lane = threadIdx.x, chain = lane & (kChains - 1);
     double sum = 0.0;
+    __syncthreads();                                                        // (the extrema)
     for (int t = 0; t < tiles; ++t) {
         __syncthreads();
         const double2 *v = reinterpret_cast<const double2 *>(fr[t & 1][chain]);
@@ -261,9 +268,10 @@ __device__ __forceinline__ void quant_offsets(const float *__restrict__ W, int n
     const double f0 = __shfl(sum, first, 64), f1 = __shfl(sum, first + 1, 64), f2 = __shfl(sum, first + 2, 64), f3 = __shfl(sum, first + 3, 64);
     const int j = group * kChainChannels + (lane >> 2);
     if (lane < kChains && (lane & 3) == 0 && j < n_in) {
-        const double fsum = (f0 + f1) + (f2 + f3), ran = q.ran[j];
-        offset[j] = q.lo[j] + (fsum / (double)n_out) * ran;                 // matmul.py:36-37
-        range[j] = (float)ran;                                              // matmul.py:39
+        const double fsum = (f0 + f1) + (f2 + f3);
+        const QuantScale sc = scale_of(lane >> 2);
+        offset[j] = sc.lo + (fsum / (double)n_out) * sc.ran;                // matmul.py:36-37
+        range[j] = (float)sc.ran;                                           // matmul.py:39
     }
 }
 
@@ -273,7 +281,7 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
                     uint8_t *__restrict__ codes, uint8_t *__restrict__ packed, uint8_t *__restrict__ packed16,
                     float *__restrict__ range, double *__restrict__ offset) {
     __shared__ __align__(16) uint32_t lds[2][8][256];
-    static_assert(kChainLds <= (int)sizeof(lds), "the fractions fit");
+    static_assert(kChainLds + 4 * kChainChannels * (int)sizeof(float2) <= (int)sizeof(lds), "the fractions and the extrema fit");
     if (blockIdx.x < q.chain_blocks) {
         // (workgroups go to the XCDs round robin: the four groups that share a 128-byte line of a row go to the same one)
         for (int64_t b = blockIdx.x; b * kChainChannels < n_in + 32 * kChainChannels; b += q.chain_blocks) {
@@ -287,20 +295,41 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
     const int64_t item = blockIdx.x - q.chain_blocks, col_block = item % q.col_blocks, part = item / q.col_blocks;
     const int cq = threadIdx.x & 31, rg = threadIdx.x >> 5;         // four channels, every eighth row
     const int64_t j0 = col_block * 128, j = j0 + 4 * cq;
-    double lo[4], ran[4], inv[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int64_t je = min(j + e, n_in - 1);
-        lo[e] = q.lo[je]; ran[e] = q.ran[je]; inv[e] = q.inv[je];
-    }
     const int64_t kbeg = part * q.part_rows, kend = min(kbeg + q.part_rows, n_out);
     const int64_t n_ct8 = (n_out + 7) >> 3, n_kb8 = (n_in + 127) >> 7, n_ct16 = (n_out + 15) >> 4, n_kb16 = (n_in + 63) >> 6;
     const bool words = (n_out & 3) == 0 && (reinterpret_cast<uintptr_t>(codes) & 3) == 0;
-    for (int64_t k0 = kbeg; k0 < kend; k0 += kEncRows) {
-        float4 x[8];
+    float4 x[8];
+    auto fetch = [&](int64_t k0) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[i] = weight4<VEC>(W + min(k0 + rg + 8 * i, n_out - 1) * n_in, j, n_in, 0.f);
-        if (k0 > kbeg) __syncthreads();                             // the tile before has been written out
+    };
+    double lo[4], ran[4], inv[4];
+    {
+        // the partials of a channel to two threads, requested ahead of the first rows
+        float2 (*ends)[128] = reinterpret_cast<float2 (*)[128]>(lds);
+        QuantScale *scales = reinterpret_cast<QuantScale *>(ends + 2);
+        const int c = threadIdx.x & 127, half = threadIdx.x >> 7;
+        const float2 *mm = q.mm + min(j0 + c, n_in - 1);
+        float2 part[kMinMaxSplits / 2];
+#pragma unroll
+        for (int i = 0; i < kMinMaxSplits / 2; ++i) part[i] = mm[min((int64_t)(2 * i + half), q.splits - 1) * n_in];
+        fetch(kbeg);
+        float2 e = part[0];
+#pragma unroll
+        for (int i = 1; i < kMinMaxSplits / 2; ++i) e = make_float2(fminf(e.x, part[i].x), fmaxf(e.y, part[i].y));
+        ends[half][c] = e;
+        __syncthreads();
+        if (half == 0) scales[c] = quant_scale(fminf(e.x, ends[1][c].x), fmaxf(e.y, ends[1][c].y));
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { const QuantScale sc = scales[4 * cq + i]; lo[i] = sc.lo; ran[i] = sc.ran; inv[i] = sc.inv; }
+        __syncthreads();                                            // before the codes take their place
+    }
+    for (int64_t k0 = kbeg; k0 < kend; k0 += kEncRows) {
+        if (k0 > kbeg) {
+            fetch(k0);
+            __syncthreads();                                        // the tile before has been written out
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const float xe[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
@@ -516,7 +545,6 @@ int rwkv_quantize_layouts(rwkv_stream_t stream, const float *weight, int64_t n_o
     const dim3 mg((unsigned)ceil_div(n_in, 256), (unsigned)q.splits), eg((unsigned)blocks);
     if (vec) hipLaunchKernelGGL(quant_minmax_kernel<true>, mg, dim3(256), 0, st, weight, n_out, n_in, q);
     else hipLaunchKernelGGL(quant_minmax_kernel<false>, mg, dim3(256), 0, st, weight, n_out, n_in, q);
-    hipLaunchKernelGGL(quant_scale_kernel, dim3((unsigned)ceil_div(n_in, 64)), dim3(64), 0, st, n_in, q);
     if (vec) hipLaunchKernelGGL(quant_encode_kernel<true>, eg, dim3(256), 0, st, weight, n_out, n_in, q, codes, packed, packed16, range, offset);
     else hipLaunchKernelGGL(quant_encode_kernel<false>, eg, dim3(256), 0, st, weight, n_out, n_in, q, codes, packed, packed16, range, offset);
     RWKV_CHECK_LAUNCH("quant_encode_kernel");
