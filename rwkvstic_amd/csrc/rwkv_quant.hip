@@ -195,7 +195,9 @@ __device__ __forceinline__ int slot16(int lane, int half) { return lane ^ (((lan
 
 // Offsets of eight channels.  The fractions of a channel are added in quantize_kernel's order, four serial float64 sums over
 // the rows k = 0, 1, 2, 3 (mod 4), so that both give the same bits (an offset that differs in its last bit moves every logit of
-// a model by rounding, and with it seeded texts).  Bound: that chain of n_out / 4 dependent additions.  Three wavefronts form
+// a model by rounding, and with it seeded texts).  Bound: not those n_out / 4 dependent additions (9 us of 10240 rows) but
+// the reading: of every 128-byte line a workgroup needs 32 bytes.  Alone these workgroups take 54 us of [10240 x 2560] and 30 of [2560 x 10240], the
+// encoding ones 26; 16 channels to a workgroup 127 and 74 with both (83 and 75 with 8), tiles of 192 rows 84 and 75.  Three wavefronts form
 // the fractions of 96 rows at a time and leave them in LDS, kChainAhead such tiles requested ahead; the fourth adds, a lane
 // per sum.  These workgroups run beside those that encode (launched first: they take longest).
 constexpr int kChainRows = 96, kChainAhead = 4, kChainStride = kChainRows / 4 + 2;     // (+ 2: 16-byte aligned, fewer bank conflicts)
@@ -204,6 +206,7 @@ constexpr int kChainLds = 2 * 4 * kChainChannels * kChainStride * 8;
 __device__ __forceinline__ void quant_offsets(const float *__restrict__ W, int n_out, int n_in, const QuantWs &q, int group, double *lds,
                                               float *__restrict__ range, double *__restrict__ offset) {
     constexpr int kChains = 4 * kChainChannels;
+    
     double (*fr)[kChains][kChainStride] = reinterpret_cast<double (*)[kChains][kChainStride]>(lds);
     const int tiles = (n_out + kChainRows - 1) / kChainRows;
     // a partial to a thread; the eight of a wavefront's channel meet in the wavefront, its four in LDS
@@ -223,13 +226,12 @@ __device__ __forceinline__ void quant_offsets(const float *__restrict__ W, int n
     if (threadIdx.x >= 64) {
         const int pt = threadIdx.x - 64, ch = pt & 7, r = pt >> 3;          // rows r, r + 24, r + 48, r + 72 of a tile
         const int j = min(group * kChainChannels + ch, n_in - 1);
-        const float *col = W + (size_t)r * n_in + j;
+        const float *col = W + j;
         float x[kChainAhead][4];
         auto fetch = [&](float (&v)[4], int t) {
             const int k = t * kChainRows;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)     // past the end: the last row again, counted as zero
-                v[e] = k + kChainRows <= n_out ? col[(size_t)(k + 24 * e) * n_in] : W[(size_t)min(k + 24 * e + r, n_out - 1) * n_in + j];
+            for (int e = 0; e < 4; ++e) v[e] = col[(size_t)min(k + 24 * e + r, n_out - 1) * n_in];      // past the end: the last row again, counted as zero
         };
 #pragma unroll
         for (int d = 0; d < kChainAhead; ++d) fetch(x[d], d);
@@ -241,12 +243,15 @@ __device__ __forceinline__ void quant_offsets(const float *__restrict__ W, int n
             for (int d = 0; d < kChainAhead; ++d) {
                 const int t = t0 + d;
                 if (t >= tiles) break;                                      // (uniform)
+                // (the four side by side, then what does not count: a branch around each would leave one chain of ten float64 operations at a time)
                 double f[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const double v = quotient((double)x[d][e] - lo, ran, inv);                      // matmul.py:32-34
-                    f[e] = ran > 0.0 && t * kChainRows + 24 * e + r < n_out ? v - trunc(v) : 0.0;   // matmul.py:35 (adding zero changes no bit)
+                    f[e] = v - trunc(v);                                                            // matmul.py:35
                 }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f[e] = ran > 0.0 && t * kChainRows + 24 * e + r < n_out ? f[e] : 0.0;   // (adding zero changes no bit)
                 fetch(x[d], t + kChainAhead);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) fr[t & 1][4 * ch + (r & 3)][(r >> 2) + 6 * e] = f[e];
@@ -295,6 +300,8 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
     const int64_t item = blockIdx.x - q.chain_blocks, col_block = item % q.col_blocks, part = item / q.col_blocks;
     const int cq = threadIdx.x & 31, rg = threadIdx.x >> 5;         // four channels, every eighth row
     const int64_t j0 = col_block * 128, j = j0 + 4 * cq;
+    // bytes of a thread's four channels: those there are, and those that have codes
+    uint32_t there = 0, coded = 0;
     const int64_t kbeg = part * q.part_rows, kend = min(kbeg + q.part_rows, n_out);
     const int64_t n_ct8 = (n_out + 7) >> 3, n_kb8 = (n_in + 127) >> 7, n_ct16 = (n_out + 15) >> 4, n_kb16 = (n_in + 63) >> 6;
     const bool words = (n_out & 3) == 0 && (reinterpret_cast<uintptr_t>(codes) & 3) == 0;
@@ -325,6 +332,12 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
         for (int i = 0; i < 4; ++i) { const QuantScale sc = scales[4 * cq + i]; lo[i] = sc.lo; ran[i] = sc.ran; inv[i] = sc.inv; }
         __syncthreads();                                            // before the codes take their place
     }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (j + e < n_in) {
+            there |= 0x80u << (8 * e);
+            if (ran[e] > 0.0) coded |= 0xffu << (8 * e);
+        }
     for (int64_t k0 = kbeg; k0 < kend; k0 += kEncRows) {
         if (k0 > kbeg) {
             fetch(k0);
@@ -334,17 +347,16 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
         for (int i = 0; i < 8; ++i) {
             const float xe[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
             const bool row = k0 + rg + 8 * i < n_out;
-            uint32_t c4 = 0, live = 0;
+            // (all four, whatever counts of them: without branches their chains of float64 operations run side by side.  A layer of width
+            // 2560 291 -> 283 us, with the same in quant_offsets)
+            uint32_t c4 = 0;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if (row && j + e < n_in) {
-                    live |= 0x80u << (8 * e);
-                    if (ran[e] > 0.0) {
-                        const double v = quotient((double)xe[e] - lo[e], ran[e], inv[e]);   // matmul.py:32-34
-                        c4 |= (uint32_t)(uint8_t)(int)v << (8 * e);                         // matmul.py:21
-                    }
-                }
+                const double v = quotient((double)xe[e] - lo[e], ran[e], inv[e]);           // matmul.py:32-34
+                c4 |= (uint32_t)(uint8_t)(int)v << (8 * e);                                 // matmul.py:21
             }
+            c4 &= row ? coded : 0u;
+            const uint32_t live = row ? there : 0u;
             // P8: block i of the tile, lane 8 s + column, dword m, with channel 32 m + 4 s + e of the block; M16: blocks
             // (i / 2, half of the 128 channels), lane 16 g + column, dword q, code - 128 with padding 0.  In LDS the
             // columns of a group are permuted (slot8, slot16) so that the 64 stores of a wavefront hit 64 banks.
