@@ -588,7 +588,7 @@ bool rows_supported(const rwkv_model *m) {
 // R rows through every layer.  sequence: rows are consecutive tokens of one sequence whose state is
 // `state` [L,5,C]; otherwise row b is one token of sequence b with state at state + b * state_stride.
 // tail: what is left to the LayerNorm kernel in front of the head: its input x, the last layer's ffn value product where it
-// is still pending (batch rows), and the last shift rows to be committed; or to the sequence's next pass.
+// is still pending, and the last shift rows to be committed; or to the sequence's next pass.
 struct RowsTailWork { const double *x = nullptr; RowsFew few{}; };
 int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R, bool sequence, double *state,
                 int64_t state_stride, const RowsWs &w, RowsTailWork &tail) {
@@ -612,6 +612,11 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     // A pending product's totals and gate are written by later launches only.
     const bool stream = weights_streamed(d.n_layer, d.n_embd, d.n_ffn, d.n_vocab);
     const bool defer = !sequence && R < kRowsDeferMax;
+    // The residual updates of a short prompt of a narrow model too, although a row of a sequence adds up the slices of the row before it as
+    // well, whose LayerNorm it needs.  Us a prompt, a launch for the sums / handed on: 12 layers of 512, 40 and 127 tokens 679, 743 / 653, 720; 24 of
+    // 1024, 77 and 127 1741, 1840 / 1695, 1788; 12 of 1536, 77 and 100 1074, 1135 / 1056, 1142; 12 of 2048, 64 and 77 1151, 1174 / 1136, 1186; 12 of
+    // 2560, 32 and 127 1067, 1502 / 1076, 1556; 8 of 4096, 32 1004 / 1036.
+    const bool hand_on = sequence ? C <= 2048 && R < kRowsDeferMax && R * C <= (1 << 17) : defer;
     RowsDeferred dk[3];
     // The LayerNorm kernels leave the new shift rows aside, and each commits what the one before it left.
     const bool aside = R < kRowsDeferMax || sequence;
@@ -643,7 +648,7 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
                           sl + 2 * (size_t)C, state_stride, reinterpret_cast<float *>(w.att), defer ? dk : nullptr));
         RWKV_TRY(rows_quant(st, R, C, w.att, true, L.att_o.range, L.att_o.offset, w.q[0], (double *)w.tot));    // att and h: float32 arrays
         const RowsProduct po = {w.q[0], L.att_o.packed16, x, stream};
-        RWKV_TRY(rows_products(st, 1, &po, w.tot, R, C, C, ROW_ADD, nullptr, defer ? &few.add : nullptr));
+        RWKV_TRY(rows_products(st, 1, &po, w.tot, R, C, C, ROW_ADD, nullptr, hand_on ? &few.add : nullptr, sequence));
         // ChannelMix (block.py:82-100)
         const float *rg2[2] = {L.ffn_k.range, L.ffn_r.range};
         const double *of2[2] = {L.ffn_k.offset, L.ffn_r.offset};
@@ -655,7 +660,7 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
         RWKV_TRY(rows_ffn_key_receptance(st, sequence, pfk, pfr, w.tot, R, C, F, L.ffn_v.range, L.ffn_v.offset, w.qv));
         const RowsProduct pfv = {w.qv, L.ffn_v.packed16, x, stream};
         // (the ffn receptance stays in the kvr slab and the totals untouched until the next LayerNorm kernel has run)
-        RWKV_TRY(rows_products(st, 1, &pfv, w.tot, R, F, C, ROW_GATE_ADD, kvr32, defer ? &few.add : nullptr));
+        RWKV_TRY(rows_products(st, 1, &pfv, w.tot, R, F, C, ROW_GATE_ADD, kvr32, hand_on ? &few.add : nullptr, sequence));
     }
     few.x_out = few.shift_out = nullptr;
     tail = RowsTailWork{x, few};
@@ -690,6 +695,12 @@ int rows_sequence(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t 
         int rc = rows_layers(m, st, tokens + t0, R, true, state, 0, rw, tail);
         if (rc) return rc;
         if (t0 + R == T) {
+            // (of a product that is pending, the last row alone)
+            RowsDeferred &add = tail.few.add;
+            if (add.tot) {
+                add.tot += (size_t)(R - 1) * add.ldd; add.S += R - 1; add.qs += R - 1; add.zp += R - 1;
+                if (add.gate) add.gate += (size_t)(R - 1) * C;
+            }
             // ln_out and the head on the last row (opt.py:72-74), as a one-row product with integer sums
             const rwkv_model_desc &d = m->d;
             const float *rg[1] = {d.head.range};

@@ -26,7 +26,7 @@ constexpr int kRowsMaxProducts = 3;     // products of equal shape and tail that
 // A product whose contraction was split, handed on unfinished: its consumer (the LayerNorm kernel for the two
 // residual updates, the WKV kernel for k, v, r) adds the slices of integer totals up itself and applies the tail,
 // which saves the launch that would otherwise do only that.  tot == nullptr: nothing is pending (the product was not
-// split and its epilogue applied the tail).  Only for batches of fewer than kRowsDeferMax independent rows.
+// split and its epilogue applied the tail).  Only for fewer than kRowsDeferMax rows; k, v, r only of independent ones.
 struct RowsDeferred {
     const long long *tot;   // [slices][slice] totals of this product; element (t, j) at t * ldd + j
     size_t slice;
@@ -40,7 +40,7 @@ constexpr int kRowsDeferSlices = 6;     // a contraction split further than this
 // What the LayerNorm kernel of fewer than kRowsDeferMax rows does besides (several workgroups share a row there, and none
 // may overwrite what another reads); of a sequence of any length, the shift rows (row 0 reads what the last row replaces).
 struct RowsFew {
-    RowsDeferred add;           // a residual update of x still pending (tot null: none); batch rows only; with mixes, its S, qs and zp are no output's
+    RowsDeferred add;           // a residual update of x still pending (tot null: none); with mixes, its S, qs and zp are no output's
     double *x_out;              // where the updated x goes: another buffer than x (null: it is not needed)
     double *shift_out;          // [R, C], of a sequence [C]: the newest shift rows, instead of the state
     const double *commit_src;   // shift rows left by the launch before (null: none) ...
@@ -73,7 +73,7 @@ int rows_quant(hipStream_t st, int64_t R, int64_t K, const void *in, bool in_f32
 // and described here (tot and the operand's row constants must stay untouched until that kernel has run); entries of
 // products that were finished here get tot = nullptr.
 int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, int64_t R, int64_t K, int64_t N, int op,
-                  const float *gate, RowsDeferred *defer = nullptr);
+                  const float *gate, RowsDeferred *defer = nullptr, bool sequence = false);
 // ffn key (relu squared) [R, C] x [C, F] and ffn receptance [R, C] x [C, C], both stored float32, and the key's rows quantised
 // for the ffn value matrix (range, offset -> out); tot as for either.
 int rows_ffn_key_receptance(hipStream_t st, bool sequence, const RowsProduct &k, const RowsProduct &r, long long *tot, int64_t R, int64_t C, int64_t F,

@@ -224,7 +224,7 @@ __device__ __forceinline__ void with_slices(int slices, F &&f) {
 struct LnQuantArgs {
     int C, R, sequence;
     const double *x;            // [R, C]
-    RowsDeferred add;           // batch rows, few-row form: x += this product first, stored to x_out (tot null: none)
+    RowsDeferred add;           // few-row form: x += this product first (and the row before, whose LayerNorm is needed), stored to x_out (tot null: none)
     double *x_out;              // null: nobody reads x again
     double *shift_out;          // few-row form of batch rows, [R, C]: the newest xy rows go here instead of to shift_dst (null: to shift_dst)
     const double *commit_src;   // few-row form or sequence: [R, C] rows (sequence: one) an earlier launch left aside (null: none) ...
@@ -377,7 +377,10 @@ __global__ void __launch_bounds__(kLnRowThreads) rows_ln_mix_quant_row_kernel(co
         // (block.py:95-100), as rows_finish_kernel would have done.
         const int c = 4 * tid, step = 4 * nt;
         double *xo = a.x_out && m == 0 ? a.x_out + (size_t)t * C : nullptr;
-        with_slices(a.add.slices, [&](auto count) { add_pending<NSEG, decltype(count)::value>(a.add, t, c, step, C, xo, xv); });
+        with_slices(a.add.slices, [&](auto count) {
+            add_pending<NSEG, decltype(count)::value>(a.add, t, c, step, C, xo, xv);
+            if (NSEG == 1 && need_prev) add_pending<NSEG, decltype(count)::value>(a.add, t - 1, c, step, C, nullptr, pv);
+        });
     }
     double s[2] = {0.0, 0.0};
 #pragma unroll
@@ -1806,14 +1809,14 @@ static bool skinny_cut(int64_t NT, int64_t KB, int n) { return ceil_div(NT, kSki
 // the two that then wait for it.  (So no power of two: 40 column blocks of 5120 channels fill 240 compute units in six slices, 160 in four.)  Us a
 // step of 32 sequences before (the power of two that brings 128 workgroups, up to eight) / now: 24 layers of 1024 1308 / 1220, 12 of 2560 1096 /
 // 1071, 8 of 4096 1023 / 1011, 8 of 5120 1289 / 1254; of 16, with four M-tiles (gemm8_skinny_kernel), 905 / 848 of 4096 and 1106 / 1031 of 5120.
-static int skinny_split(int64_t MT, int64_t NT, int64_t KB, int n, bool handed_on) {
+static int skinny_split(int64_t MT, int64_t NT, int64_t KB, int n, int readers) {
     if (!skinny_cut(NT, KB, n)) return 1;
     int best = 2;
     int64_t least = INT64_MAX;
     for (int s = 2; s <= kMaxSplit && KB >= 8 * s; ++s) {
-        const bool sum = handed_on && s <= kRowsDeferSlices;
+        const bool sum = readers && s <= kRowsDeferSlices;
         const int64_t cost = ceil_div(ceil_div(NT, kSkinnyNT) * n * s, 256) * (kSkinnyNT + (MT <= 4 ? 4 : 8)) * ceil_div(KB, s) +
-                             (sum && n > 1 ? 8 * s : sum ? 32 + (2 * s + 1) * NT / 16 : 420 + 30 * s * n);
+                             (sum && n > 1 ? 8 * s : sum ? 32 + readers * (2 * s + 1) * NT / 16 : 420 + 30 * s * n);
         if (cost < least) { least = cost; best = s; }
     }
     return best;
@@ -1825,16 +1828,16 @@ static int64_t general_cost(int64_t w4) {
     return (w4 / 512) * 64 + (rem == 0 ? 0 : rem <= 256 ? 32 : 64);
 }
 static bool general_wide(int64_t w4, int64_t w5) { return w4 >= 256 && kGemmWideNum * ceil_div(w5, 256) * 40 < kGemmWideDen * general_cost(w4); }
-static int vec_split(int64_t MT, int64_t NT, int64_t KB);
-// handed_on: the consumer adds up the slices of a contraction of at most 8 rows.
-static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n, bool handed_on = false) {
+static int vec_split(int64_t MT, int64_t NT, int64_t KB, int readers);
+// readers: who adds up the slices: 0 a launch of their own, 1 the consumer (a row of a batch), 2 the consumer, of each row and of the one before it.
+static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n, int readers = 0) {
     ProductPlan p;
     p.split = 1;
     if (vec_rows(MT, NT * n, KB)) {
         // few rows: whole contractions, as long as a digit's sum of them stays inside int32 (2^20 per block)
         p.kind = PLAN_VEC; p.gx = (int)NT; p.gy = 1;
         while (ceil_div(KB, p.split) > 1024 && p.split < kMaxSplit) p.split *= 2;
-        if (handed_on && MT <= kVecMT && n == 1 && p.split == 1) p.split = vec_split(MT, NT, KB);
+        if (readers && MT <= kVecMT && n == 1 && p.split == 1) p.split = vec_split(MT, NT, KB, readers);
         return p;
     }
     p.gy = (int)ceil_div(MT, 16);
@@ -1842,7 +1845,7 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n, bool
     if (p.kind == PLAN_GENERAL && general_wide(ceil_div(NT, kGemmNT) * p.gy * n, ceil_div(NT, kGemmWideNT) * p.gy * n)) p.kind = PLAN_WIDE;
     p.gx = (int)ceil_div(NT, p.kind == PLAN_SKINNY ? kSkinnyNT : p.kind == PLAN_WIDE ? kGemmWideNT : kGemmNT);
     // Split the contraction until the grid has a few workgroups per compute unit.
-    if (p.kind == PLAN_SKINNY) p.split = skinny_split(MT, NT, KB, n, handed_on);
+    if (p.kind == PLAN_SKINNY) p.split = skinny_split(MT, NT, KB, n, readers);
     else
         while ((int64_t)p.gx * p.gy * n * p.split < kGemmFillWgs && KB / (p.split * 2) >= 8 && p.split < kMaxSplit) p.split *= 2;
     // a long contraction on a grid still below the device: one split more (two slices at most)
@@ -1910,7 +1913,7 @@ static VecShape vec_shape(int64_t tiles, int64_t KB, int MT) {
 // (2560 channels 8.7 / 7.6 / 6.8 / 7.3) and 4096 channels gain no more than that costs (step of 8 layers 767 us both ways).  Us a step of 8
 // sequences, before (one tile to every workgroup of up to 320) / whole contractions / this: 24 layers of 1024 970 / 962 / 925, 12 of 1536
 // 589 / 579 / 560, 8 of 2048 453 / 447 / 439, 12 of 2560 764 / 744 / 722, 4 of 5120 566 / 519 / 497; all with the same bits.
-static int vec_split(int64_t MT, int64_t NT, int64_t KB) {
+static int vec_split(int64_t MT, int64_t NT, int64_t KB, int readers) {
     auto draw = [&](int s) {
         const int64_t kb = ceil_div(KB, s);
         return vec_draw(NT * s, vec_shape(NT * s, kb, (int)MT).ntw, (int)MT) * kb;
@@ -1918,7 +1921,7 @@ static int vec_split(int64_t MT, int64_t NT, int64_t KB) {
     int best = 1;
     int64_t least = draw(1) * 7 / 10;
     for (int s = 2; s <= kRowsDeferSlices; ++s) {
-        const int64_t cost = draw(s) + 32 + (2 * s + 1) * NT / 16;
+        const int64_t cost = draw(s) + 32 + readers * (2 * s + 1) * NT / 16;
         if (cost < least) { least = cost; best = s; }
     }
     return best;
@@ -2047,8 +2050,10 @@ int rows_ln_mix_quant(hipStream_t st, int n_mix, int64_t R, int C, bool sequence
     a.C = C; a.R = (int)R; a.sequence = sequence ? 1 : 0; a.x = x; a.ln_w = ln_w; a.ln_b = ln_b; a.mu = mu;
     a.add.tot = nullptr; a.x_out = nullptr; a.shift_out = nullptr; a.commit_src = nullptr; a.commit_dst = nullptr;
     if (few) {
-        if (few->add.tot && (sequence || (few->add.op != ROW_ADD && few->add.op != ROW_GATE_ADD) || few->x_out == x))
-            return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: a pending product needs batch rows, a residual tail and another buffer for the new x");
+        if (few->add.tot && ((few->add.op != ROW_ADD && few->add.op != ROW_GATE_ADD) || few->x_out == x))
+            return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: a pending product needs a residual tail and another buffer for the new x");
+        if (sequence && few->add.tot && C > 4 * kLnRowThreads)          // (the registers of wider rows do not hold the row before as well)
+            return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: a pending product of a sequence needs rows of at most %d channels", 4 * kLnRowThreads);
         if (R >= kRowsDeferMax && (few->add.tot || (!sequence && (few->shift_out || few->commit_src))))
             return set_error(RWKV_ERR_ARG, "rows_ln_mix_quant: pending work needs fewer than %d rows", (int)kRowsDeferMax);
         a.add = few->add; a.x_out = few->x_out; a.commit_src = few->commit_src; a.commit_dst = few->commit_dst;
@@ -2179,7 +2184,7 @@ static int launch_general(hipStream_t st, GemmArgs &g, bool wide, int gx, bool s
 }
 
 int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, int64_t R, int64_t K, int64_t N, int op,
-                  const float *gate, RowsDeferred *defer) {
+                  const float *gate, RowsDeferred *defer, bool sequence) {
     if (K % 64 != 0) return set_error(RWKV_ERR_SIZE, "rows_products: contraction length %lld is not a multiple of 64",
                                       (long long)K);
     if (n < 1 || n > kRowsMaxProducts) return set_error(RWKV_ERR_ARG, "rows_products: %d products in one launch", n);
@@ -2194,7 +2199,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     g.tot = tot;
     g.MT = (int)ceil_div(R, 4); g.NT = (int)ceil_div(N, 16); g.KB = (int)(K / 64); g.ldd = g.NT * 16;
     g.R = (int)R; g.N = (int)N; g.gate = gate;
-    const ProductPlan pl = plan_products(g.MT, g.NT, g.KB, n, defer && R < kRowsDeferMax);
+    const ProductPlan pl = plan_products(g.MT, g.NT, g.KB, n, defer && R < kRowsDeferMax ? (sequence ? 2 : 1) : 0);
     const int split = pl.split;
     g.kb_per_split = (int)ceil_div(g.KB, split);
     g.split = split;
@@ -2221,7 +2226,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     if (split == 1) return RWKV_OK;     // the tail was applied in the product's epilogue
     if (defer && R < kRowsDeferMax && split <= kRowsDeferSlices) {   // the consumer adds the slices up
         for (int m = 0; m < n; ++m)
-            defer[m] = RowsDeferred{tot + (size_t)m * split * g.slice, g.slice, split, g.ldd, op, g.apart != 0, pl.kind == PLAN_VEC, p[m].a.S, p[m].a.qs, p[m].a.zp, gate};
+            defer[m] = RowsDeferred{tot + (size_t)m * split * g.slice, g.slice, split, g.ldd, op, g.apart != 0, pl.kind == PLAN_VEC || sequence, p[m].a.S, p[m].a.qs, p[m].a.zp, gate};
         return RWKV_OK;
     }
 

@@ -575,6 +575,23 @@ def test_batch_steps_in_slices_that_fill_the_device_match_single_steps(C, F, B):
     test_batch_steps_of_ragged_and_wide_rows_match_single_steps(C, F, B)
 
 
+# prompts on both sides of the line up to which the residual updates are handed on in slices (2048 channels, 2^17 values), of rows that few-row,
+# skinny and general products serve; the second pass of a long prompt.  Against the same tokens one at a time.
+@pytest.mark.parametrize("C,T", [(1024, 8), (1024, 33), (1024, 127), (1024, 128), (2048, 20), (2048, 64), (2048, 65), (2112, 40), (512, 1024 + 40)])
+def test_short_prompts_match_token_by_token(C, T):
+    from rwkvstic_amd.model import HipRWKV
+    _say(f"prompt of {T} at C={C}")
+    m = HipRWKV(synth.iter_tensors(2, C, 4 * C, 100, seed=C + T, device="cuda", ln="random"))
+    toks = synth.random_tokens(T, V=100, seed=T)
+    l0, s0 = m.forward(toks.cuda(), m.emptyState.clone())
+    s1 = m.emptyState.clone()
+    for t in toks.tolist():
+        l1, s1 = m.forward([t], s1)
+    assert float((l0 - l1).norm() / l1.norm()) < 2e-6
+    for row in range(5):
+        assert float((s0[:, row] - s1[:, row]).norm() / s1[:, row].norm()) < 2e-6, row
+
+
 def test_rwkv_shell_loads_checkpoint_file_and_generates(tmp_path, tiny):
     """RWKV(path) -> RWKVMaster surface (load.py:18,42-47; rwkvMaster.py:28-105) over the HIP model."""
     from rwkvstic_amd.master import RWKV, greedy
