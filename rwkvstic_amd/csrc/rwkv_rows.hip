@@ -1132,55 +1132,64 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         frag[B][MT + wave][lane] = F.v2; frag[B][MT + 4 + wave][lane] = F.v3;                        \
     } while (0)
     // (same step as gemm8_body: the next block is parked, and its registers refilled, piece by piece between
-    // this block's groups of matrix instructions)
+    // this block's groups of matrix instructions.  With one wavefront to a SIMD nothing else hides the first LDS reads of a step: the last
+    // groups of the step before are multiplied behind its barrier.  32 sequences, before / now: 8 layers of 5120 1209 / 1179 us a step, of 4096 1010 /
+    // 986, 12 of 2560 1060 / 1050, 24 of 1024 1208 / 1182; more of them change nothing, eight blocks ahead instead of six lose 1 %, eight
+    // wavefronts of half the rows gain less than 1 % with 32 rows and lose as much with 16)
 #define RWKV_SKINNY_MOVE(FN, I, V, B, O)                                                             \
     { frag[B][((I) < 2 ? 0 : MT - 8) + wave + 4 * (I)][lane] = FN.V; FN.V = (I) < 2 ? src[I][O] : ldw<STREAM>(src[I] + (O)); }
-#define RWKV_SKINNY_STEP(FN, K)                                                                      \
+#define RWKV_SKINNY_GROUP(I, A, B)                                                                   \
+    _Pragma("unroll") for (int j = 0; j < kSkinnyGN; ++j)                                            \
+        acc[I][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, (B)[j], acc[I][j], 0, 0, 0);
+#define RWKV_SKINNY_STEP(FN, K, FIRST)                                                               \
     {                                                                                                \
         const int buf_ = (K) & 1;                                                                    \
         const size_t on_ = (size_t)((K) + 1 + kSkinnyAhead < nk ? (K) + 1 + kSkinnyAhead : nk - 1) * 64; \
         lds_barrier();                                                                               \
-        v4i Bv_[kSkinnyGN];                                                                          \
+        v4i Bv_[kSkinnyGN], Av_[MT];                                                                 \
         _Pragma("unroll") for (int j = 0; j < kSkinnyGN; ++j)                                        \
             Bv_[j] = frag[buf_][MT + wave * kSkinnyGN + j][lane];                                    \
-        v4i Av_ = frag[buf_][0][lane];                                                               \
-        _Pragma("unroll") for (int i = 0; i < MT; ++i) {                                             \
-            const v4i An_ = frag[buf_][i + 1 < MT ? i + 1 : i][lane];                                \
-            if (i == 0) RWKV_SKINNY_MOVE(FN, 0, v0, buf_ ^ 1, on_)                                   \
-            if (MT == 8 && i == 2) RWKV_SKINNY_MOVE(FN, 1, v1, buf_ ^ 1, on_)                        \
-            if (i == MT / 2) RWKV_SKINNY_MOVE(FN, 2, v2, buf_ ^ 1, on_)                              \
-            if (i == MT - (MT == 8 ? 2 : 1)) RWKV_SKINNY_MOVE(FN, 3, v3, buf_ ^ 1, on_)              \
-            _Pragma("unroll") for (int j = 0; j < kSkinnyGN; ++j)                                    \
-                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(Av_, Bv_[j], acc[i][j], 0, 0, 0);  \
-            Av_ = An_;                                                                               \
+        Av_[0] = frag[buf_][0][lane]; Av_[1] = frag[buf_][1][lane];                                  \
+        __builtin_amdgcn_sched_barrier(0);                                                           \
+        RWKV_SKINNY_MOVE(FN, 0, v0, buf_ ^ 1, on_)                                                   \
+        if (!(FIRST)) { _Pragma("unroll") for (int d = 0; d < kLate; ++d) RWKV_SKINNY_GROUP(MT - kLate + d, Al[d], Bl) }  \
+        __builtin_amdgcn_sched_barrier(0);                                                           \
+        _Pragma("unroll") for (int i = 0; i < MT - kLate; ++i) {                                     \
+            if (i + 2 < MT) Av_[i + 2] = frag[buf_][i + 2][lane];                                    \
+            if (i + 2 == MT - kLate + 1 && kLate > 1) Av_[MT - 1] = frag[buf_][MT - 1][lane];        \
+            if (MT == 8 && i == 0) RWKV_SKINNY_MOVE(FN, 1, v1, buf_ ^ 1, on_)                        \
+            if (i == (MT == 8 ? 2 : 0)) RWKV_SKINNY_MOVE(FN, 2, v2, buf_ ^ 1, on_)                   \
+            if (i == (MT == 8 ? 4 : 1)) RWKV_SKINNY_MOVE(FN, 3, v3, buf_ ^ 1, on_)                   \
+            RWKV_SKINNY_GROUP(i, Av_[i], Bv_)                                                        \
+            __builtin_amdgcn_sched_barrier(0);                                                       \
         }                                                                                            \
-        __builtin_amdgcn_sched_group_barrier(0x100, kSkinnyGN + 2, 0);                               \
-        _Pragma("unroll") for (int i = 0; i < MT; ++i) {                                             \
-            const bool moves_ = MT == 8 ? i % 2 == 0 : i != 1;                                       \
-            if (moves_) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);                           \
-            __builtin_amdgcn_sched_group_barrier(0x008, kSkinnyGN, 0);                               \
-            if (i + 2 < MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                       \
-            if (moves_) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                           \
-        }                                                                                            \
+        _Pragma("unroll") for (int d = 0; d < kLate; ++d) Al[d] = Av_[MT - kLate + d];               \
+        _Pragma("unroll") for (int j = 0; j < kSkinnyGN; ++j) Bl[j] = Bv_[j];                        \
     }
+    constexpr int kLate = MT == 8 ? 2 : 1;
+    v4i Al[kLate], Bl[kSkinnyGN];
     RWKV_SKINNY_FETCH(fly0, 0); RWKV_SKINNY_FETCH(fly1, 1); RWKV_SKINNY_FETCH(fly2, 2);
     RWKV_SKINNY_FETCH(fly3, 3); RWKV_SKINNY_FETCH(fly4, 4); RWKV_SKINNY_FETCH(fly5, 5);
     RWKV_SKINNY_PARK(fly0, 0);
     RWKV_SKINNY_FETCH(fly0, kSkinnyAhead);
-    int k0 = 0;
+    RWKV_SKINNY_STEP(fly1, 0, true)
+    int k0 = 1;
     for (; k0 + kSkinnyAhead <= nk; k0 += kSkinnyAhead) {      // whole rounds: no branch between the steps
-        RWKV_SKINNY_STEP(fly1, k0)
-        RWKV_SKINNY_STEP(fly2, k0 + 1)
-        RWKV_SKINNY_STEP(fly3, k0 + 2)
-        RWKV_SKINNY_STEP(fly4, k0 + 3)
-        RWKV_SKINNY_STEP(fly5, k0 + 4)
-        RWKV_SKINNY_STEP(fly0, k0 + 5)
+        RWKV_SKINNY_STEP(fly2, k0, false)
+        RWKV_SKINNY_STEP(fly3, k0 + 1, false)
+        RWKV_SKINNY_STEP(fly4, k0 + 2, false)
+        RWKV_SKINNY_STEP(fly5, k0 + 3, false)
+        RWKV_SKINNY_STEP(fly0, k0 + 4, false)
+        RWKV_SKINNY_STEP(fly1, k0 + 5, false)
     }
-    if (k0 < nk) RWKV_SKINNY_STEP(fly1, k0)
-    if (k0 + 1 < nk) RWKV_SKINNY_STEP(fly2, k0 + 1)
-    if (k0 + 2 < nk) RWKV_SKINNY_STEP(fly3, k0 + 2)
-    if (k0 + 3 < nk) RWKV_SKINNY_STEP(fly4, k0 + 3)
-    if (k0 + 4 < nk) RWKV_SKINNY_STEP(fly5, k0 + 4)
+    if (k0 < nk) RWKV_SKINNY_STEP(fly2, k0, false)
+    if (k0 + 1 < nk) RWKV_SKINNY_STEP(fly3, k0 + 1, false)
+    if (k0 + 2 < nk) RWKV_SKINNY_STEP(fly4, k0 + 2, false)
+    if (k0 + 3 < nk) RWKV_SKINNY_STEP(fly5, k0 + 3, false)
+    if (k0 + 4 < nk) RWKV_SKINNY_STEP(fly0, k0 + 4, false)
+#pragma unroll
+    for (int d = 0; d < kLate; ++d) RWKV_SKINNY_GROUP(MT - kLate + d, Al[d], Bl)
+#undef RWKV_SKINNY_GROUP
 #undef RWKV_SKINNY_STEP
 #undef RWKV_SKINNY_MOVE
 #undef RWKV_SKINNY_PARK
