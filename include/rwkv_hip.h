@@ -367,7 +367,7 @@ int rwkv_gemm8(rwkv_stream_t stream, int64_t T, int64_t n_in, int64_t n_out,
  * n_products (1..3) products x[T, n_in] x matrix[n_in, n_out] sharing a launch
  * (k, v, r do; matmul.py:86-94): plan = {kernel variant (0: at most 8 rows, or up to 32 of a
  * small matrix, 1: 9-32
- * rows, 2: 64 x 128 tiles, 3: 64 x 160 tiles), grid x, grid y, splits of the
+ * rows, 2: 64 x 128 tiles, 3: 64 x 160 or 64 x 80 tiles), grid x, grid y, splits of the
  * contraction}, and in *tot_bytes_per_product the bytes of integer totals the
  * workspace reserves per product.  Host-only: launches nothing. */
 int rwkv_gemm8_plan(int64_t T, int64_t n_in, int64_t n_out, int n_products,

@@ -838,7 +838,7 @@ struct GemmCols { int NT, N, tail; bool apart = false; };
 template <bool STREAM>
 __device__ __forceinline__ v4i ldw(const v4i *p) { return STREAM ? __builtin_nontemporal_load(p) : *p; }
 
-constexpr int kGemmNT = 8, kGemmWideNT = 10;     // N-tiles per workgroup (two wavefronts side by side)
+constexpr int kGemmNT = 8, kGemmWideNT = 10, kGemmNarrowNT = 5;     // N-tiles per workgroup
 constexpr int kWideRing = 4;                     // LDS buffers of the 64 x 160 variant
 
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every global load
@@ -941,15 +941,16 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, const GemmCols 
     }
 }
 
-// One workgroup of the product: 64 tokens x 32*GN columns, 2*WM wavefronts as WM x 2, each 16/WM M-tiles x GN
+// One workgroup of the product: 64 tokens x 16*WN*GN columns, WM*WN wavefronts as WM x WN, each 16/WM M-tiles x GN
 // N-tiles, RING LDS buffers.  <4, 4, 3> is the general shape (8 wavefronts of 4 x 4 tiles, two workgroups per
 // compute unit); <5, 4, 4> (4 x 5 tiles, one workgroup per compute unit) is used where it turns a grid of 1.25
-// workgroups per compute unit into exactly one (2560 columns: 16 column blocks instead of 20).
-template <int GN, int WM, int RING, bool STREAM>
+// workgroups per compute unit into exactly one (2560 columns: 16 column blocks instead of 20).  <5, 8, 1, 4> (64 x 80: eight wavefronts of 2 x 5
+// tiles) serves grids that leave compute units idle (general_narrow).
+template <int GN, int WM, int WN, int RING, bool STREAM>
 __device__ __forceinline__ void gemm8_body(const GemmArgs a) {
     // Both operands of a contraction block are fetched once per workgroup into LDS and read from there by
     // the wavefronts that need each fragment (one barrier per block).
-    constexpr int kGN = GN, kNT = 2 * GN, kGM = 16 / WM, kNW = 2 * WM;
+    constexpr int kGN = GN, kNT = WN * GN, kGM = 16 / WM, kNW = WN * WM;
     constexpr int kGemmFrags = 16 + kNT;                // fragments of one contraction block: 16 M-tiles of digits, kNT N-tiles of weights
     constexpr int kGemmLoads = (kGemmFrags + kNW - 1) / kNW;    // per thread and contraction block (wave w fetches fragments w, w + kNW, ...)
     constexpr int kSlots = kNW * kGemmLoads, kGemmRing = RING;
@@ -1061,10 +1062,13 @@ __device__ __forceinline__ void gemm8_body(const GemmArgs a) {
 
 template <bool STREAM>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) gemm8_kernel(const GemmArgs a) {
-    gemm8_body<4, 4, 3, STREAM>(a);
+    gemm8_body<4, 4, 2, 3, STREAM>(a);
 }
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) gemm8_wide_kernel(const GemmArgs a) {
-    gemm8_body<5, 4, kWideRing, false>(a);
+    gemm8_body<5, 4, 2, kWideRing, false>(a);
+}
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 4))) gemm8_narrow_kernel(const GemmArgs a) {
+    gemm8_body<5, 8, 1, kWideRing, false>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -1797,7 +1801,7 @@ constexpr int kGemmFillWgs = 96;         // larger products: split until the gri
 // Which kernel serves n products of MT row tiles x NT column tiles over KB contraction blocks, its grid and
 // the number of contraction splits.  The ONE place these are decided: the launches and the sizing of the
 // totals buffer both call it, so the buffer always holds every slice the kernel writes.
-enum { PLAN_VEC = 0, PLAN_SKINNY, PLAN_GENERAL, PLAN_WIDE };
+enum { PLAN_VEC = 0, PLAN_SKINNY, PLAN_GENERAL, PLAN_WIDE, PLAN_NARROW };
 struct ProductPlan { int kind, gx, gy, split; };
 // Which products of 9 to 32 rows go through gemv16_kernel.  Every workgroup of it reads the digits of all rows, gemm8_skinny_kernel
 // shares them between four wavefronts of eight tiles but needs slices of the contraction, and launches that add them up, to fill
@@ -1836,9 +1840,20 @@ static int64_t general_cost(int64_t w4) {
     const int64_t rem = w4 % 512;
     return (w4 / 512) * 64 + (rem == 0 ? 0 : rem <= 256 ? 32 : 64);
 }
+// (a narrow workgroup: 20, but it waits for its LDS reads, 0.7 to a matrix instruction)
+constexpr int kGemmNarrowCost = 27;
 static bool general_wide(int64_t w4, int64_t w5) { return w4 >= 256 && kGemmWideNum * ceil_div(w5, 256) * 40 < kGemmWideDen * general_cost(w4); }
 static int vec_split(int64_t MT, int64_t NT, int64_t KB, int readers);
 // readers: who adds up the slices: 0 a launch of their own, 1 the consumer (a row of a batch), 2 the consumer, of each row and of the one before it.
+// Whole contractions on a grid of the general kernel that leaves compute units idle and the others one workgroup each: 64 x 80 columns to a workgroup,
+// where those are at most one to a compute unit on every XCD (by the launch order: a grid that fits as a whole but not on each, k, v, r of 256 rows of
+// 1536 channels, 20 us a launch instead of 15), and from three row blocks on (fewer read the weights past the caches).  Us a launch, 64 x 128 / 64 x 80: 400 rows,
+// 2560 -> 2560 23.0 / 20.3, 10240 -> 2560 69 / 57.5; 256 rows, 5120 -> 5120 40 / 35.5.  A prompt of 12 layers of 2560, 320 / 400 / 512 tokens 2765,
+// 2962, 3331 -> 2619, 2746, 3186 us; of 12 of 2048, 400 and 512 2412, 2582 -> 2241, 2451; of 8 of 5120, 160 and 256 2768, 3500 -> 2712, 3413.
+static bool general_narrow(const ProductPlan &p, int64_t NT, int n) {
+    const int64_t gx = ceil_div(NT, kGemmNarrowNT), on_one = p.gy >= kXcds ? ceil_div(p.gy, kXcds) * gx : ceil_div(gx, kXcds) * p.gy;
+    return p.split == 1 && (int64_t)p.gx * p.gy * n <= 256 && p.gy > kStreamRowBlocks && on_one * n <= 256 / kXcds;
+}
 static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n, int readers = 0) {
     ProductPlan p;
     p.split = 1;
@@ -1859,6 +1874,7 @@ static ProductPlan plan_products(int64_t MT, int64_t NT, int64_t KB, int n, int 
         while ((int64_t)p.gx * p.gy * n * p.split < kGemmFillWgs && KB / (p.split * 2) >= 8 && p.split < kMaxSplit) p.split *= 2;
     // a long contraction on a grid still below the device: one split more (two slices at most)
     if (p.kind != PLAN_SKINNY && p.split == 1 && (int64_t)p.gx * p.gy * n < kGemmLongFillWgs && KB >= kGemmLongBlocks) p.split = 2;
+    if (p.kind == PLAN_GENERAL && general_narrow(p, NT, n)) { p.kind = PLAN_NARROW; p.gx = (int)ceil_div(NT, kGemmNarrowNT); }
     return p;
 }
 // Which of two roundings a product's y has: one of S (tot + 128 q) + zp, exact but for the last addition, where slices of the
@@ -2037,7 +2053,7 @@ size_t rows_quant_scratch_bytes(int64_t R, int64_t K) {
 }
 void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int out[4]) {
     const ProductPlan p = plan_products(ceil_div(R, 4), ceil_div(N, 16), K / 64, n);
-    out[0] = p.kind; out[1] = p.gx; out[2] = p.gy; out[3] = p.split;
+    out[0] = p.kind == PLAN_NARROW ? (int)PLAN_WIDE : p.kind; out[1] = p.gx; out[2] = p.gy; out[3] = p.split;
 }
 
 int rows_embed(hipStream_t st, const int64_t *tokens, int64_t R, int V, int C, const float *emb, const double *w,
@@ -2181,11 +2197,13 @@ static int launch_skinny(hipStream_t st, const GemmArgs &g, const dim3 &grid, bo
     RWKV_CHECK_LAUNCH("gemm8_skinny_kernel");
     return RWKV_OK;
 }
-static int launch_general(hipStream_t st, GemmArgs &g, bool wide, int gx, bool stream) {
+static int launch_general(hipStream_t st, GemmArgs &g, int kind, int gx, bool stream) {
+    const bool wide = kind == PLAN_WIDE;
     g.gx = gx; g.gy = (int)ceil_div(g.MT, 16); g.by_rows = g.gy >= kXcds;
     g.per_xcd = ((g.by_rows ? g.gy : gx) + kXcds - 1) / kXcds;
     const dim3 grid((unsigned)(kXcds * g.per_xcd * (g.by_rows ? gx : g.gy) * g.gz));
-    if (wide) hipLaunchKernelGGL(gemm8_wide_kernel, grid, dim3(512), 0, st, g);
+    if (kind == PLAN_NARROW) hipLaunchKernelGGL(gemm8_narrow_kernel, grid, dim3(512), 0, st, g);
+    else if (wide) hipLaunchKernelGGL(gemm8_wide_kernel, grid, dim3(512), 0, st, g);
     else if (stream && g.gy <= kStreamRowBlocks) hipLaunchKernelGGL(gemm8_kernel<true>, grid, dim3(512), 0, st, g);
     else hipLaunchKernelGGL(gemm8_kernel<false>, grid, dim3(512), 0, st, g);
     RWKV_CHECK_LAUNCH(wide ? "gemm8_wide_kernel" : "gemm8_kernel");
@@ -2228,7 +2246,7 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
         const int rc = launch_skinny(st, g, grid, p[0].stream);
         if (rc) return rc;
     } else {
-        const int rc = launch_general(st, g, pl.kind == PLAN_WIDE, pl.gx, p[0].stream);
+        const int rc = launch_general(st, g, pl.kind, pl.gx, p[0].stream);
         if (rc) return rc;
     }
     for (int m = 0; defer && m < n; ++m) defer[m].tot = nullptr;
@@ -2265,6 +2283,7 @@ static bool pair_general(int64_t MT, int64_t NT, int64_t NT2, int64_t KB) {
     auto alone = [&](int64_t nt) {                          // in ninths, as kGemmWideDen weighs the wide kernel
         const ProductPlan p = plan_products(MT, nt, KB, 1);
         if (p.split > 1) saved += 60;
+        if (p.kind == PLAN_NARROW) return (int64_t)kGemmWideDen * kGemmNarrowCost;
         return p.kind == PLAN_WIDE ? kGemmWideNum * 40 * ceil_div((int64_t)p.gx * p.gy, 256) : kGemmWideDen * general_cost((int64_t)p.gx * p.gy * p.split) / p.split;
     };
     const int64_t more = kGemmWideDen * general_cost((ceil_div(NT, kGemmNT) + ceil_div(NT2, kGemmNT)) * gy) - alone(NT) - alone(NT2);
@@ -2310,7 +2329,7 @@ int rows_ffn_key_receptance(hipStream_t st, bool sequence, const RowsProduct &k,
         const int rc = launch_skinny(st, g, grid, k.stream);
         if (rc) return rc;
     } else if (pair_general(g.MT, g.NT, g.NT2, g.KB)) {
-        const int rc = launch_general(st, g, false, (int)(ceil_div(g.NT, kGemmNT) + ceil_div(g.NT2, kGemmNT)), k.stream);
+        const int rc = launch_general(st, g, PLAN_GENERAL, (int)(ceil_div(g.NT, kGemmNT) + ceil_div(g.NT2, kGemmNT)), k.stream);
         if (rc) return rc;
     } else {
         int rc = rows_products(st, 1, &k, tot, R, C, F, ROW_RELU2, nullptr);

@@ -645,6 +645,18 @@ def test_gemm8_matches_fp64_dense(ops, T, K, N):
     assert err < 2e-7                                         # float32 rounding of x*range, nothing else
 
 
+# grids that leave compute units idle: 80 columns to a workgroup.  Ragged rows, columns and column blocks, fewer contraction blocks than
+# the ring has buffers, XCDs that share out the columns (up to 7 row blocks) and the rows
+@pytest.mark.parametrize("T,K,N", [(300, 2560, 2560), (200, 64, 4096), (130, 128, 5000), (400, 704, 2502), (520, 192, 1200), (512, 320, 2560)])
+def test_gemm8_of_narrow_workgroups_matches_fp64_dense(ops, T, K, N):
+    import ctypes
+    from rwkvstic_amd import _native
+    plan, tot = (ctypes.c_int * 4)(), ctypes.c_size_t()
+    _native.check(_native.lib().rwkv_gemm8_plan(T, K, N, 1, plan, ctypes.byref(tot)))
+    assert (plan[0], plan[1], plan[3]) == (3, -(-N // 80), 1)
+    test_gemm8_matches_fp64_dense(ops, T, K, N)
+
+
 # at most 8 rows: both sides of the column tiles at which the kernel changes its shape (256 | 320 | 512 | 1280),
 # fewer blocks than wavefronts, one block past a round, a split contraction
 @pytest.mark.parametrize("T,K,N", [(1, 64, 16), (8, 17 * 64, 4096), (8, 17 * 64, 4100), (3, 192, 5120), (5, 41 * 64, 5121), (4, 448, 8192),
