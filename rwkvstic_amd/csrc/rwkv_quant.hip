@@ -206,7 +206,6 @@ constexpr int kChainLds = 2 * 4 * kChainChannels * kChainStride * 8;
 __device__ __forceinline__ void quant_offsets(const float *__restrict__ W, int n_out, int n_in, const QuantWs &q, int group, double *lds,
                                               float *__restrict__ range, double *__restrict__ offset) {
     constexpr int kChains = 4 * kChainChannels;
-    
     double (*fr)[kChains][kChainStride] = reinterpret_cast<double (*)[kChains][kChainStride]>(lds);
     const int tiles = (n_out + kChainRows - 1) / kChainRows;
     // a partial to a thread; the eight of a wavefront's channel meet in the wavefront, its four in LDS
