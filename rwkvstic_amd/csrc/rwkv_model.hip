@@ -531,30 +531,19 @@ struct RowsWs {
     long long *tot;
 };
 
-// n_head > 0: one more product, of a single row with n_head columns (the head after a prompt)
-size_t rows_tot_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_head) {
-    const size_t a = rows_tot_bytes(R, n_wide, C), b = 3 * rows_tot_bytes(R, C, F > C ? F : C);     // k, v, r share a launch; ffn value
-    const size_t c = n_head > 0 ? rows_tot_bytes(1, n_head, C) : 0;
-    // the quantisers of the att output and of h park their partial records here before the product starts
-    const size_t q = rows_quant_scratch_bytes(R, n_wide > C ? n_wide : C);
-    const size_t m = a > b ? (a > c ? a : c) : (b > c ? b : c);
-    const size_t h = rows_deferred_bytes(R, C);         // a residual update handed on in slices
-    return std::max(std::max(m, q), h);
-}
-
-// n_wide = widest product output (n_ffn, or the vocabulary when every row needs logits)
-size_t rows_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_head) {
+// head_rows: rows that need logits (all of a batch, the last of a prompt)
+size_t rows_ws_bytes(int64_t R, int64_t C, int64_t F, int64_t V, int64_t head_rows) {
     size_t n = 0;
     n += round_up((size_t)R * C * 8, 256) * 5;          // x, kvr[3], att
     n += round_up((size_t)R * F * 8, 256);              // h
     n += round_up((size_t)(R < kRowsDeferMax ? R : kRowsDeferMax - 1) * C * 8, 256) * 3;    // x2, sh1, sh2
     n += round_up((size_t)R * 8, 256) * 12;             // S, qs, zp of four operands
     n += round_up(rows_dig_bytes(R, std::max(F, C)), 256) + 2 * round_up(rows_dig_bytes(R, C), 256);
-    n += round_up(rows_tot_ws_bytes(R, C, F, n_wide, n_head), 256);
+    n += round_up(rows_pass_tot_bytes(R, C, F, V, head_rows), 256);
     return n;
 }
 
-RowsWs rows_carve(void *ws, int64_t R, int64_t C, int64_t F, int64_t n_wide, int64_t n_head) {
+RowsWs rows_carve(void *ws, int64_t R, int64_t C, int64_t F, int64_t V, int64_t head_rows) {
     unsigned char *p = static_cast<unsigned char *>(ws);
     auto take = [&](size_t bytes) { void *q = p; p += round_up(bytes, 256); return q; };
     RowsWs w;
@@ -571,7 +560,7 @@ RowsWs rows_carve(void *ws, int64_t R, int64_t C, int64_t F, int64_t n_wide, int
     }
     w.qv.dig = w.q[0].dig;
     for (double **b : {&w.qv.S, &w.qv.qs, &w.qv.zp}) *b = (double *)take((size_t)R * 8);
-    w.tot = (long long *)take(rows_tot_ws_bytes(R, C, F, n_wide, n_head));
+    w.tot = (long long *)take(rows_pass_tot_bytes(R, C, F, V, head_rows));
     return w;
 }
 
@@ -688,7 +677,7 @@ int rows_sequence(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t 
     const int64_t C = m->d.n_embd, F = m->d.n_ffn;
     unsigned char *rows_base = static_cast<unsigned char *>(workspace) + round_up(ws_doubles(C, F) * sizeof(double), 256);
     const int64_t Rmax = T < kRowsChunk ? T : kRowsChunk;
-    const RowsWs rw = rows_carve(rows_base, Rmax, C, F, F, m->d.n_vocab);
+    const RowsWs rw = rows_carve(rows_base, Rmax, C, F, m->d.n_vocab, 1);
     RowsTailWork tail;
     for (int64_t t0 = 0; t0 < T; t0 += kRowsChunk) {
         const int64_t R = T - t0 < kRowsChunk ? T - t0 : kRowsChunk;
@@ -865,15 +854,14 @@ size_t rwkv_model_workspace_bytes(const rwkv_model *m, int64_t max_tokens) {
     size_t n = round_up(ws_doubles(m->d.n_embd, m->d.n_ffn) * sizeof(double), 256);
     if (rows_supported(m)) {            // (also where the token kernel serves eager calls: see recorded)
         const int64_t R = max_tokens < kRowsChunk ? max_tokens : kRowsChunk;
-        n += rows_ws_bytes(R, m->d.n_embd, m->d.n_ffn, m->d.n_ffn, m->d.n_vocab);
+        n += rows_ws_bytes(R, m->d.n_embd, m->d.n_ffn, m->d.n_vocab, 1);
     }
     return n;
 }
 
 size_t rwkv_model_batch_workspace_bytes(const rwkv_model *m, int64_t batch) {
     if (!m || batch <= 0 || !rows_supported(m)) return 0;
-    const int64_t wide = m->d.n_ffn > m->d.n_vocab ? m->d.n_ffn : m->d.n_vocab;
-    return rows_ws_bytes(batch, m->d.n_embd, m->d.n_ffn, wide, 0);
+    return rows_ws_bytes(batch, m->d.n_embd, m->d.n_ffn, m->d.n_vocab, batch);
 }
 
 int rwkv_model_forward(rwkv_model *m, rwkv_stream_t stream, const int64_t *tokens, int64_t T, double *state,
@@ -910,7 +898,7 @@ int rwkv_model_forward_batch(rwkv_model *m, rwkv_stream_t stream, const int64_t 
     const hipStream_t st = (hipStream_t)stream;
     const rwkv_model_desc &d = m->d;
     const int64_t C = d.n_embd, F = d.n_ffn, V = d.n_vocab;
-    const RowsWs rw = rows_carve(workspace, batch, C, F, F > V ? F : V, 0);
+    const RowsWs rw = rows_carve(workspace, batch, C, F, V, batch);
     RowsTailWork tail;
     int rc = rows_layers(m, st, tokens, batch, false, states, d.n_layer * 5 * C, rw, tail);
     if (rc) return rc;

@@ -49,6 +49,9 @@ struct RowsFew {
 size_t rows_dig_bytes(int64_t R, int64_t K);
 size_t rows_tot_bytes(int64_t R, int64_t N, int64_t K);     // integer totals of ONE product (times the products in a launch) of a contraction of up to K
 size_t rows_deferred_bytes(int64_t R, int64_t N);           // integer totals of one product handed on in slices (see RowsDeferred)
+// Integer totals that a pass of up to R rows through the layers, and head_rows of them through the head, keeps at one time, and what its
+// quantisers leave in the same place.
+size_t rows_pass_tot_bytes(int64_t R, int64_t C, int64_t F, int64_t V, int64_t head_rows);
 size_t rows_quant_scratch_bytes(int64_t R, int64_t K);   // what rows_quant writes into its scratch area (0: unused)
 // The plan rows_products follows for n products [R, K] x [K, N]: out = {kernel kind, grid x, grid y, splits}.
 void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int out[4]);

@@ -21,6 +21,7 @@
 // hands it to the matrix instruction unchanged.
 #include "rwkv_rows.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace rwkv {
@@ -2050,6 +2051,14 @@ constexpr int kLongQuantRows = 384, kLongQuantFrom = 2048;
 size_t rows_quant_scratch_bytes(int64_t R, int64_t K) {
     if (!quant_uses_parts(R, K)) return 0;
     return (size_t)(R * ceil_div(K, 4 * kRT * kQuantPartSeg) * 2 * 8);
+}
+size_t rows_pass_tot_bytes(int64_t R, int64_t C, int64_t F, int64_t V, int64_t head_rows) {
+    const int64_t K = std::max(F, C);
+    // Each product for itself: fewer columns may be cut where more are not, so the totals of the widest do not hold those of every narrower one
+    // (32 rows of 1024 channels: 16000 columns of logits are cut in two, 16384 hidden values are not).  k, v, r share a launch.
+    size_t n = std::max(3 * rows_tot_bytes(R, C, K), std::max(rows_tot_bytes(R, F, C), rows_tot_bytes(head_rows, V, C)));
+    n = std::max(n, rows_deferred_bytes(R, C));             // a residual update handed on in slices
+    return std::max(n, rows_quant_scratch_bytes(R, K));     // the quantisers' partial records, before a product starts
 }
 void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int out[4]) {
     const ProductPlan p = plan_products(ceil_div(R, 4), ceil_div(N, 16), K / 64, n);

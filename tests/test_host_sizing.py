@@ -84,6 +84,30 @@ def test_gemm8_workspace_covers_quantiser_scratch(lib):
             assert lib.rwkv_gemm8_workspace_bytes(T, K, 16) - fixed >= need, (T, K)
 
 
+def _pass_tot_bytes(lib, R, C_, F, V, head_rows):
+    fn = getattr(lib, "_ZN4rwkv19rows_pass_tot_bytesElllll")
+    fn.restype, fn.argtypes = C.c_size_t, [C.c_int64] * 5
+    return fn(R, C_, F, V, head_rows)
+
+
+@pytest.mark.parametrize("C_,F", [(64, 64), (512, 2048), (768, 640), (1024, 4096), (1024, 8192), (1024, 16384), (1536, 20480), (2048, 512), (2560, 10240),
+                                  (4096, 16384), (5120, 640), (5120, 20480)])
+def test_totals_of_a_pass_hold_those_of_every_product_in_it(lib, C_, F):
+    """Whatever the order of n_embd, n_ffn and the vocabulary: fewer columns may be cut in slices where more are not.  Of a prompt longer
+    than a pass the last one may have any number of rows."""
+    def need(rows, K, N, n):
+        (kind, gx, gy, split), _ = _plan(lib, rows, K, N, n)
+        return n * split * (-(-rows // 4) * 4 * (-(-N // 16) * 16) * 8)
+
+    layers = {R: max(need(R, C_, C_, 3), need(R, C_, F, 1), need(R, F, C_, 1)) for R in ROWS}
+    for V in (16, 100, 1000, 4000, 8000, 14000, 16000, 20000, 50277, 65536):
+        one = need(1, C_, V, 1)
+        for R in ROWS:
+            assert max(layers[R], need(R, C_, V, 1)) <= _pass_tot_bytes(lib, R, C_, F, V, R), (V, R)
+            assert max(layers[R], one) <= _pass_tot_bytes(lib, R, C_, F, V, 1), (V, R)
+        assert max(layers.values()) <= _pass_tot_bytes(lib, 1024, C_, F, V, 1), V
+
+
 def test_a_pending_product_keeps_its_row_constants_apart(lib):
     """Few rows: a row of the LayerNorm kernel has one workgroup per mix, all of which read S, qs and zp of a product handed on
     unfinished; outputs in the same arrays would be written by one while another still reads.  The call is refused on the
