@@ -31,7 +31,7 @@ struct RowsDeferred {
     const long long *tot;   // [slices][slice] totals of this product; element (t, j) at t * ldd + j
     size_t slice;
     int slices, ldd, op;    // op: the RowTail still to be applied
-    bool apart, fused;      // see rounded_apart; the gated update as one fused multiply-add, as in the product's own epilogue
+    bool apart, fused;      // see rounded_apart; the gated update as one fused multiply-add (see gate_fused)
     const double *S, *qs, *zp;
     const float *gate;      // ROW_GATE_ADD
 };

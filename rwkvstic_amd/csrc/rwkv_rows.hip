@@ -1886,6 +1886,13 @@ static bool rounded_apart(int64_t MT, int64_t NT, int64_t KB, int n) {
     if (MT > kVecMT) return MT <= kSkinnyMT ? skinny_cut(NT, KB, n) : plan_products(MT, NT, KB, n).split > 1;
     return KB >= 16 && (NT * n < 128 || (NT * n < 512 && KB >= kGemmLongBlocks));
 }
+// Whether a gated update that is handed on adds y * sigmoid(r) as one fused multiply-add, as a product's own epilogue and rows_finish_kernel do.
+// Always, but where slices of batch rows of gemm8_skinny_kernel and the general kernel have been handed on ever since: those round the
+// product for itself.  (The former takes up to eight slices, and only products of 32 column blocks and more, or of less than 64
+// contraction blocks, were handed on before six could be.)
+static bool gate_fused(int kind, bool sequence, int64_t NT, int64_t KB) {
+    return kind == PLAN_VEC || sequence || (kind == PLAN_SKINNY && 4 * ceil_div(NT, kSkinnyNT) < kSkinnyFillWgs && KB >= 64);
+}
 // Shape of the few-row kernel for a launch of so many column tiles: tiles per workgroup, wavefronts per workgroup, blocks
 // in flight per wavefront and tile (at most).  All workgroups resident at once; KB: the blocks of a workgroup's part of the contraction.
 //
@@ -2261,8 +2268,9 @@ int rows_products(hipStream_t st, int n, const RowsProduct *p, long long *tot, i
     for (int m = 0; defer && m < n; ++m) defer[m].tot = nullptr;
     if (split == 1) return RWKV_OK;     // the tail was applied in the product's epilogue
     if (defer && R < kRowsDeferMax && split <= kRowsDeferSlices) {   // the consumer adds the slices up
+        const bool fused = gate_fused(pl.kind, sequence, g.NT, g.KB);
         for (int m = 0; m < n; ++m)
-            defer[m] = RowsDeferred{tot + (size_t)m * split * g.slice, g.slice, split, g.ldd, op, g.apart != 0, pl.kind == PLAN_VEC || sequence, p[m].a.S, p[m].a.qs, p[m].a.zp, gate};
+            defer[m] = RowsDeferred{tot + (size_t)m * split * g.slice, g.slice, split, g.ldd, op, g.apart != 0, fused, p[m].a.S, p[m].a.qs, p[m].a.zp, gate};
         return RWKV_OK;
     }
 

@@ -568,6 +568,28 @@ def test_rows_of_a_small_batch_have_the_bits_of_a_batch_of_one(C, F, B):
     assert torch.equal(states, singles)
 
 
+# ffn value of up to `whole` rows as whole contractions, of more in slices that are handed on; every other product in the same kernel on
+# both sides: the gated update is one fused multiply-add in each, so the bits of a row do not depend on the others
+@pytest.mark.parametrize("C,F,whole", [(1024, 4096, 24), (1536, 6144, 16), (2560, 5632, 16), (3584, 8192, 16)])
+def test_rows_of_a_batch_have_the_same_bits_in_slices_and_in_whole_contractions(C, F, whole):
+    import ctypes
+    from rwkvstic_amd import _native as N
+    from rwkvstic_amd.model import HipRWKV
+    plan, tot = (ctypes.c_int * 4)(), ctypes.c_size_t()
+    m = HipRWKV(synth.iter_tensors(2, C, F, 100, seed=C, device="cuda", ln="random"))
+    got = {}
+    for B in (whole, whole + 1, 32):
+        _say(f"batch of {B} at C={C} F={F}")
+        N.check(N.lib().rwkv_gemm8_plan(B, F, C, 1, plan, ctypes.byref(tot)))
+        assert (plan[0], plan[3] > 1) == ((0, False) if B == whole else (1, True))
+        states = m.emptyState.repeat(B, 1, 1, 1).contiguous()
+        for step in range(3):
+            lb, states = m.forward_batch(synth.random_tokens(32, V=100, seed=60 + step)[:B].cuda(), states)
+        got[B] = (lb[:whole].clone(), states[:whole].clone())
+    for B in (whole + 1, 32):
+        assert torch.equal(got[B][0], got[whole][0]) and torch.equal(got[B][1], got[whole][1]), B
+
+
 # four and eight M-tiles, ffn value in five or six slices that are handed on, att output and k, v, r in as many as fill the device
 @pytest.mark.parametrize("C,F,B", [(4096, 16384, 9), (4096, 16384, 16), (4096, 16384, 17), (5120, 20480, 16), (5120, 20480, 32), (2560, 10240, 20),
                                    (640, 24576, 32)])
