@@ -368,8 +368,11 @@ int rwkv_gemm8(rwkv_stream_t stream, int64_t T, int64_t n_in, int64_t n_out,
  * (k, v, r do; matmul.py:86-94): plan = {kernel variant (0: at most 8 rows, or up to 32 of a
  * small matrix, 1: 9-32
  * rows, 2: 64 x 128 tiles, 3: 64 x 160 or 64 x 80 tiles), grid x, grid y, splits of the
- * contraction}, and in *tot_bytes_per_product the bytes of integer totals the
- * workspace reserves per product.  Host-only: launches nothing. */
+ * contraction}, and in *tot_bytes_per_product the bytes of integer totals
+ * rwkv_gemm8's workspace reserves per product.  Products whose slices the model
+ * leaves to the next kernel (k, v, r and the residual updates of batches, those
+ * updates in short prompts) may be cut in another number of slices than this says.
+ * Host-only: launches nothing. */
 int rwkv_gemm8_plan(int64_t T, int64_t n_in, int64_t n_out, int n_products,
                     int plan[4], size_t *tot_bytes_per_product);
 

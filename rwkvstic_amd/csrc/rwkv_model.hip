@@ -601,11 +601,7 @@ int rows_layers(rwkv_model *m, hipStream_t st, const int64_t *tokens, int64_t R,
     // A pending product's totals and gate are written by later launches only.
     const bool stream = weights_streamed(d.n_layer, d.n_embd, d.n_ffn, d.n_vocab);
     const bool defer = !sequence && R < kRowsDeferMax;
-    // The residual updates of a short prompt of a narrow model too, although a row of a sequence adds up the slices of the row before it as
-    // well, whose LayerNorm it needs.  Us a prompt, a launch for the sums / handed on: 12 layers of 512, 40 and 127 tokens 679, 743 / 653, 720; 24 of
-    // 1024, 77 and 127 1741, 1840 / 1695, 1788; 12 of 1536, 77 and 100 1074, 1135 / 1056, 1142; 12 of 2048, 64 and 77 1151, 1174 / 1136, 1186; 12 of
-    // 2560, 32 and 127 1067, 1502 / 1076, 1556; 8 of 4096, 32 1004 / 1036.
-    const bool hand_on = sequence ? C <= 2048 && R < kRowsDeferMax && R * C <= (1 << 17) : defer;
+    const bool hand_on = rows_readers(R, C, sequence) > 0;      // the residual updates
     RowsDeferred dk[3];
     // The LayerNorm kernels leave the new shift rows aside, and each commits what the one before it left.
     const bool aside = R < kRowsDeferMax || sequence;
@@ -981,7 +977,7 @@ int rwkv_gemm8_plan(int64_t T, int64_t n_in, int64_t n_out, int n_products, int 
     RWKV_CHECK_ARG(T > 0 && n_in > 0 && n_out > 0 && n_products >= 1 && n_products <= kRowsMaxProducts,
                    "rwkv_gemm8_plan: bad sizes");
     if (n_in % 64) return set_error(RWKV_ERR_SIZE, "rwkv_gemm8_plan: n_in must be a multiple of 64");
-    rows_plan_describe(T, n_in, n_out, n_products, plan);
+    rows_plan_describe(T, n_in, n_out, n_products, 0, plan);
     *tot_bytes_per_product = rows_tot_bytes(T, n_out, n_in);
     return RWKV_OK;
 }

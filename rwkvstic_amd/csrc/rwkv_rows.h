@@ -53,8 +53,12 @@ size_t rows_deferred_bytes(int64_t R, int64_t N);           // integer totals of
 // quantisers leave in the same place.
 size_t rows_pass_tot_bytes(int64_t R, int64_t C, int64_t F, int64_t V, int64_t head_rows);
 size_t rows_quant_scratch_bytes(int64_t R, int64_t K);   // what rows_quant writes into its scratch area (0: unused)
-// The plan rows_products follows for n products [R, K] x [K, N]: out = {kernel kind, grid x, grid y, splits}.
-void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int out[4]);
+// Who adds up the slices of a residual update: 0 a launch of their own, 1 its consumer, each row's once (a batch), 2 its consumer, those of
+// the row before as well (a sequence, whose LayerNorm needs both).
+int rows_readers(int64_t R, int64_t C, bool sequence);
+// The plan rows_products follows for n products [R, K] x [K, N] with so many readers of their slices (k, v, r of a batch: 1, of a sequence and
+// everything else: 0): out = {kernel kind, grid x, grid y, splits}.
+void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int readers, int out[4]);
 bool rows_ln_width_supported(int64_t C);            // widths the fused LayerNorm + mix + quantise kernel holds in registers
 
 int rows_embed(hipStream_t st, const int64_t *tokens, int64_t R, int V, int C, const float *emb, const double *w,

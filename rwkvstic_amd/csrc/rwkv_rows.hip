@@ -1799,9 +1799,9 @@ constexpr int kStreamRowBlocks = 2;
 constexpr int kSkinnyPairWgs = 64;      // ffn key and receptance of 9..32 rows in one launch from so many workgroups on
 constexpr int kGemmFillWgs = 96;         // larger products: split until the grid has this many workgroups.  A split costs a second launch and a round trip of the integer totals through memory, so it only pays for grids far below the device (3B shape, tokens/s in chunks of 64 / 128 / 256 / 512 tokens: 13,180 / 23,640 / 37,610 / 52,070 at 96; 12,480 / 21,280 / 34,650 / 49,380 at 256; 12,540 / 21,470 / 31,520 / 51,160 at 64)
 
-// Which kernel serves n products of MT row tiles x NT column tiles over KB contraction blocks, its grid and
-// the number of contraction splits.  The ONE place these are decided: the launches and the sizing of the
-// totals buffer both call it, so the buffer always holds every slice the kernel writes.
+// Which kernel serves n products of MT row tiles x NT column tiles over KB contraction blocks, its grid and the number of contraction
+// splits (plan_products; readers: who adds the slices up, see rows_readers).  The one place these are decided.  The totals' buffer is
+// sized by bounds over every number of products and readers (gemm_split_bound, rows_deferred_bytes), which a host test holds against the plans.
 enum { PLAN_VEC = 0, PLAN_SKINNY, PLAN_GENERAL, PLAN_WIDE, PLAN_NARROW };
 struct ProductPlan { int kind, gx, gy, split; };
 // Which products of 9 to 32 rows go through gemv16_kernel.  Every workgroup of it reads the digits of all rows, gemm8_skinny_kernel
@@ -1845,7 +1845,6 @@ static int64_t general_cost(int64_t w4) {
 constexpr int kGemmNarrowCost = 27;
 static bool general_wide(int64_t w4, int64_t w5) { return w4 >= 256 && kGemmWideNum * ceil_div(w5, 256) * 40 < kGemmWideDen * general_cost(w4); }
 static int vec_split(int64_t MT, int64_t NT, int64_t KB, int readers);
-// readers: who adds up the slices: 0 a launch of their own, 1 the consumer (a row of a batch), 2 the consumer, of each row and of the one before it.
 // Whole contractions on a grid of the general kernel that leaves compute units idle and the others one workgroup each: 64 x 80 columns to a workgroup,
 // where those are at most one to a compute unit on every XCD (by the launch order: a grid that fits as a whole but not on each, k, v, r of 256 rows of
 // 1536 channels, 20 us a launch instead of 15), and from three row blocks on (fewer read the weights past the caches).  Us a launch, 64 x 128 / 64 x 80: 400 rows,
@@ -2067,8 +2066,18 @@ size_t rows_pass_tot_bytes(int64_t R, int64_t C, int64_t F, int64_t V, int64_t h
     n = std::max(n, rows_deferred_bytes(R, C));             // a residual update handed on in slices
     return std::max(n, rows_quant_scratch_bytes(R, K));     // the quantisers' partial records, before a product starts
 }
-void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int out[4]) {
-    const ProductPlan p = plan_products(ceil_div(R, 4), ceil_div(N, 16), K / 64, n);
+// Batches of fewer than kRowsDeferMax rows, and the short prompts of narrow models, although a row of a sequence adds up the slices of the row
+// before it as well.  Us a prompt, a launch for the sums / handed on: 12 layers of 512, 40 and 127 tokens 679, 743 / 653, 720; 24 of
+// 1024, 77 and 127 1741, 1840 / 1695, 1788; 12 of 1536, 77 and 100 1074, 1135 / 1056, 1142; 12 of 2048, 64 and 77 1151, 1174 / 1136, 1186; 12 of
+// 2560, 32 and 127 1067, 1502 / 1076, 1556; 8 of 4096, 32 1004 / 1036.  (That is att output, and ffn value where it is cut in six at most: the general
+// kernel cuts it in eight for 33 to 127 tokens of 1024 channels, 33 to 64 of 1536 and 2048, and those slices keep their launch.)
+int rows_readers(int64_t R, int64_t C, bool sequence) {
+    if (R >= kRowsDeferMax) return 0;
+    if (!sequence) return 1;
+    return C <= 2048 && R * C <= (1 << 17) ? 2 : 0;
+}
+void rows_plan_describe(int64_t R, int64_t K, int64_t N, int n, int readers, int out[4]) {
+    const ProductPlan p = plan_products(ceil_div(R, 4), ceil_div(N, 16), K / 64, n, readers);
     out[0] = p.kind == PLAN_NARROW ? (int)PLAN_WIDE : p.kind; out[1] = p.gx; out[2] = p.gy; out[3] = p.split;
 }
 

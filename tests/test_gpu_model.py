@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+import product_plans
 from oracle import rwkv_oracle as O
 from rwkvstic_amd import synth
 
@@ -548,13 +549,14 @@ def test_batch_steps_of_more_rows_than_are_resident_match_single_steps(C, B):
         assert float((states[:, :, row] - singles[:, :, row]).norm() / singles[:, :, row].norm()) < 2e-6, row
 
 
-# at most 8 rows, ffn value handed on in 3 or 4 slices (5 to 8 rows) or finished in its own launch (a row alone, 2048 channels of
+# at most 8 rows, ffn value handed on in 3 to 5 slices (5 to 8 rows) or finished in its own launch (a row alone, 2048 channels of
 # 2048 hidden values): integer totals, exact in any order, rounded in the same place, so the bits of a row do not depend on the others
-@pytest.mark.parametrize("C,F,B", [(1024, 4096, 8), (1088, 4352, 5), (1536, 6144, 7), (2560, 10240, 8), (5120, 20480, 6), (2048, 2048, 8),
-                                   (2048, 512, 8), (1024, 64, 3)])     # the widest rows are not the hidden ones
-def test_rows_of_a_small_batch_have_the_bits_of_a_batch_of_one(C, F, B):
+@pytest.mark.parametrize("C,F,B,slices", [(1024, 4096, 8, 4), (1088, 4352, 5, 3), (1536, 6144, 7, 5), (2560, 10240, 8, 3), (5120, 20480, 6, 3),
+                                          (2048, 2048, 8, 0), (2048, 512, 8, 0), (1024, 64, 3, 0)])     # the widest rows are not the hidden ones
+def test_rows_of_a_small_batch_have_the_bits_of_a_batch_of_one(C, F, B, slices):
     from rwkvstic_amd.model import HipRWKV
     _say(f"batch of {B} at C={C} F={F}")
+    assert product_plans.handed_on(B, C, F) == slices and product_plans.handed_on(1, C, F) == 0
     m = HipRWKV(synth.iter_tensors(2, C, F, 100, seed=C + B, device="cuda", ln="random"))
     states = m.emptyState.repeat(B, 1, 1, 1).contiguous()
     singles = states.clone()
@@ -572,16 +574,13 @@ def test_rows_of_a_small_batch_have_the_bits_of_a_batch_of_one(C, F, B):
 # both sides: the gated update is one fused multiply-add in each, so the bits of a row do not depend on the others
 @pytest.mark.parametrize("C,F,whole", [(1024, 4096, 24), (1536, 6144, 16), (2560, 5632, 16), (3584, 8192, 16)])
 def test_rows_of_a_batch_have_the_same_bits_in_slices_and_in_whole_contractions(C, F, whole):
-    import ctypes
-    from rwkvstic_amd import _native as N
     from rwkvstic_amd.model import HipRWKV
-    plan, tot = (ctypes.c_int * 4)(), ctypes.c_size_t()
     m = HipRWKV(synth.iter_tensors(2, C, F, 100, seed=C, device="cuda", ln="random"))
     got = {}
     for B in (whole, whole + 1, 32):
         _say(f"batch of {B} at C={C} F={F}")
-        N.check(N.lib().rwkv_gemm8_plan(B, F, C, 1, plan, ctypes.byref(tot)))
-        assert (plan[0], plan[3] > 1) == ((0, False) if B == whole else (1, True))
+        assert product_plans.plan(B, F, C, 1, 1)[0] == (product_plans.VEC if B == whole else product_plans.SKINNY)
+        assert (product_plans.handed_on(B, C, F) > 0) == (B > whole)
         states = m.emptyState.repeat(B, 1, 1, 1).contiguous()
         for step in range(3):
             lb, states = m.forward_batch(synth.random_tokens(32, V=100, seed=60 + step)[:B].cuda(), states)
@@ -590,19 +589,23 @@ def test_rows_of_a_batch_have_the_same_bits_in_slices_and_in_whole_contractions(
         assert torch.equal(got[B][0], got[whole][0]) and torch.equal(got[B][1], got[whole][1]), B
 
 
-# four and eight M-tiles, ffn value in five or six slices that are handed on, att output and k, v, r in as many as fill the device
-@pytest.mark.parametrize("C,F,B", [(4096, 16384, 9), (4096, 16384, 16), (4096, 16384, 17), (5120, 20480, 16), (5120, 20480, 32), (2560, 10240, 20),
-                                   (640, 24576, 32)])
-def test_batch_steps_in_slices_that_fill_the_device_match_single_steps(C, F, B):
+# four and eight M-tiles, ffn value in six slices that are handed on; att output whole or in five, k, v, r whole or in two or five
+@pytest.mark.parametrize("C,F,B,att,kvr", [(4096, 16384, 9, 0, 1), (4096, 16384, 16, 0, 5), (4096, 16384, 17, 0, 5), (5120, 20480, 16, 5, 2),
+                                           (5120, 20480, 32, 5, 2), (2560, 10240, 20, 0, 1), (640, 24576, 32, 0, 1)])
+def test_batch_steps_in_slices_that_fill_the_device_match_single_steps(C, F, B, att, kvr):
+    assert product_plans.handed_on(B, C, F) == 6 and product_plans.handed_on(B, C, C) == att and product_plans.plan(B, C, C, 3, 1)[3] == kvr
     test_batch_steps_of_ragged_and_wide_rows_match_single_steps(C, F, B)
 
 
-# prompts on both sides of the line up to which the residual updates are handed on in slices (2048 channels, 2^17 values), of rows that few-row,
-# skinny and general products serve; the second pass of a long prompt.  Against the same tokens one at a time.
-@pytest.mark.parametrize("C,T", [(1024, 8), (1024, 33), (1024, 127), (1024, 128), (2048, 20), (2048, 64), (2048, 65), (2112, 40), (512, 1024 + 40)])
-def test_short_prompts_match_token_by_token(C, T):
+# prompts on both sides of the line up to which the residual updates (att output, ffn value) are handed on in slices (2048 channels, 2^17
+# values), of rows that few-row, skinny and general products serve; the second pass of a long prompt.  Against the same tokens one at a time.
+@pytest.mark.parametrize("C,T,att,ffn", [(1024, 8, 0, 0), (1024, 33, 2, 0), (1024, 127, 2, 0), (1024, 128, 0, 0), (1536, 80, 2, 4), (2048, 20, 0, 6), (2048, 64, 4, 0),
+                                         (2048, 65, 0, 0), (2112, 40, 0, 0), (512, 1024 + 40, 0, 4)])
+def test_short_prompts_match_token_by_token(C, T, att, ffn):
     from rwkvstic_amd.model import HipRWKV
     _say(f"prompt of {T} at C={C}")
+    last = T % 1024
+    assert (product_plans.handed_on(last, C, C, True), product_plans.handed_on(last, C, 4 * C, True)) == (att, ffn)
     m = HipRWKV(synth.iter_tensors(2, C, 4 * C, 100, seed=C + T, device="cuda", ln="random"))
     toks = synth.random_tokens(T, V=100, seed=T)
     l0, s0 = m.forward(toks.cuda(), m.emptyState.clone())

@@ -6,6 +6,8 @@ import os
 
 import pytest
 
+import product_plans
+
 
 @pytest.fixture(scope="module")
 def lib():
@@ -84,12 +86,6 @@ def test_gemm8_workspace_covers_quantiser_scratch(lib):
             assert lib.rwkv_gemm8_workspace_bytes(T, K, 16) - fixed >= need, (T, K)
 
 
-def _pass_tot_bytes(lib, R, C_, F, V, head_rows):
-    fn = getattr(lib, "_ZN4rwkv19rows_pass_tot_bytesElllll")
-    fn.restype, fn.argtypes = C.c_size_t, [C.c_int64] * 5
-    return fn(R, C_, F, V, head_rows)
-
-
 @pytest.mark.parametrize("C_,F", [(64, 64), (512, 2048), (768, 640), (1024, 4096), (1024, 8192), (1024, 16384), (1536, 20480), (2048, 512), (2560, 10240),
                                   (4096, 16384), (5120, 640), (5120, 20480)])
 def test_totals_of_a_pass_hold_those_of_every_product_in_it(lib, C_, F):
@@ -103,9 +99,39 @@ def test_totals_of_a_pass_hold_those_of_every_product_in_it(lib, C_, F):
     for V in (16, 100, 1000, 4000, 8000, 14000, 16000, 20000, 50277, 65536):
         one = need(1, C_, V, 1)
         for R in ROWS:
-            assert max(layers[R], need(R, C_, V, 1)) <= _pass_tot_bytes(lib, R, C_, F, V, R), (V, R)
-            assert max(layers[R], one) <= _pass_tot_bytes(lib, R, C_, F, V, 1), (V, R)
-        assert max(layers.values()) <= _pass_tot_bytes(lib, 1024, C_, F, V, 1), V
+            assert max(layers[R], need(R, C_, V, 1)) <= product_plans.pass_tot_bytes(R, C_, F, V, R), (V, R)
+            assert max(layers[R], one) <= product_plans.pass_tot_bytes(R, C_, F, V, 1), (V, R)
+        assert max(layers.values()) <= product_plans.pass_tot_bytes(1024, C_, F, V, 1), V
+
+
+@pytest.mark.parametrize("C_", [64, 320, 512, 768, 1024, 1088, 1536, 2048, 2112, 2560, 3072, 3584, 4096, 5120, 6144])
+def test_slices_left_to_the_next_kernel_are_whole_and_fit(lib, C_):
+    """The plans of k, v, r and of the two residual updates, which depend on who adds up the slices: the totals hold all of them, no slice is
+    empty (nothing would be written for it), and a few-row product has its kernel."""
+    most = 0
+    for F in (64, 640, 2 * C_, 4 * C_, 16384):
+        for R in ROWS:
+            for sequence in (False, True):
+                room, who = product_plans.pass_tot_bytes(R, C_, F, 16, 1 if sequence else R), product_plans.readers(R, C_, sequence)
+                for K, n, readers in ((C_, 1, who), (F, 1, who), (C_, 3, int(who == 1))):
+                    kind, _, _, s = product_plans.plan(R, K, C_, n, readers)
+                    MT, NT, KB = -(-R // 4), -(-C_ // 16), K // 64
+                    each = -(-KB // s)
+                    assert n * s * MT * 4 * NT * 16 * 8 <= room, (F, R, K, n, s)
+                    assert (s - 1) * each < KB, (F, R, K, n, s)
+                    if kind == product_plans.VEC:
+                        assert product_plans.vec_kernel(MT, NT * s * n, KB, each), (F, R, K, n, s)
+                    if readers:
+                        most = max(most, s)
+    assert most > 1 or C_ <= 320
+
+
+def test_what_is_handed_on(lib):
+    """Short prompts of narrow models and batches of fewer than 128 rows; slices by what they save, no more than the next kernel takes."""
+    assert [product_plans.readers(R, C_, s) for R, C_, s in ((127, 5120, False), (128, 512, False), (127, 1024, True), (128, 512, True), (64, 2048, True),
+                                                             (65, 2048, True), (4, 2112, True))] == [1, 0, 2, 0, 2, 0, 0]
+    assert [product_plans.handed_on(R, 2560, 10240) for R in (4, 8, 16, 17, 32, 127)] == [0, 3, 0, 6, 6, 4]
+    assert [product_plans.handed_on(77, C_, K, True) for C_, K in ((512, 512), (512, 2048), (1024, 1024), (1024, 4096), (1536, 6144))] == [0, 4, 2, 0, 4]
 
 
 def test_a_pending_product_keeps_its_row_constants_apart(lib):
@@ -140,8 +166,6 @@ def test_a_pending_product_keeps_its_row_constants_apart(lib):
 def test_every_few_row_product_has_its_kernel_and_every_kernel_a_product(lib):
     """gemv16_kernel: the rules that say which products it takes and in which shape, against the list of its instances."""
     import re
-    kernel_of = getattr(lib, "_ZN4rwkv13vec_kernel_ofEllll")
-    kernel_of.restype, kernel_of.argtypes = C.c_void_p, [C.c_int64] * 4
     plan, tot = (C.c_int * 4)(), C.c_size_t()
     reached = set()
     for MT in range(1, 9):
@@ -149,7 +173,7 @@ def test_every_few_row_product_has_its_kernel_and_every_kernel_a_product(lib):
             for KB in list(range(1, 130)) + [160, 175, 176, 200, 233, 234, 240, 320, 350, 351, 512, 700, 701, 1023, 1024, 1025, 2048, 2049]:
                 assert lib.rwkv_gemm8_plan(4 * MT, 64 * KB, 16 * tiles, 1, C.byref(plan), C.byref(tot)) == 0
                 kind, _, _, split = plan
-                at = kernel_of(MT, tiles * split, KB, -(-KB // split))
+                at = product_plans.vec_kernel(MT, tiles * split, KB, -(-KB // split))
                 assert (kind == 0) == bool(at), (MT, tiles, KB)
                 reached.add(at)
     source = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rwkvstic_amd", "csrc", "rwkv_rows.hip")).read()
