@@ -1823,13 +1823,17 @@ static bool skinny_cut(int64_t NT, int64_t KB, int n) { return ceil_div(NT, kSki
 // the two that then wait for it.  (So no power of two: 40 column blocks of 5120 channels fill 240 compute units in six slices, 160 in four.)  Us a
 // step of 32 sequences before (the power of two that brings 128 workgroups, up to eight) / now: 24 layers of 1024 1308 / 1220, 12 of 2560 1096 /
 // 1071, 8 of 4096 1023 / 1011, 8 of 5120 1289 / 1254; of 16, with four M-tiles (gemm8_skinny_kernel), 905 / 848 of 4096 and 1106 / 1031 of 5120.
+// The launch hands the XCDs whole column blocks, so it is the XCD with the most of them that must not start a second round: 41 blocks of 5248
+// channels in six slices are 246 workgroups, but 36 on the first XCD.  Us a step of 17 / 32 sequences of 3 layers, powers of two / 256 compute units
+// counted as one / by XCD: 3584 355, 398 / 365, 408 / 358, 401; 4224 414, 459 / 417, 465 / 402, 443; 5248 514, 579 / 545, 615 / 495, 557.
 static int skinny_split(int64_t MT, int64_t NT, int64_t KB, int n, int readers) {
     if (!skinny_cut(NT, KB, n)) return 1;
+    const int64_t on_one = ceil_div(ceil_div(NT, kSkinnyNT), kXcds) * n;        // column blocks of the XCD that has the most
     int best = 2;
     int64_t least = INT64_MAX;
     for (int s = 2; s <= kMaxSplit && KB >= 8 * s; ++s) {
         const bool sum = readers && s <= kRowsDeferSlices;
-        const int64_t cost = ceil_div(ceil_div(NT, kSkinnyNT) * n * s, 256) * (kSkinnyNT + (MT <= 4 ? 4 : 8)) * ceil_div(KB, s) +
+        const int64_t cost = ceil_div(on_one * s, 256 / kXcds) * (kSkinnyNT + (MT <= 4 ? 4 : 8)) * ceil_div(KB, s) +
                              (sum && n > 1 ? 8 * s : sum ? 32 + readers * (2 * s + 1) * NT / 16 : 420 + 30 * s * n);
         if (cost < least) { least = cost; best = s; }
     }

@@ -126,6 +126,22 @@ def test_slices_left_to_the_next_kernel_are_whole_and_fit(lib, C_):
     assert most > 1 or C_ <= 320
 
 
+def test_slices_of_9_to_32_rows_fit_each_xcd(lib):
+    """More slices must leave the compute units of the XCD that has the most column blocks (of eight tiles, dealt out in turn) less to draw:
+    rounds of 32 workgroups, times the blocks of one."""
+    seen = set()
+    for C_ in range(256, 6145, 64):
+        for R in (9, 16, 17, 32):
+            for K, n, readers in ((C_, 3, 1), (C_, 1, 1), (4 * C_, 1, 1), (C_, 1, 0), (C_, 1, 2), (4 * C_, 1, 2)):
+                kind, gx, _, s = product_plans.plan(R, K, C_, n, readers)
+                if kind == product_plans.SKINNY and s > 1:
+                    assert gx == -(-C_ // 128)
+                    draw = [-(-(-(-gx // 8) * n * t) // 32) * -(-(K // 64) // t) for t in range(1, s + 1)]
+                    assert draw[-1] == min(draw), (C_, R, K, n, s, draw)
+                    seen.add(s)
+    assert {2, 3, 4, 5, 6} <= seen
+
+
 def test_what_is_handed_on(lib):
     """Short prompts of narrow models and batches of fewer than 128 rows; slices by what they save, no more than the next kernel takes."""
     assert [product_plans.readers(R, C_, s) for R, C_, s in ((127, 5120, False), (128, 512, False), (127, 1024, True), (128, 512, True), (64, 2048, True),
