@@ -72,6 +72,12 @@ constexpr int prep_parts(int C) { return (C + kPrepThreads - 1) / kPrepThreads; 
 static unsigned prep_blocks(const DModel &m) { return (unsigned)((m.L + 1) * prep_parts(m.C)); }   // the token's parts, then each layer's
 constexpr int kRealJobs = 13;          // tile jobs per layer: k v r | o | ffn_r, 4 x ffn_k | 4 quarters of ffn_v
 constexpr unsigned kSpinLimit = 1u << 20;        // polls before a wait gives up (DArgs::spin_limit; a self-test passes a small one)
+// The front's other wavefronts look at an LDS word for what wavefront 0 polls memory for.  It must give up before they do, or they would cut short
+// a wait that is within its bound.  So they may look as often as twice its polls take: a poll (a trip to memory and 128 cycles of sleep) 0.2 to
+// 0.7 us, up to 1700 cycles; a look, without a sleep, no less than the latency of an LDS read.
+constexpr unsigned kLooksPerPoll = 64, kLookCycles = 64, kPollCycles = 1700;
+static_assert(kLooksPerPoll * kLookCycles >= 2 * kPollCycles, "wavefront 0 gives up first");
+static_assert((unsigned long long)kSpinLimit * kLooksPerPoll < 1ull << 32, "looks are counted in 32 bits");
 constexpr int kStatRows = 2;           // XR rows 0-1: sum x of a workgroup's 16 channels, and their squared deviations from the workgroup's own mean
 constexpr int kLnRows = kStatRows + 3 * 3;     // rows of the XR record table
 constexpr int kEarlyDiv = 4;           // gathers start when all but G / kEarlyDiv workgroups have published (measured flat from G/20 to G)
@@ -383,7 +389,7 @@ __device__ __forceinline__ void wait_flag(Front &fx, int which, int seq) {
     unsigned spins = 0;
     while (fx.ok && fx.flags[which] < seq) {
         __builtin_amdgcn_s_sleep(0);
-        if ((++spins & 255u) == 0u && (spins > (fx.spin_limit << 4) || fx.flags[FLAG_ABORT])) fx.fail();
+        if ((++spins & 255u) == 0u && (spins > fx.spin_limit * kLooksPerPoll || fx.flags[FLAG_ABORT])) fx.fail();
     }
 }
 
