@@ -727,7 +727,8 @@ argmax_f64_kernel(const double *__restrict__ logits, int V, int64_t *__restrict_
 // its own, 16 bytes to a lane, eight of them requested before the first is used, so that a lane keeps its columns and nothing is
 // exchanged between lanes; the 16 wavefronts' sums meet in LDS.  Us for both launches, by the other kernel / by this: 768 x 768 7.6 / 6.6,
 // 2560 x 2560 10.2 / 8.6, three of them 16.8 / 11.1, 2560 x 10240 17.0 / 12.3, 10240 x 2560 17.0 / 12.6, 5120 x 5120 17.8 / 11.7, 5120 x 20480
-// 36.6 / 26.0, 768 x 50277 21.0 / 17.8 (26 MB at copy rate: 5.5).  512 columns: 8.9 for 2560 x 2560, 14.2 for the 26 MB shapes; 256 rows,
+// 36.6 / 26.0, 768 x 50277 21.0 / 17.8 (26 MB at copy rate: 5.5).  Of fewer columns most lanes read the last piece again, which costs nothing: 64, 768, 2560
+// and 10240 rows of 16 columns 6.7, 7.4, 7.9, 8.6 / 4.8, 6.3, 6.9, 7.7, of 256 7.3, 7.6, 8.3, 10.0 / 5.5, 6.5, 7.3, 8.7.  512 columns: 8.9 for 2560 x 2560, 14.2 for the 26 MB shapes; 256 rows,
 // 16 of them in flight, 10.4 and 13.7.  Whole contractions of 16, 32 or 64 columns, one launch: 13.1, 19.9 and 32.7 at best.
 //
 // The others (mm8_ref_kernel): 128 columns (whole cache lines of the rows) and up to 256 rows, eight lanes to a row, sums
@@ -747,8 +748,6 @@ struct Mm8RefArgs {
     T *scratch;                 // [split][product][n_out]
 };
 
-// T: float (operators32.cu) or double (operators.cu:58-80, the dispatch of wrapper.cpp:60-77): the type of x, r, y and
-// of the sums.  WIDE: at least 16 columns; narrower matrices are read byte by byte.  LONG: more than 256 rows to a workgroup.
 typedef uint32_t RefPiece __attribute__((ext_vector_type(4), aligned(1)));     // 16 columns (rows may start anywhere)
 template <typename T>
 __device__ __forceinline__ void ref_piece(const RefPiece &w, T xr, T (&acc)[16]) {
@@ -817,6 +816,8 @@ __global__ void __launch_bounds__(kRefRowsThreads) mm8_ref_rows_kernel(const Mm8
     a.scratch[((size_t)blockIdx.y * gridDim.z + m) * a.n_out + k] = sum;
 }
 
+// T: float (operators32.cu) or double (operators.cu:58-80, the dispatch of wrapper.cpp:60-77): the type of x, r, y and
+// of the sums.  WIDE: at least 16 columns; narrower matrices are read byte by byte.  LONG: more than 256 rows to a workgroup.
 template <typename T, bool WIDE, bool LONG>
 __global__ void __launch_bounds__(kRefThreads) mm8_ref_kernel(const Mm8RefArgs<T> a) {
     __shared__ T xs[kRefPasses * kRefRowsPass];

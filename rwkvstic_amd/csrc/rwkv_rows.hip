@@ -943,8 +943,8 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &a, const GemmCols 
 }
 
 // One workgroup of the product: 64 tokens x 16*WN*GN columns, WM*WN wavefronts as WM x WN, each 16/WM M-tiles x GN
-// N-tiles, RING LDS buffers.  <4, 4, 3> is the general shape (8 wavefronts of 4 x 4 tiles, two workgroups per
-// compute unit); <5, 4, 4> (4 x 5 tiles, one workgroup per compute unit) is used where it turns a grid of 1.25
+// N-tiles, RING LDS buffers.  <4, 4, 2, 3> is the general shape (8 wavefronts of 4 x 4 tiles, two workgroups per
+// compute unit); <5, 4, 2, 4> (4 x 5 tiles, one workgroup per compute unit) is used where it turns a grid of 1.25
 // workgroups per compute unit into exactly one (2560 columns: 16 column blocks instead of 20).  <5, 8, 1, 4> (64 x 80: eight wavefronts of 2 x 5
 // tiles) serves grids that leave compute units idle (general_narrow).
 template <int GN, int WM, int WN, int RING, bool STREAM>
@@ -1161,7 +1161,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         __builtin_amdgcn_sched_barrier(0);                                                           \
         _Pragma("unroll") for (int i = 0; i < MT - kLate; ++i) {                                     \
             if (i + 2 < MT) Av_[i + 2] = frag[buf_][i + 2][lane];                                    \
-            if (i + 2 == MT - kLate + 1 && kLate > 1) Av_[MT - 1] = frag[buf_][MT - 1][lane];        \
             if (MT == 8 && i == 0) RWKV_SKINNY_MOVE(FN, 1, v1, buf_ ^ 1, on_)                        \
             if (i == (MT == 8 ? 2 : 0)) RWKV_SKINNY_MOVE(FN, 2, v2, buf_ ^ 1, on_)                   \
             if (i == (MT == 8 ? 4 : 1)) RWKV_SKINNY_MOVE(FN, 3, v3, buf_ ^ 1, on_)                   \
@@ -1211,7 +1210,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 // The wavefronts' sums are added in LDS, each sum by a wavefront of its own that also writes it.
 //
 // Bound: the latency of a few dependent loads per wavefront, then HBM.  So the blocks are spread over as many wavefronts
-// as are resident at once (vec_shape), which needs no split of the contraction and no second launch; wide products take
+// as are resident at once (vec_shape), which needs no second launch: whole contractions, or slices where the next kernel adds them up
+// (vec_split); wide products take
 // several tiles per wavefront, since for two M-tiles the digits are twice a tile's bytes.  8 rows at 2560 channels (us per
 // launch), 4 wavefronts of one tile with 8 blocks in flight / this: k, v, r 10.1 / 6.4, att output 7.4 / 4.9, ffn key and
 // receptance 12.7 + 6.4 / 8.4, ffn value 15.5 / 11.1 (7.5 in three slices: see vec_split), head 43 / 24.9.
@@ -1791,7 +1791,7 @@ constexpr int kGemmWideNum = 10, kGemmWideDen = 9;     // the 64 x 160 variant i
 // ... except a contraction of 200 blocks and more, which splits in two while the grid is below the device (14B shape,
 // 256-token chunks: the [256 x 20480] x [20480 x 5120] product; 14,080 against 13,190 tokens/s)
 constexpr int kGemmLongFillWgs = 256, kGemmLongBlocks = 200;
-constexpr int kSkinnyFillWgs = 128;     // 9..32 rows (weight streaming): the contraction is split until the grid has this many workgroups (batch-32 step: 8.07 ms at 128, 8.73 at 256, 9.17 at 64 for the 14B shape; 4.06 / 4.13 / 4.11 ms for the 3B shape)
+constexpr int kSkinnyFillWgs = 128;     // 9..32 rows (weight streaming): contractions of a grid below this many workgroups are cut in slices, in how many skinny_split says (when it was the number of workgroups to reach, a batch-32 step took 8.07 ms at 128, 8.73 at 256, 9.17 at 64 for the 14B shape; 4.06 / 4.13 / 4.11 ms for the 3B shape)
 // Row blocks of 64 tokens up to which the general kernel reads the weights past the caches: more of them find each other's weight
 // blocks there (prompts, kept / streamed: 77 tokens of 24 layers of 1024 2274 / 2193 us, 100 of the 3B shape 4565 / 4416, 256 of it
 // 6158 / 6248, 256 of 14B 17786 / 18992)
@@ -2235,7 +2235,7 @@ static int launch_general(hipStream_t st, GemmArgs &g, int kind, int gx, bool st
     else if (wide) hipLaunchKernelGGL(gemm8_wide_kernel, grid, dim3(512), 0, st, g);
     else if (stream && g.gy <= kStreamRowBlocks) hipLaunchKernelGGL(gemm8_kernel<true>, grid, dim3(512), 0, st, g);
     else hipLaunchKernelGGL(gemm8_kernel<false>, grid, dim3(512), 0, st, g);
-    RWKV_CHECK_LAUNCH(wide ? "gemm8_wide_kernel" : "gemm8_kernel");
+    RWKV_CHECK_LAUNCH(kind == PLAN_NARROW ? "gemm8_narrow_kernel" : wide ? "gemm8_wide_kernel" : "gemm8_kernel");
     return RWKV_OK;
 }
 
