@@ -170,11 +170,11 @@ quant_minmax_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
     }
 }
 
-// A channel's extrema -> lo, range, 1 / range.
+// A channel's extrema -> lo, range, 1 / range (0 for a constant channel: its quotients are formed all the same, and 0 * inf is no value to convert).
 struct QuantScale { double lo, ran, inv; };
 __device__ __forceinline__ QuantScale quant_scale(float lo, float hi) {
     const double ran = ((double)hi - (double)lo) / 255.0;              // matmul.py:31-33, as quantize_kernel
-    return QuantScale{(double)lo, ran, 1.0 / ran};
+    return QuantScale{(double)lo, ran, ran > 0.0 ? 1.0 / ran : 0.0};
 }
 
 // The correctly rounded quotient d / b from the correctly rounded reciprocal of b (Markstein: a quotient within one
@@ -336,7 +336,7 @@ quant_encode_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in, Qu
         if (j + e < n_in) {
             there |= 0x80u << (8 * e);
             if (ran[e] > 0.0) coded |= 0xffu << (8 * e);
-        }
+        } else lo[e] = ran[e] = inv[e] = 0.0;                       // (past the last channel x is 0, and its code must be one that converts)
     for (int64_t k0 = kbeg; k0 < kend; k0 += kEncRows) {
         if (k0 > kbeg) {
             fetch(k0);
