@@ -57,8 +57,9 @@ namespace rwkv {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-// Widths.  C = 512, 768 and 1536 are bound by the four exchanges per layer (12.3 us per layer at 768): a token of the
-// 12-layer 768 shape takes 158 us, as one-row prompts through the many-row kernels it took 630 us (146 launches).
+// Widths.  C = 512, 768 and 1536 are bound by the four exchanges per layer (at 768, stamps on, 12.5 us a layer, 12.4 with the weights in
+// the caches): a token of the 12-layer 768 shape takes 156 us, 147 of them in this kernel; as one-row prompts through the many-row kernels it
+// took 630 us (146 launches).
 // NB (template parameter throughout): 64-channel blocks of a row of C channels, C = 64 NB.  Back (streaming) waves per
 // workgroup: eight, four up to 1024 channels, where the exchanges and not the stream set the pace and a tile's sums come
 // from four parts instead of eight (24 layers of 1024: 336 us a token, with eight 344; at 1536 they are equal, at 2048 four

@@ -83,15 +83,15 @@ quantize_kernel(const float *__restrict__ W, int64_t n_out, int64_t n_in,
 }
 
 // ---------------------------------------------------------------------------
-// The same quantiser for callers with a workspace: three launches that cut the matrix both ways, and the codes leave
+// The same quantiser for callers with a workspace: two launches that cut the matrix both ways, and the codes leave
 // in any of the three layouts straight from the encoding pass.  Codes, ranges and offsets have quantize_kernel's bits.
 //
 // Bound: memory (the float32 matrix twice, the second time mostly from the memory-side cache, the codes once per
 // layout).  quantize_kernel walks all rows with one workgroup per 64 channels, 40 workgroups at 2560 channels, and
 // the packed layouts then read its codes back byte by byte.  The seven matrices of a layer of width 2560: 5.14 ms
-// that way, 0.325 ms here (host calls included; the 511 MB at copy rate: 0.108).  The offsets' serial sums are 0.03 of it, and
-// more where there are few channels for many rows: a head of 768 x 50277 takes 268 us (97 with the fractions added in
-// parallel), the layer of width 5120 1.18 ms (0.88).
+// that way, 0.282 ms here (0.319 with the host's calls in front of them; the 511 MB at copy rate: 0.108).  The offsets' serial sums cost more
+// where there are few channels for many rows: a head of 768 x 50277 takes 252 us (268 with a launch for the scales, and 97 with the fractions
+// added in parallel), the layer of width 5120 1.00 ms (1.18, and 0.88).
 //
 //   quant_minmax_kernel   256 channels x one of the row splits: partial minimum and maximum
 //   quant_encode_kernel   128 channels x kEncRows rows at a time: codes, layouts; in workgroups of its own the offsets.  Every workgroup
