@@ -342,8 +342,11 @@ __device__ __forceinline__ void add_pending(const RowsDeferred &d, int t, int c,
         }
     }
 }
-template <bool MIX, int NSEG>
-__global__ void __launch_bounds__(kLnRowThreads) rows_ln_mix_quant_row_kernel(const LnQuantArgs a) {
+// TWO: no more than 128 registers, so that two workgroups of five to eight wavefronts fit a compute unit, for grids of more than one to each.  (Of up
+// to 2048 channels it takes 132 otherwise, and the second waits for the first: us a launch of 86 / 127 rows of 1088 channels 8.2 / 9.4, with 128 7.5 /
+// 8.5, of 2048 11.6 / 12.8 and 11.1 / 12.4.  Smaller grids lose 0.1 to 0.3 us to the registers that go to scratch memory.)
+template <bool MIX, int NSEG, bool TWO = false>
+__global__ void __launch_bounds__(kLnRowThreads, TWO ? 4 : 2) rows_ln_mix_quant_row_kernel(const LnQuantArgs a) {
     __shared__ double red0[2 * 8], red1[2 * 8], red2[8], red3[8];
     __shared__ float redf[16];
     const int t = blockIdx.x, m = blockIdx.y, C = a.C, tid = threadIdx.x, nt = blockDim.x, nw = nt >> 6, lane = tid & 63;
@@ -2139,7 +2142,8 @@ int rows_ln_mix_quant(hipStream_t st, int n_mix, int64_t R, int C, bool sequence
             else if (nseg == 2) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<false, 2>), grid, block, 0, st, a);
             else hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<false, 3>), grid, block, 0, st, a);
         } else {
-            if (nseg == 1) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 1>), grid, block, 0, st, a);
+            if (nseg == 1 && threads > kLnRowThreads / 2 && R * n_out > 256) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 1, true>), grid, block, 0, st, a);
+            else if (nseg == 1) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 1>), grid, block, 0, st, a);
             else if (nseg == 2) hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 2>), grid, block, 0, st, a);
             else hipLaunchKernelGGL((rows_ln_mix_quant_row_kernel<true, 3>), grid, block, 0, st, a);
         }

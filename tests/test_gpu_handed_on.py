@@ -42,7 +42,8 @@ def _fn(name, *args):
     (True, 40, 512, 2048, ROW_GATE_ADD), (True, 127, 1024, 1024, ROW_ADD), (True, 33, 1024, 1024, ROW_ADD), (True, 28, 1024, 4096, ROW_GATE_ADD),
     (True, 80, 1536, 6144, ROW_GATE_ADD), (True, 20, 2048, 8192, ROW_GATE_ADD), (True, 64, 2048, 2048, ROW_ADD),
     (False, 8, 1024, 4096, ROW_GATE_ADD), (False, 7, 1536, 6144, ROW_GATE_ADD), (False, 8, 2560, 10240, ROW_GATE_ADD), (False, 32, 1024, 4096, ROW_GATE_ADD),
-    (False, 17, 2560, 10240, ROW_GATE_ADD), (False, 32, 3584, 14336, ROW_GATE_ADD), (False, 32, 5120, 5120, ROW_ADD), (False, 100, 2560, 2560, ROW_ADD)])
+    (False, 17, 2560, 10240, ROW_GATE_ADD), (False, 32, 3584, 14336, ROW_GATE_ADD), (False, 32, 5120, 5120, ROW_ADD), (False, 100, 2560, 2560, ROW_ADD),
+    (True, 100, 1088, 1088, ROW_ADD), (False, 86, 1536, 1536, ROW_ADD), (False, 127, 2048, 2048, ROW_ADD)])   # (more workgroups than compute units)
 def test_slices_handed_on_have_the_bits_of_a_finished_product(sequence, R, width, K, op):
     from rwkvstic_amd import ops
     print(f"handed on: sequence={sequence} R={R} C={width} K={K} op={op}", flush=True)
